@@ -148,6 +148,15 @@ int mg_fused_norm_linear(const void* x_bf16, const void* gamma_bf16, float eps, 
                          const uint8_t* sfbn, const uint8_t* sfbs, const uint8_t* sfbo,
                          int M, int N, int KN, int KS, int KO, unsigned flags,
                          void* d_bf16, void* workspace, size_t workspace_bytes, void* stream);
+/* A layer's call: mg_fused_norm_linear with what follows the GEMM done by the kernel that writes the result.
+ *   n_out     -- d_bf16 is [M, n_out]: the first n_out of the N weight rows are real, the rest padding (a layer's features
+ *                rounded up to whole tiles; N - n_out < 256).
+ *   bias_bf16 -- [n_out] or NULL: d = bf16( bf16(sum) + bias ), the two roundings of an addition after the GEMM. */
+int mg_linear(const void* x_bf16, const void* gamma_bf16, float eps, const int16_t* idx,
+              const uint8_t* bn, const uint8_t* bs, const uint8_t* bo,
+              const uint8_t* sfbn, const uint8_t* sfbs, const uint8_t* sfbo, const void* bias_bf16,
+              int M, int N, int n_out, int KN, int KS, int KO, unsigned flags,
+              void* d_bf16, void* workspace, size_t workspace_bytes, void* stream);
 size_t mg_fused_workspace_bytes(int M, int KN, int KS, int KO);
 
 /*

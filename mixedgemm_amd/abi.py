@@ -7,12 +7,15 @@ the first call raises.
 from __future__ import annotations
 
 import ctypes
+import importlib.machinery
+import importlib.util
 import os
 
 import torch
 
 _PKG = os.path.dirname(os.path.abspath(__file__))
 LIB_PATH = os.path.join(_PKG, "lib", "libmixedgemm_hip.so")
+HOST_PATH = os.path.join(_PKG, "lib", "mixedgemm_torch.so")
 
 MG_OPERAND_A = 0
 MG_OPERAND_B = 1
@@ -24,11 +27,12 @@ SYMBOLS = (
     "mg_fused_linear",
     "mg_fused_workspace_bytes", "mg_sf_bytes", "mg_sf_offset", "mg_device_synchronize", "mg_status_string",
     "mg_calibrate_reorder_index", "mg_calibrate_workspace_bytes", "mg_check_reorder_index", "mg_check_reorder_index_host",
-    "mg_fused_linear_static",
+    "mg_fused_linear_static", "mg_linear",
 )
 MG_STATIC_SCRATCH_BYTES = 20 << 20
 
 _lib = None
+_host = None
 
 
 class MixedGemmError(RuntimeError):
@@ -72,9 +76,26 @@ def lib() -> ctypes.CDLL:
         L.mg_check_reorder_index_host.restype, L.mg_check_reorder_index_host.argtypes = i, [p, i]
         L.mg_fused_linear_static.restype = i
         L.mg_fused_linear_static.argtypes = [p] * 8 + [i] * 5 + [u, p, p]
+        L.mg_linear.restype = i
+        L.mg_linear.argtypes = [p, p, f, p] + [p] * 7 + [i] * 6 + [u, p, p, z, p]
         L.mg_status_string.restype, L.mg_status_string.argtypes = ctypes.c_char_p, [i]
         _lib = L
     return _lib
+
+
+def host():
+    """The native host side of the calls below (csrc/torch_host.cpp): operand checks, allocation and launch in one
+    function.  A call it does not take as it stands returns None; the Python code of the call then says what is wrong."""
+    global _host
+    if _host is None:
+        lib()
+        if not os.path.exists(HOST_PATH):
+            raise MixedGemmError(f"{HOST_PATH} is missing: build it with `python -m mixedgemm_amd.build`")
+        loader = importlib.machinery.ExtensionFileLoader("mixedgemm_torch", HOST_PATH)
+        module = importlib.util.module_from_spec(importlib.util.spec_from_file_location("mixedgemm_torch", HOST_PATH, loader=loader))
+        loader.exec_module(module)
+        _host = module
+    return _host
 
 
 def status_string(status: int) -> str:
@@ -167,6 +188,9 @@ def _capacity(t: torch.Tensor) -> int:
 
 
 def _reorder_quantize(fn_name, operand, t, idx, kn, ks, ko, out=None):
+    got = host().reorder_quantize(operand, t, idx, kn, ks, ko, out)
+    if got is not None:
+        return got
     _require(t, torch.bfloat16, "input")
     _require(idx, torch.int16, "reorder_index")
     rows, k = t.shape
@@ -217,6 +241,9 @@ def reorder_quantize_w(w, reorder_index, kn, ks, ko, out=None):
 def matmul(an, bn, as_, bs, ao, bo, sfan, sfbn, sfas, sfbs, sfao, sfbo, out=None, w_tiled=False):
     """bf16 [M, N]; shapes are recovered from the packed operands.  w_tiled: bn, bs, bo are in the
     tile-major order of tile_weights()."""
+    got = host().matmul(an, bn, as_, bs, ao, bo, sfan, sfbn, sfas, sfbs, sfao, sfbo, out, w_tiled)
+    if got is not None:
+        return got
     for name, t in (("AN", an), ("BN", bn), ("AS", as_), ("BS", bs), ("AO", ao), ("BO", bo),
                     ("SFAN", sfan), ("SFBN", sfbn), ("SFAS", sfas), ("SFBS", sfbs), ("SFAO", sfao), ("SFBO", sfbo)):
         _require(t, torch.uint8, name)
@@ -287,6 +314,9 @@ def fused_linear(x, reorder_index, bn, bs, bo, sfbn, sfbs, sfbo, kn, ks, ko, wor
                  norm_weight=None, eps=0.0):
     """Activation reorder-quantize + mixed GEMM on one stream; returns bf16 [M, N].  With norm_weight
     (bf16 [K]) the activations pass through an RMSNorm first, inside the quantizer's row pass."""
+    got = host().fused_linear(x, reorder_index, bn, bs, bo, sfbn, sfbs, sfbo, kn, ks, ko, workspace, out, w_tiled, norm_weight, eps)
+    if got is not None:
+        return got
     _check_fused_inputs(x, reorder_index, kn, ks, ko)
     m = x.shape[0]
     n = _check_weights(x, bn, bs, bo, sfbn, sfbs, sfbo, kn, ks, ko)
@@ -362,6 +392,9 @@ def tile_weights(wn, ws, wo):
 def calibrate_reorder_index(x, out=None, workspace=None):
     """Reorder index of a bf16 activation sample x[M, K]: channels by ascending max |x| over the
     rows, ties by channel number, int16 (main.py:31-33 of the reference, there as torch calls)."""
+    got = host().calibrate(x, out, workspace)
+    if got is not None:
+        return got
     _require(x, torch.bfloat16, "x")
     if x.dim() != 2:
         raise MixedGemmError(f"x: expected a 2-D tensor [rows, channels], got {x.dim()} dimensions")

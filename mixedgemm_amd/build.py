@@ -5,6 +5,7 @@
 
 Outputs (kept out of git, shipped with the tree):
     mixedgemm_amd/lib/libmixedgemm_hip.so   hand-written gfx950 kernels + extern "C" entry points
+    mixedgemm_amd/lib/mixedgemm_torch.so    host side of the torch calls (operand checks, allocation, launch) on the C-ABI
     mixedgemm_amd/lib/libmixedgemm_bench.so measurement kernels bench.py times next to the library (not the product)
     build/mixedgemm.so                      torch extension with the reference's operator surface
     build/abi_driver                        torch-free host program (tests/c_host) on the C-ABI
@@ -23,6 +24,7 @@ LIB_DIR = os.path.join(PKG, "lib")
 LIB_PATH = os.path.join(LIB_DIR, "libmixedgemm_hip.so")
 EXT_DIR = os.path.join(ROOT, "build")
 EXT_PATH = os.path.join(EXT_DIR, "mixedgemm.so")
+HOST_PATH = os.path.join(LIB_DIR, "mixedgemm_torch.so")
 DRIVER_SRC = os.path.join(ROOT, "tests", "c_host", "abi_driver.cpp")
 DRIVER_PATH = os.path.join(EXT_DIR, "abi_driver")
 
@@ -136,32 +138,42 @@ def build_bench_library(force: bool = False, verbose: bool = False) -> str:
     return _compile_and_link(BENCH_SOURCES, BENCH_LIB_PATH, force, verbose)
 
 
-def build_torch_extension(force: bool = False, verbose: bool = False) -> str:
-    """g++ build of csrc/bindings.cpp against torch + pybind11; links the HIP
-    library through its C-ABI only (no HIP headers on this side)."""
+def _build_torch_module(src_name: str, module: str, target: str, force: bool, verbose: bool) -> str:
+    """g++ build of a torch extension against torch + pybind11; it links the HIP library through its C-ABI only (no HIP
+    kernels on this side)."""
     import torch
     from torch.utils import cpp_extension
 
-    src = os.path.join(CSRC, "bindings.cpp")
+    src = os.path.join(CSRC, src_name)
     deps = [src, os.path.join(ROOT, "include", "mixedgemm_abi.h"), LIB_PATH]
-    if force or _stale(EXT_PATH, deps):
-        os.makedirs(EXT_DIR, exist_ok=True)
+    if force or _stale(target, deps):
+        os.makedirs(os.path.dirname(target), exist_ok=True)
         torch_lib = os.path.join(os.path.dirname(torch.__file__), "lib")
         inc = [f"-I{p}" for p in cpp_extension.include_paths()]
         inc += [f"-I{sysconfig.get_paths()['include']}", f"-I{os.path.join(ROOT, 'include')}"]
         cmd = [
             "g++", "-O2", "-std=c++17", "-fPIC", "-shared", "-fvisibility=hidden",
-            "-DTORCH_EXTENSION_NAME=mixedgemm", "-DTORCH_API_INCLUDE_EXTENSION_H",
+            f"-DTORCH_EXTENSION_NAME={module}", "-DTORCH_API_INCLUDE_EXTENSION_H",
             "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM=1", "-I/opt/rocm/include",
             f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}",
-            *inc, src, "-o", EXT_PATH,
+            *inc, src, "-o", target,
             f"-L{LIB_DIR}", "-lmixedgemm_hip", f"-Wl,-rpath,{LIB_DIR}", "-Wl,-rpath,$ORIGIN/../mixedgemm_amd/lib",
-            f"-L{torch_lib}", "-ltorch", "-ltorch_cpu", "-lc10", "-lc10_hip", "-ltorch_python", f"-Wl,-rpath,{torch_lib}",
+            "-Wl,-rpath,$ORIGIN", f"-L{torch_lib}", "-ltorch", "-ltorch_cpu", "-lc10", "-lc10_hip", "-ltorch_python", f"-Wl,-rpath,{torch_lib}",
         ]
         if verbose:
             print(" ".join(cmd), flush=True)
         subprocess.check_call(cmd)
-    return EXT_PATH
+    return target
+
+
+def build_torch_extension(force: bool = False, verbose: bool = False) -> str:
+    """The module with the reference's operator surface (csrc/bindings.cpp)."""
+    return _build_torch_module("bindings.cpp", "mixedgemm", EXT_PATH, force, verbose)
+
+
+def build_torch_host(force: bool = False, verbose: bool = False) -> str:
+    """The host side of mixedgemm_amd.abi, mixedgemm_amd.linear and the registered operators (csrc/torch_host.cpp)."""
+    return _build_torch_module("torch_host.cpp", "mixedgemm_torch", HOST_PATH, force, verbose)
 
 
 def build_c_host_driver(force: bool = False, verbose: bool = False) -> str:
@@ -181,6 +193,7 @@ def build_all(force: bool = False, verbose: bool = False) -> None:
     build_hip_library(force, verbose)
     build_bench_library(force, verbose)
     build_torch_extension(force, verbose)
+    build_torch_host(force, verbose)
     build_c_host_driver(force, verbose)
 
 

@@ -15,7 +15,8 @@ hipError_t launch_reorder_quant(const void* x, const int16_t* idx, int rows, int
 hipError_t launch_mixed_gemm(const uint8_t* an, const uint8_t* bn, const uint8_t* as_, const uint8_t* bs,
                              const uint8_t* ao, const uint8_t* bo, const uint8_t* sfan, const uint8_t* sfbn,
                              const uint8_t* sfas, const uint8_t* sfbs, const uint8_t* sfao, const uint8_t* sfbo, int M,
-                             int a_rows, int N, int KN, int KS, int KO, unsigned flags, void* d, hipStream_t stream);
+                             int a_rows, int N, int KN, int KS, int KO, unsigned flags, Epilogue ep, void* d,
+                             hipStream_t stream);
 hipError_t launch_tile_weights(const uint8_t* src, uint8_t* dst, int N, int kseg, hipStream_t stream);
 bool mixed_gemm_256_supported(int M, int N, int KN, int KS, int KO);
 size_t calibrate_workspace_bytes(int K);
@@ -81,6 +82,27 @@ hipError_t scratch_ptr(uint8_t** out) {
   return hipSuccess;
 }
 
+int mixed_gemm(const uint8_t* an, const uint8_t* bn, const uint8_t* as_, const uint8_t* bs, const uint8_t* ao,
+                     const uint8_t* bo, const uint8_t* sfan, const uint8_t* sfbn, const uint8_t* sfas,
+                     const uint8_t* sfbs, const uint8_t* sfao, const uint8_t* sfbo, int M, int a_rows, int N, int KN,
+                     int KS, int KO, unsigned flags, const void* bias_bf16, int n_out, void* d_bf16, void* stream) {
+  if (int s = check_split(M, KN, KS, KO)) return s;
+  if (N < 0 || a_rows < M) return MG_ERR_BAD_SHAPE;
+  if (flags & ~MG_FLAG_W_TILED) return MG_ERR_BAD_SHAPE;
+  if ((flags & MG_FLAG_W_TILED) && !mg_weights_tileable(N, KN, KS, KO)) return MG_ERR_UNSUPPORTED;
+  if (n_out < 0 || n_out > N || N - n_out >= 256) return MG_ERR_BAD_SHAPE;
+  if (M == 0 || n_out == 0) return MG_OK;
+  if (bias_bf16 && !aligned16(bias_bf16)) return MG_ERR_BAD_POINTER;
+  if (!ptr_ok(d_bf16, true)) return MG_ERR_BAD_POINTER;
+  if (!ptr_ok(an, KN > 0) || !ptr_ok(bn, KN > 0) || !ptr_ok(as_, KS > 0) || !ptr_ok(bs, KS > 0) ||
+      !ptr_ok(ao, KO > 0) || !ptr_ok(bo, KO > 0))
+    return MG_ERR_BAD_POINTER;
+  if ((KN > 0 && (!sfan || !sfbn)) || (KS > 0 && (!sfas || !sfbs)) || (KO > 0 && (!sfao || !sfbo)))
+    return MG_ERR_BAD_POINTER;
+  return (int)mg::launch_mixed_gemm(an, bn, as_, bs, ao, bo, sfan, sfbn, sfas, sfbs, sfao, sfbo, M, a_rows, N, KN, KS, KO,
+                                    flags, mg::Epilogue{static_cast<const uint16_t*>(bias_bf16), n_out}, d_bf16, static_cast<hipStream_t>(stream));
+}
+
 }  // namespace
 
 extern "C" {
@@ -106,19 +128,8 @@ int mg_mixed_gemm_ex(const uint8_t* an, const uint8_t* bn, const uint8_t* as_, c
                      const uint8_t* bo, const uint8_t* sfan, const uint8_t* sfbn, const uint8_t* sfas,
                      const uint8_t* sfbs, const uint8_t* sfao, const uint8_t* sfbo, int M, int a_rows, int N, int KN,
                      int KS, int KO, unsigned flags, void* d_bf16, void* stream) {
-  if (int s = check_split(M, KN, KS, KO)) return s;
-  if (N < 0 || a_rows < M) return MG_ERR_BAD_SHAPE;
-  if (flags & ~MG_FLAG_W_TILED) return MG_ERR_BAD_SHAPE;
-  if ((flags & MG_FLAG_W_TILED) && !mg_weights_tileable(N, KN, KS, KO)) return MG_ERR_UNSUPPORTED;
-  if (M == 0 || N == 0) return MG_OK;
-  if (!ptr_ok(d_bf16, true)) return MG_ERR_BAD_POINTER;
-  if (!ptr_ok(an, KN > 0) || !ptr_ok(bn, KN > 0) || !ptr_ok(as_, KS > 0) || !ptr_ok(bs, KS > 0) ||
-      !ptr_ok(ao, KO > 0) || !ptr_ok(bo, KO > 0))
-    return MG_ERR_BAD_POINTER;
-  if ((KN > 0 && (!sfan || !sfbn)) || (KS > 0 && (!sfas || !sfbs)) || (KO > 0 && (!sfao || !sfbo)))
-    return MG_ERR_BAD_POINTER;
-  return (int)mg::launch_mixed_gemm(an, bn, as_, bs, ao, bo, sfan, sfbn, sfas, sfbs, sfao, sfbo, M, a_rows, N, KN, KS, KO,
-                                    flags, d_bf16, static_cast<hipStream_t>(stream));
+  return mixed_gemm(an, bn, as_, bs, ao, bo, sfan, sfbn, sfas, sfbs, sfao, sfbo, M, a_rows, N, KN, KS, KO, flags, nullptr, N,
+                    d_bf16, stream);
 }
 
 int mg_mixed_gemm(const uint8_t* an, const uint8_t* bn, const uint8_t* as_, const uint8_t* bs, const uint8_t* ao,
@@ -161,14 +172,15 @@ size_t mg_fused_workspace_bytes(int M, int KN, int KS, int KO) {
          align256(mg_sf_bytes(R, KO, MG_OPERAND_A));
 }
 
-int mg_fused_norm_linear(const void* x_bf16, const void* gamma_bf16, float eps, const int16_t* idx, const uint8_t* bn,
+int mg_linear(const void* x_bf16, const void* gamma_bf16, float eps, const int16_t* idx, const uint8_t* bn,
                          const uint8_t* bs, const uint8_t* bo, const uint8_t* sfbn, const uint8_t* sfbs,
-                         const uint8_t* sfbo, int M, int N, int KN, int KS, int KO, unsigned flags, void* d_bf16,
+                         const uint8_t* sfbo, const void* bias_bf16, int M, int N, int n_out, int KN, int KS, int KO, unsigned flags, void* d_bf16,
                          void* workspace, size_t workspace_bytes, void* stream) {
   if (gamma_bf16 != nullptr && !(eps >= 0.0f)) return MG_ERR_BAD_SHAPE;
   if (int s = check_split(M, KN, KS, KO)) return s;
-  if (N < 0) return MG_ERR_BAD_SHAPE;
-  if (M == 0 || N == 0) return MG_OK;
+  if (N < 0 || n_out < 0 || n_out > N || N - n_out >= 256) return MG_ERR_BAD_SHAPE;
+  if (M == 0 || n_out == 0) return MG_OK;
+  if (bias_bf16 && !aligned16(bias_bf16)) return MG_ERR_BAD_POINTER;
   if (!workspace || (reinterpret_cast<uintptr_t>(workspace) & 255u)) return MG_ERR_BAD_POINTER;
   if (workspace_bytes < mg_fused_workspace_bytes(M, KN, KS, KO)) return MG_ERR_BAD_SHAPE;
   const int R = mg_padded_rows(M);
@@ -183,7 +195,16 @@ int mg_fused_norm_linear(const void* x_bf16, const void* gamma_bf16, float eps, 
   if (int s = reorder_quantize<false>(x_bf16, idx, M, KN + KS + KO, KN, KS, KO, qn, qs, qo, sfn, sfs, sfo, stream, gamma_bf16, eps,
                                       /*keep_codes=*/true))
     return s;
-  return mg_mixed_gemm_ex(qn, bn, qs, bs, qo, bo, sfn, sfbn, sfs, sfbs, sfo, sfbo, M, R, N, KN, KS, KO, flags, d_bf16, stream);
+  return mixed_gemm(qn, bn, qs, bs, qo, bo, sfn, sfbn, sfs, sfbs, sfo, sfbo, M, R, N, KN, KS, KO, flags, bias_bf16, n_out, d_bf16,
+                    stream);
+}
+
+int mg_fused_norm_linear(const void* x_bf16, const void* gamma_bf16, float eps, const int16_t* idx, const uint8_t* bn,
+                         const uint8_t* bs, const uint8_t* bo, const uint8_t* sfbn, const uint8_t* sfbs,
+                         const uint8_t* sfbo, int M, int N, int KN, int KS, int KO, unsigned flags, void* d_bf16,
+                         void* workspace, size_t workspace_bytes, void* stream) {
+  return mg_linear(x_bf16, gamma_bf16, eps, idx, bn, bs, bo, sfbn, sfbs, sfbo, nullptr, M, N, N, KN, KS, KO, flags, d_bf16,
+                   workspace, workspace_bytes, stream);
 }
 
 int mg_fused_linear_ex(const void* x_bf16, const int16_t* idx, const uint8_t* bn, const uint8_t* bs, const uint8_t* bo,

@@ -55,6 +55,19 @@ inline hipError_t allow_dynamic_lds(const void* kernel, int bytes) {
   return e;
 }
 
+// What a GEMM does with its result on the way out: the first n_out of the N computed features are stored (the rest are a
+// layer's padding), rows n_out values apart, with a bias added to the rounded sum when there is one.
+struct Epilogue {
+  const uint16_t* bias;   // bf16 [n_out] (16-byte aligned), or null
+  int n_out;
+};
+
+// bf16(float(h) + float(b)): the addition of two bf16 tensors
+__device__ __forceinline__ uint16_t add_bf16(uint16_t h, uint16_t b) {
+  const float s = __uint_as_float((unsigned)h << 16) + __uint_as_float((unsigned)b << 16);
+  return __builtin_bit_cast(uint16_t, (__bf16)s);
+}
+
 // LDS bytes a workgroup may use and the number of CUs of the current device (asked once per device).
 struct DeviceLimits { int lds_bytes, cus; };
 inline hipError_t device_limits(DeviceLimits* out) {

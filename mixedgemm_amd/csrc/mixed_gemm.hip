@@ -64,6 +64,32 @@ __device__ __forceinline__ v8i load_frag(const uint8_t* __restrict__ step, int g
   return f;
 }
 
+// Up to four consecutive features n ... n + 3 of token m, rounded to bf16, with the epilogue's bias.
+__device__ __forceinline__ void store4(uint16_t* __restrict__ d, const Epilogue& ep, int m, int n, v4f sum) {
+  if (n >= ep.n_out) return;
+  uint16_t h[4];
+#pragma unroll
+  for (int v = 0; v < 4; ++v) {
+    h[v] = __builtin_bit_cast(uint16_t, (__bf16)sum[v]);
+    if (ep.bias && n + v < ep.n_out) h[v] = add_bf16(h[v], ep.bias[n + v]);
+  }
+  uint16_t* dst = d + (size_t)m * ep.n_out + n;
+  if (n + 3 < ep.n_out && (ep.n_out & 3) == 0 && (n & 3) == 0) {
+    *reinterpret_cast<v2u*>(dst) = v2u{(unsigned)h[0] | ((unsigned)h[1] << 16), (unsigned)h[2] | ((unsigned)h[3] << 16)};
+  } else {
+#pragma unroll
+    for (int v = 0; v < 4; ++v)
+      if (n + v < ep.n_out) dst[v] = h[v];
+  }
+}
+// One feature.
+__device__ __forceinline__ void store1(uint16_t* __restrict__ d, const Epilogue& ep, int m, int n, float sum) {
+  if (n >= ep.n_out) return;
+  uint16_t h = __builtin_bit_cast(uint16_t, (__bf16)sum);
+  if (ep.bias) h = add_bf16(h, ep.bias[n]);
+  d[(size_t)m * ep.n_out + n] = h;
+}
+
 // One K segment, operands read straight from global memory.  Wave tile:
 // 16 tokens x (16*NT) output features.
 template <int FMT, int NT>
@@ -101,7 +127,7 @@ mixed_gemm_direct_kernel(const uint8_t* __restrict__ an, const uint8_t* __restri
                          const uint8_t* __restrict__ sfan, const uint8_t* __restrict__ sfbn,
                          const uint8_t* __restrict__ sfas, const uint8_t* __restrict__ sfbs,
                          const uint8_t* __restrict__ sfao, const uint8_t* __restrict__ sfbo, int M, int N, int KN, int KS,
-                         int KO, uint16_t* __restrict__ d) {
+                         int KO, Epilogue ep, uint16_t* __restrict__ d) {
   constexpr int NT = 4;
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int m = blockIdx.y * 64 + wave * 16 + (lane & 15);
@@ -120,17 +146,7 @@ mixed_gemm_direct_kernel(const uint8_t* __restrict__ an, const uint8_t* __restri
 #pragma unroll
   for (int t = 0; t < NT; ++t) {
     const int n = n_base + 16 * t + 4 * (lane >> 4);
-    uint16_t h[4];
-#pragma unroll
-    for (int v = 0; v < 4; ++v) h[v] = __builtin_bit_cast(uint16_t, (__bf16)acc[t][v]);
-    uint16_t* dst = d + (size_t)m * N + n;
-    if (n + 3 < N && (N & 3) == 0) {
-      *reinterpret_cast<v2u*>(dst) = v2u{(unsigned)h[0] | ((unsigned)h[1] << 16), (unsigned)h[2] | ((unsigned)h[3] << 16)};
-    } else {
-#pragma unroll
-      for (int v = 0; v < 4; ++v)
-        if (n + v < N) dst[v] = h[v];
-    }
+    store4(d, ep, m, n, acc[t]);
   }
 }
 
@@ -163,7 +179,7 @@ __device__ __forceinline__ v4f decode_mfma(v8i wb, v8i xa, v4f acc, int sw, int 
 template <int G, int F>
 __global__ void __launch_bounds__(256)
 mixed_gemm_skinny_kernel(DecodeSeg s4, DecodeSeg s6, DecodeSeg s8, int M, int N, int steps_per_wave,
-                         int w_tiled, uint16_t* __restrict__ d) {
+                         int w_tiled, Epilogue ep, uint16_t* __restrict__ d) {
   constexpr int S = G * F >= 8 ? 1 : 8 / (G * F);   // K steps a wave keeps in flight at once
   __shared__ float partial[4][F][G][16 * 16];
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -313,13 +329,10 @@ mixed_gemm_skinny_kernel(DecodeSeg s4, DecodeSeg s6, DecodeSeg s8, int M, int N,
         for (int v = 0; v < 4; ++v) {
           const int t = 4 * g + v;
           const int row = tile_row0[f] + 16 * (2 * (t & 7) + (t >> 3));
-          if (row < N) d[(size_t)m * N + row] = __builtin_bit_cast(uint16_t, (__bf16)sum[v]);
+          store1(d, ep, m, row, sum[v]);
         }
       } else {
-        uint16_t* dst = d + (size_t)m * N + nn;
-#pragma unroll
-        for (int v = 0; v < 4; ++v)
-          if (nn + v < N) dst[v] = __builtin_bit_cast(uint16_t, (__bf16)sum[v]);
+        store4(d, ep, m, nn, sum);
       }
     }
   }
@@ -436,7 +449,7 @@ __device__ __forceinline__ void wait_vmcnt() { asm volatile("s_waitcnt vmcnt(%0)
 template <int F, bool WT, int G>
 __global__ void __launch_bounds__(256)
 mixed_gemm_decode_kernel(DecodeSeg s4, DecodeSeg s6, DecodeSeg s8, int M, int N, int steps_per_wave, DecodeLds L,
-                         uint16_t* __restrict__ d) {
+                         Epilogue ep, uint16_t* __restrict__ d) {
   static_assert(G == 1 || G == 2, "token groups of 16 per workgroup");
   constexpr int S = 4;        // K steps per round
   constexpr int PB = 4 * F;   // weight scale pieces per step
@@ -444,7 +457,7 @@ mixed_gemm_decode_kernel(DecodeSeg s4, DecodeSeg s6, DecodeSeg s8, int M, int N,
   static_assert(F == 1 || F == 2 || F == 4, "pieces per step as a power of two");
   extern __shared__ __align__(16) uint8_t lds[];
   pin_args(s4); pin_args(s6); pin_args(s8); pin_args(L);
-  asm volatile("" : "+s"(M), "+s"(N), "+s"(steps_per_wave), "+s"(d));
+  asm volatile("" : "+s"(M), "+s"(N), "+s"(steps_per_wave), "+s"(d), "+s"(ep.bias), "+s"(ep.n_out));
   const unsigned lds0 = (unsigned)(size_t)(__attribute__((address_space(3))) uint8_t*)lds;
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int i = lane & 15, g = lane >> 4;
@@ -686,30 +699,19 @@ mixed_gemm_decode_kernel(DecodeSeg s4, DecodeSeg s6, DecodeSeg s8, int M, int N,
     for (int w = 0; w < 4; ++w) sum += *reinterpret_cast<const v4f*>(partial + ((w * (F * G) + fg) * 64 + lane) * 4);
     const int m = m_base + 16 * gi + i;
     if (m < M) {
-      uint16_t h[4];
-#pragma unroll
-      for (int v = 0; v < 4; ++v) h[v] = __builtin_bit_cast(uint16_t, (__bf16)sum[v]);
       if constexpr (WT) {
         // feature slot e = 4 g + v of the block is row j + 32 (e % 8) + 16 (e / 8) of the tile
         const int bx = wg * F + f, row0 = (bx >> 4) * 256 + (bx & 15);
 #pragma unroll
         for (int v = 0; v < 4; ++v) {
           const int e = 4 * g + v, row = row0 + 32 * (e & 7) + 16 * (e >> 3);
-          if (row < N) d[(size_t)m * N + row] = h[v];
+          store1(d, ep, m, row, sum[v]);
         }
       } else {
         // feature slots 4 g ... 4 g + 3 of the group are four consecutive rows
         const int per_group = 32 / PB, group = blockIdx.x / per_group, c0 = (blockIdx.x % per_group) * PB;
         const int e = 16 * f + 4 * g;
-        const int nn = group * 128 + c0 + e % PB + 32 * (e / PB);
-        uint16_t* dst = d + (size_t)m * N + nn;
-        if (nn + 3 < N && (N & 3) == 0) {
-          *reinterpret_cast<v2u*>(dst) = v2u{(unsigned)h[0] | ((unsigned)h[1] << 16), (unsigned)h[2] | ((unsigned)h[3] << 16)};
-        } else {
-#pragma unroll
-          for (int v = 0; v < 4; ++v)
-            if (nn + v < N) dst[v] = h[v];
-        }
+        store4(d, ep, m, group * 128 + c0 + e % PB + 32 * (e / PB), sum);
       }
     }
   }
@@ -770,14 +772,14 @@ static int decode2_feature_groups(const DecodeSeg& d4, const DecodeSeg& d6, cons
 }
 
 hipError_t launch_skinny(const DecodeSeg& d4, const DecodeSeg& d6, const DecodeSeg& d8, int M, int N,
-                         bool w_tiled, uint16_t* d, hipStream_t stream) {
+                         bool w_tiled, Epilogue ep, uint16_t* d, hipStream_t stream) {
   const int rows = M;
   DeviceLimits lim;
   if (hipError_t e = device_limits(&lim); e != hipSuccess) return e;
   // decode: the kernel that stages everything but the weight codes in LDS
   // (a segment's weight codes below 4 GB: the kernel addresses them with 32-bit per-lane offsets)
   const size_t widest = (size_t)(d4.nblk > d6.nblk ? (d4.nblk > d8.nblk ? d4.nblk : d8.nblk) : (d6.nblk > d8.nblk ? d6.nblk : d8.nblk));
-  typedef void (*kernel_t)(DecodeSeg, DecodeSeg, DecodeSeg, int, int, int, DecodeLds, uint16_t*);
+  typedef void (*kernel_t)(DecodeSeg, DecodeSeg, DecodeSeg, int, int, int, DecodeLds, Epilogue, uint16_t*);
   const bool whole_steps = ((d4.nblk | d6.nblk | d8.nblk) & 3) == 0 && (size_t)N * widest * 16 < ((size_t)1 << 32);
   const int spw = (d4.steps + d6.steps + d8.steps + 3) / 4;
   if (M <= 16 && whole_steps) {
@@ -795,7 +797,7 @@ hipError_t launch_skinny(const DecodeSeg& d4, const DecodeSeg& d6, const DecodeS
           {mixed_gemm_decode_kernel<1, true, 1>, mixed_gemm_decode_kernel<2, true, 1>, mixed_gemm_decode_kernel<4, true, 1>}};
       const kernel_t kernel = kernels[w_tiled ? 1 : 0][f == 4 ? 2 : f - 1];
       if (hipError_t e = allow_dynamic_lds(reinterpret_cast<const void*>(kernel), kDecodeLds1); e != hipSuccess) return e;
-      hipLaunchKernelGGL(kernel, grid, dim3(256), (size_t)L.total, stream, d4, d6, d8, M, N, spw, L, d);
+      hipLaunchKernelGGL(kernel, grid, dim3(256), (size_t)L.total, stream, d4, d6, d8, M, N, spw, L, ep, d);
       return hipGetLastError();
     }
   }
@@ -814,7 +816,7 @@ hipError_t launch_skinny(const DecodeSeg& d4, const DecodeSeg& d6, const DecodeS
           {mixed_gemm_decode_kernel<1, true, 2>, mixed_gemm_decode_kernel<2, true, 2>, mixed_gemm_decode_kernel<4, true, 2>}};
       const kernel_t kernel = kernels[w_tiled ? 1 : 0][f == 4 ? 2 : f - 1];
       if (hipError_t e = allow_dynamic_lds(reinterpret_cast<const void*>(kernel), kDecodeLds2); e != hipSuccess) return e;
-      hipLaunchKernelGGL(kernel, grid, dim3(256), (size_t)L.total, stream, d4, d6, d8, M, N, spw, L, d);
+      hipLaunchKernelGGL(kernel, grid, dim3(256), (size_t)L.total, stream, d4, d6, d8, M, N, spw, L, ep, d);
       return hipGetLastError();
     }
   }
@@ -825,16 +827,16 @@ hipError_t launch_skinny(const DecodeSeg& d4, const DecodeSeg& d6, const DecodeS
   const int wt = w_tiled ? 1 : 0;
   switch (g) {
     case 1:
-      if (f == 2) hipLaunchKernelGGL((mixed_gemm_skinny_kernel<1, 2>), grid, dim3(256), 0, stream, d4, d6, d8, M, N, steps_per_wave, wt, d);
-      else hipLaunchKernelGGL((mixed_gemm_skinny_kernel<1, 1>), grid, dim3(256), 0, stream, d4, d6, d8, M, N, steps_per_wave, wt, d);
+      if (f == 2) hipLaunchKernelGGL((mixed_gemm_skinny_kernel<1, 2>), grid, dim3(256), 0, stream, d4, d6, d8, M, N, steps_per_wave, wt, ep, d);
+      else hipLaunchKernelGGL((mixed_gemm_skinny_kernel<1, 1>), grid, dim3(256), 0, stream, d4, d6, d8, M, N, steps_per_wave, wt, ep, d);
       break;
     case 2:
-      if (f == 2) hipLaunchKernelGGL((mixed_gemm_skinny_kernel<2, 2>), grid, dim3(256), 0, stream, d4, d6, d8, M, N, steps_per_wave, wt, d);
-      else hipLaunchKernelGGL((mixed_gemm_skinny_kernel<2, 1>), grid, dim3(256), 0, stream, d4, d6, d8, M, N, steps_per_wave, wt, d);
+      if (f == 2) hipLaunchKernelGGL((mixed_gemm_skinny_kernel<2, 2>), grid, dim3(256), 0, stream, d4, d6, d8, M, N, steps_per_wave, wt, ep, d);
+      else hipLaunchKernelGGL((mixed_gemm_skinny_kernel<2, 1>), grid, dim3(256), 0, stream, d4, d6, d8, M, N, steps_per_wave, wt, ep, d);
       break;
     default:   // 4 token groups: skinny_groups takes no more
-      if (f == 2) hipLaunchKernelGGL((mixed_gemm_skinny_kernel<4, 2>), grid, dim3(256), 0, stream, d4, d6, d8, M, N, steps_per_wave, wt, d);
-      else hipLaunchKernelGGL((mixed_gemm_skinny_kernel<4, 1>), grid, dim3(256), 0, stream, d4, d6, d8, M, N, steps_per_wave, wt, d);
+      if (f == 2) hipLaunchKernelGGL((mixed_gemm_skinny_kernel<4, 2>), grid, dim3(256), 0, stream, d4, d6, d8, M, N, steps_per_wave, wt, ep, d);
+      else hipLaunchKernelGGL((mixed_gemm_skinny_kernel<4, 1>), grid, dim3(256), 0, stream, d4, d6, d8, M, N, steps_per_wave, wt, ep, d);
       break;
   }
   return hipGetLastError();
@@ -847,8 +849,8 @@ bool mixed_gemm_256_supported(int M, int N, int KN, int KS, int KO);
 hipError_t launch_mixed_gemm_256(const uint8_t* an, const uint8_t* bn, const uint8_t* as_, const uint8_t* bs,
                                  const uint8_t* ao, const uint8_t* bo, const uint8_t* sfan, const uint8_t* sfbn,
                                  const uint8_t* sfas, const uint8_t* sfbs, const uint8_t* sfao, const uint8_t* sfbo,
-                                 int m_store, int a_rows, int N, int KN, int KS, int KO, bool w_tiled, void* d,
-                                 hipStream_t stream);
+                                 int m_store, int a_rows, int N, int KN, int KS, int KO, bool w_tiled, Epilogue ep,
+                                 void* d, hipStream_t stream);
 
 // Rough launch times in microseconds, only to choose between the kernels for fewer than 256 tokens (measured on
 // MI355X, 256 CUs, K = 4096: the whole-tile kernel runs such problems as 256 x 128 tiles when that is at most one
@@ -880,7 +882,8 @@ static double skinny_us(const DecodeSeg& d4, const DecodeSeg& d6, const DecodeSe
 hipError_t launch_mixed_gemm(const uint8_t* an, const uint8_t* bn, const uint8_t* as_, const uint8_t* bs,
                              const uint8_t* ao, const uint8_t* bo, const uint8_t* sfan, const uint8_t* sfbn,
                              const uint8_t* sfas, const uint8_t* sfbs, const uint8_t* sfao, const uint8_t* sfbo, int M,
-                             int a_rows, int N, int KN, int KS, int KO, unsigned flags, void* d, hipStream_t stream) {
+                             int a_rows, int N, int KN, int KS, int KO, unsigned flags, Epilogue ep, void* d,
+                             hipStream_t stream) {
   if (M == 0 || N == 0) return hipSuccess;
   const bool w_tiled = (flags & 1u) != 0;   // MG_FLAG_W_TILED
   // tile-major weights exist only for shapes the 256x256 kernel takes
@@ -901,13 +904,13 @@ hipError_t launch_mixed_gemm(const uint8_t* an, const uint8_t* bn, const uint8_t
   if (mixed_gemm_256_supported(m_pad, N, KN, KS, KO) &&
       (M >= 256 || pipelined_us(M, N, steps, cus) < skinny_us(d4, d6, d8, M, N, steps, cus, w_tiled)))
     return launch_mixed_gemm_256(an, bn, as_, bs, ao, bo, sfan, sfbn, sfas, sfbs, sfao, sfbo, M, a_rows, N, KN, KS, KO,
-                                 w_tiled, d, stream);
-  if (M < 256 && KN + KS + KO > 0) return launch_skinny(d4, d6, d8, M, N, w_tiled, static_cast<uint16_t*>(d), stream);
+                                 w_tiled, ep, d, stream);
+  if (M < 256 && KN + KS + KO > 0) return launch_skinny(d4, d6, d8, M, N, w_tiled, ep, static_cast<uint16_t*>(d), stream);
   // what is left (256 tokens or more with N not a multiple of 8, or with a segment that is not whole 128-wide
   // stages next to an empty one): the direct kernel
   dim3 grid(ceil_div(N, 64), ceil_div(M, 64));
   hipLaunchKernelGGL(mixed_gemm_direct_kernel, grid, dim3(256), 0, stream, an, bn, as_, bs, ao, bo, sfan, sfbn, sfas, sfbs,
-                     sfao, sfbo, M, N, KN, KS, KO, static_cast<uint16_t*>(d));
+                     sfao, sfbo, M, N, KN, KS, KO, ep, static_cast<uint16_t*>(d));
   return hipGetLastError();
 }
 

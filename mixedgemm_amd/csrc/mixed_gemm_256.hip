@@ -50,6 +50,8 @@ constexpr int kCopySlots = kWCopies + kXSlots + 1;     // + the scale copy
 constexpr int kSplit = 3;                              // slots [0, kSplit) go out in the second half of a stage, the rest in the next first half
 
 typedef int v6i __attribute__((ext_vector_type(6)));
+typedef uint16_t v8h __attribute__((ext_vector_type(8)));
+typedef v4u v4u_any __attribute__((aligned(2)));   // a 16-byte piece anywhere in a bf16 row
 
 // Kernel arguments: per K segment (0: E2M1, 1: E3M2, 2: E4M3 activations) the code and scale
 // pointers and the number of 128-wide stages.
@@ -935,10 +937,11 @@ __device__ __forceinline__ int stages_of(const Plan& p) {
 // NLAST: see run_segment (the launcher picks the instance from the plan).
 // Computes one tile of 256 features x 128 * TM tokens: feature tile tile_n, token tile tile_m (of 128 * TM rows).
 template <bool REGULAR, bool REM, bool WT, int SEGS, int TM, int NLAST>
-__device__ __forceinline__ void compute_tile(const Plan& plan, int tile_n, int tile_m, int tiles_n, int N, int m_store,
-                                             int a_rows, uint16_t* __restrict__ d, uint8_t* lds) {
+__device__ __forceinline__ void compute_tile(const Plan& plan, int tile_n, int tile_m, int tiles_n, const Epilogue& ep,
+                                             int m_store, int a_rows, uint16_t* __restrict__ d, uint8_t* lds) {
   static_assert(TM == 2 || TM == 1, "wave tiles of 128 features x 32 * TM tokens");
   const int tid = threadIdx.x;
+  const int N = ep.n_out;   // features past it are padding: computed where a tile has them, never stored
   Ctx c;
   c.lane = tid & 63;
   c.wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -1093,26 +1096,58 @@ __device__ __forceinline__ void compute_tile(const Plan& plan, int tile_n, int t
     const uint8_t* rd = stage + r * kPitch + cc * 16;
     uint16_t* out = d + (size_t)(c.m0 + c.wm * (32 * TM) + r) * N + c.n0 + c.wn * 128 + cc * 8;
     // token rows at or past m_store are not written, nor the 8-feature pieces past the layer's last feature
-    const int rows_left = (c.wn * 128 + cc * 8 < c.cols_avail) ? m_store - (c.m0 + c.wm * (32 * TM) + r) : 0;
+    const int cols_left = c.cols_avail - (c.wn * 128 + cc * 8);
+    const int rows_left = cols_left > 0 ? m_store - (c.m0 + c.wm * (32 * TM) + r) : 0;
+    // the lane's eight features' bias, added to the rounded sums
+    v8h bias = {0, 0, 0, 0, 0, 0, 0, 0};
+    if (ep.bias != nullptr) {   // wave-uniform
+      const uint16_t* bp = ep.bias + c.n0 + c.wn * 128 + cc * 8;
+      if (cols_left >= 8) bias = *reinterpret_cast<const v8h*>(bp);
+      else
+#pragma unroll
+        for (int e = 0; e < 8; ++e) bias[e] = e < cols_left ? bp[e] : (uint16_t)0;
+    }
+    auto with_bias = [&](v4u v) {
+      v8h h = __builtin_bit_cast(v8h, v);
+#pragma unroll
+      for (int e = 0; e < 8; ++e) h[e] = add_bf16(h[e], bias[e]);
+      return __builtin_bit_cast(v4u, h);
+    };
     // Eight reads in flight, then their eight stores: a read that is waited for before its own store costs a
     // full LDS latency per row (which is what the compiler makes of the predicated form: it sinks each read
     // into its store's block -- hence the separate path for tiles that are stored whole).  Streaming stores: the result is not read again here, and the XCD's L2 is
-    // better spent on the operands.
+    // better spent on the operands.  A feature count that is not a multiple of 8 makes the rows start at odd places: the
+    // same 16-byte stores, unaligned, and single values in the last piece of a row.
     auto write_rows = [&](auto whole) {
 #pragma unroll
       for (int b = 0; b < TM; ++b) {
         v4u v[8];
 #pragma unroll
         for (int j = 0; j < 8; ++j) v[j] = *reinterpret_cast<const v4u*>(rd + (b * 8 + j) * 4 * kPitch);
+        if (ep.bias != nullptr)
+#pragma unroll
+          for (int j = 0; j < 8; ++j) v[j] = with_bias(v[j]);
 #pragma unroll
         for (int j = 0; j < 8; ++j) {
           const int i = b * 8 + j;
-          if (decltype(whole)::value || i * 4 < rows_left)
-            __builtin_nontemporal_store(v[j], reinterpret_cast<v4u*>(out + (size_t)i * 4 * N));
+          uint16_t* dst = out + (size_t)i * 4 * N;
+          if constexpr (decltype(whole)::value) {
+            __builtin_nontemporal_store(v[j], reinterpret_cast<v4u*>(dst));
+          } else if (i * 4 < rows_left) {
+            if (cols_left >= 8) {
+              __builtin_nontemporal_store(v[j], reinterpret_cast<v4u_any*>(dst));
+            } else {
+              const v8h h = __builtin_bit_cast(v8h, v[j]);
+#pragma unroll
+              for (int e = 0; e < 7; ++e)
+                if (e < cols_left) dst[e] = h[e];
+            }
+          }
         }
       }
     };
-    if (m_store - c.m0 >= kTokens && c.cols_avail == kT) write_rows(std::true_type{});   // wave-uniform: the whole tile is stored
+    // wave-uniform: the whole tile is stored, in aligned pieces
+    if (m_store - c.m0 >= kTokens && c.cols_avail == kT && (N & 7) == 0) write_rows(std::true_type{});
     else write_rows(std::false_type{});
   }
 }
@@ -1120,13 +1155,13 @@ __device__ __forceinline__ void compute_tile(const Plan& plan, int tile_n, int t
 
 template <bool REGULAR, bool REM, bool WT, int SEGS = 7, int TM = 2, int NLAST = 0>
 __global__ void __launch_bounds__(64 * kWaves) __attribute__((amdgpu_waves_per_eu(2, 2)))
-mixed_gemm_256_kernel(Plan plan_arg, int tiles_n, int N, int m_store, int a_rows, uint16_t* __restrict__ d, int first_round,
+mixed_gemm_256_kernel(Plan plan_arg, int tiles_n, Epilogue ep, int m_store, int a_rows, uint16_t* __restrict__ d, int first_round,
                       int skew) {
   extern __shared__ __align__(16) uint8_t lds[];
   const Plan plan = start_workgroup<WT>(plan_arg, first_round, skew);
   int tile_n, tile_m;
   tile_of(blockIdx.x, gridDim.x, tiles_n, tile_n, tile_m, first_round, 128 * TM);
-  compute_tile<REGULAR, REM, WT, SEGS, TM, NLAST>(plan, tile_n, tile_m, tiles_n, N, m_store, a_rows, d, lds);
+  compute_tile<REGULAR, REM, WT, SEGS, TM, NLAST>(plan, tile_n, tile_m, tiles_n, ep, m_store, a_rows, d, lds);
 }
 
 // The same for problems whose last round of 256 x 256 tiles would leave at least half of the CUs idle: the first
@@ -1136,7 +1171,7 @@ mixed_gemm_256_kernel(Plan plan_arg, int tiles_n, int N, int m_store, int a_rows
 // and the CUs that work while the others idle get the clock the others do not use.
 template <bool REM, bool WT, int NLAST>
 __global__ void __launch_bounds__(64 * kWaves) __attribute__((amdgpu_waves_per_eu(2, 2)))
-mixed_gemm_256_tail_kernel(Plan plan_arg, int tiles_n, int N, int m_store, int a_rows, uint16_t* __restrict__ d, int first_round,
+mixed_gemm_256_tail_kernel(Plan plan_arg, int tiles_n, Epilogue ep, int m_store, int a_rows, uint16_t* __restrict__ d, int first_round,
                            int skew, int n_whole) {
   extern __shared__ __align__(16) uint8_t lds[];
   const Plan plan = start_workgroup<WT>(plan_arg, first_round, skew);
@@ -1145,7 +1180,7 @@ mixed_gemm_256_tail_kernel(Plan plan_arg, int tiles_n, int N, int m_store, int a
   int tile_n, tile_m;
   if (wg < n_whole) {
     tile_of(wg, ntiles, tiles_n, tile_n, tile_m);
-    compute_tile<true, REM, WT, 7, 2, NLAST>(plan, tile_n, tile_m, tiles_n, N, m_store, a_rows, d, lds);
+    compute_tile<true, REM, WT, 7, 2, NLAST>(plan, tile_n, tile_m, tiles_n, ep, m_store, a_rows, d, lds);
   } else {
     // Where the XCDs walk bands of feature tiles, the two halves of a tile go to the XCD that holds the tile's band
     // (workgroups 8 apart): its L2 then fetches the weight tile once for both, and the tiles left over in a band
@@ -1162,7 +1197,7 @@ mixed_gemm_256_tail_kernel(Plan plan_arg, int tiles_n, int N, int m_store, int a
     }
     const int half_m = 2 * tile_m + upper;
     if (half_m * 128 >= m_store) return;   // the lower half of a ragged last tile: no token of it exists
-    compute_tile<true, REM, WT, 7, 1, NLAST>(plan, tile_n, half_m, tiles_n, N, m_store, a_rows, d, lds);
+    compute_tile<true, REM, WT, 7, 1, NLAST>(plan, tile_n, half_m, tiles_n, ep, m_store, a_rows, d, lds);
   }
 }
 
@@ -1189,7 +1224,7 @@ static int tile_tokens(int m_store, int N, int cus) {
   return tiles <= cus / 2 ? 128 : 256;
 }
 
-typedef void (*kernel_t)(Plan, int, int, int, int, uint16_t*, int, int);
+typedef void (*kernel_t)(Plan, int, Epilogue, int, int, uint16_t*, int, int);
 
 // The kernel for a plan: segs = which activation segments exist (bit 0 E2M1, 1 E3M2, 2 E4M3), nlast = stages of the
 // last one (3 = three or more), regular = every segment but the last has at least three stages.  Plans with an empty
@@ -1219,7 +1254,7 @@ static kernel_t select_kernel(bool regular, int segs, int nlast) {
   return nullptr;
 }
 
-typedef void (*tail_kernel_t)(Plan, int, int, int, int, uint16_t*, int, int, int);
+typedef void (*tail_kernel_t)(Plan, int, Epilogue, int, int, uint16_t*, int, int, int);
 
 template <bool REM, bool WT>
 static tail_kernel_t select_tail_kernel(int nlast) {
@@ -1230,14 +1265,14 @@ static tail_kernel_t select_tail_kernel(int nlast) {
 hipError_t launch_mixed_gemm_256(const uint8_t* an, const uint8_t* bn, const uint8_t* as_, const uint8_t* bs,
                                  const uint8_t* ao, const uint8_t* bo, const uint8_t* sfan, const uint8_t* sfbn,
                                  const uint8_t* sfas, const uint8_t* sfbs, const uint8_t* sfao, const uint8_t* sfbo,
-                                 int m_store, int a_rows, int N, int KN, int KS, int KO, bool w_tiled, void* d,
-                                 hipStream_t stream) {
+                                 int m_store, int a_rows, int N, int KN, int KS, int KO, bool w_tiled, Epilogue ep,
+                                 void* d, hipStream_t stream) {
   // m_store tokens are computed in whole tiles of 256 or 128 token rows; rows past m_store are computed but not
   // stored; the activation buffers are read up to row a_rows - 1 only
   if (m_store <= 0 || a_rows < m_store) return hipErrorInvalidValue;
   DeviceLimits lim;
   if (hipError_t e = device_limits(&lim); e != hipSuccess) return e;
-  const int tokens = tile_tokens(m_store, N, lim.cus);
+  const int tokens = tile_tokens(m_store, ep.n_out, lim.cus);
   const int M = (m_store + tokens - 1) / tokens * tokens;
   const bool rem = (KN | KS | KO) % 128 != 0;
   const int half = tokens == 128 ? 1 : 0;
@@ -1257,7 +1292,7 @@ hipError_t launch_mixed_gemm_256(const uint8_t* an, const uint8_t* bn, const uin
   }
   if (kernel == nullptr) return hipErrorInvalidValue;
   // a last round of whole tiles on at most half of the CUs: those tiles as twice as many half tiles
-  const int whole_tiles = ((N + kT - 1) / kT) * (M / tokens);
+  const int whole_tiles = ((ep.n_out + kT - 1) / kT) * (M / tokens);
   const int rest = whole_tiles % lim.cus;
   const bool tail = !half && regular && segs == 7 && whole_tiles > lim.cus && rest > 0 && 2 * rest <= lim.cus;
   tail_kernel_t tail_kernel = nullptr;
@@ -1277,15 +1312,15 @@ hipError_t launch_mixed_gemm_256(const uint8_t* an, const uint8_t* bn, const uin
   p.total = p.st0 + p.st1 + p.st2;
   p.w_tiled = w_tiled ? 1 : 0;
   if (w_tiled && N % kT != 0) return hipErrorInvalidValue;
-  const int tiles_n = (N + kT - 1) / kT, tiles_m = M / tokens;
+  const int tiles_n = (ep.n_out + kT - 1) / kT, tiles_m = M / tokens;
   // more tiles than CUs: staggered start (see the kernel), up to kStartSkew ticks of the shader's clock counter
   const int ntiles = tiles_n * tiles_m;
   const int skew = ntiles > lim.cus ? kStartSkew : 0;
   if (tail)
-    hipLaunchKernelGGL(tail_kernel, dim3(ntiles + rest), dim3(64 * kWaves), kBuffers * kStage, stream, p, tiles_n, N, m_store, a_rows,
+    hipLaunchKernelGGL(tail_kernel, dim3(ntiles + rest), dim3(64 * kWaves), kBuffers * kStage, stream, p, tiles_n, ep, m_store, a_rows,
                        static_cast<uint16_t*>(d), lim.cus, skew, ntiles - rest);
   else
-    hipLaunchKernelGGL(kernel, dim3(ntiles), dim3(64 * kWaves), kBuffers * kStage, stream, p, tiles_n, N, m_store, a_rows,
+    hipLaunchKernelGGL(kernel, dim3(ntiles), dim3(64 * kWaves), kBuffers * kStage, stream, p, tiles_n, ep, m_store, a_rows,
                        static_cast<uint16_t*>(d), lim.cus, skew);
   return hipGetLastError();
 }

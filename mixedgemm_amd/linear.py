@@ -206,20 +206,20 @@ def read_header(path: str):
 # ------------------------------------------------------------------ torch operators
 # Same names and argument order as the reference's module (bindings.cpp:315-341), in the
 # namespace mixedgemm_amd; they enqueue on the current stream and return without synchronizing.
+# The GPU kernels and the derivative (an error: inference only) are native (csrc/torch_host.cpp); for other devices the
+# functions of abi say that there is none.
+_ops = torch.library.Library("mixedgemm_amd", "DEF")
+_QUANT = "(Tensor {}, Tensor reorder_index, SymInt KN, SymInt KS, SymInt KO) -> (Tensor, Tensor, Tensor, Tensor, Tensor, Tensor)"
+_WEIGHTS = "Tensor BN, Tensor BS, Tensor BO, Tensor SFBN, Tensor SFBS, Tensor SFBO, SymInt KN, SymInt KS, SymInt KO, bool w_tiled=False"
+
+
+def _fused_norm(X, norm_weight, eps, reorder_index, BN, BS, BO, SFBN, SFBS, SFBO, KN, KS, KO, w_tiled=False):
+    return abi.fused_linear(X, reorder_index, BN, BS, BO, SFBN, SFBS, SFBO, KN, KS, KO, w_tiled=w_tiled,
+                            norm_weight=norm_weight, eps=eps)
+
+
 def _sf_len(rows: int, kseg: int, operand: int) -> int:
     return abi.sf_bytes(rows, kseg, operand)
-
-
-@torch.library.custom_op("mixedgemm_amd::reorder_quantize_x", mutates_args=())
-def reorder_quantize_x_op(X: torch.Tensor, reorder_index: torch.Tensor, KN: int, KS: int, KO: int
-                          ) -> tuple[torch.Tensor, torch.Tensor, torch.Tensor, torch.Tensor, torch.Tensor, torch.Tensor]:
-    return abi.reorder_quantize_x(X, reorder_index, KN, KS, KO)
-
-
-@torch.library.custom_op("mixedgemm_amd::reorder_quantize_w", mutates_args=())
-def reorder_quantize_w_op(W: torch.Tensor, reorder_index: torch.Tensor, KN: int, KS: int, KO: int
-                          ) -> tuple[torch.Tensor, torch.Tensor, torch.Tensor, torch.Tensor, torch.Tensor, torch.Tensor]:
-    return abi.reorder_quantize_w(W, reorder_index, KN, KS, KO)
 
 
 def _fake_quant(operand):
@@ -236,57 +236,45 @@ def _fake_quant(operand):
     return fake
 
 
-reorder_quantize_x_op.register_fake(_fake_quant(abi.MG_OPERAND_A))
-reorder_quantize_w_op.register_fake(_fake_quant(abi.MG_OPERAND_B))
-
-
-@torch.library.custom_op("mixedgemm_amd::matmul", mutates_args=())
-def matmul_op(AN: torch.Tensor, BN: torch.Tensor, AS: torch.Tensor, BS: torch.Tensor, AO: torch.Tensor, BO: torch.Tensor,
-              SFAN: torch.Tensor, SFBN: torch.Tensor, SFAS: torch.Tensor, SFBS: torch.Tensor, SFAO: torch.Tensor,
-              SFBO: torch.Tensor, w_tiled: bool = False) -> torch.Tensor:
-    return abi.matmul(AN, BN, AS, BS, AO, BO, SFAN, SFBN, SFAS, SFBS, SFAO, SFBO, w_tiled=w_tiled)
-
-
-@matmul_op.register_fake
-def _(AN, BN, AS, BS, AO, BO, SFAN, SFBN, SFAS, SFBS, SFAO, SFBO, w_tiled=False):
+def _fake_matmul(AN, BN, AS, BS, AO, BO, SFAN, SFBN, SFAS, SFBS, SFAO, SFBO, w_tiled=False):
     return torch.empty((AN.shape[0], BN.shape[0]), dtype=torch.bfloat16, device=AN.device)
 
 
-@torch.library.custom_op("mixedgemm_amd::fused_linear", mutates_args=())
-def fused_linear_op(X: torch.Tensor, reorder_index: torch.Tensor, BN: torch.Tensor, BS: torch.Tensor, BO: torch.Tensor,
-                    SFBN: torch.Tensor, SFBS: torch.Tensor, SFBO: torch.Tensor, KN: int, KS: int, KO: int,
-                    w_tiled: bool = False) -> torch.Tensor:
-    return abi.fused_linear(X, reorder_index, BN, BS, BO, SFBN, SFBS, SFBO, KN, KS, KO, w_tiled=w_tiled)
-
-
-@fused_linear_op.register_fake
-def _(X, reorder_index, BN, BS, BO, SFBN, SFBS, SFBO, KN, KS, KO, w_tiled=False):
+def _fake_fused(X, reorder_index, BN, BS, BO, SFBN, SFBS, SFBO, KN, KS, KO, w_tiled=False):
     n = BN.shape[0] if KN else (BS.shape[0] if KS else BO.shape[0])
     return torch.empty((X.shape[0], n), dtype=torch.bfloat16, device=X.device)
 
 
-@torch.library.custom_op("mixedgemm_amd::fused_norm_linear", mutates_args=())
-def fused_norm_linear_op(X: torch.Tensor, norm_weight: torch.Tensor, eps: float, reorder_index: torch.Tensor,
-                         BN: torch.Tensor, BS: torch.Tensor, BO: torch.Tensor, SFBN: torch.Tensor, SFBS: torch.Tensor,
-                         SFBO: torch.Tensor, KN: int, KS: int, KO: int, w_tiled: bool = False) -> torch.Tensor:
-    return abi.fused_linear(X, reorder_index, BN, BS, BO, SFBN, SFBS, SFBO, KN, KS, KO, w_tiled=w_tiled,
-                            norm_weight=norm_weight, eps=eps)
+def _fake_fused_norm(X, norm_weight, eps, reorder_index, *weights_and_split):
+    return _fake_fused(X, reorder_index, *weights_and_split)
 
 
-@fused_norm_linear_op.register_fake
-def _(X, norm_weight, eps, reorder_index, BN, BS, BO, SFBN, SFBS, SFBO, KN, KS, KO, w_tiled=False):
-    n = BN.shape[0] if KN else (BS.shape[0] if KS else BO.shape[0])
-    return torch.empty((X.shape[0], n), dtype=torch.bfloat16, device=X.device)
-
-
-@torch.library.custom_op("mixedgemm_amd::calibrate_reorder_index", mutates_args=())
-def calibrate_reorder_index_op(X: torch.Tensor) -> torch.Tensor:
-    return abi.calibrate_reorder_index(X)
-
-
-@calibrate_reorder_index_op.register_fake
-def _(X):
+def _fake_calibrate(X):
     return torch.empty((X.shape[1],), dtype=torch.int16, device=X.device)
+
+
+for _name, _schema, _other, _fake in (
+        ("reorder_quantize_x", _QUANT.format("X"), abi.reorder_quantize_x, _fake_quant(abi.MG_OPERAND_A)),
+        ("reorder_quantize_w", _QUANT.format("W"), abi.reorder_quantize_w, _fake_quant(abi.MG_OPERAND_B)),
+        ("matmul", "(Tensor AN, Tensor BN, Tensor AS, Tensor BS, Tensor AO, Tensor BO, Tensor SFAN, Tensor SFBN, Tensor SFAS, "
+                   "Tensor SFBS, Tensor SFAO, Tensor SFBO, bool w_tiled=False) -> Tensor",
+         lambda *a: abi.matmul(*a[:12], w_tiled=len(a) > 12 and a[12]), _fake_matmul),
+        ("fused_linear", f"(Tensor X, Tensor reorder_index, {_WEIGHTS}) -> Tensor",
+         lambda *a: abi.fused_linear(*a[:11], w_tiled=len(a) > 11 and a[11]), _fake_fused),
+        ("fused_norm_linear", f"(Tensor X, Tensor norm_weight, float eps, Tensor reorder_index, {_WEIGHTS}) -> Tensor",
+         _fused_norm, _fake_fused_norm),
+        ("calibrate_reorder_index", "(Tensor X) -> Tensor", abi.calibrate_reorder_index, _fake_calibrate)):
+    _ops.define(_name + _schema, tags=(torch.Tag.pt2_compliant_tag,))
+    _ops.impl(_name, _other, "CompositeExplicitAutograd")
+    torch.library.register_fake(f"mixedgemm_amd::{_name}", _fake, lib=_ops)
+reorder_quantize_x_op = torch.ops.mixedgemm_amd.reorder_quantize_x
+reorder_quantize_w_op = torch.ops.mixedgemm_amd.reorder_quantize_w
+matmul_op = torch.ops.mixedgemm_amd.matmul
+fused_linear_op = torch.ops.mixedgemm_amd.fused_linear
+fused_norm_linear_op = torch.ops.mixedgemm_amd.fused_norm_linear
+calibrate_reorder_index_op = torch.ops.mixedgemm_amd.calibrate_reorder_index
+if os.path.exists(abi.HOST_PATH) and os.path.exists(abi.LIB_PATH):
+    abi.host()   # registers the GPU kernels; without them a GPU tensor gets the error of abi.host()
 
 
 # ------------------------------------------------------------------ the layer
@@ -326,6 +314,12 @@ class MixedLinear(torch.nn.Module):
                              self.tiled, self.out_features if self.out_features != self.wn.shape[0] else 0)
 
     def forward(self, x: torch.Tensor) -> torch.Tensor:
+        # One native call for what nothing intercepts: norm, quantization, GEMM, bias and the real features of a padded
+        # layer.  Everything else -- tracing, other dtypes and layouts -- goes through the operators.
+        if not torch.compiler.is_compiling():
+            y = abi.host().layer(x, self._buffers, self.split, self.tiled, self.out_features, self.eps)
+            if y is not None:
+                return y
         lead = x.shape[:-1]
         x2 = x.reshape(-1, self.in_features)
         if x2.dtype != torch.bfloat16:

@@ -217,3 +217,23 @@ def test_layer_with_a_plan_that_has_no_e3m2_or_e4m3_segment(linear, tmp_path, sp
     torch.cuda.synchronize()
     ref, slack = _oracle_linear(x, w, idx, split)
     _close(y, ref, slack)
+
+
+@pytest.mark.parametrize("m", [1, 16, 40, 300])
+@pytest.mark.parametrize("n", [24, 1001, 1004, 1280])
+@pytest.mark.parametrize("bias", [False, True])
+def test_layer_stores_the_real_features_and_adds_the_bias(linear, m, n, bias):
+    """The kernels' own slice and bias against the operators' result, sliced and added to by torch: the same roundings in
+    the same order, so the same bits.  Feature counts with whole, half and odd 16-byte pieces in the last tile."""
+    k = 1088                                     # (640, 320, 128): two blocks past the last whole step of a segment
+    split = linear.default_split(k)
+    x = H.make_activations(m, k, 300 + m).to(DEV)
+    w = H.make_weights(n, k, 301 + n).to(DEV)
+    b = torch.randn(n, generator=torch.Generator().manual_seed(n)).to(torch.bfloat16).to(DEV) if bias else None
+    pw = linear.PackedWeights.from_float(w, torch.ops.mixedgemm_amd.calibrate_reorder_index(x), split)
+    want = torch.ops.mixedgemm_amd.fused_linear(x, pw.reorder_index, *pw.tensors(), *split, pw.tiled)[:, :n]
+    want = want + b if bias else want
+    got = linear.MixedLinear(pw, bias=b)(x.view(m, 1, k))
+    torch.cuda.synchronize()
+    assert got.shape == (m, 1, n) and got.is_contiguous()
+    assert torch.equal(got[:, 0], want)
