@@ -19,7 +19,7 @@
 //                [64+16g, 64+16g+16) in registers 4-7 (two 16-byte pieces);
 // and, for every format, the E8M0 scale of block g of row i in the byte of the
 // scale register that op_sel selects.
-#include <stdlib.h>
+#include <type_traits>
 
 #include "mg_common.h"
 
@@ -152,15 +152,24 @@ mixed_gemm_direct_kernel(const uint8_t* __restrict__ an, const uint8_t* __restri
 
 
 // ---------------------------------------------------------------------------
-// Skinny kernel: few tokens (decode, small batches), weights streamed once per
-// 16 * G tokens (HBM- or L2-bound).
+// Skinny kernel: few tokens (decode, small batches) where the decode kernel's LDS image does not fit or a segment
+// ends in a partial 128-wide step.  Weights are streamed once per 16 * G tokens (HBM- or L2-bound).
 //
-// A workgroup of 4 waves owns F groups of 16 output features and G groups of 16 tokens; the K
-// steps (128 elements each, counted over the three segments) are dealt to the 4
-// waves in contiguous quarters.  A wave issues every load of a round of steps
-// (weights, the G token groups, scales; addresses clamped, no branches) before
-// the round's first MFMA; the 4 partial 16x16 tiles per group are summed through
-// LDS and rounded to bf16 once.  G = 1 is the decode case.
+// A workgroup of 4 waves owns F groups of 16 output features and G groups of 16 tokens; the K steps (128 elements
+// each, counted over the three segments) are dealt to the waves in contiguous quarters (as in the decode kernel below:
+// the same sums in the same order, whichever of the two a shape goes to).  Each wave runs a pipeline of its own: a
+// ring of NS slots in LDS, one step each (weight codes, token codes, the 16-byte pieces of the scale atoms that hold
+// its rows), filled by global -> LDS copies NS - 1 steps ahead and refilled as soon as its fragments are in registers.
+// No barrier until the waves' partial 16x16 tiles are summed; nothing in flight occupies a register.
+//
+// What bounds it is the address unit (~33 cycles per copy of 16 rows x 64 bytes) and, with one workgroup per CU, the
+// latency of the first copies: about 2.3 us + 0.07 ... 0.12 us per K step.  So the token fragments of a step are as
+// many copies as their format has kilobytes, and all scales of a step are one copy.  The 16-byte pieces of a row are
+// copied by neighbouring lanes and permuted inside the row (XOR with bits of the row number), so that the fragment
+// reads spread over the LDS banks.  Before (fragments and scale bytes loaded into registers, each round of steps
+// waited for as a whole; same shapes, K = 14336, N = 4096): M = 16 17.5 -> 11.0 us, 32 23 -> 12.2, 64 28 -> 13.1,
+// 128 47 (whole-tile kernel) -> 16.8, 200 47 -> 30.8; K = 4096, N = 4096, M = 128 9.0 -> 7.9 (decode kernel with 32
+// tokens per workgroup, which this replaces).
 // ---------------------------------------------------------------------------
 struct DecodeSeg {
   const uint8_t* a;
@@ -176,176 +185,255 @@ __device__ __forceinline__ v4f decode_mfma(v8i wb, v8i xa, v4f acc, int sw, int 
   return __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(wb, xa, acc, kFmtE2M1, FMT, 0, sw, 0, sx);
 }
 
+template <int N>
+__device__ __forceinline__ void wait_vmcnt() { asm volatile("s_waitcnt vmcnt(%0)" : : "n"(N) : "memory"); }
+
+__device__ __forceinline__ void dma16_at(const uint8_t* base, unsigned voff, unsigned lds_off) {
+  // base and lds_off are wave-uniform; say so to the compiler
+  const uint64_t bv = reinterpret_cast<uint64_t>(base);
+  // (the builtin returns int: without the casts the low half would be sign-extended over the high half)
+  const uint32_t lo = (uint32_t)__builtin_amdgcn_readfirstlane((uint32_t)bv);
+  const uint32_t hi = (uint32_t)__builtin_amdgcn_readfirstlane((uint32_t)(bv >> 32));
+  base = reinterpret_cast<const uint8_t*>(((uint64_t)hi << 32) | lo);
+  lds_off = __builtin_amdgcn_readfirstlane(lds_off);
+  asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1"
+               : : "v"(voff), "s"(base), "s"(lds_off) : "memory", "m0");
+}
+// the same with a 64-bit address per lane
+__device__ __forceinline__ void dma16_lane(const uint8_t* p, unsigned lds_off) {
+  lds_off = __builtin_amdgcn_readfirstlane(lds_off);
+  asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off" : : "v"(p), "s"(lds_off) : "memory", "m0");
+}
+
+// copies of 1 KB per step for 16 G tokens of a format
+template <int FMT, int G>
+constexpr int kTokenCopies = (16 * G * 4 * Frag<FMT>::kBytes + 1023) / 1024;
+// LDS bytes of a slot, and slots per wave
 template <int G, int F>
+constexpr int kSkinnySlot = 1024 * (1 + F + 2 * G);
+template <int G, int F>
+constexpr int kSkinnySlots = 156 * 1024 / (4 * kSkinnySlot<G, F>) < 8 ? 156 * 1024 / (4 * kSkinnySlot<G, F>) : 8;
+
+template <int G, int F, bool WT>
 __global__ void __launch_bounds__(256)
-mixed_gemm_skinny_kernel(DecodeSeg s4, DecodeSeg s6, DecodeSeg s8, int M, int N, int steps_per_wave,
-                         int w_tiled, Epilogue ep, uint16_t* __restrict__ d) {
-  constexpr int S = G * F >= 8 ? 1 : 8 / (G * F);   // K steps a wave keeps in flight at once
-  __shared__ float partial[4][F][G][16 * 16];
+mixed_gemm_skinny_kernel(DecodeSeg s4, DecodeSeg s6, DecodeSeg s8, int M, int N, int steps_per_wave, Epilogue ep,
+                         uint16_t* __restrict__ d) {
+  constexpr int NS = kSkinnySlots<G, F>, kSlot = kSkinnySlot<G, F>;
+  constexpr int PA = G == 1 ? 16 : 32, PB = 4 * F;   // scale pieces per step: tokens, weights
+  static_assert(NS >= 3 && PA + PB <= 64, "a pipeline; one copy for all scales of a step");
+  extern __shared__ __align__(16) uint8_t lds[];
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int i = lane & 15, g = lane >> 4;
-  // The workgroup owns F groups of 16 features (group index bx = blockIdx.x * F + f) and G groups of 16
-  // tokens; an activation fragment is loaded once and used for the F feature groups.
-  // Row-major weights: a group is 16 consecutive features.  Tile-major weights: the 16 rows of one
-  // 1 KB copy block (block j = bx % 16 of feature tile bx / 16), i.e. features
-  // j + 16 * (2 * (t % 8) + t / 8) of the tile for t = 0..15, so that a weight load reads 1 KB of
-  // consecutive bytes.
-  int tile_row0[F], n[F], nc[F];
-  bool n_ok[F];
+  uint8_t* const ring = lds + wave * (NS * kSlot);
+  const unsigned ring0 = (unsigned)(size_t)(__attribute__((address_space(3))) uint8_t*)lds + (unsigned)wave * (NS * kSlot);
+  const int t6 = s4.steps, t8 = s4.steps + s6.steps, total = t8 + s8.steps;
+  const int t_begin = wave * steps_per_wave, t_end = min(total, t_begin + steps_per_wave);
+
+  // ---- the workgroup's rows: the mapping of the decode kernel below (feature group f, lane row i -> its scale piece
+  // and its dword in the piece), and the weight row this lane copies, row lane / 4 of the group
+  int wg = blockIdx.x;
+  if constexpr (WT) {   // the workgroups of a 256-feature tile on one XCD (see the decode kernel)
+    constexpr int kPer = 16 / F;
+    if ((int)gridDim.x % (8 * kPer) == 0) {
+      const int xcd = wg & 7, slot = wg >> 3;
+      wg = ((slot / kPer) * 8 + xcd) * kPer + slot % kPer;
+    }
+  }
+  constexpr int per_group = 32 / PB;
+  const int tile = (wg * F) >> 4, j0 = (wg * F) & 15;                    // tile-major
+  const int group = wg / per_group, c0 = (wg % per_group) * PB;          // row-major
+  auto feature = [&](int f, int e) {   // feature e of group f
+    if constexpr (WT) return tile * 256 + j0 + f + 32 * (e & 7) + 16 * (e >> 3);
+    else return group * 128 + c0 + (16 * f + e) % PB + 32 * ((16 * f + e) / PB);
+  };
+  int sw_off[F];   // this lane's weight scale byte in a step's pieces
+  int wrow[F];     // the weight row it copies
 #pragma unroll
   for (int f = 0; f < F; ++f) {
-    const int bx = blockIdx.x * F + f;
-    tile_row0[f] = (bx >> 4) * 256 + (bx & 15);
-    n[f] = w_tiled ? tile_row0[f] + 16 * (2 * (i & 7) + (i >> 3)) : bx * 16 + i;
-    n_ok[f] = n[f] < N;
-    nc[f] = min(n[f], N - 1);   // clamped rows: every load is in bounds and unconditional
+    if constexpr (WT) sw_off[f] = (PA + (((i & 7) >> 2) * 2 + (i >> 3)) * F + f) * 16 + (i & 3) * 4 + g;
+    else sw_off[f] = (PA + (16 * f + i) % PB) * 16 + ((16 * f + i) / PB) * 4 + g;
+    wrow[f] = min(feature(f, lane >> 2), N - 1);   // rows past N: read again, never stored
   }
-  const int m0 = blockIdx.y * (G * 16) + i;      // this lane's token in group 0
-  const int total = s4.steps + s6.steps + s8.steps;
+  const int m_base = (int)blockIdx.y * 16 * G, last_row = min(M - m_base, 16 * G) - 1;
+  // the scale piece this lane copies, as an address in each segment's first step
+  const uint8_t *sc4, *sc6, *sc8;
+  {
+    const int pl = min(lane, PA + PB - 1) - PA;
+    unsigned piece;
+    int mul;
+    if (pl < 0) {
+      piece = (unsigned)((m_base & 31) + pl + PA);
+      mul = m_base >> 7;
+    } else if constexpr (WT) {
+      piece = (unsigned)(j0 + pl % F + 16 * ((pl / F) & 1));
+      mul = tile * 2 + pl / (2 * F);
+    } else {
+      piece = (unsigned)(c0 + pl);
+      mul = group;
+    }
+    sc4 = (pl < 0 ? s4.sfa : s4.sfb) + (size_t)mul * s4.steps * 512 + piece * 16;
+    sc6 = (pl < 0 ? s6.sfa : s6.sfb) + (size_t)mul * s6.steps * 512 + piece * 16;
+    sc8 = (pl < 0 ? s8.sfa : s8.sfb) + (size_t)mul * s8.steps * 512 + piece * 16;
+  }
+
+  // ---- requests step q of a segment into a slot
+  const int wpos = (lane & 3) ^ ((lane >> 4) & 3);   // the 16-byte piece of its row that this lane copies
+  auto request_seg = [&](auto fmt_c, const DecodeSeg& s, const uint8_t* sc, int q, unsigned slot) __attribute__((always_inline)) {
+    constexpr int FMT = decltype(fmt_c)::value;
+    const int left = min(s.nblk - 4 * q, 4);
+    dma16_lane(sc + (size_t)q * 512, slot);
+    const unsigned wp = (unsigned)min(wpos, left - 1) * 16u;
+#pragma unroll
+    for (int f = 0; f < F; ++f) {
+      const unsigned at = slot + 1024u * (1 + f);
+      if constexpr (WT) {
+        // 16 KB per (256-feature tile, whole step), the group's block in it; the blocks past the last whole step as
+        // rows of nblk % 4 blocks behind the tiled part
+        const int whole = s.nblk >> 2;
+        if (q < whole) dma16_at(s.b + (((size_t)tile * whole + q) * 16 + j0 + f) * 1024, (unsigned)(lane >> 2) * 64u + wp, at);
+        else dma16_at(s.b + (size_t)(N >> 8) * whole * 16384, (unsigned)wrow[f] * (unsigned)(s.nblk & 3) * 16u + wp, at);
+      } else {
+        dma16_at(s.b + (size_t)q * 64, (unsigned)wrow[f] * (unsigned)s.nblk * 16u + wp, at);
+      }
+    }
+    const unsigned pitch = (unsigned)s.nblk * Frag<FMT>::kBytes;
+    const uint8_t* a = s.a + (size_t)m_base * pitch + (size_t)q * (4 * Frag<FMT>::kBytes);
+    constexpr int kPieces = Frag<FMT>::kBytes / 4;   // 16-byte pieces of a row's step
+#pragma unroll
+    for (int c = 0; c < kTokenCopies<FMT, G>; ++c) {
+      const int chunk = min(c * 64 + lane, 16 * G * kPieces - 1), row = chunk / kPieces, p = chunk % kPieces;
+      unsigned off;
+      if constexpr (FMT == kFmtE2M1) off = (unsigned)min(p ^ ((row >> 2) & 3), left - 1) * 16u;
+      else if constexpr (FMT == kFmtE3M2) off = (unsigned)min(p * 16, left * 24 - 16);
+      else off = (unsigned)min(p ^ (row & 7), 2 * left - 1) * 16u;
+      dma16_at(a, (unsigned)min(row, last_row) * pitch + off, slot + 1024u * (1 + F + c));
+    }
+  };
+  auto request = [&](int t, unsigned slot) __attribute__((always_inline)) {
+    if (t >= t_end) return;
+    if (t < t6) request_seg(std::integral_constant<int, kFmtE2M1>{}, s4, sc4, t, slot);
+    else if (t < t8) request_seg(std::integral_constant<int, kFmtE3M2>{}, s6, sc6, t - t6, slot);
+    else request_seg(std::integral_constant<int, kFmtE4M3>{}, s8, sc8, t - t8, slot);
+  };
+
   v4f acc[F][G];
 #pragma unroll
   for (int f = 0; f < F; ++f)
 #pragma unroll
     for (int gi = 0; gi < G; ++gi) acc[f][gi] = v4f{0.f, 0.f, 0.f, 0.f};
-
-  for (int r0 = 0; r0 < steps_per_wave; r0 += S) {
-    const int t0 = wave * steps_per_wave + r0, t_end = min(total, wave * steps_per_wave + steps_per_wave);
-
-    // Straight-line issue of every load of this round, so all of them are in
-    // flight together; masking comes afterwards.
-    v4i wq[S][F], xa[S][G], xb[S][G];
-    int sw[S][F], sx[S][G];
+  int sx_off[G];   // this lane's token scale byte in a step's pieces
 #pragma unroll
-    for (int k = 0; k < S; ++k) {
-      const int t = min(t0 + k, total - 1);
-      const int seg = t < s4.steps ? 0 : (t < s4.steps + s6.steps ? 1 : 2);
-      const int q = seg == 0 ? t : (seg == 1 ? t - s4.steps : t - s4.steps - s6.steps);
-      const uint8_t* pa = seg == 0 ? s4.a : (seg == 1 ? s6.a : s8.a);
-      const uint8_t* pb = seg == 0 ? s4.b : (seg == 1 ? s6.b : s8.b);
-      const uint8_t* psa = seg == 0 ? s4.sfa : (seg == 1 ? s6.sfa : s8.sfa);
-      const uint8_t* psb = seg == 0 ? s4.sfb : (seg == 1 ? s6.sfb : s8.sfb);
-      const int nblk = seg == 0 ? s4.nblk : (seg == 1 ? s6.nblk : s8.nblk);
-      const int katoms = seg == 0 ? s4.steps : (seg == 1 ? s6.steps : s8.steps);
-      const int xbytes = seg == 0 ? 16 : (seg == 1 ? 24 : 32);   // activation bytes per 32-element block
-      const int left = nblk - 4 * q;
-      const int gc = min(g, left - 1);
-      // tile-major weights: 16 KB per (256-feature tile, whole step), the group's block in it, lane
-      // quad i, piece g; the blocks past the last whole step as rows of (nblk % 4) blocks behind the tiled part
-      const int whole = nblk >> 2, rblk = nblk & 3;
+  for (int gi = 0; gi < G; ++gi) {
+    const int m = m_base + 16 * gi + i;
+    sx_off[gi] = ((m - m_base) & (PA - 1)) * 16 + ((m >> 5) & 3) * 4 + g;
+  }
+
+  int t = t_begin, slot = 0;
+#pragma unroll
+  for (int k = 0; k < NS - 1; ++k) request(t_begin + k, ring0 + k * kSlot);
+  // the wave's steps of one segment
+  auto run = [&](auto fmt_c, const DecodeSeg& s, int t_first, int t_next) __attribute__((always_inline)) {
+    constexpr int FMT = decltype(fmt_c)::value;
+    for (const int last = min(t_next, t_end); t < last; ++t) {
+      // The slot after this one was read one step ago and is free.  Wait for this step: NS - 1 steps are younger, each
+      // with at least as many copies as this one (a token takes more bytes in every later segment's format).
+      const int ahead = t + NS - 1;
+      request(ahead, ring0 + (unsigned)(slot == 0 ? NS - 1 : slot - 1) * kSlot);
+      if (ahead < t_end) wait_vmcnt<(NS - 1) * (1 + F + kTokenCopies<FMT, G>)>();
+      else wait_vmcnt<0>();
+      const uint8_t* sl = ring + slot * kSlot;
+      slot = slot == NS - 1 ? 0 : slot + 1;
+      const int left = s.nblk - 4 * (t - t_first);
+      int s_w[F], s_x[G];
+      v4i w[F];
+      v8i x[G];
 #pragma unroll
       for (int f = 0; f < F; ++f) {
-        const int bx = blockIdx.x * F + f;
-        const size_t w_tiled_off =
-            q < whole ? ((((size_t)(bx >> 4) * whole + q) * 16 + (bx & 15)) * 1024 + i * 64 + g * 16)
-                      : ((size_t)(N >> 8) * whole * 16384 + (size_t)nc[f] * rblk * 16 + gc * 16);
-        const size_t w_off = w_tiled ? w_tiled_off : ((size_t)nc[f] * nblk * 16 + q * 64 + gc * 16);
-        wq[k][f] = *reinterpret_cast<const v4i*>(pb + w_off);
-        sw[k][f] = psb[sf_offset(nc[f], 4 * q + gc, katoms)];
+        s_w[f] = sl[sw_off[f]];
+        w[f] = *reinterpret_cast<const v4i*>(sl + 1024 * (1 + f) + i * 64 + (g ^ ((i >> 2) & 3)) * 16);
       }
-      // activations: two 16-byte pieces.  E2M1: block g (second piece unused);
-      // E3M2: bytes [0,16) and [8,24) of block g; E4M3: K [16g,+16) and [64+16g,+16).
-      const int a_blk = seg == 2 ? (g >> 1) : g, b_blk = seg == 2 ? 2 + (g >> 1) : g;
-      int off_a = seg == 1 ? g * 24 : g * 16;
-      int off_b = seg == 0 ? g * 16 : (seg == 1 ? g * 24 + 8 : 64 + g * 16);
-      off_a = a_blk < left ? off_a : 0;
-      off_b = b_blk < left ? off_b : 0;
 #pragma unroll
       for (int gi = 0; gi < G; ++gi) {
-        const int mc = min(m0 + gi * 16, M - 1);
-        const uint8_t* xrow = pa + (size_t)mc * nblk * xbytes + q * 4 * xbytes;
-        xa[k][gi] = *reinterpret_cast<const v4i*>(xrow + off_a);
-        // E2M1 needs one piece only; a wave-uniform branch around the second load pays for G = 4 only (measured)
-        if (G != 4 || seg != 0) xb[k][gi] = *reinterpret_cast<const v4i*>(xrow + off_b);
-        else xb[k][gi] = v4i{0, 0, 0, 0};
-        sx[k][gi] = psa[sf_offset(mc, 4 * q + gc, katoms)];
+        s_x[gi] = sl[sx_off[gi]];
+        const uint8_t* row = sl + 1024 * (1 + F) + (16 * gi + i) * (4 * Frag<FMT>::kBytes);
+        if constexpr (FMT == kFmtE2M1) {
+          const v4i a = *reinterpret_cast<const v4i*>(row + (g ^ ((i >> 2) & 3)) * 16);
+          x[gi] = v8i{a[0], a[1], a[2], a[3], 0, 0, 0, 0};
+        } else if constexpr (FMT == kFmtE3M2) {
+          const v2i* p = reinterpret_cast<const v2i*>(row + g * 24);
+          // a partial step of 24 or 72 bytes: its last 16 bytes were copied, of which these are the second half
+          const v2i a = p[0], b = p[1], e = p[(left & 1) && g == left - 1 ? 3 : 2];
+          x[gi] = v8i{a[0], a[1], b[0], b[1], e[0], e[1], 0, 0};
+        } else {   // K [16g, 16g+16) and [64+16g, 64+16g+16)
+          const v4i a = *reinterpret_cast<const v4i*>(row + (g ^ (i & 7)) * 16);
+          const v4i b = *reinterpret_cast<const v4i*>(row + ((4 + g) ^ (i & 7)) * 16);
+          x[gi] = v8i{a[0], a[1], a[2], a[3], b[0], b[1], b[2], b[3]};
+        }
       }
-    }
-
-#pragma unroll
-    for (int k = 0; k < S; ++k) {
-      const int t = t0 + k;
-      if (t < t_end) {   // wave-uniform
-        const int seg = t < s4.steps ? 0 : (t < s4.steps + s6.steps ? 1 : 2);
-        const int q = seg == 0 ? t : (seg == 1 ? t - s4.steps : t - s4.steps - s6.steps);
-        const int nblk = seg == 0 ? s4.nblk : (seg == 1 ? s6.nblk : s8.nblk);
-        const int left = nblk - 4 * q;
-        const bool blk_ok = g < left;
-        const v4i z = {0, 0, 0, 0};
-        v8i wf[F];
-        int s_w[F];
+      if (left < 4) {   // wave-uniform: the segment's last, partial step; what lies past its end is zero
+        const bool ok = g < left, lo_ok = FMT == kFmtE4M3 ? (g >> 1) < left : ok, hi_ok = FMT == kFmtE4M3 ? 2 + (g >> 1) < left : ok;
 #pragma unroll
         for (int f = 0; f < F; ++f) {
-          const bool w_ok = n_ok[f] && blk_ok;
-          const v4i w4 = w_ok ? wq[k][f] : z;
-          wf[f] = v8i{w4[0], w4[1], w4[2], w4[3], 0, 0, 0, 0};
-          s_w[f] = w_ok ? sw[k][f] : 127;
+          s_w[f] = ok ? s_w[f] : 127;
+#pragma unroll
+          for (int e = 0; e < 4; ++e) w[f][e] = ok ? w[f][e] : 0;
         }
 #pragma unroll
         for (int gi = 0; gi < G; ++gi) {
-          const bool m_ok = m0 + gi * 16 < M;
-          const int s_x = (m_ok && blk_ok) ? sx[k][gi] : 127;
-          if (seg == 0) {
-            const v4i a4 = (m_ok && blk_ok) ? xa[k][gi] : z;
-            const v8i xf = {a4[0], a4[1], a4[2], a4[3], 0, 0, 0, 0};
+          s_x[gi] = ok ? s_x[gi] : 127;
 #pragma unroll
-            for (int f = 0; f < F; ++f) acc[f][gi] = decode_mfma<kFmtE2M1>(wf[f], xf, acc[f][gi], s_w[f], s_x);
-          } else if (seg == 1) {
-            const v4i a4 = (m_ok && blk_ok) ? xa[k][gi] : z;
-            const v4i b4 = (m_ok && blk_ok) ? xb[k][gi] : z;
-            const v8i xf = {a4[0], a4[1], a4[2], a4[3], b4[2], b4[3], 0, 0};
-#pragma unroll
-            for (int f = 0; f < F; ++f) acc[f][gi] = decode_mfma<kFmtE3M2>(wf[f], xf, acc[f][gi], s_w[f], s_x);
-          } else {
-            const v4i a4 = (m_ok && (g >> 1) < left) ? xa[k][gi] : z;
-            const v4i b4 = (m_ok && 2 + (g >> 1) < left) ? xb[k][gi] : z;
-            const v8i xf = {a4[0], a4[1], a4[2], a4[3], b4[0], b4[1], b4[2], b4[3]};
-#pragma unroll
-            for (int f = 0; f < F; ++f) acc[f][gi] = decode_mfma<kFmtE4M3>(wf[f], xf, acc[f][gi], s_w[f], s_x);
+          for (int e = 0; e < 4; ++e) {
+            x[gi][e] = lo_ok ? x[gi][e] : 0;
+            x[gi][4 + e] = hi_ok ? x[gi][4 + e] : 0;
           }
         }
       }
+      // the fragments are in registers before a later request may fill this slot again
+      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+#pragma unroll
+      for (int gi = 0; gi < G; ++gi)
+#pragma unroll
+        for (int f = 0; f < F; ++f)
+          acc[f][gi] = decode_mfma<FMT>(v8i{w[f][0], w[f][1], w[f][2], w[f][3], 0, 0, 0, 0}, x[gi], acc[f][gi], s_w[f], s_x[gi]);
     }
-  }
+  };
+  run(std::integral_constant<int, kFmtE2M1>{}, s4, 0, t6);
+  run(std::integral_constant<int, kFmtE3M2>{}, s6, t6, t8);
+  run(std::integral_constant<int, kFmtE4M3>{}, s8, t8, total);
 
-  // result tile is D^T: lane holds token m = lane % 16, features 4 * (lane / 16) + v
+  // ---- sum the four waves' partial tiles (D^T: lane holds token lane % 16, features 4 * (lane / 16) + v of a group)
+  __syncthreads();   // every wave is done with its ring, which nothing fills any more
+  float* partial = reinterpret_cast<float*>(lds);
 #pragma unroll
   for (int f = 0; f < F; ++f)
 #pragma unroll
-    for (int gi = 0; gi < G; ++gi) *reinterpret_cast<v4f*>(&partial[wave][f][gi][lane * 4]) = acc[f][gi];
+    for (int gi = 0; gi < G; ++gi)
+      *reinterpret_cast<v4f*>(partial + ((wave * (F * G) + f * G + gi) * 64 + lane) * 4) = acc[f][gi];
   __syncthreads();
-  // the F * G partial tiles are dealt to the 4 waves round-robin
 #pragma unroll
   for (int fg = 0; fg < F * G; ++fg) {
     if ((fg & 3) != wave) continue;
     const int f = fg / G, gi = fg % G;
     v4f sum = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-    for (int w = 0; w < 4; ++w) sum += *reinterpret_cast<const v4f*>(&partial[w][f][gi][lane * 4]);
-    const int nn = (blockIdx.x * F + f) * 16 + 4 * g;
-    const int m = m0 + gi * 16;
+    for (int w = 0; w < 4; ++w) sum += *reinterpret_cast<const v4f*>(partial + ((w * (F * G) + fg) * 64 + lane) * 4);
+    const int m = m_base + 16 * gi + i;
     if (m < M) {
-      if (w_tiled) {   // feature 4g + v of the group is row tile_row0 + 16 * (2 * (t % 8) + t / 8), t = 4g + v
+      if constexpr (WT) {
 #pragma unroll
-        for (int v = 0; v < 4; ++v) {
-          const int t = 4 * g + v;
-          const int row = tile_row0[f] + 16 * (2 * (t & 7) + (t >> 3));
-          store1(d, ep, m, row, sum[v]);
-        }
+        for (int v = 0; v < 4; ++v) store1(d, ep, m, feature(f, 4 * g + v), sum[v]);
       } else {
-        store4(d, ep, m, nn, sum);
+        store4(d, ep, m, feature(f, 4 * g), sum);
       }
     }
   }
 }
 
 // ---------------------------------------------------------------------------
-// Decode kernel: 16 G tokens per workgroup (G = 1: up to 16 tokens in all; G = 2: up to 255 tokens, 32 per workgroup,
-// where their codes fit the LDS), whole 128-wide K steps.
+// Decode kernel: up to 16 tokens, whole 128-wide K steps.
 //
-// The skinny kernel above issues seven loads per K step and wave, five of them for a few bytes each (the
-// token fragment twice, three scale bytes); the address unit handles those as slowly as the two 1 KB weight
-// loads, and with 31 MB to stream in a few microseconds that is what bounds it.  Here everything that is not
-// a weight code goes global -> LDS once per workgroup in 1 KB copies (global_load_lds_dwordx4): the token
+// The skinny kernel above copies every step's token codes and scales for itself, for 16 tokens whether they exist or
+// not: as many copies as the weights need.  Here everything that is not a weight code goes global -> LDS once per workgroup in 1 KB copies (global_load_lds_dwordx4): the token
 // codes of all three segments (M x 2464 bytes for K = 4096) and, per K step, the 16-byte pieces of the scale
 // atoms that hold the workgroup's rows; the K loop reads them from LDS.  The weight codes go to registers,
 // eight K steps per wave in flight at a time, in two rounds of four.  All
@@ -367,7 +455,7 @@ struct DecodeLds {
   int sfb0, sfb1, sfb2;  // of the weight scale pieces: per step 4 F pieces
   int partial;           // of the partial sums
   int total;
-  int pa;                // 8 (up to 8 tokens), 16, or 32 (G = 2: the whole atom of the workgroup's group of 128 tokens)
+  int pa;                // 8 (up to 8 tokens) or 16
 };
 
 // value of segment seg (0, 1, 2) by masking: a select between struct fields invites the compiler to index a private
@@ -379,18 +467,6 @@ __device__ __forceinline__ const uint8_t* sel3p(int seg, const uint8_t* p0, cons
   const uint64_t m0 = seg == 0 ? ~0ull : 0ull, m1 = seg == 1 ? ~0ull : 0ull, m2 = seg == 2 ? ~0ull : 0ull;
   return reinterpret_cast<const uint8_t*>((reinterpret_cast<uint64_t>(p0) & m0) | (reinterpret_cast<uint64_t>(p1) & m1) |
                                           (reinterpret_cast<uint64_t>(p2) & m2));
-}
-
-__device__ __forceinline__ void dma16_at(const uint8_t* base, unsigned voff, unsigned lds_off) {
-  // base and lds_off are wave-uniform; say so to the compiler
-  const uint64_t bv = reinterpret_cast<uint64_t>(base);
-  // (the builtin returns int: without the casts the low half would be sign-extended over the high half)
-  const uint32_t lo = (uint32_t)__builtin_amdgcn_readfirstlane((uint32_t)bv);
-  const uint32_t hi = (uint32_t)__builtin_amdgcn_readfirstlane((uint32_t)(bv >> 32));
-  base = reinterpret_cast<const uint8_t*>(((uint64_t)hi << 32) | lo);
-  lds_off = __builtin_amdgcn_readfirstlane(lds_off);
-  asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1"
-               : : "v"(voff), "s"(base), "s"(lds_off) : "memory", "m0");
 }
 
 // Copies `bytes` (a multiple of 16) from src to LDS offset dst in units of 1 KB, unit u by wave u % 4; lanes past
@@ -443,14 +519,11 @@ __device__ __forceinline__ void load16_uncounted(v4i& dst, const uint8_t* sbase,
   else asm volatile("global_load_dwordx4 %0, %1, %2 offset:%3" : "=v"(dst) : "v"(voff), "s"(u), "n"(OFF) : "memory");
 }
 __device__ __forceinline__ void tie(v4i& r) { asm volatile("" : "+v"(r)); }
-template <int N>
-__device__ __forceinline__ void wait_vmcnt() { asm volatile("s_waitcnt vmcnt(%0)" : : "n"(N) : "memory"); }
 
-template <int F, bool WT, int G>
+template <int F, bool WT>
 __global__ void __launch_bounds__(256)
 mixed_gemm_decode_kernel(DecodeSeg s4, DecodeSeg s6, DecodeSeg s8, int M, int N, int steps_per_wave, DecodeLds L,
                          Epilogue ep, uint16_t* __restrict__ d) {
-  static_assert(G == 1 || G == 2, "token groups of 16 per workgroup");
   constexpr int S = 4;        // K steps per round
   constexpr int PB = 4 * F;   // weight scale pieces per step
   constexpr int PBLOG = F == 1 ? 2 : (F == 2 ? 3 : 4);
@@ -538,12 +611,11 @@ mixed_gemm_decode_kernel(DecodeSeg s4, DecodeSeg s6, DecodeSeg s8, int M, int N,
       if constexpr (WT) {
         const int nst = sel3(seg, nblk4, nblk6, nblk8) >> 2;
         const uint8_t* sb = pb + (((size_t)wtile * nst + q) * 16 + wj0) * 1024;
-        constexpr bool kStream = G == 1;   // several token groups' workgroups read the same weights: those stay ordinary loads
-        if constexpr (F >= 1) load16_uncounted<0, kStream>(wq[B][k][0], sb, vlane);
-        if constexpr (F >= 2) load16_uncounted<1024, kStream>(wq[B][k][F >= 2 ? 1 : 0], sb, vlane);
+        if constexpr (F >= 1) load16_uncounted<0, true>(wq[B][k][0], sb, vlane);
+        if constexpr (F >= 2) load16_uncounted<1024, true>(wq[B][k][F >= 2 ? 1 : 0], sb, vlane);
         if constexpr (F >= 4) {
-          load16_uncounted<2048, kStream>(wq[B][k][F >= 4 ? 2 : 0], sb, vlane);
-          load16_uncounted<3072, kStream>(wq[B][k][F >= 4 ? 3 : 0], sb, vlane);
+          load16_uncounted<2048, true>(wq[B][k][F >= 4 ? 2 : 0], sb, vlane);
+          load16_uncounted<3072, true>(wq[B][k][F >= 4 ? 3 : 0], sb, vlane);
         }
       } else {
         const uint8_t* sb = pb + (size_t)q * 64;
@@ -555,20 +627,16 @@ mixed_gemm_decode_kernel(DecodeSeg s4, DecodeSeg s6, DecodeSeg s8, int M, int N,
   };
   // ---- what is not a weight code, into LDS: requested first (measured: with the first round of weights ahead of
   // them the kernel is slower, by 2 % on tile-major and 7 % on row-major weights)
-  // the workgroup's tokens: m_base ... m_base + rows_here - 1 (G = 2: workgroup blockIdx.y takes 32 of them)
-  const int m_base = G == 1 ? 0 : (int)blockIdx.y * 32;
-  const int rows_here = min(M - m_base, 16 * G);
-  copy_region(s4.a + (size_t)m_base * nblk4 * 16, rows_here * nblk4 * 16, lds0 + L.x0, wave, lane);
-  copy_region(s6.a + (size_t)m_base * nblk6 * 24, rows_here * nblk6 * 24, lds0 + L.x1, wave, lane);
-  copy_region(s8.a + (size_t)m_base * nblk8 * 32, rows_here * nblk8 * 32, lds0 + L.x2, wave, lane);
+  copy_region(s4.a, M * nblk4 * 16, lds0 + L.x0, wave, lane);
+  copy_region(s6.a, M * nblk6 * 24, lds0 + L.x1, wave, lane);
+  copy_region(s8.a, M * nblk8 * 32, lds0 + L.x2, wave, lane);
   {
-    const int palog = L.pa == 8 ? 3 : (L.pa == 16 ? 4 : 5);
-    // token scale pieces 0 ... pa - 1 of the tokens' group of 128 rows
+    const int palog = L.pa == 8 ? 3 : 4;
+    // token scale pieces 0 ... pa - 1
     const unsigned pa_off = (unsigned)(lane & (L.pa - 1)) * 16u;
-    const unsigned agrp = (unsigned)(m_base >> 7) * 512u;   // times the segment's atoms along K
-    if (s4.steps) copy_pieces(s4.sfa, s4.steps, palog, pa_off + agrp * (unsigned)s4.steps, lds0 + L.sfa0, wave, lane);
-    if (s6.steps) copy_pieces(s6.sfa, s6.steps, palog, pa_off + agrp * (unsigned)s6.steps, lds0 + L.sfa1, wave, lane);
-    if (s8.steps) copy_pieces(s8.sfa, s8.steps, palog, pa_off + agrp * (unsigned)s8.steps, lds0 + L.sfa2, wave, lane);
+    if (s4.steps) copy_pieces(s4.sfa, s4.steps, palog, pa_off, lds0 + L.sfa0, wave, lane);
+    if (s6.steps) copy_pieces(s6.sfa, s6.steps, palog, pa_off, lds0 + L.sfa1, wave, lane);
+    if (s8.steps) copy_pieces(s8.sfa, s8.steps, palog, pa_off, lds0 + L.sfa2, wave, lane);
     if (s4.steps) copy_pieces(s4.sfb, s4.steps, PBLOG, sfb_piece_off + (unsigned)(sfb_katoms_mul * s4.steps) * 512u, lds0 + L.sfb0, wave, lane);
     if (s6.steps) copy_pieces(s6.sfb, s6.steps, PBLOG, sfb_piece_off + (unsigned)(sfb_katoms_mul * s6.steps) * 512u, lds0 + L.sfb1, wave, lane);
     if (s8.steps) copy_pieces(s8.sfb, s8.steps, PBLOG, sfb_piece_off + (unsigned)(sfb_katoms_mul * s8.steps) * 512u, lds0 + L.sfb2, wave, lane);
@@ -582,20 +650,11 @@ mixed_gemm_decode_kernel(DecodeSeg s4, DecodeSeg s6, DecodeSeg s8, int M, int N,
   else wait_vmcnt<0>();
   asm volatile("s_barrier" ::: "memory");
 
-  v4f acc[F][G];
+  v4f acc[F];
 #pragma unroll
-  for (int f = 0; f < F; ++f)
-#pragma unroll
-    for (int gi = 0; gi < G; ++gi) acc[f][gi] = v4f{0.f, 0.f, 0.f, 0.f};
-  // token of this lane in token group gi, as a row of the workgroup's LDS image (tokens past M: the last one again,
-  // never stored), and where its scale bytes sit in a step's pieces
-  int mc[G], sx_off[G];
-#pragma unroll
-  for (int gi = 0; gi < G; ++gi) {
-    mc[gi] = min(16 * gi + i, rows_here - 1);
-    const int mg = m_base + mc[gi];
-    sx_off[gi] = (mg & (L.pa - 1)) * 16 + ((mg >> 5) & 3) * 4;
-  }
+  for (int f = 0; f < F; ++f) acc[f] = v4f{0.f, 0.f, 0.f, 0.f};
+  // this lane's token (tokens past M: the last one again, never stored), and where its scale bytes sit in a step's pieces
+  const int mc = min(i, M - 1), sx_off = mc * 16;
   const int pa16 = L.pa * 16;
 
   auto compute_round = [&](int r, auto buf_c) {
@@ -608,9 +667,7 @@ mixed_gemm_decode_kernel(DecodeSeg s4, DecodeSeg s6, DecodeSeg s8, int M, int N,
         const int q = seg == 0 ? t : (seg == 1 ? t - s4.steps : t - s4.steps - s6.steps);
         const uint8_t* sfa_l = lds + sel3(seg, L.sfa0, L.sfa1, L.sfa2) + q * pa16;
         const uint8_t* sfb_l = lds + sel3(seg, L.sfb0, L.sfb1, L.sfb2) + q * (PB * 16);
-        int s_x[G];
-#pragma unroll
-        for (int gi = 0; gi < G; ++gi) s_x[gi] = sfa_l[sx_off[gi] + g];
+        const int s_x = sfa_l[sx_off + g];
         v8i wf[F];
         int s_w[F];
 #pragma unroll
@@ -619,26 +676,23 @@ mixed_gemm_decode_kernel(DecodeSeg s4, DecodeSeg s6, DecodeSeg s8, int M, int N,
           const v4i w4 = wq[B][k][f];
           wf[f] = v8i{w4[0], w4[1], w4[2], w4[3], 0, 0, 0, 0};
         }
+        if (seg == 0) {
+          const v4i a4 = *reinterpret_cast<const v4i*>(lds + L.x0 + mc * (nblk4 * 16) + q * 64 + g * 16);
+          const v8i xf = {a4[0], a4[1], a4[2], a4[3], 0, 0, 0, 0};
 #pragma unroll
-        for (int gi = 0; gi < G; ++gi) {
-          if (seg == 0) {
-            const v4i a4 = *reinterpret_cast<const v4i*>(lds + L.x0 + mc[gi] * (nblk4 * 16) + q * 64 + g * 16);
-            const v8i xf = {a4[0], a4[1], a4[2], a4[3], 0, 0, 0, 0};
+          for (int f = 0; f < F; ++f) acc[f] = decode_mfma<kFmtE2M1>(wf[f], xf, acc[f], s_w[f], s_x);
+        } else if (seg == 1) {
+          const v2i* p = reinterpret_cast<const v2i*>(lds + L.x1 + mc * (nblk6 * 24) + q * 96 + g * 24);
+          const v2i a = p[0], b = p[1], c = p[2];
+          const v8i xf = {a[0], a[1], b[0], b[1], c[0], c[1], 0, 0};
 #pragma unroll
-            for (int f = 0; f < F; ++f) acc[f][gi] = decode_mfma<kFmtE2M1>(wf[f], xf, acc[f][gi], s_w[f], s_x[gi]);
-          } else if (seg == 1) {
-            const v2i* p = reinterpret_cast<const v2i*>(lds + L.x1 + mc[gi] * (nblk6 * 24) + q * 96 + g * 24);
-            const v2i a = p[0], b = p[1], c = p[2];
-            const v8i xf = {a[0], a[1], b[0], b[1], c[0], c[1], 0, 0};
+          for (int f = 0; f < F; ++f) acc[f] = decode_mfma<kFmtE3M2>(wf[f], xf, acc[f], s_w[f], s_x);
+        } else {
+          const uint8_t* p = lds + L.x2 + mc * (nblk8 * 32) + q * 128 + g * 16;
+          const v4i a4 = *reinterpret_cast<const v4i*>(p), b4v = *reinterpret_cast<const v4i*>(p + 64);
+          const v8i xf = {a4[0], a4[1], a4[2], a4[3], b4v[0], b4v[1], b4v[2], b4v[3]};
 #pragma unroll
-            for (int f = 0; f < F; ++f) acc[f][gi] = decode_mfma<kFmtE3M2>(wf[f], xf, acc[f][gi], s_w[f], s_x[gi]);
-          } else {
-            const uint8_t* p = lds + L.x2 + mc[gi] * (nblk8 * 32) + q * 128 + g * 16;
-            const v4i a4 = *reinterpret_cast<const v4i*>(p), b4v = *reinterpret_cast<const v4i*>(p + 64);
-            const v8i xf = {a4[0], a4[1], a4[2], a4[3], b4v[0], b4v[1], b4v[2], b4v[3]};
-#pragma unroll
-            for (int f = 0; f < F; ++f) acc[f][gi] = decode_mfma<kFmtE4M3>(wf[f], xf, acc[f][gi], s_w[f], s_x[gi]);
-          }
+          for (int f = 0; f < F; ++f) acc[f] = decode_mfma<kFmtE4M3>(wf[f], xf, acc[f], s_w[f], s_x);
         }
       }
     }
@@ -685,161 +739,125 @@ mixed_gemm_decode_kernel(DecodeSeg s4, DecodeSeg s6, DecodeSeg s8, int M, int N,
   // ---- sum the four waves' partial tiles (D^T: lane holds token lane % 16, feature slots 4 * (lane / 16) + v of a group)
   float* partial = reinterpret_cast<float*>(lds + L.partial);
 #pragma unroll
-  for (int f = 0; f < F; ++f)
-#pragma unroll
-    for (int gi = 0; gi < G; ++gi)
-      *reinterpret_cast<v4f*>(partial + ((wave * (F * G) + f * G + gi) * 64 + lane) * 4) = acc[f][gi];
+  for (int f = 0; f < F; ++f) *reinterpret_cast<v4f*>(partial + ((wave * F + f) * 64 + lane) * 4) = acc[f];
   __syncthreads();
+  if (wave >= F) return;
+  const int f = wave;
+  v4f sum = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-  for (int fg = 0; fg < F * G; ++fg) {
-    if ((fg & 3) != wave) continue;
-    const int f = fg / G, gi = fg % G;
-    v4f sum = {0.f, 0.f, 0.f, 0.f};
+  for (int w = 0; w < 4; ++w) sum += *reinterpret_cast<const v4f*>(partial + ((w * F + f) * 64 + lane) * 4);
+  if (i >= M) return;
+  if constexpr (WT) {
+    // feature slot e = 4 g + v of the block is row j + 32 (e % 8) + 16 (e / 8) of the tile
+    const int bx = wg * F + f, row0 = (bx >> 4) * 256 + (bx & 15);
 #pragma unroll
-    for (int w = 0; w < 4; ++w) sum += *reinterpret_cast<const v4f*>(partial + ((w * (F * G) + fg) * 64 + lane) * 4);
-    const int m = m_base + 16 * gi + i;
-    if (m < M) {
-      if constexpr (WT) {
-        // feature slot e = 4 g + v of the block is row j + 32 (e % 8) + 16 (e / 8) of the tile
-        const int bx = wg * F + f, row0 = (bx >> 4) * 256 + (bx & 15);
-#pragma unroll
-        for (int v = 0; v < 4; ++v) {
-          const int e = 4 * g + v, row = row0 + 32 * (e & 7) + 16 * (e >> 3);
-          store1(d, ep, m, row, sum[v]);
-        }
-      } else {
-        // feature slots 4 g ... 4 g + 3 of the group are four consecutive rows
-        const int per_group = 32 / PB, group = blockIdx.x / per_group, c0 = (blockIdx.x % per_group) * PB;
-        const int e = 16 * f + 4 * g;
-        store4(d, ep, m, group * 128 + c0 + e % PB + 32 * (e / PB), sum);
-      }
+    for (int v = 0; v < 4; ++v) {
+      const int e = 4 * g + v;
+      store1(d, ep, i, row0 + 32 * (e & 7) + 16 * (e >> 3), sum[v]);
     }
+  } else {
+    // feature slots 4 g ... 4 g + 3 of the group are four consecutive rows
+    const int per_group = 32 / PB, group = blockIdx.x / per_group, c0 = (blockIdx.x % per_group) * PB;
+    const int e = 16 * f + 4 * g;
+    store4(d, ep, i, group * 128 + c0 + e % PB + 32 * (e / PB), sum);
   }
 }
 
 static int round_up_1k(int v) { return (v + 1023) & ~1023; }
 
-// The decode kernel takes whole 128-wide steps in every segment and, with one token group per workgroup (G = 1), up to
-// 16 tokens and an LDS image of at most 76 KB (two workgroups per CU); with two (G = 2: 32 tokens per workgroup, any
-// number of tokens below 256) whatever fits the LDS of a CU.
-constexpr int kDecodeLds1 = 76 * 1024, kDecodeLds2 = 156 * 1024;
-static bool decode_lds_plan(const DecodeSeg& d4, const DecodeSeg& d6, const DecodeSeg& d8, int M, int F, int G, DecodeLds* L) {
+// The decode kernel takes whole 128-wide steps in every segment and an LDS image of at most 76 KB.
+constexpr int kDecodeLds = 76 * 1024;
+static bool decode_lds_plan(const DecodeSeg& d4, const DecodeSeg& d6, const DecodeSeg& d8, int M, int F, DecodeLds* L) {
   int pos = 0;
   auto take = [&](int bytes) { const int at = pos; pos += round_up_1k(bytes); return at; };
-  const int rows = G == 1 ? M : (M < 32 ? M : 32);   // token rows of a workgroup's image
-  L->pa = G == 2 ? 32 : (M <= 8 ? 8 : 16);
-  L->x0 = take(rows * d4.nblk * 16); L->x1 = take(rows * d6.nblk * 24); L->x2 = take(rows * d8.nblk * 32);
+  L->pa = M <= 8 ? 8 : 16;
+  L->x0 = take(M * d4.nblk * 16); L->x1 = take(M * d6.nblk * 24); L->x2 = take(M * d8.nblk * 32);
   L->sfa0 = take(d4.steps * L->pa * 16); L->sfa1 = take(d6.steps * L->pa * 16); L->sfa2 = take(d8.steps * L->pa * 16);
   L->sfb0 = take(d4.steps * F * 64); L->sfb1 = take(d6.steps * F * 64); L->sfb2 = take(d8.steps * F * 64);
   L->partial = pos;
-  pos += 4 * F * G * 1024;
+  pos += 4 * F * 1024;
   L->total = pos;
-  return pos <= (G == 1 ? kDecodeLds1 : kDecodeLds2);
+  return pos <= kDecodeLds;
 }
 
-// Feature groups of 16 per workgroup of the decode kernel (and what the cost model below assumes of the skinny one).
-static int skinny_feature_groups(int rows, int N, int cus) {
-  const int g = rows <= 16 ? 1 : (rows <= 32 ? 2 : (rows <= 64 ? 4 : 8));
-  return ceil_div(N, 32) * ceil_div(rows, 16 * g) >= cus ? 2 : 1;
+// Token groups (g) and feature groups (f) of 16 per workgroup of the skinny kernel, and its launch time in microseconds:
+// the pair with the lowest estimate.  A workgroup has its CU to itself (LDS) and takes ~2.3 us to fill and drain its
+// pipeline plus the table's nanoseconds per K step; what a further round of workgroups costs above that was fitted.
+// Measured (tile-major weights, N = 4096, K = 14336, 113 steps; estimate): M = 16 11.0 (10.9) us, 32 12.2 (12.0),
+// 64 13.1 (13.0), 128 16.8 (15.7), 200 30.8 (31.7); N = 5120, K = 5120: M = 8 7.0 (6.5), 128 17.5 (16.7); N = 28672,
+// K = 4096, M = 16: 15.0 (13.6).
+struct SkinnyPlan { int g, f; double us; };
+static SkinnyPlan skinny_plan(int M, int N, int steps, int cus) {
+  static const struct { int g, f; double ns; } kForms[] = {{1, 1, 67}, {1, 2, 77}, {1, 4, 102}, {2, 1, 83},
+                                                           {2, 2, 86}, {2, 4, 117}, {4, 1, 99}, {4, 2, 110}};
+  SkinnyPlan best = {0, 0, 0.0};
+  for (const auto& k : kForms) {
+    const int rounds = (int)(((int64_t)ceil_div(N, 16 * k.f) * ceil_div(M, 16 * k.g) + cus - 1) / cus);
+    const double us = 1.0 + rounds * (2.3 + steps * k.ns * 1e-3) + 1.5 * (rounds - 1);
+    if (best.g == 0 || us < best.us) best = {k.g, k.f, us};
+  }
+  return best;
 }
 
-// Token groups (g) and feature groups (f) of 16 per workgroup of the skinny kernel.  A wave's loads per K step are
-// f weight fragments, 2 g token fragments and f + g scale bytes, and the token fragments (16 rows x 16 bytes each)
-// are what the address unit is slowest at: two feature groups per workgroup halve them per output, and more than
-// four token groups per workgroup never paid (M = 128, N = 4096, K = 4096: g = 8, f = 1 22.3 us; g = 4, f = 2 16.9 us;
-// M = 64: g = 4, f = 1 12.0 us; g = 2, f = 2 10.5 us; M = 200: g = 8, f = 2 26.4 us; g = 4, f = 2 23.0 us).  The largest of
-// these that still gives every CU a workgroup.
-static void skinny_groups(int rows, int N, int cus, int* g_out, int* f_out) {
-  const int gmax = rows <= 16 ? 1 : (rows <= 32 ? 2 : 4);
-  for (int f = 2; f >= 1; --f)
-    for (int g = gmax; g >= 1; g >>= 1)
-      if (ceil_div(N, 16 * f) * ceil_div(rows, 16 * g) >= cus) {
-        *g_out = g;
-        *f_out = f;
-        return;
-      }
-  *g_out = 1;
-  *f_out = 1;
-}
-// Feature groups of 16 per workgroup (4, 2 or 1) for the decode kernel with two token groups per workgroup: the most
-// that still leave most CUs a workgroup and whose LDS image fits; 0 if none does (then *L is not valid).
-static int decode2_feature_groups(const DecodeSeg& d4, const DecodeSeg& d6, const DecodeSeg& d8, int M, int N, int cus,
-                                  DecodeLds* L) {
-  const int tg = ceil_div(M, 32);
-  int f = ceil_div(N, 64) * tg >= cus * 3 / 4 ? 4 : (ceil_div(N, 32) * tg >= cus * 3 / 4 ? 2 : 1);
-  while (f > 1 && !decode_lds_plan(d4, d6, d8, M, f, 2, L)) f >>= 1;
-  return decode_lds_plan(d4, d6, d8, M, f, 2, L) ? f : 0;
+// Feature groups of 16 per workgroup of the decode kernel: 4 (tile-major weights; measured on N = 14336: 9.0 against 9.6 us)
+// or 2 as long as that leaves most CUs a workgroup.
+static int decode_feature_groups(int N, bool w_tiled, int cus) {
+  if (w_tiled && ceil_div(N, 64) >= cus * 3 / 4) return 4;
+  return ceil_div(N, 32) >= cus ? 2 : 1;
 }
 
 hipError_t launch_skinny(const DecodeSeg& d4, const DecodeSeg& d6, const DecodeSeg& d8, int M, int N,
                          bool w_tiled, Epilogue ep, uint16_t* d, hipStream_t stream) {
-  const int rows = M;
   DeviceLimits lim;
   if (hipError_t e = device_limits(&lim); e != hipSuccess) return e;
-  // decode: the kernel that stages everything but the weight codes in LDS
+  // The decode kernel, which brings the tokens' codes and all scales into LDS once per workgroup, for whole 128-wide
+  // steps.  Measured against the skinny kernel on tile-major weights, K = 4096:
+  //   N = 4096 (1 feature group per workgroup): M = 1 4.8 against 5.3 us, 8 5.3 against 5.4, 16 5.5 against 5.3;
+  //   N = 6144 (1, a second round of workgroups): M = 8 6.2 against 5.8;
+  //   N = 14336 (4): M = 8 7.5 against 8.3, 16 8.0 against 8.6;  N = 28672 (4, two per CU): 12.6 / 13.6 against 14.8 / 15.3.
+  // So: four feature groups (two such workgroups fit a CU), or one round of workgroups and at most 8 tokens.
   // (a segment's weight codes below 4 GB: the kernel addresses them with 32-bit per-lane offsets)
   const size_t widest = (size_t)(d4.nblk > d6.nblk ? (d4.nblk > d8.nblk ? d4.nblk : d8.nblk) : (d6.nblk > d8.nblk ? d6.nblk : d8.nblk));
   typedef void (*kernel_t)(DecodeSeg, DecodeSeg, DecodeSeg, int, int, int, DecodeLds, Epilogue, uint16_t*);
   const bool whole_steps = ((d4.nblk | d6.nblk | d8.nblk) & 3) == 0 && (size_t)N * widest * 16 < ((size_t)1 << 32);
-  const int spw = (d4.steps + d6.steps + d8.steps + 3) / 4;
+  const int total = d4.steps + d6.steps + d8.steps;
   if (M <= 16 && whole_steps) {
-    // feature groups of 16 per workgroup: 4 (tile-major weights; measured on N = 14336: 9.0 against 9.6 us) or 2 as
-    // long as that leaves most CUs a workgroup
-    int f = skinny_feature_groups(rows, N, lim.cus);
-    if (w_tiled && ceil_div(N, 64) >= lim.cus * 3 / 4) f = 4;
+    const int f = decode_feature_groups(N, w_tiled, lim.cus);
+    // row-major: per group of 128 rows 8 / F workgroups (the last group whole, rows past N clamped and not stored)
+    const dim3 grid(w_tiled ? ceil_div(N, 16 * f) : ceil_div(N, 128) * (8 / f));
     DecodeLds L;
-    if (f == 4 && !decode_lds_plan(d4, d6, d8, M, f, 1, &L)) f = 2;
-    if (decode_lds_plan(d4, d6, d8, M, f, 1, &L)) {
-      // row-major: per group of 128 rows 8 / F workgroups (the last group whole, rows past N clamped and not stored)
-      const dim3 grid(w_tiled ? ceil_div(N, 16 * f) : ceil_div(N, 128) * (8 / f));
+    if ((f == 4 || (M <= 8 && (int)grid.x <= lim.cus)) && decode_lds_plan(d4, d6, d8, M, f, &L)) {
       const kernel_t kernels[2][3] = {
-          {mixed_gemm_decode_kernel<1, false, 1>, mixed_gemm_decode_kernel<2, false, 1>, mixed_gemm_decode_kernel<4, false, 1>},
-          {mixed_gemm_decode_kernel<1, true, 1>, mixed_gemm_decode_kernel<2, true, 1>, mixed_gemm_decode_kernel<4, true, 1>}};
+          {mixed_gemm_decode_kernel<1, false>, mixed_gemm_decode_kernel<2, false>, nullptr},
+          {mixed_gemm_decode_kernel<1, true>, mixed_gemm_decode_kernel<2, true>, mixed_gemm_decode_kernel<4, true>}};
       const kernel_t kernel = kernels[w_tiled ? 1 : 0][f == 4 ? 2 : f - 1];
-      if (hipError_t e = allow_dynamic_lds(reinterpret_cast<const void*>(kernel), kDecodeLds1); e != hipSuccess) return e;
-      hipLaunchKernelGGL(kernel, grid, dim3(256), (size_t)L.total, stream, d4, d6, d8, M, N, spw, L, ep, d);
+      if (hipError_t e = allow_dynamic_lds(reinterpret_cast<const void*>(kernel), kDecodeLds); e != hipSuccess) return e;
+      hipLaunchKernelGGL(kernel, grid, dim3(256), (size_t)L.total, stream, d4, d6, d8, M, N, (total + 3) / 4, L, ep, d);
       return hipGetLastError();
     }
   }
-  // More tokens, in groups of 32 per workgroup, while their codes fit the LDS (K = 4096: 79 KB; not K = 14336): the
-  // token fragments and scales then come from LDS once per workgroup instead of from memory in every K step, which
-  // is what the kernel below spends most of its time on (M = 128, N = 4096, K = 4096: 17 -> 9 us).  The most feature
-  // groups per workgroup (4, 2, 1) that still leave most CUs a workgroup.
-  if (M > 16 && whole_steps) {
-    const int tg = ceil_div(M, 32);
-    DecodeLds L;
-    const int f = decode2_feature_groups(d4, d6, d8, M, N, lim.cus, &L);
-    if (f > 0) {
-      const dim3 grid(w_tiled ? ceil_div(N, 16 * f) : ceil_div(N, 128) * (8 / f), tg);
-      const kernel_t kernels[2][3] = {
-          {mixed_gemm_decode_kernel<1, false, 2>, mixed_gemm_decode_kernel<2, false, 2>, mixed_gemm_decode_kernel<4, false, 2>},
-          {mixed_gemm_decode_kernel<1, true, 2>, mixed_gemm_decode_kernel<2, true, 2>, mixed_gemm_decode_kernel<4, true, 2>}};
-      const kernel_t kernel = kernels[w_tiled ? 1 : 0][f == 4 ? 2 : f - 1];
-      if (hipError_t e = allow_dynamic_lds(reinterpret_cast<const void*>(kernel), kDecodeLds2); e != hipSuccess) return e;
-      hipLaunchKernelGGL(kernel, grid, dim3(256), (size_t)L.total, stream, d4, d6, d8, M, N, spw, L, ep, d);
-      return hipGetLastError();
-    }
-  }
-  const int steps_per_wave = (d4.steps + d6.steps + d8.steps + 3) / 4;
-  int g, f;
-  skinny_groups(rows, N, lim.cus, &g, &f);
-  const dim3 grid(ceil_div(N, 16 * f), ceil_div(rows, 16 * g));
-  const int wt = w_tiled ? 1 : 0;
-  switch (g) {
-    case 1:
-      if (f == 2) hipLaunchKernelGGL((mixed_gemm_skinny_kernel<1, 2>), grid, dim3(256), 0, stream, d4, d6, d8, M, N, steps_per_wave, wt, ep, d);
-      else hipLaunchKernelGGL((mixed_gemm_skinny_kernel<1, 1>), grid, dim3(256), 0, stream, d4, d6, d8, M, N, steps_per_wave, wt, ep, d);
-      break;
-    case 2:
-      if (f == 2) hipLaunchKernelGGL((mixed_gemm_skinny_kernel<2, 2>), grid, dim3(256), 0, stream, d4, d6, d8, M, N, steps_per_wave, wt, ep, d);
-      else hipLaunchKernelGGL((mixed_gemm_skinny_kernel<2, 1>), grid, dim3(256), 0, stream, d4, d6, d8, M, N, steps_per_wave, wt, ep, d);
-      break;
-    default:   // 4 token groups: skinny_groups takes no more
-      if (f == 2) hipLaunchKernelGGL((mixed_gemm_skinny_kernel<4, 2>), grid, dim3(256), 0, stream, d4, d6, d8, M, N, steps_per_wave, wt, ep, d);
-      else hipLaunchKernelGGL((mixed_gemm_skinny_kernel<4, 1>), grid, dim3(256), 0, stream, d4, d6, d8, M, N, steps_per_wave, wt, ep, d);
-      break;
-  }
-  return hipGetLastError();
+  const SkinnyPlan plan = skinny_plan(M, N, total, lim.cus);
+  const dim3 grid(w_tiled ? ceil_div(N, 16 * plan.f) : ceil_div(N, 128) * (8 / plan.f), ceil_div(M, 16 * plan.g));
+  auto launch = [&](auto g_c, auto f_c, auto wt_c) {
+    constexpr int G = decltype(g_c)::value, F = decltype(f_c)::value;
+    constexpr int kLds = 4 * kSkinnySlots<G, F> * kSkinnySlot<G, F>;
+    const auto kernel = mixed_gemm_skinny_kernel<G, F, decltype(wt_c)::value>;
+    if (hipError_t e = allow_dynamic_lds(reinterpret_cast<const void*>(kernel), kLds); e != hipSuccess) return e;
+    hipLaunchKernelGGL(kernel, grid, dim3(256), kLds, stream, d4, d6, d8, M, N, (total + 3) / 4, ep, d);
+    return hipGetLastError();
+  };
+  auto with_f = [&](auto g_c, auto wt_c) {
+    if (plan.f == 1) return launch(g_c, std::integral_constant<int, 1>{}, wt_c);
+    if constexpr (decltype(g_c)::value < 4)   // 4 x 4 groups: no room for a pipeline in the LDS
+      if (plan.f == 4) return launch(g_c, std::integral_constant<int, 4>{}, wt_c);
+    return launch(g_c, std::integral_constant<int, 2>{}, wt_c);
+  };
+  auto with_g = [&](auto wt_c) {
+    if (plan.g == 4) return with_f(std::integral_constant<int, 4>{}, wt_c);
+    if (plan.g == 2) return with_f(std::integral_constant<int, 2>{}, wt_c);
+    return with_f(std::integral_constant<int, 1>{}, wt_c);
+  };
+  return w_tiled ? with_g(std::true_type{}) : with_g(std::false_type{});
 }
 
 }  // namespace
@@ -852,30 +870,15 @@ hipError_t launch_mixed_gemm_256(const uint8_t* an, const uint8_t* bn, const uin
                                  int m_store, int a_rows, int N, int KN, int KS, int KO, bool w_tiled, Epilogue ep,
                                  void* d, hipStream_t stream);
 
-// Rough launch times in microseconds, only to choose between the kernels for fewer than 256 tokens (measured on
-// MI355X, 256 CUs, K = 4096: the whole-tile kernel runs such problems as 256 x 128 tiles when that is at most one
+// Rough launch time of the whole-tile kernel in microseconds, only to choose between the kernels for fewer than 256
+// tokens (measured on MI355X, 256 CUs, K = 4096: it runs such problems as 256 x 128 tiles when that is at most one
 // round -- a 128-wide stage then takes ~0.42 us with at most half of the CUs busy, ~0.45 us with more, plus ~2.5 us --
-// and as 256 x 256 tiles at ~0.95 us a stage plus ~3 us a round otherwise; the decode kernel with two token groups
-// per workgroup takes ~5.5 us plus 22 ns per K step and feature group for each round of one workgroup per CU; the
-// skinny kernel 0.25-0.33 ns per 16 tokens x 16 features x 128 K plus ~5 us: K = 14336, N = 4096, 64 / 128 tokens 28 / 62 us).
+// and as 256 x 256 tiles at ~0.95 us a stage plus ~3 us a round otherwise).  Against it the skinny kernel, measured:
+// N = 18944, K = 3584: M = 32 14.9 against 15.5 us, 64 15.1 against 21.5; N = 4096, K = 14336, M = 200: 47 against 31.
 static double pipelined_us(int M, int N, int stages, int cus) {
   const int whole = ceil_div(M, 256) * ceil_div(N, 256);
   if (whole <= cus / 2) return stages * (ceil_div(M, 128) * ceil_div(N, 256) <= cus / 2 ? 0.42 : 0.45) + 2.5;
   return (double)ceil_div(whole, cus) * (stages * 0.95 + 3.0);
-}
-static double skinny_us(const DecodeSeg& d4, const DecodeSeg& d6, const DecodeSeg& d8, int rows, int N, int steps, int cus,
-                        bool w_tiled) {
-  if (rows > 16 && ((d4.nblk | d6.nblk | d8.nblk) & 3) == 0) {
-    DecodeLds L;
-    const int f2 = decode2_feature_groups(d4, d6, d8, rows, N, cus, &L);
-    if (f2 > 0) {
-      const int wgs = (w_tiled ? ceil_div(N, 16 * f2) : ceil_div(N, 128) * (8 / f2)) * ceil_div(rows, 32);
-      return 1.0 + ceil_div(wgs, cus) * (5.5 + steps * f2 * 0.022);
-    }
-  }
-  int g, f;
-  skinny_groups(rows, N, cus, &g, &f);
-  return 5.0 + (double)ceil_div(rows, 16) * ceil_div(N, 16) * steps * (f == 2 ? 0.25e-3 : 0.33e-3);
 }
 
 // a_rows: token rows for which the activation codes and scales are readable (>= M)
@@ -902,10 +905,12 @@ hipError_t launch_mixed_gemm(const uint8_t* an, const uint8_t* bn, const uint8_t
   const DecodeSeg d6 = {as_, bs, sfas, sfbs, KS / 32, (KS + 127) / 128};
   const DecodeSeg d8 = {ao, bo, sfao, sfbo, KO / 32, (KO + 127) / 128};
   if (mixed_gemm_256_supported(m_pad, N, KN, KS, KO) &&
-      (M >= 256 || pipelined_us(M, N, steps, cus) < skinny_us(d4, d6, d8, M, N, steps, cus, w_tiled)))
+      (M >= 256 || pipelined_us(M, N, steps, cus) < skinny_plan(M, N, steps, cus).us))
     return launch_mixed_gemm_256(an, bn, as_, bs, ao, bo, sfan, sfbn, sfas, sfbs, sfao, sfbo, M, a_rows, N, KN, KS, KO,
                                  w_tiled, ep, d, stream);
-  if (M < 256 && KN + KS + KO > 0) return launch_skinny(d4, d6, d8, M, N, w_tiled, ep, static_cast<uint16_t*>(d), stream);
+  // (the skinny kernel addresses a segment's row-major weight codes with 32-bit offsets)
+  const int widest = KN > KS ? (KN > KO ? KN : KO) : (KS > KO ? KS : KO);
+  if (M < 256 && KN + KS + KO > 0 && (w_tiled || (size_t)N * (size_t)(widest / 2) < ((size_t)1 << 32))) return launch_skinny(d4, d6, d8, M, N, w_tiled, ep, static_cast<uint16_t*>(d), stream);
   // what is left (256 tokens or more with N not a multiple of 8, or with a segment that is not whole 128-wide
   // stages next to an empty one): the direct kernel
   dim3 grid(ceil_div(N, 64), ceil_div(M, 64));

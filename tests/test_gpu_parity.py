@@ -160,7 +160,7 @@ GEMM_SHAPES = [
     (20, 64, 448, 224, 64), (1, 16, 32, 32, 32),
     # decode kernel (M <= 16): ragged N, partial K steps, more K steps than one pass keeps in flight
     (8, 200, 96, 160, 64), (3, 1000, 2560, 1408, 128), (16, 48, 8192, 4096, 1024), (5, 40, 0, 4928, 448),
-    # 128 tokens x 256 features and whole 128-wide K stages (the decode kernel with two token groups per workgroup, or 256 x 128 tiles where they are estimated faster)
+    # 128 tokens x 256 features and whole 128-wide K stages (the skinny kernel, or 256 x 128 tiles where they are estimated faster)
     (128, 256, 256, 0, 0), (128, 256, 0, 256, 0), (128, 256, 0, 0, 128), (128, 256, 128, 0, 128),
     (256, 512, 384, 256, 128), (128, 256, 2560, 1408, 128), (384, 768, 1280, 640, 128),
     # whole tiles with all three segments: the one-workgroup-per-CU kernel
@@ -224,9 +224,8 @@ def test_decode_kernel_matches_oracle(abi, m, n, kn, ks, ko, tiled):
     _check_gemm(d, qx, qw, f"decode {m}x{n}x{k}")
 
 
-# 17 to 255 tokens with whole 128-wide steps: the decode kernel with two token groups (32 tokens) per workgroup where
-# the tokens' codes fit the LDS, one to four feature groups per workgroup, ragged token and feature counts, an empty
-# segment, a token count whose last workgroup has a single token group; K = 14336 does not fit (skinny kernel)
+# 17 to 255 tokens: the skinny kernel, one to four token and feature groups per workgroup, ragged token and feature counts, an
+# empty segment, a token count whose last workgroup has a single token group
 SMALL_M_SHAPES = [
     (128, 4096, 2560, 1408, 128), (32, 512, 2560, 1408, 128), (100, 4096, 2560, 1408, 128), (255, 512, 384, 256, 128),
     (40, 14336, 2560, 1408, 128), (64, 256, 0, 384, 128), (130, 1000, 1280, 0, 256), (17, 264, 128, 128, 128),
@@ -558,9 +557,26 @@ def test_tile_weights_matches_the_layout_formula(abi, n, kseg):
     del z
 
 
+# The skinny kernel's pipelines: fewer K steps than waves, than ring slots, and one more than a ring holds; a last step of
+# 1, 2 and 3 blocks per format (an E3M2 one of 24 or 72 bytes is copied shifted); every (token, feature) group count that
+# the plan picks; the tokens of one scale atom on both sides of row 32, 64 and 128.
+SKINNY_SHAPES = [
+    (9, 256, 32, 32, 32), (16, 256, 128, 96, 0), (31, 256, 0, 32, 96), (64, 512, 3840, 288, 32), (65, 1024, 3584, 160, 96),
+    (129, 2048, 1056, 608, 160), (255, 256, 4224, 2080, 352), (33, 8192, 416, 224, 64), (70, 8192, 416, 480, 160),
+    (200, 4096, 1280, 736, 96), (10, 14336, 416, 480, 160), (40, 18944, 288, 160, 64),
+]
+
+
+@pytest.mark.parametrize("m,n,kn,ks,ko", SKINNY_SHAPES)
+def test_skinny_kernel_at_the_edges_of_its_pipeline(abi, m, n, kn, ks, ko):
+    test_small_batches_match_oracle(abi, m, n, kn, ks, ko, False)
+    if abi.weights_tileable(n, kn, ks, ko):
+        test_small_batches_match_oracle(abi, m, n, kn, ks, ko, True)
+
+
 TILED_SHAPES = [
     # M, N, KN, KS, KO: the 256x256 kernel (plain and with compiled-in segment-boundary copies), ragged
-    # token counts, and the skinny kernel with 1, 2, 4 and 8 token groups
+    # token counts, and the skinny kernel with 1, 2 and 4 token groups
     (256, 256, 128, 128, 128), (512, 512, 256, 384, 128), (256, 768, 2560, 1408, 128), (512, 256, 384, 512, 256),
     (300, 512, 2560, 1408, 128), (1000, 256, 384, 384, 384),
     (8, 512, 2560, 1408, 128), (20, 256, 128, 256, 128), (50, 768, 384, 128, 128), (130, 256, 2560, 896, 128),
