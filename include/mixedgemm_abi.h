@@ -65,6 +65,12 @@ int mg_reorder_quantize_w(const void* w_bf16, const int16_t* idx, int N, int K, 
                           uint8_t* qn, uint8_t* qs, uint8_t* qo,
                           uint8_t* sfn, uint8_t* sfs, uint8_t* sfo, void* stream);
 
+/* mg_reorder_quantize_w and mg_tile_weights in one pass: w_bf16 has n rows, the result N (a multiple of 256, at most 255
+ * more); rows n ... N - 1 are quantized as zeros.  Codes in the tile-major order of mg_tile_weights, scales as
+ * mg_reorder_quantize_w writes them. */
+int mg_reorder_quantize_w_tiled(const void* w_bf16, const int16_t* reorder_index, int n, int N, int K, int KN, int KS, int KO,
+                                uint8_t* qn, uint8_t* qs, uint8_t* qo, uint8_t* sfn, uint8_t* sfs, uint8_t* sfo, void* stream);
+
 /*
  * mg_reorder_quantize_x with an RMSNorm in front, in the same pass over the rows (the layer that feeds
  * a quantized linear in a transformer block; the reference leaves it to the caller and reads the

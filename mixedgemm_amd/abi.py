@@ -23,6 +23,7 @@ MG_FLAG_W_TILED = 1
 
 SYMBOLS = (
     "mg_reorder_quantize_x", "mg_reorder_quantize_w", "mg_mixed_gemm", "mg_mixed_gemm_ex", "mg_padded_rows", "mg_tile_weights",
+    "mg_reorder_quantize_w_tiled",
     "mg_weights_tileable", "mg_fused_linear_ex", "mg_rmsnorm_reorder_quantize_x", "mg_fused_norm_linear",
     "mg_fused_linear",
     "mg_fused_workspace_bytes", "mg_sf_bytes", "mg_sf_offset", "mg_device_synchronize", "mg_status_string",
@@ -51,6 +52,8 @@ def lib() -> ctypes.CDLL:
         for name in ("mg_reorder_quantize_x", "mg_reorder_quantize_w"):
             fn = getattr(L, name)
             fn.restype, fn.argtypes = i, [p, p, i, i, i, i, i, p, p, p, p, p, p, p]
+        L.mg_reorder_quantize_w_tiled.restype = i
+        L.mg_reorder_quantize_w_tiled.argtypes = [p, p, i, i, i, i, i, i, p, p, p, p, p, p, p]
         L.mg_mixed_gemm.restype, L.mg_mixed_gemm.argtypes = i, [p] * 12 + [i] * 5 + [p, p]
         u = ctypes.c_uint
         L.mg_mixed_gemm_ex.restype, L.mg_mixed_gemm_ex.argtypes = i, [p] * 12 + [i] * 6 + [u, p, p]
@@ -238,6 +241,25 @@ def reorder_quantize_w(w, reorder_index, kn, ks, ko, out=None):
     return _reorder_quantize("mg_reorder_quantize_w", MG_OPERAND_B, w, reorder_index, kn, ks, ko, out)
 
 
+def reorder_quantize_w_tiled(w, reorder_index, kn, ks, ko):
+    """reorder_quantize_w with the codes in the tile-major order of tile_weights(), in one pass.  Row counts that are no
+    multiple of 256 are padded to one, the rows past the last quantized as zeros."""
+    got = host().reorder_quantize(MG_OPERAND_B, w, reorder_index, kn, ks, ko, True)
+    if got is not None:
+        return got
+    _require(w, torch.bfloat16, "input")
+    _require(reorder_index, torch.int16, "reorder_index")
+    if w.dim() != 2 or reorder_index.numel() != w.shape[1] or reorder_index.device != w.device:
+        raise MixedGemmError("expected a 2-D weight and an index with an entry per column on its GPU")
+    n, k = w.shape
+    stored = (n + 255) // 256 * 256
+    out = alloc_quant_outputs(stored, kn, ks, ko, MG_OPERAND_B, w.device)
+    status = lib().mg_reorder_quantize_w_tiled(_ptr(w), _ptr(reorder_index), n, stored, k, kn, ks, ko, *(_ptr(t) for t in out),
+                                               _stream(w))
+    check(status, "mg_reorder_quantize_w_tiled")
+    return out
+
+
 def matmul(an, bn, as_, bs, ao, bo, sfan, sfbn, sfas, sfbs, sfao, sfbo, out=None, w_tiled=False):
     """bf16 [M, N]; shapes are recovered from the packed operands.  w_tiled: bn, bs, bo are in the
     tile-major order of tile_weights()."""
@@ -361,16 +383,40 @@ def fused_linear_static(x, reorder_index, bn, bs, bo, sfbn, sfbs, sfbo, kn, ks, 
 
 def check_reorder_index(reorder_index, k=None) -> None:
     """Raises MixedGemmError unless every entry of the int16 index lies in [0, K).  Blocks for a GPU tensor."""
-    if reorder_index.dtype != torch.int16 or not reorder_index.is_contiguous():
-        raise MixedGemmError("reorder_index: expected a contiguous int16 tensor")
-    k = reorder_index.numel() if k is None else int(k)
-    if reorder_index.numel() != k:
-        raise MixedGemmError(f"reorder_index has {reorder_index.numel()} entries, expected {k}")
+    k = _index_entries(reorder_index, k)
     if reorder_index.is_cuda:
         status = lib().mg_check_reorder_index(_ptr(reorder_index), k, _stream(reorder_index))
     else:
         status = lib().mg_check_reorder_index_host(ctypes.c_void_p(reorder_index.data_ptr()), k)
     check(status, "mg_check_reorder_index")
+
+
+def start_check_reorder_index(reorder_index, k=None):
+    """check_reorder_index in two halves: the copy of a GPU tensor's entries to the host is enqueued here, and the function
+    returned waits for it and raises.  What is launched in between does not wait for the check."""
+    k = _index_entries(reorder_index, k)
+    if not reorder_index.is_cuda or k > 32767:
+        check_reorder_index(reorder_index, k)
+        return lambda: None
+    entries = torch.empty(k, dtype=torch.int16, pin_memory=True)
+    with torch.cuda.device(reorder_index.device):
+        entries.copy_(reorder_index.view(-1), non_blocking=True)
+        copied = torch.cuda.Event()
+        copied.record()
+
+    def finish() -> None:
+        copied.synchronize()
+        check(lib().mg_check_reorder_index_host(ctypes.c_void_p(entries.data_ptr()), k), "mg_check_reorder_index")
+    return finish
+
+
+def _index_entries(reorder_index, k) -> int:
+    if reorder_index.dtype != torch.int16 or not reorder_index.is_contiguous():
+        raise MixedGemmError("reorder_index: expected a contiguous int16 tensor")
+    k = reorder_index.numel() if k is None else int(k)
+    if reorder_index.numel() != k:
+        raise MixedGemmError(f"reorder_index has {reorder_index.numel()} entries, expected {k}")
+    return k
 
 
 def weights_tileable(n: int, kn: int, ks: int, ko: int) -> bool:

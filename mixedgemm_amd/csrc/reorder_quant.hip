@@ -16,6 +16,7 @@
 #include <type_traits>
 
 #include "mg_common.h"
+#include "quantize.h"
 
 namespace mg {
 
@@ -24,25 +25,6 @@ namespace {
 __device__ __forceinline__ unsigned perm(unsigned hi, unsigned lo, unsigned sel) {
   return __builtin_amdgcn_perm(hi, lo, sel);
 }
-
-// E8M0 byte of the block scale from the bits of amax (a non-negative float).
-// MAX = fm * 2^pm with fm in [0.5,1): the exponent steps up by one when the
-// mantissa of amax exceeds the mantissa of MAX, which the add below carries
-// into the exponent field.  `fmt` may differ between the lanes of a wave.
-__device__ __forceinline__ int scale_byte(float amax, int fmt) {
-  const unsigned thr = fmt == kFmtE2M1 ? 0x400000u : 0x600000u;  // 6 = 1.5*4, 28 = 1.75*16, 448 = 1.75*256
-  const int pm = fmt == kFmtE2M1 ? 3 : (fmt == kFmtE3M2 ? 5 : 9);
-  const unsigned bits = __float_as_uint(amax);
-  int byte = (int)((bits + (0x7FFFFFu - thr)) >> 23) + 1 - pm;
-  byte = byte < 0 ? 0 : byte;
-  return amax == 0.0f ? 126 : byte;
-}
-
-// roundf(x * rs) for a bf16 value x and a power of two rs, as one multiplication and one round-to-nearest-even:
-// rs1 = rs * (1 + 2^-12).  x * rs has at most 8 significant bits, so x * rs1 is exact in fp32 (21 bits), a
-// tie n + 0.5 moves off the tie away from zero, and every other value stays on its side of the nearest tie
-// (it is at least one 8-bit step from it, the nudge is 2^-12 of the value).  The sign of zero is kept.
-__device__ __forceinline__ float round_scaled(float x, float rs1) { return __builtin_rintf(x * rs1); }
 
 // Stores of the codes and the scale byte.  COUNTED: as inline assembly, one instruction each, so that a kernel
 // which waits with s_waitcnt vmcnt(n) on older requests knows exactly how many stores it has issued since;
@@ -148,31 +130,6 @@ __device__ __forceinline__ void quantize_store(const float (&f)[32], int fmt, ui
 // T > 0: blockDim.x == T and the slot offsets are immediates of the LDS reads; T == 0: any blockDim.x, the
 // slot offset is added to the addresses per row.
 // ---------------------------------------------------------------------------------------------
-// Sum of a double over the 64 lanes of a wave, the same value in every lane: four data-parallel-primitive steps inside
-// the rows of 16 lanes (two register moves and an add each, no trip through the LDS crossbar), then the four row sums
-// through scalar registers.
-template <int CTRL>
-__device__ __forceinline__ double dpp_add(double v) {
-  const uint64_t b = __builtin_bit_cast(uint64_t, v);
-  const int lo = __builtin_amdgcn_mov_dpp((int)(uint32_t)b, CTRL, 0xF, 0xF, true);
-  const int hi = __builtin_amdgcn_mov_dpp((int)(uint32_t)(b >> 32), CTRL, 0xF, 0xF, true);
-  return v + __builtin_bit_cast(double, ((uint64_t)(uint32_t)hi << 32) | (uint32_t)lo);
-}
-__device__ __forceinline__ double wave_sum(double v) {
-  v = dpp_add<0xB1>(v);    // quad_perm [1, 0, 3, 2]
-  v = dpp_add<0x4E>(v);    // quad_perm [2, 3, 0, 1]
-  v = dpp_add<0x141>(v);   // row_half_mirror: the other quad of the 8
-  v = dpp_add<0x140>(v);   // row_mirror: the other 8 of the 16
-  const uint64_t b = __builtin_bit_cast(uint64_t, v);
-  double rows[4];
-#pragma unroll
-  for (int r = 0; r < 4; ++r) {
-    const uint32_t lo = __builtin_amdgcn_readlane((int)(uint32_t)b, 16 * r), hi = __builtin_amdgcn_readlane((int)(uint32_t)(b >> 32), 16 * r);
-    rows[r] = __builtin_bit_cast(double, ((uint64_t)hi << 32) | lo);
-  }
-  return (rows[0] + rows[1]) + (rows[2] + rows[3]);
-}
-
 __device__ __forceinline__ void dma16(const uint8_t* base, unsigned voff, unsigned lds_off) {
   asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1"
                : : "v"(voff), "s"(base), "s"(lds_off) : "memory", "m0");
@@ -217,64 +174,21 @@ __device__ __forceinline__ void gather_wait(unsigned (&u)[16]) {
                  "+v"(u[8]), "+v"(u[9]), "+v"(u[10]), "+v"(u[11]), "+v"(u[12]), "+v"(u[13]), "+v"(u[14]), "+v"(u[15]));
 }
 
-// Half a block (16 gathered values, lane pair 2b / 2b + 1 holds block b): the pair's absmax by one cross-lane
-// step, then the same arithmetic as quantize_store; `half` (0 or 1) says which 16 elements these are.
-template <bool KEEP = false>
-__device__ __forceinline__ void quantize_store_half(const float (&f)[16], int fmt, int half, uint8_t* __restrict__ q,
-                                                    uint8_t* __restrict__ sf) {
-  float amax = 0.0f;
-#pragma unroll
-  for (int p = 0; p < 16; p += 2) amax = __builtin_fmaxf(__builtin_fmaxf(amax, __builtin_fabsf(f[p])), __builtin_fabsf(f[p + 1]));
-  // quad_perm [1, 0, 3, 2]: the other lane of the pair
-  const float other = __uint_as_float((unsigned)__builtin_amdgcn_mov_dpp((int)__float_as_uint(amax), 0xB1, 0xF, 0xF, true));
-  amax = __builtin_fmaxf(amax, other);
-  const int byte = scale_byte(amax, fmt);
-  const float rs1 = __uint_as_float(((unsigned)(254 - byte) << 23) | 0x800u);
-  float v[16];
-#pragma unroll
-  for (int p = 0; p < 16; ++p) v[p] = round_scaled(f[p], rs1);
-  if (half == 0) store1<true>(sf, byte);
-  if (fmt == kFmtE2M1) {
-    v2u out;
-#pragma unroll
-    for (int j = 0; j < 2; ++j) {
-      unsigned w = 0;
-      w = __builtin_amdgcn_cvt_scalef32_pk_fp4_f32(w, v[8 * j + 0], v[8 * j + 1], 1.0f, 0);
-      w = __builtin_amdgcn_cvt_scalef32_pk_fp4_f32(w, v[8 * j + 2], v[8 * j + 3], 1.0f, 1);
-      w = __builtin_amdgcn_cvt_scalef32_pk_fp4_f32(w, v[8 * j + 4], v[8 * j + 5], 1.0f, 2);
-      w = __builtin_amdgcn_cvt_scalef32_pk_fp4_f32(w, v[8 * j + 6], v[8 * j + 7], 1.0f, 3);
-      out[j] = w;
-    }
-    store8<true, KEEP>(q + half * 8, out);
-  } else {
-    if (fmt == kFmtE3M2) {
-      // 16 codes are the first 96 bits of the 32-code conversion
-      v32bf h;
-#pragma unroll
-      for (int p = 0; p < 16; ++p) h[p] = (__bf16)v[p];
-#pragma unroll
-      for (int p = 16; p < 32; ++p) h[p] = (__bf16)0.0f;
-      const v6u w = __builtin_amdgcn_cvt_scalef32_pk32_bf6_bf16(h, 1.0f);
-      typedef unsigned v3u __attribute__((ext_vector_type(3)));
-      const v3u w3 = {w[0], w[1], w[2]};
-      if constexpr (KEEP) asm volatile("global_store_dwordx3 %0, %1, off" : : "v"(q + half * 12), "v"(w3) : "memory");
-      else asm volatile("global_store_dwordx3 %0, %1, off nt" : : "v"(q + half * 12), "v"(w3) : "memory");
-    } else {
-      unsigned out[4];
-#pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        const v2bf lo = {(__bf16)v[4 * j + 0], (__bf16)v[4 * j + 1]};
-        const v2bf hi = {(__bf16)v[4 * j + 2], (__bf16)v[4 * j + 3]};
-        v2s z = {0, 0};
-        z = __builtin_amdgcn_cvt_scalef32_pk_fp8_bf16(z, lo, 1.0f, false);
-        z = __builtin_amdgcn_cvt_scalef32_pk_fp8_bf16(z, hi, 1.0f, true);
-        out[j] = __builtin_bit_cast(unsigned, z);
-      }
-      store16<true, KEEP>(q + half * 16, v4u{out[0], out[1], out[2], out[3]});
-    }
-  }
-}
 
+// Codes and scale byte of half a block to memory, counted stores.
+template <bool KEEP>
+struct StoreHalf {
+  uint8_t* q;    // of the block
+  uint8_t* sf;
+  int half;
+  __device__ __forceinline__ void scale(int byte) const { store1<true>(sf, byte); }
+  __device__ __forceinline__ void codes(v2u v) const { store8<true, KEEP>(q + half * 8, v); }
+  __device__ __forceinline__ void codes(v3u v) const {
+    if constexpr (KEEP) asm volatile("global_store_dwordx3 %0, %1, off" : : "v"(q + half * 12), "v"(v) : "memory");
+    else asm volatile("global_store_dwordx3 %0, %1, off nt" : : "v"(q + half * 12), "v"(v) : "memory");
+  }
+  __device__ __forceinline__ void codes(v4u v) const { store16<true, KEEP>(q + half * 16, v); }
+};
 
 // Which rows a workgroup takes (see the kernel).  With a whole number `a` of rows per workgroup the plain schedule
 // is `a` full iterations; the skewed one is a - 1 full iterations, one without the last generation of workgroups
@@ -288,12 +202,16 @@ struct RowSchedule {
   int width[3];   // then: the first width[j] workgroups take one (0: nobody)
 };
 
-template <int EPL, int T, int NS, bool IS_W, int MAXT, bool KEEP = false, bool NORM = false>
+// TILED (weights): the codes go out in the tile-major order of mg_tile_weights, and rows past src_rows (up to whole
+// tiles) are quantized as zeros.  A row's stores are then 64-byte pieces 16 KB apart instead of one run; the two rows that
+// share a line go to workgroups of one XCD, whose L2 joins them, and the pass is as fast as the row-major one:
+// W[14336, 4096] 38.7 us for quantizing and tiling one after the other, 24.6 in one pass (5.9 TB/s of what it has to move).
+template <int EPL, int T, int NS, bool IS_W, int MAXT, bool KEEP = false, bool NORM = false, bool TILED = false>
 __global__ void __launch_bounds__(MAXT)
 reorder_quant_dma_kernel(const uint8_t* __restrict__ x, const int16_t* __restrict__ idx, int rows, int K, int KN, int KS,
                          int KO, uint8_t* __restrict__ qn, uint8_t* __restrict__ qs, uint8_t* __restrict__ qo,
                          uint8_t* __restrict__ sfn, uint8_t* __restrict__ sfs, uint8_t* __restrict__ sfo, RowSchedule sched,
-                         const uint16_t* __restrict__ gamma, float eps) {
+                         const uint16_t* __restrict__ gamma, float eps, int src_rows) {
   extern __shared__ __align__(16) uint8_t lds[];
   __shared__ double row_sums[NORM ? 2 : 1][NORM ? MAXT / 64 : 1];   // RMSNorm: the waves' sums of squares, by row parity
   static_assert(EPL == 32 || EPL == 16, "one or two lanes per block");
@@ -335,6 +253,8 @@ reorder_quant_dma_kernel(const uint8_t* __restrict__ x, const int16_t* __restric
     return off + first;
   };
   const size_t row_bytes = (size_t)K * 2;
+  // the row to read for a row of the result: past the last one that exists the last one again (its values are dropped)
+  auto src_row = [&](int row) { return TILED ? min(row, src_rows - 1) : row; };
 
   // per-lane byte offsets of the lane's 16-byte pieces of a row (pieces past the row's end: the last one
   // again, into the slot's padding)
@@ -368,7 +288,7 @@ reorder_quant_dma_kernel(const uint8_t* __restrict__ x, const int16_t* __restric
   }
 #pragma unroll
   for (int s = 0; s < NS; ++s)
-    if (s < count) request(x + (size_t)row_of(s) * row_bytes, s * stride);
+    if (s < count) request(x + (size_t)src_row(row_of(s)) * row_bytes, s * stride);
   // RMSNorm: the weights of this lane's pieces of a row (the same for every row); ordinary loads, which the compiler
   // waits for itself where they are first used (with vmcnt(0): once, in the first row)
   v4u gv[kPieces];
@@ -385,8 +305,16 @@ reorder_quant_dma_kernel(const uint8_t* __restrict__ x, const int16_t* __restric
   const int katoms = (kseg + 127) >> 7;
   const int fmt = IS_W ? kFmtE2M1 : (seg == 0 ? kFmtE2M1 : (seg == 1 ? kFmtE3M2 : kFmtE4M3));
   const int blk_bytes = fmt == kFmtE2M1 ? 16 : (fmt == kFmtE3M2 ? 24 : 32);
-  const size_t pitch = (size_t)(kseg >> 5) * blk_bytes;
+  size_t pitch = (size_t)(kseg >> 5) * blk_bytes;
   uint8_t* qbase = (seg == 0 ? qn : (seg == 1 ? qs : qo)) + j * blk_bytes;
+  // Tile-major: a whole 128-wide step of a 256-row tile is 16 KB, of which row r has 64 bytes in copy block r % 16; the
+  // blocks past the last whole step follow as `rows` rows of (blocks % 4).
+  const int whole = kseg >> 7;
+  const bool in_tile = TILED && (j >> 2) < whole;
+  if constexpr (TILED) {
+    qbase = (seg == 0 ? qn : (seg == 1 ? qs : qo)) + (in_tile ? (size_t)(j >> 2) * 16384 : (size_t)rows * whole * 64) + (j & 3) * 16;
+    pitch = in_tile ? (size_t)whole * 16384 : (size_t)((kseg >> 5) & 3) * 16;   // per tile, or per row
+  }
   uint8_t* sfbase = seg == 0 ? sfn : (seg == 1 ? sfs : sfo);
 
   // ---- the index entries are the oldest requests: they are there when at most the row copies are in flight
@@ -450,20 +378,15 @@ reorder_quant_dma_kernel(const uint8_t* __restrict__ x, const int16_t* __restric
       __builtin_amdgcn_s_waitcnt(0xC07F);   // lgkmcnt(0): the sum is in the LDS (a raw barrier implies no wait of the compiler's)
       asm volatile("s_barrier" ::: "memory");   // also: every wave's copies of row i have landed, every wave is past its gather of row i - 1
       if (i >= 1 && i - 1 + NS < count)
-        request(x + (size_t)row_of(i + NS - 1) * row_bytes, ((S + NS - 1) % NS) * stride);
+        request(x + (size_t)src_row(row_of(i + NS - 1)) * row_bytes, ((S + NS - 1) % NS) * stride);
       double tot = 0.0;
       for (int w = 0; w < (nthr >> 6); ++w) tot += row_sums[i & 1][w];
-      const float var = (float)(tot / (double)K);
-      const float rn = (float)(1.0 / __builtin_sqrt((double)(var + eps)));
+      const float rn = rms_scale(tot, K, eps);
 #pragma unroll
       for (int it = 0; it < kPieces; ++it) {
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
-          const unsigned d = a[it][e], g = gv[it][e];
-          const float h0 = (float)(__bf16)(__uint_as_float(d << 16) * rn);
-          const float h1 = (float)(__bf16)(__uint_as_float(d & 0xffff0000u) * rn);
-          const v2bf y = {(__bf16)(__uint_as_float(g << 16) * h0), (__bf16)(__uint_as_float(g & 0xffff0000u) * h1)};
-          a[it][e] = __builtin_bit_cast(unsigned, y);
+          a[it][e] = rms_apply(a[it][e], gv[it][e], rn);
         }
         if (it * nthr + tid < nchunks) *reinterpret_cast<v4u*>(slot + (size_t)(it * nthr + tid) * 16) = a[it];
       }
@@ -473,7 +396,7 @@ reorder_quant_dma_kernel(const uint8_t* __restrict__ x, const int16_t* __restric
       asm volatile("s_barrier" ::: "memory");
       // every wave is past its gather of row i - 1: refill that row's slot
       if (i >= 1 && i - 1 + NS < count)
-        request(x + (size_t)row_of(i + NS - 1) * row_bytes, ((S + NS - 1) % NS) * stride);
+        request(x + (size_t)src_row(row_of(i + NS - 1)) * row_bytes, ((S + NS - 1) % NS) * stride);
     }
     if (has_block) {
       constexpr int kOff = kImm ? S * 2 * EPL * T : -1;
@@ -482,6 +405,18 @@ reorder_quant_dma_kernel(const uint8_t* __restrict__ x, const int16_t* __restric
 #pragma unroll
       for (int h = 0; h < kParts; ++h) gather_wait(u[h]);
       uint8_t* q = qbase + (size_t)row * pitch;
+      if constexpr (TILED) {
+        if (in_tile) {
+          const int h = (row >> 4) & 15;   // rows 16 h ... of the tile: lane quad h / 2 + 8 (h % 2) of the copy block
+          q = qbase + (size_t)(row >> 8) * pitch + (row & 15) * 1024 + ((h >> 1) + 8 * (h & 1)) * 64;
+        }
+        if (row >= src_rows) {   // workgroup-uniform
+#pragma unroll
+          for (int h = 0; h < kParts; ++h)
+#pragma unroll
+            for (int p = 0; p < 16; ++p) u[h][p] = 0u;
+        }
+      }
       uint8_t* sf = sfbase + sf_offset(row, j, katoms);
       if constexpr (EPL == 32) {
         float f[32];
@@ -492,7 +427,7 @@ reorder_quant_dma_kernel(const uint8_t* __restrict__ x, const int16_t* __restric
         float f[16];
 #pragma unroll
         for (int p = 0; p < 16; ++p) f[p] = __uint_as_float(u[0][p]);
-        quantize_store_half<KEEP>(f, fmt, half, q, sf);
+        quantize_half(f, fmt, half, StoreHalf<KEEP>{q, sf, half});
       }
     }
   };
@@ -509,13 +444,14 @@ reorder_quant_dma_kernel(const uint8_t* __restrict__ x, const int16_t* __restric
 
 }  // namespace
 
-// gamma != nullptr: RMSNorm with that weight and eps before the gather (activations only)
+// gamma != nullptr: RMSNorm with that weight and eps before the gather (activations only).  src_rows != 0 (weights only):
+// codes in tile-major order, x has src_rows rows and the result `rows`, a multiple of 256.
 template <bool IS_W>
 hipError_t launch_reorder_quant(const void* x, const int16_t* idx, int rows, int K, int KN, int KS, int KO, uint8_t* qn,
                                 uint8_t* qs, uint8_t* qo, uint8_t* sfn, uint8_t* sfs, uint8_t* sfo,
-                                const void* gamma, float eps, bool keep_codes, hipStream_t stream) {
+                                const void* gamma, float eps, bool keep_codes, int src_rows, hipStream_t stream) {
   if (rows == 0 || K == 0) return hipSuccess;
-  if (gamma != nullptr && IS_W) return hipErrorInvalidValue;
+  if ((gamma != nullptr && IS_W) || (src_rows != 0 && (!IS_W || src_rows > rows || rows % 256 != 0))) return hipErrorInvalidValue;
   const uint16_t* gm = static_cast<const uint16_t*>(gamma);
   const int threads = ((K >> 5) + 63) & ~63;
   const uint8_t* xb = static_cast<const uint8_t*>(x);
@@ -543,7 +479,7 @@ hipError_t launch_reorder_quant(const void* x, const int16_t* idx, int rows, int
     err = allow_dynamic_lds(reinterpret_cast<const void*>(kernel), usable);
     if (err != hipSuccess) return;
     hipLaunchKernelGGL(kernel, dim3(grid), dim3(nthreads), (size_t)lds, stream, xb, idx, rows, K, KN, KS, KO, qn, qs, qo, sfn,
-                       sfs, sfo, sched, gm, eps);
+                       sfs, sfo, sched, gm, eps, src_rows);
     err = hipGetLastError();
   };
   // Measured on M = 4096 ... 16384 rows of K = 3584 ... 18944: two row slots per workgroup, and per CU up to four
@@ -553,50 +489,52 @@ hipError_t launch_reorder_quant(const void* x, const int16_t* idx, int rows, int
   constexpr int kPerCu = 4;
   // keep: the codes stay in the L2 for the kernel that reads them next (activations only); norm: RMSNorm of the row
   // before the gather (activations only; its codes are always kept: what follows a norm is the layer's GEMM)
-  auto dispatch = [&](auto keep_c, auto norm_c) {
+  auto dispatch = [&](auto keep_c, auto norm_c, auto tiled_c) {
+    constexpr bool TI = decltype(tiled_c)::value;
     constexpr bool KP = decltype(keep_c)::value;
     constexpr bool NM = decltype(norm_c)::value;
     if (K <= 8192) {
       // two lanes per block: K/16 lanes, rounded up to whole waves
       const int t2 = ((K >> 4) + 63) & ~63;
       switch (t2) {
-        case 64: launch_dma(reorder_quant_dma_kernel<16, 64, kNS, IS_W, 64, KP, NM>, 16, kNS, 64, kPerCu); break;
-        case 128: launch_dma(reorder_quant_dma_kernel<16, 128, kNS, IS_W, 128, KP, NM>, 16, kNS, 128, kPerCu); break;
-        case 192: launch_dma(reorder_quant_dma_kernel<16, 192, kNS, IS_W, 192, KP, NM>, 16, kNS, 192, kPerCu); break;
-        case 256: launch_dma(reorder_quant_dma_kernel<16, 256, kNS, IS_W, 256, KP, NM>, 16, kNS, 256, kPerCu); break;
-        case 320: launch_dma(reorder_quant_dma_kernel<16, 320, kNS, IS_W, 320, KP, NM>, 16, kNS, 320, kPerCu); break;
-        case 384: launch_dma(reorder_quant_dma_kernel<16, 384, kNS, IS_W, 384, KP, NM>, 16, kNS, 384, kPerCu); break;
-        case 448: launch_dma(reorder_quant_dma_kernel<16, 448, kNS, IS_W, 448, KP, NM>, 16, kNS, 448, kPerCu); break;
-        default: launch_dma(reorder_quant_dma_kernel<16, 512, kNS, IS_W, 512, KP, NM>, 16, kNS, 512, kPerCu); break;
+        case 64: launch_dma(reorder_quant_dma_kernel<16, 64, kNS, IS_W, 64, KP, NM, TI>, 16, kNS, 64, kPerCu); break;
+        case 128: launch_dma(reorder_quant_dma_kernel<16, 128, kNS, IS_W, 128, KP, NM, TI>, 16, kNS, 128, kPerCu); break;
+        case 192: launch_dma(reorder_quant_dma_kernel<16, 192, kNS, IS_W, 192, KP, NM, TI>, 16, kNS, 192, kPerCu); break;
+        case 256: launch_dma(reorder_quant_dma_kernel<16, 256, kNS, IS_W, 256, KP, NM, TI>, 16, kNS, 256, kPerCu); break;
+        case 320: launch_dma(reorder_quant_dma_kernel<16, 320, kNS, IS_W, 320, KP, NM, TI>, 16, kNS, 320, kPerCu); break;
+        case 384: launch_dma(reorder_quant_dma_kernel<16, 384, kNS, IS_W, 384, KP, NM, TI>, 16, kNS, 384, kPerCu); break;
+        case 448: launch_dma(reorder_quant_dma_kernel<16, 448, kNS, IS_W, 448, KP, NM, TI>, 16, kNS, 448, kPerCu); break;
+        default: launch_dma(reorder_quant_dma_kernel<16, 512, kNS, IS_W, 512, KP, NM, TI>, 16, kNS, 512, kPerCu); break;
       }
     } else if (K <= 20480) {
       // one lane per block: the workgroups are large enough as it is, and LDS (two rows per workgroup) bounds how
       // many a CU holds
       switch (threads) {
-        case 320: launch_dma(reorder_quant_dma_kernel<32, 320, kNS, IS_W, 320, KP, NM>, 32, kNS, 320, kPerCu); break;
-        case 384: launch_dma(reorder_quant_dma_kernel<32, 384, kNS, IS_W, 384, KP, NM>, 32, kNS, 384, kPerCu); break;
-        case 448: launch_dma(reorder_quant_dma_kernel<32, 448, kNS, IS_W, 448, KP, NM>, 32, kNS, 448, kPerCu); break;
-        case 512: launch_dma(reorder_quant_dma_kernel<32, 512, kNS, IS_W, 512, KP, NM>, 32, kNS, 512, kPerCu); break;
-        case 576: launch_dma(reorder_quant_dma_kernel<32, 576, kNS, IS_W, 576, KP, NM>, 32, kNS, 576, kPerCu); break;
-        default: launch_dma(reorder_quant_dma_kernel<32, 640, kNS, IS_W, 640, KP, NM>, 32, kNS, 640, kPerCu); break;
+        case 320: launch_dma(reorder_quant_dma_kernel<32, 320, kNS, IS_W, 320, KP, NM, TI>, 32, kNS, 320, kPerCu); break;
+        case 384: launch_dma(reorder_quant_dma_kernel<32, 384, kNS, IS_W, 384, KP, NM, TI>, 32, kNS, 384, kPerCu); break;
+        case 448: launch_dma(reorder_quant_dma_kernel<32, 448, kNS, IS_W, 448, KP, NM, TI>, 32, kNS, 448, kPerCu); break;
+        case 512: launch_dma(reorder_quant_dma_kernel<32, 512, kNS, IS_W, 512, KP, NM, TI>, 32, kNS, 512, kPerCu); break;
+        case 576: launch_dma(reorder_quant_dma_kernel<32, 576, kNS, IS_W, 576, KP, NM, TI>, 32, kNS, 576, kPerCu); break;
+        default: launch_dma(reorder_quant_dma_kernel<32, 640, kNS, IS_W, 640, KP, NM, TI>, 32, kNS, 640, kPerCu); break;
       }
     } else {
-      launch_dma(reorder_quant_dma_kernel<32, 0, 2, IS_W, 1024, KP, NM>, 32, 2, threads, kPerCu);
+      launch_dma(reorder_quant_dma_kernel<32, 0, 2, IS_W, 1024, KP, NM, TI>, 32, 2, threads, kPerCu);
     }
   };
   if constexpr (IS_W) {
-    dispatch(std::false_type{}, std::false_type{});
+    if (src_rows != 0) dispatch(std::false_type{}, std::false_type{}, std::true_type{});
+    else dispatch(std::false_type{}, std::false_type{}, std::false_type{});
   } else {
-    if (gamma != nullptr) dispatch(std::true_type{}, std::true_type{});
-    else if (keep_codes) dispatch(std::true_type{}, std::false_type{});
-    else dispatch(std::false_type{}, std::false_type{});
+    if (gamma != nullptr) dispatch(std::true_type{}, std::true_type{}, std::false_type{});
+    else if (keep_codes) dispatch(std::true_type{}, std::false_type{}, std::false_type{});
+    else dispatch(std::false_type{}, std::false_type{}, std::false_type{});
   }
   return err;
 }
 
 template hipError_t launch_reorder_quant<false>(const void*, const int16_t*, int, int, int, int, int, uint8_t*, uint8_t*,
-                                                uint8_t*, uint8_t*, uint8_t*, uint8_t*, const void*, float, bool, hipStream_t);
+                                                uint8_t*, uint8_t*, uint8_t*, uint8_t*, const void*, float, bool, int, hipStream_t);
 template hipError_t launch_reorder_quant<true>(const void*, const int16_t*, int, int, int, int, int, uint8_t*, uint8_t*,
-                                               uint8_t*, uint8_t*, uint8_t*, uint8_t*, const void*, float, bool, hipStream_t);
+                                               uint8_t*, uint8_t*, uint8_t*, uint8_t*, const void*, float, bool, int, hipStream_t);
 
 }  // namespace mg

@@ -146,15 +146,17 @@ Six quant_outputs(int64_t rows, int64_t kn, int64_t ks, int64_t ko, int operand,
   return {codes(kn / 2), codes(w ? ks / 2 : ks / 4 * 3), codes(w ? ko / 2 : ko), scales(kn), scales(ks), scales(ko)};
 }
 
+// `tiled` (weights, no `out`): codes in tile-major order, rows padded to whole 256-row tiles.
 std::optional<Six> reorder_quantize(const Tensor& t, const Tensor& index, int64_t kn, int64_t ks, int64_t ko, int operand,
-                                    const Six* out) {
+                                    const Six* out, bool tiled = false) {
   const int64_t k = kn + ks + ko;
   if (!split_ok(kn, ks, ko) || !on_gpu(t, at::kBFloat16) || t.dim() != 2 || t.size(1) != k || t.size(0) > INT32_MAX)
     return std::nullopt;
   const at::Device device = t.device();
   if (!on_gpu(index, at::kShort, device) || index.numel() != k) return std::nullopt;
-  const int64_t rows = t.size(0);
+  const int64_t n = t.size(0), rows = tiled ? (n + 255) / 256 * 256 : n;
   const bool w = operand == MG_OPERAND_B;
+  if ((tiled && (!w || out || n == 0)) || rows > INT32_MAX) return std::nullopt;
   const c10::hip::HIPGuard guard(device.index());
   Six q;
   if (out) {
@@ -168,9 +170,13 @@ std::optional<Six> reorder_quantize(const Tensor& t, const Tensor& index, int64_
   } else {
     q = quant_outputs(rows, kn, ks, ko, operand, device);
   }
-  const int status = (w ? mg_reorder_quantize_w : mg_reorder_quantize_x)(
-      ptr<void>(t), ptr<int16_t>(index), (int)rows, (int)k, (int)kn, (int)ks, (int)ko, ptr<uint8_t>(q[0]), ptr<uint8_t>(q[1]),
-      ptr<uint8_t>(q[2]), ptr<uint8_t>(q[3]), ptr<uint8_t>(q[4]), ptr<uint8_t>(q[5]), stream_of(t));
+  const int status =
+      tiled ? mg_reorder_quantize_w_tiled(ptr<void>(t), ptr<int16_t>(index), (int)n, (int)rows, (int)k, (int)kn, (int)ks, (int)ko,
+                                          ptr<uint8_t>(q[0]), ptr<uint8_t>(q[1]), ptr<uint8_t>(q[2]), ptr<uint8_t>(q[3]),
+                                          ptr<uint8_t>(q[4]), ptr<uint8_t>(q[5]), stream_of(t))
+            : (w ? mg_reorder_quantize_w : mg_reorder_quantize_x)(
+                  ptr<void>(t), ptr<int16_t>(index), (int)rows, (int)k, (int)kn, (int)ks, (int)ko, ptr<uint8_t>(q[0]),
+                  ptr<uint8_t>(q[1]), ptr<uint8_t>(q[2]), ptr<uint8_t>(q[3]), ptr<uint8_t>(q[4]), ptr<uint8_t>(q[5]), stream_of(t));
   if (status != MG_OK) return std::nullopt;
   return q;
 }
@@ -316,18 +322,18 @@ PyObject* py_layer(PyObject*, PyObject* const* a, Py_ssize_t n) {
   });
 }
 
-// (operand, t, reorder_index, kn, ks, ko, out)
+// (operand, t, reorder_index, kn, ks, ko, out or None, or True: weights in tile-major order)
 PyObject* py_reorder_quantize(PyObject*, PyObject* const* a, Py_ssize_t n) {
   return guarded([&]() -> PyObject* {
     if (n != 7) throw NotTaken{};
     Six out;
-    const bool given = a[6] != Py_None;
+    const bool tiled = a[6] == Py_True, given = a[6] != Py_None && !tiled;
     if (given) {
       if (!PyTuple_Check(a[6]) || PyTuple_GET_SIZE(a[6]) != 6) throw NotTaken{};
       for (int i = 0; i < 6; ++i) out[i] = tensor_arg(PyTuple_GET_ITEM(a[6], i));
     }
     std::optional<Six> q = reorder_quantize(tensor_arg(a[1]), tensor_arg(a[2]), int_arg(a[3]), int_arg(a[4]), int_arg(a[5]),
-                                            (int)int_arg(a[0]), given ? &out : nullptr);
+                                            (int)int_arg(a[0]), given ? &out : nullptr, tiled);
     if (q && given) {
       Py_INCREF(a[6]);
       return a[6];

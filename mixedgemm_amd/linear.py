@@ -82,14 +82,16 @@ class PackedWeights:
         bindings.cpp:188-305); with `tile`, shapes that allow it are then put in tile-major order."""
         split = tuple(split) if split is not None else default_split(weight.shape[1])
         n = weight.shape[0]
-        abi.check_reorder_index(reorder_index, weight.shape[1])
+        check = abi.start_check_reorder_index(reorder_index, weight.shape[1])   # (the kernels read any index safely)
         # the whole-tile kernel wants a multiple of 256 features: zero rows are cheap, the layer drops their outputs
-        if tile and n > 256 and n % 256 and abi.weights_tileable((n + 255) // 256 * 256, *split):
-            pad = torch.zeros(((n + 255) // 256 * 256 - n, weight.shape[1]), dtype=weight.dtype, device=weight.device)
-            weight = torch.cat([weight, pad])
-        q = abi.reorder_quantize_w(weight, reorder_index, *split)
-        pw = cls(*q, reorder_index, split, False, n if weight.shape[0] != n else 0)
-        return pw.tile() if tile and pw.tileable() else pw
+        stored = (n + 255) // 256 * 256
+        if tile and (n == stored or n > 256) and abi.weights_tileable(stored, *split):
+            q = abi.reorder_quantize_w_tiled(weight, reorder_index, *split)
+            pw = cls(*q, reorder_index, split, True, n if stored != n else 0)
+        else:
+            pw = cls(*abi.reorder_quantize_w(weight, reorder_index, *split), reorder_index, split)
+        check()
+        return pw
 
     def tileable(self) -> bool:
         return abi.weights_tileable(self.rows, *self.split)

@@ -574,6 +574,29 @@ def test_skinny_kernel_at_the_edges_of_its_pipeline(abi, m, n, kn, ks, ko):
         test_small_batches_match_oracle(abi, m, n, kn, ks, ko, True)
 
 
+# Codes and scales of the one-pass weight packing against quantizing (with rows of zeros) and tiling one after the other:
+# whole tiles and a last tile of 1, 8 and 255 rows, one and two lanes per block, a run-time workgroup size (K > 20480),
+# and 1 to 3 blocks past a segment's last whole step.
+@pytest.mark.parametrize("n,kn,ks,ko", [
+    (256, 128, 128, 128), (512, 2560, 1408, 128), (257, 416, 224, 160), (264, 512, 0, 0), (511, 384, 0, 128),
+    (2048, 8960, 4928, 448), (300, 11776, 6560, 608), (256, 20224, 256, 128), (1100, 512, 160, 352)])
+def test_weights_quantized_straight_into_tile_major_order(abi, n, kn, ks, ko):
+    k, stored = kn + ks + ko, (n + 255) // 256 * 256
+    assert abi.weights_tileable(stored, kn, ks, ko)
+    w = H.make_weights(n, k, 41 + n).to(DEV)
+    idx = torch.randperm(k, generator=torch.Generator().manual_seed(n)).to(torch.int16).to(DEV)
+    got = abi.reorder_quantize_w_tiled(w, idx, kn, ks, ko)
+    q = abi.reorder_quantize_w(torch.cat([w, torch.zeros(stored - n, k, dtype=w.dtype, device=DEV)]), idx, kn, ks, ko)
+    want = abi.tile_weights(*q[:3])
+    for a, b in zip(got[:3], want):
+        assert torch.equal(a, b)
+    rows = torch.arange(stored)
+    for a, b, kseg in zip(got[3:], q[3:], (kn, ks, ko)):
+        for kb in range(kseg // 32):   # the bytes of blocks that exist
+            at = torch.tensor([abi.lib().mg_sf_offset(int(r), kb, kseg) for r in rows[::37]], device=DEV)
+            assert torch.equal(a[at], b[at])
+
+
 TILED_SHAPES = [
     # M, N, KN, KS, KO: the 256x256 kernel (plain and with compiled-in segment-boundary copies), ragged
     # token counts, and the skinny kernel with 1, 2 and 4 token groups
