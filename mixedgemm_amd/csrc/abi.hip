@@ -17,6 +17,9 @@ hipError_t launch_mixed_gemm(const uint8_t* an, const uint8_t* bn, const uint8_t
                              const uint8_t* sfas, const uint8_t* sfbs, const uint8_t* sfao, const uint8_t* sfbo, int M,
                              int a_rows, int N, int KN, int KS, int KO, unsigned flags, Epilogue ep, void* d,
                              hipStream_t stream);
+hipError_t launch_token_linear(const void* x, const int16_t* idx, const void* gamma, float eps, const uint8_t* bn, const uint8_t* bs,
+                               const uint8_t* bo, const uint8_t* sfbn, const uint8_t* sfbs, const uint8_t* sfbo, int M, int N,
+                               int KN, int KS, int KO, bool w_tiled, Epilogue ep, void* d, hipStream_t stream, bool* taken);
 hipError_t launch_tile_weights(const uint8_t* src, uint8_t* dst, int N, int kseg, hipStream_t stream);
 bool mixed_gemm_256_supported(int M, int N, int KN, int KS, int KO);
 size_t calibrate_workspace_bytes(int K);
@@ -190,6 +193,17 @@ int mg_linear(const void* x_bf16, const void* gamma_bf16, float eps, const int16
   if (bias_bf16 && !aligned16(bias_bf16)) return MG_ERR_BAD_POINTER;
   if (!workspace || (reinterpret_cast<uintptr_t>(workspace) & 255u)) return MG_ERR_BAD_POINTER;
   if (workspace_bytes < mg_fused_workspace_bytes(M, KN, KS, KO)) return MG_ERR_BAD_SHAPE;
+  // a token or two: one launch, where it is the faster way (what is wrong with the operands is for the calls below to say)
+  const bool tiled = (flags & MG_FLAG_W_TILED) != 0;
+  if ((flags & ~MG_FLAG_W_TILED) == 0 && (!tiled || mg_weights_tileable(N, KN, KS, KO)) && ptr_ok(x_bf16, true) && ptr_ok(idx, true) &&
+      ptr_ok(d_bf16, true) && ptr_ok(bn, KN > 0) && ptr_ok(bs, KS > 0) && ptr_ok(bo, KO > 0) && (KN == 0 || sfbn) &&
+      (KS == 0 || sfbs) && (KO == 0 || sfbo)) {
+    bool taken = false;
+    const hipError_t e = mg::launch_token_linear(x_bf16, idx, gamma_bf16, eps, bn, bs, bo, sfbn, sfbs, sfbo, M, N, KN, KS, KO, tiled,
+                                                 mg::Epilogue{static_cast<const uint16_t*>(bias_bf16), n_out}, d_bf16,
+                                                 static_cast<hipStream_t>(stream), &taken);
+    if (e != hipSuccess || taken) return (int)e;
+  }
   const int R = mg_padded_rows(M);
   uint8_t* p = static_cast<uint8_t*>(workspace);
   uint8_t* qn = p;  p += align256((size_t)R * (KN / 2));

@@ -22,6 +22,7 @@
 #include <type_traits>
 
 #include "mg_common.h"
+#include "quantize.h"
 
 namespace mg {
 
@@ -469,23 +470,25 @@ __device__ __forceinline__ const uint8_t* sel3p(int seg, const uint8_t* p0, cons
                                           (reinterpret_cast<uint64_t>(p2) & m2));
 }
 
-// Copies `bytes` (a multiple of 16) from src to LDS offset dst in units of 1 KB, unit u by wave u % 4; lanes past
+// Copies `bytes` (a multiple of 16) from src to LDS offset dst in units of 1 KB, unit u by wave u % W; lanes past
 // the end copy the last 16 bytes again (into the padding that rounds every region up to whole units).
+template <int W = 4>
 __device__ __forceinline__ void copy_region(const uint8_t* src, int bytes, unsigned dst, int wave, int lane) {
   const int units = (bytes + 1023) >> 10, chunks = bytes >> 4;
-  for (int u = wave; u < units; u += 4)
+  for (int u = wave; u < units; u += W)
     dma16_at(src, (unsigned)min(u * 64 + lane, chunks - 1) * 16u, dst + (unsigned)u * 1024u);
 }
 
 // Copies P (4, 8 or 16, a power of two) 16-byte pieces per K step of a segment's scale atoms (512 bytes per step)
 // to LDS as [step][piece]; piece_off is this lane's piece (lane % P) as a byte offset inside the atom (and, for
-// pieces of another group of 128 rows, that group's distance).  Units of 1 KB = 64 / P steps, unit u by wave u % 4;
+// pieces of another group of 128 rows, that group's distance).  Units of 1 KB = 64 / P steps, unit u by wave u % W;
 // steps past the last one copy it again (into the region's padding).
 // P = 1 << plog pieces per step (a power of two: no divisions by a run-time value here)
+template <int W = 4>
 __device__ __forceinline__ void copy_pieces(const uint8_t* src, int steps, int plog, unsigned piece_off, unsigned dst,
                                             int wave, int lane) {
   const int per_unit = 64 >> plog, units = (steps + per_unit - 1) >> (6 - plog);
-  for (int u = wave; u < units; u += 4) {
+  for (int u = wave; u < units; u += W) {
     const int q = min(u * per_unit + (lane >> plog), steps - 1);
     dma16_at(src, (unsigned)q * 512u + piece_off, dst + (unsigned)u * 1024u);
   }
@@ -763,6 +766,288 @@ mixed_gemm_decode_kernel(DecodeSeg s4, DecodeSeg s6, DecodeSeg s8, int M, int N,
   }
 }
 
+// ---------------------------------------------------------------------------
+// Token kernel: quantization and GEMM of a few tokens in one launch.
+//
+// For a token or two the quantizer is a launch of as many workgroups whose 2.5 us are latency, one memory round trip
+// after the other, in front of a GEMM that waits for a round trip of its own.  Here every workgroup quantizes the tokens
+// for itself, in LDS, while its first weights are on their way: x, the index (and the RMSNorm's weight) are copied to
+// LDS, then the weight scales, then the first NS - 1 steps of weight codes of each ring; the tokens are gathered and
+// quantized, their codes and scale bytes written to LDS, while the weights arrive.  The K loop is the skinny kernel's
+// with one token group, its slots holding weight codes only.  The codes are the quantizer's and the sums are added in the
+// order of the decode and the skinny kernel: the same bits.
+//
+// What bounds it is latency: launch, first copies, LDS gathers (~0.5 us for every 8192 channels of the tokens), then the
+// weights' arrival.  N = 4096, K = 4096, tile-major, in a graph, two launches -> one: M = 1 7.5 -> 6.0 us, 2 7.9 -> 6.4, 4
+// 7.7 -> 7.5 (8: 7.8 -> 10.0, not taken); N = 14336, M = 1 10.3 -> 8.0, 4 10.2 -> 9.3; with RMSNorm, N = 4096: M = 1
+// 8.2 -> 7.1, 2 8.4 -> 8.0 (4: 8.4 -> 9.7, not taken).  A layer call of one token from Python: 9.1 -> 7.0 us.
+// ---------------------------------------------------------------------------
+constexpr int kTokenRows = 8;    // most tokens (a wave each in the RMSNorm)
+constexpr int kTokenWaves = 8;   // all quantize; four of them also run the K loop
+struct TokenLds {   // byte offsets behind the rings
+  int x, idx, gamma;     // bf16 rows, index, RMSNorm weight
+  int q0, q1, q2;        // codes per segment
+  int sx0, sx1, sx2;     // their scale bytes: per step kTokenRows x 4
+  int sw0, sw1, sw2;     // weight scale pieces: per step 4 F x 16
+  int sums;              // RMSNorm: the waves' sums of squares
+  int total;
+};
+// slots per wave: 48 ... 80 KB of weight codes in flight per CU
+template <int F>
+constexpr int kTokenSlots = F == 1 ? 12 : (F == 2 ? 8 : 5);
+
+// waits until at most `steps` (wave-uniform) steps of PER copies each are in flight
+template <int PER>
+__device__ __forceinline__ void wait_steps(int steps) {
+  switch (steps) {
+#define MG_STEPS_CASE(N) case N: wait_vmcnt<N * PER>(); break;
+    MG_STEPS_CASE(1) MG_STEPS_CASE(2) MG_STEPS_CASE(3) MG_STEPS_CASE(4) MG_STEPS_CASE(5) MG_STEPS_CASE(6)
+    MG_STEPS_CASE(7) MG_STEPS_CASE(8) MG_STEPS_CASE(9) MG_STEPS_CASE(10) MG_STEPS_CASE(11)
+#undef MG_STEPS_CASE
+    default: wait_vmcnt<0>(); break;
+  }
+}
+
+// Codes and scale byte of half a block to LDS.
+struct LdsHalf {
+  uint8_t* q;    // of the block
+  uint8_t* sf;
+  int half;
+  __device__ __forceinline__ void scale(int byte) const { *sf = (uint8_t)byte; }
+  __device__ __forceinline__ void codes(v2u v) const { *reinterpret_cast<v2u*>(q + half * 8) = v; }
+  __device__ __forceinline__ void codes(v3u v) const {
+    unsigned* p = reinterpret_cast<unsigned*>(q + half * 12);
+    p[0] = v[0]; p[1] = v[1]; p[2] = v[2];
+  }
+  __device__ __forceinline__ void codes(v4u v) const { *reinterpret_cast<v4u*>(q + half * 16) = v; }
+};
+
+__device__ __forceinline__ void lds_barrier() {   // this wave's LDS accesses are done, then every wave's
+  asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+}
+
+template <int F, bool WT, bool NORM>
+__global__ void __launch_bounds__(64 * kTokenWaves)
+mixed_gemm_token_kernel(const uint8_t* __restrict__ x, const uint8_t* __restrict__ gamma, const uint8_t* __restrict__ idx,
+                        float eps, int K, DecodeSeg s4, DecodeSeg s6, DecodeSeg s8, int M, int N, int steps_per_wave,
+                        TokenLds L, Epilogue ep, uint16_t* __restrict__ d) {
+  constexpr int NS = kTokenSlots<F>, kSlot = 1024 * F;
+  constexpr int PB = 4 * F, PBLOG = F == 1 ? 2 : (F == 2 ? 3 : 4);
+  static_assert(NS - 1 <= 11, "wait_steps");
+  extern __shared__ __align__(16) uint8_t lds[];
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int i = lane & 15, g = lane >> 4;
+  const unsigned lds0 = (unsigned)(size_t)(__attribute__((address_space(3))) uint8_t*)lds;
+  // four waves share the K steps, as in the other kernels
+  const uint8_t* const ring = lds + wave * (NS * kSlot);
+  const unsigned ring0 = lds0 + (unsigned)wave * (NS * kSlot);
+  const int t6 = s4.steps, t8 = s4.steps + s6.steps, total = t8 + s8.steps;
+  const int t_begin = wave < 4 ? wave * steps_per_wave : total, t_end = min(total, t_begin + steps_per_wave);
+
+  // ---- what everybody waits for first: tokens, index, RMSNorm weight, weight scales
+  copy_region<kTokenWaves>(x, M * K * 2, lds0 + L.x, wave, lane);
+  copy_region<kTokenWaves>(idx, K * 2, lds0 + L.idx, wave, lane);
+  if constexpr (NORM) copy_region<kTokenWaves>(gamma, K * 2, lds0 + L.gamma, wave, lane);
+
+  // ---- the workgroup's weight rows, as in the skinny kernel
+  int wg = blockIdx.x;
+  if constexpr (WT) {
+    constexpr int kPer = 16 / F;
+    if ((int)gridDim.x % (8 * kPer) == 0) {
+      const int xcd = wg & 7, slot = wg >> 3;
+      wg = ((slot / kPer) * 8 + xcd) * kPer + slot % kPer;
+    }
+  }
+  constexpr int per_group = 32 / PB;
+  const int tile = (wg * F) >> 4, j0 = (wg * F) & 15;                    // tile-major
+  const int group = wg / per_group, c0 = (wg % per_group) * PB;          // row-major
+  auto feature = [&](int f, int e) {
+    if constexpr (WT) return tile * 256 + j0 + f + 32 * (e & 7) + 16 * (e >> 3);
+    else return group * 128 + c0 + (16 * f + e) % PB + 32 * ((16 * f + e) / PB);
+  };
+  int sw_off[F], wrow[F];
+#pragma unroll
+  for (int f = 0; f < F; ++f) {
+    if constexpr (WT) sw_off[f] = (((i & 7) >> 2) * 2 * F + (i >> 3) * F + f) * 16 + (i & 3) * 4 + g;
+    else sw_off[f] = ((16 * f + i) % PB) * 16 + ((16 * f + i) / PB) * 4 + g;
+    wrow[f] = min(feature(f, lane >> 2), N - 1);   // rows past N: read again, never stored
+  }
+  {
+    const int pl = lane % PB;
+    const unsigned piece = WT ? (unsigned)(j0 + pl % F + 16 * ((pl / F) & 1)) * 16u : (unsigned)(c0 + pl) * 16u;
+    const unsigned mul = WT ? (unsigned)(tile * 2 + pl / (2 * F)) : (unsigned)group;
+    if (s4.steps) copy_pieces<kTokenWaves>(s4.sfb, s4.steps, PBLOG, piece + mul * (unsigned)s4.steps * 512u, lds0 + L.sw0, wave, lane);
+    if (s6.steps) copy_pieces<kTokenWaves>(s6.sfb, s6.steps, PBLOG, piece + mul * (unsigned)s6.steps * 512u, lds0 + L.sw1, wave, lane);
+    if (s8.steps) copy_pieces<kTokenWaves>(s8.sfb, s8.steps, PBLOG, piece + mul * (unsigned)s8.steps * 512u, lds0 + L.sw2, wave, lane);
+  }
+
+  // ---- the first steps of weight codes
+  const int wpos = (lane & 3) ^ ((lane >> 4) & 3);   // the 16-byte piece of its row that this lane copies
+  auto request = [&](int t, unsigned slot) __attribute__((always_inline)) {
+    if (t >= t_end) return;
+    const int seg = t < t6 ? 0 : (t < t8 ? 1 : 2), q = t - sel3(seg, 0, t6, t8);
+    const uint8_t* b = sel3p(seg, s4.b, s6.b, s8.b);
+    const int nblk = sel3(seg, s4.nblk, s6.nblk, s8.nblk), whole = nblk >> 2, left = min(nblk - 4 * q, 4);
+    const unsigned wp = (unsigned)min(wpos, left - 1) * 16u;
+#pragma unroll
+    for (int f = 0; f < F; ++f) {
+      const unsigned at = slot + 1024u * f;
+      if constexpr (WT) {
+        if (q < whole) dma16_at(b + (((size_t)tile * whole + q) * 16 + j0 + f) * 1024, (unsigned)(lane >> 2) * 64u + wp, at);
+        else dma16_at(b + (size_t)(N >> 8) * whole * 16384, (unsigned)wrow[f] * (unsigned)(nblk & 3) * 16u + wp, at);
+      } else {
+        dma16_at(b + (size_t)q * 64, (unsigned)wrow[f] * (unsigned)nblk * 16u + wp, at);
+      }
+    }
+  };
+#pragma unroll
+  for (int k = 0; k < NS - 1; ++k) request(t_begin + k, ring0 + k * kSlot);
+  wait_steps<F>(min(NS - 1, t_end - t_begin));   // everything older has landed
+  lds_barrier();
+
+  // ---- RMSNorm of the tokens, in place (see the quantizer); the waves are dealt to the tokens
+  if constexpr (NORM) {
+    double* sums = reinterpret_cast<double*>(lds + L.sums);
+    // token wave >> shift, shared by `of` waves of which this is the rank-th
+    const int shift = M == 1 ? 3 : (M == 2 ? 2 : (M <= 4 ? 1 : 0)), of = 1 << shift;
+    const int m = wave >> shift, rank = wave & (of - 1), pieces = m < M ? K >> 3 : 0;
+    uint8_t* row = lds + L.x + m * K * 2;
+    double part[4] = {0.0, 0.0, 0.0, 0.0};
+    for (int p = rank * 64 + lane; p < pieces; p += of * 64) {
+      const v4u a = *reinterpret_cast<const v4u*>(row + p * 16);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const double lo = (double)__uint_as_float(a[e] << 16), hi = (double)__uint_as_float(a[e] & 0xffff0000u);
+        part[e] = __builtin_fma(lo, lo, part[e]);
+        part[e] = __builtin_fma(hi, hi, part[e]);
+      }
+    }
+    const double ss = wave_sum((part[0] + part[1]) + (part[2] + part[3]));
+    if (lane == 0) sums[wave] = ss;
+    lds_barrier();
+    double tot = 0.0;
+    for (int w = 0; w < of; ++w) tot += sums[m * of + w];
+    const float r = rms_scale(tot, K, eps);
+    for (int p = rank * 64 + lane; p < pieces; p += of * 64) {
+      v4u* at = reinterpret_cast<v4u*>(row + p * 16);
+      const v4u gm = *reinterpret_cast<const v4u*>(lds + L.gamma + p * 16);
+      v4u a = *at;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) a[e] = rms_apply(a[e], gm[e], r);
+      *at = a;
+    }
+    lds_barrier();
+  }
+
+  // ---- quantization: two lanes per block of 32 (a pair is always both inside or both outside)
+  const int halves = K >> 4;
+  for (int m = 0, h = tid; ; h += 64 * kTokenWaves) {
+    while (h >= halves && m < M) {   // on to the next token
+      h -= halves;
+      ++m;
+    }
+    if (m >= M) break;
+    const int b = h >> 1, half = h & 1;
+    const int seg = b < s4.nblk ? 0 : (b < s4.nblk + s6.nblk ? 1 : 2);
+    const int j = b - sel3(seg, 0, s4.nblk, s4.nblk + s6.nblk);
+    const int fmt = sel3(seg, kFmtE2M1, kFmtE3M2, kFmtE4M3), bytes = sel3(seg, 16, 24, 32);
+    uint8_t* q = lds + sel3(seg, L.q0 + m * s4.nblk * 16, L.q1 + m * s6.nblk * 24, L.q2 + m * s8.nblk * 32) + j * bytes;
+    uint8_t* sf = lds + sel3(seg, L.sx0, L.sx1, L.sx2) + (j >> 2) * (4 * kTokenRows) + m * 4 + (j & 3);
+    const v4u i0 = *reinterpret_cast<const v4u*>(lds + L.idx + h * 32), i1 = *reinterpret_cast<const v4u*>(lds + L.idx + h * 32 + 16);
+    int at[16];   // an entry outside [0, K) reads channel K - 1
+#pragma unroll
+    for (int e = 0; e < 16; ++e) {
+      const unsigned w = e < 8 ? i0[e >> 1] : i1[(e - 8) >> 1];
+      at[e] = L.x + m * K * 2 + (int)min((e & 1) ? w >> 16 : w & 0xffffu, (unsigned)(K - 1)) * 2;
+    }
+    float f[16];
+#pragma unroll
+    for (int e = 0; e < 16; ++e) f[e] = __uint_as_float((unsigned)*reinterpret_cast<const uint16_t*>(lds + at[e]) << 16);
+    quantize_half(f, fmt, half, LdsHalf{q, sf, half});
+  }
+  lds_barrier();
+
+  // ---- the K loop
+  v4f acc[F];
+#pragma unroll
+  for (int f = 0; f < F; ++f) acc[f] = v4f{0.f, 0.f, 0.f, 0.f};
+  const int mc = min(i, M - 1);   // tokens past M: the last one again, never stored
+  int t = t_begin, slot = 0;
+  auto run = [&](auto fmt_c, const DecodeSeg& s, int codes, int sfx, int sfw, int t_first, int t_next) __attribute__((always_inline)) {
+    constexpr int FMT = decltype(fmt_c)::value;
+    const uint8_t* row = lds + codes + mc * (s.nblk * Frag<FMT>::kBytes);
+    for (const int last = min(t_next, t_end); t < last; ++t) {
+      request(t + NS - 1, ring0 + (unsigned)(slot == 0 ? NS - 1 : slot - 1) * kSlot);
+      wait_steps<F>(min(NS - 1, t_end - 1 - t));
+      const uint8_t* sl = ring + slot * kSlot;
+      slot = slot == NS - 1 ? 0 : slot + 1;
+      const int q = t - t_first, left = s.nblk - 4 * q;
+      v4i w[F];
+      int s_w[F], s_x = lds[sfx + q * (4 * kTokenRows) + mc * 4 + g];
+#pragma unroll
+      for (int f = 0; f < F; ++f) {
+        s_w[f] = lds[sfw + q * (PB * 16) + sw_off[f]];
+        w[f] = *reinterpret_cast<const v4i*>(sl + 1024 * f + i * 64 + (g ^ ((i >> 2) & 3)) * 16);
+      }
+      v8i x8;
+      if constexpr (FMT == kFmtE2M1) {
+        const v4i a = *reinterpret_cast<const v4i*>(row + q * 64 + g * 16);
+        x8 = v8i{a[0], a[1], a[2], a[3], 0, 0, 0, 0};
+      } else if constexpr (FMT == kFmtE3M2) {
+        const v2i* p = reinterpret_cast<const v2i*>(row + q * 96 + g * 24);
+        const v2i a = p[0], b = p[1], e = p[2];
+        x8 = v8i{a[0], a[1], b[0], b[1], e[0], e[1], 0, 0};
+      } else {
+        const v4i a = *reinterpret_cast<const v4i*>(row + q * 128 + g * 16);
+        const v4i b = *reinterpret_cast<const v4i*>(row + q * 128 + 64 + g * 16);
+        x8 = v8i{a[0], a[1], a[2], a[3], b[0], b[1], b[2], b[3]};
+      }
+      if (left < 4) {   // wave-uniform: the segment's last, partial step; what lies past its end is zero
+        const bool ok = g < left, lo_ok = FMT == kFmtE4M3 ? (g >> 1) < left : ok, hi_ok = FMT == kFmtE4M3 ? 2 + (g >> 1) < left : ok;
+        s_x = ok ? s_x : 127;
+#pragma unroll
+        for (int f = 0; f < F; ++f) {
+          s_w[f] = ok ? s_w[f] : 127;
+#pragma unroll
+          for (int e = 0; e < 4; ++e) w[f][e] = ok ? w[f][e] : 0;
+        }
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          x8[e] = lo_ok ? x8[e] : 0;
+          x8[4 + e] = hi_ok ? x8[4 + e] : 0;
+        }
+      }
+      // the weights are in registers before a later request may fill this slot again
+      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+#pragma unroll
+      for (int f = 0; f < F; ++f)
+        acc[f] = decode_mfma<FMT>(v8i{w[f][0], w[f][1], w[f][2], w[f][3], 0, 0, 0, 0}, x8, acc[f], s_w[f], s_x);
+    }
+  };
+  run(std::integral_constant<int, kFmtE2M1>{}, s4, L.q0, L.sx0, L.sw0, 0, t6);
+  run(std::integral_constant<int, kFmtE3M2>{}, s6, L.q1, L.sx1, L.sw1, t6, t8);
+  run(std::integral_constant<int, kFmtE4M3>{}, s8, L.q2, L.sx2, L.sw2, t8, total);
+
+  // ---- sum the four waves' partial tiles, in the rings' place
+  lds_barrier();
+  float* partial = reinterpret_cast<float*>(lds);
+#pragma unroll
+  for (int f = 0; f < F; ++f)
+    if (wave < 4) *reinterpret_cast<v4f*>(partial + ((wave * F + f) * 64 + lane) * 4) = acc[f];
+  __syncthreads();
+  if (wave >= F || i >= M) return;
+  const int f = wave;
+  v4f sum = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+  for (int w = 0; w < 4; ++w) sum += *reinterpret_cast<const v4f*>(partial + ((w * F + f) * 64 + lane) * 4);
+  if constexpr (WT) {
+#pragma unroll
+    for (int v = 0; v < 4; ++v) store1(d, ep, i, feature(f, 4 * g + v), sum[v]);
+  } else {
+    store4(d, ep, i, feature(f, 4 * g), sum);
+  }
+}
+
 static int round_up_1k(int v) { return (v + 1023) & ~1023; }
 
 // The decode kernel takes whole 128-wide steps in every segment and an LDS image of at most 76 KB.
@@ -917,6 +1202,59 @@ hipError_t launch_mixed_gemm(const uint8_t* an, const uint8_t* bn, const uint8_t
   hipLaunchKernelGGL(mixed_gemm_direct_kernel, grid, dim3(256), 0, stream, an, bn, as_, bs, ao, bo, sfan, sfbn, sfas, sfbs,
                      sfao, sfbo, M, N, KN, KS, KO, ep, static_cast<uint16_t*>(d));
   return hipGetLastError();
+}
+
+// Quantization and GEMM of a few tokens in one launch, where that is the faster way; *taken says whether it was.
+// Every workgroup repeats the quantization, so it pays up to 16384 channels in all (M = 4, K = 4096 7.7 -> 7.5 us, M = 8
+// 7.8 -> 10.0; M = 2, K = 8192 13.0 -> 11.0), with RMSNorm up to 10240 (M = 2, K = 4096 8.4 -> 8.0, K = 5120 10.7 -> 10.3;
+// M = 4, K = 4096 8.4 -> 9.7), for rows of at most 8192 (M = 1, K = 14336: 13.7 -> 14.0), and in one round of workgroups.
+hipError_t launch_token_linear(const void* x, const int16_t* idx, const void* gamma, float eps, const uint8_t* bn, const uint8_t* bs,
+                               const uint8_t* bo, const uint8_t* sfbn, const uint8_t* sfbs, const uint8_t* sfbo, int M, int N,
+                               int KN, int KS, int KO, bool w_tiled, Epilogue ep, void* d, hipStream_t stream, bool* taken) {
+  *taken = false;
+  const int K = KN + KS + KO;
+  // (row-major weight codes are addressed with 32-bit offsets; the copies of gamma want it aligned)
+  const int widest = KN > KS ? (KN > KO ? KN : KO) : (KS > KO ? KS : KO);
+  if (M < 1 || M > kTokenRows || K == 0 || K > 8192 || M * K > (gamma ? 10240 : 16384) || N == 0 || (!w_tiled && (size_t)N * (size_t)(widest / 2) >= ((size_t)1 << 32)) ||
+      (reinterpret_cast<uintptr_t>(gamma) & 15u))
+    return hipSuccess;
+  // tile-major weights exist only for shapes the 256x256 kernel takes
+  if (w_tiled && (N % 256 != 0 || !mixed_gemm_256_supported(256, N, KN, KS, KO))) return hipErrorInvalidValue;
+  DeviceLimits lim;
+  if (hipError_t e = device_limits(&lim); e != hipSuccess) return e;
+  const DecodeSeg d4 = {nullptr, bn, nullptr, sfbn, KN / 32, ceil_div(KN, 128)};
+  const DecodeSeg d6 = {nullptr, bs, nullptr, sfbs, KS / 32, ceil_div(KS, 128)};
+  const DecodeSeg d8 = {nullptr, bo, nullptr, sfbo, KO / 32, ceil_div(KO, 128)};
+  const int total = d4.steps + d6.steps + d8.steps;
+  const int f = ceil_div(N, 16) <= lim.cus ? 1 : (ceil_div(N, 32) <= lim.cus ? 2 : 4);
+  const int grid = w_tiled ? ceil_div(N, 16 * f) : ceil_div(N, 128) * (8 / f);
+  if (grid > lim.cus) return hipSuccess;
+  TokenLds L;
+  int pos = 4 * 1024 * (f == 1 ? kTokenSlots<1> : (f == 2 ? 2 * kTokenSlots<2> : 4 * kTokenSlots<4>));
+  auto take = [&](int bytes) { const int at = pos; pos += round_up_1k(bytes); return at; };
+  L.x = take(M * K * 2); L.idx = take(K * 2); L.gamma = gamma ? take(K * 2) : 0;
+  L.sw0 = take(d4.steps * f * 64); L.sw1 = take(d6.steps * f * 64); L.sw2 = take(d8.steps * f * 64);
+  L.sx0 = take(d4.steps * 4 * kTokenRows); L.sx1 = take(d6.steps * 4 * kTokenRows); L.sx2 = take(d8.steps * 4 * kTokenRows);
+  L.q0 = take(M * d4.nblk * 16); L.q1 = take(M * d6.nblk * 24); L.q2 = take(M * d8.nblk * 32);
+  L.sums = take(128);   // also what a last, partial step reads past the last codes (and drops)
+  L.total = pos;
+  if (pos > lim.lds_bytes) return hipSuccess;
+  auto launch = [&](auto f_c, auto wt_c, auto norm_c) {
+    const auto kernel = mixed_gemm_token_kernel<decltype(f_c)::value, decltype(wt_c)::value, decltype(norm_c)::value>;
+    if (hipError_t e = allow_dynamic_lds(reinterpret_cast<const void*>(kernel), lim.lds_bytes); e != hipSuccess) return e;
+    hipLaunchKernelGGL(kernel, dim3(grid), dim3(64 * kTokenWaves), (size_t)L.total, stream, static_cast<const uint8_t*>(x),
+                       static_cast<const uint8_t*>(gamma), reinterpret_cast<const uint8_t*>(idx), eps, K, d4, d6, d8, M, N,
+                       (total + 3) / 4, L, ep, static_cast<uint16_t*>(d));
+    return hipGetLastError();
+  };
+  auto with_norm = [&](auto f_c, auto wt_c) {
+    return gamma ? launch(f_c, wt_c, std::true_type{}) : launch(f_c, wt_c, std::false_type{});
+  };
+  auto with_layout = [&](auto f_c) { return w_tiled ? with_norm(f_c, std::true_type{}) : with_norm(f_c, std::false_type{}); };
+  *taken = true;
+  if (f == 1) return with_layout(std::integral_constant<int, 1>{});
+  if (f == 2) return with_layout(std::integral_constant<int, 2>{});
+  return with_layout(std::integral_constant<int, 4>{});
 }
 
 }  // namespace mg

@@ -237,3 +237,33 @@ def test_layer_stores_the_real_features_and_adds_the_bias(linear, m, n, bias):
     torch.cuda.synchronize()
     assert got.shape == (m, 1, n) and got.is_contiguous()
     assert torch.equal(got[:, 0], want)
+
+
+# A few tokens in one launch against the quantizer and the GEMM one after the other: the same bits.  One to eight tokens on
+# both sides of the largest count it takes, with and without RMSNorm, all three feature group counts, ragged features, one
+# and several rounds of blocks per lane, a last step of 1 to 3 blocks, an index with entries out of range.
+@pytest.mark.parametrize("n,split", [(256, (128, 128, 128)), (4096, (2560, 1408, 128)), (8192, (1024, 480, 160)), (14336, (2560, 1408, 128)),
+                                     (1000, (416, 224, 96)), (40, (32, 32, 32)), (520, (5120, 2560, 512)), (264, (0, 1056, 0)),
+                                     (300, (96, 0, 672))])
+@pytest.mark.parametrize("norm", [False, True])
+@pytest.mark.parametrize("tiled", [False, True])
+def test_few_tokens_in_one_launch(linear, n, split, norm, tiled):
+    from mixedgemm_amd import abi
+    k = sum(split)
+    if tiled and not (n % 256 == 0 and abi.weights_tileable(n, *split)):
+        pytest.skip("shape cannot be tiled")
+    g = torch.Generator().manual_seed(n + k)
+    idx = torch.randperm(k, generator=g).to(torch.int16)
+    idx[3], idx[k - 1] = -5, 32767   # read as channel K - 1 on both ways
+    idx, w = idx.to(DEV), H.make_weights(n, k, 7).to(DEV)
+    b = abi.reorder_quantize_w(w, idx, *split)
+    if tiled:
+        b = abi.tile_weights(*b[:3]) + tuple(b[3:])
+    gamma = (1 + 0.1 * torch.randn(k, generator=g)).to(torch.bfloat16).to(DEV) if norm else None
+    for m in (1, 2, 3, 5, 8):
+        x = H.make_activations(m, k, 100 + m, n_out=max(1, k // 32)).to(DEV)
+        got = abi.fused_linear(x, idx, *b, *split, w_tiled=tiled, norm_weight=gamma, eps=1e-5)
+        a = abi.rmsnorm_reorder_quantize_x(x, gamma, 1e-5, idx, *split) if norm else abi.reorder_quantize_x(x, idx, *split)
+        want = abi.matmul(a[0], b[0], a[1], b[1], a[2], b[2], a[3], b[3], a[4], b[4], a[5], b[5], w_tiled=tiled)
+        torch.cuda.synchronize()
+        assert torch.equal(got, want), m
