@@ -42,7 +42,7 @@ constexpr int kStartSkew = 8000;          // see the kernel: largest start delay
 // tile is 256 x 256; TM = 1: 256 x 128), 64 * TM accumulator registers, so that two waves fit a SIMD's register file
 // and one wave's copy and fragment-read instructions issue while the other's MFMA runs.  A stage's copies are dealt to
 // the waves so that the workgroup moves every byte exactly once: per wave 2 weight blocks, 2 / 3 / 4 token copies
-// (E2M1 / E3M2 / E4M3) and a quarter of a scale atom pair (a 4-byte copy).
+// (E2M1 / E3M2 / E4M3; TM = 1: 1 / 2 / 2) and a quarter of a scale atom pair (a 4-byte copy).
 constexpr int kWaves = 8;
 constexpr int kWCopies = 2;                            // weight copy blocks per wave and stage
 constexpr int kXSlots = 4;                             // token copy slots per wave and stage (E4M3 uses them all)
@@ -103,6 +103,10 @@ template <> struct Fmt<kFmtNone> { static constexpr int seg = 3, row_bytes = 0, 
 template <> struct Fmt<kFmtE2M1> { static constexpr int seg = 0, row_bytes = 64, x_copies = 4; typedef v4i xfrag; };
 template <> struct Fmt<kFmtE3M2> { static constexpr int seg = 1, row_bytes = 96, x_copies = 6; typedef v6i xfrag; };
 template <> struct Fmt<kFmtE4M3> { static constexpr int seg = 2, row_bytes = 128, x_copies = 8; typedef v8i xfrag; };
+
+// Token copies per wave and stage.  Half tiles (TM = 1): half of them, E3M2's 1.5 rounded up.
+template <int FMT, int TM>
+constexpr int kTokenCopies = TM == 2 ? Fmt<FMT>::x_copies / 2 : (Fmt<FMT>::x_copies / 2 + 1) / 2;
 
 // ---------------------------------------------------------------------------------------------
 // Copies.  One instruction moves 64 x 16 B to 1 KB of consecutive LDS.  Weights and E2M1 / E4M3
@@ -198,10 +202,19 @@ struct LaneOffsets {
   // Byte offset, from the tile's first token row, that this lane reads in token copy kx of a stage of
   // segment sg (row pitch lda).  E2M1: rows 2 * wave + kx + 16 * pr, 16-byte piece lane % 4; E4M3: rows
   // 4 * (wave % 4) + kx + 16 * pr; E3M2: piece c % 6 of row wave + 8 * (c / 6), c = 64 * kx + lane.
+  // Half tiles (TM = 1) have rows 0 ... 127: a block holds rows 2 j and 2 j + 1, + 16 u + 32 t (u < 2, t < 4) at quad
+  // 8 u + 4 (t / 2) + 2 (row % 2) + t % 2, which keeps the 16 rows of a fragment read on different banks; E2M1 block
+  // j = wave, E4M3 block j = 2 * (wave % 4) + kx.
+  template <int TM>
   __device__ __forceinline__ unsigned xoff(int sg, int kx, unsigned lda) const {
     if (sg == 1) {
       const int c = 64 * kx + lane;
       return (unsigned)min(8 * (c / 6) + wave, last_row) * lda + (c % 6) * 16;
+    }
+    if constexpr (TM == 1) {
+      const int k = lane >> 2, row = ((k >> 1) & 1) + 16 * (k >> 3) + 32 * (2 * ((k >> 2) & 1) + (k & 1));
+      const int j = sg == 0 ? wave : 2 * (wave & 3) + kx;
+      return (unsigned)min(row + 2 * j, last_row) * lda + (lane & 3) * 16;
     }
     const int first = sg == 0 ? 2 * wave : 4 * (wave & 3);
     return (unsigned)min(prow + first + kx, last_row) * lda + (lane & 3) * 16;
@@ -245,6 +258,7 @@ struct StageBases {
 };
 
 // Copies of a stage whose format is only known at run time (segment boundaries, prologue).
+template <int TM>
 struct GenericCopy {
   StageBases b;
   unsigned buf;   // LDS byte offset of the target stage buffer
@@ -254,7 +268,7 @@ struct GenericCopy {
       : b(plan, q, c), buf(c.lds_base + (q % kBuffers) * kStage) {}
 
   __device__ __forceinline__ int count() const {
-    return b.seg < 0 ? 0 : kWCopies + (b.seg == 0 ? kXSlots / 2 : (b.seg == 1 ? 3 * kXSlots / 4 : kXSlots)) + 1;
+    return b.seg < 0 ? 0 : kWCopies + (b.seg == 0 ? kTokenCopies<kFmtE2M1, TM> : (b.seg == 1 ? kTokenCopies<kFmtE3M2, TM> : kTokenCopies<kFmtE4M3, TM>)) + 1;
   }
 
   template <int K>
@@ -266,11 +280,13 @@ struct GenericCopy {
     } else if constexpr (K < kCopySlots - 1) {
       constexpr int kx = K - kWCopies;
       if (b.seg == 0) {
-        if constexpr (kx < kXSlots / 2) copy16(b.x, lo.xoff(0, kx, b.lda), buf + kXOff + (wave * (kXSlots / 2) + kx) * kBlk);
+        constexpr int n = kTokenCopies<kFmtE2M1, TM>;
+        if constexpr (kx < n) copy16(b.x, lo.xoff<TM>(0, kx, b.lda), buf + kXOff + (wave * n + kx) * kBlk);
       } else if (b.seg == 1) {
-        if constexpr (kx < 3 * kXSlots / 4) copy16(b.x, lo.xoff(1, kx, b.lda), buf + kXOff + wave * kBlk6 + kx * 1024);
+        if constexpr (kx < kTokenCopies<kFmtE3M2, TM>) copy16(b.x, lo.xoff<TM>(1, kx, b.lda), buf + kXOff + wave * kBlk6 + kx * 1024);
       } else {
-        copy16(b.x, lo.xoff(2, kx, b.lda), buf + kXOff + (wave * kXSlots + kx) * kBlk);
+        constexpr int n = kTokenCopies<kFmtE4M3, TM>;
+        if constexpr (kx < n) copy16(b.x, lo.xoff<TM>(2, kx, b.lda), buf + kXOff + (wave * n + kx) * kBlk);
       }
     } else {
       copy4(b.s, pick3u(b.seg, lo.s0, lo.s1, lo.s2), buf + kSOff + wave * 256);
@@ -278,8 +294,8 @@ struct GenericCopy {
   }
 };
 
-template <int K0, int K1>
-__device__ __forceinline__ void issue_range(const GenericCopy& cp, const LaneOffsets& lo, int wave) {
+template <int K0, int K1, int TM>
+__device__ __forceinline__ void issue_range(const GenericCopy<TM>& cp, const LaneOffsets& lo, int wave) {
   if constexpr (K0 < K1) {
     cp.template issue<K0>(lo, wave);
     issue_range<K0 + 1, K1>(cp, lo, wave);
@@ -290,14 +306,15 @@ __device__ __forceinline__ void issue_range(const GenericCopy& cp, const LaneOff
 // per-lane offsets (one register per copy, the row step of the copy folded in) fixed.
 // WT: weights in tile-major order -- one per-lane offset (16 * lane) and immediates for all four
 // weight copies; vw[] is then unused.
-template <int FMT, bool WT>
+template <int FMT, bool WT, int TM>
 struct LeanCopy {
   static constexpr int WC = kWCopies;
-  static constexpr int NX = Fmt<FMT>::x_copies / 2;
+  static constexpr int NX = kTokenCopies<FMT, TM>;
   // token copies, rows clamped to the last readable one.  E2M1, E3M2: one offset per copy.  E4M3, of which
   // there are few stages: the first copy's offset, and in its bits 0-2 how many of the three row steps that
-  // follow stay inside the readable rows.  (These offsets are multiples of 16.)
-  static constexpr int NV = FMT == kFmtE4M3 ? 1 : (FMT == kFmtE3M2 ? 3 : NX);
+  // follow stay inside the readable rows (whole tiles).  (These offsets are multiples of 16.)
+  static constexpr bool kSteps = FMT == kFmtE4M3 && TM == 2;
+  static constexpr int NV = kSteps ? 1 : NX;
   const uint8_t *w, *x, *s;        // bases of the stage being copied
   unsigned lds_w, lds_x, lds_s;    // LDS offsets of the wave's first weight / token block and scale atom pair in buffer 0
   unsigned lda;
@@ -316,15 +333,12 @@ struct LeanCopy {
       for (int k = 0; k < WC; ++k) vw[k] = lo.woff(k, b.ldb);
     }
     lda = __builtin_amdgcn_readfirstlane(b.lda);
-    if constexpr (FMT == kFmtE4M3) {
+    if constexpr (kSteps) {
       const int row0 = lo.prow + 4 * (c.wave & 3);
-      vx[0] = lo.xoff(2, 0, b.lda) | (unsigned)min(max(lo.last_row - row0, 0), NX - 1);
-    } else if constexpr (FMT == kFmtE3M2) {
-#pragma unroll
-      for (int t = 0; t < 3; ++t) vx[t] = lo.xoff(1, t, b.lda);
+      vx[0] = lo.xoff<TM>(2, 0, b.lda) | (unsigned)min(max(lo.last_row - row0, 0), NX - 1);
     } else {
 #pragma unroll
-      for (int k = 0; k < NX; ++k) vx[k] = lo.xoff(0, k, b.lda);
+      for (int k = 0; k < NX; ++k) vx[k] = lo.xoff<TM>(sg, k, b.lda);
     }
     vs = sg == 0 ? lo.s0 : (sg == 1 ? lo.s1 : lo.s2);
     lds_w = __builtin_amdgcn_readfirstlane(c.lds_base + kWOff + c.wave * WC * kBlk);
@@ -350,7 +364,7 @@ struct LeanCopy {
     } else if constexpr (K < WC + NX) {
       constexpr int kx = K - WC;
       if constexpr (FMT == kFmtE3M2) copy16i<kx * 1024>(x, vx[kx], lds_x + boff);
-      else if constexpr (FMT == kFmtE4M3)
+      else if constexpr (kSteps)
         copy16i<kx * kBlk>(x, (vx[0] & ~15u) + min((unsigned)kx, vx[0] & 7u) * lda, lds_x + boff);
       else copy16i<kx * kBlk>(x, vx[kx], lds_x + boff);
     } else if constexpr (K == kCopySlots - 1) {
@@ -359,8 +373,8 @@ struct LeanCopy {
   }
 };
 
-template <bool WT>
-struct LeanCopy<kFmtNone, WT> {
+template <bool WT, int TM>
+struct LeanCopy<kFmtNone, WT, TM> {
   __device__ __forceinline__ void init(const Plan&, int, const LaneOffsets&, const Ctx&) {}
   __device__ __forceinline__ void advance() {}
   static constexpr int count() { return 0; }
@@ -368,8 +382,8 @@ struct LeanCopy<kFmtNone, WT> {
   __device__ __forceinline__ void issue(unsigned) const {}
 };
 
-template <int K0, int K1, int FMT, bool WT>
-__device__ __forceinline__ void issue_range(const LeanCopy<FMT, WT>& lc, unsigned boff) {
+template <int K0, int K1, int FMT, bool WT, int TM>
+__device__ __forceinline__ void issue_range(const LeanCopy<FMT, WT, TM>& lc, unsigned boff) {
   if constexpr (K0 < K1) {
     lc.template issue<K0>(boff);
     issue_range<K0 + 1, K1>(lc, boff);
@@ -438,7 +452,8 @@ struct TokenPtrs {
       // row 32*rt + i: block i%8, row slot 4*rt + i/8, fragment 2h+g of 24 bytes
       x = lds + kXOff + (i & 7) * kBlk6 + (4 * TM * c.wm + (i >> 3)) * 96 + g * 24;
     } else {
-      x = lds + kXOff + (i & 15) * kBlk + (i >> 4) * 512 + c.wm * (64 * TM) + g * 16;
+      if constexpr (TM == 2) x = lds + kXOff + (i & 15) * kBlk + (i >> 4) * 512 + c.wm * 128 + g * 16;
+      else x = lds + kXOff + ((i & 15) >> 1) * kBlk + (i >> 4) * 512 + (c.wm >> 1) * 256 + (i & 1) * 128 + (c.wm & 1) * 64 + g * 16;
     }
   }
 };
@@ -473,7 +488,7 @@ struct FragReader {
         const v2i a = p[0], b = p[1], c = p[2];
         f.x[t] = v6i{a[0], a[1], b[0], b[1], c[0], c[1]};
       } else {
-        const uint8_t* p = px + H * 16 * kBlk + t * 64;
+        const uint8_t* p = px + H * (8 * TM) * kBlk + t * 64;
         const v4i a = *reinterpret_cast<const v4i*>(p);        // K [16g, 16g+16) of the half
         const v4i b = *reinterpret_cast<const v4i*>(p + 32);   // K [32+16g, 32+16g+16)
         f.x[t] = __builtin_shufflevector(a, b, 0, 1, 2, 3, 4, 5, 6, 7);
@@ -534,9 +549,9 @@ __device__ __forceinline__ void mfma_one(v16f& acc, v4i w, const typename Fmt<FM
 }
 
 // first copy slot >= K that a stage of format FMT has (the token slots past the format's copies are empty)
-template <int FMT>
+template <int FMT, int TM>
 constexpr int next_slot(int k) {
-  return (k >= kWCopies + Fmt<FMT>::x_copies / 2 && k < kCopySlots - 1) ? kCopySlots - 1 : k;
+  return (k >= kWCopies + kTokenCopies<FMT, TM> && k < kCopySlots - 1) ? kCopySlots - 1 : k;
 }
 
 // The 4 * TM MFMAs of one K half.  Between them: the fragment reads of `rd` (for the next half: one after
@@ -547,7 +562,7 @@ constexpr int next_slot(int k) {
 // otherwise slots of the run-time plan `gc`.
 template <int FMT, int H, bool LEAN, int CF, int M0, int K0, int K1, class Reader, bool WT, int TM>
 __device__ __forceinline__ void mfma_half(v16f (&acc)[4][TM], const HalfFrags<FMT, TM>& f, const Scales<TM>& sc, const Reader& rd,
-                                          const LeanCopy<CF, WT>& lc, bool on, unsigned boff, const GenericCopy& gc,
+                                          const LeanCopy<CF, WT, TM>& lc, bool on, unsigned boff, const GenericCopy<TM>& gc,
                                           const LaneOffsets& lo, int wave) {
   if constexpr (M0 < 4 * TM) {
     constexpr int tn = M0 / TM, tm = M0 % TM;
@@ -556,7 +571,7 @@ __device__ __forceinline__ void mfma_half(v16f (&acc)[4][TM], const HalfFrags<FM
     // without one: what is read last is needed first afterwards, and its LDS latency would stand between two halves.
     constexpr int RP = (Reader::kReads + 4 * TM - 3) / (4 * TM - 2);
     read_some<M0 * RP, (M0 + 1) * RP>(rd);
-    constexpr int KS = LEAN ? (CF == kFmtNone ? K1 : next_slot<CF>(K0)) : K0;
+    constexpr int KS = LEAN ? (CF == kFmtNone ? K1 : next_slot<CF, TM>(K0)) : K0;
     // a copy slot after every second MFMA where a wave has twice as many MFMAs per half as copy slots, else after every one
     constexpr bool kEvery = 4 * TM <= kCopySlots - kSplit;
     if constexpr ((kEvery || (M0 & 1) == 1) && KS < K1) {
@@ -598,8 +613,8 @@ struct Ring {
 // !LEAN: both from the run-time plan `gc`.  next_on: there is a stage q+1.
 template <int FMT, int FR, bool LEAN, int CL, int CE, int MID, bool WT, int TM>
 __device__ __forceinline__ void stage_body(v16f (&acc)[4][TM], HalfFrags<FMT, TM>& a, HalfFrags<FR, TM>& a_next, Scales<TM>& sc,
-                                           const LeanCopy<CL, WT>& lcl, bool late_on, LeanCopy<CE, WT>& lce, bool early_on,
-                                           GenericCopy& gc, const LaneOffsets& lo, const Plan& plan, int q,
+                                           const LeanCopy<CL, WT, TM>& lcl, bool late_on, LeanCopy<CE, WT, TM>& lce, bool early_on,
+                                           GenericCopy<TM>& gc, const LaneOffsets& lo, const Plan& plan, int q,
                                            bool next_on, const Ring& ring, const WeightPtrs& wp, const TokenPtrs<FMT, TM>& xp,
                                            const TokenPtrs<FR, TM>& xpn, const Ctx& c) {
   HalfFrags<FMT, TM> b;
@@ -612,7 +627,7 @@ __device__ __forceinline__ void stage_body(v16f (&acc)[4][TM], HalfFrags<FMT, TM
   __builtin_amdgcn_sched_barrier(0);
   wait_lds_reads();
   if constexpr (LEAN) {
-    if (late_on) wait_copies_but_imm<LeanCopy<CL, WT>::count()>();
+    if (late_on) wait_copies_but_imm<LeanCopy<CL, WT, TM>::count()>();
     else wait_copies_but_imm<0>();
   } else {
     wait_copies_but(gc.count());
@@ -622,7 +637,7 @@ __device__ __forceinline__ void stage_body(v16f (&acc)[4][TM], HalfFrags<FMT, TM
   if constexpr (LEAN) {
     if constexpr (MID == 1) lce.advance();   // MID == 2: lce was set up for its segment's first stage before the K loop
   } else {
-    gc = GenericCopy(plan, q + 3, c);
+    gc = GenericCopy<TM>(plan, q + 3, c);
   }
   // second half; reads the first half and the scales of stage q+1; the first copies of stage q+3
   // go to the buffer this stage just released
@@ -652,7 +667,7 @@ __device__ __forceinline__ void stage_body(v16f (&acc)[4][TM], HalfFrags<FMT, TM
 // stages that copy across a segment boundary take the run-time path.
 template <int FMT, int F1, int FR1, bool REGULAR, int NLAST = 0, bool WT, int TM>
 __device__ __forceinline__ void run_segment(v16f (&acc)[4][TM], HalfFrags<FMT, TM>& a, Scales<TM>& sc, HalfFrags<FR1, TM>& a_next,
-                                            LeanCopy<FMT, WT>& lc, LeanCopy<F1, WT>& lcn, GenericCopy& gc, const LaneOffsets& lo,
+                                            LeanCopy<FMT, WT, TM>& lc, LeanCopy<F1, WT, TM>& lcn, GenericCopy<TM>& gc, const LaneOffsets& lo,
                                             const Plan& plan, int n, int n1, int q0, const WeightPtrs& wp,
                                             const uint8_t* lds, const Ctx& c) {
   const TokenPtrs<FMT, TM> xp(lds, c);
@@ -710,7 +725,7 @@ __device__ __forceinline__ void run_segment(v16f (&acc)[4][TM], HalfFrags<FMT, T
                                                 xp, xp, c);
         ring.rotate();
       }
-      gc = GenericCopy(plan, q0 + ql + 2, c);
+      gc = GenericCopy<TM>(plan, q0 + ql + 2, c);
     }
     for (; ql + 1 < n; ++ql) {
       stage_body<FMT, FMT, false, FMT, FMT, 0>(acc, a, unused, sc, lc, true, lc, true, gc, lo, plan, q0 + ql, true, ring, wp, xp,
@@ -931,9 +946,11 @@ __device__ __forceinline__ int stages_of(const Plan& p) {
 // SEGS: which activation segments the plan has, bit 0 E2M1, bit 1 E3M2, bit 2 E4M3 -- the
 // prefetched fragments pass from a segment to the next one that exists, and their types are fixed here.
 // TM: token tiles of 32 per wave.  2: the workgroup's tile is 256 features x 256 tokens.  1: 256 x 128, for
-// problems with fewer than 256 whole tiles (every CU still gets a workgroup): same copies (the lanes of token
-// rows 128 ... 255 read the last row again, which costs the address unit next to nothing), same LDS image,
-// half the MFMAs per stage, a copy slot after every MFMA instead of every second one.
+// problems with fewer than 256 whole tiles (every CU still gets a workgroup): the same weight copies, 1 / 2 / 2 token
+// copies per wave and stage instead of 2 / 3 / 4, half the MFMAs per stage, a copy slot after every MFMA instead of every
+// second one.  (With a whole tile's token copies, whose lanes past row 127 read the last row again, the address unit was
+// busy 87 % of M = 2048, N = 4096, K = 14336; without them 79.9 -> 78.2 us for that layer call, 62.9 -> 61.4 for M = 1024,
+// N = 4096, K = 4096 through the module.)
 // NLAST: see run_segment (the launcher picks the instance from the plan).
 // Computes one tile of 256 features x 128 * TM tokens: feature tile tile_n, token tile tile_m (of 128 * TM rows).
 template <bool REGULAR, bool REM, bool WT, int SEGS, int TM, int NLAST>
@@ -976,8 +993,8 @@ __device__ __forceinline__ void compute_tile(const Plan& plan, int tile_n, int t
   constexpr int FA = nth_format(SEGS, 0), FB = nth_format(SEGS, 1), FC = nth_format(SEGS, 2);   // the segments that exist, in order
   static_assert(FA != kFmtNone, "a plan has at least one segment");
   const int nA = stages_of<FA>(plan), nB = stages_of<FB>(plan), nC = stages_of<FC>(plan);
-  GenericCopy gc;
-  LeanCopy<FA, WT> la;
+  GenericCopy<TM> gc;
+  LeanCopy<FA, WT, TM> la;
   int in_flight;   // copies that may stay in flight while stage 0 is awaited
   if constexpr (REGULAR) {
     la.init(plan, 0, lo, c);
@@ -994,18 +1011,18 @@ __device__ __forceinline__ void compute_tile(const Plan& plan, int tile_n, int t
       in_flight += kSplit;
     }
   } else {
-    const GenericCopy g0(plan, 0, c);
+    const GenericCopy<TM> g0(plan, 0, c);
     issue_range<0, kCopySlots>(g0, lo, c.wave);
-    const GenericCopy g1(plan, 1, c);
+    const GenericCopy<TM> g1(plan, 1, c);
     issue_range<0, kCopySlots>(g1, lo, c.wave);
-    gc = GenericCopy(plan, 2, c);
+    gc = GenericCopy<TM>(plan, 2, c);
     issue_range<0, kSplit>(gc, lo, c.wave);
     in_flight = g1.count() + (gc.b.seg < 0 ? 0 : kSplit);
   }
   // the copy state of the later segments, while the first copies are in flight: set up between two halves of a
   // stage it would hold up the MFMAs for several hundred cycles
-  LeanCopy<FB, WT> lb;
-  LeanCopy<FC, WT> lcc;
+  LeanCopy<FB, WT, TM> lb;
+  LeanCopy<FC, WT, TM> lcc;
   if constexpr (REGULAR) {
     lb.init(plan, nA, lo, c);          // (no-ops for segments that do not exist)
     lcc.init(plan, nA + nB, lo, c);
@@ -1055,7 +1072,7 @@ __device__ __forceinline__ void compute_tile(const Plan& plan, int tile_n, int t
     wait_lds_reads();
     shift_scales(sc, sw, sx, c.lane);
   }
-  LeanCopy<kFmtNone, WT> l0;
+  LeanCopy<kFmtNone, WT, TM> l0;
   // NLAST goes to the plan's last segment and the one before it (see run_segment)
   if constexpr (FB == kFmtNone) {
     run_segment<FA, kFmtNone, FA, REGULAR>(acc, fa, sc, da, la, l0, gc, lo, plan, nA, 0, 0, wp, lds, c);
