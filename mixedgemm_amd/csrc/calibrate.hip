@@ -9,7 +9,8 @@
 // rows --, folds its row lanes through LDS and writes one row of partial maxima (the bf16 bit patterns with
 // the sign cleared order like the values).  The strips are few (kStrips), so that pass 2 can afford to fold
 // them in every workgroup: each folds the partials of all K channels into unique 32-bit keys
-// (absmax bits << 16 | channel) in LDS and ranks 16 channels against all keys.
+// (absmax bits << 16 | channel) in LDS and ranks 16 channels against all keys.  Wide layers sort and search instead, in
+// two launches (see kRankMost).
 #include "mg_common.h"
 
 namespace mg {
@@ -127,10 +128,87 @@ rank_channels_kernel(const uint16_t* __restrict__ partial, int nstrips, int K, i
   }
 }
 
+// Wide layers (K > kRankMost): K^2 compares, and K/16 workgroups that each fold all partial maxima, are most of the time.
+// So two launches instead: each workgroup of the first folds 256 channels and sorts their keys (every key ranked against
+// the 256), one of the second holds all sorted chunks in LDS and ranks 128 keys by binary search in every chunk, four
+// threads per key with a quarter of the chunks each: 9 K / 256 steps per key instead of K.  Bound by latency and the
+// LDS reads of the searches.  Calibration as a whole, M = 300: K = 6144 11.1 -> 12.3 us (not taken), 8192
+// 13.0 -> 12.1, 14336 27.4 -> 15.0, 18944 40.6 -> 17.0, 32736 131 -> 23; M = 4096, K = 14336 46 -> 34.
+constexpr int kRankMost = 7168;
+constexpr int kChunk = 256, kSearchKeys = 128, kSearchThreads = 4 * kSearchKeys;
+
+__global__ void __launch_bounds__(kChunk)
+sort_chunks_kernel(const uint16_t* __restrict__ partial, int nstrips, int K, unsigned* __restrict__ sorted) {
+  __shared__ __align__(16) unsigned keys[kChunk];
+  const int c0 = blockIdx.x * kChunk, t = threadIdx.x;
+  keys[t] = 0xffffffffu;   // past the last channel: larger than every key
+  __syncthreads();
+  if (t < kChunk / 8 && c0 + t * 8 < K) {   // K is a multiple of 32: a lane's 8 channels are all inside or all outside
+    const uint16_t* p = partial + c0 + t * 8;
+    v4u m = *reinterpret_cast<const v4u*>(p);
+#pragma unroll
+    for (int s = 1; s < kStrips; ++s) absmax_fold(m, *reinterpret_cast<const v4u*>(p + (size_t)min(s, nstrips - 1) * K));
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      keys[t * 8 + 2 * j] = (m[j] << 16) | (unsigned)(c0 + t * 8 + 2 * j);
+      keys[t * 8 + 2 * j + 1] = (m[j] & 0xffff0000u) | (unsigned)(c0 + t * 8 + 2 * j + 1);
+    }
+  }
+  __syncthreads();
+  const unsigned mine = keys[t];
+  int rank = 0;
+#pragma unroll 8
+  for (int j = 0; j < kChunk; j += 4) {
+    const v4u q = *reinterpret_cast<const v4u*>(keys + j);
+#pragma unroll
+    for (int e = 0; e < 4; ++e) rank += q[e] < mine ? 1 : 0;
+  }
+  // (the keys past the last channel are equal: they keep their places at the end)
+  sorted[c0 + (c0 + t < K ? rank : t)] = mine;
+}
+
+__global__ void __launch_bounds__(kSearchThreads)
+rank_sorted_kernel(const unsigned* __restrict__ sorted, int K, int16_t* __restrict__ idx) {
+  extern __shared__ __align__(16) unsigned chunks[];   // all chunks, then four counts per key
+  const int nchunks = ceil_div(K, kChunk), total = nchunks * kChunk;
+  int* counts = reinterpret_cast<int*>(chunks + total);
+#pragma unroll 4
+  for (int j = threadIdx.x * 4; j < total; j += kSearchThreads * 4)
+    *reinterpret_cast<v4u*>(chunks + j) = *reinterpret_cast<const v4u*>(sorted + j);
+  __syncthreads();
+  const int key = threadIdx.x % kSearchKeys, part = threadIdx.x / kSearchKeys;
+  const unsigned mine = chunks[blockIdx.x * kSearchKeys + key];
+  int rank = 0;
+  // several chunks at once: the steps of one search wait for each other
+  constexpr int kAtOnce = 4;
+  for (int c = part; c < nchunks; c += 4 * kAtOnce) {
+    const unsigned* at[kAtOnce];
+    int pos[kAtOnce];
+#pragma unroll
+    for (int u = 0; u < kAtOnce; ++u) {
+      at[u] = chunks + min(c + 4 * u, nchunks - 1) * kChunk;
+      pos[u] = 0;
+    }
+#pragma unroll
+    for (int step = kChunk / 2; step >= 1; step >>= 1)
+#pragma unroll
+      for (int u = 0; u < kAtOnce; ++u) pos[u] += at[u][pos[u] + step - 1] < mine ? step : 0;
+#pragma unroll
+    for (int u = 0; u < kAtOnce; ++u)
+      if (c + 4 * u < nchunks) rank += pos[u] + (at[u][pos[u]] < mine ? 1 : 0);
+  }
+  counts[part * kSearchKeys + key] = rank;
+  __syncthreads();
+  if (threadIdx.x < kSearchKeys && mine != 0xffffffffu)
+    idx[counts[key] + counts[kSearchKeys + key] + counts[2 * kSearchKeys + key] + counts[3 * kSearchKeys + key]] = (int16_t)(mine & 0xffffu);
+}
+
 }  // namespace
 
-// kStrips rows of partial maxima (K x 2 B each, a multiple of 16)
-size_t calibrate_workspace_bytes(int K) { return (size_t)kStrips * K * sizeof(uint16_t); }
+// kStrips rows of partial maxima (K x 2 B each, a multiple of 16), and the sorted chunks of a wide layer
+size_t calibrate_workspace_bytes(int K) {
+  return (size_t)kStrips * K * sizeof(uint16_t) + (K > kRankMost ? (size_t)ceil_div(K, kChunk) * kChunk * sizeof(unsigned) : 0);
+}
 
 hipError_t launch_calibrate(const void* x, int rows, int K, int16_t* idx, void* workspace, hipStream_t stream) {
   uint16_t* partial = static_cast<uint16_t*>(workspace);
@@ -140,6 +218,19 @@ hipError_t launch_calibrate(const void* x, int rows, int K, int16_t* idx, void* 
                      static_cast<const uint16_t*>(x), rows, K, partial);
   hipError_t e = hipGetLastError();
   if (e != hipSuccess) return e;
+  if (K > kRankMost) {
+    unsigned* sorted = reinterpret_cast<unsigned*>(partial + (size_t)kStrips * K);
+    const int nchunks = ceil_div(K, kChunk);
+    constexpr int kMostLds = 32768 * (int)sizeof(unsigned) + kSearchThreads * (int)sizeof(int);
+    e = allow_dynamic_lds(reinterpret_cast<const void*>(rank_sorted_kernel), kMostLds);
+    if (e != hipSuccess) return e;
+    hipLaunchKernelGGL(sort_chunks_kernel, dim3(nchunks), dim3(kChunk), 0, stream, partial, nstrips, K, sorted);
+    e = hipGetLastError();
+    if (e != hipSuccess) return e;
+    hipLaunchKernelGGL(rank_sorted_kernel, dim3(nchunks * (kChunk / kSearchKeys)), dim3(kSearchThreads),
+                       (size_t)nchunks * kChunk * sizeof(unsigned) + kSearchThreads * sizeof(int), stream, sorted, K, idx);
+    return hipGetLastError();
+  }
   const size_t lds = (size_t)(K + kRankSlices * kRankChannels) * sizeof(unsigned);
   e = allow_dynamic_lds(reinterpret_cast<const void*>(rank_channels_kernel),
                         (32768 + kRankSlices * kRankChannels) * (int)sizeof(unsigned));

@@ -495,6 +495,19 @@ def test_calibrate_reorder_index_matches_oracle(abi, m, k):
     np.testing.assert_array_equal(idx.cpu().numpy(), mo.calibrate_reorder_index(H.bf16_bits(x)))
 
 
+# Wide layers sort chunks of 256 keys and search them: the last width of the other way and the first of this one, a last
+# chunk of 32 and of 224 channels, the widest; few distinct values (ties across chunks), zeros and infinities.
+@pytest.mark.parametrize("k", [7168, 7200, 8160, 14336, 32736])
+def test_calibration_of_wide_layers(abi, k):
+    g = torch.Generator().manual_seed(k)
+    x = torch.randn(3, k, generator=g).to(torch.bfloat16)
+    x[:, ::5] = 0
+    x[1, ::7] = 2.0
+    x[2, 3::1001] = float("inf")
+    idx = abi.calibrate_reorder_index(x.cuda())
+    np.testing.assert_array_equal(idx.cpu().numpy(), mo.calibrate_reorder_index(H.bf16_bits(x)))
+
+
 # ------------------------------------------------------------------ committed golden vectors
 import glob as _glob
 import os as _os
