@@ -31,7 +31,7 @@ DRIVER_PATH = os.path.join(EXT_DIR, "abi_driver")
 BENCH_LIB_PATH = os.path.join(LIB_DIR, "libmixedgemm_bench.so")
 OBJ_DIR = os.path.join(EXT_DIR, "obj")
 
-HIP_SOURCES = ["abi.hip", "reorder_quant.hip", "mixed_gemm.hip", "mixed_gemm_256.hip", "calibrate.hip"]
+HIP_SOURCES = ["abi.hip", "reorder_quant.hip", "mixed_gemm.hip", "mixed_gemm_256.hip", "mixed_gemm_tile.hip", "calibrate.hip"]
 BENCH_SOURCES = ["bench_kernels.hip"]
 HIP_HEADERS = ["mg_common.h", "quantize.h", os.path.join(ROOT, "include", "mixedgemm_abi.h")]
 
@@ -54,7 +54,7 @@ def _stale(target: str, deps: list[str]) -> bool:
 # is still to fill must never be moved or spilled, so these kernels must compile without scratch memory.  (The
 # whole-tile GEMM is listed for speed: a spill inside its K loop costs more than anything else there.)
 NO_SCRATCH_KERNELS = ("mixed_gemm_decode_kernel", "reorder_quant_dma_kernel", "mixed_gemm_256_kernel",
-                      "mixed_gemm_256_tail_kernel")
+                      "mixed_gemm_256_tail_kernel", "mixed_gemm_tile_kernel")
 
 
 # ... except the quantizer for K > 20480 (run-time workgroup size, up to 1024 lanes of 128 registers): it spills, and

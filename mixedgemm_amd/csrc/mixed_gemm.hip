@@ -19,6 +19,8 @@
 //                [64+16g, 64+16g+16) in registers 4-7 (two 16-byte pieces);
 // and, for every format, the E8M0 scale of block g of row i in the byte of the
 // scale register that op_sel selects.
+#include <math.h>
+
 #include <type_traits>
 
 #include "mg_common.h"
@@ -33,37 +35,6 @@ struct Frag;
 template <> struct Frag<kFmtE2M1> { static constexpr int kBytes = 16; };
 template <> struct Frag<kFmtE3M2> { static constexpr int kBytes = 24; };
 template <> struct Frag<kFmtE4M3> { static constexpr int kBytes = 32; };
-
-// Load one lane's fragment of a 128-wide K step into the low dwords of v8i.
-// `step` points at the start of the K step in the lane's row; blocks at or past
-// `blocks_left` (counted from the start of the step) read as zero.
-template <int FMT>
-__device__ __forceinline__ v8i load_frag(const uint8_t* __restrict__ step, int g, int blocks_left, bool row_ok) {
-  v8i f = {0, 0, 0, 0, 0, 0, 0, 0};
-  if constexpr (FMT == kFmtE2M1) {
-    if (row_ok && g < blocks_left) {
-      const v4i t = *reinterpret_cast<const v4i*>(step + g * 16);
-      f[0] = t[0]; f[1] = t[1]; f[2] = t[2]; f[3] = t[3];
-    }
-  } else if constexpr (FMT == kFmtE3M2) {
-    if (row_ok && g < blocks_left) {
-      const v2i* q = reinterpret_cast<const v2i*>(step + g * 24);
-      const v2i t0 = q[0], t1 = q[1], t2 = q[2];
-      f[0] = t0[0]; f[1] = t0[1]; f[2] = t1[0]; f[3] = t1[1]; f[4] = t2[0]; f[5] = t2[1];
-    }
-  } else {
-    // two 16-element pieces: K [16g, 16g+16) in block g/2 and K [64+16g, ...) in block 2 + g/2
-    if (row_ok && (g >> 1) < blocks_left) {
-      const v4i t = *reinterpret_cast<const v4i*>(step + g * 16);
-      f[0] = t[0]; f[1] = t[1]; f[2] = t[2]; f[3] = t[3];
-    }
-    if (row_ok && 2 + (g >> 1) < blocks_left) {
-      const v4i t = *reinterpret_cast<const v4i*>(step + 64 + g * 16);
-      f[4] = t[0]; f[5] = t[1]; f[6] = t[2]; f[7] = t[3];
-    }
-  }
-  return f;
-}
 
 // Up to four consecutive features n ... n + 3 of token m, rounded to bf16, with the epilogue's bias.
 __device__ __forceinline__ void store4(uint16_t* __restrict__ d, const Epilogue& ep, int m, int n, v4f sum) {
@@ -90,67 +61,6 @@ __device__ __forceinline__ void store1(uint16_t* __restrict__ d, const Epilogue&
   if (ep.bias) h = add_bf16(h, ep.bias[n]);
   d[(size_t)m * ep.n_out + n] = h;
 }
-
-// One K segment, operands read straight from global memory.  Wave tile:
-// 16 tokens x (16*NT) output features.
-template <int FMT, int NT>
-__device__ __forceinline__ void segment_direct(v4f (&acc)[NT], const uint8_t* __restrict__ a, const uint8_t* __restrict__ sfa,
-                                               const uint8_t* __restrict__ b, const uint8_t* __restrict__ sfb, int kseg,
-                                               int m, bool m_ok, int n_base, int N, int lane) {
-  const int nblk = kseg >> 5;
-  if (nblk == 0) return;
-  const int katoms = (kseg + 127) >> 7;
-  const int g = lane >> 4, i = lane & 15;
-  const size_t lda = (size_t)nblk * Frag<FMT>::kBytes;
-  const size_t ldb = (size_t)nblk * 16;
-  for (int q = 0; q < katoms; ++q) {
-    const int kb = 4 * q + g;
-    const int left = nblk - 4 * q;
-    const bool k_ok = kb < nblk;
-    const v8i xa = load_frag<FMT>(a + (size_t)m * lda + (size_t)q * 4 * Frag<FMT>::kBytes, g, left, m_ok);
-    const int sx = (k_ok && m_ok) ? (int)sfa[sf_offset(m, kb, katoms)] : 127;
-#pragma unroll
-    for (int t = 0; t < NT; ++t) {
-      const int n = n_base + 16 * t + i;
-      const bool b_ok = k_ok && n < N;
-      const v8i wb = load_frag<kFmtE2M1>(b + (size_t)n * ldb + (size_t)q * 64, g, left, n < N);
-      const int sw = b_ok ? (int)sfb[sf_offset(n, kb, katoms)] : 127;
-      acc[t] = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(wb, xa, acc[t], kFmtE2M1, FMT, 0, sw, 0, sx);
-    }
-  }
-}
-
-// Generic kernel for any M, N and 32-granular segments: no LDS, every wave
-// fetches its own fragments.  Workgroup = 4 waves = 64 tokens x 64 features.
-__global__ void __launch_bounds__(256)
-mixed_gemm_direct_kernel(const uint8_t* __restrict__ an, const uint8_t* __restrict__ bn, const uint8_t* __restrict__ as_,
-                         const uint8_t* __restrict__ bs, const uint8_t* __restrict__ ao, const uint8_t* __restrict__ bo,
-                         const uint8_t* __restrict__ sfan, const uint8_t* __restrict__ sfbn,
-                         const uint8_t* __restrict__ sfas, const uint8_t* __restrict__ sfbs,
-                         const uint8_t* __restrict__ sfao, const uint8_t* __restrict__ sfbo, int M, int N, int KN, int KS,
-                         int KO, Epilogue ep, uint16_t* __restrict__ d) {
-  constexpr int NT = 4;
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  const int m = blockIdx.y * 64 + wave * 16 + (lane & 15);
-  const int n_base = blockIdx.x * 64;
-  const bool m_ok = m < M;
-  v4f acc[NT];
-#pragma unroll
-  for (int t = 0; t < NT; ++t) acc[t] = v4f{0.f, 0.f, 0.f, 0.f};
-
-  segment_direct<kFmtE2M1, NT>(acc, an, sfan, bn, sfbn, KN, m, m_ok, n_base, N, lane);
-  segment_direct<kFmtE3M2, NT>(acc, as_, sfas, bs, sfbs, KS, m, m_ok, n_base, N, lane);
-  segment_direct<kFmtE4M3, NT>(acc, ao, sfao, bo, sfbo, KO, m, m_ok, n_base, N, lane);
-
-  // result tile is D^T: lane holds token m = lane%16, features 4*(lane/16) + v
-  if (!m_ok) return;
-#pragma unroll
-  for (int t = 0; t < NT; ++t) {
-    const int n = n_base + 16 * t + 4 * (lane >> 4);
-    store4(d, ep, m, n, acc[t]);
-  }
-}
-
 
 // ---------------------------------------------------------------------------
 // Skinny kernel: few tokens (decode, small batches), any 32-granular K, wherever the rules below do not find another kernel
@@ -1183,6 +1093,15 @@ hipError_t launch_mixed_gemm_256(const uint8_t* an, const uint8_t* bn, const uin
                                  int m_store, int a_rows, int N, int KN, int KS, int KO, bool w_tiled, Epilogue ep,
                                  void* d, hipStream_t stream);
 
+// tiles of 64 or 128 features x 64 or 128 tokens (mixed_gemm_tile.hip)
+struct TilePlanChoice { int tf, tt; double us; };
+TilePlanChoice mixed_gemm_tile_plan(int M, int N, int KN, int KS, int KO, int cus);
+hipError_t launch_mixed_gemm_tile(const uint8_t* an, const uint8_t* bn, const uint8_t* as_, const uint8_t* bs,
+                                  const uint8_t* ao, const uint8_t* bo, const uint8_t* sfan, const uint8_t* sfbn,
+                                  const uint8_t* sfas, const uint8_t* sfbs, const uint8_t* sfao, const uint8_t* sfbo,
+                                  int m_store, int a_rows, int N, int KN, int KS, int KO, bool w_tiled, const TilePlanChoice& choice,
+                                  Epilogue ep, void* d, hipStream_t stream);
+
 // Rough launch time of the whole-tile kernel in microseconds, only to choose between the kernels for fewer than 256
 // tokens (measured on MI355X, 256 CUs).  It runs such problems as 256 x 128 tiles when that is at most one round: ~2.5 us
 // plus, per 128-wide stage, ~0.42 us on tile-major weights with at most half of the CUs busy and ~0.45 us with more; on
@@ -1196,6 +1115,18 @@ static double pipelined_us(int M, int N, int stages, int cus, bool w_tiled) {
   const int whole = ceil_div(M, 256) * ceil_div(N, 256), halves = ceil_div(M, 128) * ceil_div(N, 256);
   if (whole <= cus / 2) return stages * (w_tiled ? (halves <= cus / 2 ? 0.42 : 0.45) : 0.487 + 0.0027 * halves) + 2.5;
   return (double)ceil_div(whole, cus) * (stages * 0.95 + 3.0);
+}
+
+// The same on tile-major weights for 256 tokens and more, fitted to 148 measured calls (rms error 7 %): half tiles (at most cus / 2
+// whole ones) or rounds of whole tiles, of which a last one on at most half of the CUs counts 0.62; microseconds per stage, per
+// MB of results, and what the blocks past whole stages cost.
+static double whole_tiles_us(int M, int N, int stages, bool rest, bool three_segments, int cus) {
+  const int whole = ceil_div(M, 256) * ceil_div(N, 256), halves = ceil_div(M, 128) * ceil_div(N, 256);
+  const double mb = 2e-6 * M * N;
+  if (whole <= cus / 2) return 3.46 + stages * (0.354 + 0.104 * fmin(1.0, (double)halves / cus)) + 0.19 * mb + (rest ? 2.2 : 0.0);
+  const int full = whole / cus, left = whole % cus;
+  const double rounds = full + (left == 0 ? 0.0 : (left <= cus / 2 && full > 0 && three_segments ? 0.62 : 1.0));
+  return fmax(1.44 + rounds * (stages * 0.748 - 9.1 + (rest ? 2.1 : 0.0)) + 0.68 * mb, rounds * stages * 0.6);
 }
 
 // a_rows: token rows for which the activation codes and scales are readable (>= M)
@@ -1213,33 +1144,33 @@ hipError_t launch_mixed_gemm(const uint8_t* an, const uint8_t* bn, const uint8_t
   const DecodeSeg d6 = {as_, bs, sfas, sfbs, KS / 32, (KS + 127) / 128};
   const DecodeSeg d8 = {ao, bo, sfao, sfbo, KO / 32, (KO + 127) / 128};
   const bool whole_tiles = mixed_gemm_256_supported(m_pad, N, KN, KS, KO);
-  SkinnyPlan skinny = {0, 0, 0.0};   // fewer than 256 tokens: the kernel that runs if whole tiles are not faster
-  bool pipelined = whole_tiles;
-  if (M < 256 && KN + KS + KO > 0) {
-    DeviceLimits lim;
-    if (hipError_t e = device_limits(&lim); e != hipSuccess) return e;
+  DeviceLimits lim;
+  if (hipError_t e = device_limits(&lim); e != hipSuccess) return e;
+  const int steps = d4.steps + d6.steps + d8.steps;
+  // (the skinny kernel addresses a segment's row-major weight codes with 32-bit offsets)
+  const int widest = KN > KS ? (KN > KO ? KN : KO) : (KS > KO ? KS : KO);
+  const bool few = M < 256 && KN + KS + KO > 0, skinny_ok = few && (w_tiled || (size_t)N * (size_t)(widest / 2) < ((size_t)1 << 32));
+  if (few) {
     DecodeLds L;
     if (const int f = decode_plan(d4, d6, d8, M, N, w_tiled, lim.cus, &L))
       return launch_decode(d4, d6, d8, M, N, w_tiled, f, L, ep, static_cast<uint16_t*>(d), stream);
-    const int steps = d4.steps + d6.steps + d8.steps;
-    skinny = skinny_plan(M, N, steps, lim.cus, w_tiled);
-    pipelined = whole_tiles && pipelined_us(M, N, steps, lim.cus, w_tiled) < skinny.us;
   }
+  // Small tiles where they are estimated to be the fastest by a margin (the estimates of both sides are off by 10 %), and for
+  // what no other kernel takes.  Both weight layouts go the same way: the estimates compared are those on tile-major weights.
+  const TilePlanChoice tile = mixed_gemm_tile_plan(M, N, KN, KS, KO, lim.cus);
+  const double others = few ? (whole_tiles ? fmin(pipelined_us(M, N, steps, lim.cus, true), skinny_plan(M, N, steps, lim.cus, true).us)
+                                           : skinny_plan(M, N, steps, lim.cus, true).us)
+                            : whole_tiles_us(M, N, steps, (KN | KS | KO) % 128 != 0, KN > 0 && KS > 0 && KO > 0, lim.cus);
+  if ((M > 16 || !few) && ((!whole_tiles && !skinny_ok) || tile.us < 0.95 * others))
+    return launch_mixed_gemm_tile(an, bn, as_, bs, ao, bo, sfan, sfbn, sfas, sfbs, sfao, sfbo, M, a_rows, N, KN, KS, KO, w_tiled, tile,
+                                  ep, d, stream);
+  const SkinnyPlan skinny = skinny_ok ? skinny_plan(M, N, steps, lim.cus, w_tiled) : SkinnyPlan{0, 0, 0.0};
   // whole 256-row tiles; the last one does not write rows past M and reads no activation row past
   // a_rows (lanes that would are pointed at the last readable row)
-  if (pipelined)
+  if (whole_tiles && (!skinny_ok || pipelined_us(M, N, steps, lim.cus, w_tiled) < skinny.us))
     return launch_mixed_gemm_256(an, bn, as_, bs, ao, bo, sfan, sfbn, sfas, sfbs, sfao, sfbo, M, a_rows, N, KN, KS, KO,
                                  w_tiled, ep, d, stream);
-  // (the skinny kernel addresses a segment's row-major weight codes with 32-bit offsets)
-  const int widest = KN > KS ? (KN > KO ? KN : KO) : (KS > KO ? KS : KO);
-  if (skinny.g != 0 && (w_tiled || (size_t)N * (size_t)(widest / 2) < ((size_t)1 << 32)))
-    return launch_skinny(d4, d6, d8, M, N, w_tiled, skinny, ep, static_cast<uint16_t*>(d), stream);
-  // what is left (256 tokens or more with N not a multiple of 8, or with a segment that is not whole 128-wide
-  // stages next to an empty one): the direct kernel
-  dim3 grid(ceil_div(N, 64), ceil_div(M, 64));
-  hipLaunchKernelGGL(mixed_gemm_direct_kernel, grid, dim3(256), 0, stream, an, bn, as_, bs, ao, bo, sfan, sfbn, sfas, sfbs,
-                     sfao, sfbo, M, N, KN, KS, KO, ep, static_cast<uint16_t*>(d));
-  return hipGetLastError();
+  return launch_skinny(d4, d6, d8, M, N, w_tiled, skinny, ep, static_cast<uint16_t*>(d), stream);
 }
 
 // Quantization and GEMM of a few tokens in one launch, where that is the faster way; *taken says whether it was.

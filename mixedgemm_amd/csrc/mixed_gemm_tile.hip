@@ -1,0 +1,729 @@
+// Mixed block-scaled GEMM on small workgroup tiles, 64 or 128 features x 64 or 128 tokens, for problems with too few tiles of
+// 256 x 256 or 256 x 128 to fill the chip: waves that only copy and waves that only multiply.
+//
+// What bounded such launches on 256 x 128 tiles was not the memory (a tile alone on the chip took 0.30 us per stage of 128 K elements):
+// a global -> LDS copy holds the wave that issues it for ~64 cycles (its addresses go out one per cycle; a CU accepts one
+// from each of its SIMDs at a time, 1 KB per 16 cycles in all, whatever rows it is put together from, as long as the lines are in
+// the L2), so that waves that copy and multiply in turn leave the matrix cores idle.  Here four waves, one per SIMD, issue
+// all copies, eight waves, two per SIMD, read fragments and multiply, and one barrier hands over WS stages at a time, each of them the
+// work of 8 / WS of the math waves (fragments are read once per 2 x 2 tiles of 32 x 32 rather than once per 1 x 2).
+// What bounds it now (stamps of an instrumented build): LDS bandwidth, ~16 cycles per KB copied and 4.4 per KB read: 64 x 64 tiles, K =
+// 4096, one per CU: 270 cycles per stage, of which 64 are MFMAs' (150 without copies); a launch of them takes 1.2 us until the
+// first stages have landed, 2.7 us for 20 E2M1 and 1.3 for 12 later stages, 1.2 us to add the partial sums and store.
+// Tile-major / row-major weights, of two or three layers in turn, before (skinny kernel or 256 x 128 tiles) -> now, us:
+//   M = 256, N = 4096, K = 4096: 16.4 / 19.6 -> 8.5 / 8.5;   K = 14336: 45.6 / 59.9 -> 19.7 / 22.3
+//   M = 512, N = 4096, K = 4096: 16.6 / 19.6 -> 10.5 / 11.8;  N = 1024, K = 8192: 27.6 / 34.8 -> 11.6 / 13.2
+//   M = 64, N = 14336, K = 4096: 16.4 / 16.8 -> 8.8 / 9.3;   M = 128: 16.9 / 20.3 -> 10.3 / 12.3
+// Tiles of 256 x 128 with the same division of work were level with the mixed waves of the 256 x 256 kernel (M = 2048, N =
+// 4096, K = 12288: 57.6 against 56.3 us: 15 % fewer cycles at a clock as much lower; the chip is at its power limit there), tiles of
+// 64 and 128 x 32 slower than 64 x 64 at every shape tried.
+#include "mg_common.h"
+
+#include <type_traits>
+
+namespace mg {
+
+namespace {
+
+constexpr int kCopyWaves = 4, kMathWaves = 8, kTileWaves = kCopyWaves + kMathWaves;
+constexpr int kRingBytes = 156 * 1024;   // LDS for the ring of batches
+
+typedef int v6i __attribute__((ext_vector_type(6)));
+
+struct TileSeg {
+  const uint8_t *a, *b, *sfa, *sfb;
+  int blk;    // 32-element blocks
+  int whole;  // whole 128-wide stages
+};
+
+struct TilePlan {
+  TileSeg s4, s6, s8;
+  int total;      // whole stages of all segments
+  int N;          // weight rows
+  int m_store;    // token rows that are stored
+  int a_rows;     // token rows that may be read
+  // Workgroup -> tile (see tile_at): a rectangle of `div` x div2 tiles per XCD, 2^xlog rectangles along the features, or
+  // (xlog < 0) tiles in feature-major order, div = token tiles, div2 = tiles per XCD or 0
+  int xlog, div, div2;
+  unsigned magic;   // 2^32 / div, rounded up (div > 1)
+};
+
+template <int FMT> struct Form;
+template <> struct Form<kFmtE2M1> { static constexpr int row = 64; typedef v4i frag; };
+template <> struct Form<kFmtE3M2> { static constexpr int row = 96; typedef v6i frag; };
+template <> struct Form<kFmtE4M3> { static constexpr int row = 128; typedef v8i frag; };
+
+__device__ __forceinline__ const uint8_t* uniform(const uint8_t* p) {
+  const uint64_t v = reinterpret_cast<uint64_t>(p);
+  const uint32_t lo = (uint32_t)__builtin_amdgcn_readfirstlane((uint32_t)v), hi = (uint32_t)__builtin_amdgcn_readfirstlane((uint32_t)(v >> 32));
+  return reinterpret_cast<const uint8_t*>(((uint64_t)hi << 32) | lo);
+}
+
+// global[base + voff(lane)] -> LDS[lds_off + 16 * lane]; base and lds_off wave-uniform
+__device__ __forceinline__ void copy_at(const uint8_t* base, unsigned voff, unsigned lds_off) {
+  base = uniform(base);
+  lds_off = __builtin_amdgcn_readfirstlane(lds_off);
+  asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1"
+               : : "v"(voff), "s"(base), "s"(lds_off) : "memory", "m0");
+}
+// the same with a 64-bit address per lane
+__device__ __forceinline__ void copy_lane(const uint8_t* p, unsigned lds_off) {
+  lds_off = __builtin_amdgcn_readfirstlane(lds_off);
+  asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off" : : "v"(p), "s"(lds_off) : "memory", "m0");
+}
+
+template <int N>
+__device__ __forceinline__ void wait_vm() { asm volatile("s_waitcnt vmcnt(%0)" : : "n"(N) : "memory"); }
+__device__ __forceinline__ void workgroup_barrier() { asm volatile("s_barrier" ::: "memory"); }
+// the barriers of the last YOUNGER + 2 batches, with nothing more to issue; the last PARTIAL of them count for nothing
+template <int YOUNGER, int PER, int PARTIAL>
+__device__ __forceinline__ void drain() {
+  wait_vm<(YOUNGER > PARTIAL ? YOUNGER - PARTIAL : 0) * PER>();
+  workgroup_barrier();
+  if constexpr (YOUNGER > 0) drain<YOUNGER - 1, PER, PARTIAL>();
+  else workgroup_barrier();
+}
+// s_waitcnt lgkmcnt(0) that the compiler's own counting sees
+__device__ __forceinline__ void wait_lds() { __builtin_amdgcn_s_waitcnt(0xC07F); }
+
+// Geometry of an instance.  TF x TT: the workgroup's tile; WT: tile-major weights; a batch of WS stages per barrier, each the
+// work of 8 / WS math waves (WF along the features).
+template <int TF_, int TT_, int WF_, int WS_, bool WT_>
+struct Geo {
+  static constexpr int TF = TF_, TT = TT_, WF = WF_, WS = WS_;
+  static constexpr bool WT = WT_;
+  static constexpr int WM = kMathWaves / WF / WS;                          // math waves along tokens
+  static constexpr int TN = TF / 32 / WF, TM = TT / 32 / WM;               // a wave's 32 x 32 tiles
+  // a stage in LDS: 1 KB of scales (32 pieces of the features, 32 of the tokens), weights, tokens
+  static constexpr int kW = 1024, kX = kW + TF * 64;
+  static constexpr int kSlot = kX + TT * 128;
+  static constexpr int kBatch = WS * kSlot;
+  static constexpr int NB = kRingBytes / kBatch < 8 ? kRingBytes / kBatch : 8;   // batches in the ring
+  // the partial sums on their way out: per stage of a batch, fp32 rows of tokens
+  static constexpr int kPitch = TF * 4 + 16, kPart = TT * kPitch;
+  static_assert(WS > 1 && TN == 2 && (TM == 1 || TM == 2) && NB >= 3 && WS * kPart <= NB * kBatch, "tile geometry");
+};
+
+template <class G>
+struct TileCtx {
+  int lane, n0, m0;        // row-major: first feature of the tile
+  int tile, j0;            // tile-major: 256-feature tile and first copy block in it
+  int last_col, last_row;  // last readable weight / token row, from the tile's first
+};
+
+// Which weight row is row i of a 32-row fragment T of the tile.  Row-major: rows 32 T + i.  Tile-major (copy block b, row e of
+// its 16): block 4 (T / 2) + i % 4, row i / 4 + 8 (T % 2), so that four consecutive fragment rows are four consecutive features.
+template <class G>
+__device__ __forceinline__ int weight_row(const TileCtx<G>& c, int T, int i) {
+  if constexpr (G::WT) return c.tile * 256 + c.j0 + 4 * (T >> 1) + (i & 3) + 32 * (i >> 2) + 16 * (T & 1);
+  else return c.n0 + min(32 * T + i, c.last_col);
+}
+// Position in the tile's output row (features in ascending order) of fragment rows 8 vq + 4 g ... + 3.
+template <class G>
+__device__ __forceinline__ int out_position(int T, int vq, int g) {
+  if constexpr (G::WT) return (2 * (2 * vq + g) + (T & 1)) * (G::TF / 16) + 4 * (T >> 1);
+  else return 32 * T + 8 * vq + 4 * g;
+}
+
+// ---------------------------------------------------------------------------------------------
+// Copies of one whole stage, dealt to the four copy waves.  Weights and E2M1 tokens: 16 rows x 64 B per copy, the 16-byte
+// pieces of row r permuted by XOR with r / 4 (tile-major weights: with the block's number), E4M3: 8 rows x 128 B, permuted by XOR
+// with r / 2, E3M2: rows of 96 B one after the other, their pieces rotated by one in rows 8 ... 15 of every 16: the 16 rows that a
+// fragment read touches at a time lie on different banks (E3M2 rows as they are: 0.85 instead of 0.36 us per stage of 128 x 128).
+// Scales: the 16-byte pieces (rows c, c + 32, c + 64, c + 96 of an atom of 128 rows) that hold the tile's rows, one copy; on
+// tile-major weights in the order that makes the scales of a 32-row fragment 128 consecutive bytes.
+// ---------------------------------------------------------------------------------------------
+template <int FMT, class G>
+constexpr int kTokenCopiesAll = G::TT * Form<FMT>::row / 1024;
+// copies that every copy wave issues per whole batch, at least (a stage of a later segment has as many or more)
+template <class G>
+constexpr int kBatchCopies = G::WS * (G::TF / 64) + G::WS * kTokenCopiesAll<kFmtE2M1, G> / kCopyWaves + G::WS / kCopyWaves;
+
+template <int FMT, class G>
+struct StageCopy {
+  static constexpr int NW = G::TF / 64, NX = kTokenCopiesAll<FMT, G>, KX = (NX + kCopyWaves - 1) / kCopyWaves;
+  const uint8_t *w, *x;         // bases of the next stage
+  const uint8_t* sc;            // this lane's scale piece
+  unsigned vw[G::WT ? 1 : NW], vx[KX];
+  int wave;
+
+  // token copies come in fours, a last pair is dealt to waves 0, 1 and 2, 3 in turn
+  static_assert(NX % 2 == 0, "token copies in pairs");
+  __device__ __forceinline__ int block(int k) const { return (k + 1) * kCopyWaves <= NX ? wave + kCopyWaves * k : (wave & 1) + kCopyWaves * k; }
+
+  __device__ __forceinline__ void init(const TileCtx<G>& c, const TileSeg& s, int wave_) {
+    wave = wave_;
+    const int r = c.lane >> 2, p = (c.lane & 3) ^ ((c.lane >> 4) & 3);
+    if constexpr (G::WT) {
+      w = s.b + ((size_t)c.tile * s.whole * 16 + c.j0 + wave) * 1024;
+      vw[0] = (unsigned)(r * 64 + ((c.lane & 3) ^ wave) * 16);
+    } else {
+      w = s.b + (size_t)c.n0 * s.blk * 16;
+#pragma unroll
+      for (int k = 0; k < NW; ++k) vw[k] = (unsigned)min(16 * (wave + kCopyWaves * k) + r, c.last_col) * (unsigned)s.blk * 16u + p * 16;
+    }
+    const unsigned pitch = (unsigned)s.blk * (Form<FMT>::row / 4);
+    x = s.a + (size_t)c.m0 * pitch;
+#pragma unroll
+    for (int k = 0; k < KX; ++k) {
+      const int b = block(k);
+      if constexpr (FMT == kFmtE2M1) {
+        vx[k] = (unsigned)min(16 * b + r, c.last_row) * pitch + p * 16;
+      } else if constexpr (FMT == kFmtE3M2) {   // the pieces of rows 8 ... 15 of every 16 rotated by one
+        const int chunk = 64 * b + c.lane, row = chunk / 6, at = chunk % 6;
+        const int piece = (row & 8) ? (at == 0 ? 5 : at - 1) : at;
+        vx[k] = (unsigned)min(row, c.last_row) * pitch + piece * 16;
+      } else {
+        const int row = 8 * b + (c.lane >> 3);
+        vx[k] = (unsigned)min(row, c.last_row) * pitch + (((c.lane & 7) ^ ((row >> 1) & 7)) * 16);
+      }
+    }
+    const int katoms = (s.blk + 3) >> 2;
+    const int pl = c.lane & 31;
+    int atom, piece;   // of the features
+    if constexpr (G::WT) {
+      const int at = pl % (G::TF / 4), T = at >> 3;   // (64 features: 16 pieces, copied twice)
+      atom = c.tile * 2 + ((at >> 2) & 1);
+      piece = c.j0 + 4 * (T >> 1) + (at & 3) + 16 * (T & 1);
+    } else {
+      atom = c.n0 >> 7;
+      piece = pl;
+    }
+    const uint8_t* of_rows = s.sfa + (size_t)(c.m0 >> 7) * katoms * 512 + (c.lane & 31) * 16;
+    const uint8_t* of_features = s.sfb + (size_t)atom * katoms * 512 + piece * 16;
+    sc = c.lane < 32 ? of_features : of_rows;
+  }
+
+  // the next stage, t-th of all, into a slot.  What does not divide by the copy waves goes to other ones in every stage.
+  __device__ __forceinline__ void issue(int t, unsigned slot) {
+#pragma unroll
+    for (int k = 0; k < NW; ++k) {
+      if constexpr (G::WT) copy_at(w + k * (kCopyWaves * 1024), vw[0], slot + G::kW + 1024u * (wave + kCopyWaves * k));
+      else copy_at(w, vw[k], slot + G::kW + 1024u * (wave + kCopyWaves * k));
+    }
+#pragma unroll
+    for (int k = 0; k < KX; ++k)
+      if ((k + 1) * kCopyWaves <= NX || (wave >> 1) == (t & 1)) copy_at(x, vx[k], slot + G::kX + 1024u * block(k));
+    const int turn = 2 * (~t & 1) + ((t >> 1) & 1);   // every wave once in four stages
+    if (turn == wave) copy_lane(sc, slot);
+    w += G::WT ? 16384 : 64;
+    x += Form<FMT>::row;
+    sc += 512;
+  }
+};
+
+// ---------------------------------------------------------------------------------------------
+// Fragments of one 64-wide K half
+// ---------------------------------------------------------------------------------------------
+template <int FMT, class G>
+struct TileFrags {
+  v4i w[G::TN];
+  typename Form<FMT>::frag x[G::TM];
+};
+
+template <class G>
+struct ReadAt {   // per-lane LDS offsets inside a slot
+  int w, x4, x6, x8, sw, sx;
+  int xor4, xor8, xorw;
+  int p6a, p6b, h6a, h6b;   // E3M2: the lane's whole and half piece of K half 0, 1
+};
+
+__device__ __forceinline__ v8i widened(v4i v) { return __builtin_shufflevector(v, v, 0, 1, 2, 3, -1, -1, -1, -1); }
+__device__ __forceinline__ v8i widened(v6i v) { return __builtin_shufflevector(v, v, 0, 1, 2, 3, 4, 5, -1, -1); }
+__device__ __forceinline__ v8i widened(v8i v) { return v; }
+
+template <int FMT, int H, class G>
+__device__ __forceinline__ void read_half(TileFrags<FMT, G>& f, const uint8_t* slot, const ReadAt<G>& r, int g) {
+  const int piece = ((2 * H + g) ^ r.xor4) * 16, wpiece = G::WT ? ((2 * H + g) ^ r.xorw) * 16 : piece;
+#pragma unroll
+  for (int t = 0; t < G::TN; ++t) f.w[t] = *reinterpret_cast<const v4i*>(slot + r.w + t * (G::WT ? 512 : 2048) + wpiece);
+#pragma unroll
+  for (int t = 0; t < G::TM; ++t) {
+    if constexpr (FMT == kFmtE2M1) {
+      f.x[t] = *reinterpret_cast<const v4i*>(slot + r.x4 + t * 2048 + piece);
+    } else if constexpr (FMT == kFmtE3M2) {
+      // block 2H is piece 3H and the first half of piece 3H + 1, block 2H + 1 the other half and piece 3H + 2
+      const uint8_t* row = slot + r.x6 + t * 3072;
+      const v4i a = *reinterpret_cast<const v4i*>(row + (H ? r.p6b : r.p6a));
+      const v2i b = *reinterpret_cast<const v2i*>(row + (H ? r.h6b : r.h6a));
+      f.x[t] = g ? v6i{b[0], b[1], a[0], a[1], a[2], a[3]} : v6i{a[0], a[1], a[2], a[3], b[0], b[1]};
+    } else {   // K [16g, 16g+16) and [32+16g, ...) of the half
+      const v4i a = *reinterpret_cast<const v4i*>(slot + r.x8 + t * 4096 + ((4 * H + g) ^ r.xor8) * 16);
+      const v4i b = *reinterpret_cast<const v4i*>(slot + r.x8 + t * 4096 + ((4 * H + 2 + g) ^ r.xor8) * 16);
+      f.x[t] = __builtin_shufflevector(a, b, 0, 1, 2, 3, 4, 5, 6, 7);
+    }
+  }
+}
+
+template <class G>
+struct TileScales {
+  int w[G::TN], x[G::TM];
+};
+// Scale dwords of the wave's fragments in a stage.  Of two fragments the lower 32 lanes read the first one's and the upper
+// ones the second one's (a dword read occupies the LDS for as long as a 16-byte one).
+template <class G>
+struct RawScales {
+  int w, x;
+};
+template <class G>
+__device__ __forceinline__ void read_scales(RawScales<G>& s, const uint8_t* slot, const ReadAt<G>& r) {
+  s.w = *reinterpret_cast<const int*>(slot + r.sw);
+  s.x = *reinterpret_cast<const int*>(slot + r.sx);
+}
+__device__ __forceinline__ void both_halves(int v, int& lower, int& upper) {
+  const auto p = __builtin_amdgcn_permlane32_swap((unsigned)v, (unsigned)v, false, false);
+  lower = (int)p[0];   // the lower lanes' value in all lanes
+  upper = (int)p[1];
+}
+template <class G>
+__device__ __forceinline__ TileScales<G> shifted(const RawScales<G>& s, int g) {
+  TileScales<G> o;
+  both_halves(s.w, o.w[0], o.w[1]);
+  if constexpr (G::TM == 2) both_halves(s.x, o.x[0], o.x[1]);
+  else o.x[0] = s.x;
+#pragma unroll
+  for (int t = 0; t < G::TN; ++t) o.w[t] = (int)((unsigned)o.w[t] >> (8 * g));
+#pragma unroll
+  for (int t = 0; t < G::TM; ++t) o.x[t] = (int)((unsigned)o.x[t] >> (8 * g));
+  return o;
+}
+
+// MFMAs [M0, M1) of a K half
+template <int FMT, int H, class G, int M0, int M1>
+__device__ __forceinline__ void multiply(v16f (&acc)[G::TN][G::TM], const TileFrags<FMT, G>& f, const TileScales<G>& sc) {
+#pragma unroll
+  for (int k = M0; k < M1; ++k) {
+    const int tn = k / G::TM, tm = k % G::TM;
+    acc[tn][tm] = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(widened(f.w[tn]), widened(f.x[tm]), acc[tn][tm], kFmtE2M1, FMT, 2 * H, sc.w[tn],
+                                                                  2 * H, sc.x[tm]);
+  }
+}
+
+// The 0 ... 3 blocks of 32 a segment has beyond its whole stages, straight from global memory, before the K loop; each segment's
+// by the waves of another stage of the batch.
+template <int FMT, class G>
+struct Rest {
+  TileFrags<FMT, G> f;
+  TileScales<G> sc;
+};
+template <int FMT, int H, class G>
+__device__ __forceinline__ void rest_load(Rest<FMT, G>& r, const TileCtx<G>& c, const TileSeg& s, int N, int wf, int wm) {
+  const int rem = s.blk & 3;
+  const int i = c.lane & 31, g = c.lane >> 5, q = s.blk >> 2, katoms = (s.blk + 3) >> 2;
+  const int kb = 4 * q + min(2 * H + g, rem - 1), kb0 = 4 * q + 2 * H, kb1 = 4 * q + min(2 * H + 1, rem - 1);   // blocks that exist
+#pragma unroll
+  for (int t = 0; t < G::TN; ++t) {
+    const int n = weight_row<G>(c, wf * G::TN + t, i);
+    const uint8_t* p = G::WT ? s.b + (size_t)(N >> 8) * q * 16384 + ((size_t)n * rem + (kb - 4 * q)) * 16 : s.b + ((size_t)n * s.blk + kb) * 16;
+    r.f.w[t] = *reinterpret_cast<const v4i*>(p);
+    r.sc.w[t] = s.sfb[sf_offset(n, kb, katoms)];
+  }
+#pragma unroll
+  for (int t = 0; t < G::TM; ++t) {
+    const int m = c.m0 + min((wm * G::TM + t) * 32 + i, c.last_row);
+    const uint8_t* row = s.a + (size_t)m * s.blk * (Form<FMT>::row / 4);
+    r.sc.x[t] = s.sfa[sf_offset(m, kb, katoms)];
+    if constexpr (FMT == kFmtE2M1) {
+      r.f.x[t] = *reinterpret_cast<const v4i*>(row + (size_t)kb * 16);
+    } else if constexpr (FMT == kFmtE3M2) {
+      const v2i* v = reinterpret_cast<const v2i*>(row + (size_t)kb * 24);
+      const v2i a = v[0], b = v[1], e = v[2];
+      r.f.x[t] = v6i{a[0], a[1], b[0], b[1], e[0], e[1]};
+    } else {
+      const v4i a = *reinterpret_cast<const v4i*>(row + (size_t)kb0 * 32 + g * 16), b = *reinterpret_cast<const v4i*>(row + (size_t)kb1 * 32 + g * 16);
+      r.f.x[t] = __builtin_shufflevector(a, b, 0, 1, 2, 3, 4, 5, 6, 7);
+    }
+  }
+}
+// what lies past the segment's end is zero
+template <int FMT, int H, class G>
+__device__ __forceinline__ void rest_multiply(v16f (&acc)[G::TN][G::TM], Rest<FMT, G>& r, const TileSeg& s, int g) {
+  const int rem = s.blk & 3;
+  const bool ok = 2 * H + g < rem, ok1 = 2 * H + 1 < rem;
+#pragma unroll
+  for (int t = 0; t < G::TN; ++t) {
+#pragma unroll
+    for (int e = 0; e < 4; ++e) r.f.w[t][e] = ok ? r.f.w[t][e] : 0;
+    r.sc.w[t] = ok ? r.sc.w[t] : 127;
+  }
+#pragma unroll
+  for (int t = 0; t < G::TM; ++t) {
+    r.sc.x[t] = ok ? r.sc.x[t] : 127;
+    if constexpr (FMT == kFmtE4M3) {
+#pragma unroll
+      for (int e = 4; e < 8; ++e) r.f.x[t][e] = ok1 ? r.f.x[t][e] : 0;
+    } else {
+#pragma unroll
+      for (int e = 0; e < (FMT == kFmtE2M1 ? 4 : 6); ++e) r.f.x[t][e] = ok ? r.f.x[t][e] : 0;
+    }
+  }
+  multiply<FMT, 0, G, 0, G::TN * G::TM>(acc, r.f, r.sc);
+}
+template <int H, class G>
+__device__ __forceinline__ void rest_half(v16f (&acc)[G::TN][G::TM], const TileCtx<G>& c, const TilePlan& p, int wf, int wm, int ws, int g) {
+  const bool has4 = (p.s4.blk & 3) > 2 * H && ws == 1 % G::WS, has6 = (p.s6.blk & 3) > 2 * H && ws == 2 % G::WS,
+             has8 = (p.s8.blk & 3) > 2 * H && ws == 3 % G::WS;   // wave-uniform
+  Rest<kFmtE2M1, G> r4;
+  Rest<kFmtE3M2, G> r6;
+  Rest<kFmtE4M3, G> r8;
+  if (has4) rest_load<kFmtE2M1, H, G>(r4, c, p.s4, p.N, wf, wm);
+  if (has6) rest_load<kFmtE3M2, H, G>(r6, c, p.s6, p.N, wf, wm);
+  if (has8) rest_load<kFmtE4M3, H, G>(r8, c, p.s8, p.N, wf, wm);
+  __builtin_amdgcn_sched_barrier(0);
+  if (has4) rest_multiply<kFmtE2M1, H, G>(acc, r4, p.s4, g);
+  if (has6) rest_multiply<kFmtE3M2, H, G>(acc, r6, p.s6, g);
+  if (has8) rest_multiply<kFmtE4M3, H, G>(acc, r8, p.s8, g);
+}
+
+// Workgroup -> tile.  Workgroups go to the 8 XCDs round-robin; an XCD (an L2) gets a rectangle of tiles where the counts divide,
+// the one with the fewest operand bytes per stage, else consecutive tiles in feature-major order.
+__device__ __forceinline__ void tile_at(const TilePlan& p, int wg, int& tn, int& tm) {
+  const int xcd = wg & 7;
+  int j = wg >> 3;
+  if (p.xlog < 0) j = p.div2 > 0 ? xcd * p.div2 + j : wg;
+  const int q = p.div > 1 ? (int)__umulhi((unsigned)j, p.magic) : j, r = j - q * p.div;
+  if (p.xlog < 0) {
+    tn = q;
+    tm = r;
+  } else {
+    tn = (xcd & ((1 << p.xlog) - 1)) * p.div + r;
+    tm = (xcd >> p.xlog) * p.div2 + q;
+  }
+}
+
+// All arguments into scalar registers in one batch of loads: fetched where they are first used they cost a round trip to the
+// argument buffer each time, before the first copy goes out.
+__device__ __forceinline__ void pin_plan(const TilePlan& p, const Epilogue& ep, const uint16_t* d) {
+  asm volatile("" : : "s"(p.s4.a), "s"(p.s4.b), "s"(p.s4.sfa), "s"(p.s4.sfb), "s"(p.s4.blk), "s"(p.s4.whole), "s"(p.s6.a), "s"(p.s6.b),
+               "s"(p.s6.sfa), "s"(p.s6.sfb), "s"(p.s6.blk), "s"(p.s6.whole), "s"(p.s8.a), "s"(p.s8.b), "s"(p.s8.sfa), "s"(p.s8.sfb),
+               "s"(p.s8.blk), "s"(p.s8.whole), "s"(p.total), "s"(p.N), "s"(p.m_store), "s"(p.a_rows), "s"(p.xlog), "s"(p.div), "s"(p.div2),
+               "s"(p.magic), "s"(ep.bias), "s"(ep.n_out), "s"(d));
+}
+
+template <int TF, int TT, int WF, int WS, bool WT, bool REM>
+__global__ void __launch_bounds__(64 * kTileWaves)
+mixed_gemm_tile_kernel(TilePlan plan, Epilogue ep, uint16_t* __restrict__ d) {
+  typedef Geo<TF, TT, WF, WS, WT> G;
+  constexpr int NB = G::NB;
+  extern __shared__ __align__(16) uint8_t lds[];
+  const unsigned lds0 = (unsigned)(size_t)(__attribute__((address_space(3))) uint8_t*)lds;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  pin_plan(plan, ep, d);
+  int tn, tm;
+  tile_at(plan, blockIdx.x, tn, tm);
+  TileCtx<G> c;
+  c.lane = threadIdx.x & 63;
+  c.n0 = tn * TF;
+  c.m0 = tm * TT;
+  c.tile = c.n0 >> 8;
+  c.j0 = (c.n0 & 255) >> 4;
+  c.last_col = min(plan.N - c.n0, TF) - 1;
+  c.last_row = min(plan.a_rows - c.m0, TT) - 1;
+  const int total = plan.total, t6 = plan.s4.whole, t8 = t6 + plan.s6.whole, batches = (total + WS - 1) / WS;
+
+  if (wave < kCopyWaves) {
+    // ------------------------------------------------------------------ copy waves
+    StageCopy<kFmtE2M1, G> k4;
+    StageCopy<kFmtE3M2, G> k6;
+    StageCopy<kFmtE4M3, G> k8;
+    unsigned slot = lds0;
+    const unsigned ring_end = lds0 + NB * G::kBatch;
+    auto advance = [&]() __attribute__((always_inline)) {
+      slot += G::kSlot;
+      slot = slot == ring_end ? lds0 : slot;
+    };
+    // The first NB batches at once, then one more behind each barrier.  Before the barrier that hands over a batch, all but
+    // the copies of the NB - 2 younger ones have landed (kBatchCopies each at least; a last, partial one is counted as none).
+    constexpr int LB = kBatchCopies<G>;
+    auto stages = [&](auto& k, int& t, int last) __attribute__((always_inline)) {
+      for (; t < last; ++t) {
+        k.issue(t, slot);
+        advance();
+      }
+    };
+    // whole batches of one segment
+    auto stream = [&](auto& k, int& t, int last) __attribute__((always_inline)) {
+      for (; t + WS <= last; t += WS) {
+        wait_vm<(NB - 2) * LB>();
+        workgroup_barrier();
+#pragma unroll
+        for (int u = 0; u < WS; ++u) {
+          k.issue(t + u, slot);
+          advance();
+        }
+      }
+    };
+    // a run of stages whatever their segments
+    auto mixed = [&](int& t, int last) __attribute__((always_inline)) {
+      stages(k4, t, min(last, t6));
+      stages(k6, t, min(last, t8));
+      stages(k8, t, last);
+    };
+    int t = 0;
+    constexpr int kFirst = NB * WS;
+    k4.init(c, plan.s4, wave);
+    const bool short4 = t6 < kFirst;
+    if (short4) {
+      k6.init(c, plan.s6, wave);
+      k8.init(c, plan.s8, wave);
+    }
+    if (total >= kFirst) {
+      // two batches, then the multiplying starts on the first of them, then the rest of the ring
+      mixed(t, 2 * WS);
+      wait_vm<LB>();
+      workgroup_barrier();   // batch 0 has landed
+      mixed(t, kFirst);
+      if (!short4) {
+        k6.init(c, plan.s6, wave);
+        k8.init(c, plan.s8, wave);
+      }
+      stream(k4, t, t6);
+      if (t < t6 && t + WS <= total) {   // a batch of two or three segments
+        wait_vm<(NB - 2) * LB>();
+        workgroup_barrier();
+        mixed(t, t + WS);
+      }
+      stream(k6, t, t8);
+      if (t < t8 && t + WS <= total) {
+        wait_vm<(NB - 2) * LB>();
+        workgroup_barrier();
+        mixed(t, t + WS);
+      }
+      stream(k8, t, total);
+      if (t < total) {   // the last, partial batch
+        wait_vm<(NB - 2) * LB>();
+        workgroup_barrier();
+        mixed(t, total);
+        drain<NB - 2, LB, 1>();
+      } else {
+        drain<NB - 2, LB, 0>();
+      }
+    } else {   // all of them at once
+      mixed(t, total);
+      wait_vm<0>();
+      for (int q = 0; q <= batches; ++q) workgroup_barrier();
+    }
+  } else {
+    // ------------------------------------------------------------------ math waves
+    const int mw = wave - kCopyWaves, wf = mw % WF, wm = (mw / WF) % G::WM, ws = mw / (WF * G::WM);
+    const int i = c.lane & 31, g = c.lane >> 5;
+    ReadAt<G> at;
+    at.xor4 = (i >> 2) & 3;
+    at.xor8 = (i >> 1) & 7;
+    at.xorw = i & 3;
+    at.w = G::kW + (WT ? ((wf * G::TN) >> 1) * 4096 + ((wf * G::TN) & 1) * 512 + (i & 3) * 1024 + (i >> 2) * 64 : (wf * G::TN) * 2048 + i * 64);
+    at.x4 = G::kX + (wm * G::TM) * 2048 + i * 64;
+    at.x6 = G::kX + (wm * G::TM) * 3072 + i * 96;
+    {
+      const int turn = (i >> 3) & 1;
+      auto piece = [&](int p) { return (p + turn == 6 ? 0 : p + turn) * 16; };
+      at.p6a = piece(2 * g);
+      at.p6b = piece(3 + 2 * g);
+      at.h6a = piece(1) + 8 * g;
+      at.h6b = piece(4) + 8 * g;
+    }
+    at.x8 = G::kX + (wm * G::TM) * 4096 + i * 128;
+    if constexpr (WT) at.sw = (wf * G::TN + g) * 128 + ((i >> 4) * 4 + (i & 3)) * 16 + ((i >> 2) & 3) * 4;
+    else at.sw = i * 16 + ((((c.n0 & 127) >> 5) + wf * G::TN + g) & 3) * 4;
+    at.sx = 512 + i * 16 + (((c.m0 & 127) >> 5) + wm * G::TM + (G::TM == 2 ? g : 0)) * 4;
+
+    v16f acc[G::TN][G::TM];
+#pragma unroll
+    for (int a = 0; a < G::TN; ++a)
+#pragma unroll
+      for (int b = 0; b < G::TM; ++b)
+#pragma unroll
+        for (int v = 0; v < 16; ++v) acc[a][b][v] = 0.0f;
+    if constexpr (REM) {
+      rest_half<0, G>(acc, c, plan, wf, wm, ws, g);
+      rest_half<1, G>(acc, c, plan, wf, wm, ws, g);
+    }
+    workgroup_barrier();   // batch 0 has landed
+    const uint8_t* slot = lds + ws * G::kSlot;
+    const uint8_t* const ring_end = slot + NB * G::kBatch;
+    // This wave's stages of one segment.  Everything between two barriers is one basic block with its order fixed by scheduling
+    // barriers: an MFMA, the reads of the next half, the other MFMAs (the compiler would sink them behind the barrier).
+    auto run = [&](auto fmt_c, int stages) __attribute__((always_inline)) {
+      constexpr int FMT = decltype(fmt_c)::value;
+      if (stages == 0) return;
+      TileFrags<FMT, G> fa, fb, fn;
+      RawScales<G> raw;
+      TileScales<G> sc;
+      read_scales<G>(raw, slot, at);
+      read_half<FMT, 0, G>(fa, slot, at, g);
+      auto first_half = [&]() __attribute__((always_inline)) {
+        wait_lds();
+        sc = shifted<G>(raw, g);
+        multiply<FMT, 0, G, 0, 1>(acc, fa, sc);
+        __builtin_amdgcn_sched_barrier(0);
+        read_half<FMT, 1, G>(fb, slot, at, g);
+        __builtin_amdgcn_sched_barrier(0);
+        multiply<FMT, 0, G, 1, G::TN * G::TM>(acc, fa, sc);
+        __builtin_amdgcn_sched_barrier(0);
+        wait_lds();
+        workgroup_barrier();   // the next batch has landed; this one is in registers
+        slot += G::kBatch;
+        slot = slot == ring_end ? slot - NB * G::kBatch : slot;
+        __builtin_amdgcn_sched_barrier(0);
+        multiply<FMT, 1, G, 0, 1>(acc, fb, sc);
+        __builtin_amdgcn_sched_barrier(0);
+      };
+      for (int q = 1; q < stages; ++q) {
+        first_half();
+        read_scales<G>(raw, slot, at);
+        read_half<FMT, 0, G>(fn, slot, at, g);
+        __builtin_amdgcn_sched_barrier(0);
+        multiply<FMT, 1, G, 1, G::TN * G::TM>(acc, fb, sc);
+        __builtin_amdgcn_sched_barrier(0);
+        fa = fn;
+      }
+      first_half();
+      multiply<FMT, 1, G, 1, G::TN * G::TM>(acc, fb, sc);
+    };
+    auto mine = [&](int t) { return (max(t - ws, 0) + WS - 1) / WS; };   // of the first t stages
+    run(std::integral_constant<int, kFmtE2M1>{}, mine(t6));
+    run(std::integral_constant<int, kFmtE3M2>{}, mine(t8) - mine(t6));
+    run(std::integral_constant<int, kFmtE4M3>{}, mine(total) - mine(t8));
+    if (mine(total) < batches) workgroup_barrier();
+
+    // Nothing reads or fills the ring any more.  The partial sums to LDS, as rows of tokens: a lane holds token i of its 32 x 32
+    // tiles and fragment rows 8 (v / 4) + 4 g + v % 4, four consecutive features at a time.
+#pragma unroll
+    for (int b = 0; b < G::TM; ++b) {
+      uint8_t* row = lds + ws * G::kPart + ((wm * G::TM + b) * 32 + i) * G::kPitch;
+#pragma unroll
+      for (int a = 0; a < G::TN; ++a)
+#pragma unroll
+        for (int vq = 0; vq < 4; ++vq)
+          *reinterpret_cast<v4f*>(row + out_position<G>(wf * G::TN + a, vq, g) * 4) =
+              v4f{acc[a][b][4 * vq], acc[a][b][4 * vq + 1], acc[a][b][4 * vq + 2], acc[a][b][4 * vq + 3]};
+    }
+    wait_lds();
+  }
+  workgroup_barrier();
+
+  // All waves add the partial sums of a batch's stages, in their order, and store pieces of eight features (tile-major weights, 64
+  // features: four).  On tile-major weights a piece is one run out of every sixteen features; its neighbours are other
+  // workgroups' of the same XCD, whose L2 puts them together (so these are ordinary stores).
+  {
+    constexpr int E = WT && TF == 64 ? 4 : 8;                  // features per piece
+    constexpr int PR = TF / E, RI = 64 / PR;                   // pieces per row, rows per instruction
+    typedef uint16_t vh __attribute__((ext_vector_type(E)));
+    typedef vh vh_any __attribute__((aligned(2)));
+    const int piece = c.lane % PR, sub = c.lane / PR;
+    const int col = WT ? c.tile * 256 + 16 * piece + c.j0 : c.n0 + piece * E;
+    const int n_out = ep.n_out, cols_left = n_out - col;
+    vh bias = {};
+    if (ep.bias != nullptr) {   // wave-uniform
+#pragma unroll
+      for (int e = 0; e < E; ++e) bias[e] = e < cols_left ? ep.bias[col + e] : (uint16_t)0;
+    }
+    const bool aligned = (n_out & (E - 1)) == 0;
+    for (int r0 = wave * RI; r0 < TT; r0 += kTileWaves * RI) {
+      const int r = r0 + sub, m = c.m0 + r;
+      if (r >= TT || m >= plan.m_store || cols_left <= 0) continue;
+      vh h;
+      const uint8_t* at = lds + r * G::kPitch + piece * (4 * E);
+#pragma unroll
+      for (int e = 0; e < E; e += 4) {
+        v4f sum = *reinterpret_cast<const v4f*>(at + 4 * e);
+#pragma unroll
+        for (int o = 1; o < WS; ++o) sum += *reinterpret_cast<const v4f*>(at + o * G::kPart + 4 * e);
+#pragma unroll
+        for (int x = 0; x < 4; ++x) h[e + x] = __builtin_bit_cast(uint16_t, (__bf16)sum[x]);
+      }
+      if (ep.bias != nullptr) {
+#pragma unroll
+        for (int e = 0; e < E; ++e) h[e] = add_bf16(h[e], bias[e]);
+      }
+      uint16_t* dst = d + (size_t)m * n_out + col;
+      if (cols_left >= E) {
+        if constexpr (WT) *reinterpret_cast<vh_any*>(dst) = h;
+        else if (aligned) __builtin_nontemporal_store(h, reinterpret_cast<vh*>(dst));
+        else __builtin_nontemporal_store(h, reinterpret_cast<vh_any*>(dst));
+      } else {
+#pragma unroll
+        for (int e = 0; e < E - 1; ++e)
+          if (e < cols_left) dst[e] = h[e];
+      }
+    }
+  }
+}
+
+template <int TF, int TT, int WF, int WS>
+hipError_t launch_geo(const TilePlan& p, int nwg, bool w_tiled, bool rem, const Epilogue& ep, uint16_t* d, hipStream_t stream) {
+  const auto kernel = w_tiled ? (rem ? mixed_gemm_tile_kernel<TF, TT, WF, WS, true, true> : mixed_gemm_tile_kernel<TF, TT, WF, WS, true, false>)
+                              : (rem ? mixed_gemm_tile_kernel<TF, TT, WF, WS, false, true> : mixed_gemm_tile_kernel<TF, TT, WF, WS, false, false>);
+  typedef Geo<TF, TT, WF, WS, false> G;
+  constexpr int kLds = G::NB * G::kBatch;
+  if (hipError_t e = allow_dynamic_lds(reinterpret_cast<const void*>(kernel), kLds); e != hipSuccess) return e;
+  hipLaunchKernelGGL(kernel, dim3(nwg), dim3(64 * kTileWaves), kLds, stream, p, ep, d);
+  return hipGetLastError();
+}
+
+}  // namespace
+
+struct TilePlanChoice { int tf, tt; double us; };
+
+// The tile with the lowest estimate.  A workgroup has its CU to itself (LDS), so a launch is rounds of them; microseconds: fixed,
+// per round, per stage and round, per stage with all CUs busy, per MB of results, per round with blocks past the whole stages.
+// Fitted to 290 measured calls each (24 ... 3000 tokens, N 384 ... 28672, K 1024 ... 18944, tile-major weights; rms error 9 %):
+// the tile taken is in the mean 1 % slower than the best of the three.
+TilePlanChoice mixed_gemm_tile_plan(int M, int N, int KN, int KS, int KO, int cus) {
+  static const struct { int tf, tt; double fixed, round, stage, fill, mb, rest; } kTiles[] = {
+      {128, 128, 2.02, 0.19, 0.253, 0.096, 0.56, 2.1}, {128, 64, 1.29, 1.36, 0.167, 0.059, 0.45, 1.2}, {64, 64, 1.51, 0.99, 0.124, 0.028, 0.78, 1.1}};
+  const int stages = KN / 128 + KS / 128 + KO / 128;
+  const bool rest = ((KN | KS | KO) & 127) != 0;
+  TilePlanChoice best = {0, 0, 0.0};
+  for (const auto& t : kTiles) {
+    const int64_t tiles = (int64_t)ceil_div(N, t.tf) * ceil_div(M, t.tt);
+    const double rounds = (double)((tiles + cus - 1) / cus), busy = tiles < cus ? (double)tiles / cus : 1.0;
+    const double us = t.fixed + rounds * (t.round + stages * t.stage + (rest ? t.rest : 0.0)) + stages * t.fill * busy + 2e-6 * M * N * t.mb;
+    if (best.tf == 0 || us < best.us) best = {t.tf, t.tt, us};
+  }
+  return best;
+}
+
+hipError_t launch_mixed_gemm_tile(const uint8_t* an, const uint8_t* bn, const uint8_t* as_, const uint8_t* bs,
+                                  const uint8_t* ao, const uint8_t* bo, const uint8_t* sfan, const uint8_t* sfbn,
+                                  const uint8_t* sfas, const uint8_t* sfbs, const uint8_t* sfao, const uint8_t* sfbo,
+                                  int m_store, int a_rows, int N, int KN, int KS, int KO, bool w_tiled, const TilePlanChoice& choice,
+                                  Epilogue ep, void* d, hipStream_t stream) {
+  const int tf = choice.tf, tt = choice.tt;
+  if (m_store <= 0 || a_rows < m_store) return hipErrorInvalidValue;
+  TilePlan p;
+  p.s4 = {an, bn, sfan, sfbn, KN / 32, KN / 128};
+  p.s6 = {as_, bs, sfas, sfbs, KS / 32, KS / 128};
+  p.s8 = {ao, bo, sfao, sfbo, KO / 32, KO / 128};
+  p.total = p.s4.whole + p.s6.whole + p.s8.whole;
+  p.N = N;
+  p.m_store = m_store;
+  p.a_rows = a_rows;
+  const int tiles_n = ceil_div(ep.n_out, tf), tiles_m = ceil_div(m_store, tt), nwg = tiles_n * tiles_m;
+  p.xlog = -1;
+  p.div = tiles_m;
+  p.div2 = (nwg & 7) == 0 ? nwg >> 3 : 0;
+  if ((nwg & 7) == 0) {
+    int best = 0x7fffffff;
+    for (int x = 3; x >= 0; --x) {
+      const int gx = 1 << x, gy = 8 >> x;
+      if (tiles_n % gx || tiles_m % gy) continue;
+      const int cost = (tiles_n / gx) * tf * 64 + (tiles_m / gy) * tt * 80;   // operand bytes per stage of a rectangle
+      if (cost < best) {
+        best = cost;
+        p.xlog = x;
+        p.div = tiles_n / gx;
+        p.div2 = tiles_m / gy;
+      }
+    }
+  }
+  p.magic = p.div > 1 ? (unsigned)(((1ull << 32) + p.div - 1) / p.div) : 0;
+  const bool rem = ((KN | KS | KO) & 127) != 0;
+  uint16_t* out = static_cast<uint16_t*>(d);
+  if (tf == 128 && tt == 128) return launch_geo<128, 128, 2, 2>(p, nwg, w_tiled, rem, ep, out, stream);
+  if (tf == 128 && tt == 64) return launch_geo<128, 64, 2, 2>(p, nwg, w_tiled, rem, ep, out, stream);
+  if (tf == 64 && tt == 64) return launch_geo<64, 64, 1, 4>(p, nwg, w_tiled, rem, ep, out, stream);
+  return hipErrorInvalidValue;
+}
+
+}  // namespace mg

@@ -721,6 +721,40 @@ def test_exact_size_activation_buffers_on_the_whole_tile_kernel(abi, m, n, kn, k
     assert torch.equal(d_pad, d_tight)
 
 
+# Small tiles (64 x 64, 128 x 64, 128 x 128): token counts at and past the edges of 64 and 128, feature counts of whole, ragged and
+# single tiles, fewer stages than the ring holds, a last batch that is not whole, batches across segment boundaries (stage counts
+# that are no multiples of 2 and 4), empty segments, 1 to 3 blocks past the whole stages, a segment without a whole stage.
+SMALL_TILE_SHAPES = [
+    (256, 256, 128, 128, 128), (257, 264, 128, 0, 0), (319, 1000, 0, 256, 128), (320, 520, 640, 384, 128), (321, 768, 1152, 640, 256),
+    (450, 1001, 1152, 640, 256), (300, 60, 416, 224, 96), (300, 40, 64, 32, 0), (511, 1280, 480, 480, 480), (256, 8, 32, 0, 0),
+    (300, 5120, 256, 160, 128), (384, 4352, 640, 416, 128), (385, 4100, 640, 384, 128), (512, 2816, 0, 0, 640),
+    (260, 6656, 384, 160, 128), (513, 3584, 384, 384, 384), (640, 3080, 1024, 0, 128), (385, 6400, 448, 416, 224), (257, 6401, 640, 256, 0),
+]
+
+
+@pytest.mark.parametrize("m,n,kn,ks,ko", SMALL_TILE_SHAPES)
+def test_small_tiles_match_oracle(abi, m, n, kn, ks, ko):
+    """Row-major against the oracle, tile-major weights and exact-size activation buffers bit for bit like them."""
+    _say("small tiles", m, n, kn, ks, ko)
+    k = kn + ks + ko
+    x = H.make_activations(m, k, 81 + m, n_out=max(1, k // 32))
+    w = H.make_weights(n, k, 82 + n)
+    idx = H.absmax_sort_index(x)
+    bq = abi.reorder_quantize_w(w.to(DEV), idx.to(DEV), kn, ks, ko)
+    aq = abi.reorder_quantize_x(x.to(DEV), idx.to(DEV), kn, ks, ko)
+    tight = [t.clone() for t in aq]
+    args = lambda a, b: (a[0], b[0], a[1], b[1], a[2], b[2], a[3], bq[3], a[4], bq[4], a[5], bq[5])
+    d = abi.matmul(*args(aq, bq))
+    d_tight = abi.matmul(*args(tight, bq))
+    torch.cuda.synchronize()
+    _check_gemm(d, *_oracle_operands(x, w, idx, kn, ks, ko), "small tiles")
+    assert torch.equal(d, d_tight)
+    if abi.weights_tileable(n, kn, ks, ko):
+        d_tiled = abi.matmul(*args(tight, abi.tile_weights(*bq[:3])), w_tiled=True)
+        torch.cuda.synchronize()
+        assert torch.equal(d, d_tiled)
+
+
 def _seeded_shapes(count, seed):
     """Shapes drawn across the dispatcher's cases: token counts on both sides of 256 and of whole tiles, feature
     counts with and without whole 256-feature tiles, segments of 0 or 32..1024 channels in steps of 32."""
