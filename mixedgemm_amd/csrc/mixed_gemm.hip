@@ -1117,16 +1117,16 @@ static double pipelined_us(int M, int N, int stages, int cus, bool w_tiled) {
   return (double)ceil_div(whole, cus) * (stages * 0.95 + 3.0);
 }
 
-// The same on tile-major weights for 256 tokens and more, fitted to 148 measured calls (rms error 7 %): half tiles (at most cus / 2
+// The same on tile-major weights for 256 tokens and more, fitted to 184 measured calls (rms error 7 %): half tiles (at most cus / 2
 // whole ones) or rounds of whole tiles, of which a last one on at most half of the CUs counts 0.62; microseconds per stage, per
 // MB of results, and what the blocks past whole stages cost.
 static double whole_tiles_us(int M, int N, int stages, bool rest, bool three_segments, int cus) {
   const int whole = ceil_div(M, 256) * ceil_div(N, 256), halves = ceil_div(M, 128) * ceil_div(N, 256);
   const double mb = 2e-6 * M * N;
-  if (whole <= cus / 2) return 3.46 + stages * (0.354 + 0.104 * fmin(1.0, (double)halves / cus)) + 0.19 * mb + (rest ? 2.2 : 0.0);
+  if (whole <= cus / 2) return 3.8 + stages * (0.346 + 0.084 * fmin(1.0, (double)halves / cus)) + 0.26 * mb + (rest ? 2.0 : 0.0);
   const int full = whole / cus, left = whole % cus;
   const double rounds = full + (left == 0 ? 0.0 : (left <= cus / 2 && full > 0 && three_segments ? 0.62 : 1.0));
-  return fmax(1.44 + rounds * (stages * 0.748 - 9.1 + (rest ? 2.1 : 0.0)) + 0.68 * mb, rounds * stages * 0.6);
+  return fmax(1.4 + rounds * (stages * 0.741 - 7.0 + (rest ? 2.5 : 0.0)) + 0.63 * mb, rounds * stages * 0.6);
 }
 
 // a_rows: token rows for which the activation codes and scales are readable (>= M)

@@ -11,9 +11,10 @@
 // 4096, one per CU: 270 cycles per stage, of which 64 are MFMAs' (150 without copies); a launch of them takes 1.2 us until the
 // first stages have landed, 2.7 us for 20 E2M1 and 1.3 for 12 later stages, 1.2 us to add the partial sums and store.
 // Tile-major / row-major weights, of two or three layers in turn, before (skinny kernel or 256 x 128 tiles) -> now, us:
-//   M = 256, N = 4096, K = 4096: 16.4 / 19.6 -> 8.5 / 8.5;   K = 14336: 45.6 / 59.9 -> 19.7 / 22.3
-//   M = 512, N = 4096, K = 4096: 16.6 / 19.6 -> 10.5 / 11.8;  N = 1024, K = 8192: 27.6 / 34.8 -> 11.6 / 13.2
-//   M = 64, N = 14336, K = 4096: 16.4 / 16.8 -> 8.8 / 9.3;   M = 128: 16.9 / 20.3 -> 10.3 / 12.3
+//   M = 256, N = 4096, K = 4096: 16.4 / 19.6 -> 8.3 / 8.6;   K = 14336: 45.6 / 59.9 -> 20.2 / 22.3
+//   M = 512, N = 4096, K = 4096: 16.6 / 19.6 -> 10.0 / 12.0;  N = 1024, K = 8192: 27.6 / 34.8 -> 11.6 / 13.2
+//   M = 64, N = 14336, K = 4096: 16.4 / 16.8 -> 8.8 / 9.3;   M = 128: 16.8 / 20.1 -> 10.1 / 12.3
+//   M = 1024, N = 4096, K = 4096: 17.0 / 19.7 -> 14.7 / 17.0
 // Tiles of 256 x 128 with the same division of work were level with the mixed waves of the 256 x 256 kernel (M = 2048, N =
 // 4096, K = 12288: 57.6 against 56.3 us: 15 % fewer cycles at a clock as much lower; the chip is at its power limit there), tiles of
 // 64 and 128 x 32 slower than 64 x 64 at every shape tried.
@@ -29,6 +30,8 @@ constexpr int kCopyWaves = 4, kMathWaves = 8, kTileWaves = kCopyWaves + kMathWav
 constexpr int kRingBytes = 156 * 1024;   // LDS for the ring of batches
 
 typedef int v6i __attribute__((ext_vector_type(6)));
+typedef uint16_t v8h __attribute__((ext_vector_type(8)));
+typedef v8h v8h_any __attribute__((aligned(2)));
 
 struct TileSeg {
   const uint8_t *a, *b, *sfa, *sfb;
@@ -106,33 +109,59 @@ struct Geo {
 
 template <class G>
 struct TileCtx {
-  int lane, n0, m0;        // row-major: first feature of the tile
-  int tile, j0;            // tile-major: 256-feature tile and first copy block in it
+  int lane, n0, m0;        // first feature, first token of the tile
   int last_col, last_row;  // last readable weight / token row, from the tile's first
 };
 
-// Which weight row is row i of a 32-row fragment T of the tile.  Row-major: rows 32 T + i.  Tile-major (copy block b, row e of
-// its 16): block 4 (T / 2) + i % 4, row i / 4 + 8 (T % 2), so that four consecutive fragment rows are four consecutive features.
-template <class G>
-__device__ __forceinline__ int weight_row(const TileCtx<G>& c, int T, int i) {
-  if constexpr (G::WT) return c.tile * 256 + c.j0 + 4 * (T >> 1) + (i & 3) + 32 * (i >> 2) + 16 * (T & 1);
-  else return c.n0 + min(32 * T + i, c.last_col);
-}
-// Position in the tile's output row (features in ascending order) of fragment rows 8 vq + 4 g ... + 3.
-template <class G>
-__device__ __forceinline__ int out_position(int T, int vq, int g) {
-  if constexpr (G::WT) return (2 * (2 * vq + g) + (T & 1)) * (G::TF / 16) + 4 * (T >> 1);
-  else return 32 * T + 8 * vq + 4 * g;
-}
-
 // ---------------------------------------------------------------------------------------------
 // Copies of one whole stage, dealt to the four copy waves.  Weights and E2M1 tokens: 16 rows x 64 B per copy, the 16-byte
-// pieces of row r permuted by XOR with r / 4 (tile-major weights: with the block's number), E4M3: 8 rows x 128 B, permuted by XOR
-// with r / 2, E3M2: rows of 96 B one after the other, their pieces rotated by one in rows 8 ... 15 of every 16: the 16 rows that a
-// fragment read touches at a time lie on different banks (E3M2 rows as they are: 0.85 instead of 0.36 us per stage of 128 x 128).
-// Scales: the 16-byte pieces (rows c, c + 32, c + 64, c + 96 of an atom of 128 rows) that hold the tile's rows, one copy; on
-// tile-major weights in the order that makes the scales of a 32-row fragment 128 consecutive bytes.
+// pieces of row r permuted by XOR with r / 4, E4M3: 8 rows x 128 B, permuted by XOR with r / 2, E3M2: rows of 96 B one after the other,
+// their pieces rotated by one in rows 8 ... 15 of every 16: the 16 rows that a fragment read touches at a time lie on different
+// banks (E3M2 rows as they are: 0.85 instead of 0.36 us per stage of 128 x 128).  Scales: the two atoms of 128 rows that hold the
+// tile's rows, one copy.
+// Tile-major weights (16 KB per 256 features and stage: 1 KB per j = feature % 16, in it 64 bytes per feature / 16, even ones
+// first): a copy takes what the tile's features have of 128 / TF blocks of 1 KB, whole lines, and row i of a 32-row fragment is the
+// feature that WeightRows says.  (A workgroup has consecutive features: with whole 1 KB blocks, i.e. every other run of eight, two
+// workgroups shared each line of the result: M = 1024, N = K = 4096 from warm L2s 17.1 us, now 13.9; with one feature's 64 bytes
+// per four lanes, half lines, M = 256, N = 4096, K = 14336 21.9 us, now 20.2.)
 // ---------------------------------------------------------------------------------------------
+// Rows of a weight fragment.  Row-major: row i of fragment T is feature 32 T + i of the tile, in copy block 2 T + i / 16.
+// Tile-major, 128 features: copy block j / 2 holds [j % 2][feature / 16 % 2][feature / 32]; 64: j / 4 [j % 4][...][...].  Four
+// consecutive rows of a fragment are four consecutive features, and the 16 rows read at a time (0-3, 12-15, 20-27 and the others)
+// are four different feature / 16 with all four j % 4 each: with the pieces permuted by XOR with j, on different banks.
+template <class G>
+struct WeightRows {
+  static __device__ __forceinline__ int feature(int T, int i) {
+    if constexpr (!G::WT) return 32 * T + i;
+    else if constexpr (G::TF == 128) return 16 * (2 * ((i >> 2) & 3) + (i >> 4)) + 4 * T + (i & 3);
+    else return 16 * (2 * ((i >> 2) & 1) + ((i >> 3) & 1)) + 8 * T + 4 * (i >> 4) + (i & 3);
+  }
+  // of its 64 bytes in the stage's weights
+  static __device__ __forceinline__ int lds(int T, int i) {
+    if constexpr (!G::WT) return T * 2048 + i * 64;
+    else if constexpr (G::TF == 128) return T * 2048 + ((i >> 1) & 1) * 1024 + (i & 1) * 512 + (i >> 4) * 256 + ((i >> 2) & 3) * 64;
+    else return T * 2048 + (i >> 4) * 1024 + (i & 3) * 256 + ((i >> 3) & 1) * 128 + ((i >> 2) & 1) * 64;
+  }
+  // of its scale dword in the stage's scales; first: the tile's first feature in its atom of 128, / 32
+  static __device__ __forceinline__ int scale(int T, int i, int first) {
+    if constexpr (!G::WT) return i * 16 + ((first + T) & 3) * 4;
+    else if constexpr (G::TF == 128) return T * 128 + (i >> 4) * 64 + (i & 3) * 16 + ((i >> 2) & 3) * 4;
+    else return T * 256 + ((i >> 3) & 1) * 128 + (i >> 4) * 64 + (i & 3) * 16 + (first + ((i >> 2) & 1)) * 4;
+  }
+  // what a lane copies: the 16-byte piece of the atom (32 lanes) ...
+  static __device__ __forceinline__ int scale_piece(int l) {
+    if constexpr (!G::WT) return l;
+    else if constexpr (G::TF == 128) return 16 * ((l >> 2) & 1) + 4 * (l >> 3) + (l & 3);
+    else return 16 * ((l >> 3) & 1) + 8 * (l >> 4) + 4 * ((l >> 2) & 1) + (l & 3);
+  }
+  // ... and the offset of its 16 bytes of copy block b in the stage's 16 KB of tile-major weights
+  static __device__ __forceinline__ unsigned tiled_offset(int b, int l, int n0) {
+    const int j = G::TF == 128 ? 2 * b + (l >> 5) : 4 * b + (l >> 4);
+    const int odd = G::TF == 128 ? (l >> 4) & 1 : (l >> 3) & 1, pair = G::TF == 128 ? (l >> 2) & 3 : (l >> 2) & 1;
+    return (unsigned)(j * 1024 + (((n0 & 255) >> 5) + pair + 8 * odd) * 64 + (((l & 3) ^ (j & 3)) * 16));
+  }
+};
+
 template <int FMT, class G>
 constexpr int kTokenCopiesAll = G::TT * Form<FMT>::row / 1024;
 // copies that every copy wave issues per whole batch, at least (a stage of a later segment has as many or more)
@@ -144,7 +173,7 @@ struct StageCopy {
   static constexpr int NW = G::TF / 64, NX = kTokenCopiesAll<FMT, G>, KX = (NX + kCopyWaves - 1) / kCopyWaves;
   const uint8_t *w, *x;         // bases of the next stage
   const uint8_t* sc;            // this lane's scale piece
-  unsigned vw[G::WT ? 1 : NW], vx[KX];
+  unsigned vw[NW], vx[KX];
   int wave;
 
   // token copies come in fours, a last pair is dealt to waves 0, 1 and 2, 3 in turn
@@ -155,8 +184,9 @@ struct StageCopy {
     wave = wave_;
     const int r = c.lane >> 2, p = (c.lane & 3) ^ ((c.lane >> 4) & 3);
     if constexpr (G::WT) {
-      w = s.b + ((size_t)c.tile * s.whole * 16 + c.j0 + wave) * 1024;
-      vw[0] = (unsigned)(r * 64 + ((c.lane & 3) ^ wave) * 16);
+      w = s.b + (size_t)(c.n0 >> 8) * s.whole * 16384;
+#pragma unroll
+      for (int k = 0; k < NW; ++k) vw[k] = WeightRows<G>::tiled_offset(wave + kCopyWaves * k, c.lane, c.n0);
     } else {
       w = s.b + (size_t)c.n0 * s.blk * 16;
 #pragma unroll
@@ -179,28 +209,15 @@ struct StageCopy {
       }
     }
     const int katoms = (s.blk + 3) >> 2;
-    const int pl = c.lane & 31;
-    int atom, piece;   // of the features
-    if constexpr (G::WT) {
-      const int at = pl % (G::TF / 4), T = at >> 3;   // (64 features: 16 pieces, copied twice)
-      atom = c.tile * 2 + ((at >> 2) & 1);
-      piece = c.j0 + 4 * (T >> 1) + (at & 3) + 16 * (T & 1);
-    } else {
-      atom = c.n0 >> 7;
-      piece = pl;
-    }
-    const uint8_t* of_rows = s.sfa + (size_t)(c.m0 >> 7) * katoms * 512 + (c.lane & 31) * 16;
-    const uint8_t* of_features = s.sfb + (size_t)atom * katoms * 512 + piece * 16;
-    sc = c.lane < 32 ? of_features : of_rows;
+    const uint8_t* const of_features = s.sfb + (size_t)(c.n0 >> 7) * katoms * 512;
+    const uint8_t* const of_rows = s.sfa + (size_t)(c.m0 >> 7) * katoms * 512;
+    sc = c.lane < 32 ? of_features + WeightRows<G>::scale_piece(c.lane) * 16 : of_rows + (c.lane & 31) * 16;
   }
 
   // the next stage, t-th of all, into a slot.  What does not divide by the copy waves goes to other ones in every stage.
   __device__ __forceinline__ void issue(int t, unsigned slot) {
 #pragma unroll
-    for (int k = 0; k < NW; ++k) {
-      if constexpr (G::WT) copy_at(w + k * (kCopyWaves * 1024), vw[0], slot + G::kW + 1024u * (wave + kCopyWaves * k));
-      else copy_at(w, vw[k], slot + G::kW + 1024u * (wave + kCopyWaves * k));
-    }
+    for (int k = 0; k < NW; ++k) copy_at(w, vw[k], slot + G::kW + 1024u * (wave + kCopyWaves * k));
 #pragma unroll
     for (int k = 0; k < KX; ++k)
       if ((k + 1) * kCopyWaves <= NX || (wave >> 1) == (t & 1)) copy_at(x, vx[k], slot + G::kX + 1024u * block(k));
@@ -234,9 +251,9 @@ __device__ __forceinline__ v8i widened(v8i v) { return v; }
 
 template <int FMT, int H, class G>
 __device__ __forceinline__ void read_half(TileFrags<FMT, G>& f, const uint8_t* slot, const ReadAt<G>& r, int g) {
-  const int piece = ((2 * H + g) ^ r.xor4) * 16, wpiece = G::WT ? ((2 * H + g) ^ r.xorw) * 16 : piece;
+  const int piece = ((2 * H + g) ^ r.xor4) * 16, wpiece = ((2 * H + g) ^ r.xorw) * 16;
 #pragma unroll
-  for (int t = 0; t < G::TN; ++t) f.w[t] = *reinterpret_cast<const v4i*>(slot + r.w + t * (G::WT ? 512 : 2048) + wpiece);
+  for (int t = 0; t < G::TN; ++t) f.w[t] = *reinterpret_cast<const v4i*>(slot + r.w + t * 2048 + wpiece);
 #pragma unroll
   for (int t = 0; t < G::TM; ++t) {
     if constexpr (FMT == kFmtE2M1) {
@@ -313,7 +330,7 @@ __device__ __forceinline__ void rest_load(Rest<FMT, G>& r, const TileCtx<G>& c, 
   const int kb = 4 * q + min(2 * H + g, rem - 1), kb0 = 4 * q + 2 * H, kb1 = 4 * q + min(2 * H + 1, rem - 1);   // blocks that exist
 #pragma unroll
   for (int t = 0; t < G::TN; ++t) {
-    const int n = weight_row<G>(c, wf * G::TN + t, i);
+    const int n = c.n0 + min(WeightRows<G>::feature(wf * G::TN + t, i), c.last_col);
     const uint8_t* p = G::WT ? s.b + (size_t)(N >> 8) * q * 16384 + ((size_t)n * rem + (kb - 4 * q)) * 16 : s.b + ((size_t)n * s.blk + kb) * 16;
     r.f.w[t] = *reinterpret_cast<const v4i*>(p);
     r.sc.w[t] = s.sfb[sf_offset(n, kb, katoms)];
@@ -415,8 +432,6 @@ mixed_gemm_tile_kernel(TilePlan plan, Epilogue ep, uint16_t* __restrict__ d) {
   c.lane = threadIdx.x & 63;
   c.n0 = tn * TF;
   c.m0 = tm * TT;
-  c.tile = c.n0 >> 8;
-  c.j0 = (c.n0 & 255) >> 4;
   c.last_col = min(plan.N - c.n0, TF) - 1;
   c.last_row = min(plan.a_rows - c.m0, TT) - 1;
   const int total = plan.total, t6 = plan.s4.whole, t8 = t6 + plan.s6.whole, batches = (total + WS - 1) / WS;
@@ -510,8 +525,8 @@ mixed_gemm_tile_kernel(TilePlan plan, Epilogue ep, uint16_t* __restrict__ d) {
     ReadAt<G> at;
     at.xor4 = (i >> 2) & 3;
     at.xor8 = (i >> 1) & 7;
-    at.xorw = i & 3;
-    at.w = G::kW + (WT ? ((wf * G::TN) >> 1) * 4096 + ((wf * G::TN) & 1) * 512 + (i & 3) * 1024 + (i >> 2) * 64 : (wf * G::TN) * 2048 + i * 64);
+    at.xorw = WT ? i & 3 : (i >> 2) & 3;
+    at.w = G::kW + WeightRows<G>::lds(wf * G::TN, i);
     at.x4 = G::kX + (wm * G::TM) * 2048 + i * 64;
     at.x6 = G::kX + (wm * G::TM) * 3072 + i * 96;
     {
@@ -523,8 +538,7 @@ mixed_gemm_tile_kernel(TilePlan plan, Epilogue ep, uint16_t* __restrict__ d) {
       at.h6b = piece(4) + 8 * g;
     }
     at.x8 = G::kX + (wm * G::TM) * 4096 + i * 128;
-    if constexpr (WT) at.sw = (wf * G::TN + g) * 128 + ((i >> 4) * 4 + (i & 3)) * 16 + ((i >> 2) & 3) * 4;
-    else at.sw = i * 16 + ((((c.n0 & 127) >> 5) + wf * G::TN + g) & 3) * 4;
+    at.sw = WeightRows<G>::scale(wf * G::TN + g, i, (c.n0 & 127) >> 5);
     at.sx = 512 + i * 16 + (((c.m0 & 127) >> 5) + wm * G::TM + (G::TM == 2 ? g : 0)) * 4;
 
     v16f acc[G::TN][G::TM];
@@ -595,37 +609,31 @@ mixed_gemm_tile_kernel(TilePlan plan, Epilogue ep, uint16_t* __restrict__ d) {
       for (int a = 0; a < G::TN; ++a)
 #pragma unroll
         for (int vq = 0; vq < 4; ++vq)
-          *reinterpret_cast<v4f*>(row + out_position<G>(wf * G::TN + a, vq, g) * 4) =
+          *reinterpret_cast<v4f*>(row + WeightRows<G>::feature(wf * G::TN + a, 8 * vq + 4 * g) * 4) =
               v4f{acc[a][b][4 * vq], acc[a][b][4 * vq + 1], acc[a][b][4 * vq + 2], acc[a][b][4 * vq + 3]};
     }
     wait_lds();
   }
   workgroup_barrier();
 
-  // All waves add the partial sums of a batch's stages, in their order, and store pieces of eight features (tile-major weights, 64
-  // features: four).  On tile-major weights a piece is one run out of every sixteen features; its neighbours are other
-  // workgroups' of the same XCD, whose L2 puts them together (so these are ordinary stores).
+  // All waves add the partial sums of a batch's stages, in their order, and store pieces of eight features.
   {
-    constexpr int E = WT && TF == 64 ? 4 : 8;                  // features per piece
-    constexpr int PR = TF / E, RI = 64 / PR;                   // pieces per row, rows per instruction
-    typedef uint16_t vh __attribute__((ext_vector_type(E)));
-    typedef vh vh_any __attribute__((aligned(2)));
-    const int piece = c.lane % PR, sub = c.lane / PR;
-    const int col = WT ? c.tile * 256 + 16 * piece + c.j0 : c.n0 + piece * E;
+    constexpr int PR = TF / 8, RI = 64 / PR;   // pieces per row, rows per instruction
+    const int piece = c.lane % PR, sub = c.lane / PR, col = c.n0 + piece * 8;
     const int n_out = ep.n_out, cols_left = n_out - col;
-    vh bias = {};
+    v8h bias = {};
     if (ep.bias != nullptr) {   // wave-uniform
 #pragma unroll
-      for (int e = 0; e < E; ++e) bias[e] = e < cols_left ? ep.bias[col + e] : (uint16_t)0;
+      for (int e = 0; e < 8; ++e) bias[e] = e < cols_left ? ep.bias[col + e] : (uint16_t)0;
     }
-    const bool aligned = (n_out & (E - 1)) == 0;
+    const bool aligned = (n_out & 7) == 0;
     for (int r0 = wave * RI; r0 < TT; r0 += kTileWaves * RI) {
       const int r = r0 + sub, m = c.m0 + r;
       if (r >= TT || m >= plan.m_store || cols_left <= 0) continue;
-      vh h;
-      const uint8_t* at = lds + r * G::kPitch + piece * (4 * E);
+      v8h h;
+      const uint8_t* at = lds + r * G::kPitch + piece * 32;
 #pragma unroll
-      for (int e = 0; e < E; e += 4) {
+      for (int e = 0; e < 8; e += 4) {
         v4f sum = *reinterpret_cast<const v4f*>(at + 4 * e);
 #pragma unroll
         for (int o = 1; o < WS; ++o) sum += *reinterpret_cast<const v4f*>(at + o * G::kPart + 4 * e);
@@ -634,16 +642,15 @@ mixed_gemm_tile_kernel(TilePlan plan, Epilogue ep, uint16_t* __restrict__ d) {
       }
       if (ep.bias != nullptr) {
 #pragma unroll
-        for (int e = 0; e < E; ++e) h[e] = add_bf16(h[e], bias[e]);
+        for (int e = 0; e < 8; ++e) h[e] = add_bf16(h[e], bias[e]);
       }
       uint16_t* dst = d + (size_t)m * n_out + col;
-      if (cols_left >= E) {
-        if constexpr (WT) *reinterpret_cast<vh_any*>(dst) = h;
-        else if (aligned) __builtin_nontemporal_store(h, reinterpret_cast<vh*>(dst));
-        else __builtin_nontemporal_store(h, reinterpret_cast<vh_any*>(dst));
+      if (cols_left >= 8) {
+        if (aligned) __builtin_nontemporal_store(h, reinterpret_cast<v8h*>(dst));
+        else __builtin_nontemporal_store(h, reinterpret_cast<v8h_any*>(dst));
       } else {
 #pragma unroll
-        for (int e = 0; e < E - 1; ++e)
+        for (int e = 0; e < 7; ++e)
           if (e < cols_left) dst[e] = h[e];
       }
     }
@@ -667,11 +674,11 @@ struct TilePlanChoice { int tf, tt; double us; };
 
 // The tile with the lowest estimate.  A workgroup has its CU to itself (LDS), so a launch is rounds of them; microseconds: fixed,
 // per round, per stage and round, per stage with all CUs busy, per MB of results, per round with blocks past the whole stages.
-// Fitted to 290 measured calls each (24 ... 3000 tokens, N 384 ... 28672, K 1024 ... 18944, tile-major weights; rms error 9 %):
-// the tile taken is in the mean 1 % slower than the best of the three.
+// Fitted to 450 measured calls each (17 ... 2600 tokens, N 384 ... 28672, K 1024 ... 18944, tile-major weights; rms error 10 %):
+// the tile taken is in the mean 0.5 % slower than the best of the three.
 TilePlanChoice mixed_gemm_tile_plan(int M, int N, int KN, int KS, int KO, int cus) {
   static const struct { int tf, tt; double fixed, round, stage, fill, mb, rest; } kTiles[] = {
-      {128, 128, 2.02, 0.19, 0.253, 0.096, 0.56, 2.1}, {128, 64, 1.29, 1.36, 0.167, 0.059, 0.45, 1.2}, {64, 64, 1.51, 0.99, 0.124, 0.028, 0.78, 1.1}};
+      {128, 128, 2.87, -0.24, 0.260, 0.075, 0.41, 1.8}, {128, 64, 1.47, 1.29, 0.170, 0.051, 0.39, 1.0}, {64, 64, 1.55, 1.07, 0.125, 0.039, 0.46, 0.9}};
   const int stages = KN / 128 + KS / 128 + KO / 128;
   const bool rest = ((KN | KS | KO) & 127) != 0;
   TilePlanChoice best = {0, 0, 0.0};
