@@ -850,7 +850,7 @@ mixed_gemm_token_kernel(const uint8_t* __restrict__ x, const uint8_t* __restrict
     lds_barrier();
     double tot = 0.0;
     for (int w = 0; w < of; ++w) tot += sums[m * of + w];
-    const float r = rms_scale(tot, K, eps);
+    const float r = rms_scale(tot, K, 1.0 / (double)K, eps);
     for (int p = rank * 64 + lane; p < pieces; p += of * 64) {
       v4u* at = reinterpret_cast<v4u*>(row + p * 16);
       const v4u gm = *reinterpret_cast<const v4u*>(lds + L.gamma + p * 16);

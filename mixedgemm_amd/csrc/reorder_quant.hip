@@ -211,14 +211,18 @@ __global__ void __launch_bounds__(MAXT)
 reorder_quant_dma_kernel(const uint8_t* __restrict__ x, const int16_t* __restrict__ idx, int rows, int K, int KN, int KS,
                          int KO, uint8_t* __restrict__ qn, uint8_t* __restrict__ qs, uint8_t* __restrict__ qo,
                          uint8_t* __restrict__ sfn, uint8_t* __restrict__ sfs, uint8_t* __restrict__ sfo, RowSchedule sched,
-                         const uint16_t* __restrict__ gamma, float eps, int src_rows) {
+                         const uint16_t* __restrict__ gamma, float eps, double inv_k, int src_rows) {
   extern __shared__ __align__(16) uint8_t lds[];
   __shared__ double row_sums[NORM ? 2 : 1][NORM ? MAXT / 64 : 1];   // RMSNorm: the waves' sums of squares, by row parity
   static_assert(EPL == 32 || EPL == 16, "one or two lanes per block");
   constexpr int kPieces = EPL / 8;   // 16-byte pieces of a row (and of the index) per lane
   constexpr int kParts = EPL / 16;   // gathers of 16 per lane and row
   constexpr bool kImm = T > 0;
-  static_assert(!kImm || (NS - 1) * 2 * EPL * T <= 65535, "slot offsets must fit the LDS instructions' immediate");
+  // RMSNorm: two lanes per block normalize the channels they have gathered; one lane per block, whose gathered weights would take
+  // 32 registers, normalizes the row in place before the gather
+  constexpr bool kLate = NORM && EPL == 16;
+  static_assert(!kLate || kImm, "the weight's loads are counted");
+  static_assert(!kImm || (kLate ? NS : NS - 1) * 2 * EPL * T <= 65535, "slot offsets must fit the LDS instructions' immediate");
   const int tid = threadIdx.x;
   const int nthr = kImm ? T : (int)blockDim.x;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -286,13 +290,19 @@ reorder_quant_dma_kernel(const uint8_t* __restrict__ x, const int16_t* __restric
       else iv[q] = ip[q];
     }
   }
+  // RMSNorm: the weights of this lane's pieces of a row (the same for every row).  kLate: uncounted loads, older than the rows
+  // and there when the first one is; else ordinary loads, which the compiler waits for itself where they are first used (with
+  // vmcnt(0): once, in the first row).
+  v4u gv[kPieces];
+  if constexpr (kLate) {
+#pragma unroll
+    for (int it = 0; it < kPieces; ++it)
+      asm volatile("global_load_dwordx4 %0, %1, off" : "=v"(gv[it]) : "v"(gamma + (size_t)min(it * nthr + tid, nchunks - 1) * 8) : "memory");
+  }
 #pragma unroll
   for (int s = 0; s < NS; ++s)
     if (s < count) request(x + (size_t)src_row(row_of(s)) * row_bytes, s * stride);
-  // RMSNorm: the weights of this lane's pieces of a row (the same for every row); ordinary loads, which the compiler
-  // waits for itself where they are first used (with vmcnt(0): once, in the first row)
-  v4u gv[kPieces];
-  if constexpr (NORM) {
+  if constexpr (NORM && !kLate) {
 #pragma unroll
     for (int it = 0; it < kPieces; ++it)
       gv[it] = *reinterpret_cast<const v4u*>(gamma + (size_t)min(it * nthr + tid, nchunks - 1) * 8);
@@ -318,7 +328,7 @@ reorder_quant_dma_kernel(const uint8_t* __restrict__ x, const int16_t* __restric
   uint8_t* sfbase = seg == 0 ? sfn : (seg == 1 ? sfs : sfo);
 
   // ---- the index entries are the oldest requests: they are there when at most the row copies are in flight
-  wait_vm(kPieces * min(NS, count));
+  wait_vm(kPieces * min(NS, count) + (kLate ? kPieces : 0));
   if constexpr (kPieces == 4) asm volatile("" : "+v"(iv[0]), "+v"(iv[1]), "+v"(iv[2]), "+v"(iv[3]));
   else asm volatile("" : "+v"(iv[0]), "+v"(iv[1]));
   // LDS byte addresses of the lane's gathered channels in slot 0.  An entry outside [0, K) is read as
@@ -342,6 +352,8 @@ reorder_quant_dma_kernel(const uint8_t* __restrict__ x, const int16_t* __restric
       (__builtin_amdgcn_ballot_w64(fmt_or_none == kFmtE3M2) ? (EPL == 32 ? code_stores(kFmtE3M2) : 1) : 0) +
       (__builtin_amdgcn_ballot_w64(fmt_or_none == kFmtE4M3) ? (EPL == 32 ? code_stores(kFmtE4M3) : 1) : 0);
 
+  unsigned gw[kLate ? 16 : 1];   // kLate: the weights of the lane's gathered channels, in the upper halves
+
   int i = 0;
   auto body = [&](auto slot_c) {
     constexpr int S = decltype(slot_c)::value;
@@ -351,12 +363,15 @@ reorder_quant_dma_kernel(const uint8_t* __restrict__ x, const int16_t* __restric
     // iterations -- and the stores of the iterations since, at most NS - 1 of them.
     wait_vm(kPieces * min(i == 0 ? NS - 1 : NS - 2, count - 1 - i) + row_stores * min(i, NS - 1));
     if constexpr (NORM) {
-      // RMSNorm of the row, in place, before anyone gathers from it (the arithmetic of the usual fp32 implementation):
+      // RMSNorm of the row (the arithmetic of the usual fp32 implementation):
       //   var = fl32( (sum over the row of x^2, accumulated in fp64) / K )
       //   r   = fl32( 1 / sqrt( fl32(var + eps) ) )      (division and square root in fp64)
       //   y   = bf16( gamma * bf16( x * r ) )            (both products in fp32)
       // The fp64 sum makes the result independent of the order in which the lanes add their parts (up to the last
-      // bit of a double, which the rounding to fp32 all but never sees).  A lane works on the pieces it copied.
+      // bit of a double, which the rounding to fp32 all but never sees).  A lane sums over the pieces it copied.
+      // kLate: one barrier per row as without RMSNorm, nothing written back, and the vector ALUs, which bound it, have 220
+      // instructions per row and wave next to the quantizer's 110 instead of 280: M = 4096, K = 4096 17.1 us normalized in place, now
+      // 15.8; 8192 rows 28.9 -> 26.5, 1024 7.1 -> 6.7.
       uint8_t* slot = lds + S * stride;
       v4u a[kPieces];
       double part[4] = {0.0, 0.0, 0.0, 0.0};   // four chains: one chain of dependent fp64 fmas would wait for each in turn
@@ -375,28 +390,55 @@ reorder_quant_dma_kernel(const uint8_t* __restrict__ x, const int16_t* __restric
       }
       double ss = wave_sum((part[0] + part[1]) + (part[2] + part[3]));
       if ((tid & 63) == 0) row_sums[i & 1][tid >> 6] = ss;
+      if constexpr (kLate) {
+        if (i == 0) {   // the weights to LDS, behind the row slots, for the other lanes
+#pragma unroll
+          for (int it = 0; it < kPieces; ++it) {
+            asm volatile("" : "+v"(gv[it]));   // (older than the row: landed)
+            *reinterpret_cast<v4u*>(lds + NS * stride + (size_t)(it * nthr + tid) * 16) = gv[it];
+          }
+        }
+      }
       __builtin_amdgcn_s_waitcnt(0xC07F);   // lgkmcnt(0): the sum is in the LDS (a raw barrier implies no wait of the compiler's)
       asm volatile("s_barrier" ::: "memory");   // also: every wave's copies of row i have landed, every wave is past its gather of row i - 1
       if (i >= 1 && i - 1 + NS < count)
         request(x + (size_t)src_row(row_of(i + NS - 1)) * row_bytes, ((S + NS - 1) % NS) * stride);
-      double tot = 0.0;
-      for (int w = 0; w < (nthr >> 6); ++w) tot += row_sums[i & 1][w];
-      const float rn = rms_scale(tot, K, eps);
+      if constexpr (!kLate) {
+        double tot = 0.0;
+        for (int w = 0; w < (nthr >> 6); ++w) tot += row_sums[i & 1][w];
+        const float rn = rms_scale(tot, K, inv_k, eps);
 #pragma unroll
-      for (int it = 0; it < kPieces; ++it) {
+        for (int it = 0; it < kPieces; ++it) {
 #pragma unroll
-        for (int e = 0; e < 4; ++e) {
-          a[it][e] = rms_apply(a[it][e], gv[it][e], rn);
+          for (int e = 0; e < 4; ++e) {
+            a[it][e] = rms_apply(a[it][e], gv[it][e], rn);
+          }
+          if (it * nthr + tid < nchunks) *reinterpret_cast<v4u*>(slot + (size_t)(it * nthr + tid) * 16) = a[it];
         }
-        if (it * nthr + tid < nchunks) *reinterpret_cast<v4u*>(slot + (size_t)(it * nthr + tid) * 16) = a[it];
+        __builtin_amdgcn_s_waitcnt(0xC07F);
+        asm volatile("s_barrier" ::: "memory");   // the normalized row is complete
       }
-      __builtin_amdgcn_s_waitcnt(0xC07F);
-      asm volatile("s_barrier" ::: "memory");   // the normalized row is complete
     } else {
       asm volatile("s_barrier" ::: "memory");
       // every wave is past its gather of row i - 1: refill that row's slot
       if (i >= 1 && i - 1 + NS < count)
         request(x + (size_t)src_row(row_of(i + NS - 1)) * row_bytes, ((S + NS - 1) % NS) * stride);
+    }
+    // (the sums of row i: written again, for row i + 2, behind the barrier of row i + 1)
+    float rn = 0.0f;
+    if constexpr (kLate) {
+      double tot = 0.0;
+      for (int w = 0; w < (nthr >> 6); ++w) tot += row_sums[i & 1][w];
+      rn = rms_scale(tot, K, inv_k, eps);
+      if (i == 0) {
+        if (has_block) gather16<NS * 2 * EPL * T>(u[0], ga[0], 0u);
+        gather_wait(u[0]);
+#pragma unroll
+        for (int p = 0; p < 16; ++p) {
+          gw[p] = u[0][p];
+          u[0][p] = 0u;
+        }
+      }
     }
     if (has_block) {
       constexpr int kOff = kImm ? S * 2 * EPL * T : -1;
@@ -427,6 +469,9 @@ reorder_quant_dma_kernel(const uint8_t* __restrict__ x, const int16_t* __restric
         float f[16];
 #pragma unroll
         for (int p = 0; p < 16; ++p) f[p] = __uint_as_float(u[0][p]);
+        if constexpr (kLate)
+#pragma unroll
+          for (int p = 0; p < 16; p += 2) rms_apply(f[p], f[p + 1], gw[p], gw[p + 1], rn);
         quantize_half(f, fmt, half, StoreHalf<KEEP>{q, sf, half});
       }
     }
@@ -461,7 +506,7 @@ hipError_t launch_reorder_quant(const void* x, const int16_t* idx, int rows, int
   // rows global -> LDS directly; NS row slots per workgroup, as many workgroups per CU as fit
   const int usable = lim.lds_bytes - 1024;   // the kernels' static LDS (row sums of the RMSNorm) stays below 1 KB
   auto launch_dma = [&](auto kernel, int epl, int NS, int nthreads, int max_per_cu) {
-    const int lds = NS * 2 * epl * nthreads;   // NS row slots
+    const int lds = (NS + (gm && epl == 16 ? 1 : 0)) * 2 * epl * nthreads;   // NS row slots, and the RMSNorm's weight
     if (lds > usable) { err = hipErrorInvalidValue; return; }
     int per_cu = usable / lds;
     per_cu = per_cu > max_per_cu ? max_per_cu : per_cu;
@@ -479,7 +524,7 @@ hipError_t launch_reorder_quant(const void* x, const int16_t* idx, int rows, int
     err = allow_dynamic_lds(reinterpret_cast<const void*>(kernel), usable);
     if (err != hipSuccess) return;
     hipLaunchKernelGGL(kernel, dim3(grid), dim3(nthreads), (size_t)lds, stream, xb, idx, rows, K, KN, KS, KO, qn, qs, qo, sfn,
-                       sfs, sfo, sched, gm, eps, src_rows);
+                       sfs, sfo, sched, gm, eps, 1.0 / K, src_rows);
     err = hipGetLastError();
   };
   // Measured on M = 4096 ... 16384 rows of K = 3584 ... 18944: two row slots per workgroup, and per CU up to four
