@@ -71,6 +71,14 @@ int mg_reorder_quantize_w(const void* w_bf16, const int16_t* idx, int N, int K, 
 int mg_reorder_quantize_w_tiled(const void* w_bf16, const int16_t* reorder_index, int n, int N, int K, int KN, int KS, int KO,
                                 uint8_t* qn, uint8_t* qs, uint8_t* qo, uint8_t* sfn, uint8_t* sfs, uint8_t* sfo, void* stream);
 
+/* mg_reorder_quantize_w (N = n) or, with MG_FLAG_W_TILED, mg_reorder_quantize_w_tiled, which also looks at the index: soon after
+ * it starts, and not only when it is done, the launch writes verdict[0 ... 15], each 1 or 2; all of them are 1 if every entry
+ * lies in [0, K).  verdict is memory that the GPU can write and the host reads while the launch runs (hipHostMalloc), all 0
+ * before the call. */
+int mg_pack_weights(const void* w_bf16, const int16_t* reorder_index, int n, int N, int K, int KN, int KS, int KO, unsigned flags,
+                    uint8_t* qn, uint8_t* qs, uint8_t* qo, uint8_t* sfn, uint8_t* sfs, uint8_t* sfo, uint32_t* verdict,
+                    void* stream);
+
 /*
  * mg_reorder_quantize_x with an RMSNorm in front, in the same pass over the rows (the layer that feeds
  * a quantized linear in a transformer block; the reference leaves it to the caller and reads the

@@ -20,10 +20,11 @@ HOST_PATH = os.path.join(_PKG, "lib", "mixedgemm_torch.so")
 MG_OPERAND_A = 0
 MG_OPERAND_B = 1
 MG_FLAG_W_TILED = 1
+MG_OK, MG_ERR_BAD_INDEX = 0, 10003
 
 SYMBOLS = (
     "mg_reorder_quantize_x", "mg_reorder_quantize_w", "mg_mixed_gemm", "mg_mixed_gemm_ex", "mg_padded_rows", "mg_tile_weights",
-    "mg_reorder_quantize_w_tiled",
+    "mg_reorder_quantize_w_tiled", "mg_pack_weights",
     "mg_weights_tileable", "mg_fused_linear_ex", "mg_rmsnorm_reorder_quantize_x", "mg_fused_norm_linear",
     "mg_fused_linear",
     "mg_fused_workspace_bytes", "mg_sf_bytes", "mg_sf_offset", "mg_device_synchronize", "mg_status_string",
@@ -258,6 +259,20 @@ def reorder_quantize_w_tiled(w, reorder_index, kn, ks, ko):
                                                _stream(w))
     check(status, "mg_reorder_quantize_w_tiled")
     return out
+
+
+def pack_weights(w, reorder_index, kn, ks, ko, tiled):
+    """reorder_quantize_w_tiled or reorder_quantize_w, and check_reorder_index: returns once the index is known to be good, with
+    the launch still running."""
+    _index_entries(reorder_index, w.shape[1])
+    got = host().pack(w, reorder_index, kn, ks, ko, tiled)
+    if got is not None:
+        check(MG_OK if got[1] else MG_ERR_BAD_INDEX, "mg_check_reorder_index")
+        return got[0]
+    finish = start_check_reorder_index(reorder_index, w.shape[1])   # (the kernels read any index safely)
+    q = (reorder_quantize_w_tiled if tiled else reorder_quantize_w)(w, reorder_index, kn, ks, ko)
+    finish()
+    return q
 
 
 def matmul(an, bn, as_, bs, ao, bo, sfan, sfbn, sfas, sfbs, sfao, sfbo, out=None, w_tiled=False):

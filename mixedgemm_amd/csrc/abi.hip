@@ -11,7 +11,7 @@ namespace mg {
 template <bool IS_W>
 hipError_t launch_reorder_quant(const void* x, const int16_t* idx, int rows, int K, int KN, int KS, int KO, uint8_t* qn,
                                 uint8_t* qs, uint8_t* qo, uint8_t* sfn, uint8_t* sfs, uint8_t* sfo, const void* gamma,
-                                float eps, bool keep_codes, int src_rows, hipStream_t stream);
+                                float eps, bool keep_codes, int src_rows, unsigned* verdict, hipStream_t stream);
 hipError_t launch_mixed_gemm(const uint8_t* an, const uint8_t* bn, const uint8_t* as_, const uint8_t* bs,
                              const uint8_t* ao, const uint8_t* bo, const uint8_t* sfan, const uint8_t* sfbn,
                              const uint8_t* sfas, const uint8_t* sfbs, const uint8_t* sfao, const uint8_t* sfbo, int M,
@@ -43,7 +43,8 @@ int check_split(int rows, int KN, int KS, int KO) {
 template <bool IS_W>
 int reorder_quantize(const void* x, const int16_t* idx, int rows, int K, int KN, int KS, int KO, uint8_t* qn,
                      uint8_t* qs, uint8_t* qo, uint8_t* sfn, uint8_t* sfs, uint8_t* sfo, void* stream,
-                     const void* gamma = nullptr, float eps = 0.0f, bool keep_codes = false, int src_rows = 0) {
+                     const void* gamma = nullptr, float eps = 0.0f, bool keep_codes = false, int src_rows = 0,
+                     unsigned* verdict = nullptr) {
   if (int s = check_split(rows, KN, KS, KO)) return s;
   if (K != KN + KS + KO) return MG_ERR_BAD_SHAPE;
   if (rows == 0 || K == 0) return MG_OK;
@@ -51,7 +52,7 @@ int reorder_quantize(const void* x, const int16_t* idx, int rows, int K, int KN,
   if (!ptr_ok(qn, KN > 0) || !ptr_ok(qs, KS > 0) || !ptr_ok(qo, KO > 0)) return MG_ERR_BAD_POINTER;
   if ((KN > 0 && !sfn) || (KS > 0 && !sfs) || (KO > 0 && !sfo)) return MG_ERR_BAD_POINTER;
   return (int)mg::launch_reorder_quant<IS_W>(x, idx, rows, K, KN, KS, KO, qn, qs, qo, sfn, sfs, sfo, gamma, eps, keep_codes, src_rows,
-                                             static_cast<hipStream_t>(stream));
+                                             verdict, static_cast<hipStream_t>(stream));
 }
 
 size_t align256(size_t v) { return (v + 255) & ~(size_t)255; }
@@ -132,6 +133,14 @@ int mg_reorder_quantize_w_tiled(const void* w_bf16, const int16_t* idx, int n, i
   if (int s = check_split(N, KN, KS, KO)) return s;
   if (n <= 0 || n > N || N - n >= 256 || N % 256 != 0) return MG_ERR_BAD_SHAPE;
   return reorder_quantize<true>(w_bf16, idx, N, K, KN, KS, KO, qn, qs, qo, sfn, sfs, sfo, stream, nullptr, 0.0f, false, n);
+}
+
+int mg_pack_weights(const void* w_bf16, const int16_t* idx, int n, int N, int K, int KN, int KS, int KO, unsigned flags, uint8_t* qn,
+                    uint8_t* qs, uint8_t* qo, uint8_t* sfn, uint8_t* sfs, uint8_t* sfo, uint32_t* verdict, void* stream) {
+  const bool tiled = (flags & MG_FLAG_W_TILED) != 0;
+  if ((flags & ~MG_FLAG_W_TILED) != 0 || n <= 0 || n > N || (tiled ? N - n >= 256 || N % 256 != 0 : n != N)) return MG_ERR_BAD_SHAPE;
+  if (verdict == nullptr || K <= 0) return verdict == nullptr ? MG_ERR_BAD_POINTER : MG_ERR_BAD_SHAPE;
+  return reorder_quantize<true>(w_bf16, idx, N, K, KN, KS, KO, qn, qs, qo, sfn, sfs, sfo, stream, nullptr, 0.0f, false, tiled ? n : 0, verdict);
 }
 
 int mg_mixed_gemm_ex(const uint8_t* an, const uint8_t* bn, const uint8_t* as_, const uint8_t* bs, const uint8_t* ao,

@@ -211,7 +211,8 @@ __global__ void __launch_bounds__(MAXT)
 reorder_quant_dma_kernel(const uint8_t* __restrict__ x, const int16_t* __restrict__ idx, int rows, int K, int KN, int KS,
                          int KO, uint8_t* __restrict__ qn, uint8_t* __restrict__ qs, uint8_t* __restrict__ qo,
                          uint8_t* __restrict__ sfn, uint8_t* __restrict__ sfs, uint8_t* __restrict__ sfo, RowSchedule sched,
-                         const uint16_t* __restrict__ gamma, float eps, double inv_k, int src_rows) {
+                         const uint16_t* __restrict__ gamma, float eps, double inv_k, int src_rows,
+                         unsigned* __restrict__ verdict) {
   extern __shared__ __align__(16) uint8_t lds[];
   __shared__ double row_sums[NORM ? 2 : 1][NORM ? MAXT / 64 : 1];   // RMSNorm: the waves' sums of squares, by row parity
   static_assert(EPL == 32 || EPL == 16, "one or two lanes per block");
@@ -331,6 +332,22 @@ reorder_quant_dma_kernel(const uint8_t* __restrict__ x, const int16_t* __restric
   wait_vm(kPieces * min(NS, count) + (kLate ? kPieces : 0));
   if constexpr (kPieces == 4) asm volatile("" : "+v"(iv[0]), "+v"(iv[1]), "+v"(iv[2]), "+v"(iv[3]));
   else asm volatile("" : "+v"(iv[0]), "+v"(iv[1]));
+  // Is the index good?  A workgroup has all of it in its registers: the first one says so while its first rows arrive, every
+  // wave for its part, in 16 words of host memory which the caller watches.  (A store that the counts of what is in flight leave
+  // out makes their waits stricter, not laxer.)  N = 14336, K = 4096 with the entries copied to the host in front of the kernel,
+  // 3.5 us and a gap on either side: 41.1 us, now 29.5.
+  if constexpr (IS_W) {
+    if (verdict != nullptr && blockIdx.x == 0) {
+      bool bad = false;
+#pragma unroll
+      for (int q = 0; q < kPieces; ++q)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) bad |= (iv[q][e] & 0xffffu) >= (unsigned)K || (iv[q][e] >> 16) >= (unsigned)K;
+      const unsigned word = __builtin_amdgcn_ballot_w64(bad) != 0 ? 2u : 1u;
+      const int lane = tid & 63;
+      if (lane < 16 && lane % (nthr >> 6) == wave) __hip_atomic_store(verdict + lane, word, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+    }
+  }
   // LDS byte addresses of the lane's gathered channels in slot 0.  An entry outside [0, K) is read as
   // channel K - 1, so that the gather stays inside the row whatever the index holds.
   unsigned ga[kParts][16];
@@ -490,13 +507,13 @@ reorder_quant_dma_kernel(const uint8_t* __restrict__ x, const int16_t* __restric
 }  // namespace
 
 // gamma != nullptr: RMSNorm with that weight and eps before the gather (activations only).  src_rows != 0 (weights only):
-// codes in tile-major order, x has src_rows rows and the result `rows`, a multiple of 256.
+// codes in tile-major order, x has src_rows rows and the result `rows`, a multiple of 256.  verdict (weights only): 16 words, see the kernel.
 template <bool IS_W>
 hipError_t launch_reorder_quant(const void* x, const int16_t* idx, int rows, int K, int KN, int KS, int KO, uint8_t* qn,
                                 uint8_t* qs, uint8_t* qo, uint8_t* sfn, uint8_t* sfs, uint8_t* sfo,
-                                const void* gamma, float eps, bool keep_codes, int src_rows, hipStream_t stream) {
+                                const void* gamma, float eps, bool keep_codes, int src_rows, unsigned* verdict, hipStream_t stream) {
   if (rows == 0 || K == 0) return hipSuccess;
-  if ((gamma != nullptr && IS_W) || (src_rows != 0 && (!IS_W || src_rows > rows || rows % 256 != 0))) return hipErrorInvalidValue;
+  if ((gamma != nullptr && IS_W) || (verdict != nullptr && !IS_W) || (src_rows != 0 && (!IS_W || src_rows > rows || rows % 256 != 0))) return hipErrorInvalidValue;
   const uint16_t* gm = static_cast<const uint16_t*>(gamma);
   const int threads = ((K >> 5) + 63) & ~63;
   const uint8_t* xb = static_cast<const uint8_t*>(x);
@@ -524,7 +541,7 @@ hipError_t launch_reorder_quant(const void* x, const int16_t* idx, int rows, int
     err = allow_dynamic_lds(reinterpret_cast<const void*>(kernel), usable);
     if (err != hipSuccess) return;
     hipLaunchKernelGGL(kernel, dim3(grid), dim3(nthreads), (size_t)lds, stream, xb, idx, rows, K, KN, KS, KO, qn, qs, qo, sfn,
-                       sfs, sfo, sched, gm, eps, 1.0 / K, src_rows);
+                       sfs, sfo, sched, gm, eps, 1.0 / K, src_rows, verdict);
     err = hipGetLastError();
   };
   // Measured on M = 4096 ... 16384 rows of K = 3584 ... 18944: two row slots per workgroup, and per CU up to four
@@ -578,8 +595,8 @@ hipError_t launch_reorder_quant(const void* x, const int16_t* idx, int rows, int
 }
 
 template hipError_t launch_reorder_quant<false>(const void*, const int16_t*, int, int, int, int, int, uint8_t*, uint8_t*,
-                                                uint8_t*, uint8_t*, uint8_t*, uint8_t*, const void*, float, bool, int, hipStream_t);
+                                                uint8_t*, uint8_t*, uint8_t*, uint8_t*, const void*, float, bool, int, unsigned*, hipStream_t);
 template hipError_t launch_reorder_quant<true>(const void*, const int16_t*, int, int, int, int, int, uint8_t*, uint8_t*,
-                                               uint8_t*, uint8_t*, uint8_t*, uint8_t*, const void*, float, bool, int, hipStream_t);
+                                               uint8_t*, uint8_t*, uint8_t*, uint8_t*, const void*, float, bool, int, unsigned*, hipStream_t);
 
 }  // namespace mg

@@ -21,7 +21,10 @@
 #include <ATen/record_function.h>
 #include <c10/core/impl/LocalDispatchKeySet.h>
 #include <c10/hip/HIPGuard.h>
+#include <c10/hip/HIPGraphsC10Utils.h>
 #include <c10/hip/HIPStream.h>
+
+#include <immintrin.h>
 
 #include <optional>
 
@@ -212,6 +215,46 @@ std::optional<Six> reorder_quantize(const Tensor& t, const Tensor& index, int64_
   return q;
 }
 
+// Quantized weights and whether every entry of the index lies inside, as the launch says soon after it has started: the call
+// returns when it has, with the launch still running.  Not taken in a stream capture, where it does not start.
+struct Packed {
+  Six q;
+  bool index_ok;
+};
+std::optional<Packed> pack(const Tensor& t, const Tensor& index, int64_t kn, int64_t ks, int64_t ko, bool tiled) {
+  const int64_t k = kn + ks + ko;
+  if (!split_ok(kn, ks, ko) || !on_gpu(t, at::kBFloat16) || t.dim() != 2 || t.size(1) != k || k == 0 || t.size(0) == 0)
+    return std::nullopt;
+  const at::Device device = t.device();
+  if (!on_gpu(index, at::kShort, device) || index.numel() != k) return std::nullopt;
+  const int64_t n = t.size(0), rows = tiled ? (n + 255) / 256 * 256 : n;
+  if (rows > INT32_MAX) return std::nullopt;
+  const c10::hip::HIPGuard guard(device.index());
+  if (c10::hip::currentStreamCaptureStatusMayInitCtx() != c10::hip::CaptureStatus::None) return std::nullopt;
+  const c10::hip::HIPStream stream = c10::hip::getCurrentHIPStream(device.index());
+  Packed p;
+  p.q = quant_outputs(rows, kn, ks, ko, MG_OPERAND_B, device);
+  const Tensor words = at::empty({16}, at::TensorOptions().dtype(at::kInt).pinned_memory(true));
+  volatile uint32_t* const verdict = static_cast<uint32_t*>(words.data_ptr());
+  for (int i = 0; i < 16; ++i) verdict[i] = 0;
+  const int status = mg_pack_weights(ptr<void>(t), ptr<int16_t>(index), (int)n, (int)rows, (int)k, (int)kn, (int)ks, (int)ko,
+                                     tiled ? MG_FLAG_W_TILED : 0u, ptr<uint8_t>(p.q[0]), ptr<uint8_t>(p.q[1]), ptr<uint8_t>(p.q[2]),
+                                     ptr<uint8_t>(p.q[3]), ptr<uint8_t>(p.q[4]), ptr<uint8_t>(p.q[5]), const_cast<uint32_t*>(verdict),
+                                     static_cast<void*>(stream.stream()));
+  if (!enqueued(status, "mg_pack_weights")) return std::nullopt;
+  p.index_ok = true;
+  bool ended = false;
+  for (int i = 0; i < 16; ++i) {
+    for (unsigned spins = 1; verdict[i] == 0; ++spins) {
+      TORCH_CHECK(!ended, "mixedgemm: the launch ended without a word about the reorder index");
+      if (spins % 1024 == 0) ended = stream.query();   // throws what the stream has failed with
+      _mm_pause();
+    }
+    p.index_ok &= verdict[i] == 1;
+  }
+  return p;
+}
+
 int64_t capacity(const Tensor& t) {
   return static_cast<int64_t>(t.storage().nbytes()) - t.storage_offset() * static_cast<int64_t>(t.element_size());
 }
@@ -392,6 +435,20 @@ PyObject* py_reorder_quantize(PyObject*, PyObject* const* a, Py_ssize_t n) {
   });
 }
 
+// (weight, reorder_index, kn, ks, ko, tiled) -> (the six tensors, whether the index is good)
+PyObject* py_pack(PyObject*, PyObject* const* a, Py_ssize_t n) {
+  return guarded([&]() -> PyObject* {
+    if (n != 6) throw NotTaken{};
+    const Tensor t = tensor_arg(a[0]), index = tensor_arg(a[1]);
+    const int64_t kn = int_arg(a[2]), ks = int_arg(a[3]), ko = int_arg(a[4]);
+    const bool tiled = a[5] == Py_True;
+    std::optional<Packed> p = unlocked([&] { return pack(t, index, kn, ks, ko, tiled); });
+    if (!p) return wrap(std::optional<Six>());
+    py::object q = py::reinterpret_steal<py::object>(wrap(std::optional<Six>(std::move(p->q))));
+    return py::make_tuple(q, p->index_ok).release().ptr();
+  });
+}
+
 // the twelve operands in the order of the reference's matmul, out, w_tiled
 PyObject* py_matmul(PyObject*, PyObject* const* a, Py_ssize_t n) {
   return guarded([&]() -> PyObject* {
@@ -421,6 +478,7 @@ PyMethodDef kMethods[] = {
     {"fused_linear", MG_FASTCALL(py_fused_linear), METH_FASTCALL, nullptr},
     {"layer", MG_FASTCALL(py_layer), METH_FASTCALL, nullptr},
     {"reorder_quantize", MG_FASTCALL(py_reorder_quantize), METH_FASTCALL, nullptr},
+    {"pack", MG_FASTCALL(py_pack), METH_FASTCALL, nullptr},
     {"matmul", MG_FASTCALL(py_matmul), METH_FASTCALL, nullptr},
     {"calibrate", MG_FASTCALL(py_calibrate), METH_FASTCALL, nullptr},
     {nullptr, nullptr, 0, nullptr}};

@@ -82,18 +82,13 @@ class PackedWeights:
         bindings.cpp:188-305); with `tile`, shapes that allow it are then put in tile-major order."""
         split = tuple(split) if split is not None else default_split(weight.shape[1])
         n = weight.shape[0]
-        check = abi.start_check_reorder_index(reorder_index, weight.shape[1])   # (the kernels read any index safely)
         # the whole-tile kernel wants a multiple of 256 features: zero rows are cheap, the layer drops their outputs
         stored = (n + 255) // 256 * 256
         if tile and (n == stored or n > 256) and abi.weights_tileable(stored, *split):
             if n != stored and (not weight.is_contiguous() or weight.data_ptr() % 16):
                 weight = weight.clone(memory_format=torch.contiguous_format)   # any view packs where rows are appended
-            q = abi.reorder_quantize_w_tiled(weight, reorder_index, *split)
-            pw = cls(*q, reorder_index, split, True, n if stored != n else 0)
-        else:
-            pw = cls(*abi.reorder_quantize_w(weight, reorder_index, *split), reorder_index, split)
-        check()
-        return pw
+            return cls(*abi.pack_weights(weight, reorder_index, *split, True), reorder_index, split, True, n if stored != n else 0)
+        return cls(*abi.pack_weights(weight, reorder_index, *split, False), reorder_index, split)
 
     def tileable(self) -> bool:
         return abi.weights_tileable(self.rows, *self.split)

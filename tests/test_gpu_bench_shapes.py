@@ -130,3 +130,34 @@ def test_out_of_range_index_is_reported_and_clamped(abi):
     got = abi.reorder_quantize_x(x.to(DEV), bad.to(DEV), kn, ks, ko)
     torch.cuda.synchronize()
     H.assert_quant_equal(got, sc.quantize_x(H.bf16_bits(x), clamped.numpy(), kn, ks, ko), rows, (kn, ks, ko), what="clamped index")
+
+
+# one wave; waves that share the 16 words unevenly (3, 13); one and two blocks per lane; the kernel of any workgroup size
+@pytest.mark.parametrize("rows,split,tiled", [(1, (32, 0, 0), False), (5, (1024, 512, 960), False), (300, (2048, 512, 1536), True),
+                                              (3, (8192, 2048, 2880), False), (257, (8192, 64, 128), True), (2, (20000 - 32, 512, 512), False),
+                                              (2, (30720, 1024, 992), False)])
+def test_packing_reports_a_bad_index(abi, rows, split, tiled):
+    """pack_weights: the tensors of the quantizer alone, and an entry outside [0, K) is refused wherever it stands."""
+    k = sum(split)
+    w = H.make_weights(rows, k, 5).to(DEV)
+    idx = H.random_index(k, 6)
+    got = abi.pack_weights(w, idx.to(DEV), *split, tiled)
+    want = (abi.reorder_quantize_w_tiled if tiled else abi.reorder_quantize_w)(w, idx.to(DEV), *split)
+    torch.cuda.synchronize()
+    stored = (rows + 255) // 256 * 256 if tiled else rows
+    for g, w_, kseg in zip(got, want, (*split, *split)):
+        assert g.shape == w_.shape
+        if g.dim() == 2:
+            assert torch.equal(g, w_), f"codes of {rows} x {split}"
+        else:
+            np.testing.assert_array_equal(H.gather_logical_scales(g, stored, kseg), H.gather_logical_scales(w_, stored, kseg))
+    for i, v in {0: -1, 1: k, k // 2: -32768, k // 3: 32767, k - 1: k if k < 32768 else -2}.items():
+        if 0 <= v < k:
+            continue
+        bad = idx.clone()
+        bad[i] = v
+        with pytest.raises(abi.MixedGemmError, match="out of range"):
+            abi.pack_weights(w, bad.to(DEV), *split, tiled)
+    with pytest.raises(abi.MixedGemmError):
+        abi.pack_weights(w, idx[:-1].contiguous().to(DEV), *split, tiled)
+    torch.cuda.synchronize()
