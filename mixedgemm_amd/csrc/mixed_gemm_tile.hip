@@ -675,17 +675,20 @@ struct TilePlanChoice { int tf, tt; double us; };
 // The tile with the lowest estimate.  A workgroup has its CU to itself (LDS), so a launch is rounds of them; microseconds: fixed,
 // per round, per stage and round, per stage with all CUs busy, per MB of results, per round with blocks past the whole stages.
 // Fitted to 450 measured calls each (17 ... 2600 tokens, N 384 ... 28672, K 1024 ... 18944, tile-major weights; rms error 10 %):
-// the tile taken is in the mean 0.5 % slower than the best of the three.
+// the tile taken is in the mean 0.5 % slower than the best of the three.  Long launches are held back by the clock that the power
+// limit leaves: no faster than the table's PFLOP/s on whole tiles (M = 1894, N = 8448, K = 13824: 198 us where the sum says 135, 170
+// on 256 x 256 tiles; over 55 calls of 35 ... 135 us the choice against those is then the faster one every time).
 TilePlanChoice mixed_gemm_tile_plan(int M, int N, int KN, int KS, int KO, int cus) {
-  static const struct { int tf, tt; double fixed, round, stage, fill, mb, rest; } kTiles[] = {
-      {128, 128, 2.87, -0.24, 0.260, 0.075, 0.41, 1.8}, {128, 64, 1.47, 1.29, 0.170, 0.051, 0.39, 1.0}, {64, 64, 1.55, 1.07, 0.125, 0.039, 0.46, 0.9}};
+  static const struct { int tf, tt; double fixed, round, stage, fill, mb, rest, pflops; } kTiles[] = {
+      {128, 128, 2.87, -0.24, 0.260, 0.075, 0.41, 1.8, 2.3}, {128, 64, 1.47, 1.29, 0.170, 0.051, 0.39, 1.0, 2.0}, {64, 64, 1.55, 1.07, 0.125, 0.039, 0.46, 0.9, 1.5}};
   const int stages = KN / 128 + KS / 128 + KO / 128;
   const bool rest = ((KN | KS | KO) & 127) != 0;
   TilePlanChoice best = {0, 0, 0.0};
   for (const auto& t : kTiles) {
     const int64_t tiles = (int64_t)ceil_div(N, t.tf) * ceil_div(M, t.tt);
     const double rounds = (double)((tiles + cus - 1) / cus), busy = tiles < cus ? (double)tiles / cus : 1.0;
-    const double us = t.fixed + rounds * (t.round + stages * t.stage + (rest ? t.rest : 0.0)) + stages * t.fill * busy + 2e-6 * M * N * t.mb;
+    const double power = 2e-9 * (double)tiles * t.tf * t.tt * (KN + KS + KO) / t.pflops;
+    const double us = fmax(power, t.fixed + rounds * (t.round + stages * t.stage + (rest ? t.rest : 0.0)) + stages * t.fill * busy + 2e-6 * M * N * t.mb);
     if (best.tf == 0 || us < best.us) best = {t.tf, t.tt, us};
   }
   return best;
