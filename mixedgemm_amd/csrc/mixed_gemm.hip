@@ -102,6 +102,7 @@ __device__ __forceinline__ v4f decode_mfma(v8i wb, v8i xa, v4f acc, int sw, int 
 template <int N>
 __device__ __forceinline__ void wait_vmcnt() { asm volatile("s_waitcnt vmcnt(%0)" : : "n"(N) : "memory"); }
 
+template <bool STREAM = false>
 __device__ __forceinline__ void dma16_at(const uint8_t* base, unsigned voff, unsigned lds_off) {
   // base and lds_off are wave-uniform; say so to the compiler
   const uint64_t bv = reinterpret_cast<uint64_t>(base);
@@ -110,8 +111,10 @@ __device__ __forceinline__ void dma16_at(const uint8_t* base, unsigned voff, uns
   const uint32_t hi = (uint32_t)__builtin_amdgcn_readfirstlane((uint32_t)(bv >> 32));
   base = reinterpret_cast<const uint8_t*>(((uint64_t)hi << 32) | lo);
   lds_off = __builtin_amdgcn_readfirstlane(lds_off);
-  asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1"
-               : : "v"(voff), "s"(base), "s"(lds_off) : "memory", "m0");
+  if constexpr (STREAM) asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1 nt"
+                                     : : "v"(voff), "s"(base), "s"(lds_off) : "memory", "m0");
+  else asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1"
+                    : : "v"(voff), "s"(base), "s"(lds_off) : "memory", "m0");
 }
 // the same with a 64-bit address per lane
 __device__ __forceinline__ void dma16_lane(const uint8_t* p, unsigned lds_off) {
@@ -134,6 +137,10 @@ mixed_gemm_skinny_kernel(DecodeSeg s4, DecodeSeg s6, DecodeSeg s8, int M, int N,
                          uint16_t* __restrict__ d) {
   constexpr int NS = kSkinnySlots<G, F>, kSlot = kSkinnySlot<G, F>;
   constexpr int PA = G == 1 ? 16 : 32, PB = 4 * F;   // scale pieces per step: tokens, weights
+  // The widest layers' weight codes, whole lines that nobody reads again, as streaming loads: they leave the last-level cache to
+  // what follows.  N = 28672, K = 4096, M = 16 from HBM 15.3 -> 14.2 us, 20480 13.4 -> 12.7 (from that cache 12.3 -> 13.3); a decoder
+  // layer's four projections of 16 tokens, whose others (58 MB) then stay in it, 62.5 -> 56.3.
+  constexpr bool kStream = WT && F == 8;
   static_assert(NS >= 3 && PA + PB <= 64, "a pipeline; one copy for all scales of a step");
   extern __shared__ __align__(16) uint8_t lds[];
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -204,7 +211,7 @@ mixed_gemm_skinny_kernel(DecodeSeg s4, DecodeSeg s6, DecodeSeg s8, int M, int N,
         // 16 KB per (256-feature tile, whole step), the group's block in it; the blocks past the last whole step as
         // rows of nblk % 4 blocks behind the tiled part
         const int whole = s.nblk >> 2;
-        if (q < whole) dma16_at(s.b + (((size_t)tile * whole + q) * 16 + j0 + f) * 1024, (unsigned)(lane >> 2) * 64u + wp, at);
+        if (q < whole) dma16_at<kStream>(s.b + (((size_t)tile * whole + q) * 16 + j0 + f) * 1024, (unsigned)(lane >> 2) * 64u + wp, at);
         else dma16_at(s.b + (size_t)(N >> 8) * whole * 16384, (unsigned)wrow[f] * (unsigned)(s.nblk & 3) * 16u + wp, at);
       } else {
         dma16_at(s.b + (size_t)q * 64, (unsigned)wrow[f] * (unsigned)s.nblk * 16u + wp, at);
@@ -1002,15 +1009,20 @@ static bool decode_lds_plan(const DecodeSeg& d4, const DecodeSeg& d6, const Deco
 //   row-major, N = 4096, K = 14336: M = 16 8.5 against 9.8 / 12.7 us, 128 18.4 against 20.7 / 25.6, 200 37 against 35 / 40;
 //     N = 5120, K = 5120: M = 8 5.8 against 6.4 / 8.1, 128 18.1 against 17.3 / 18.8;  N = 14336, K = 4096, M = 64 15.7
 //     against 16.3 / 20.5
+// Eight feature groups are for 64 to 128 features per CU and up to 16 tokens, where four need a second round (from HBM, M = 16,
+// tile-major / row-major weights, us): N = 20480, K = 5120 19.3 -> 16.3 / 23.6 -> 20.6, N = 28672, K = 5120 22.0 -> 17.1 / 25.9 -> 22.6, N =
+// 18944, K = 3584 15.7 -> 11.6.  Up to 64 features per CU they are slower (N = 16384, K = 5120 15.2 against 12.3), and so they are
+// with two token groups (M = 32, N = 24576, K = 8192 21.4 against 19.1 on small tiles).
 // Over 1511 calls of 17 to 255 tokens (N 256 ... 28672, K 1024 ... 18944) the form taken, whole tiles included, is in the
 // mean 1.2 / 3.0 % (row-major) and 2.0 / 3.2 % (tile-major) slower than the best one, 22 / 60 % and 27 / 40 % at most; with the
 // tile-major figures row-major weights were at 3.0 / 5.2 and 68 / 77 %.
 struct SkinnyPlan { int g, f; double us; };
 static SkinnyPlan skinny_plan(int M, int N, int steps, int cus, bool w_tiled) {
   static const struct { int g, f; double ns[2]; } kForms[] = {   // row-major, tile-major weights
-      {1, 1, {46, 67}}, {1, 2, {62, 77}}, {1, 4, {104, 102}}, {2, 2, {89, 86}}, {2, 4, {145, 117}}, {4, 2, {134, 110}}};
+      {1, 1, {46, 67}}, {1, 2, {62, 77}}, {1, 4, {104, 102}}, {2, 2, {89, 86}}, {2, 4, {145, 117}}, {4, 2, {134, 110}}, {1, 8, {230, 225}}};
   SkinnyPlan best = {0, 0, 0.0};
   for (const auto& k : kForms) {
+    if (k.f == 8 && M > 16) continue;
     const int across = w_tiled ? ceil_div(N, 16 * k.f) : ceil_div(N, 128) * (8 / k.f);
     const int rounds = (int)(((int64_t)across * ceil_div(M, 16 * k.g) + cus - 1) / cus);
     const double us = 1.0 + rounds * (2.3 + steps * k.ns[w_tiled] * 1e-3) + 1.5 * (rounds - 1);
@@ -1021,19 +1033,20 @@ static SkinnyPlan skinny_plan(int M, int N, int steps, int cus, bool w_tiled) {
 
 // The decode kernel, which brings the tokens' codes and all scales into LDS once per workgroup, for up to 16 tokens and
 // whole 128-wide steps: its feature groups of 16 per workgroup, or 0 where another kernel is taken.
-// Measured against the skinny kernel on tile-major weights, K = 4096:
-//   N = 4096 (1 feature group per workgroup): M = 1 4.8 against 5.3 us, 8 5.3 against 5.4, 16 5.5 against 5.3 (two layers'
-//     weights in turn; from HBM 5.6 against 5.8, 5.9 against 6.1);
-//   N = 6144 (1, a second round of workgroups): M = 8 6.2 against 5.8;
-//   N = 14336 (4): M = 8 7.5 against 8.3, 16 8.0 against 8.6;  N = 28672 (4, two per CU): 12.6 / 13.6 against 14.8 / 15.3.
-// So: four feature groups (two such workgroups fit a CU; 9.0 against 9.6 us with two groups at N = 14336), or one round
-// of workgroups and at most 8 tokens.
-// On row-major weights the skinny kernel is ahead or level up to 64 features per CU (in the caches / from HBM, N = 4096, K =
-// 4096, M = 1: 5.1 against 5.6 / 5.4 against 5.7 us; N = 14336, M = 8: 8.4 against 9.0 / 10.4 against 10.3, 16: 8.6 against
-// 9.3 / 10.9 against 10.7), then needs a second round, where two workgroups of this kernel with two feature groups fit a CU: N = 18944,
-// K = 3584: M = 8 10.7 against 12.2 / 12.5 against 15.5, 16 11.9 against 12.8 / 13.5 against 16.3; K = 12288, M = 1 26.6 against
-// 31.4 / 29.7 against 38.6; N = 28672, K = 4096, M = 16 17.1 against 18.4 / 18.1 against 19.8 (K = 8192, M = 8, in the caches, the
-// exception: 26.2 against 23.3).
+// Against the skinny kernel on tile-major weights, K = 4096, from the caches / from HBM (layers of 120 and of 700 MB in turn, us):
+//   N = 4096 (1 feature group per workgroup): M = 4 5.3 against 5.5 / 5.5 against 5.9, 16 (skinny) 5.5 against 5.3 / 5.8 against 6.6;
+//   N = 14336 (4): M = 8 8.9 against 8.6 / 8.7 against 9.4, 16 9.3 against 8.8 / 9.2 against 10.1;
+//   N = 28672 (4, two per CU; skinny with 8): M = 4 12.4 against 12.1 / 14.0 against 14.2, 16 13.3 against 13.3 / 15.3 against 14.2;
+//   K = 8192, M = 4: N = 4096 8.6 against 7.7 / 8.7 against 8.1, 14336 15.6 against 13.1 / 14.5 against 14.9;
+//   N = 18944, M = 16: K = 1024 7.8 against 7.2 / 7.2 against 6.7, 2048 8.9 against 8.8 / 8.8 against 8.7 (N = 28672: 8.7 against
+//     9.5 / 9.1 against 9.6), 2560 12.0 against 9.7 / 12.1 against 9.7;  N = 36864, K = 3584, M = 16 18.7 against 20.9 / 19.0 against 23.1.
+// So: four feature groups (two such workgroups fit a CU), or one round of workgroups and at most 8 tokens; up to 32 K steps, so
+// that all of a wave's weights are in flight at once; up to 16 where the skinny kernel has eight feature groups; above 128
+// features per CU, where that needs two rounds, always.
+// On row-major weights the skinny kernel is ahead or level up to 64 features per CU (N = 4096, K = 4096, M = 1: 5.1 against 5.6 / 5.4
+// against 5.7; N = 14336, M = 16: 8.6 against 9.3 / 11.1 against 10.7), then needs eight feature groups or a second round, where two
+// workgroups of this kernel with two feature groups fit a CU: N = 18944, M = 16: K = 2048 8.0 against 7.9 / 8.8 against 9.6, K = 3584
+// 11.9 against 10.6 / 13.6 against 14.9, K = 4096 - / 14.0 against 16.1.
 // The whole-tile kernel was slower than the form taken here at every shape measured (N = 28672, K = 2048: 11.4 against 8.8).
 // (a segment's weight codes below 4 GB: the kernel addresses them with 32-bit per-lane offsets)
 static int decode_plan(const DecodeSeg& d4, const DecodeSeg& d6, const DecodeSeg& d8, int M, int N, bool w_tiled, int cus,
@@ -1042,8 +1055,10 @@ static int decode_plan(const DecodeSeg& d4, const DecodeSeg& d6, const DecodeSeg
   if (M > 16 || widest == 0 || ((d4.nblk | d6.nblk | d8.nblk) & 3) != 0 || (size_t)N * widest * 16 >= ((size_t)1 << 32)) return 0;
   int f = 2;
   if (w_tiled) {
+    const int steps = d4.steps + d6.steps + d8.steps;
     f = ceil_div(N, 64) >= cus * 3 / 4 ? 4 : (ceil_div(N, 32) >= cus ? 2 : 1);
     if (f < 4 && (M > 8 || ceil_div(N, 16 * f) > cus)) return 0;
+    if (ceil_div(N, 128) <= cus && steps > (ceil_div(N, 64) <= cus ? 32 : 16)) return 0;
   } else if (ceil_div(N, 128) * 2 <= cus) {
     return 0;
   }
@@ -1078,9 +1093,10 @@ hipError_t launch_skinny(const DecodeSeg& d4, const DecodeSeg& d6, const DecodeS
   const std::integral_constant<int, 1> one;
   const std::integral_constant<int, 2> two;
   const std::integral_constant<int, 4> four;
+  const std::integral_constant<int, 8> eight;
   if (plan.g == 4) return launch(four, two);
   if (plan.g == 2) return plan.f == 4 ? launch(two, four) : launch(two, two);
-  return plan.f == 4 ? launch(one, four) : (plan.f == 2 ? launch(one, two) : launch(one, one));
+  return plan.f == 8 ? launch(one, eight) : plan.f == 4 ? launch(one, four) : (plan.f == 2 ? launch(one, two) : launch(one, one));
 }
 
 }  // namespace
@@ -1102,28 +1118,26 @@ hipError_t launch_mixed_gemm_tile(const uint8_t* an, const uint8_t* bn, const ui
                                   int m_store, int a_rows, int N, int KN, int KS, int KO, bool w_tiled, const TilePlanChoice& choice,
                                   Epilogue ep, void* d, hipStream_t stream);
 
-// Rough launch time of the whole-tile kernel in microseconds, only to choose between the kernels for fewer than 256
-// tokens (measured on MI355X, 256 CUs).  It runs such problems as 256 x 128 tiles when that is at most one round: ~2.5 us
-// plus, per 128-wide stage, ~0.42 us on tile-major weights with at most half of the CUs busy and ~0.45 us with more; on
-// row-major ones, whose copies touch twice the lines, 0.49 us and 2.7 ns more for every workgroup that shares the memory (all
-// of it with weights in the caches; 0.59 and 0.78 us a stage when they come from HBM).  As 256 x 256 tiles ~0.95 us a stage
-// plus ~3 us a round otherwise.  Against it the skinny kernel, measured:
-//   tile-major, N = 18944, K = 3584: M = 32 14.9 against 15.5 us, 64 15.1 against 21.5; N = 4096, K = 14336, M = 200: 31 against 47
-//   row-major, N = 14336, K = 12288, M = 91: 55 against 73; N = 9600, K = 2656, M = 63: 12.5 against 16.7; N = 8192, K = 3584, M =
-//     191: 20.4 against 17.5
-static double pipelined_us(int M, int N, int stages, int cus, bool w_tiled) {
+// Rough launch time of the whole-tile kernel in microseconds for fewer than 256 tokens, only to choose between the kernels: as
+// 256 x 128 tiles when that is at most one round (fitted to 771 calls on tile-major weights, rms error 8 %), else as 256 x 256.
+// What the blocks past whole stages, the hand-over between three segments and an E3M2 segment shorter than its pipeline cost is
+// counted: with 4.5 us for the last (K = 1024: N = 24576, M = 64 was 12.9 us here, and is 6.4 on small tiles).
+static bool short_middle(int KN, int KS, int KO) { return KN > 0 && KO > 0 && KS > 0 && KS < 384; }
+static double pipelined_us(int M, int N, int stages, int KN, int KS, int KO, int cus) {
   const int whole = ceil_div(M, 256) * ceil_div(N, 256), halves = ceil_div(M, 128) * ceil_div(N, 256);
-  if (whole <= cus / 2) return stages * (w_tiled ? (halves <= cus / 2 ? 0.42 : 0.45) : 0.487 + 0.0027 * halves) + 2.5;
-  return (double)ceil_div(whole, cus) * (stages * 0.95 + 3.0);
+  if (whole > cus / 2) return (double)ceil_div(whole, cus) * (stages * 0.95 + 3.0);
+  return 1.9 + stages * (0.342 + 0.28 * fmin(1.0, (double)halves / cus)) + ((KN | KS | KO) % 128 != 0 ? 1.0 : 0.0) +
+         (KN > 0 && KS > 0 && KO > 0 ? 2.0 : 0.0) + (short_middle(KN, KS, KO) ? 4.5 : 0.0);
 }
 
 // The same on tile-major weights for 256 tokens and more, fitted to 184 measured calls (rms error 7 %): half tiles (at most cus / 2
 // whole ones) or rounds of whole tiles, of which a last one on at most half of the CUs counts 0.62; microseconds per stage, per
 // MB of results, and what the blocks past whole stages cost.
-static double whole_tiles_us(int M, int N, int stages, bool rest, bool three_segments, int cus) {
+static double whole_tiles_us(int M, int N, int stages, int KN, int KS, int KO, int cus) {
+  const bool rest = (KN | KS | KO) % 128 != 0, three_segments = KN > 0 && KS > 0 && KO > 0;
   const int whole = ceil_div(M, 256) * ceil_div(N, 256), halves = ceil_div(M, 128) * ceil_div(N, 256);
   const double mb = 2e-6 * M * N;
-  if (whole <= cus / 2) return 3.8 + stages * (0.346 + 0.084 * fmin(1.0, (double)halves / cus)) + 0.26 * mb + (rest ? 2.0 : 0.0);
+  if (whole <= cus / 2) return 3.8 + stages * (0.346 + 0.084 * fmin(1.0, (double)halves / cus)) + 0.26 * mb + (rest ? 2.0 : 0.0) + (short_middle(KN, KS, KO) ? 4.5 : 0.0);
   const int full = whole / cus, left = whole % cus;
   const double rounds = full + (left == 0 ? 0.0 : (left <= cus / 2 && full > 0 && three_segments ? 0.62 : 1.0));
   return fmax(1.4 + rounds * (stages * 0.741 - 7.0 + (rest ? 2.5 : 0.0)) + 0.63 * mb, rounds * stages * 0.6);
@@ -1158,16 +1172,16 @@ hipError_t launch_mixed_gemm(const uint8_t* an, const uint8_t* bn, const uint8_t
   // Small tiles where they are estimated to be the fastest by a margin (the estimates of both sides are off by 10 %), and for
   // what no other kernel takes.  Both weight layouts go the same way: the estimates compared are those on tile-major weights.
   const TilePlanChoice tile = mixed_gemm_tile_plan(M, N, KN, KS, KO, lim.cus);
-  const double others = few ? (whole_tiles ? fmin(pipelined_us(M, N, steps, lim.cus, true), skinny_plan(M, N, steps, lim.cus, true).us)
-                                           : skinny_plan(M, N, steps, lim.cus, true).us)
-                            : whole_tiles_us(M, N, steps, (KN | KS | KO) % 128 != 0, KN > 0 && KS > 0 && KO > 0, lim.cus);
+  const SkinnyPlan skinny_t = few ? skinny_plan(M, N, steps, lim.cus, true) : SkinnyPlan{0, 0, 0.0};
+  const double whole_us = few ? pipelined_us(M, N, steps, KN, KS, KO, lim.cus) : whole_tiles_us(M, N, steps, KN, KS, KO, lim.cus);
+  const double others = few ? (whole_tiles ? fmin(whole_us, skinny_t.us) : skinny_t.us) : whole_us;
   if ((M > 16 || !few) && ((!whole_tiles && !skinny_ok) || tile.us < 0.95 * others))
     return launch_mixed_gemm_tile(an, bn, as_, bs, ao, bo, sfan, sfbn, sfas, sfbs, sfao, sfbo, M, a_rows, N, KN, KS, KO, w_tiled, tile,
                                   ep, d, stream);
-  const SkinnyPlan skinny = skinny_ok ? skinny_plan(M, N, steps, lim.cus, w_tiled) : SkinnyPlan{0, 0, 0.0};
+  const SkinnyPlan skinny = skinny_ok && !w_tiled ? skinny_plan(M, N, steps, lim.cus, false) : skinny_t;
   // whole 256-row tiles; the last one does not write rows past M and reads no activation row past
   // a_rows (lanes that would are pointed at the last readable row)
-  if (whole_tiles && (!skinny_ok || pipelined_us(M, N, steps, lim.cus, w_tiled) < skinny.us))
+  if (whole_tiles && (!skinny_ok || whole_us < skinny.us))
     return launch_mixed_gemm_256(an, bn, as_, bs, ao, bo, sfan, sfbn, sfas, sfbs, sfao, sfbo, M, a_rows, N, KN, KS, KO,
                                  w_tiled, ep, d, stream);
   return launch_skinny(d4, d6, d8, M, N, w_tiled, skinny, ep, static_cast<uint16_t*>(d), stream);

@@ -203,9 +203,8 @@ DECODE_SHAPES = [
     # needs a CU's whole LDS (and fewer feature groups per workgroup for 16 tokens)
     (8, 512, 416, 480, 160), (16, 768, 160, 224, 352), (4, 1024, 480, 448, 192), (9, 520, 64, 96, 32),
     (8, 4096, 8960, 4928, 448), (16, 4096, 7680, 4224, 384), (1, 3584, 11776, 6560, 608),
-    # the decode kernel with two feature groups per workgroup: row-major weights of more than 64 features per CU (1, 8, 9 and 16
-    # tokens, a ragged last group of rows, an empty segment, K beyond the first two rounds of steps), and the tile-major
-    # width that has a workgroup per CU with two groups; at most 8 and more tokens on the widest tile-major layers
+    # more than 64 features per CU (1, 8, 9 and 16 tokens, a ragged last group of rows, an empty segment, many steps per wave), and
+    # the tile-major width that has a workgroup of the decode kernel per CU with two groups
     (1, 18944, 384, 0, 128), (8, 16520, 384, 384, 128), (9, 16888, 128, 128, 128), (16, 18944, 512, 384, 128), (5, 16392, 2560, 1536, 512),
     (8, 8192, 640, 512, 384), (5, 8192, 2560, 1408, 128), (4, 28672, 1280, 640, 128), (16, 28672, 256, 128, 128),
 ]
@@ -596,6 +595,23 @@ def test_skinny_kernel_at_the_edges_of_its_pipeline(abi, m, n, kn, ks, ko):
         test_small_batches_match_oracle(abi, m, n, kn, ks, ko, True)
 
 
+# Up to 16 tokens on more than 64 features per CU.  Up to 128: the skinny kernel with eight feature groups (a ragged last group of
+# 128 rows, whole tiles, 1 to 3 blocks past whole steps, fewer steps than waves, an empty segment).  More: the decode kernel with
+# four and two feature groups, from the first width on, and the skinny kernel where a segment is not whole steps.  On both layouts
+# of the weights, which give the same bits where one kernel takes both.
+WIDE_SHAPES = [
+    (1, 16392, 384, 0, 128), (16, 16640, 416, 224, 160), (9, 18944, 640, 384, 128), (3, 18943, 64, 32, 96), (8, 32768, 128, 128, 128),
+    (2, 20480, 2560, 1408, 128), (1, 32776, 384, 0, 128), (16, 33024, 256, 128, 128), (9, 33024, 416, 0, 0), (8, 33000, 1152, 640, 256),
+]
+
+
+@pytest.mark.parametrize("m,n,kn,ks,ko", WIDE_SHAPES)
+def test_few_tokens_on_many_features(abi, m, n, kn, ks, ko):
+    test_small_batches_match_oracle(abi, m, n, kn, ks, ko, False)
+    if abi.weights_tileable(n, kn, ks, ko):
+        test_small_batches_match_oracle(abi, m, n, kn, ks, ko, True)
+
+
 # Codes and scales of the one-pass weight packing against quantizing (with rows of zeros) and tiling one after the other:
 # whole tiles and a last tile of 1, 8 and 255 rows, one and two lanes per block, a run-time workgroup size (K > 20480),
 # and 1 to 3 blocks past a segment's last whole step.
@@ -728,7 +744,7 @@ SMALL_TILE_SHAPES = [
     (256, 256, 128, 128, 128), (257, 264, 128, 0, 0), (319, 1000, 0, 256, 128), (320, 520, 640, 384, 128), (321, 768, 1152, 640, 256),
     (450, 1001, 1152, 640, 256), (300, 60, 416, 224, 96), (300, 40, 64, 32, 0), (511, 1280, 480, 480, 480), (256, 8, 32, 0, 0),
     (300, 5120, 256, 160, 128), (384, 4352, 640, 416, 128), (385, 4100, 640, 384, 128), (512, 2816, 0, 0, 640),
-    (260, 6656, 384, 160, 128), (513, 3584, 384, 384, 384), (640, 3080, 1024, 0, 128), (385, 6400, 448, 416, 224), (257, 6401, 640, 256, 0),
+    (260, 6656, 384, 160, 128), (64, 8192, 640, 256, 128), (200, 1032, 640, 256, 128), (513, 3584, 384, 384, 384), (640, 3080, 1024, 0, 128), (385, 6400, 448, 416, 224), (257, 6401, 640, 256, 0),
 ]
 
 
