@@ -297,6 +297,10 @@ BIG_TILE_SHAPES = [
     # launches of at most one tile per CU whose tile counts divide among the 8 XCDs as rectangles of tiles
     # (8 x 8, 16 x 12 and 8 x 16 tiles of 256 x 128; 16 x 8 tiles of 256 x 256), ragged tokens among them
     (1024, 2048, 384, 384, 128), (1536, 4096, 384, 384, 256), (2000, 2048, 384, 128, 0), (2048, 4096, 256, 128, 128),
+    # 256 x 128 tiles where no smaller ones are taken: a last segment of 1, 2, 3 stages, without and with blocks past the whole
+    # stages, tokens that end in either half of a tile, fewer than 256 tokens
+    (300, 11264, 128, 384, 128), (385, 11264, 384, 384, 256), (300, 11264, 256, 384, 384), (300, 11264, 416, 480, 160),
+    (300, 11272, 480, 448, 288), (512, 11264, 160, 416, 416), (170, 18944, 256, 384, 128), (170, 18944, 640, 416, 128),
 ]
 
 
