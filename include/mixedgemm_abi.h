@@ -135,6 +135,15 @@ int mg_tile_weights(const uint8_t* src, uint8_t* dst, int N, int kseg, void* str
  * the others multiples of 128 (pure E3M2 x E2M1 and E4M3 x E2M1 products among them: what matmul_host6 and
  * matmul_host8 of the reference, src/fp6.cu:35 and src/fp8.cu:35, compute on their own). */
 int mg_weights_tileable(int N, int KN, int KS, int KO);
+/* Which kernel mg_mixed_gemm_ex runs on a GPU with `cus` compute units (MI355X: 256): out[0] one of the MG_KERNEL_* below, out[1] and
+ * out[2] the features and tokens per workgroup (whole tiles: 256 x 256, some or all of them as 256 x 128).  Host only; for tests and
+ * for whoever wants to know what a shape costs. */
+#define MG_KERNEL_NONE 0   /* nothing to compute */
+#define MG_KERNEL_DECODE 1
+#define MG_KERNEL_SKINNY 2
+#define MG_KERNEL_TILE 3
+#define MG_KERNEL_WHOLE 4
+int mg_gemm_kernel(int M, int N, int KN, int KS, int KO, unsigned flags, int cus, int out[3]);
 /* M rounded up to whole 256-token tiles. */
 int mg_padded_rows(int M);
 

@@ -21,11 +21,12 @@ MG_OPERAND_A = 0
 MG_OPERAND_B = 1
 MG_FLAG_W_TILED = 1
 MG_OK, MG_ERR_BAD_INDEX = 0, 10003
+GEMM_KERNELS = ("none", "decode", "skinny", "tile", "whole")   # MG_KERNEL_*
 
 SYMBOLS = (
     "mg_reorder_quantize_x", "mg_reorder_quantize_w", "mg_mixed_gemm", "mg_mixed_gemm_ex", "mg_padded_rows", "mg_tile_weights",
     "mg_reorder_quantize_w_tiled", "mg_pack_weights",
-    "mg_weights_tileable", "mg_fused_linear_ex", "mg_rmsnorm_reorder_quantize_x", "mg_fused_norm_linear",
+    "mg_weights_tileable", "mg_gemm_kernel", "mg_fused_linear_ex", "mg_rmsnorm_reorder_quantize_x", "mg_fused_norm_linear",
     "mg_fused_linear",
     "mg_fused_workspace_bytes", "mg_sf_bytes", "mg_sf_offset", "mg_device_synchronize", "mg_status_string",
     "mg_calibrate_reorder_index", "mg_calibrate_workspace_bytes", "mg_check_reorder_index", "mg_check_reorder_index_host",
@@ -60,6 +61,7 @@ def lib() -> ctypes.CDLL:
         L.mg_mixed_gemm_ex.restype, L.mg_mixed_gemm_ex.argtypes = i, [p] * 12 + [i] * 6 + [u, p, p]
         L.mg_tile_weights.restype, L.mg_tile_weights.argtypes = i, [p, p, i, i, p]
         L.mg_weights_tileable.restype, L.mg_weights_tileable.argtypes = i, [i, i, i, i]
+        L.mg_gemm_kernel.restype, L.mg_gemm_kernel.argtypes = i, [i] * 5 + [u, i, p]
         f = ctypes.c_float
         L.mg_rmsnorm_reorder_quantize_x.restype = i
         L.mg_rmsnorm_reorder_quantize_x.argtypes = [p, p, f, p, i, i, i, i, i, p, p, p, p, p, p, p]
@@ -436,6 +438,14 @@ def _index_entries(reorder_index, k) -> int:
 
 def weights_tileable(n: int, kn: int, ks: int, ko: int) -> bool:
     return bool(lib().mg_weights_tileable(n, kn, ks, ko))
+
+
+def gemm_kernel(m: int, n: int, kn: int, ks: int, ko: int, w_tiled: bool = False, cus: int = 256):
+    """(kernel, features, tokens): what matmul runs for a shape on a GPU with `cus` compute units, one of GEMM_KERNELS, and what a
+    workgroup of it computes.  Host only."""
+    out = (ctypes.c_int * 3)()
+    check(lib().mg_gemm_kernel(m, n, kn, ks, ko, MG_FLAG_W_TILED if w_tiled else 0, cus, out), "mg_gemm_kernel")
+    return GEMM_KERNELS[out[0]], out[1], out[2]
 
 
 def tile_weights(wn, ws, wo):

@@ -12,6 +12,7 @@ template <bool IS_W>
 hipError_t launch_reorder_quant(const void* x, const int16_t* idx, int rows, int K, int KN, int KS, int KO, uint8_t* qn,
                                 uint8_t* qs, uint8_t* qo, uint8_t* sfn, uint8_t* sfs, uint8_t* sfo, const void* gamma,
                                 float eps, bool keep_codes, int src_rows, unsigned* verdict, hipStream_t stream);
+void mixed_gemm_choice(int M, int N, int KN, int KS, int KO, bool w_tiled, int cus, int out[3]);
 hipError_t launch_mixed_gemm(const uint8_t* an, const uint8_t* bn, const uint8_t* as_, const uint8_t* bs,
                              const uint8_t* ao, const uint8_t* bo, const uint8_t* sfan, const uint8_t* sfbn,
                              const uint8_t* sfas, const uint8_t* sfbs, const uint8_t* sfao, const uint8_t* sfbo, int M,
@@ -162,6 +163,16 @@ int mg_padded_rows(int M) { return M <= 0 ? 0 : (M + 255) / 256 * 256; }
 
 int mg_weights_tileable(int N, int KN, int KS, int KO) {
   return N > 0 && N % 256 == 0 && mg::mixed_gemm_256_supported(256, N, KN, KS, KO);   // what the whole-tile kernel takes
+}
+
+int mg_gemm_kernel(int M, int N, int KN, int KS, int KO, unsigned flags, int cus, int out[3]) {
+  if (int s = check_split(M, KN, KS, KO)) return s;
+  if (N < 0 || (flags & ~MG_FLAG_W_TILED) || cus <= 0) return MG_ERR_BAD_SHAPE;
+  const bool tiled = (flags & MG_FLAG_W_TILED) != 0;
+  if (tiled && !mg_weights_tileable(N, KN, KS, KO)) return MG_ERR_UNSUPPORTED;
+  if (out == nullptr) return MG_ERR_BAD_POINTER;
+  mg::mixed_gemm_choice(M, N, KN, KS, KO, tiled, cus, out);
+  return MG_OK;
 }
 
 int mg_tile_weights(const uint8_t* src, uint8_t* dst, int N, int kseg, void* stream) {

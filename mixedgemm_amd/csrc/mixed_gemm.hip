@@ -1143,6 +1143,71 @@ static double whole_tiles_us(int M, int N, int stages, int KN, int KS, int KO, i
   return fmax(1.4 + rounds * (stages * 0.741 - 7.0 + (rest ? 2.5 : 0.0)) + 0.63 * mb, rounds * stages * 0.6);
 }
 
+// The kernel a problem runs on.  A function of the shape, the weights' layout and the number of CUs alone.
+enum class GemmKernel { kNone, kDecode, kSkinny, kTile, kWhole };
+struct GemmChoice {
+  GemmKernel kernel;
+  int decode_f;          // kDecode: feature groups of 16 per workgroup
+  DecodeLds lds;         //   and the LDS image
+  SkinnyPlan skinny;     // kSkinny
+  TilePlanChoice tile;   // kTile
+};
+
+static GemmChoice choose_gemm(const DecodeSeg& d4, const DecodeSeg& d6, const DecodeSeg& d8, int M, int N, int KN, int KS, int KO,
+                              bool w_tiled, int cus) {
+  GemmChoice c = {};
+  if (M == 0 || N == 0) return c;
+  const int m_pad = (M + 255) / 256 * 256;
+  const bool whole_tiles = mixed_gemm_256_supported(m_pad, N, KN, KS, KO);
+  const int steps = d4.steps + d6.steps + d8.steps;
+  // (the skinny kernel addresses a segment's row-major weight codes with 32-bit offsets)
+  const int widest = KN > KS ? (KN > KO ? KN : KO) : (KS > KO ? KS : KO);
+  const bool few = M < 256 && KN + KS + KO > 0, skinny_ok = few && (w_tiled || (size_t)N * (size_t)(widest / 2) < ((size_t)1 << 32));
+  if (few) {
+    c.decode_f = decode_plan(d4, d6, d8, M, N, w_tiled, cus, &c.lds);
+    if (c.decode_f != 0) {
+      c.kernel = GemmKernel::kDecode;
+      return c;
+    }
+  }
+  // What no other kernel takes, whatever the number of tokens, goes to small tiles; so does what they are estimated to be the
+  // fastest for by a margin (the estimates of both sides are off by 10 %), above 16 tokens.  Both weight layouts go the same way
+  // there (they give the same bits): the estimates compared are those on
+  // tile-major weights.  Below 256 tokens the kernel taken is in the mean 0.7 % slower than the best one with the weights in the
+  // caches (1542 calls) and 0.03 % from HBM (710 calls), where the skinny kernel keeps more on its way: 128 tokens, N = K = 4096,
+  // the nearest of the estimates, 9.6 against 8.2 us on small tiles in the caches, 10.8 against 10.9 from HBM (row-major 10.7
+  // against 11.3).
+  c.tile = mixed_gemm_tile_plan(M, N, KN, KS, KO, cus);
+  const SkinnyPlan skinny_t = few ? skinny_plan(M, N, steps, cus, true) : SkinnyPlan{0, 0, 0.0};
+  const double whole_us = few ? pipelined_us(M, N, steps, KN, KS, KO, cus) : whole_tiles_us(M, N, steps, KN, KS, KO, cus);
+  const double others = few ? (whole_tiles ? fmin(whole_us, skinny_t.us) : skinny_t.us) : whole_us;
+  if ((!whole_tiles && !skinny_ok) || ((M > 16 || !few) && c.tile.us < 0.95 * others)) {
+    c.kernel = GemmKernel::kTile;
+    return c;
+  }
+  c.skinny = skinny_ok && !w_tiled ? skinny_plan(M, N, steps, cus, false) : skinny_t;
+  // whole 256-row tiles; the last one does not write rows past M and reads no activation row past
+  // a_rows (lanes that would are pointed at the last readable row)
+  c.kernel = whole_tiles && (!skinny_ok || whole_us < c.skinny.us) ? GemmKernel::kWhole : GemmKernel::kSkinny;
+  return c;
+}
+
+// The choice for the host alone: out[0] the kernel (MG_KERNEL_*), out[1] features and out[2] tokens per workgroup.
+void mixed_gemm_choice(int M, int N, int KN, int KS, int KO, bool w_tiled, int cus, int out[3]) {
+  const DecodeSeg d4 = {nullptr, nullptr, nullptr, nullptr, KN / 32, ceil_div(KN, 128)};
+  const DecodeSeg d6 = {nullptr, nullptr, nullptr, nullptr, KS / 32, ceil_div(KS, 128)};
+  const DecodeSeg d8 = {nullptr, nullptr, nullptr, nullptr, KO / 32, ceil_div(KO, 128)};
+  const GemmChoice c = choose_gemm(d4, d6, d8, M, N, KN, KS, KO, w_tiled, cus);
+  out[0] = (int)c.kernel;
+  switch (c.kernel) {
+    case GemmKernel::kDecode: out[1] = 16 * c.decode_f; out[2] = 16; break;
+    case GemmKernel::kSkinny: out[1] = 16 * c.skinny.f; out[2] = 16 * c.skinny.g; break;
+    case GemmKernel::kTile: out[1] = c.tile.tf; out[2] = c.tile.tt; break;
+    case GemmKernel::kWhole: out[1] = out[2] = 256; break;
+    default: out[1] = out[2] = 0;
+  }
+}
+
 // a_rows: token rows for which the activation codes and scales are readable (>= M)
 hipError_t launch_mixed_gemm(const uint8_t* an, const uint8_t* bn, const uint8_t* as_, const uint8_t* bs,
                              const uint8_t* ao, const uint8_t* bo, const uint8_t* sfan, const uint8_t* sfbn,
@@ -1153,42 +1218,25 @@ hipError_t launch_mixed_gemm(const uint8_t* an, const uint8_t* bn, const uint8_t
   const bool w_tiled = (flags & 1u) != 0;   // MG_FLAG_W_TILED
   // tile-major weights exist only for shapes the 256x256 kernel takes
   if (w_tiled && (N % 256 != 0 || !mixed_gemm_256_supported(256, N, KN, KS, KO))) return hipErrorInvalidValue;
-  const int m_pad = (M + 255) / 256 * 256;
-  const DecodeSeg d4 = {an, bn, sfan, sfbn, KN / 32, (KN + 127) / 128};
-  const DecodeSeg d6 = {as_, bs, sfas, sfbs, KS / 32, (KS + 127) / 128};
-  const DecodeSeg d8 = {ao, bo, sfao, sfbo, KO / 32, (KO + 127) / 128};
-  const bool whole_tiles = mixed_gemm_256_supported(m_pad, N, KN, KS, KO);
+  const DecodeSeg d4 = {an, bn, sfan, sfbn, KN / 32, ceil_div(KN, 128)};
+  const DecodeSeg d6 = {as_, bs, sfas, sfbs, KS / 32, ceil_div(KS, 128)};
+  const DecodeSeg d8 = {ao, bo, sfao, sfbo, KO / 32, ceil_div(KO, 128)};
   DeviceLimits lim;
   if (hipError_t e = device_limits(&lim); e != hipSuccess) return e;
-  const int steps = d4.steps + d6.steps + d8.steps;
-  // (the skinny kernel addresses a segment's row-major weight codes with 32-bit offsets)
-  const int widest = KN > KS ? (KN > KO ? KN : KO) : (KS > KO ? KS : KO);
-  const bool few = M < 256 && KN + KS + KO > 0, skinny_ok = few && (w_tiled || (size_t)N * (size_t)(widest / 2) < ((size_t)1 << 32));
-  if (few) {
-    DecodeLds L;
-    if (const int f = decode_plan(d4, d6, d8, M, N, w_tiled, lim.cus, &L))
-      return launch_decode(d4, d6, d8, M, N, w_tiled, f, L, ep, static_cast<uint16_t*>(d), stream);
+  const GemmChoice c = choose_gemm(d4, d6, d8, M, N, KN, KS, KO, w_tiled, lim.cus);
+  switch (c.kernel) {
+    case GemmKernel::kDecode:
+      return launch_decode(d4, d6, d8, M, N, w_tiled, c.decode_f, c.lds, ep, static_cast<uint16_t*>(d), stream);
+    case GemmKernel::kSkinny:
+      return launch_skinny(d4, d6, d8, M, N, w_tiled, c.skinny, ep, static_cast<uint16_t*>(d), stream);
+    case GemmKernel::kTile:
+      return launch_mixed_gemm_tile(an, bn, as_, bs, ao, bo, sfan, sfbn, sfas, sfbs, sfao, sfbo, M, a_rows, N, KN, KS, KO, w_tiled,
+                                    c.tile, ep, d, stream);
+    case GemmKernel::kWhole:
+      return launch_mixed_gemm_256(an, bn, as_, bs, ao, bo, sfan, sfbn, sfas, sfbs, sfao, sfbo, M, a_rows, N, KN, KS, KO, w_tiled,
+                                   ep, d, stream);
+    default: return hipErrorInvalidValue;
   }
-  // Small tiles where they are estimated to be the fastest by a margin (the estimates of both sides are off by 10 %), and for
-  // what no other kernel takes.  Both weight layouts go the same way (they give the same bits): the estimates compared are those on
-  // tile-major weights.  Below 256 tokens the kernel taken is in the mean 0.7 % slower than the best one with the weights in the
-  // caches (1542 calls) and 0.03 % from HBM (710 calls), where the skinny kernel keeps more on its way: 128 tokens, N = K = 4096,
-  // the nearest of the estimates, 9.6 against 8.2 us on small tiles in the caches, 10.8 against 10.9 from HBM (row-major 10.7
-  // against 11.3).
-  const TilePlanChoice tile = mixed_gemm_tile_plan(M, N, KN, KS, KO, lim.cus);
-  const SkinnyPlan skinny_t = few ? skinny_plan(M, N, steps, lim.cus, true) : SkinnyPlan{0, 0, 0.0};
-  const double whole_us = few ? pipelined_us(M, N, steps, KN, KS, KO, lim.cus) : whole_tiles_us(M, N, steps, KN, KS, KO, lim.cus);
-  const double others = few ? (whole_tiles ? fmin(whole_us, skinny_t.us) : skinny_t.us) : whole_us;
-  if ((M > 16 || !few) && ((!whole_tiles && !skinny_ok) || tile.us < 0.95 * others))
-    return launch_mixed_gemm_tile(an, bn, as_, bs, ao, bo, sfan, sfbn, sfas, sfbs, sfao, sfbo, M, a_rows, N, KN, KS, KO, w_tiled, tile,
-                                  ep, d, stream);
-  const SkinnyPlan skinny = skinny_ok && !w_tiled ? skinny_plan(M, N, steps, lim.cus, false) : skinny_t;
-  // whole 256-row tiles; the last one does not write rows past M and reads no activation row past
-  // a_rows (lanes that would are pointed at the last readable row)
-  if (whole_tiles && (!skinny_ok || whole_us < skinny.us))
-    return launch_mixed_gemm_256(an, bn, as_, bs, ao, bo, sfan, sfbn, sfas, sfbs, sfao, sfbo, M, a_rows, N, KN, KS, KO,
-                                 w_tiled, ep, d, stream);
-  return launch_skinny(d4, d6, d8, M, N, w_tiled, skinny, ep, static_cast<uint16_t*>(d), stream);
 }
 
 // Quantization and GEMM of a few tokens in one launch, where that is the faster way; *taken says whether it was.

@@ -293,3 +293,38 @@ def test_static_entry_point_refuses_what_does_not_fit(abi):
     # shape errors come first, empty problems succeed without touching the GPU
     assert lib.mg_fused_linear_static(*[null] * 8, 16, 256, 2560, 1400, 136, 0, null, null) == 10001
     assert lib.mg_fused_linear_static(*[null] * 8, 0, 256, 2560, 1408, 128, 0, null, null) == 0
+
+
+# ------------------------------------------------------------------ which kernel a shape runs on
+def test_gemm_kernel_query(abi):
+    import torch  # noqa: F401
+    assert abi.gemm_kernel(0, 256, 128, 0, 0) == ("none", 0, 0) and abi.gemm_kernel(4, 0, 128, 0, 0) == ("none", 0, 0)
+    assert abi.gemm_kernel(8, 14336, 2560, 1408, 128, True)[0] == "decode"
+    assert abi.gemm_kernel(8, 4104, 2560, 1408, 96)[0] == "skinny"
+    assert abi.gemm_kernel(256, 4096, 2560, 1408, 128) == ("tile", 64, 64)
+    assert abi.gemm_kernel(4096, 14336, 2560, 1408, 128, True) == ("whole", 256, 256)
+    assert abi.gemm_kernel(300, 1001, 2560, 1408, 128)[0] == "tile"     # an odd number of features: nothing else takes it
+    lib, three = abi.lib(), (ctypes.c_int * 3)()
+    assert lib.mg_gemm_kernel(8, 256, 100, 0, 0, 0, 256, three) == 10001
+    assert lib.mg_gemm_kernel(8, 256, 128, 0, 0, 2, 256, three) == 10001
+    assert lib.mg_gemm_kernel(8, 256, 128, 0, 0, 0, 0, three) == 10001
+    assert lib.mg_gemm_kernel(8, 200, 128, 128, 128, 1, 256, three) == 10004
+    assert lib.mg_gemm_kernel(8, 256, 128, 0, 0, 0, 256, None) == 10002
+
+
+@pytest.mark.parametrize("cus", [256, 64])
+def test_segments_of_4_gb_of_row_major_weights_never_meet_32_bit_offsets(abi, cus):
+    """The skinny and decode kernels address a segment's row-major weight codes with 32-bit offsets: whatever the number of tokens,
+    a segment of 2^32 bytes and more runs on one of the kernels that do not, and one row less on either side of the line keeps its own."""
+    # all E2M1 and no whole stages; whole 128-wide stages; three segments; a feature count that is no multiple of 8
+    for kn, ks, ko in ((32736, 0, 0), (32640, 0, 0), (0, 32736, 0), (0, 0, 32672), (20480, 8192, 4064), (2048, 64, 30624)):
+        widest = max(kn, ks, ko)
+        line = -(-(1 << 32) // (widest // 2))          # the fewest rows that reach 2^32 bytes
+        for n in (line, line + 3, line + 256 - line % 256, 2 * line):
+            assert n * (widest // 2) >= 1 << 32
+            for m in (*range(1, 18), 31, 32, 33, 64, 100, 128, 200, 255, 256, 300):
+                kernel, tf, tt = abi.gemm_kernel(m, n, kn, ks, ko, cus=cus)
+                assert kernel in ("tile", "whole"), (m, n, kn, ks, ko, kernel)
+                assert tf >= 64 and tt >= 64
+        if (line - 1) % 8:                             # (not for whole tiles: the choice above does not depend on them)
+            assert abi.gemm_kernel(1, line - 1, kn, ks, ko, cus=cus)[0] in ("skinny", "decode")

@@ -775,6 +775,31 @@ def test_small_tiles_match_oracle(abi, m, n, kn, ks, ko):
         assert torch.equal(d, d_tiled)
 
 
+@pytest.mark.parametrize("m", [1, 8, 16, 17])
+def test_row_major_weights_of_more_than_4_gb(abi, m):
+    """Features behind the first 2^32 bytes of a segment's codes are multiplied with their own rows.  All scales are 1 and the sums
+    (multiples of 1/4 below 36 * K) exact in fp32, so the part of the weights on its own has the same bits on whatever kernel."""
+    n, k, part = 262464 + 3, 32736, 300          # no whole stages, an odd number of features: 4.3 GB of codes
+    _say("4 GB", m, n, k)
+    g = torch.Generator(device=DEV).manual_seed(m)
+    codes = lambda rows: torch.randint(0, 256, (rows, k // 2), dtype=torch.uint8, device=DEV, generator=g)
+    ones = lambda rows, operand: torch.full((abi.sf_bytes(rows, k, operand),), 127, dtype=torch.uint8, device=DEV)
+    none = lambda rows: torch.empty((rows, 0), dtype=torch.uint8, device=DEV)
+    empty = torch.empty(0, dtype=torch.uint8, device=DEV)
+    a, b = codes(m), codes(n)
+    sfa = ones(m, abi.MG_OPERAND_A)
+
+    def product(w):
+        r = w.shape[0]
+        return abi.matmul(a, w, none(m), none(r), none(m), none(r), sfa, ones(r, abi.MG_OPERAND_B), empty, empty, empty, empty)
+
+    d = product(b)
+    for at in (0, n // 2, n - part):
+        want = product(b[at:at + part].contiguous())
+        torch.cuda.synchronize()
+        assert torch.equal(d[:, at:at + part], want), f"features {at} ... {at + part}"
+
+
 def _seeded_shapes(count, seed):
     """Shapes drawn across the dispatcher's cases: token counts on both sides of 256 and of whole tiles, feature
     counts with and without whole 256-feature tiles, segments of 0 or 32..1024 channels in steps of 32."""
