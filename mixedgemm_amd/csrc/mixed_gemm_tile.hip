@@ -19,6 +19,7 @@
 // 4096, K = 12288: 57.6 against 56.3 us: 15 % fewer cycles at a clock as much lower; the chip is at its power limit there), tiles of
 // 64 and 128 x 32 slower than 64 x 64 at every shape tried.
 #include "mg_common.h"
+#include "tile_order.h"
 
 #include <type_traits>
 
@@ -45,10 +46,7 @@ struct TilePlan {
   int N;          // weight rows
   int m_store;    // token rows that are stored
   int a_rows;     // token rows that may be read
-  // Workgroup -> tile (see tile_at): a rectangle of `div` x div2 tiles per XCD, 2^xlog rectangles along the features, or
-  // (xlog < 0) tiles in feature-major order, div = token tiles, div2 = tiles per XCD or 0
-  int xlog, div, div2;
-  unsigned magic;   // 2^32 / div, rounded up (div > 1)
+  TileOrder order;   // workgroup -> tile
 };
 
 template <int FMT> struct Form;
@@ -392,29 +390,13 @@ __device__ __forceinline__ void rest_half(v16f (&acc)[G::TN][G::TM], const TileC
   if (has8) rest_multiply<kFmtE4M3, H, G>(acc, r8, p.s8, g);
 }
 
-// Workgroup -> tile.  Workgroups go to the 8 XCDs round-robin; an XCD (an L2) gets a rectangle of tiles where the counts divide,
-// the one with the fewest operand bytes per stage, else consecutive tiles in feature-major order.
-__device__ __forceinline__ void tile_at(const TilePlan& p, int wg, int& tn, int& tm) {
-  const int xcd = wg & 7;
-  int j = wg >> 3;
-  if (p.xlog < 0) j = p.div2 > 0 ? xcd * p.div2 + j : wg;
-  const int q = p.div > 1 ? (int)__umulhi((unsigned)j, p.magic) : j, r = j - q * p.div;
-  if (p.xlog < 0) {
-    tn = q;
-    tm = r;
-  } else {
-    tn = (xcd & ((1 << p.xlog) - 1)) * p.div + r;
-    tm = (xcd >> p.xlog) * p.div2 + q;
-  }
-}
-
 // All arguments into scalar registers in one batch of loads: fetched where they are first used they cost a round trip to the
 // argument buffer each time, before the first copy goes out.
 __device__ __forceinline__ void pin_plan(const TilePlan& p, const Epilogue& ep, const uint16_t* d) {
   asm volatile("" : : "s"(p.s4.a), "s"(p.s4.b), "s"(p.s4.sfa), "s"(p.s4.sfb), "s"(p.s4.blk), "s"(p.s4.whole), "s"(p.s6.a), "s"(p.s6.b),
                "s"(p.s6.sfa), "s"(p.s6.sfb), "s"(p.s6.blk), "s"(p.s6.whole), "s"(p.s8.a), "s"(p.s8.b), "s"(p.s8.sfa), "s"(p.s8.sfb),
-               "s"(p.s8.blk), "s"(p.s8.whole), "s"(p.total), "s"(p.N), "s"(p.m_store), "s"(p.a_rows), "s"(p.xlog), "s"(p.div), "s"(p.div2),
-               "s"(p.magic), "s"(ep.bias), "s"(ep.n_out), "s"(d));
+               "s"(p.s8.blk), "s"(p.s8.whole), "s"(p.total), "s"(p.N), "s"(p.m_store), "s"(p.a_rows), "s"(p.order.xlog), "s"(p.order.div),
+               "s"(p.order.div2), "s"(p.order.magic), "s"(ep.bias), "s"(ep.n_out), "s"(d));
 }
 
 template <int TF, int TT, int WF, int WS, bool WT, bool REM>
@@ -427,7 +409,7 @@ mixed_gemm_tile_kernel(TilePlan plan, Epilogue ep, uint16_t* __restrict__ d) {
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   pin_plan(plan, ep, d);
   int tn, tm;
-  tile_at(plan, blockIdx.x, tn, tm);
+  tile_at(plan.order, blockIdx.x, tn, tm);
   TileCtx<G> c;
   c.lane = threadIdx.x & 63;
   c.n0 = tn * TF;
@@ -710,24 +692,7 @@ hipError_t launch_mixed_gemm_tile(const uint8_t* an, const uint8_t* bn, const ui
   p.m_store = m_store;
   p.a_rows = a_rows;
   const int tiles_n = ceil_div(ep.n_out, tf), tiles_m = ceil_div(m_store, tt), nwg = tiles_n * tiles_m;
-  p.xlog = -1;
-  p.div = tiles_m;
-  p.div2 = (nwg & 7) == 0 ? nwg >> 3 : 0;
-  if ((nwg & 7) == 0) {
-    int best = 0x7fffffff;
-    for (int x = 3; x >= 0; --x) {
-      const int gx = 1 << x, gy = 8 >> x;
-      if (tiles_n % gx || tiles_m % gy) continue;
-      const int cost = (tiles_n / gx) * tf * 64 + (tiles_m / gy) * tt * 80;   // operand bytes per stage of a rectangle
-      if (cost < best) {
-        best = cost;
-        p.xlog = x;
-        p.div = tiles_n / gx;
-        p.div2 = tiles_m / gy;
-      }
-    }
-  }
-  p.magic = p.div > 1 ? (unsigned)(((1ull << 32) + p.div - 1) / p.div) : 0;
+  p.order = tile_order(tiles_n, tiles_m, tf, tt);
   const bool rem = ((KN | KS | KO) & 127) != 0;
   uint16_t* out = static_cast<uint16_t*>(d);
   if (tf == 128 && tt == 128) return launch_geo<128, 128, 2, 2>(p, nwg, w_tiled, rem, ep, out, stream);

@@ -1,0 +1,61 @@
+// Which tile of the result a workgroup of the small-tile GEMM computes: integer arithmetic for the kernel and for the host.
+#pragma once
+#include <hip/hip_runtime.h>
+#include <stdint.h>
+
+namespace mg {
+
+// Workgroups go to the 8 XCDs round-robin; an XCD (an L2) gets a rectangle of tiles where the counts divide, the one with the fewest
+// operand bytes per stage, else consecutive tiles in feature-major order.
+struct TileOrder {
+  // A rectangle of `div` x div2 tiles per XCD, 2^xlog rectangles along the features, or (xlog < 0) tiles in feature-major order,
+  // div = token tiles, div2 = tiles per XCD or 0
+  int xlog, div, div2;
+  unsigned magic;   // 2^32 / div, rounded up (div > 1)
+};
+
+// tf x tt: features and tokens of a tile
+inline TileOrder tile_order(int tiles_n, int tiles_m, int tf, int tt) {
+  const int nwg = tiles_n * tiles_m;
+  TileOrder o = {-1, tiles_m, (nwg & 7) == 0 ? nwg >> 3 : 0, 0};
+  if ((nwg & 7) == 0) {
+    double best = 0.0;
+    for (int x = 3; x >= 0; --x) {
+      const int gx = 1 << x, gy = 8 >> x;
+      if (tiles_n % gx || tiles_m % gy) continue;
+      const double cost = (double)(tiles_n / gx) * tf * 64 + (double)(tiles_m / gy) * tt * 80;   // operand bytes per stage of a rectangle
+      if (o.xlog < 0 || cost < best) {
+        best = cost;
+        o = {x, tiles_n / gx, tiles_m / gy, 0};
+      }
+    }
+  }
+  o.magic = o.div > 1 ? (unsigned)(((1ull << 32) + o.div - 1) / o.div) : 0;
+  return o;
+}
+
+__host__ __device__ inline void tile_at(const TileOrder& o, int wg, int& tn, int& tm) {
+  const int xcd = wg & 7;
+  int j = wg >> 3;
+  if (o.xlog < 0) j = o.div2 > 0 ? xcd * o.div2 + j : wg;
+  int q = j, r = 0;
+  if (o.div > 1) {
+    // magic * div = 2^32 + e with 0 <= e < div, so the product is j / div + (j * e / div) / 2^32: less than one too large for any
+    // 31-bit j, and its whole part is j / div or, for some of the j that lie just below a multiple of div, one more.
+    q = (int)(((uint64_t)(uint32_t)j * o.magic) >> 32);
+    r = j - q * o.div;
+    if (r < 0) {
+      q -= 1;
+      r += o.div;
+    }
+  }
+  if (o.xlog < 0) {
+    tn = q;
+    tm = r;
+  } else {
+    tn = (xcd & ((1 << o.xlog) - 1)) * o.div + r;
+    tm = (xcd >> o.xlog) * o.div2 + q;
+  }
+}
+
+}  // namespace mg

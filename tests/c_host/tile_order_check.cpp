@@ -1,0 +1,28 @@
+// Host program of tests/test_tile_order_cpu.py: maps every workgroup of each grid given as "tiles_n tiles_m tf tt" on stdin to its
+// tile and prints the grids where some tile is not computed exactly once.
+#include <stdio.h>
+
+#include <vector>
+
+#include "../../mixedgemm_amd/csrc/tile_order.h"
+
+int main() {
+  int tiles_n, tiles_m, tf, tt, grids = 0;
+  while (scanf("%d %d %d %d", &tiles_n, &tiles_m, &tf, &tt) == 4) {
+    const mg::TileOrder order = mg::tile_order(tiles_n, tiles_m, tf, tt);
+    const int nwg = tiles_n * tiles_m;
+    std::vector<bool> seen(nwg, false);
+    for (int wg = 0; wg < nwg; ++wg) {
+      int tn = -1, tm = -1;
+      mg::tile_at(order, wg, tn, tm);
+      if (tn < 0 || tn >= tiles_n || tm < 0 || tm >= tiles_m || seen[(size_t)tn * tiles_m + tm]) {
+        printf("%d x %d tiles of %d x %d: workgroup %d -> (%d, %d)\n", tiles_n, tiles_m, tf, tt, wg, tn, tm);
+        break;
+      }
+      seen[(size_t)tn * tiles_m + tm] = true;
+    }
+    ++grids;
+  }
+  printf("%d grids\n", grids);
+  return 0;
+}

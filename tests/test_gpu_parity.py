@@ -800,6 +800,31 @@ def test_row_major_weights_of_more_than_4_gb(abi, m):
         assert torch.equal(d[:, at:at + part], want), f"features {at} ... {at + part}"
 
 
+def test_small_tiles_of_a_grid_beyond_a_32_bit_reciprocal(abi):
+    """30819 x 5 tiles of 128 x 128: the last workgroup's tile is the last one.  Scales of 1 and K = 64: exact sums, so that parts of
+    the problem on their own have the same bits."""
+    m, n, k, part = 3944818, 545, 64, 200
+    _say("large grid", m, n, k)
+    assert abi.gemm_kernel(m, n, k, 0, 0) == ("tile", 128, 128)
+    g = torch.Generator(device=DEV).manual_seed(3)
+    codes = lambda rows: torch.randint(0, 256, (rows, k // 2), dtype=torch.uint8, device=DEV, generator=g)
+    ones = lambda rows, operand: torch.full((abi.sf_bytes(rows, k, operand),), 127, dtype=torch.uint8, device=DEV)
+    none = lambda rows: torch.empty((rows, 0), dtype=torch.uint8, device=DEV)
+    empty = torch.empty(0, dtype=torch.uint8, device=DEV)
+    a, b = codes(m), codes(n)
+
+    def product(x, **kw):
+        return abi.matmul(x, b, none(x.shape[0]), none(n), none(x.shape[0]), none(n), ones(x.shape[0], abi.MG_OPERAND_A),
+                          ones(n, abi.MG_OPERAND_B), empty, empty, empty, empty, **kw)
+
+    d = product(a, out=torch.full((m, n), float("nan"), dtype=torch.bfloat16, device=DEV))
+    assert not bool(torch.isnan(d).any())
+    for at in (0, m // 2 // 128 * 128, m - part):
+        want = product(a[at:at + part].contiguous())
+        torch.cuda.synchronize()
+        assert torch.equal(d[at:at + part], want), f"tokens {at} ... {at + part}"
+
+
 def _seeded_shapes(count, seed):
     """Shapes drawn across the dispatcher's cases: token counts on both sides of 256 and of whole tiles, feature
     counts with and without whole 256-feature tiles, segments of 0 or 32..1024 channels in steps of 32."""
