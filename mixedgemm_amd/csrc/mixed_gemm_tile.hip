@@ -396,7 +396,7 @@ __device__ __forceinline__ void pin_plan(const TilePlan& p, const Epilogue& ep, 
   asm volatile("" : : "s"(p.s4.a), "s"(p.s4.b), "s"(p.s4.sfa), "s"(p.s4.sfb), "s"(p.s4.blk), "s"(p.s4.whole), "s"(p.s6.a), "s"(p.s6.b),
                "s"(p.s6.sfa), "s"(p.s6.sfb), "s"(p.s6.blk), "s"(p.s6.whole), "s"(p.s8.a), "s"(p.s8.b), "s"(p.s8.sfa), "s"(p.s8.sfb),
                "s"(p.s8.blk), "s"(p.s8.whole), "s"(p.total), "s"(p.N), "s"(p.m_store), "s"(p.a_rows), "s"(p.order.xlog), "s"(p.order.div),
-               "s"(p.order.div2), "s"(p.order.magic), "s"(ep.bias), "s"(ep.n_out), "s"(d));
+               "s"(p.order.div2), "s"(p.order.magic), "s"(p.order.grid_x), "s"(p.order.tiles), "s"(ep.bias), "s"(ep.n_out), "s"(d));
 }
 
 template <int TF, int TT, int WF, int WS, bool WT, bool REM>
@@ -408,8 +408,10 @@ mixed_gemm_tile_kernel(TilePlan plan, Epilogue ep, uint16_t* __restrict__ d) {
   const unsigned lds0 = (unsigned)(size_t)(__attribute__((address_space(3))) uint8_t*)lds;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   pin_plan(plan, ep, d);
+  const int wg = blockIdx.y * plan.order.grid_x + blockIdx.x;
+  if (wg >= plan.order.tiles) return;   // (the last row of a grid of several)
   int tn, tm;
-  tile_at(plan.order, blockIdx.x, tn, tm);
+  tile_at(plan.order, wg, tn, tm);
   TileCtx<G> c;
   c.lane = threadIdx.x & 63;
   c.n0 = tn * TF;
@@ -640,13 +642,14 @@ mixed_gemm_tile_kernel(TilePlan plan, Epilogue ep, uint16_t* __restrict__ d) {
 }
 
 template <int TF, int TT, int WF, int WS>
-hipError_t launch_geo(const TilePlan& p, int nwg, bool w_tiled, bool rem, const Epilogue& ep, uint16_t* d, hipStream_t stream) {
+hipError_t launch_geo(const TilePlan& p, bool w_tiled, bool rem, const Epilogue& ep, uint16_t* d, hipStream_t stream) {
   const auto kernel = w_tiled ? (rem ? mixed_gemm_tile_kernel<TF, TT, WF, WS, true, true> : mixed_gemm_tile_kernel<TF, TT, WF, WS, true, false>)
                               : (rem ? mixed_gemm_tile_kernel<TF, TT, WF, WS, false, true> : mixed_gemm_tile_kernel<TF, TT, WF, WS, false, false>);
+  static_assert((int64_t)kMostTilesAcross * 64 * kTileWaves < (int64_t)1 << 32, "threads along a dimension of the grid");
   typedef Geo<TF, TT, WF, WS, false> G;
   constexpr int kLds = G::NB * G::kBatch;
   if (hipError_t e = allow_dynamic_lds(reinterpret_cast<const void*>(kernel), kLds); e != hipSuccess) return e;
-  hipLaunchKernelGGL(kernel, dim3(nwg), dim3(64 * kTileWaves), kLds, stream, p, ep, d);
+  hipLaunchKernelGGL(kernel, dim3(p.order.grid_x, grid_rows(p.order)), dim3(64 * kTileWaves), kLds, stream, p, ep, d);
   return hipGetLastError();
 }
 
@@ -691,13 +694,12 @@ hipError_t launch_mixed_gemm_tile(const uint8_t* an, const uint8_t* bn, const ui
   p.N = N;
   p.m_store = m_store;
   p.a_rows = a_rows;
-  const int tiles_n = ceil_div(ep.n_out, tf), tiles_m = ceil_div(m_store, tt), nwg = tiles_n * tiles_m;
-  p.order = tile_order(tiles_n, tiles_m, tf, tt);
+  p.order = tile_order(ceil_div(ep.n_out, tf), ceil_div(m_store, tt), tf, tt);
   const bool rem = ((KN | KS | KO) & 127) != 0;
   uint16_t* out = static_cast<uint16_t*>(d);
-  if (tf == 128 && tt == 128) return launch_geo<128, 128, 2, 2>(p, nwg, w_tiled, rem, ep, out, stream);
-  if (tf == 128 && tt == 64) return launch_geo<128, 64, 2, 2>(p, nwg, w_tiled, rem, ep, out, stream);
-  if (tf == 64 && tt == 64) return launch_geo<64, 64, 1, 4>(p, nwg, w_tiled, rem, ep, out, stream);
+  if (tf == 128 && tt == 128) return launch_geo<128, 128, 2, 2>(p, w_tiled, rem, ep, out, stream);
+  if (tf == 128 && tt == 64) return launch_geo<128, 64, 2, 2>(p, w_tiled, rem, ep, out, stream);
+  if (tf == 64 && tt == 64) return launch_geo<64, 64, 1, 4>(p, w_tiled, rem, ep, out, stream);
   return hipErrorInvalidValue;
 }
 

@@ -12,12 +12,16 @@ struct TileOrder {
   // div = token tiles, div2 = tiles per XCD or 0
   int xlog, div, div2;
   unsigned magic;   // 2^32 / div, rounded up (div > 1)
+  int grid_x, tiles;   // workgroups per row of the launch grid, and of all
 };
+
+// HIP takes fewer than 2^32 threads along a dimension of a grid; a launch of more tiles than this has several rows of workgroups.
+constexpr int kMostTilesAcross = 1 << 22;   // of at most 1023 threads each
 
 // tf x tt: features and tokens of a tile
 inline TileOrder tile_order(int tiles_n, int tiles_m, int tf, int tt) {
   const int nwg = tiles_n * tiles_m;
-  TileOrder o = {-1, tiles_m, (nwg & 7) == 0 ? nwg >> 3 : 0, 0};
+  TileOrder o = {-1, tiles_m, (nwg & 7) == 0 ? nwg >> 3 : 0, 0, nwg < kMostTilesAcross ? nwg : kMostTilesAcross, nwg};
   if ((nwg & 7) == 0) {
     double best = 0.0;
     for (int x = 3; x >= 0; --x) {
@@ -26,7 +30,9 @@ inline TileOrder tile_order(int tiles_n, int tiles_m, int tf, int tt) {
       const double cost = (double)(tiles_n / gx) * tf * 64 + (double)(tiles_m / gy) * tt * 80;   // operand bytes per stage of a rectangle
       if (o.xlog < 0 || cost < best) {
         best = cost;
-        o = {x, tiles_n / gx, tiles_m / gy, 0};
+        o.xlog = x;
+        o.div = tiles_n / gx;
+        o.div2 = tiles_m / gy;
       }
     }
   }
@@ -34,6 +40,9 @@ inline TileOrder tile_order(int tiles_n, int tiles_m, int tf, int tt) {
   return o;
 }
 
+inline int grid_rows(const TileOrder& o) { return (int)(((int64_t)o.tiles + o.grid_x - 1) / o.grid_x); }
+
+// wg: the workgroup's number in launch order, below o.tiles
 __host__ __device__ inline void tile_at(const TileOrder& o, int wg, int& tn, int& tm) {
   const int xcd = wg & 7;
   int j = wg >> 3;

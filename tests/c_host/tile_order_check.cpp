@@ -12,6 +12,9 @@ int main() {
     const mg::TileOrder order = mg::tile_order(tiles_n, tiles_m, tf, tt);
     const int nwg = tiles_n * tiles_m;
     std::vector<bool> seen(nwg, false);
+    const int rows = mg::grid_rows(order);
+    if (order.grid_x > mg::kMostTilesAcross || (long long)order.grid_x * rows < nwg || (long long)order.grid_x * (rows - 1) >= nwg)
+      printf("%d x %d tiles of %d x %d: a grid of %d x %d\n", tiles_n, tiles_m, tf, tt, order.grid_x, rows);
     for (int wg = 0; wg < nwg; ++wg) {
       int tn = -1, tm = -1;
       mg::tile_at(order, wg, tn, tm);

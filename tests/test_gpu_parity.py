@@ -825,6 +825,31 @@ def test_small_tiles_of_a_grid_beyond_a_32_bit_reciprocal(abi):
         assert torch.equal(d[at:at + part], want), f"tokens {at} ... {at + part}"
 
 
+def test_small_tiles_of_a_grid_of_several_rows(abi):
+    """One token, 716 million features: more workgroups than one dimension of a grid takes.  Exact sums as above."""
+    n, k, part = 128 * 5593000 + 3, 32, 300
+    _say("grid of several rows", n, k)
+    kernel, tf, _ = abi.gemm_kernel(1, n, k, 0, 0)
+    assert kernel == "tile" and n / tf * 768 > 1 << 32
+    g = torch.Generator(device=DEV).manual_seed(4)
+    a = torch.randint(0, 256, (1, k // 2), dtype=torch.uint8, device=DEV, generator=g)
+    b = torch.randint(0, 256, (n, k // 2), dtype=torch.uint8, device=DEV, generator=g)
+    ones = lambda rows, operand: torch.full((abi.sf_bytes(rows, k, operand),), 127, dtype=torch.uint8, device=DEV)
+    none = lambda rows: torch.empty((rows, 0), dtype=torch.uint8, device=DEV)
+    empty = torch.empty(0, dtype=torch.uint8, device=DEV)
+
+    def product(w, **kw):
+        return abi.matmul(a, w, none(1), none(w.shape[0]), none(1), none(w.shape[0]), ones(1, abi.MG_OPERAND_A),
+                          ones(w.shape[0], abi.MG_OPERAND_B), empty, empty, empty, empty, **kw)
+
+    d = product(b, out=torch.full((1, n), float("nan"), dtype=torch.bfloat16, device=DEV))
+    assert not bool(torch.isnan(d).any())
+    for at in (0, (1 << 22) * tf - part // 2, n - part):
+        want = product(b[at:at + part].contiguous())
+        torch.cuda.synchronize()
+        assert torch.equal(d[:, at:at + part], want), f"features {at} ... {at + part}"
+
+
 def _seeded_shapes(count, seed):
     """Shapes drawn across the dispatcher's cases: token counts on both sides of 256 and of whole tiles, feature
     counts with and without whole 256-feature tiles, segments of 0 or 32..1024 channels in steps of 32."""

@@ -38,3 +38,10 @@ def test_every_tile_of_grids_beyond_a_32_bit_reciprocal(check):
         if n * m < 4_000_000 and n * m * m >= 1 << 32:
             grids.append((n, m, *rng.choice(FORMS)))
     assert check(grids) == []
+
+
+def test_grids_of_more_tiles_than_one_row_of_workgroups_takes(check):
+    """Fewer than 2^32 threads along a dimension: 4194304 workgroups of 768."""
+    most = 1 << 22
+    grids = [(most - 1, 1), (most, 1), (most + 1, 1), (1, most + 1), (5593752, 1), (11187503, 1), (2, 4194305), (3001, 2003)]
+    assert check([(n, m, *f) for n, m in grids for f in FORMS]) == []
