@@ -24,6 +24,18 @@ int main() {
       }
       seen[(size_t)tn * tiles_m + tm] = true;
     }
+    // where the counts do not divide into rectangles, an XCD's tiles are a run in feature-major order
+    for (int xcd = 0; xcd < 8 && (nwg & 7) != 0; ++xcd) {
+      int tn, tm, next = -1;
+      for (int wg = xcd; wg < nwg; wg += 8) {
+        mg::tile_at(order, wg, tn, tm);
+        if (next >= 0 && tn * tiles_m + tm != next) {
+          printf("%d x %d tiles of %d x %d: no run on XCD %d at workgroup %d\n", tiles_n, tiles_m, tf, tt, xcd, wg);
+          break;
+        }
+        next = tn * tiles_m + tm + 1;
+      }
+    }
     ++grids;
   }
   printf("%d grids\n", grids);
