@@ -1172,16 +1172,24 @@ static GemmChoice choose_gemm(const DecodeSeg& d4, const DecodeSeg& d6, const De
   }
   // What no other kernel takes, whatever the number of tokens, goes to small tiles; so does what they are estimated to be the
   // fastest for by a margin (the estimates of both sides are off by 10 %), above 16 tokens.  Both weight layouts go the same way
-  // there (they give the same bits): the estimates compared are those on
-  // tile-major weights.  Below 256 tokens the kernel taken is in the mean 0.7 % slower than the best one with the weights in the
-  // caches (1542 calls) and 0.03 % from HBM (710 calls), where the skinny kernel keeps more on its way: 128 tokens, N = K = 4096,
-  // the nearest of the estimates, 9.6 against 8.2 us on small tiles in the caches, 10.8 against 10.9 from HBM (row-major 10.7
-  // against 11.3).
+  // there (they give the same bits): the estimates compared are those on tile-major weights.
+  // (128 tokens, N = K = 4096, the nearest of the estimates: 9.6 against 8.2 us on small tiles with the weights in the caches, 10.8
+  // against 10.9 from HBM.)
+  // The margins: 5 %; 0.6 us more against the skinny kernel up to 9 steps, where the launch ramps are all there is (from HBM, small tile
+  // against skinny: M = 18, N = 2560, K = 1024 5.0 against 3.3 us, M = 21, N = 8360 5.4 against 4.6); 7 % against whole tiles below 256
+  // tokens where the small ones need a second round (M = 171, N = 20480, K = 11008, row-major 48.6 against 44.3).
+  // Against the choice between the other kernels alone, 4882 drawn calls of 17 ... 255 tokens: 1.22 times as fast in the mean with the
+  // weights in the caches, 1.17 from HBM, 13 of them slower by more than 3 %; 2297 of 256 ... 3000 tokens: 1.22 and 1.24, 4 slower.  Most
+  // of these are row-major weights of 100 MB and more in a tile or two of tokens (M = 23, N = 17984, K = 13824 43.6 against 41.8), at worst N =
+  // 16440, K = 18944 as MXFP4 and MXFP8, M = 19 67 against 52 us; the mean over their neighbours is 1.05.
   c.tile = mixed_gemm_tile_plan(M, N, KN, KS, KO, cus);
   const SkinnyPlan skinny_t = few ? skinny_plan(M, N, steps, cus, true) : SkinnyPlan{0, 0, 0.0};
   const double whole_us = few ? pipelined_us(M, N, steps, KN, KS, KO, cus) : whole_tiles_us(M, N, steps, KN, KS, KO, cus);
-  const double others = few ? (whole_tiles ? fmin(whole_us, skinny_t.us) : skinny_t.us) : whole_us;
-  if ((!whole_tiles && !skinny_ok) || ((M > 16 || !few) && c.tile.us < 0.95 * others)) {
+  const bool second_round = (int64_t)ceil_div(N, c.tile.tf) * ceil_div(M, c.tile.tt) > cus;
+  const bool before_whole = c.tile.us < (few && second_round ? 0.93 : 0.95) * whole_us;
+  const bool before_skinny = c.tile.us + (steps <= 9 ? 0.6 : 0.0) < 0.95 * skinny_t.us;
+  const bool fastest = few ? M > 16 && before_skinny && (!whole_tiles || before_whole) : before_whole;
+  if ((!whole_tiles && !skinny_ok) || fastest) {
     c.kernel = GemmKernel::kTile;
     return c;
   }

@@ -328,3 +328,18 @@ def test_segments_of_4_gb_of_row_major_weights_never_meet_32_bit_offsets(abi, cu
                 assert tf >= 64 and tt >= 64
         if (line - 1) % 8:                             # (not for whole tiles: the choice above does not depend on them)
             assert abi.gemm_kernel(1, line - 1, kn, ks, ko, cus=cus)[0] in ("skinny", "decode")
+
+
+@pytest.mark.parametrize("m,n,kn,ks,ko,others", [
+    # few stages: the skinny kernel, whose launch ramp is the shorter one
+    (18, 2560, 640, 256, 128, True), (34, 3072, 1024, 0, 0, True), (49, 2560, 1024, 0, 0, True), (21, 8360, 640, 256, 128, True),
+    (17, 10328, 640, 256, 128, True), (21, 9240, 768, 256, 128, True),
+    # a second round of small tiles against one of half tiles
+    (149, 20480, 2304, 1152, 128, True), (171, 20480, 11008, 0, 0, True),
+    # ... and where small tiles are the faster ones
+    (49, 9600, 1024, 0, 0, False), (85, 8192, 640, 256, 128, False), (140, 18944, 5120, 2816, 256, False), (136, 18944, 11968, 0, 128, False),
+])
+def test_small_tiles_are_not_taken_where_they_were_measured_slower(abi, m, n, kn, ks, ko, others):
+    for tiled in (False, True):
+        if not tiled or abi.weights_tileable(n, kn, ks, ko):
+            assert (abi.gemm_kernel(m, n, kn, ks, ko, tiled)[0] != "tile") == others
