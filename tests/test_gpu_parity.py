@@ -743,7 +743,8 @@ def test_exact_size_activation_buffers_on_the_whole_tile_kernel(abi, m, n, kn, k
 
 # Small tiles (64 x 64, 128 x 64, 128 x 128): token counts at and past the edges of 64 and 128, feature counts of whole, ragged and
 # single tiles, fewer stages than the ring holds, a last batch that is not whole, batches across segment boundaries (stage counts
-# that are no multiples of 2 and 4), empty segments, 1 to 3 blocks past the whole stages, a segment without a whole stage.
+# that are no multiples of 2 and 4), empty segments, 1 to 3 blocks past the whole stages, a segment without a whole stage.  (The two
+# of fewer than 256 tokens lie on the other side of the dispatcher's line and run on the skinny kernel.)
 SMALL_TILE_SHAPES = [
     (256, 256, 128, 128, 128), (257, 264, 128, 0, 0), (319, 1000, 0, 256, 128), (320, 520, 640, 384, 128), (321, 768, 1152, 640, 256),
     (450, 1001, 1152, 640, 256), (300, 60, 416, 224, 96), (300, 40, 64, 32, 0), (511, 1280, 480, 480, 480), (256, 8, 32, 0, 0),
@@ -752,10 +753,8 @@ SMALL_TILE_SHAPES = [
 ]
 
 
-@pytest.mark.parametrize("m,n,kn,ks,ko", SMALL_TILE_SHAPES)
-def test_small_tiles_match_oracle(abi, m, n, kn, ks, ko):
+def _check_small_tiles(abi, m, n, kn, ks, ko):
     """Row-major against the oracle, tile-major weights and exact-size activation buffers bit for bit like them."""
-    _say("small tiles", m, n, kn, ks, ko)
     k = kn + ks + ko
     x = H.make_activations(m, k, 81 + m, n_out=max(1, k // 32))
     w = H.make_weights(n, k, 82 + n)
@@ -773,6 +772,38 @@ def test_small_tiles_match_oracle(abi, m, n, kn, ks, ko):
         d_tiled = abi.matmul(*args(tight, abi.tile_weights(*bq[:3])), w_tiled=True)
         torch.cuda.synchronize()
         assert torch.equal(d, d_tiled)
+
+
+@pytest.mark.parametrize("m,n,kn,ks,ko", SMALL_TILE_SHAPES)
+def test_small_tiles_match_oracle(abi, m, n, kn, ks, ko):
+    _say("small tiles", m, n, kn, ks, ko)
+    _check_small_tiles(abi, m, n, kn, ks, ko)
+
+
+# Every instance (tile, weights' layout, with and without blocks past the whole stages) with more E2M1 stages than its ring holds and
+# at least two whole batches of each later segment, so that all three refill it; a last batch that is whole and one that is not,
+# batches of two segments, ragged token counts below and above 256.
+RING_SHAPES = [
+    (64, 64, 262, 256, 2816, 1024, 1280), (64, 64, 69, 5632, 2304, 1024, 1152), (64, 64, 70, 5632, 2720, 1120, 1440),
+    (64, 64, 267, 256, 2912, 1184, 1088),
+    (128, 64, 145, 5632, 1408, 512, 640), (128, 64, 296, 3328, 1408, 512, 512), (128, 64, 460, 2304, 1440, 576, 704),
+    (128, 64, 137, 5632, 1504, 1056, 576),
+    (128, 128, 399, 4864, 1408, 640, 512), (128, 128, 333, 5632, 1408, 512, 512), (128, 128, 390, 5120, 1440, 736, 576),
+    (128, 128, 339, 5632, 1504, 608, 544),
+]
+
+
+@pytest.mark.parametrize("tf,tt,m,n,kn,ks,ko", RING_SHAPES)
+def test_small_tiles_refill_their_ring(abi, tf, tt, m, n, kn, ks, ko):
+    _say("rings of small tiles", tf, tt, m, n, kn, ks, ko)
+    cus = torch.cuda.get_device_properties(0).multi_processor_count
+    for w_tiled in (False, True):
+        assert abi.gemm_kernel(m, n, kn, ks, ko, w_tiled, cus) == ("tile", tf, tt)
+    stage = 1024 + 64 * tf + 128 * tt                      # bytes in LDS: scales, weights, tokens
+    batch = 4 if tf == tt == 64 else 2                     # stages per barrier
+    ring = min(8, 156 * 1024 // (batch * stage)) * batch   # stages in the ring
+    assert kn // 128 >= ring + batch and min(ks, ko) // 128 >= 2 * batch
+    _check_small_tiles(abi, m, n, kn, ks, ko)
 
 
 @pytest.mark.parametrize("m", [1, 8, 16, 17])
