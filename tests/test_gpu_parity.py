@@ -961,6 +961,8 @@ def test_tiled_flag_is_refused_for_shapes_that_cannot_be_tiled(abi):
     (1030, 256, 128, 128, 1e-5),     # more rows than resident workgroups: several rows per workgroup
     (5, 20480, 11264, 992, 1e-5),    # K = 32736, the largest: the kernel with a run-time workgroup size (1024 lanes)
     (300, 15360, 8448, 768, 1e-6),   # K = 24576 on the same kernel, two rows per workgroup for some
+    # two lanes per block, whose gathered channels are normalized in registers, in workgroups of 3, 5, 6 and 7 waves, whole and not
+    (6, 1920, 1024, 64, 1e-5), (9, 3200, 1792, 128, 1e-5), (5, 3840, 2112, 160, 1e-6), (1200, 4480, 2432, 256, 1e-5),
 ])
 def test_rmsnorm_reorder_quantize_matches_oracle(abi, rows, kn, ks, ko, eps):
     k = kn + ks + ko

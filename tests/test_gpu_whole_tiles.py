@@ -1,0 +1,85 @@
+"""The GEMM on whole tiles (256 x 256 and 256 x 128): every instance of the kernel, bit for bit.
+
+The kernel is compiled per set of segments, length of the last segment, tile, weight layout, and with or without segment boundaries in
+the K loop and blocks past the whole stages.  Each of these runs here, on a shape that the dispatcher gives to it."""
+import numpy as np
+import pytest
+import torch
+
+from oracle import mx_oracle as mo
+
+pytestmark = pytest.mark.gpu
+
+DEV = "cuda"
+FORMATS = ("e2m1", "e3m2", "e4m3")
+
+
+@pytest.fixture(scope="module")
+def abi():
+    from mixedgemm_amd import abi as module
+    module.lib()
+    return module
+
+
+# last segments of 1, 2 and 3 stages behind segments of fewer than 3 stages (2) and more; one, two and three segments; 1 to 3 blocks of
+# 32 past the whole stages
+SPLITS = (
+    [s for a in (256, 512) for last in (128, 256, 384) for s in ((a, last, 0), (a, 0, last), (0, a, last))]
+    + [(512, 0, 0), (0, 512, 0), (0, 0, 512)]
+    + [(a, b, last) for a in (256, 512) for b in (256, 512) for last in (128, 256, 384)]
+    + [s for last in (160, 288, 416) for s in ((544, 448, last), (416, 160, last))]
+)
+# 148 tiles of 256 x 128, the last 44 tokens long; 135 tiles of 256 x 256; 272 of them, the last 16 as half tiles; ragged tokens and features
+SIZES = [(300, 18944), (2304, 3840), (4352, 4096), (4300, 4104)]
+
+
+def _table(fmt):
+    """(codes, their values): all of a format, of E4M3 those up to 16 that are multiples of 1/16."""
+    codes = np.arange(1 << mo.BITS[fmt])
+    values = mo.decode_codes(codes, fmt).astype(np.float64)
+    if fmt == "e4m3":
+        keep = np.isfinite(values) & (np.abs(values) <= 16) & (np.mod(values * 16, 1) == 0)
+        codes, values = codes[keep], values[keep]
+    return torch.from_numpy(codes).to(DEV), torch.from_numpy(values).to(DEV)
+
+
+def _operand(rows, kseg, fmt, operand, g):
+    """Packed codes, scale buffer and values (fp64) of random codes with scales of 1/2, 1 and 2."""
+    codes, values = _table(fmt)
+    pick = torch.randint(0, len(codes), (rows, kseg), device=DEV, generator=g)
+    c = codes[pick].int()
+    if fmt == "e2m1":
+        packed = c[:, 0::2] | c[:, 1::2] << 4
+    elif fmt == "e3m2":   # a little-endian stream of 6-bit codes
+        word = c[:, 0::4] | c[:, 1::4] << 6 | c[:, 2::4] << 12 | c[:, 3::4] << 18
+        packed = torch.stack((word & 255, word >> 8 & 255, word >> 16), dim=2).flatten(1)
+    else:
+        packed = c
+    scale = torch.randint(126, 129, (rows, kseg // 32), device=DEV, generator=g)
+    buffer = torch.from_numpy(mo.sf_scatter(scale.to(torch.uint8).cpu().numpy(), kseg, operand)).to(DEV)
+    return packed.to(torch.uint8).contiguous(), buffer, values[pick] * torch.exp2((scale - 127).double()).repeat_interleave(32, dim=1)
+
+
+@pytest.mark.parametrize("m,n", SIZES)
+@pytest.mark.parametrize("kn,ks,ko", SPLITS)
+def test_every_instance_of_the_whole_tile_kernel(abi, m, n, kn, ks, ko):
+    """Products are multiples of 2^-7 and their absolute values sum up to less than 2^17, so that every fp32 sum in any order is the
+    exact one: the result is the fp64 product rounded once."""
+    print("whole tiles", m, n, kn, ks, ko, flush=True)
+    cus = torch.cuda.get_device_properties(0).multi_processor_count
+    tileable = abi.weights_tileable(n, kn, ks, ko)
+    assert abi.gemm_kernel(m, n, kn, ks, ko, False, cus)[0] == "whole" and (not tileable or abi.gemm_kernel(m, n, kn, ks, ko, True, cus)[0] == "whole")
+    g = torch.Generator(device=DEV).manual_seed(m + 3 * kn + 5 * ks + 7 * ko)
+    a = [_operand(m, k, fmt, "a", g) for k, fmt in zip((kn, ks, ko), FORMATS)]
+    b = [_operand(n, k, "e2m1", "b", g) for k in (kn, ks, ko)]
+    av, bv = torch.cat([x[2] for x in a], dim=1), torch.cat([x[2] for x in b], dim=1)
+    assert float((av.abs() @ bv.abs().T.contiguous()).max()) < 2 ** 17
+    want = (av @ bv.T.contiguous()).to(torch.float32).to(torch.bfloat16)
+    scales = (a[0][1], b[0][1], a[1][1], b[1][1], a[2][1], b[2][1])
+    layouts = [([x[0] for x in b], False)]
+    if tileable:
+        layouts.append((abi.tile_weights(*(x[0] for x in b)), True))
+    for w, w_tiled in layouts:
+        d = abi.matmul(a[0][0], w[0], a[1][0], w[1], a[2][0], w[2], *scales, w_tiled=w_tiled)
+        torch.cuda.synchronize()
+        assert torch.equal(d.view(torch.int16), want.view(torch.int16)), f"w_tiled={w_tiled}: {int((d != want).sum())} of {d.numel()} differ"
