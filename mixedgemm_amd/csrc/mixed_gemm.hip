@@ -1121,7 +1121,8 @@ hipError_t launch_mixed_gemm_tile(const uint8_t* an, const uint8_t* bn, const ui
 // Rough launch time of the whole-tile kernel in microseconds for fewer than 256 tokens, only to choose between the kernels: as
 // 256 x 128 tiles when that is at most one round (fitted to 771 calls on tile-major weights, rms error 8 %), else as 256 x 256.
 // What the blocks past whole stages, the hand-over between three segments and an E3M2 segment shorter than its pipeline cost is
-// counted: with 4.5 us for the last (K = 1024: N = 24576, M = 64 was 12.9 us here, and is 6.4 on small tiles).
+// counted: with 4.5 us for the last (K = 1024: N = 24576, M = 64 was 12.9 us here, and is 6.4 on small tiles; not counted for more than
+// cus / 2 whole tiles).
 static bool short_middle(int KN, int KS, int KO) { return KN > 0 && KO > 0 && KS > 0 && KS < 384; }
 static double pipelined_us(int M, int N, int stages, int KN, int KS, int KO, int cus) {
   const int whole = ceil_div(M, 256) * ceil_div(N, 256), halves = ceil_div(M, 128) * ceil_div(N, 256);

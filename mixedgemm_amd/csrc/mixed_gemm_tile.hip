@@ -7,14 +7,17 @@
 // the L2), so that waves that copy and multiply in turn leave the matrix cores idle.  Here four waves, one per SIMD, issue
 // all copies, eight waves, two per SIMD, read fragments and multiply, and one barrier hands over WS stages at a time, each of them the
 // work of 8 / WS of the math waves (fragments are read once per 2 x 2 tiles of 32 x 32 rather than once per 1 x 2).
-// What bounds it now (stamps of an instrumented build): LDS bandwidth, ~16 cycles per KB copied and 4.4 per KB read: 64 x 64 tiles, K =
-// 4096, one per CU: 270 cycles per stage, of which 64 are MFMAs' (150 without copies); a launch of them takes 1.2 us until the
-// first stages have landed, 2.7 us for 20 E2M1 and 1.3 for 12 later stages, 1.2 us to add the partial sums and store.
-// Tile-major / row-major weights, of two or three layers in turn, before (skinny kernel or 256 x 128 tiles) -> now, us:
+// What bounds it now: with many stages the copies (address unit busy 72 % of the cycles on tile-major and 77 % on row-major weights at
+// M = 256, N = 4096, K = 14336, where the matrix cores are 19 and 16 %, the LDS's fragment reads 25 %), with 32 stages latency as well
+// (address unit 45 ... 65 %, waves waiting 50 ... 63 %; M = 1024, N = K = 4096: matrix cores 29 and 25 %).  Clock stamps of an instrumented
+// build: 64 x 64 tiles, K = 4096, one per CU: 270 cycles per stage, of which 64 are MFMAs' (150 without copies); a launch of them takes 1.2
+// us until the first stages have landed, 2.7 us for 20 E2M1 and 1.3 for 12 later stages, 1.2 us to add the partial sums and store.
+// Tile-major / row-major weights, of two or three layers in turn in the caches, before (skinny kernel or 256 x 128 tiles) -> now, us:
 //   M = 256, N = 4096, K = 4096: 16.4 / 19.6 -> 8.3 / 8.6;   K = 14336: 45.6 / 59.9 -> 20.2 / 22.3
 //   M = 512, N = 4096, K = 4096: 16.6 / 19.6 -> 10.0 / 12.0;  N = 1024, K = 8192: 27.6 / 34.8 -> 11.6 / 13.2
 //   M = 64, N = 14336, K = 4096: 16.4 / 16.8 -> 8.8 / 9.3;   M = 128: 16.8 / 20.1 -> 10.1 / 12.3
-//   M = 1024, N = 4096, K = 4096: 17.0 / 19.7 -> 14.7 / 17.0
+//   M = 1024, N = 4096, K = 4096: 17.0 / 19.7 -> 14.5 / 16.5
+// (from HBM: M = 256 10.6 / 10.8 and 30 / 30, M = 512 12.5 / 15.2 and 16.1 / 16.0, M = 64 13.7 / 14.1, M = 1024 17.6 / 19.2)
 // Tiles of 256 x 128 with the same division of work were level with the mixed waves of the 256 x 256 kernel (M = 2048, N =
 // 4096, K = 12288: 57.6 against 56.3 us: 15 % fewer cycles at a clock as much lower; the chip is at its power limit there), tiles of
 // 64 and 128 x 32 slower than 64 x 64 at every shape tried.
@@ -120,8 +123,8 @@ struct TileCtx {
 // Tile-major weights (16 KB per 256 features and stage: 1 KB per j = feature % 16, in it 64 bytes per feature / 16, even ones
 // first): a copy takes what the tile's features have of 128 / TF blocks of 1 KB, whole lines, and row i of a 32-row fragment is the
 // feature that WeightRows says.  (A workgroup has consecutive features: with whole 1 KB blocks, i.e. every other run of eight, two
-// workgroups shared each line of the result: M = 1024, N = K = 4096 from warm L2s 17.1 us, now 13.9; with one feature's 64 bytes
-// per four lanes, half lines, M = 256, N = 4096, K = 14336 21.9 us, now 20.2.)
+// workgroups shared each line of the result: M = 1024, N = K = 4096 with the same operands in each launch 17.1 us, now 13.9; with one
+// feature's 64 bytes per four lanes, half lines, M = 256, N = 4096, K = 14336 21.9 us, now 20.2.)
 // ---------------------------------------------------------------------------------------------
 // Rows of a weight fragment.  Row-major: row i of fragment T is feature 32 T + i of the tile, in copy block 2 T + i / 16.
 // Tile-major, 128 features: copy block j / 2 holds [j % 2][feature / 16 % 2][feature / 32]; 64: j / 4 [j % 4][...][...].  Four
@@ -659,7 +662,8 @@ struct TilePlanChoice { int tf, tt; double us; };
 
 // The tile with the lowest estimate.  A workgroup has its CU to itself (LDS), so a launch is rounds of them; microseconds: fixed,
 // per round, per stage and round, per stage with all CUs busy, per MB of results, per round with blocks past the whole stages.
-// Fitted to 450 measured calls each (17 ... 2600 tokens, N 384 ... 28672, K 1024 ... 18944, tile-major weights; rms error 10 %):
+// Fitted to 450 measured calls each (17 ... 2600 tokens, N 384 ... 28672, K 1024 ... 18944, tile-major weights; rms error 10 %,
+// before the runs of tiles per XCD of tile_order.h, which made launches of other than 8 n tiles up to 1.4 times as fast):
 // the tile taken is in the mean 0.5 % slower than the best of the three.  Long launches are held back by the clock that the power
 // limit leaves: no faster than the table's PFLOP/s on whole tiles (M = 1894, N = 8448, K = 13824: 198 us where the sum says 135, 170
 // on 256 x 256 tiles; over 55 calls of 35 ... 135 us the choice against those is then the faster one every time).

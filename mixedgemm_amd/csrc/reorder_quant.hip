@@ -382,7 +382,7 @@ reorder_quant_dma_kernel(const uint8_t* __restrict__ x, const int16_t* __restric
     if constexpr (NORM) {
       // RMSNorm of the row (the arithmetic of the usual fp32 implementation):
       //   var = fl32( (sum over the row of x^2, accumulated in fp64) / K )
-      //   r   = fl32( 1 / sqrt( fl32(var + eps) ) )      (division and square root in fp64)
+      //   r   = fl32( 1 / sqrt( fl32(var + eps) ) )      (quotient and root to a unit in the last place of a double: rms_scale)
       //   y   = bf16( gamma * bf16( x * r ) )            (both products in fp32)
       // The fp64 sum makes the result independent of the order in which the lanes add their parts (up to the last
       // bit of a double, which the rounding to fp32 all but never sees).  A lane sums over the pieces it copied.

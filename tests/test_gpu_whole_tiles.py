@@ -29,8 +29,9 @@ SPLITS = (
     + [(a, b, last) for a in (256, 512) for b in (256, 512) for last in (128, 256, 384)]
     + [s for last in (160, 288, 416) for s in ((544, 448, last), (416, 160, last))]
 )
-# 148 tiles of 256 x 128, the last 44 tokens long; 135 tiles of 256 x 256; 272 of them, the last 16 as half tiles; ragged tokens and features
-SIZES = [(300, 18944), (2304, 3840), (4352, 4096), (4300, 4104)]
+# 224 tiles of 256 x 128, half of them without their last token; 135 tiles of 256 x 256, 148 of which every other one has 44 tokens, 272 of
+# which the last 16 run as half tiles; ragged tokens and features
+SIZES = [(255, 28672), (2304, 3840), (300, 18944), (4352, 4096), (4300, 4104)]
 
 
 def _table(fmt):
