@@ -172,16 +172,16 @@ GEMM_SHAPES = [
     # 17 to 255 tokens: ragged M and N, partial K steps (skinny kernel), an empty segment
     (17, 48, 256, 128, 128), (32, 200, 96, 160, 64), (50, 40, 2560, 1408, 128), (64, 64, 0, 4928, 448),
     (100, 256, 448, 224, 64), (128, 4096, 2560, 1408, 128), (255, 272, 128, 128, 128), (200, 1000, 640, 256, 256),
-    # ragged token counts: the last 256-row tile stores only part of its rows
+    # ragged token counts: the last tile stores only part of its rows
     (300, 512, 2560, 1408, 128), (257, 256, 384, 384, 384), (767, 256, 448, 416, 224),
-    # plans without E3M2 and / or E4M3 activations on the whole-tile kernel (fragments pass to the next segment that exists)
+    # plans without E3M2 and / or E4M3 activations (fragments pass to the next segment that exists)
     (256, 256, 512, 0, 0), (512, 512, 128, 0, 0), (300, 256, 384, 0, 128), (256, 512, 1024, 0, 256), (256, 256, 384, 256, 0),
     (300, 512, 2560, 1536, 0), (1000, 256, 4096, 0, 0), (256, 256, 512, 0, 384), (256, 256, 384, 128, 0),
     # feature counts that are not whole 256-feature tiles (multiples of 8): the last tile's lanes read the last
     # weight row again and store only the pieces that exist
     (300, 1000, 2560, 1408, 128), (256, 264, 384, 384, 384), (512, 136, 448, 416, 224), (700, 8, 128, 128, 128),
     (256, 392, 512, 0, 0), (384, 648, 384, 0, 128),
-    # plans without E2M1 activations on the whole-tile kernel: pure E3M2 x E2M1 and E4M3 x E2M1 products (the reference's
+    # plans without E2M1 activations: pure E3M2 x E2M1 and E4M3 x E2M1 products (the reference's
     # matmul_host6 / matmul_host8 alone), E3M2 + E4M3 with and without three stages in the first of them; and plans
     # whose first segment is shorter than three stages next to an empty one (run-time segment-boundary copies)
     (256, 256, 0, 256, 0), (512, 256, 0, 1024, 0), (300, 264, 0, 128, 0), (256, 256, 0, 0, 128), (256, 512, 0, 0, 640),
@@ -277,7 +277,8 @@ def test_mixed_gemm_matches_oracle(abi, m, n, kn, ks, ko):
     _check_gemm(d, qx, qw, f"gemm {m}x{n}x{k}")
 
 
-# More than 128 whole tiles: 256 x 256 tiles (smaller problems run 256 x 128).  One plan per kernel family: all three
+# More than 128 whole tiles: 256 x 256 tiles (smaller problems run 256 x 128; (1024, 2048) and (2048, 4096, 256, 128, 128) run on small
+# tiles).  One plan per kernel family: all three
 # segments with a last segment of 1, 2 and 3 stages (the kernels are compiled per length of the last segment),
 # segments with a remainder, and the plans with an empty segment.
 BIG_TILE_SHAPES = [
@@ -364,7 +365,7 @@ def test_gemm_operand_bit_order_one_hot(abi, seg):
 
 @pytest.mark.parametrize("m,n,kn,ks,ko", [
     (96, 256, 2560, 1408, 128),
-    # ragged token counts: the last 256-row tile reads rows past M from the padded buffers and does not write them
+    # ragged token counts: the last tile reads rows past M from the padded buffers and does not write them
     (300, 512, 2560, 1408, 128), (130, 2560, 384, 384, 384), (1000, 256, 448, 416, 224), (255, 4096, 2560, 896, 128),
     (70, 14336, 2560, 1408, 128),
 ])
@@ -718,7 +719,9 @@ def test_mixed_tile_heights_equal_the_plain_launch_bit_for_bit(abi, m, m_part, n
 def test_exact_size_activation_buffers_on_the_whole_tile_kernel(abi, m, n, kn, ks, ko):
     """Activation buffers with no room past row M: the lanes of the last tile that would read past the last row
     read that row again, and the result equals the padded-buffer one bit for bit.  Row counts around the lengths
-    of the runs of rows a lane copies (2, 4, 8), the 16-row copy blocks and the second scale atom (128 rows)."""
+    of the runs of rows a lane copies (2, 4, 8), the 16-row copy blocks and the second scale atom (128 rows).
+    (At these sizes small tiles and the skinny kernel are the faster ones and run; whole tiles at the same row counts:
+    test_gpu_whole_tiles.py.)"""
     _say("exact-size", m, n, kn, ks, ko)
     k = kn + ks + ko
     x = H.make_activations(m, k, 71 + m, n_out=max(1, k // 32))
@@ -898,7 +901,7 @@ def _seeded_shapes(count, seed):
 
 
 def _seeded_tile_shapes(count, seed):
-    """Shapes the whole-tile kernel takes: ragged token counts, segments of whole stages or with 32, 64, 96 channels
+    """Shapes that the whole-tile kernel can take (small tiles are mostly faster): ragged token counts, segments of whole stages or with 32, 64, 96 channels
     past them, with and without three stages before a boundary, plans without E3M2 and / or E4M3."""
     rng = np.random.default_rng(seed)
     out = []

@@ -61,11 +61,9 @@ def _operand(rows, kseg, fmt, operand, g):
     return packed.to(torch.uint8).contiguous(), buffer, values[pick] * torch.exp2((scale - 127).double()).repeat_interleave(32, dim=1)
 
 
-@pytest.mark.parametrize("m,n", SIZES)
-@pytest.mark.parametrize("kn,ks,ko", SPLITS)
-def test_every_instance_of_the_whole_tile_kernel(abi, m, n, kn, ks, ko):
+def _check(abi, m, n, kn, ks, ko):
     """Products are multiples of 2^-7 and their absolute values sum up to less than 2^17, so that every fp32 sum in any order is the
-    exact one: the result is the fp64 product rounded once."""
+    exact one: the result is the fp64 product rounded once.  The activation buffers end with row m."""
     print("whole tiles", m, n, kn, ks, ko, flush=True)
     cus = torch.cuda.get_device_properties(0).multi_processor_count
     tileable = abi.weights_tileable(n, kn, ks, ko)
@@ -84,3 +82,17 @@ def test_every_instance_of_the_whole_tile_kernel(abi, m, n, kn, ks, ko):
         d = abi.matmul(a[0][0], w[0], a[1][0], w[1], a[2][0], w[2], *scales, w_tiled=w_tiled)
         torch.cuda.synchronize()
         assert torch.equal(d.view(torch.int16), want.view(torch.int16)), f"w_tiled={w_tiled}: {int((d != want).sum())} of {d.numel()} differ"
+
+
+@pytest.mark.parametrize("m,n", SIZES)
+@pytest.mark.parametrize("kn,ks,ko", SPLITS)
+def test_every_instance_of_the_whole_tile_kernel(abi, m, n, kn, ks, ko):
+    _check(abi, m, n, kn, ks, ko)
+
+
+# around the lengths of the runs of rows that a lane copies (2, 4, 8), the copy blocks of 16 rows and the second scale atom: tiles of 256 x 128
+# (16384 features; fewer than 256 tokens) and of 256 x 256
+@pytest.mark.parametrize("m,n", [(m, n) for m in (257, 258, 261, 263, 271, 272, 273, 384, 385, 511) for n in (16384, 28672)] + [(129, 28672), (200, 28672)])
+@pytest.mark.parametrize("kn,ks,ko", [(480, 448, 160), (384, 384, 256)])
+def test_rows_up_to_the_last_one_on_whole_tiles(abi, m, n, kn, ks, ko):
+    _check(abi, m, n, kn, ks, ko)
