@@ -39,13 +39,13 @@ MEASURED_TRAFFIC = {
     "gemm_c3": {"bytes": int((110305.8 * 1.99983 + 114721.1 * 1.0) * 1024),      # 343 MB against 159 MB algorithmic: operands re-read 5.5x past L2
                 "source": "mixedgemm_amd/csrc/mixed_gemm_256.hip", "sha": "48aa4ca44f075236"},
     "quant_c1": {"bytes": int((16463.5 * 1.99983 + 10524.5 * 1.0) * 1024),       # 44.5 MB against 44.2 MB algorithmic
-                 "source": "mixedgemm_amd/csrc/reorder_quant.hip", "sha": "a0c72180cdddeb67"},
+                 "source": "mixedgemm_amd/csrc/reorder_quant.hip", "sha": "bc16441704e8f575"},
     "quant_w_c3": {"bytes": int((57431.0 * 1.99983 + 30849.8 * 1.0) * 1024),     # 149.2 MB against 148.6 MB algorithmic
-                   "source": "mixedgemm_amd/csrc/reorder_quant.hip", "sha": "a0c72180cdddeb67"},
+                   "source": "mixedgemm_amd/csrc/reorder_quant.hip", "sha": "bc16441704e8f575"},
     "tile_w_c3": {"bytes": int((14412.5 * 1.99983 + 28672.0 * 1.0) * 1024),      # 58.9 MB against 58.7 MB (three launches)
                   "source": "mixedgemm_amd/csrc/mixed_gemm_256.hip", "sha": "48aa4ca44f075236"},
     "decode_c2": {"bytes": int((15416.0 * 1.99983 + 224.0 * 1.0) * 1024),        # 31.8 MB against 31.4 MB algorithmic (tile-major weights)
-                  "source": "mixedgemm_amd/csrc/mixed_gemm.hip", "sha": "e02818cbe03feda7"},
+                  "source": "mixedgemm_amd/csrc/mixed_gemm.hip", "sha": "2ac458ac7f9d0388"},
     "calibrate_c1": {"bytes": int(((16427.0 + 286.0) * 1.99983 + (64.0 + 56.2) * 1.0) * 1024),   # two kernels: 34.3 MB against 33.6 MB
                      "source": "mixedgemm_amd/csrc/calibrate.hip", "sha": "71587112b192334b"},
 }
