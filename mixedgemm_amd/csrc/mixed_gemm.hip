@@ -25,6 +25,7 @@
 
 #include "mg_common.h"
 #include "quantize.h"
+#include "tile_order.h"
 
 namespace mg {
 
@@ -70,7 +71,9 @@ __device__ __forceinline__ void store1(uint16_t* __restrict__ d, const Epilogue&
 // each, counted over the three segments) are dealt to the waves in contiguous quarters (as in the decode kernel below:
 // the same sums in the same order, whichever of the two a shape goes to).  Each wave runs a pipeline of its own: a
 // ring of NS slots in LDS, one step each (weight codes, token codes, the 16-byte pieces of the scale atoms that hold
-// its rows), filled by global -> LDS copies NS - 1 steps ahead and refilled as soon as its fragments are in registers.
+// its rows), filled by global -> LDS copies NS - 1 steps ahead and refilled as soon as its fragments are in registers,
+// whole steps two at a time: one wait for two steps' fragments.  Requests of whole steps are addresses that advance and offsets that
+// stay; the steps around a segment's end, and the first ones, are addressed one by one.
 // No barrier until the waves' partial 16x16 tiles are summed; nothing in flight occupies a register.
 //
 // What bounds it, from counters: a launch takes about 2.3 us + 0.07 ... 0.14 us per K step.  With few steps that is the
@@ -84,6 +87,10 @@ __device__ __forceinline__ void store1(uint16_t* __restrict__ d, const Epilogue&
 // of two layers in turn, K = 14336, N = 4096): M = 16 17.5 -> 11.0 us, 32 23 -> 12.2, 64 28 -> 13.1, 128 47 (whole-tile
 // kernel) -> 16.8, 200 47 -> 30.8; K = 4096, N = 4096, M = 128 9.0 -> 7.9 (decode kernel with 32 tokens per workgroup,
 // which this replaces).
+// Layer call (quantizer and this kernel) from HBM, tile-major weights, us, with eight slots, one step at a time -> shorter rings 8.9, two
+// steps at a time 8.75, all arguments fetched in one batch 8.55: M = 16, N = K = 4096 9.4 -> 8.55; M = 32, N = 4096, K = 14336 19.5 -> 18.3; M =
+// 128, N = K = 4096 13.8 -> 13.1 (eight slots of the form with half the features before); 370 calls of 1 ... 255 tokens 1.03 times as
+// fast in the mean, two of them 3 % slower (row-major weights in the caches, K = 6144).
 // ---------------------------------------------------------------------------
 struct DecodeSeg {
   const uint8_t* a;
@@ -101,6 +108,18 @@ __device__ __forceinline__ v4f decode_mfma(v8i wb, v8i xa, v4f acc, int sw, int 
 
 template <int N>
 __device__ __forceinline__ void wait_vmcnt() { asm volatile("s_waitcnt vmcnt(%0)" : : "n"(N) : "memory"); }
+
+// waits until at most `steps` (wave-uniform, at most MOST) steps of PER copies each are in flight
+template <int PER, int MOST>
+__device__ __forceinline__ void wait_steps(int steps) {
+  switch (steps) {
+#define MG_STEPS_CASE(N) case N: if constexpr (N <= MOST) { wait_vmcnt<N * PER>(); break; } [[fallthrough]];
+    MG_STEPS_CASE(1) MG_STEPS_CASE(2) MG_STEPS_CASE(3) MG_STEPS_CASE(4) MG_STEPS_CASE(5) MG_STEPS_CASE(6)
+    MG_STEPS_CASE(7) MG_STEPS_CASE(8) MG_STEPS_CASE(9) MG_STEPS_CASE(10) MG_STEPS_CASE(11)
+#undef MG_STEPS_CASE
+    default: wait_vmcnt<0>(); break;
+  }
+}
 
 template <bool STREAM = false>
 __device__ __forceinline__ void dma16_at(const uint8_t* base, unsigned voff, unsigned lds_off) {
@@ -125,24 +144,33 @@ __device__ __forceinline__ void dma16_lane(const uint8_t* p, unsigned lds_off) {
 // copies of 1 KB per step for 16 G tokens of a format
 template <int FMT, int G>
 constexpr int kTokenCopies = (16 * G * 4 * Frag<FMT>::kBytes + 1023) / 1024;
-// LDS bytes of a slot, and slots per wave
+// LDS bytes of a slot, and slots per wave.  Four slots, three where four do not fit: a wave that has more to request before its first step stands at
+// its requests -- a CU takes no more than some 40 KB of them ahead of the data -- while the first steps' data is there.  Layer call, M = 16, N = K =
+// 4096 from HBM with 3 / 4 / 5 / 6 / 8 / 12 slots 9.1 / 8.7 / 8.9 / 9.0 / 9.4 / 9.7 us, K = 14336 17.9 / 16.5 / 16.7 / 16.9 / 17.3 / 18.2.
 template <int G, int F>
-constexpr int kSkinnySlot = 1024 * (1 + F + 2 * G);
+constexpr int kSkinnyPieces = (G == 1 ? 16 : 32) + 4 * F;   // scale pieces of a step: tokens, weights
 template <int G, int F>
-constexpr int kSkinnySlots = 156 * 1024 / (4 * kSkinnySlot<G, F>) < 8 ? 156 * 1024 / (4 * kSkinnySlot<G, F>) : 8;
+constexpr int kSkinnySlot = 1024 * (F + 2 * G) + 16 * kSkinnyPieces<G, F>;
+template <int G, int F>
+constexpr int kSkinnySlots = 159 * 1024 / (4 * kSkinnySlot<G, F>) < 4 ? 3 : 4;
 
 template <int G, int F, bool WT>
 __global__ void __launch_bounds__(256)
-mixed_gemm_skinny_kernel(DecodeSeg s4, DecodeSeg s6, DecodeSeg s8, int M, int N, int steps_per_wave, Epilogue ep,
-                         uint16_t* __restrict__ d) {
+mixed_gemm_skinny_kernel(DecodeSeg s4, DecodeSeg s6, DecodeSeg s8, int M, int N, int steps_per_wave, TileOrder order,
+                         Epilogue ep, uint16_t* __restrict__ d) {
   constexpr int NS = kSkinnySlots<G, F>, kSlot = kSkinnySlot<G, F>;
   constexpr int PA = G == 1 ? 16 : 32, PB = 4 * F;   // scale pieces per step: tokens, weights
   // The widest layers' weight codes, whole lines that nobody reads again, as streaming loads: they leave the last-level cache to
   // what follows.  N = 28672, K = 4096, M = 16 from HBM 15.3 -> 14.2 us, 20480 13.4 -> 12.7 (from that cache 12.3 -> 13.3); a decoder
   // layer's four projections of 16 tokens, whose others (58 MB) then stay in it, 62.5 -> 56.3.
   constexpr bool kStream = WT && F == 8;
+  constexpr int kScales = 1024 * (F + 2 * G);   // where a slot's scales begin
   static_assert(NS >= 3 && PA + PB <= 64, "a pipeline; one copy for all scales of a step");
   extern __shared__ __align__(16) uint8_t lds[];
+  // all arguments in one batch of loads (see pin_args)
+  asm volatile("" : : "s"(s4.a), "s"(s4.sfb), "s"(s4.nblk), "s"(s4.steps), "s"(s6.a), "s"(s6.sfb), "s"(s6.nblk), "s"(s6.steps), "s"(s8.a),
+               "s"(s8.sfb), "s"(s8.nblk), "s"(s8.steps), "s"(M), "s"(N), "s"(steps_per_wave), "s"(order.xlog), "s"(order.magic),
+               "s"(order.tiles), "s"(ep.bias), "s"(ep.n_out), "s"(d));
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int i = lane & 15, g = lane >> 4;
   uint8_t* const ring = lds + wave * (NS * kSlot);
@@ -152,14 +180,13 @@ mixed_gemm_skinny_kernel(DecodeSeg s4, DecodeSeg s6, DecodeSeg s8, int M, int N,
 
   // ---- the workgroup's rows: the mapping of the decode kernel below (feature group f, lane row i -> its scale piece
   // and its dword in the piece), and the weight row this lane copies, row lane / 4 of the group
-  int wg = blockIdx.x;
-  if constexpr (WT) {   // the workgroups of a 256-feature tile on one XCD (see the decode kernel)
-    constexpr int kPer = 16 / F;
-    if ((int)gridDim.x % (8 * kPer) == 0) {
-      const int xcd = wg & 7, slot = wg >> 3;
-      wg = ((slot / kPer) * 8 + xcd) * kPer + slot % kPer;
-    }
-  }
+  // (an XCD has runs of workgroups: those of the same features, for other tokens, find the weights in its L2 -- M = 19, N = 7424, K =
+  // 18944, whose two token groups were on different XCDs, 31.9 -> 28.0 us --, and those of a 256-feature tile of tile-major weights
+  // put their sectors of the result together there, see the decode kernel)
+  const int launched = (int)blockIdx.x + order.grid_x * (int)blockIdx.y;
+  if (launched >= order.tiles) return;
+  int wg, token_group;
+  tile_at(order, launched, wg, token_group);
   constexpr int per_group = 32 / PB;
   const int tile = (wg * F) >> 4, j0 = (wg * F) & 15;                    // tile-major
   const int group = wg / per_group, c0 = (wg % per_group) * PB;          // row-major
@@ -175,7 +202,7 @@ mixed_gemm_skinny_kernel(DecodeSeg s4, DecodeSeg s6, DecodeSeg s8, int M, int N,
     else sw_off[f] = (PA + (16 * f + i) % PB) * 16 + ((16 * f + i) / PB) * 4 + g;
     wrow[f] = min(feature(f, lane >> 2), N - 1);   // rows past N: read again, never stored
   }
-  const int m_base = (int)blockIdx.y * 16 * G, last_row = min(M - m_base, 16 * G) - 1;
+  const int m_base = token_group * 16 * G, last_row = min(M - m_base, 16 * G) - 1;
   // the scale piece this lane copies, as an address in each segment's first step
   const uint8_t *sc4, *sc6, *sc8;
   {
@@ -202,11 +229,11 @@ mixed_gemm_skinny_kernel(DecodeSeg s4, DecodeSeg s6, DecodeSeg s8, int M, int N,
   auto request_seg = [&](auto fmt_c, const DecodeSeg& s, const uint8_t* sc, int q, unsigned slot) __attribute__((always_inline)) {
     constexpr int FMT = decltype(fmt_c)::value;
     const int left = min(s.nblk - 4 * q, 4);
-    dma16_lane(sc + (size_t)q * 512, slot);
+    if (lane < kSkinnyPieces<G, F>) dma16_lane(sc + (size_t)q * 512, slot + kScales);
     const unsigned wp = (unsigned)min(wpos, left - 1) * 16u;
 #pragma unroll
     for (int f = 0; f < F; ++f) {
-      const unsigned at = slot + 1024u * (1 + f);
+      const unsigned at = slot + 1024u * f;
       if constexpr (WT) {
         // 16 KB per (256-feature tile, whole step), the group's block in it; the blocks past the last whole step as
         // rows of nblk % 4 blocks behind the tiled part
@@ -227,7 +254,7 @@ mixed_gemm_skinny_kernel(DecodeSeg s4, DecodeSeg s6, DecodeSeg s8, int M, int N,
       if constexpr (FMT == kFmtE2M1) off = (unsigned)min(p ^ ((row >> 2) & 3), left - 1) * 16u;
       else if constexpr (FMT == kFmtE3M2) off = (unsigned)min(p * 16, left * 24 - 16);
       else off = (unsigned)min(p ^ (row & 7), 2 * left - 1) * 16u;
-      dma16_at(a, (unsigned)min(row, last_row) * pitch + off, slot + 1024u * (1 + F + c));
+      dma16_at(a, (unsigned)min(row, last_row) * pitch + off, slot + 1024u * (F + c));
     }
   };
   auto request = [&](int t, unsigned slot) __attribute__((always_inline)) {
@@ -252,75 +279,136 @@ mixed_gemm_skinny_kernel(DecodeSeg s4, DecodeSeg s6, DecodeSeg s8, int M, int N,
   int t = t_begin, slot = 0;
 #pragma unroll
   for (int k = 0; k < NS - 1; ++k) request(t_begin + k, ring0 + k * kSlot);
-  // the wave's steps of one segment
-  auto run = [&](auto fmt_c, const DecodeSeg& s, int t_first, int t_next) __attribute__((always_inline)) {
+  // the fragments of a step in a slot
+  struct Fragments { v4i w[F]; v8i x[G]; int s_w[F], s_x[G]; };
+  const int frag4 = i * 64 + (g ^ ((i >> 2) & 3)) * 16;   // of 64-byte rows
+  auto read = [&](auto fmt_c, Fragments& r, const uint8_t* sl, int left) __attribute__((always_inline)) {
     constexpr int FMT = decltype(fmt_c)::value;
-    for (const int last = min(t_next, t_end); t < last; ++t) {
-      // The slot after this one was read one step ago and is free.  Wait for this step: NS - 1 steps are younger, each
-      // with at least as many copies as this one (a token takes more bytes in every later segment's format).
-      const int ahead = t + NS - 1;
-      request(ahead, ring0 + (unsigned)(slot == 0 ? NS - 1 : slot - 1) * kSlot);
-      if (ahead < t_end) wait_vmcnt<(NS - 1) * (1 + F + kTokenCopies<FMT, G>)>();
-      else wait_vmcnt<0>();
-      const uint8_t* sl = ring + slot * kSlot;
-      slot = slot == NS - 1 ? 0 : slot + 1;
-      const int left = s.nblk - 4 * (t - t_first);
-      int s_w[F], s_x[G];
-      v4i w[F];
-      v8i x[G];
 #pragma unroll
-      for (int f = 0; f < F; ++f) {
-        s_w[f] = sl[sw_off[f]];
-        w[f] = *reinterpret_cast<const v4i*>(sl + 1024 * (1 + f) + i * 64 + (g ^ ((i >> 2) & 3)) * 16);
+    for (int f = 0; f < F; ++f) {
+      r.s_w[f] = sl[kScales + sw_off[f]];
+      r.w[f] = *reinterpret_cast<const v4i*>(sl + 1024 * f + frag4);
+    }
+#pragma unroll
+    for (int gi = 0; gi < G; ++gi) {
+      r.s_x[gi] = sl[kScales + sx_off[gi]];
+      const uint8_t* row = sl + 1024 * F + (16 * gi) * (4 * Frag<FMT>::kBytes);
+      if constexpr (FMT == kFmtE2M1) {
+        const v4i a = *reinterpret_cast<const v4i*>(row + frag4);
+        r.x[gi] = v8i{a[0], a[1], a[2], a[3], 0, 0, 0, 0};
+      } else if constexpr (FMT == kFmtE3M2) {
+        const v2i* p = reinterpret_cast<const v2i*>(row + i * 96 + g * 24);
+        // a partial step of 24 or 72 bytes: its last 16 bytes were copied, of which these are the second half
+        const v2i a = p[0], b = p[1], e = p[(left & 1) && g == left - 1 ? 3 : 2];
+        r.x[gi] = v8i{a[0], a[1], b[0], b[1], e[0], e[1], 0, 0};
+      } else {   // K [16g, 16g+16) and [64+16g, 64+16g+16)
+        const v4i a = *reinterpret_cast<const v4i*>(row + i * 128 + (g ^ (i & 7)) * 16);
+        const v4i b = *reinterpret_cast<const v4i*>(row + i * 128 + ((4 + g) ^ (i & 7)) * 16);
+        r.x[gi] = v8i{a[0], a[1], a[2], a[3], b[0], b[1], b[2], b[3]};
       }
-#pragma unroll
-      for (int gi = 0; gi < G; ++gi) {
-        s_x[gi] = sl[sx_off[gi]];
-        const uint8_t* row = sl + 1024 * (1 + F) + (16 * gi + i) * (4 * Frag<FMT>::kBytes);
-        if constexpr (FMT == kFmtE2M1) {
-          const v4i a = *reinterpret_cast<const v4i*>(row + (g ^ ((i >> 2) & 3)) * 16);
-          x[gi] = v8i{a[0], a[1], a[2], a[3], 0, 0, 0, 0};
-        } else if constexpr (FMT == kFmtE3M2) {
-          const v2i* p = reinterpret_cast<const v2i*>(row + g * 24);
-          // a partial step of 24 or 72 bytes: its last 16 bytes were copied, of which these are the second half
-          const v2i a = p[0], b = p[1], e = p[(left & 1) && g == left - 1 ? 3 : 2];
-          x[gi] = v8i{a[0], a[1], b[0], b[1], e[0], e[1], 0, 0};
-        } else {   // K [16g, 16g+16) and [64+16g, 64+16g+16)
-          const v4i a = *reinterpret_cast<const v4i*>(row + (g ^ (i & 7)) * 16);
-          const v4i b = *reinterpret_cast<const v4i*>(row + ((4 + g) ^ (i & 7)) * 16);
-          x[gi] = v8i{a[0], a[1], a[2], a[3], b[0], b[1], b[2], b[3]};
-        }
-      }
-      if (left < 4) {   // wave-uniform: the segment's last, partial step; what lies past its end is zero
-        const bool ok = g < left, lo_ok = FMT == kFmtE4M3 ? (g >> 1) < left : ok, hi_ok = FMT == kFmtE4M3 ? 2 + (g >> 1) < left : ok;
-#pragma unroll
-        for (int f = 0; f < F; ++f) {
-          s_w[f] = ok ? s_w[f] : 127;
-#pragma unroll
-          for (int e = 0; e < 4; ++e) w[f][e] = ok ? w[f][e] : 0;
-        }
-#pragma unroll
-        for (int gi = 0; gi < G; ++gi) {
-          s_x[gi] = ok ? s_x[gi] : 127;
-#pragma unroll
-          for (int e = 0; e < 4; ++e) {
-            x[gi][e] = lo_ok ? x[gi][e] : 0;
-            x[gi][4 + e] = hi_ok ? x[gi][4 + e] : 0;
-          }
-        }
-      }
-      // the fragments are in registers before a later request may fill this slot again
-      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-#pragma unroll
-      for (int gi = 0; gi < G; ++gi)
-#pragma unroll
-        for (int f = 0; f < F; ++f)
-          acc[f][gi] = decode_mfma<FMT>(v8i{w[f][0], w[f][1], w[f][2], w[f][3], 0, 0, 0, 0}, x[gi], acc[f][gi], s_w[f], s_x[gi]);
     }
   };
-  run(std::integral_constant<int, kFmtE2M1>{}, s4, 0, t6);
-  run(std::integral_constant<int, kFmtE3M2>{}, s6, t6, t8);
-  run(std::integral_constant<int, kFmtE4M3>{}, s8, t8, total);
+  auto multiply = [&](auto fmt_c, const Fragments& r) __attribute__((always_inline)) {
+    constexpr int FMT = decltype(fmt_c)::value;
+#pragma unroll
+    for (int gi = 0; gi < G; ++gi)
+#pragma unroll
+      for (int f = 0; f < F; ++f)
+        acc[f][gi] = decode_mfma<FMT>(v8i{r.w[f][0], r.w[f][1], r.w[f][2], r.w[f][3], 0, 0, 0, 0}, r.x[gi], acc[f][gi], r.s_w[f], r.s_x[gi]);
+  };
+  // the wave's steps of one segment, two at a time
+  auto run = [&](auto fmt_c, const DecodeSeg& s, const uint8_t* sc, int t_first, int t_next) __attribute__((always_inline)) {
+    constexpr int FMT = decltype(fmt_c)::value, TC = kTokenCopies<FMT, G>, PER = 1 + F + TC;
+    const int last = min(t_next, t_end);
+    if (t >= last) return;
+    const int whole = s.nblk >> 2, whole_end = min(last, t_first + whole);   // steps before whole_end are whole ones
+    // Requests of whole steps of this segment, which most are: addresses that advance, and offsets that stay.
+    const int q_next = t + NS - 1 - t_first;
+    const uint8_t* sc_next = sc + (ptrdiff_t)q_next * 512;
+    const uint8_t* w_next = WT ? s.b + (((ptrdiff_t)tile * whole + q_next) * 16 + j0) * 1024 : s.b + (ptrdiff_t)q_next * 64;
+    const unsigned pitch = (unsigned)s.nblk * Frag<FMT>::kBytes;
+    const uint8_t* a_next = s.a + (size_t)m_base * pitch + (ptrdiff_t)q_next * (4 * Frag<FMT>::kBytes);
+    unsigned w_off[F], a_off[TC];
+    if (t + NS - 1 < whole_end) {
+#pragma unroll
+      for (int f = 0; f < F; ++f) w_off[f] = WT ? (unsigned)(lane >> 2) * 64u + wpos * 16u : (unsigned)wrow[f] * (unsigned)s.nblk * 16u + wpos * 16u;
+#pragma unroll
+      for (int c = 0; c < TC; ++c) {
+        constexpr int kPieces = Frag<FMT>::kBytes / 4;
+        const int chunk = min(c * 64 + lane, 16 * G * kPieces - 1), row = chunk / kPieces, p = chunk % kPieces;
+        a_off[c] = (unsigned)min(row, last_row) * pitch + (FMT == kFmtE2M1 ? p ^ ((row >> 2) & 3) : FMT == kFmtE3M2 ? p : p ^ (row & 7)) * 16u;
+      }
+    }
+    auto next = [&](int ahead, unsigned to) __attribute__((always_inline)) {
+      if (ahead < whole_end) {
+        if (lane < kSkinnyPieces<G, F>) dma16_lane(sc_next, to + kScales);
+#pragma unroll
+        for (int f = 0; f < F; ++f) dma16_at<kStream>(WT ? w_next + f * 1024 : w_next, w_off[f], to + 1024u * f);
+#pragma unroll
+        for (int c = 0; c < TC; ++c) dma16_at(a_next, a_off[c], to + 1024u * (F + c));
+        sc_next += 512;
+        w_next += WT ? 16384 : 64;
+        a_next += 4 * Frag<FMT>::kBytes;
+      } else {
+        request(ahead, to);
+      }
+    };
+    // Steps up to t + NS - 2 have been requested.  What is waited for has at least `younger` steps behind it, each with at
+    // least as many copies as this segment's (a token takes more bytes in every later segment's format).
+    while (t < last) {
+      const uint8_t* sl = ring + slot * kSlot;
+      const unsigned freed = ring0 + (unsigned)(slot == 0 ? NS - 1 : slot - 1) * kSlot;   // read a step ago
+      if (t + 1 < whole_end) {
+        const int after = slot == NS - 1 ? 0 : slot + 1;
+        const unsigned this_slot = ring0 + (unsigned)slot * kSlot;
+        next(t + NS - 1, freed);
+        if (t + NS - 1 < t_end) wait_vmcnt<(NS - 2) * PER>();
+        else wait_steps<PER, NS - 3>(t_end - 2 - t);
+        Fragments r0, r1;
+        read(fmt_c, r0, sl, 4);
+        read(fmt_c, r1, ring + after * kSlot, 4);
+        // the fragments are in registers before a later request may fill these slots again
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+        next(t + NS, this_slot);
+        multiply(fmt_c, r0);
+        multiply(fmt_c, r1);
+        slot = after == NS - 1 ? 0 : after + 1;
+        t += 2;
+      } else {
+        next(t + NS - 1, freed);
+        if (t + NS - 1 < t_end) wait_vmcnt<(NS - 1) * PER>();
+        else wait_steps<PER, NS - 2>(t_end - 1 - t);
+        slot = slot == NS - 1 ? 0 : slot + 1;
+        const int left = s.nblk - 4 * (t - t_first);
+        Fragments r;
+        read(fmt_c, r, sl, left);
+        if (left < 4) {   // wave-uniform: the segment's last, partial step; what lies past its end is zero
+          const bool ok = g < left, lo_ok = FMT == kFmtE4M3 ? (g >> 1) < left : ok, hi_ok = FMT == kFmtE4M3 ? 2 + (g >> 1) < left : ok;
+#pragma unroll
+          for (int f = 0; f < F; ++f) {
+            r.s_w[f] = ok ? r.s_w[f] : 127;
+#pragma unroll
+            for (int e = 0; e < 4; ++e) r.w[f][e] = ok ? r.w[f][e] : 0;
+          }
+#pragma unroll
+          for (int gi = 0; gi < G; ++gi) {
+            r.s_x[gi] = ok ? r.s_x[gi] : 127;
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+              r.x[gi][e] = lo_ok ? r.x[gi][e] : 0;
+              r.x[gi][4 + e] = hi_ok ? r.x[gi][4 + e] : 0;
+            }
+          }
+        }
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+        multiply(fmt_c, r);
+        ++t;
+      }
+    }
+  };
+  run(std::integral_constant<int, kFmtE2M1>{}, s4, sc4, 0, t6);
+  run(std::integral_constant<int, kFmtE3M2>{}, s6, sc6, t6, t8);
+  run(std::integral_constant<int, kFmtE4M3>{}, s8, sc8, t8, total);
 
   // ---- sum the four waves' partial tiles (D^T: lane holds token lane % 16, features 4 * (lane / 16) + v of a group)
   __syncthreads();   // every wave is done with its ring, which nothing fills any more
@@ -726,18 +814,6 @@ struct TokenLds {   // byte offsets behind the rings
 template <int F>
 constexpr int kTokenSlots = F == 1 ? 12 : (F == 2 ? 8 : 5);
 
-// waits until at most `steps` (wave-uniform) steps of PER copies each are in flight
-template <int PER>
-__device__ __forceinline__ void wait_steps(int steps) {
-  switch (steps) {
-#define MG_STEPS_CASE(N) case N: wait_vmcnt<N * PER>(); break;
-    MG_STEPS_CASE(1) MG_STEPS_CASE(2) MG_STEPS_CASE(3) MG_STEPS_CASE(4) MG_STEPS_CASE(5) MG_STEPS_CASE(6)
-    MG_STEPS_CASE(7) MG_STEPS_CASE(8) MG_STEPS_CASE(9) MG_STEPS_CASE(10) MG_STEPS_CASE(11)
-#undef MG_STEPS_CASE
-    default: wait_vmcnt<0>(); break;
-  }
-}
-
 // Codes and scale byte of half a block to LDS.
 struct LdsHalf {
   uint8_t* q;    // of the block
@@ -832,7 +908,7 @@ mixed_gemm_token_kernel(const uint8_t* __restrict__ x, const uint8_t* __restrict
   };
 #pragma unroll
   for (int k = 0; k < NS - 1; ++k) request(t_begin + k, ring0 + k * kSlot);
-  wait_steps<F>(min(NS - 1, t_end - t_begin));   // everything older has landed
+  wait_steps<F, NS - 1>(min(NS - 1, t_end - t_begin));   // everything older has landed
   lds_barrier();
 
   // ---- RMSNorm of the tokens, in place (see the quantizer); the waves are dealt to the tokens
@@ -908,7 +984,7 @@ mixed_gemm_token_kernel(const uint8_t* __restrict__ x, const uint8_t* __restrict
     const uint8_t* row = lds + codes + mc * (s.nblk * Frag<FMT>::kBytes);
     for (const int last = min(t_next, t_end); t < last; ++t) {
       request(t + NS - 1, ring0 + (unsigned)(slot == 0 ? NS - 1 : slot - 1) * kSlot);
-      wait_steps<F>(min(NS - 1, t_end - 1 - t));
+      wait_steps<F, NS - 1>(min(NS - 1, t_end - 1 - t));
       const uint8_t* sl = ring + slot * kSlot;
       slot = slot == NS - 1 ? 0 : slot + 1;
       const int q = t - t_first, left = s.nblk - 4 * q;
@@ -1018,14 +1094,17 @@ static bool decode_lds_plan(const DecodeSeg& d4, const DecodeSeg& d6, const Deco
 // tile-major figures row-major weights were at 3.0 / 5.2 and 68 / 77 %.
 struct SkinnyPlan { int g, f; double us; };
 static SkinnyPlan skinny_plan(int M, int N, int steps, int cus, bool w_tiled) {
-  static const struct { int g, f; double ns[2]; } kForms[] = {   // row-major, tile-major weights
-      {1, 1, {46, 67}}, {1, 2, {62, 77}}, {1, 4, {104, 102}}, {2, 2, {89, 86}}, {2, 4, {145, 117}}, {4, 2, {134, 110}}, {1, 8, {230, 225}}};
+  // row-major, tile-major weights; `even`: with an even number of token groups, where the form of half the features and twice the tokens
+  // has as many workgroups
+  static const struct { int g, f; double ns[2], even[2]; } kForms[] = {
+      {1, 1, {46, 67}, {46, 67}}, {1, 2, {62, 77}, {62, 77}}, {1, 4, {104, 102}, {104, 85}}, {2, 2, {89, 86}, {89, 86}},
+      {2, 4, {145, 117}, {145, 106}}, {4, 2, {134, 110}, {134, 110}}, {1, 8, {230, 225}, {230, 225}}};
   SkinnyPlan best = {0, 0, 0.0};
   for (const auto& k : kForms) {
     if (k.f == 8 && M > 16) continue;
     const int across = w_tiled ? ceil_div(N, 16 * k.f) : ceil_div(N, 128) * (8 / k.f);
-    const int rounds = (int)(((int64_t)across * ceil_div(M, 16 * k.g) + cus - 1) / cus);
-    const double us = 1.0 + rounds * (2.3 + steps * k.ns[w_tiled] * 1e-3) + 1.5 * (rounds - 1);
+    const int groups = ceil_div(M, 16 * k.g), rounds = (int)(((int64_t)across * groups + cus - 1) / cus);
+    const double us = 1.0 + rounds * (2.3 + steps * (groups % 2 == 0 ? k.even : k.ns)[w_tiled] * 1e-3) + 1.5 * (rounds - 1);
     if (best.g == 0 || us < best.us) best = {k.g, k.f, us};
   }
   return best;
@@ -1081,13 +1160,13 @@ hipError_t launch_decode(const DecodeSeg& d4, const DecodeSeg& d6, const DecodeS
 hipError_t launch_skinny(const DecodeSeg& d4, const DecodeSeg& d6, const DecodeSeg& d8, int M, int N, bool w_tiled,
                          const SkinnyPlan& plan, Epilogue ep, uint16_t* d, hipStream_t stream) {
   const int total = d4.steps + d6.steps + d8.steps;
-  const dim3 grid(w_tiled ? ceil_div(N, 16 * plan.f) : ceil_div(N, 128) * (8 / plan.f), ceil_div(M, 16 * plan.g));
+  const TileOrder order = tile_runs(w_tiled ? ceil_div(N, 16 * plan.f) : ceil_div(N, 128) * (8 / plan.f), ceil_div(M, 16 * plan.g));
   auto launch = [&](auto g_c, auto f_c) {
     constexpr int G = decltype(g_c)::value, F = decltype(f_c)::value;
     constexpr int kLds = 4 * kSkinnySlots<G, F> * kSkinnySlot<G, F>;
     const auto kernel = w_tiled ? mixed_gemm_skinny_kernel<G, F, true> : mixed_gemm_skinny_kernel<G, F, false>;
     if (hipError_t e = allow_dynamic_lds(reinterpret_cast<const void*>(kernel), kLds); e != hipSuccess) return e;
-    hipLaunchKernelGGL(kernel, grid, dim3(256), kLds, stream, d4, d6, d8, M, N, (total + 3) / 4, ep, d);
+    hipLaunchKernelGGL(kernel, dim3(order.grid_x, grid_rows(order)), dim3(256), kLds, stream, d4, d6, d8, M, N, (total + 3) / 4, order, ep, d);
     return hipGetLastError();
   };
   const std::integral_constant<int, 1> one;

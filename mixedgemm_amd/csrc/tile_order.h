@@ -21,10 +21,17 @@ struct TileOrder {
 // HIP takes fewer than 2^32 threads along a dimension of a grid; a launch of more tiles than this has several rows of workgroups.
 constexpr int kMostTilesAcross = 1 << 22;   // of at most 1023 threads each
 
+// Runs of consecutive tiles, token tile after token tile, whatever the counts.
+inline TileOrder tile_runs(int tiles_n, int tiles_m) {
+  const int nwg = tiles_n * tiles_m;
+  return {-1, tiles_m, nwg >> 3, tiles_m > 1 ? (unsigned)(((1ull << 32) + tiles_m - 1) / tiles_m) : 0,
+          nwg < kMostTilesAcross ? nwg : kMostTilesAcross, nwg};
+}
+
 // tf x tt: features and tokens of a tile
 inline TileOrder tile_order(int tiles_n, int tiles_m, int tf, int tt) {
-  const int nwg = tiles_n * tiles_m;
-  TileOrder o = {-1, tiles_m, nwg >> 3, 0, nwg < kMostTilesAcross ? nwg : kMostTilesAcross, nwg};
+  TileOrder o = tile_runs(tiles_n, tiles_m);
+  const int nwg = o.tiles;
   if ((nwg & 7) == 0) {
     double best = 0.0;
     for (int x = 3; x >= 0; --x) {

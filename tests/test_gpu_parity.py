@@ -600,6 +600,23 @@ def test_skinny_kernel_at_the_edges_of_its_pipeline(abi, m, n, kn, ks, ko):
         test_small_batches_match_oracle(abi, m, n, kn, ks, ko, True)
 
 
+# Steps two at a time out of rings of three or four slots: 1 ... 10 steps per wave (odd and even, fewer than a ring, one more, twice as
+# many), the segments' borders at either step of a pair, with and without partial last steps; one, two and an odd number of
+# token groups, in runs of workgroups that do and do not divide by the eight XCDs.
+@pytest.mark.parametrize("per_wave", range(1, 11))
+@pytest.mark.parametrize("m,n", [(5, 1280), (24, 1536), (70, 768)])
+@pytest.mark.parametrize("rest", [(0, 0, 0), (32, 64, 96), (96, 0, 32)])
+def test_skinny_kernel_takes_steps_in_pairs(abi, per_wave, m, n, rest):
+    steps = 4 * per_wave
+    s4 = steps // 2 + (per_wave & 1)
+    s6 = max(1, steps - s4 - 1 - (per_wave % 3 == 0))
+    s8 = max(1, steps - s4 - s6)
+    kn, ks, ko = (128 * s - ((128 - r) if r else 0) for s, r in zip((s4, s6, s8), rest))
+    test_small_batches_match_oracle(abi, m, n, kn, ks, ko, False)
+    if abi.weights_tileable(n, kn, ks, ko):
+        test_small_batches_match_oracle(abi, m, n, kn, ks, ko, True)
+
+
 # Up to 16 tokens on more than 64 features per CU.  Up to 128: the skinny kernel with eight feature groups (a ragged last group of
 # 128 rows, whole tiles, 1 to 3 blocks past whole steps, fewer steps than waves, an empty segment).  More: the decode kernel with
 # four and two feature groups, from the first width on, and the skinny kernel where a segment is not whole steps.  On both layouts
