@@ -799,6 +799,8 @@ mixed_gemm_decode_kernel(DecodeSeg s4, DecodeSeg s6, DecodeSeg s8, int M, int N,
 // 12 %).  N = 4096, K = 4096, tile-major, in a graph, two launches -> one: M = 1 7.5 -> 6.0 us, 2 7.9 -> 6.4, 4 7.7 -> 7.5
 // (8: 7.8 -> 10.0, not taken); N = 14336, M = 1 10.3 -> 8.0, 4 10.2 -> 9.3; with RMSNorm, N = 4096: M = 1 8.2 -> 7.1, 2
 // 8.4 -> 8.0 (4: 8.4 -> 9.7, not taken).  A layer call of one token from Python: 9.1 -> 7.0 us.
+// With shorter rings and whole steps two at a time (from HBM, one launch before and after): N = K = 4096, M = 1 6.2 -> 5.9, 2 6.6 -> 6.35, with
+// RMSNorm 7.15 -> 6.9; N = K = 8192, M = 1 10.7 -> 9.9; N = 4096, K = 8192 9.1 -> 8.4; 200 drawn calls 1.035 times as fast in the mean.
 // ---------------------------------------------------------------------------
 constexpr int kTokenRows = 8;    // most tokens (a wave each in the RMSNorm)
 constexpr int kTokenWaves = 8;   // all quantize; four of them also run the K loop
@@ -810,9 +812,10 @@ struct TokenLds {   // byte offsets behind the rings
   int sums;              // RMSNorm: the waves' sums of squares
   int total;
 };
-// slots per wave: 48 ... 80 KB of weight codes in flight per CU
+// Slots per wave: 20 ... 64 KB of weight codes in flight per CU (see kSkinnySlots; with 12 / 8 / 5 of them, us: N = K = 4096 6.2, now 5.9; N = K =
+// 8192 10.7, now 9.9; N = 14336, K = 4096 8.6, now 8.5; 2 to 5 steps per wave on row-major weights 4.5 ... 4.8, now 4.65 ... 4.9)
 template <int F>
-constexpr int kTokenSlots = F == 1 ? 12 : (F == 2 ? 8 : 5);
+constexpr int kTokenSlots = F == 1 ? 5 : (F == 2 ? 5 : 4);
 
 // Codes and scale byte of half a block to LDS.
 struct LdsHalf {
@@ -979,55 +982,85 @@ mixed_gemm_token_kernel(const uint8_t* __restrict__ x, const uint8_t* __restrict
   for (int f = 0; f < F; ++f) acc[f] = v4f{0.f, 0.f, 0.f, 0.f};
   const int mc = min(i, M - 1);   // tokens past M: the last one again, never stored
   int t = t_begin, slot = 0;
+  struct Fragments { v4i w[F]; v8i x; int s_w[F], s_x; };
+  // the wave's steps of one segment, whole ones two at a time as in the skinny kernel
   auto run = [&](auto fmt_c, const DecodeSeg& s, int codes, int sfx, int sfw, int t_first, int t_next) __attribute__((always_inline)) {
     constexpr int FMT = decltype(fmt_c)::value;
-    const uint8_t* row = lds + codes + mc * (s.nblk * Frag<FMT>::kBytes);
-    for (const int last = min(t_next, t_end); t < last; ++t) {
-      request(t + NS - 1, ring0 + (unsigned)(slot == 0 ? NS - 1 : slot - 1) * kSlot);
-      wait_steps<F, NS - 1>(min(NS - 1, t_end - 1 - t));
-      const uint8_t* sl = ring + slot * kSlot;
-      slot = slot == NS - 1 ? 0 : slot + 1;
-      const int q = t - t_first, left = s.nblk - 4 * q;
-      v4i w[F];
-      int s_w[F], s_x = lds[sfx + q * (4 * kTokenRows) + mc * 4 + g];
+    const int last = min(t_next, t_end);
+    if (t >= last) return;
+    const int whole_end = min(last, t_first + (s.nblk >> 2));
+    const uint8_t* row = lds + codes + mc * (s.nblk * Frag<FMT>::kBytes) + g * (FMT == kFmtE3M2 ? 24 : 16);
+    const uint8_t* sx = lds + sfx + mc * 4 + g;
+    const uint8_t* sw = lds + sfw;
+    auto read = [&](Fragments& r, const uint8_t* sl, int q) __attribute__((always_inline)) {
+      r.s_x = sx[q * (4 * kTokenRows)];
 #pragma unroll
       for (int f = 0; f < F; ++f) {
-        s_w[f] = lds[sfw + q * (PB * 16) + sw_off[f]];
-        w[f] = *reinterpret_cast<const v4i*>(sl + 1024 * f + i * 64 + (g ^ ((i >> 2) & 3)) * 16);
+        r.s_w[f] = sw[q * (PB * 16) + sw_off[f]];
+        r.w[f] = *reinterpret_cast<const v4i*>(sl + 1024 * f + i * 64 + (g ^ ((i >> 2) & 3)) * 16);
       }
-      v8i x8;
       if constexpr (FMT == kFmtE2M1) {
-        const v4i a = *reinterpret_cast<const v4i*>(row + q * 64 + g * 16);
-        x8 = v8i{a[0], a[1], a[2], a[3], 0, 0, 0, 0};
+        const v4i a = *reinterpret_cast<const v4i*>(row + q * 64);
+        r.x = v8i{a[0], a[1], a[2], a[3], 0, 0, 0, 0};
       } else if constexpr (FMT == kFmtE3M2) {
-        const v2i* p = reinterpret_cast<const v2i*>(row + q * 96 + g * 24);
+        const v2i* p = reinterpret_cast<const v2i*>(row + q * 96);
         const v2i a = p[0], b = p[1], e = p[2];
-        x8 = v8i{a[0], a[1], b[0], b[1], e[0], e[1], 0, 0};
+        r.x = v8i{a[0], a[1], b[0], b[1], e[0], e[1], 0, 0};
       } else {
-        const v4i a = *reinterpret_cast<const v4i*>(row + q * 128 + g * 16);
-        const v4i b = *reinterpret_cast<const v4i*>(row + q * 128 + 64 + g * 16);
-        x8 = v8i{a[0], a[1], a[2], a[3], b[0], b[1], b[2], b[3]};
+        const v4i a = *reinterpret_cast<const v4i*>(row + q * 128);
+        const v4i b = *reinterpret_cast<const v4i*>(row + q * 128 + 64);
+        r.x = v8i{a[0], a[1], a[2], a[3], b[0], b[1], b[2], b[3]};
       }
+    };
+    auto multiply = [&](const Fragments& r) __attribute__((always_inline)) {
+#pragma unroll
+      for (int f = 0; f < F; ++f)
+        acc[f] = decode_mfma<FMT>(v8i{r.w[f][0], r.w[f][1], r.w[f][2], r.w[f][3], 0, 0, 0, 0}, r.x, acc[f], r.s_w[f], r.s_x);
+    };
+    while (t < last) {
+      const uint8_t* sl = ring + slot * kSlot;
+      const unsigned this_slot = ring0 + (unsigned)slot * kSlot;
+      request(t + NS - 1, ring0 + (unsigned)(slot == 0 ? NS - 1 : slot - 1) * kSlot);
+      slot = slot == NS - 1 ? 0 : slot + 1;
+      const int q = t - t_first;
+      if (F < 4 && t + 1 < whole_end) {   // (four feature groups: 8.45 us one at a time, 8.6 in pairs)
+        if (t + NS - 1 < t_end) wait_vmcnt<(NS - 2) * F>();
+        else wait_steps<F, NS - 3>(t_end - 2 - t);
+        Fragments r0, r1;
+        read(r0, sl, q);
+        read(r1, ring + slot * kSlot, q + 1);
+        // the weights are in registers before a later request may fill these slots again
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+        request(t + NS, this_slot);
+        multiply(r0);
+        multiply(r1);
+        slot = slot == NS - 1 ? 0 : slot + 1;
+        t += 2;
+        continue;
+      }
+      if (t + NS - 1 < t_end) wait_vmcnt<(NS - 1) * F>();
+      else wait_steps<F, NS - 2>(t_end - 1 - t);
+      const int left = s.nblk - 4 * q;
+      Fragments r;
+      read(r, sl, q);
       if (left < 4) {   // wave-uniform: the segment's last, partial step; what lies past its end is zero
         const bool ok = g < left, lo_ok = FMT == kFmtE4M3 ? (g >> 1) < left : ok, hi_ok = FMT == kFmtE4M3 ? 2 + (g >> 1) < left : ok;
-        s_x = ok ? s_x : 127;
+        r.s_x = ok ? r.s_x : 127;
 #pragma unroll
         for (int f = 0; f < F; ++f) {
-          s_w[f] = ok ? s_w[f] : 127;
+          r.s_w[f] = ok ? r.s_w[f] : 127;
 #pragma unroll
-          for (int e = 0; e < 4; ++e) w[f][e] = ok ? w[f][e] : 0;
+          for (int e = 0; e < 4; ++e) r.w[f][e] = ok ? r.w[f][e] : 0;
         }
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
-          x8[e] = lo_ok ? x8[e] : 0;
-          x8[4 + e] = hi_ok ? x8[4 + e] : 0;
+          r.x[e] = lo_ok ? r.x[e] : 0;
+          r.x[4 + e] = hi_ok ? r.x[4 + e] : 0;
         }
       }
-      // the weights are in registers before a later request may fill this slot again
       asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-#pragma unroll
-      for (int f = 0; f < F; ++f)
-        acc[f] = decode_mfma<FMT>(v8i{w[f][0], w[f][1], w[f][2], w[f][3], 0, 0, 0, 0}, x8, acc[f], s_w[f], s_x);
+      multiply(r);
+      ++t;
     }
   };
   run(std::integral_constant<int, kFmtE2M1>{}, s4, L.q0, L.sx0, L.sw0, 0, t6);
@@ -1328,11 +1361,10 @@ hipError_t launch_mixed_gemm(const uint8_t* an, const uint8_t* bn, const uint8_t
 }
 
 // Quantization and GEMM of a few tokens in one launch, where that is the faster way; *taken says whether it was.
-// Every workgroup repeats the quantization, so it pays up to 16384 channels in all (M = 4, K = 4096 7.7 -> 7.5 us, M = 8
-// 7.8 -> 10.0; M = 2, K = 8192 13.0 -> 11.0), with RMSNorm up to 10240 (M = 2, K = 4096 8.4 -> 8.0, K = 5120 10.7 -> 10.3;
-// M = 4, K = 4096 8.4 -> 9.7), from 5 tokens on, where a token's norm is one wave's work, 8192 (launch time, one against two,
-// N = 4096: M = 8, K = 1024 0.97, 1152 1.09, 2048 1.18; M = 5, K = 1536 1.00, 1792 1.07; M = 4, K = 2560 1.03), for rows of at
-// most 8192 (M = 1, K = 14336: 13.7 -> 14.0), and in one round of workgroups.
+// Every workgroup repeats the quantization, so it pays up to 20480 channels in all (us, two launches against one, N = 4096 / 14336, K = 4096: M =
+// 5 8.2 against 7.8 / 11.4 against 10.3, M = 6 8.3 against 8.6), with RMSNorm up to 10240 (M = 3 9.0 against 9.0 / 12.2 against 11.4, but 10.5 against
+// 11.1 with the weights in the caches, N = 13312), from 5 tokens on, where a token's norm is one wave's work, 8192 (M = 8, K = 1024 level, K =
+// 2048 7.6 against 8.8), for rows of at most 8192 (M = 1, K = 14336, with longer rings: 13.7 against 14.0), and in one round of workgroups.
 hipError_t launch_token_linear(const void* x, const int16_t* idx, const void* gamma, float eps, const uint8_t* bn, const uint8_t* bs,
                                const uint8_t* bo, const uint8_t* sfbn, const uint8_t* sfbs, const uint8_t* sfbo, int M, int N,
                                int KN, int KS, int KO, bool w_tiled, Epilogue ep, void* d, hipStream_t stream, bool* taken) {
@@ -1340,7 +1372,7 @@ hipError_t launch_token_linear(const void* x, const int16_t* idx, const void* ga
   const int K = KN + KS + KO;
   // (row-major weight codes are addressed with 32-bit offsets; the copies of gamma want it aligned)
   const int widest = KN > KS ? (KN > KO ? KN : KO) : (KS > KO ? KS : KO);
-  if (M < 1 || M > kTokenRows || K == 0 || K > 8192 || M * K > (gamma ? (M > 4 ? 8192 : 10240) : 16384) || N == 0 || (!w_tiled && (size_t)N * (size_t)(widest / 2) >= ((size_t)1 << 32)) ||
+  if (M < 1 || M > kTokenRows || K == 0 || K > 8192 || M * K > (gamma ? (M > 4 ? 8192 : 10240) : 20480) || N == 0 || (!w_tiled && (size_t)N * (size_t)(widest / 2) >= ((size_t)1 << 32)) ||
       (reinterpret_cast<uintptr_t>(gamma) & 15u))
     return hipSuccess;
   // tile-major weights exist only for shapes the 256x256 kernel takes

@@ -269,6 +269,15 @@ def test_few_tokens_in_one_launch(linear, n, split, norm, tiled):
         assert torch.equal(got, want), m
 
 
+# Rings of five slots and steps two at a time with one and two feature groups, four slots with four: 2 ... 16 steps per wave, odd and even, the
+# segments' borders at either step of a pair, with and without partial last steps.
+@pytest.mark.parametrize("n,split", [(264, (640, 256, 128)), (264, (1216, 480, 96)), (264, (1920, 896, 256)), (264, (4096, 3072, 1024)),
+                                     (6144, (640, 256, 128)), (6144, (1216, 480, 96)), (6144, (2688, 1024, 384)), (14336, (1216, 480, 96))])
+@pytest.mark.parametrize("tiled", [False, True])
+def test_few_tokens_take_steps_in_pairs(linear, n, split, tiled):
+    test_few_tokens_in_one_launch(linear, n, split, False, tiled)
+
+
 # The same with rows that no random draw gives: zeros of both signs, the smallest subnormals, the largest finite values, one
 # infinity, one NaN.  A block that holds an infinity or a NaN has no specified codes, but both ways run the same arithmetic.
 @pytest.mark.parametrize("n,split", [(256, (128, 128, 128)), (1000, (416, 224, 96)), (4096, (1280, 640, 128))])
