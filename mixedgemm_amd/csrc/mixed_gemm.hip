@@ -358,12 +358,12 @@ mixed_gemm_skinny_kernel(DecodeSeg s4, DecodeSeg s6, DecodeSeg s8, int M, int N,
     while (t < last) {
       const uint8_t* sl = ring + slot * kSlot;
       const unsigned freed = ring0 + (unsigned)(slot == 0 ? NS - 1 : slot - 1) * kSlot;   // read a step ago
-      if (t + 1 < whole_end) {
+      if (NS > 3 && t + 1 < whole_end) {   // (out of three slots, with one step in flight: N = 20480, K = 5120, M = 16 18.0 us, in pairs 18.5)
         const int after = slot == NS - 1 ? 0 : slot + 1;
         const unsigned this_slot = ring0 + (unsigned)slot * kSlot;
         next(t + NS - 1, freed);
         if (t + NS - 1 < t_end) wait_vmcnt<(NS - 2) * PER>();
-        else wait_steps<PER, NS - 3>(t_end - 2 - t);
+        else wait_steps<PER, (NS > 3 ? NS - 3 : 0)>(t_end - 2 - t);
         Fragments r0, r1;
         read(fmt_c, r0, sl, 4);
         read(fmt_c, r1, ring + after * kSlot, 4);
@@ -446,7 +446,7 @@ mixed_gemm_skinny_kernel(DecodeSeg s4, DecodeSeg s6, DecodeSeg s8, int M, int N,
 // workgroup in 1 KB copies (global_load_lds_dwordx4): the token codes of all three segments (M x 2464 bytes for
 // K = 4096) and, per K step, the 16-byte pieces of the scale
 // atoms that hold the workgroup's rows; the K loop reads them from LDS.  The weight codes go to registers,
-// eight K steps per wave in flight at a time, in two rounds of four.  All
+// eight K steps per wave at a time, in two rounds of four.  All
 // requests are inline assembly, so that the waits can count them (requests complete in order).
 //
 // Which features a workgroup owns follows the scale atoms: a 16-byte piece of an atom holds rows c, c + 32,
@@ -539,6 +539,15 @@ __device__ __forceinline__ void load16_uncounted(v4i& dst, const uint8_t* sbase,
 }
 __device__ __forceinline__ void tie(v4i& r) { asm volatile("" : "+v"(r)); }
 
+// f of the integral constants N ... END - 1
+template <int N, int END, class Fn>
+__device__ __forceinline__ void for_each_step(Fn f) {
+  if constexpr (N < END) {
+    f(std::integral_constant<int, N>{});
+    for_each_step<N + 1, END>(f);
+  }
+}
+
 template <int F, bool WT>
 __global__ void __launch_bounds__(256)
 mixed_gemm_decode_kernel(DecodeSeg s4, DecodeSeg s6, DecodeSeg s8, int M, int N, int steps_per_wave, DecodeLds L,
@@ -618,10 +627,9 @@ mixed_gemm_decode_kernel(DecodeSeg s4, DecodeSeg s6, DecodeSeg s8, int M, int N,
     vrow8[f] = (unsigned)nc[f] * (unsigned)nblk8 * 16u + (unsigned)g * 16u;
   }
   const int wtile = (wg * F) >> 4, wj0 = (wg * F) & 15;
-  auto request_round = [&](int r, auto buf_c) {
-    constexpr int B = decltype(buf_c)::value;
-#pragma unroll
-    for (int k = 0; k < S; ++k) {
+  auto request_step = [&](int r, auto buf_c, auto k_c) __attribute__((always_inline)) {
+    constexpr int B = decltype(buf_c)::value, k = decltype(k_c)::value;
+    {
       const int t = min(t_begin + r * S + k, total - 1);
       const int seg = t < s4.steps ? 0 : (t < s4.steps + s6.steps ? 1 : 2);
       const int q = seg == 0 ? t : (seg == 1 ? t - s4.steps : t - s4.steps - s6.steps);
@@ -643,6 +651,12 @@ mixed_gemm_decode_kernel(DecodeSeg s4, DecodeSeg s6, DecodeSeg s8, int M, int N,
       }
     }
   };
+  auto request_round = [&](int r, auto buf_c) __attribute__((always_inline)) {
+    request_step(r, buf_c, std::integral_constant<int, 0>{});
+    request_step(r, buf_c, std::integral_constant<int, 1>{});
+    request_step(r, buf_c, std::integral_constant<int, 2>{});
+    request_step(r, buf_c, std::integral_constant<int, 3>{});
+  };
   // ---- what is not a weight code, into LDS: requested first (measured: with the first round of weights ahead of
   // them the kernel is slower, by 2 % on tile-major and 7 % on row-major weights)
   copy_region(s4.a, M * nblk4 * 16, lds0 + L.x0, wave, lane);
@@ -660,11 +674,21 @@ mixed_gemm_decode_kernel(DecodeSeg s4, DecodeSeg s6, DecodeSeg s8, int M, int N,
     if (s8.steps) copy_pieces(s8.sfb, s8.steps, PBLOG, sfb_piece_off + (unsigned)(sfb_katoms_mul * s8.steps) * 512u, lds0 + L.sfb2, wave, lane);
   }
 
-  if (rounds > 0) request_round(0, std::integral_constant<int, 0>{});
-  if (rounds > 1) request_round(1, std::integral_constant<int, 1>{});
+  // The first two rounds: kAhead steps are requested up front, another one as each is used (a wave that requests more stands at its
+  // requests while its first steps' codes are there).  Layer call from HBM, us, with both rounds requested and each waited for as a whole /
+  // a window of 2 / 3 / 4 / 5 / 6 / 8 steps: N = 14336, K = 4096 (F = 4), M = 8 11.6 / 11.0 / 10.8 / 10.8 / 10.7 / 10.9 / 11.6, from the caches 10.0 / 10.0 /
+  // 9.3 / 9.3 / 9.5 / 9.6 / 10.0; row-major, N = 18944, K = 3584 (F = 2), M = 16 17.0 / - / 16.85 / 16.3 / 16.4 / 16.3 / 16.7; N = K = 4096 (F = 1) 8.3, now 7.75.
+  constexpr int kAhead = F == 4 ? 4 : (F == 2 ? 5 : 8);
+  auto request_nth = [&](auto n_c) __attribute__((always_inline)) {
+    constexpr int n = decltype(n_c)::value;
+    request_step(n / S, std::integral_constant<int, n / S>{}, std::integral_constant<int, n % S>{});
+  };
+  if (rounds > 1) for_each_step<0, kAhead>(request_nth);
+  else if (rounds > 0) request_round(0, std::integral_constant<int, 0>{});
 
-  // ---- the copies and the first round are older than the second round: done when only that is in flight
-  if (rounds > 1) wait_vmcnt<S * F>();
+  // ---- the copies are older than all of them
+  if (rounds > 1) wait_vmcnt<kAhead * F>();
+  else if (rounds > 0) wait_vmcnt<S * F>();
   else wait_vmcnt<0>();
   asm volatile("s_barrier" ::: "memory");
 
@@ -675,10 +699,9 @@ mixed_gemm_decode_kernel(DecodeSeg s4, DecodeSeg s6, DecodeSeg s8, int M, int N,
   const int mc = min(i, M - 1), sx_off = mc * 16;
   const int pa16 = L.pa * 16;
 
-  auto compute_round = [&](int r, auto buf_c) {
-    constexpr int B = decltype(buf_c)::value;
-#pragma unroll
-    for (int k = 0; k < S; ++k) {
+  auto compute_step = [&](int r, auto buf_c, auto k_c) __attribute__((always_inline)) {
+    constexpr int B = decltype(buf_c)::value, k = decltype(k_c)::value;
+    {
       const int t = t_begin + r * S + k;
       if (t < t_end) {   // wave-uniform
         const int seg = t < s4.steps ? 0 : (t < s4.steps + s6.steps ? 1 : 2);
@@ -715,6 +738,12 @@ mixed_gemm_decode_kernel(DecodeSeg s4, DecodeSeg s6, DecodeSeg s8, int M, int N,
       }
     }
   };
+  auto compute_round = [&](int r, auto buf_c) __attribute__((always_inline)) {
+    compute_step(r, buf_c, std::integral_constant<int, 0>{});
+    compute_step(r, buf_c, std::integral_constant<int, 1>{});
+    compute_step(r, buf_c, std::integral_constant<int, 2>{});
+    compute_step(r, buf_c, std::integral_constant<int, 3>{});
+  };
   // the registers of a round are tied to the wait that precedes their use
   auto settle = [&](auto buf_c, auto n_c) {
     constexpr int B = decltype(buf_c)::value;
@@ -728,17 +757,17 @@ mixed_gemm_decode_kernel(DecodeSeg s4, DecodeSeg s6, DecodeSeg s8, int M, int N,
   // Two rounds at a time, both requested before the first is used.  The first pair (requested above) is straight-line
   // code, the loop requests its pairs itself: nothing is in flight across a loop edge (a register that an uncounted
   // load is still to fill must not be moved by the compiler, which a value carried around a loop may be).
-  if (rounds > 0) {
+  // step n of TOTAL, with AHEAD requested before it
+  auto nth_step = [&](auto n_c, auto total_c) __attribute__((always_inline)) {
+    constexpr int n = decltype(n_c)::value, kTotal = decltype(total_c)::value, kWin = kTotal > S ? kAhead : S;
+    wait_vmcnt<(kWin - 1 < kTotal - 1 - n ? kWin - 1 : kTotal - 1 - n) * F>();
 #pragma unroll
-    for (int k = 0; k < S; ++k)
-#pragma unroll
-      for (int f = 0; f < F; ++f) tie(wq[0][k][f]);
-    compute_round(0, std::integral_constant<int, 0>{});
-  }
-  if (rounds > 1) {
-    settle(std::integral_constant<int, 1>{}, std::integral_constant<int, 0>{});
-    compute_round(1, std::integral_constant<int, 1>{});
-  }
+    for (int f = 0; f < F; ++f) tie(wq[n / S][n % S][f]);
+    compute_step(n / S, std::integral_constant<int, n / S>{}, std::integral_constant<int, n % S>{});
+    if constexpr (n + kWin < kTotal) request_nth(std::integral_constant<int, n + kWin>{});
+  };
+  if (rounds > 1) for_each_step<0, 2 * S>([&](auto n_c) __attribute__((always_inline)) { nth_step(n_c, std::integral_constant<int, 2 * S>{}); });
+  else if (rounds > 0) for_each_step<0, S>([&](auto n_c) __attribute__((always_inline)) { nth_step(n_c, std::integral_constant<int, S>{}); });
   for (int r = 2; r < rounds; r += 2) {
     request_round(r, std::integral_constant<int, 0>{});
     if (r + 1 < rounds) {

@@ -229,6 +229,19 @@ def test_decode_kernel_matches_oracle(abi, m, n, kn, ks, ko, tiled):
     _check_gemm(d, qx, qw, f"decode {m}x{n}x{k}")
 
 
+# The decode kernel's window of requested steps: 1 to 8 steps per wave (one round of four, and two), a last wave with fewer, for one,
+# two and four feature groups, whose windows are eight, five and four steps.
+@pytest.mark.parametrize("per_wave", range(1, 9))
+@pytest.mark.parametrize("m,n,tiled", [(3, 256, True), (9, 16640, False), (8, 12288, True)])
+def test_decode_kernel_requests_steps_as_it_goes(abi, per_wave, m, n, tiled):
+    steps = 4 * per_wave - per_wave % 3
+    s8 = 1 if steps > 2 else 0
+    s6 = (steps - s8) // 3
+    shape = (128 * (steps - s6 - s8), 128 * s6, 128 * s8)
+    if per_wave > 1 or not tiled:   # (plans of two segments, one stage each, are not tile-major)
+        test_decode_kernel_matches_oracle(abi, m, n, *shape, tiled)
+
+
 # 17 to 255 tokens: the skinny kernel (whole tiles where they are estimated faster), ragged token and feature counts, an
 # empty segment, a token count whose last workgroup has a single token group
 SMALL_M_SHAPES = [
