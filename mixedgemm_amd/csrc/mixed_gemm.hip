@@ -1181,6 +1181,10 @@ static SkinnyPlan skinny_plan(int M, int N, int steps, int cus, bool w_tiled) {
 //   K = 8192, M = 4: N = 4096 8.6 against 7.7 / 8.7 against 8.1, 14336 15.6 against 13.1 / 14.5 against 14.9;
 //   N = 18944, M = 16: K = 1024 7.8 against 7.2 / 7.2 against 6.7, 2048 8.9 against 8.8 / 8.8 against 8.7 (N = 28672: 8.7 against
 //     9.5 / 9.1 against 9.6), 2560 12.0 against 9.7 / 12.1 against 9.7;  N = 36864, K = 3584, M = 16 18.7 against 20.9 / 19.0 against 23.1.
+// (Both sides before the skinny kernel's shorter rings and this kernel's window of requested steps.  With them, layer calls from HBM / from the
+// caches, skinny against this kernel, M = 16, K = 4096: N = 4096 8.5 against 8.1 / 8.0 against 8.5 us, 6144 9.7 against 8.9 / 8.4 against 8.8, 8192
+// 10.0 against 9.1 / 8.5 against 8.9; the four projections of a decoder layer, 116 MB in a graph, 53.6 with the rule as it is, 55.9 with this
+// kernel for up to 16 tokens on 4096 and 6144 features.)
 // So: four feature groups (two such workgroups fit a CU), or one round of workgroups and at most 8 tokens; up to 32 K steps, so
 // that all of a wave's weights are in flight at once; up to 16 where the skinny kernel has eight feature groups; above 128
 // features per CU, where that needs two rounds, always.
