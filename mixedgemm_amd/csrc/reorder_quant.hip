@@ -522,12 +522,12 @@ hipError_t launch_reorder_quant(const void* x, const int16_t* idx, int rows, int
   hipError_t err = hipSuccess;
   // rows global -> LDS directly; NS row slots per workgroup, as many workgroups per CU as fit
   const int usable = lim.lds_bytes - 1024;   // the kernels' static LDS (row sums of the RMSNorm) stays below 1 KB
-  auto launch_dma = [&](auto kernel, int epl, int NS, int nthreads, int max_per_cu) {
+  auto launch_dma = [&](auto kernel, int epl, int NS, int nthreads, int max_per_cu, int most_waves = 16) {
     const int lds = (NS + (gm && epl == 16 ? 1 : 0)) * 2 * epl * nthreads;   // NS row slots, and the RMSNorm's weight
     if (lds > usable) { err = hipErrorInvalidValue; return; }
     int per_cu = usable / lds;
     per_cu = per_cu > max_per_cu ? max_per_cu : per_cu;
-    const int by_waves = 16 / (nthreads / 64);
+    const int by_waves = most_waves / (nthreads / 64);
     per_cu = per_cu > by_waves ? (by_waves < 1 ? 1 : by_waves) : per_cu;
     const int resident = lim.cus * per_cu;
     const int grid = rows < resident ? rows : resident;
@@ -549,15 +549,31 @@ hipError_t launch_reorder_quant(const void* x, const int16_t* idx, int rows, int
   // in front of a workgroup's first row and was slower.
   constexpr int kNS = 2;
   constexpr int kPerCu = 4;
+  // Activations of 8192 < K <= 16384 with two lanes per block as well, i.e. 9 ... 16 waves per workgroup, where that is the faster way (us, one
+  // lane per block against two; without RMSNorm):
+  //   9 and 10 waves, one workgroup per CU: K = 9216 rows 16 3.9 against 3.55, 128 4.3 / 4.15, 256 4.2 / 4.2, 512 5.9 / 6.2, 700 8.2 / 7.8, 1024 10.5 /
+  //     9.0, 4096 25.0 / 23.5; K = 10240 256 4.2 / 4.3, 512 6.2 / 6.45, 2048 15.2 / 14.6 (three per CU: 2048 rows of 9216 15 % slower than one lane);
+  //   11 and 12 waves, two per CU: K = 12288 rows 16 3.9 / 3.7, 512 6.9 / 6.3, 1024 10.2 / 9.5, 4096 28.3 / 26.6; K = 11008 512 6.8 / 6.35, 4096 25.9 /
+  //     24.8 (one per CU: up to 5 % slower than one lane);
+  //   13 ... 16 waves, one per CU: K = 14336 rows 16 4.05 / 4.0, 256 4.95 / 4.9, 512 7.6 / 7.75, 700 9.1 / 9.5, 1024 11.8 / 11.5, 2048 18.2 / 17.9, 4096
+  //     33.0 / 30.8; K = 16384 1024 13.1 / 12.05, 4096 37.3 / 34.3 (two per CU: up to 15 % slower).
+  // With RMSNorm, whose form for one lane per block normalizes the row in place: K = 9216 rows 16 5.2 / 5.1, 512 11.3 / 9.1, 2048 30.3 / 24.1; K = 12288
+  // 16 5.6 / 5.3, 2048 31.7 / 24.8; K = 14336 16 5.7 / 6.0, 100 6.3 / 6.3, 256 7.3 / 7.0, 700 17.4 / 14.9, 2048 33.9 / 29.3 (up to K = 15360: the
+  // LDS offsets of its three rows are immediates).
+  auto two_lanes = [&](int t2, bool norm) {
+    if (norm) return t2 <= 768 || (t2 <= 960 && 2 * rows >= lim.cus);
+    if (t2 > 1024) return false;
+    if (t2 < 704) return 2 * rows <= lim.cus || 2 * rows >= 5 * lim.cus;
+    return t2 <= 768 || rows <= lim.cus || rows >= 4 * lim.cus;
+  };
   // keep: the codes stay in the L2 for the kernel that reads them next (activations only); norm: RMSNorm of the row
   // before the gather (activations only; its codes are always kept: what follows a norm is the layer's GEMM)
   auto dispatch = [&](auto keep_c, auto norm_c, auto tiled_c) {
     constexpr bool TI = decltype(tiled_c)::value;
     constexpr bool KP = decltype(keep_c)::value;
     constexpr bool NM = decltype(norm_c)::value;
+    const int t2 = ((K >> 4) + 63) & ~63;   // two lanes per block: K/16 lanes, rounded up to whole waves
     if (K <= 8192) {
-      // two lanes per block: K/16 lanes, rounded up to whole waves
-      const int t2 = ((K >> 4) + 63) & ~63;
       switch (t2) {
         case 64: launch_dma(reorder_quant_dma_kernel<16, 64, kNS, IS_W, 64, KP, NM, TI>, 16, kNS, 64, kPerCu); break;
         case 128: launch_dma(reorder_quant_dma_kernel<16, 128, kNS, IS_W, 128, KP, NM, TI>, 16, kNS, 128, kPerCu); break;
@@ -567,6 +583,25 @@ hipError_t launch_reorder_quant(const void* x, const int16_t* idx, int rows, int
         case 384: launch_dma(reorder_quant_dma_kernel<16, 384, kNS, IS_W, 384, KP, NM, TI>, 16, kNS, 384, kPerCu); break;
         case 448: launch_dma(reorder_quant_dma_kernel<16, 448, kNS, IS_W, 448, KP, NM, TI>, 16, kNS, 448, kPerCu); break;
         default: launch_dma(reorder_quant_dma_kernel<16, 512, kNS, IS_W, 512, KP, NM, TI>, 16, kNS, 512, kPerCu); break;
+      }
+    } else if (!IS_W && two_lanes(t2, NM)) {
+      if constexpr (!IS_W) {
+        auto wide = [&](auto t_c) {
+          constexpr int T2 = decltype(t_c)::value;
+          launch_dma(reorder_quant_dma_kernel<16, T2, kNS, IS_W, T2, KP, NM, TI>, 16, kNS, T2, kPerCu, !NM && (T2 == 704 || T2 == 768) ? 24 : 16);
+        };
+        switch (t2) {
+          case 576: wide(std::integral_constant<int, 576>{}); break;
+          case 640: wide(std::integral_constant<int, 640>{}); break;
+          case 704: wide(std::integral_constant<int, 704>{}); break;
+          case 768: wide(std::integral_constant<int, 768>{}); break;
+          case 832: wide(std::integral_constant<int, 832>{}); break;
+          case 896: wide(std::integral_constant<int, 896>{}); break;
+          case 960: wide(std::integral_constant<int, 960>{}); break;
+          default:
+            if constexpr (!NM) wide(std::integral_constant<int, 1024>{});
+            break;
+        }
       }
     } else if (K <= 20480) {
       // one lane per block: the workgroups are large enough as it is, and LDS (two rows per workgroup) bounds how

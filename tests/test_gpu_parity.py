@@ -57,6 +57,29 @@ def test_reorder_quantize_matches_oracle(abi, which, rows, kn, ks, ko):
     H.assert_quant_equal(got, want, rows, (kn, ks, ko), what=f"{which} {rows}x{k}")
 
 
+# Activations of 8192 < K <= 16384: every workgroup size with two lanes per block, the smallest K of each and the largest, row counts on both
+# sides of where one lane per block takes over (of 128, 256, 640 and 1024), with RMSNorm (up to K = 15360), and with the codes kept for the
+# GEMM of a layer call.
+@pytest.mark.parametrize("k", [8224, 9248, 10272, 11296, 12320, 13344, 14368, 15360, 15392, 16384])
+@pytest.mark.parametrize("rows", [3, 129, 257, 641, 1025])
+def test_wide_rows_with_two_lanes_per_block(abi, k, rows):
+    kn, ko = k * 5 // 8 // 32 * 32, k // 32 // 32 * 32 + 32
+    ks = k - kn - ko
+    _say("wide rows", rows, kn, ks, ko)
+    test_reorder_quantize_matches_oracle(abi, "x", rows, kn, ks, ko)
+    if rows <= 257:
+        test_rmsnorm_reorder_quantize_matches_oracle(abi, rows, kn, ks, ko, 1e-5)
+    if rows <= 129:
+        x, idx = _quant_inputs(rows, k, 400 + rows)
+        x, idx, w = x.to(DEV), idx.to(DEV), H.make_weights(256, k, 401).to(DEV)
+        b = abi.reorder_quantize_w(w, idx, kn, ks, ko)
+        a = abi.reorder_quantize_x(x, idx, kn, ks, ko)
+        d = abi.fused_linear(x, idx, *b, kn, ks, ko)
+        want = abi.matmul(a[0], b[0], a[1], b[1], a[2], b[2], a[3], b[3], a[4], b[4], a[5], b[5])
+        torch.cuda.synchronize()
+        assert torch.equal(d, want)
+
+
 def _adversarial(k):
     rows = []
     z = np.zeros(k, np.float32)
