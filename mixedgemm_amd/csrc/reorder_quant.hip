@@ -560,11 +560,13 @@ hipError_t launch_reorder_quant(const void* x, const int16_t* idx, int rows, int
   // With RMSNorm, whose form for one lane per block normalizes the row in place: K = 9216 rows 16 5.2 / 5.1, 512 11.3 / 9.1, 2048 30.3 / 24.1; K = 12288
   // 16 5.6 / 5.3, 2048 31.7 / 24.8; K = 14336 16 5.7 / 6.0, 100 6.3 / 6.3, 256 7.3 / 7.0, 700 17.4 / 14.9, 2048 33.9 / 29.3 (up to K = 15360: the
   // LDS offsets of its three rows are immediates).
-  auto two_lanes = [&](int t2, bool norm) {
+  // Codes kept for the GEMM that follows, many rows, the call with the GEMM: 2048 rows of 14336 79.9 / 80.9, 4096 138.0 / 140.9, of 9216 69.6 / 70.4 --
+  // not taken there; of 12288 81.2 / 80.6.
+  auto two_lanes = [&](int t2, bool norm, bool kept) {
     if (norm) return t2 <= 768 || (t2 <= 960 && 2 * rows >= lim.cus);
     if (t2 > 1024) return false;
-    if (t2 < 704) return 2 * rows <= lim.cus || 2 * rows >= 5 * lim.cus;
-    return t2 <= 768 || rows <= lim.cus || rows >= 4 * lim.cus;
+    if (t2 < 704) return 2 * rows <= lim.cus || (!kept && 2 * rows >= 5 * lim.cus);
+    return t2 <= 768 || rows <= lim.cus || (!kept && rows >= 4 * lim.cus);
   };
   // keep: the codes stay in the L2 for the kernel that reads them next (activations only); norm: RMSNorm of the row
   // before the gather (activations only; its codes are always kept: what follows a norm is the layer's GEMM)
@@ -584,7 +586,7 @@ hipError_t launch_reorder_quant(const void* x, const int16_t* idx, int rows, int
         case 448: launch_dma(reorder_quant_dma_kernel<16, 448, kNS, IS_W, 448, KP, NM, TI>, 16, kNS, 448, kPerCu); break;
         default: launch_dma(reorder_quant_dma_kernel<16, 512, kNS, IS_W, 512, KP, NM, TI>, 16, kNS, 512, kPerCu); break;
       }
-    } else if (!IS_W && two_lanes(t2, NM)) {
+    } else if (!IS_W && two_lanes(t2, NM, KP)) {
       if constexpr (!IS_W) {
         auto wide = [&](auto t_c) {
           constexpr int T2 = decltype(t_c)::value;
