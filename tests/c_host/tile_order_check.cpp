@@ -36,6 +36,23 @@ int main() {
         next = tn * tiles_m + tm + 1;
       }
     }
+    // runs whatever the counts (the skinny kernel's): every tile once, consecutive on an XCD
+    const mg::TileOrder runs = mg::tile_runs(tiles_n, tiles_m);
+    std::vector<bool> ran(nwg, false);
+    for (int xcd = 0; xcd < 8; ++xcd) {
+      int next = -1;
+      for (int wg = xcd; wg < nwg; wg += 8) {
+        int tn = -1, tm = -1;
+        mg::tile_at(runs, wg, tn, tm);
+        const bool inside = tn >= 0 && tn < tiles_n && tm >= 0 && tm < tiles_m;
+        if (!inside || ran[(size_t)tn * tiles_m + tm] || (next >= 0 && tn * tiles_m + tm != next)) {
+          printf("%d x %d tiles in runs: workgroup %d -> (%d, %d)\n", tiles_n, tiles_m, wg, tn, tm);
+          break;
+        }
+        ran[(size_t)tn * tiles_m + tm] = true;
+        next = tn * tiles_m + tm + 1;
+      }
+    }
     ++grids;
   }
   printf("%d grids\n", grids);
