@@ -62,6 +62,11 @@ NO_SCRATCH_KERNELS = ("mixed_gemm_decode_kernel", "reorder_quant_dma_kernel", "m
 MAY_SPILL = ("reorder_quant_dma_kernelILi32ELi0E",)
 
 
+# Kernels in whose loops every step begins with scalar address arithmetic: scalars spilled to vector lanes come back one
+# instruction at a time in front of each request.
+NO_SCALAR_SPILL_KERNELS = ("mixed_gemm_skinny_kernel", "mixed_gemm_token_kernel", "mixed_gemm_decode_kernel")
+
+
 def _split_remarks(stderr: str) -> tuple[str, str]:
     """(resource-usage remarks, everything else) of a hipcc run with -Rpass-analysis=kernel-resource-usage."""
     remarks, other, skip = [], [], 0
@@ -76,7 +81,7 @@ def _split_remarks(stderr: str) -> tuple[str, str]:
     return "\n".join(remarks), "\n".join(other)
 
 
-def _check_no_scratch(src: str, remarks: str) -> None:
+def _check_spills(src: str, remarks: str) -> None:
     import re
     name, bad = None, []
     for line in remarks.splitlines():
@@ -86,6 +91,9 @@ def _check_no_scratch(src: str, remarks: str) -> None:
         m = re.search(r"ScratchSize \[bytes/lane\]: (\d+)", line)
         if m and name and int(m.group(1)) and any(k in name for k in NO_SCRATCH_KERNELS) and not any(k in name for k in MAY_SPILL):
             bad.append(f"{name}: {m.group(1)} bytes of scratch per lane")
+        m = re.search(r"SGPRs Spill: (\d+)", line)
+        if m and name and int(m.group(1)) and any(k in name for k in NO_SCALAR_SPILL_KERNELS):
+            bad.append(f"{name}: {m.group(1)} scalar registers spilled")
     if bad:
         raise RuntimeError(f"{os.path.basename(src)}: kernels that must not spill do:\n  " + "\n  ".join(bad))
 
@@ -113,7 +121,7 @@ def _compile_and_link(sources: list[str], target: str, force: bool, verbose: boo
             if done.returncode != 0:
                 raise subprocess.CalledProcessError(done.returncode, cmd)
             try:
-                _check_no_scratch(src, remarks)
+                _check_spills(src, remarks)
             except Exception:
                 os.remove(obj)
                 raise

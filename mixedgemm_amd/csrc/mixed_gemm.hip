@@ -165,6 +165,12 @@ mixed_gemm_skinny_kernel(DecodeSeg s4, DecodeSeg s6, DecodeSeg s8, int M, int N,
   // layer's four projections of 16 tokens, whose others (58 MB) then stay in it, 62.5 -> 56.3.
   constexpr bool kStream = WT && F == 8;
   constexpr int kScales = 1024 * (F + 2 * G);   // where a slot's scales begin
+  // Whole steps two at a time where the ring has four slots.  Out of three, with one step in flight, pairs are slower (N = 20480, K = 5120, M =
+  // 16 18.5 against 18.0 us).
+  constexpr bool kPairs = NS > 3;
+  // Requests of whole steps by advancing addresses, which single steps out of three slots use on row-major weights alone: on tile-major ones
+  // both ways of addressing are more scalars than there are (8 and 9 were spilled; 24 calls of (1, 8) 1.0 % and 1.8 % faster without).
+  constexpr bool kAdvance = kPairs || !WT;
   static_assert(NS >= 3 && PA + PB <= 64, "a pipeline; one copy for all scales of a step");
   extern __shared__ __align__(16) uint8_t lds[];
   // all arguments in one batch of loads (see pin_args)
@@ -316,7 +322,7 @@ mixed_gemm_skinny_kernel(DecodeSeg s4, DecodeSeg s6, DecodeSeg s8, int M, int N,
       for (int f = 0; f < F; ++f)
         acc[f][gi] = decode_mfma<FMT>(v8i{r.w[f][0], r.w[f][1], r.w[f][2], r.w[f][3], 0, 0, 0, 0}, r.x[gi], acc[f][gi], r.s_w[f], r.s_x[gi]);
   };
-  // the wave's steps of one segment, two at a time
+  // the wave's steps of one segment
   auto run = [&](auto fmt_c, const DecodeSeg& s, const uint8_t* sc, int t_first, int t_next) __attribute__((always_inline)) {
     constexpr int FMT = decltype(fmt_c)::value, TC = kTokenCopies<FMT, G>, PER = 1 + F + TC;
     const int last = min(t_next, t_end);
@@ -329,7 +335,7 @@ mixed_gemm_skinny_kernel(DecodeSeg s4, DecodeSeg s6, DecodeSeg s8, int M, int N,
     const unsigned pitch = (unsigned)s.nblk * Frag<FMT>::kBytes;
     const uint8_t* a_next = s.a + (size_t)m_base * pitch + (ptrdiff_t)q_next * (4 * Frag<FMT>::kBytes);
     unsigned w_off[F], a_off[TC];
-    if (t + NS - 1 < whole_end) {
+    if (kAdvance && t + NS - 1 < whole_end) {
 #pragma unroll
       for (int f = 0; f < F; ++f) w_off[f] = WT ? (unsigned)(lane >> 2) * 64u + wpos * 16u : (unsigned)wrow[f] * (unsigned)s.nblk * 16u + wpos * 16u;
 #pragma unroll
@@ -340,7 +346,7 @@ mixed_gemm_skinny_kernel(DecodeSeg s4, DecodeSeg s6, DecodeSeg s8, int M, int N,
       }
     }
     auto next = [&](int ahead, unsigned to) __attribute__((always_inline)) {
-      if (ahead < whole_end) {
+      if (kAdvance && ahead < whole_end) {
         if (lane < kSkinnyPieces<G, F>) dma16_lane(sc_next, to + kScales);
 #pragma unroll
         for (int f = 0; f < F; ++f) dma16_at<kStream>(WT ? w_next + f * 1024 : w_next, w_off[f], to + 1024u * f);
@@ -353,12 +359,12 @@ mixed_gemm_skinny_kernel(DecodeSeg s4, DecodeSeg s6, DecodeSeg s8, int M, int N,
         request(ahead, to);
       }
     };
-    // Steps up to t + NS - 2 have been requested.  What is waited for has at least `younger` steps behind it, each with at
-    // least as many copies as this segment's (a token takes more bytes in every later segment's format).
+    // Steps up to t + NS - 2 have been requested.  A wait counts the steps behind the one waited for, each with at least as
+    // many copies as this segment's (a token takes more bytes in every later segment's format).
     while (t < last) {
       const uint8_t* sl = ring + slot * kSlot;
       const unsigned freed = ring0 + (unsigned)(slot == 0 ? NS - 1 : slot - 1) * kSlot;   // read a step ago
-      if (NS > 3 && t + 1 < whole_end) {   // (out of three slots, with one step in flight: N = 20480, K = 5120, M = 16 18.0 us, in pairs 18.5)
+      if (kPairs && t + 1 < whole_end) {
         const int after = slot == NS - 1 ? 0 : slot + 1;
         const unsigned this_slot = ring0 + (unsigned)slot * kSlot;
         next(t + NS - 1, freed);

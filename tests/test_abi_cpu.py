@@ -343,3 +343,18 @@ def test_small_tiles_are_not_taken_where_they_were_measured_slower(abi, m, n, kn
     for tiled in (False, True):
         if not tiled or abi.weights_tileable(n, kn, ks, ko):
             assert (abi.gemm_kernel(m, n, kn, ks, ko, tiled)[0] != "tile") == others
+
+
+def test_build_refuses_kernels_that_spill():
+    """Scratch memory where inline-assembly loads are in flight, and scalars spilled in the few-token kernels' loops."""
+    from mixedgemm_amd import build
+
+    def remarks(name, scratch, scalars):
+        return "\n".join(f"mixed_gemm.hip:1:1: remark:     {text} [-Rpass-analysis=kernel-resource-usage]" for text in
+                         (f"Function Name: {name}", f"ScratchSize [bytes/lane]: {scratch}", f"SGPRs Spill: {scalars}"))
+
+    skinny, decode = "_ZN2mg24mixed_gemm_skinny_kernelILi1ELi8ELb1EEE", "_ZN2mg24mixed_gemm_decode_kernelILi4ELb1EEE"
+    build._check_spills("mixed_gemm.hip", remarks(skinny, 0, 0) + "\n" + remarks(decode, 0, 0) + "\n" + remarks("other", 16, 9))
+    for bad in (remarks(skinny, 0, 9), remarks(decode, 0, 1), remarks(decode, 16, 0)):
+        with pytest.raises(RuntimeError):
+            build._check_spills("mixed_gemm.hip", bad)
