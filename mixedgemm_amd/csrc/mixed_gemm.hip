@@ -166,11 +166,12 @@ mixed_gemm_skinny_kernel(DecodeSeg s4, DecodeSeg s6, DecodeSeg s8, int M, int N,
   constexpr bool kStream = WT && F == 8;
   constexpr int kScales = 1024 * (F + 2 * G);   // where a slot's scales begin
   // Whole steps two at a time where the ring has four slots.  Out of three, with one step in flight, pairs are slower (N = 20480, K = 5120, M =
-  // 16 18.5 against 18.0 us).
-  constexpr bool kPairs = NS > 3;
+  // 16 18.5 against 18.0 us), and so they are with two token and four feature groups on row-major weights, where the copies of half
+  // lines are what a step waits for (24 calls, from HBM / from the caches 1.5 % and 1.4 % faster one at a time; M = 20, N = 11264, K = 2496 9.1 -> 8.8).
+  constexpr bool kPairs = NS > 3 && (WT || G != 2 || F != 4);
   // Requests of whole steps by advancing addresses, which single steps out of three slots use on row-major weights alone: on tile-major ones
   // both ways of addressing are more scalars than there are (8 and 9 were spilled; 24 calls of (1, 8) 1.0 % and 1.8 % faster without).
-  constexpr bool kAdvance = kPairs || !WT;
+  constexpr bool kAdvance = NS > 3 ? kPairs : !WT;
   static_assert(NS >= 3 && PA + PB <= 64, "a pipeline; one copy for all scales of a step");
   extern __shared__ __align__(16) uint8_t lds[];
   // all arguments in one batch of loads (see pin_args)
