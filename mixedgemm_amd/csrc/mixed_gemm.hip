@@ -849,7 +849,7 @@ struct TokenLds {   // byte offsets behind the rings
   int total;
 };
 // Slots per wave: 20 ... 64 KB of weight codes in flight per CU (see kSkinnySlots; with 12 / 8 / 5 of them, us: N = K = 4096 6.2, now 5.9; N = K =
-// 8192 10.7, now 9.9; N = 14336, K = 4096 8.6, now 8.5; 2 to 5 steps per wave on row-major weights 4.5 ... 4.8, now 4.65 ... 4.9)
+// 8192 10.7, now 9.9; N = 14336, K = 4096 8.6, now 8.5)
 template <int F>
 constexpr int kTokenSlots = F == 1 ? 5 : (F == 2 ? 5 : 4);
 
@@ -879,6 +879,9 @@ mixed_gemm_token_kernel(const uint8_t* __restrict__ x, const uint8_t* __restrict
   constexpr int NS = kTokenSlots<F>, kSlot = 1024 * F;
   constexpr int PB = 4 * F, PBLOG = F == 1 ? 2 : (F == 2 ? 3 : 4);
   static_assert(NS - 1 <= 11, "wait_steps");
+  // (four feature groups: 8.45 us one at a time, 8.6 in pairs; two on row-major weights: 80 calls from HBM / from the caches 1.6 % and 1.3 %
+  // faster one at a time, N = 7936, K = 2048, M = 2 5.05 -> 4.9)
+  constexpr bool kPairs = F == 1 || (F == 2 && WT);
   extern __shared__ __align__(16) uint8_t lds[];
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int i = lane & 15, g = lane >> 4;
@@ -1059,7 +1062,7 @@ mixed_gemm_token_kernel(const uint8_t* __restrict__ x, const uint8_t* __restrict
       request(t + NS - 1, ring0 + (unsigned)(slot == 0 ? NS - 1 : slot - 1) * kSlot);
       slot = slot == NS - 1 ? 0 : slot + 1;
       const int q = t - t_first;
-      if (F < 4 && t + 1 < whole_end) {   // (four feature groups: 8.45 us one at a time, 8.6 in pairs)
+      if (kPairs && t + 1 < whole_end) {
         if (t + NS - 1 < t_end) wait_vmcnt<(NS - 2) * F>();
         else wait_steps<F, NS - 3>(t_end - 2 - t);
         Fragments r0, r1;
