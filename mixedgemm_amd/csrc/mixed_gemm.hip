@@ -1404,8 +1404,11 @@ hipError_t launch_mixed_gemm(const uint8_t* an, const uint8_t* bn, const uint8_t
 }
 
 // Quantization and GEMM of a few tokens in one launch, where that is the faster way; *taken says whether it was.
-// Every workgroup repeats the quantization, so it pays up to 20480 channels in all (us, two launches against one, N = 4096 / 14336, K = 4096: M =
-// 5 8.2 against 7.8 / 11.4 against 10.3, M = 6 8.3 against 8.6), with RMSNorm up to 10240 (M = 3 9.0 against 9.0 / 12.2 against 11.4, but 10.5 against
+// Every workgroup repeats the quantization, so it pays up to 16384 channels in all, up to 20480 for 5 tokens, 6 and 8 of them on row-major weights
+// with two and four feature groups (120 shapes above 16384, two launches over one from HBM / from the caches: tile-major M = 3 ... 5 0.99 ... 1.13
+// / 0.94 ... 1.08, 6 0.98 ... 1.07 / 0.95 ... 1.00, 7 0.98 ... 1.04 / 0.93 ... 0.97, 8 0.95 ... 1.05 / 0.92 ... 0.99; row-major with one group M = 4 and 5 1.02 ... 1.06 /
+// 1.00 ... 1.03, 6 1.00 / 0.99, 8 0.96 / 0.93, with two M = 6 1.13 / 1.01, 7 1.09 / 0.97, with four M = 8 1.12 / 1.04), with RMSNorm up to 10240
+// (M = 3, N = 4096 / 14336, K = 4096 9.0 against 9.0 / 12.2 against 11.4, but 10.5 against
 // 11.1 with the weights in the caches, N = 13312), from 5 tokens on, where a token's norm is one wave's work, 8192 (M = 8, K = 1024 level, K =
 // 2048 7.6 against 8.8), for rows of at most 8192 (M = 1, K = 14336, with longer rings: 13.7 against 14.0), and in one round of workgroups.
 hipError_t launch_token_linear(const void* x, const int16_t* idx, const void* gamma, float eps, const uint8_t* bn, const uint8_t* bs,
@@ -1428,7 +1431,7 @@ hipError_t launch_token_linear(const void* x, const int16_t* idx, const void* ga
   const int total = d4.steps + d6.steps + d8.steps;
   const int f = ceil_div(N, 16) <= lim.cus ? 1 : (ceil_div(N, 32) <= lim.cus ? 2 : 4);
   const int grid = w_tiled ? ceil_div(N, 16 * f) : ceil_div(N, 128) * (8 / f);
-  if (grid > lim.cus) return hipSuccess;
+  if (grid > lim.cus || (M * K > 16384 && M > (w_tiled ? 5 : 4 + f))) return hipSuccess;
   TokenLds L;
   int pos = 4 * 1024 * (f == 1 ? kTokenSlots<1> : (f == 2 ? 2 * kTokenSlots<2> : 4 * kTokenSlots<4>));
   auto take = [&](int bytes) { const int at = pos; pos += round_up_1k(bytes); return at; };
