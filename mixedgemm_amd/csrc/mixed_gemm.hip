@@ -690,8 +690,10 @@ mixed_gemm_decode_kernel(DecodeSeg s4, DecodeSeg s6, DecodeSeg s8, int M, int N,
     constexpr int n = decltype(n_c)::value;
     request_step(n / S, std::integral_constant<int, n / S>{}, std::integral_constant<int, n % S>{});
   };
-  if (rounds > 1) for_each_step<0, kAhead>(request_nth);
-  else if (rounds > 0) request_round(0, std::integral_constant<int, 0>{});
+  // (the first round in one place for both cases: a register that is still to be filled must not have two loads meeting in it where branches join)
+  static_assert(kAhead >= S, "the first round is requested up front");
+  if (rounds > 0) for_each_step<0, S>(request_nth);
+  if (rounds > 1) for_each_step<S, kAhead>(request_nth);
 
   // ---- the copies are older than all of them
   if (rounds > 1) wait_vmcnt<kAhead * F>();
