@@ -555,18 +555,20 @@ hipError_t launch_reorder_quant(const void* x, const int16_t* idx, int rows, int
   //     9.0, 4096 25.0 / 23.5; K = 10240 256 4.2 / 4.3, 512 6.2 / 6.45, 2048 15.2 / 14.6 (three per CU: 2048 rows of 9216 15 % slower than one lane);
   //   11 and 12 waves, two per CU: K = 12288 rows 16 3.9 / 3.7, 512 6.9 / 6.3, 1024 10.2 / 9.5, 4096 28.3 / 26.6; K = 11008 512 6.8 / 6.35, 4096 25.9 /
   //     24.8 (one per CU: up to 5 % slower than one lane);
-  //   13 ... 16 waves, one per CU: K = 14336 rows 16 4.05 / 4.0, 256 4.95 / 4.9, 512 7.6 / 7.75, 700 9.1 / 9.5, 1024 11.8 / 11.5, 2048 18.2 / 17.9, 4096
-  //     33.0 / 30.8; K = 16384 1024 13.1 / 12.05, 4096 37.3 / 34.3 (two per CU: up to 15 % slower).
+  //   13 ... 16 waves, one per CU: 1 ... 256 rows 0.05 ... 0.15 faster with two (K = 12800 1.02, 14336 1.01, 16384 1.03 times as fast; medians, single runs differ by
+  //     1 %); K = 14336 512 7.6 / 7.75, 700 9.1 / 9.5, 1024 11.8 / 11.5, 2048 18.2 / 17.9, 4096 33.0 / 30.8; K = 16384 1024 13.1 / 12.05, 4096 37.3 / 34.3;
+  //     with 13 waves (K = 12800) 1024 level, 1200 0.97 times as fast, 2048 level, 4096 1.08 (two per CU: up to 15 % slower).
   // With RMSNorm, whose form for one lane per block normalizes the row in place: K = 9216 rows 16 5.2 / 5.1, 512 11.3 / 9.1, 2048 30.3 / 24.1; K = 12288
-  // 16 5.6 / 5.3, 2048 31.7 / 24.8; K = 14336 16 5.7 / 6.0, 100 6.3 / 6.3, 256 7.3 / 7.0, 700 17.4 / 14.9, 2048 33.9 / 29.3 (up to K = 15360: the
-  // LDS offsets of its three rows are immediates).
-  // Codes kept for the GEMM that follows, many rows, the call with the GEMM: 2048 rows of 14336 79.9 / 80.9, 4096 138.0 / 140.9, of 9216 69.6 / 70.4 --
-  // not taken there; of 12288 81.2 / 80.6.
+  // 16 5.6 / 5.3, 2048 31.7 / 24.8; K = 14336 16 5.7 / 6.0, 100 6.3 / 6.3, 256 7.3 / 7.0, 700 17.4 / 14.9, 2048 33.9 / 29.3; K = 12800 and 15360, one over two: 64
+  // rows 0.95, 128 0.96 and 0.98, 200 0.98 and 1.02, 256 1.00 and 1.02, 300 1.14 and 1.18 (up to K = 15360: the LDS offsets of its three rows are immediates).
+  // Codes kept for the GEMM that follows, gain of two lanes per layer call, us (N = 2048 and 4096; two figures of one side differ by 0.1 %): 9 and 10
+  // waves, 1 ... 128 rows 0.25 ... 0.3, 200 0.2, 384 -0.1 ... -0.6, 1024 0.1 ... 0.7, 2048 -0.5 ... -0.6, 4096 -0.7 ... -0.8; 11 and 12, up to 128 rows 0.1 ... 0.25, 512
+  // 0.4 ... 0.5, 700 0.7, 1024 0.3, 2048 0.2 ... 0.4, 4096 -0.1 ... 0.1; 13 ... 16, up to 256 rows 0.05 ... 0.25, 512 -0.3 ... -0.5, 1024 -0.1 ... 0.2, 4096 -1.1 ... -2.1.
   auto two_lanes = [&](int t2, bool norm, bool kept) {
-    if (norm) return t2 <= 768 || (t2 <= 960 && 2 * rows >= lim.cus);
+    if (norm) return t2 <= 768 || (t2 <= 960 && 4 * rows >= 3 * lim.cus);
     if (t2 > 1024) return false;
     if (t2 < 704) return 2 * rows <= lim.cus || (!kept && 2 * rows >= 5 * lim.cus);
-    return t2 <= 768 || rows <= lim.cus || (!kept && rows >= 4 * lim.cus);
+    return t2 <= 768 || rows <= lim.cus || (!kept && rows >= (t2 == 832 ? 8 : 4) * lim.cus);
   };
   // keep: the codes stay in the L2 for the kernel that reads them next (activations only); norm: RMSNorm of the row
   // before the gather (activations only; its codes are always kept: what follows a norm is the layer's GEMM)
