@@ -57,27 +57,51 @@ def test_reorder_quantize_matches_oracle(abi, which, rows, kn, ks, ko):
     H.assert_quant_equal(got, want, rows, (kn, ks, ko), what=f"{which} {rows}x{k}")
 
 
+def _wide_split(k):
+    kn, ko = k * 5 // 8 // 32 * 32, k // 32 // 32 * 32 + 32
+    return kn, k - kn - ko, ko
+
+
+def _check_kept_codes(abi, rows, k):
+    """A layer call, whose quantizer keeps the codes in the caches, against the quantizer and the GEMM one after the other."""
+    split = _wide_split(k)
+    x, idx = _quant_inputs(rows, k, 400 + rows)
+    x, idx, w = x.to(DEV), idx.to(DEV), H.make_weights(256, k, 401).to(DEV)
+    b = abi.reorder_quantize_w(w, idx, *split)
+    a = abi.reorder_quantize_x(x, idx, *split)
+    d = abi.fused_linear(x, idx, *b, *split)
+    want = abi.matmul(a[0], b[0], a[1], b[1], a[2], b[2], a[3], b[3], a[4], b[4], a[5], b[5])
+    torch.cuda.synchronize()
+    assert torch.equal(d, want)
+
+
 # Activations of 8192 < K <= 16384: every workgroup size with two lanes per block, the smallest K of each and the largest, row counts on both
-# sides of where one lane per block takes over (of 128, 256, 640 and 1024), with RMSNorm (up to K = 15360), and with the codes kept for the
+# sides of where one lane per block takes over (of 128, 192, 256, 640 and 1024), with RMSNorm (up to K = 15360), and with the codes kept for the
 # GEMM of a layer call.
 @pytest.mark.parametrize("k", [8224, 9248, 10272, 11296, 12320, 13344, 14368, 15360, 15392, 16384])
 @pytest.mark.parametrize("rows", [3, 129, 257, 641, 1025])
 def test_wide_rows_with_two_lanes_per_block(abi, k, rows):
-    kn, ko = k * 5 // 8 // 32 * 32, k // 32 // 32 * 32 + 32
-    ks = k - kn - ko
-    _say("wide rows", rows, kn, ks, ko)
-    test_reorder_quantize_matches_oracle(abi, "x", rows, kn, ks, ko)
+    split = _wide_split(k)
+    _say("wide rows", rows, *split)
+    test_reorder_quantize_matches_oracle(abi, "x", rows, *split)
     if rows <= 257:
-        test_rmsnorm_reorder_quantize_matches_oracle(abi, rows, kn, ks, ko, 1e-5)
+        test_rmsnorm_reorder_quantize_matches_oracle(abi, rows, *split, 1e-5)
     if rows <= 129:
-        x, idx = _quant_inputs(rows, k, 400 + rows)
-        x, idx, w = x.to(DEV), idx.to(DEV), H.make_weights(256, k, 401).to(DEV)
-        b = abi.reorder_quantize_w(w, idx, kn, ks, ko)
-        a = abi.reorder_quantize_x(x, idx, kn, ks, ko)
-        d = abi.fused_linear(x, idx, *b, kn, ks, ko)
-        want = abi.matmul(a[0], b[0], a[1], b[1], a[2], b[2], a[3], b[3], a[4], b[4], a[5], b[5])
-        torch.cuda.synchronize()
-        assert torch.equal(d, want)
+        _check_kept_codes(abi, rows, k)
+
+
+# The same instances with more rows than both slots of every workgroup hold, so that slots are filled again and the RMSNorm's sums change
+# places: one workgroup per CU has three or four of 900 rows and eight or nine of 2100 (where 13 waves take over again), two per CU, with 11 and
+# 12 waves and no RMSNorm, two or three of 1100.
+@pytest.mark.parametrize("k", [8224, 9248, 10272, 11296, 12288, 12320, 13344, 14368, 15360])
+def test_wide_rows_refill_their_slots_with_rmsnorm(abi, k):
+    test_rmsnorm_reorder_quantize_matches_oracle(abi, 900, *_wide_split(k), 1e-5)
+
+
+@pytest.mark.parametrize("rows,k", [(1100, 10272), (1100, 11296), (1100, 12288), (2100, 12320)])
+def test_wide_rows_refill_their_slots(abi, rows, k):
+    test_reorder_quantize_matches_oracle(abi, "x", rows, *_wide_split(k))
+    _check_kept_codes(abi, rows, k)
 
 
 def _adversarial(k):
