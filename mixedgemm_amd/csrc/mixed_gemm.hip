@@ -1146,19 +1146,21 @@ static bool decode_lds_plan(const DecodeSeg& d4, const DecodeSeg& d6, const Deco
 }
 
 // Token groups (g) and feature groups (f) of 16 per workgroup of the skinny kernel, and its launch time in microseconds:
-// the pair with the lowest estimate.  A workgroup has its CU to itself (LDS) and takes ~2.3 us to fill and drain its
-// pipeline plus the table's nanoseconds per K step; a further round of workgroups costs more than the first (fitted).
+// the pair with the lowest estimate.  A workgroup takes ~2.3 us to fill and drain its pipeline plus the table's nanoseconds per
+// K step; a further round of workgroups costs more than the first (fitted).  A round is a workgroup per CU, also for (1, 1) and
+// (1, 2), of which three and two fit a CU's LDS: side by side they share its requests, and the form with half as many workgroups is
+// faster (M = 16, K = 4096, us from the caches / from HBM, two workgroups of (1, 1) per CU against one of (1, 2): N = 8192 tile-major 6.4
+// against 5.4 / 8.15 against 6.6, row-major 6.45 against 5.6 / 8.3 against 7.4; two of (1, 2) against one of (1, 4), N = 12288 7.9 against 7.5 / 10.3
+// against 8.9, row-major 8.4 against 8.2 / 11.3 against 10.2).
 // Row-major weights have a column of their own (a weight copy touches 16 half lines there, 8 lines on tile-major ones): the
 // smallest forms are cheaper than on tile-major weights, the two largest dearer, which changes their order.  Two and four
 // token groups with one feature group are not among the forms: half the token groups with twice the feature groups are never
 // more workgroups, and cheaper (83 against 77 and 99 against 86 ns on tile-major weights, 69 / 62 and 96 / 89 on row-major).
-// Estimate against measurement, with the weights in the caches / from HBM (rotating over more than 600 MB):
-//   tile-major, N = 4096, K = 14336: M = 16 10.9 against 10.3 / 12.5 us, 128 15.7 against 19.9 / 24.5, 200 32 against 34 / 40;
-//     N = 5120, K = 5120: M = 8 6.5 against 6.8 / 7.7, 128 16.1 against 19.0 / 20.3;  N = 14336, K = 4096, M = 64 15.6
-//     against 16.0 / 20.1
-//   row-major, N = 4096, K = 14336: M = 16 8.5 against 9.8 / 12.7 us, 128 18.4 against 20.7 / 25.6, 200 37 against 35 / 40;
-//     N = 5120, K = 5120: M = 8 5.8 against 6.4 / 8.1, 128 18.1 against 17.3 / 18.8;  N = 14336, K = 4096, M = 64 15.7
-//     against 16.3 / 20.5
+// Estimate against measurement, with the weights in the caches / from HBM (rotating over 1.3 GB), us:
+//   tile-major, N = 4096, K = 14336: M = 16 10.9 against 9.3 / 11.6, 128 15.7 against 17.1 / 22.7; N = K = 5120: M = 8 6.5 against
+//     5.75 / 6.7; N = 2560, K = 5120, M = 128 7.8 against 8.6 / 11.0
+//   row-major, N = 4096, K = 14336: M = 16 8.5 against 8.95 / 12.2, 128 18.4 against 20.2 / 25.2; N = K = 5120: M = 8 5.8 against
+//     5.3 / 7.5
 // Eight feature groups are for 64 to 128 features per CU and up to 16 tokens, where four need a second round (from HBM, M = 16,
 // tile-major / row-major weights, us): N = 20480, K = 5120 19.3 -> 16.3 / 23.6 -> 20.6, N = 28672, K = 5120 22.0 -> 17.1 / 25.9 -> 22.6, N =
 // 18944, K = 3584 15.7 -> 11.6.  Up to 64 features per CU they are slower (N = 16384, K = 5120 15.2 against 12.3), and so they are
@@ -1166,21 +1168,22 @@ static bool decode_lds_plan(const DecodeSeg& d4, const DecodeSeg& d6, const Deco
 // Over 1511 calls of 17 to 255 tokens (N 256 ... 28672, K 1024 ... 18944) the form taken, whole tiles included, is in the
 // mean 1.2 / 3.0 % (row-major) and 2.0 / 3.2 % (tile-major) slower than the best one, 22 / 60 % and 27 / 40 % at most; with the
 // tile-major figures row-major weights were at 3.0 / 5.2 and 68 / 77 %.
+// On tile-major weights (2, 2) and (4, 2) give way to half the tokens and twice the features wherever those are as many workgroups: M = 56, N =
+// 3584, K = 8192 (1, 4) against (2, 2) 8.6 / 11.2 against 8.6 / 11.6; M = 64, N = K = 4096 6.35 / 7.7 against 6.0 / 8.1; M = 128, N = K = 4096 (2, 4)
+// against (4, 2) 7.8 / 9.7 against 8.3 / 10.2, K = 14336 17.1 / 22.7 against 19.1 / 24.5.  The estimate is the same for both.
 struct SkinnyPlan { int g, f; double us; };
 static SkinnyPlan skinny_plan(int M, int N, int steps, int cus, bool w_tiled) {
-  // row-major, tile-major weights; `even`: with an even number of token groups, where the form of half the features and twice the tokens
-  // has as many workgroups
-  static const struct { int g, f; double ns[2], even[2]; } kForms[] = {
-      {1, 1, {46, 67}, {46, 67}}, {1, 2, {62, 77}, {62, 77}}, {1, 4, {104, 102}, {104, 85}}, {2, 2, {89, 86}, {89, 86}},
-      {2, 4, {145, 117}, {145, 106}}, {4, 2, {134, 110}, {134, 110}}, {1, 8, {230, 225}, {230, 225}}};
+  static const struct { int g, f; double ns[2]; } kForms[] = {   // row-major, tile-major weights
+      {1, 1, {46, 67}}, {1, 2, {62, 77}}, {1, 4, {104, 102}}, {2, 2, {89, 86}}, {2, 4, {145, 117}}, {4, 2, {134, 110}}, {1, 8, {230, 225}}};
   SkinnyPlan best = {0, 0, 0.0};
   for (const auto& k : kForms) {
     if (k.f == 8 && M > 16) continue;
     const int across = w_tiled ? ceil_div(N, 16 * k.f) : ceil_div(N, 128) * (8 / k.f);
-    const int groups = ceil_div(M, 16 * k.g), rounds = (int)(((int64_t)across * groups + cus - 1) / cus);
-    const double us = 1.0 + rounds * (2.3 + steps * (groups % 2 == 0 ? k.even : k.ns)[w_tiled] * 1e-3) + 1.5 * (rounds - 1);
+    const int rounds = (int)(((int64_t)across * ceil_div(M, 16 * k.g) + cus - 1) / cus);
+    const double us = 1.0 + rounds * (2.3 + steps * k.ns[w_tiled] * 1e-3) + 1.5 * (rounds - 1);
     if (best.g == 0 || us < best.us) best = {k.g, k.f, us};
   }
+  if (w_tiled && best.g >= 2 && best.f == 2 && ceil_div(M, 8 * best.g) == 2 * ceil_div(M, 16 * best.g)) best = {best.g / 2, 4, best.us};
   return best;
 }
 

@@ -345,6 +345,17 @@ def test_small_tiles_are_not_taken_where_they_were_measured_slower(abi, m, n, kn
             assert (abi.gemm_kernel(m, n, kn, ks, ko, tiled)[0] != "tile") == others
 
 
+# Tile-major weights: of two forms of the skinny kernel with as many workgroups the one with the fewer tokens, whose preference is not part
+# of the time that the kernels are compared by (the last two went to the skinny kernel with it).
+@pytest.mark.parametrize("m,n,kn,ks,ko,want", [
+    (64, 4096, 2560, 1408, 128, ("skinny", 64, 16)), (48, 4096, 2560, 1408, 128, ("skinny", 32, 32)),
+    (128, 4096, 2560, 1408, 128, ("skinny", 64, 32)), (80, 4096, 3200, 1760, 160, ("skinny", 32, 64)),
+    (51, 4189, 768, 384, 128, ("tile", 64, 64)), (50, 4143, 1280, 0, 0, ("tile", 64, 64)),
+])
+def test_forms_of_the_skinny_kernel_with_as_many_workgroups(abi, m, n, kn, ks, ko, want):
+    assert abi.gemm_kernel(m, n, kn, ks, ko, abi.weights_tileable(n, kn, ks, ko)) == want
+
+
 def test_build_refuses_kernels_that_spill():
     """Scratch memory where inline-assembly loads are in flight, and scalars spilled in the few-token kernels' loops."""
     from mixedgemm_amd import build
