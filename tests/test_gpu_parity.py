@@ -641,9 +641,9 @@ def test_tile_weights_matches_the_layout_formula(abi, n, kseg):
 
 
 # The skinny kernel's pipelines: fewer K steps than waves, than ring slots, and one more than a ring holds; a last step of
-# 1, 2 and 3 blocks per format (an E3M2 one of 24 or 72 bytes is copied shifted); every pair of token and feature group
-# counts that the plan picks, on both weight layouts, with and without a partial last step (two token groups with four
-# feature groups: the last row); the tokens of one scale atom on both sides of row 32, 64 and 128.
+# 1, 2 and 3 blocks per format (an E3M2 one of 24 or 72 bytes is copied shifted); most pairs of token and feature group
+# counts that the plan picks, on both weight layouts, with and without a partial last step (all of them by step counts in the tests
+# below); the tokens of one scale atom on both sides of row 32, 64 and 128.
 SKINNY_SHAPES = [
     (9, 256, 32, 32, 32), (16, 256, 128, 96, 0), (31, 256, 0, 32, 96), (64, 512, 3840, 288, 32), (65, 1024, 3584, 160, 96),
     (129, 2048, 1056, 608, 160), (255, 256, 4224, 2080, 352), (33, 8192, 416, 224, 64), (70, 8192, 416, 480, 160),
@@ -660,21 +660,51 @@ def test_skinny_kernel_at_the_edges_of_its_pipeline(abi, m, n, kn, ks, ko):
         test_small_batches_match_oracle(abi, m, n, kn, ks, ko, True)
 
 
-# Steps two at a time out of rings of three or four slots: 1 ... 10 steps per wave (odd and even, fewer than a ring, one more, twice as
-# many), the segments' borders at either step of a pair, with and without partial last steps; one, two and an odd number of
-# token groups, in runs of workgroups that do and do not divide by the eight XCDs.
-@pytest.mark.parametrize("per_wave", range(1, 11))
-@pytest.mark.parametrize("m,n", [(5, 1280), (24, 1536), (70, 768)])
-@pytest.mark.parametrize("rest", [(0, 0, 0), (32, 64, 96), (96, 0, 32)])
-def test_skinny_kernel_takes_steps_in_pairs(abi, per_wave, m, n, rest):
+# 1 ... 10 steps per wave (all requested up front; odd and even, as many as a ring holds, one more, twice as many), the segments' borders at
+# either step of a pair, with and without partial last steps; one, two and an odd number of token groups, in runs of workgroups that do and
+# do not divide by the eight XCDs.  These are the form with one group of tokens and of features; the test below has the others.
+def _steps_per_wave(per_wave, rest):
     steps = 4 * per_wave
     s4 = steps // 2 + (per_wave & 1)
     s6 = max(1, steps - s4 - 1 - (per_wave % 3 == 0))
     s8 = max(1, steps - s4 - s6)
-    kn, ks, ko = (128 * s - ((128 - r) if r else 0) for s, r in zip((s4, s6, s8), rest))
+    return tuple(128 * s - ((128 - r) if r else 0) for s, r in zip((s4, s6, s8), rest))
+
+
+@pytest.mark.parametrize("per_wave", range(1, 11))
+@pytest.mark.parametrize("m,n", [(5, 1280), (24, 1536), (70, 768)])
+@pytest.mark.parametrize("rest", [(0, 0, 0), (32, 64, 96), (96, 0, 32)])
+def test_skinny_kernel_takes_steps_in_pairs(abi, per_wave, m, n, rest):
+    kn, ks, ko = _steps_per_wave(per_wave, rest)
     test_small_batches_match_oracle(abi, m, n, kn, ks, ko, False)
     if abi.weights_tileable(n, kn, ks, ko):
         test_small_batches_match_oracle(abi, m, n, kn, ks, ko, True)
+
+
+# The same for each wider form, on both layouts: rings of four slots in pairs and one at a time, rings of three slots.  The weights are 640
+# distinct rows (five groups of 128, which is no divisor of a form's tiles) over and over, so that the oracle multiplies them once and all
+# repetitions must have the same bits.  Up to 16 tokens on more than 64 features per CU whole steps go to the decode kernel.
+@pytest.mark.parametrize("per_wave", range(1, 11))
+@pytest.mark.parametrize("features,tokens,m,n", [
+    (32, 16, 9, 5120), (64, 16, 12, 10240), (128, 16, 16, 17920), (32, 32, 40, 3840), (64, 32, 24, 8960), (32, 64, 70, 3840)])
+@pytest.mark.parametrize("rest", [(0, 0, 0), (32, 64, 96), (96, 0, 32)])
+def test_wide_forms_of_the_skinny_kernel(abi, per_wave, features, tokens, m, n, rest):
+    kn, ks, ko = _steps_per_wave(per_wave, rest)
+    k, base = kn + ks + ko, 640
+    _say("wide forms", m, n, kn, ks, ko)
+    x, w = H.make_activations(m, k, 51 + m + per_wave, n_out=max(1, k // 32)), H.make_weights(base, k, 53 + per_wave)
+    qx, qw = _oracle_operands(x, w, H.absmax_sort_index(x), kn, ks, ko)
+    a, b = _to_dev(qx), [t.repeat(n // base, *[1] * (t.dim() - 1)) for t in _to_dev(qw)]
+    for tiled in (False, True):
+        if tiled and not abi.weights_tileable(n, kn, ks, ko):
+            continue
+        kernel = abi.gemm_kernel(m, n, kn, ks, ko, tiled)
+        assert kernel == ("skinny", features, tokens) or (features == 128 and rest == (0, 0, 0) and kernel[0] == "decode"), kernel
+        c = list(abi.tile_weights(*b[:3])) + b[3:] if tiled else b
+        d = abi.matmul(a[0], c[0], a[1], c[1], a[2], c[2], a[3], c[3], a[4], c[4], a[5], c[5], w_tiled=tiled)
+        torch.cuda.synchronize()
+        _check_gemm(d[:, :base].contiguous(), qx, qw, f"{features} x {tokens}")
+        assert torch.equal(d, d[:, :base].repeat(1, n // base))
 
 
 # Up to 16 tokens on more than 64 features per CU.  Up to 128: the skinny kernel with eight feature groups (a ragged last group of
