@@ -112,10 +112,10 @@ __device__ __forceinline__ void wait_vmcnt() { asm volatile("s_waitcnt vmcnt(%0)
 // waits until at most `steps` (wave-uniform, at most MOST) steps of PER copies each are in flight
 template <int PER, int MOST>
 __device__ __forceinline__ void wait_steps(int steps) {
+  static_assert(MOST <= 4, "cases");
   switch (steps) {
 #define MG_STEPS_CASE(N) case N: if constexpr (N <= MOST) { wait_vmcnt<N * PER>(); break; } [[fallthrough]];
-    MG_STEPS_CASE(1) MG_STEPS_CASE(2) MG_STEPS_CASE(3) MG_STEPS_CASE(4) MG_STEPS_CASE(5) MG_STEPS_CASE(6)
-    MG_STEPS_CASE(7) MG_STEPS_CASE(8) MG_STEPS_CASE(9) MG_STEPS_CASE(10) MG_STEPS_CASE(11)
+    MG_STEPS_CASE(1) MG_STEPS_CASE(2) MG_STEPS_CASE(3) MG_STEPS_CASE(4)
 #undef MG_STEPS_CASE
     default: wait_vmcnt<0>(); break;
   }
@@ -172,6 +172,10 @@ mixed_gemm_skinny_kernel(DecodeSeg s4, DecodeSeg s6, DecodeSeg s8, int M, int N,
   // Requests of whole steps by advancing addresses, which single steps out of three slots use on row-major weights alone: on tile-major ones
   // both ways of addressing are more scalars than there are (8 and 9 were spilled; 24 calls of (1, 8) 1.0 % and 1.8 % faster without).
   constexpr bool kAdvance = NS > 3 ? kPairs : !WT;
+  // A wave's last NS - 1 steps are waited for at once, or (four and eight feature groups, whose steps are 4 and 8 KB of weights) each by
+  // itself: 200 layer calls of K < 2000, the steps each by itself over at once from HBM / from the caches, (1, 1) 1.4 % and 0.9 % slower,
+  // (1, 2) level / 0.3 % slower, (1, 4) 1.2 % faster / 0.9 % slower, (2, 4) 1.5 % faster / 0.9 % slower.
+  constexpr bool kLastAtOnce = F < 4;
   static_assert(NS >= 3 && PA + PB <= 64, "a pipeline; one copy for all scales of a step");
   extern __shared__ __align__(16) uint8_t lds[];
   // all arguments in one batch of loads (see pin_args)
@@ -360,8 +364,14 @@ mixed_gemm_skinny_kernel(DecodeSeg s4, DecodeSeg s6, DecodeSeg s8, int M, int N,
         request(ahead, to);
       }
     };
-    // Steps up to t + NS - 2 have been requested.  A wait counts the steps behind the one waited for, each with at least as
+    // Waits for steps t ... t + STEPS - 1, those up to t + NS - 1 requested: a wait counts the steps behind, each with at least as
     // many copies as this segment's (a token takes more bytes in every later segment's format).
+    auto wait_for = [&](auto steps_c) __attribute__((always_inline)) {
+      constexpr int kSteps = decltype(steps_c)::value;
+      if (t + NS - 1 < t_end) wait_vmcnt<(NS - kSteps) * PER>();
+      else if constexpr (kLastAtOnce) wait_vmcnt<0>();
+      else wait_steps<PER, NS - 1 - kSteps>(t_end - kSteps - t);
+    };
     while (t < last) {
       const uint8_t* sl = ring + slot * kSlot;
       const unsigned freed = ring0 + (unsigned)(slot == 0 ? NS - 1 : slot - 1) * kSlot;   // read a step ago
@@ -369,8 +379,7 @@ mixed_gemm_skinny_kernel(DecodeSeg s4, DecodeSeg s6, DecodeSeg s8, int M, int N,
         const int after = slot == NS - 1 ? 0 : slot + 1;
         const unsigned this_slot = ring0 + (unsigned)slot * kSlot;
         next(t + NS - 1, freed);
-        if (t + NS - 1 < t_end) wait_vmcnt<(NS - 2) * PER>();
-        else wait_steps<PER, (NS > 3 ? NS - 3 : 0)>(t_end - 2 - t);
+        wait_for(std::integral_constant<int, 2>{});
         Fragments r0, r1;
         read(fmt_c, r0, sl, 4);
         read(fmt_c, r1, ring + after * kSlot, 4);
@@ -383,8 +392,7 @@ mixed_gemm_skinny_kernel(DecodeSeg s4, DecodeSeg s6, DecodeSeg s8, int M, int N,
         t += 2;
       } else {
         next(t + NS - 1, freed);
-        if (t + NS - 1 < t_end) wait_vmcnt<(NS - 1) * PER>();
-        else wait_steps<PER, NS - 2>(t_end - 1 - t);
+        wait_for(std::integral_constant<int, 1>{});
         slot = slot == NS - 1 ? 0 : slot + 1;
         const int left = s.nblk - 4 * (t - t_first);
         Fragments r;
@@ -880,7 +888,6 @@ mixed_gemm_token_kernel(const uint8_t* __restrict__ x, const uint8_t* __restrict
                         TokenLds L, Epilogue ep, uint16_t* __restrict__ d) {
   constexpr int NS = kTokenSlots<F>, kSlot = 1024 * F;
   constexpr int PB = 4 * F, PBLOG = F == 1 ? 2 : (F == 2 ? 3 : 4);
-  static_assert(NS - 1 <= 11, "wait_steps");
   // (four feature groups: 8.45 us one at a time, 8.6 in pairs; two on row-major weights: 80 calls from HBM / from the caches 1.6 % and 1.3 %
   // faster one at a time, N = 7936, K = 2048, M = 2 5.05 -> 4.9)
   constexpr bool kPairs = F == 1 || (F == 2 && WT);
