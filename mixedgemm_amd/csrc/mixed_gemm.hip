@@ -154,7 +154,10 @@ constexpr int kSkinnySlot = 1024 * (F + 2 * G) + 16 * kSkinnyPieces<G, F>;
 template <int G, int F>
 constexpr int kSkinnySlots = 159 * 1024 / (4 * kSkinnySlot<G, F>) < 4 ? 3 : 4;
 
-template <int G, int F, bool WT>
+// ONCE: launches of at most NS - 1 steps per wave, which are all requested up front.  One step at a time and nothing requested in the loop: the
+// less code such a launch fetches, the sooner it ends (300 layer calls of K < 2000, those of 3 steps per wave, against the pipeline's form from the
+// caches / from HBM 1.8 % / 1.6 % faster, in pairs 0.8 % each; both loops in one kernel made the longer launches 5 % slower).
+template <int G, int F, bool WT, bool ONCE>
 __global__ void __launch_bounds__(256)
 mixed_gemm_skinny_kernel(DecodeSeg s4, DecodeSeg s6, DecodeSeg s8, int M, int N, int steps_per_wave, TileOrder order,
                          Epilogue ep, uint16_t* __restrict__ d) {
@@ -168,10 +171,10 @@ mixed_gemm_skinny_kernel(DecodeSeg s4, DecodeSeg s6, DecodeSeg s8, int M, int N,
   // Whole steps two at a time where the ring has four slots.  Out of three, with one step in flight, pairs are slower (N = 20480, K = 5120, M =
   // 16 18.5 against 18.0 us), and so they are with two token and four feature groups on row-major weights, where the copies of half
   // lines are what a step waits for (24 calls, from HBM / from the caches 1.5 % and 1.4 % faster one at a time; M = 20, N = 11264, K = 2496 9.1 -> 8.8).
-  constexpr bool kPairs = NS > 3 && (WT || G != 2 || F != 4);
+  constexpr bool kPairs = !ONCE && NS > 3 && (WT || G != 2 || F != 4);
   // Requests of whole steps by advancing addresses, which single steps out of three slots use on row-major weights alone: on tile-major ones
   // both ways of addressing are more scalars than there are (8 and 9 were spilled; 24 calls of (1, 8) 1.0 % and 1.8 % faster without).
-  constexpr bool kAdvance = NS > 3 ? kPairs : !WT;
+  constexpr bool kAdvance = !ONCE && (NS > 3 ? kPairs : !WT);
   // A wave's last NS - 1 steps are waited for at once, or (four and eight feature groups, whose steps are 4 and 8 KB of weights) each by
   // itself: 200 layer calls of K < 2000, the steps each by itself over at once from HBM / from the caches, (1, 1) 1.4 % and 0.9 % slower,
   // (1, 2) level / 0.3 % slower, (1, 4) 1.2 % faster / 0.9 % slower, (2, 4) 1.5 % faster / 0.9 % slower.
@@ -290,6 +293,7 @@ mixed_gemm_skinny_kernel(DecodeSeg s4, DecodeSeg s6, DecodeSeg s8, int M, int N,
   int t = t_begin, slot = 0;
 #pragma unroll
   for (int k = 0; k < NS - 1; ++k) request(t_begin + k, ring0 + k * kSlot);
+  if constexpr (ONCE && kLastAtOnce) wait_vmcnt<0>();
   // the fragments of a step in a slot
   struct Fragments { v4i w[F]; v8i x[G]; int s_w[F], s_x[G]; };
   const int frag4 = i * 64 + (g ^ ((i >> 2) & 3)) * 16;   // of 64-byte rows
@@ -351,6 +355,7 @@ mixed_gemm_skinny_kernel(DecodeSeg s4, DecodeSeg s6, DecodeSeg s8, int M, int N,
       }
     }
     auto next = [&](int ahead, unsigned to) __attribute__((always_inline)) {
+      if constexpr (ONCE) return;
       if (kAdvance && ahead < whole_end) {
         if (lane < kSkinnyPieces<G, F>) dma16_lane(sc_next, to + kScales);
 #pragma unroll
@@ -368,7 +373,8 @@ mixed_gemm_skinny_kernel(DecodeSeg s4, DecodeSeg s6, DecodeSeg s8, int M, int N,
     // many copies as this segment's (a token takes more bytes in every later segment's format).
     auto wait_for = [&](auto steps_c) __attribute__((always_inline)) {
       constexpr int kSteps = decltype(steps_c)::value;
-      if (t + NS - 1 < t_end) wait_vmcnt<(NS - kSteps) * PER>();
+      if constexpr (ONCE && kLastAtOnce) return;
+      if (!ONCE && t + NS - 1 < t_end) wait_vmcnt<(NS - kSteps) * PER>();
       else if constexpr (kLastAtOnce) wait_vmcnt<0>();
       else wait_steps<PER, NS - 1 - kSteps>(t_end - kSteps - t);
     };
@@ -415,7 +421,7 @@ mixed_gemm_skinny_kernel(DecodeSeg s4, DecodeSeg s6, DecodeSeg s8, int M, int N,
             }
           }
         }
-        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+        if constexpr (!ONCE) asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
         multiply(fmt_c, r);
         ++t;
       }
@@ -1252,7 +1258,9 @@ hipError_t launch_skinny(const DecodeSeg& d4, const DecodeSeg& d6, const DecodeS
   auto launch = [&](auto g_c, auto f_c) {
     constexpr int G = decltype(g_c)::value, F = decltype(f_c)::value;
     constexpr int kLds = 4 * kSkinnySlots<G, F> * kSkinnySlot<G, F>;
-    const auto kernel = w_tiled ? mixed_gemm_skinny_kernel<G, F, true> : mixed_gemm_skinny_kernel<G, F, false>;
+    const bool once = (total + 3) / 4 < kSkinnySlots<G, F>;
+    const auto kernel = w_tiled ? (once ? mixed_gemm_skinny_kernel<G, F, true, true> : mixed_gemm_skinny_kernel<G, F, true, false>)
+                                : (once ? mixed_gemm_skinny_kernel<G, F, false, true> : mixed_gemm_skinny_kernel<G, F, false, false>);
     if (hipError_t e = allow_dynamic_lds(reinterpret_cast<const void*>(kernel), kLds); e != hipSuccess) return e;
     hipLaunchKernelGGL(kernel, dim3(order.grid_x, grid_rows(order)), dim3(256), kLds, stream, d4, d6, d8, M, N, (total + 3) / 4, order, ep, d);
     return hipGetLastError();
