@@ -89,8 +89,9 @@ __device__ __forceinline__ void store1(uint16_t* __restrict__ d, const Epilogue&
 // which this replaces).
 // Layer call (quantizer and this kernel) from HBM, tile-major weights, us, with eight slots, one step at a time -> shorter rings 8.9, two
 // steps at a time 8.75, all arguments fetched in one batch 8.55: M = 16, N = K = 4096 9.4 -> 8.55; M = 32, N = 4096, K = 14336 19.5 -> 18.3; M =
-// 128, N = K = 4096 13.8 -> 13.1 (eight slots of the form with half the features before); 370 calls of 1 ... 255 tokens 1.03 times as
-// fast in the mean, two of them 3 % slower (row-major weights in the caches, K = 6144).
+// 128, N = K = 4096 13.8 -> 13.1 (eight slots of the form with half the features before).  With what the kernel's constants say below, 400
+// calls of 1 ... 255 tokens are 1.053 / 1.044 times as fast from the caches / from HBM as with eight slots, three and one of them slower by more than
+// 2.5 % (two runs of one side differ by 2); slowest are row-major weights with four and eight feature groups, 0.996 ... 1.009 in the mean.
 // ---------------------------------------------------------------------------
 struct DecodeSeg {
   const uint8_t* a;
@@ -777,10 +778,10 @@ mixed_gemm_decode_kernel(DecodeSeg s4, DecodeSeg s6, DecodeSeg s8, int M, int N,
 #pragma unroll
       for (int f = 0; f < F; ++f) tie(wq[B][k][f]);
   };
-  // Two rounds at a time, both requested before the first is used.  The first pair (requested above) is straight-line
-  // code, the loop requests its pairs itself: nothing is in flight across a loop edge (a register that an uncounted
-  // load is still to fill must not be moved by the compiler, which a value carried around a loop may be).
-  // step n of TOTAL, with AHEAD requested before it
+  // The first two rounds are straight-line code, a window of requested steps (above); the loop behind them requests two whole rounds itself
+  // and uses them: nothing is in flight across a loop edge (a register that an uncounted load is still to fill must not be
+  // moved by the compiler, which a value carried around a loop may be).
+  // Step n of kTotal; those up to n + kWin - 1 are requested.
   auto nth_step = [&](auto n_c, auto total_c) __attribute__((always_inline)) {
     constexpr int n = decltype(n_c)::value, kTotal = decltype(total_c)::value, kWin = kTotal > S ? kAhead : S;
     wait_vmcnt<(kWin - 1 < kTotal - 1 - n ? kWin - 1 : kTotal - 1 - n) * F>();
@@ -1220,8 +1221,10 @@ static SkinnyPlan skinny_plan(int M, int N, int steps, int cus, bool w_tiled) {
 // caches, skinny against this kernel, M = 16, K = 4096: N = 4096 8.5 against 8.1 / 8.0 against 8.5 us, 6144 9.7 against 8.9 / 8.4 against 8.8, 8192
 // 10.0 against 9.1 / 8.5 against 8.9; the four projections of a decoder layer, 116 MB in a graph, 53.6 with the rule as it is, 55.9 with this
 // kernel for up to 16 tokens on 4096 and 6144 features.)
-// So: four feature groups (two such workgroups fit a CU), or one round of workgroups and at most 8 tokens; up to 32 K steps, so
-// that all of a wave's weights are in flight at once; up to 16 where the skinny kernel has eight feature groups; above 128
+// So: four feature groups (two such workgroups fit a CU), or one round of workgroups and at most 8 tokens; up to 32 K steps, which are
+// the two rounds per wave that have a window of requests (the loop behind them starts with nothing in flight; M = 4, this kernel against
+// the skinny one from the caches / from HBM, 32 and 36 steps: N = 4096 5.0 against 4.7 / 5.05 against 5.4 and 6.2 against 4.85 / 6.2 against 5.8, N =
+// 14336 7.3 against 7.7 / 7.7 against 8.5 and 9.5 against 8.3 / 9.9 against 9.3); up to 16 where the skinny kernel has eight feature groups; above 128
 // features per CU, where that needs two rounds, always.
 // On row-major weights the skinny kernel is ahead or level up to 64 features per CU (N = 4096, K = 4096, M = 1: 5.1 against 5.6 / 5.4
 // against 5.7; N = 14336, M = 16: 8.6 against 9.3 / 11.1 against 10.7), then needs eight feature groups or a second round, where two
