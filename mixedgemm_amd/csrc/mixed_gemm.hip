@@ -155,9 +155,9 @@ constexpr int kSkinnySlot = 1024 * (F + 2 * G) + 16 * kSkinnyPieces<G, F>;
 template <int G, int F>
 constexpr int kSkinnySlots = 159 * 1024 / (4 * kSkinnySlot<G, F>) < 4 ? 3 : 4;
 
-// ONCE: launches of at most NS - 1 steps per wave, which are all requested up front.  One step at a time and nothing requested in the loop: the
-// less code such a launch fetches, the sooner it ends (300 layer calls of K < 2000, those of 3 steps per wave, against the pipeline's form from the
-// caches / from HBM 1.8 % / 1.6 % faster, in pairs 0.8 % each; both loops in one kernel made the longer launches 5 % slower).
+// ONCE: launches of at most NS - 1 steps per wave, which are all requested up front.  One step at a time and nothing requested in the loop: with
+// less code around them so few steps end sooner (172 layer calls of 3 steps per wave, K < 2000, against the pipeline's form from the caches /
+// from HBM 1.8 % / 1.6 % faster, in pairs 0.8 % each; both loops in one kernel made the longer launches 5 % slower).
 template <int G, int F, bool WT, bool ONCE>
 __global__ void __launch_bounds__(256)
 mixed_gemm_skinny_kernel(DecodeSeg s4, DecodeSeg s6, DecodeSeg s8, int M, int N, int steps_per_wave, TileOrder order,
