@@ -549,26 +549,30 @@ hipError_t launch_reorder_quant(const void* x, const int16_t* idx, int rows, int
   // in front of a workgroup's first row and was slower.
   constexpr int kNS = 2;
   constexpr int kPerCu = 4;
-  // Activations of 8192 < K <= 16384 with two lanes per block as well, i.e. 9 ... 16 waves per workgroup, where that is the faster way (us, one
-  // lane per block against two; without RMSNorm):
-  //   9 and 10 waves, one workgroup per CU: K = 9216 rows 16 3.9 against 3.55, 128 4.3 / 4.15, 256 4.2 / 4.2, 512 5.9 / 6.2, 700 8.2 / 7.8, 1024 10.5 /
-  //     9.0, 4096 25.0 / 23.5; K = 10240 256 4.2 / 4.3, 512 6.2 / 6.45, 2048 15.2 / 14.6 (three per CU: 2048 rows of 9216 15 % slower than one lane);
-  //   11 and 12 waves, two per CU: K = 12288 rows 16 3.9 / 3.7, 512 6.9 / 6.3, 1024 10.2 / 9.5, 4096 28.3 / 26.6; K = 11008 512 6.8 / 6.35, 4096 25.9 /
-  //     24.8 (one per CU: up to 5 % slower than one lane);
-  //   13 ... 16 waves, one per CU: 1 ... 256 rows 0.05 ... 0.15 faster with two (K = 12800 1.02, 14336 1.01, 16384 1.03 times as fast; medians, single runs differ by
-  //     1 %); K = 14336 512 7.6 / 7.75, 700 9.1 / 9.5, 1024 11.8 / 11.5, 2048 18.2 / 17.9, 4096 33.0 / 30.8; K = 16384 1024 13.1 / 12.05, 4096 37.3 / 34.3;
-  //     with 13 waves (K = 12800) 1024 level, 1200 0.97 times as fast, 2048 level, 4096 1.08 (two per CU: up to 15 % slower).
-  // With RMSNorm, whose form for one lane per block normalizes the row in place: K = 9216 rows 16 5.2 / 5.1, 512 11.3 / 9.1, 2048 30.3 / 24.1; K = 12288
-  // 16 5.6 / 5.3, 2048 31.7 / 24.8; K = 14336 16 5.7 / 6.0, 100 6.3 / 6.3, 256 7.3 / 7.0, 700 17.4 / 14.9, 2048 33.9 / 29.3; K = 12800 and 15360, one over two: 64
-  // rows 0.95, 128 0.96 and 0.98, 200 0.98 and 1.02, 256 1.00 and 1.02, 300 1.14 and 1.18 (up to K = 15360: the LDS offsets of its three rows are immediates).
-  // Codes kept for the GEMM that follows, gain of two lanes per layer call, us (N = 2048 and 4096; two figures of one side differ by 0.1 %): 9 and 10
-  // waves, 1 ... 128 rows 0.25 ... 0.3, 200 0.2, 384 -0.1 ... -0.6, 1024 0.1 ... 0.7, 2048 -0.5 ... -0.6, 4096 -0.7 ... -0.8; 11 and 12, up to 128 rows 0.1 ... 0.25, 512
-  // 0.4 ... 0.5, 700 0.7, 1024 0.3, 2048 0.2 ... 0.4, 4096 -0.1 ... 0.1; 13 ... 16, up to 256 rows 0.05 ... 0.25, 512 -0.3 ... -0.5, 1024 -0.1 ... 0.2, 4096 -1.1 ... -2.1.
+  // Activations of 8192 < K <= 16384 with two lanes per block as well, i.e. 9 ... 16 waves per workgroup, where that is the faster way or level with the
+  // rows in the caches, where the kernel before left them, and from HBM (us, one lane per block against two, from the caches / from HBM; two runs of one
+  // side differ by 1 %).  Without RMSNorm:
+  //   9 and 10 waves, one workgroup per CU: K = 9216 rows 16 4.35 against 4.05 / 3.95 against 3.7, 128 4.55, 4.25 / 4.35, 4.3, 256 4.4, 4.4 / 4.4, 4.45, 512
+  //     5.05, 5.4 / 6.1, 6.35, 640 7.2, 6.75 / 7.9, 7.55, 1024 8.2, 7.8 / 10.4, 8.9, 1025 8.2, 8.55 / 10.4, 9.4, 1600 9.9, 11.4 / 12.4, 12.25, 4096 22.2, 22.7 /
+  //     24.6, 23.25; K = 10240 1024 8.1, 8.1 / 10.9, 9.3, 2048 13.1, 13.9 / 15.0, 14.4 (three per CU: 2048 rows of 9216 15 % slower than one lane);
+  //   11 and 12 waves, two per CU: K = 12288 rows 16 4.35, 4.15 / 3.95, 3.85, 256 4.55, 4.35 / 4.85, 4.65, 512 5.3, 5.6 / 6.9, 6.4, 1024 7.8, 7.6 / 10.0, 9.15, 1600
+  //     11.0, 11.5 / 13.15, 12.4, 2048 13.7, 12.9 / 15.2, 14.2, 8192 45.9, 40.0 / 52.3, 49.1; K = 11008 1700 10.45, 10.7 / 12.55, 12.1, 4096 22.6, 20.8 / 25.4, 23.9;
+  //   13 ... 16 waves, one per CU: K = 14336 rows 16 4.45, 4.4 / 4.1, 4.15, 256 4.75, 4.75 / 5.2, 5.1, 320 5.5, 6.1 / 7.1, 6.95, 1024 9.1, 9.3 / 11.4, 11.3, 1600 12.8, 14.9 /
+  //     15.3, 15.6, 3500 24.3, 24.6 / 27.7, 26.4, 4096 27.1, 27.2 / 32.0, 29.8, 8192 52.0, 49.5 / 61.3, 55.3; K = 12800 4096 25.3, 26.0 / 28.85, 27.15, 6144 36.4, 36.1 / 42.55,
+  //     38.2; K = 15360 2560 20.1, 19.6 / 23.4, 22.2, K = 16384 2048 17.0, 17.35 / 20.2, 19.3, 3072 24.2, 22.9 / 27.6, 26.0 (two per CU: up to 15 % slower).
+  // With RMSNorm, whose form for one lane per block normalizes the row in place: K = 9216 rows 16 5.6, 5.5 / 5.4, 5.3, 512 9.8, 8.4 / 11.0, 8.8, 2048 28.5, 23.55 / 29.6,
+  // 23.8; K = 12288 16 6.25, 5.75 / 5.85, 5.45, 2048 30.4, 24.4 / 31.3, 24.7; K = 14336 128 6.35, 6.6 / 6.85, 6.65, 256 6.6, 6.85 / 7.3, 7.05, 257 10.3, 9.35 / 11.7, 9.5, 2048
+  // 31.9, 28.4 / 33.0, 28.7; K = 12800 4096 51.0, 50.8 / 52.1, 51.0, 8192 93.8, 96.5 / 94.6, 96.6 (up to K = 15360: the LDS offsets of its three rows are
+  // immediates).
+  // Codes kept for the GEMM that follows, gain of two lanes per layer call (N = 4096): 9 and 10 waves, 1 ... 128 rows 1 ... 5 % / 0 ... 3 %, 512 -2 % / -1 %, 2048 and
+  // 4096 -1 % / 0.5 %; 11 and 12, 1 ... 900 rows 0 ... 4 % / 0 ... 4 %, from 1300 on 0 / 1 %; 13 ... 16, up to 256 rows 0 ... 2 % / 0 ... 2 %, 512 -1 % / 0, 2048 and 4096 -2 % / -1 ... 1 %.
   auto two_lanes = [&](int t2, bool norm, bool kept) {
-    if (norm) return t2 <= 768 || (t2 <= 960 && 4 * rows >= 3 * lim.cus);
+    const int64_t r = rows, cus = lim.cus;
+    if (norm) return t2 <= 768 || (t2 <= 960 && r > cus && (t2 > 832 || r <= 16 * cus));
     if (t2 > 1024) return false;
-    if (t2 < 704) return 2 * rows <= lim.cus || (!kept && 2 * rows >= 5 * lim.cus);
-    return t2 <= 768 || rows <= lim.cus || (!kept && rows >= (t2 == 832 ? 8 : 4) * lim.cus);
+    if (t2 < 704) return 2 * r <= cus || (!kept && 2 * r >= 5 * cus && r <= 4 * cus);
+    if (t2 <= 768) return kept || r <= cus || r >= 4 * cus;
+    return r <= cus || (!kept && r >= (t2 == 832 ? 24 : t2 == 896 ? 16 : 12) * cus);
   };
   // keep: the codes stay in the L2 for the kernel that reads them next (activations only); norm: RMSNorm of the row
   // before the gather (activations only; its codes are always kept: what follows a norm is the layer's GEMM)

@@ -76,8 +76,8 @@ def _check_kept_codes(abi, rows, k):
 
 
 # Activations of 8192 < K <= 16384: every workgroup size with two lanes per block, the smallest K of each and the largest, row counts on both
-# sides of where one lane per block takes over (of 128, 192, 256, 640 and 1024), with RMSNorm (up to K = 15360), and with the codes kept for the
-# GEMM of a layer call.
+# sides of where one lane per block takes over (of 128, 256, 640 and 1024; the lines further up: the test of many rows), with RMSNorm (up to K =
+# 15360), and with the codes kept for the GEMM of a layer call.
 @pytest.mark.parametrize("k", [8224, 9248, 10272, 11296, 12320, 13344, 14368, 15360, 15392, 16384])
 @pytest.mark.parametrize("rows", [3, 129, 257, 641, 1025])
 def test_wide_rows_with_two_lanes_per_block(abi, k, rows):
@@ -91,17 +91,43 @@ def test_wide_rows_with_two_lanes_per_block(abi, k, rows):
 
 
 # The same instances with more rows than both slots of every workgroup hold, so that slots are filled again and the RMSNorm's sums change
-# places: one workgroup per CU has three or four of 900 rows and eight or nine of 2100 (where 13 waves take over again), two per CU, with 11 and
-# 12 waves and no RMSNorm, two or three of 1100.
+# places: one workgroup per CU has three or four of 900 rows (9 and 10 waves: of 1000 without RMSNorm), two per CU, with 11 and 12 waves and no
+# RMSNorm, two or three of 1100.
 @pytest.mark.parametrize("k", [8224, 9248, 10272, 11296, 12288, 12320, 13344, 14368, 15360])
 def test_wide_rows_refill_their_slots_with_rmsnorm(abi, k):
     test_rmsnorm_reorder_quantize_matches_oracle(abi, 900, *_wide_split(k), 1e-5)
 
 
-@pytest.mark.parametrize("rows,k", [(1100, 10272), (1100, 11296), (1100, 12288), (2100, 12320)])
+@pytest.mark.parametrize("rows,k", [(1000, 8224), (1000, 9248), (1100, 10272), (1100, 11296), (1100, 12288), (2100, 12320)])
 def test_wide_rows_refill_their_slots(abi, rows, k):
     test_reorder_quantize_matches_oracle(abi, "x", rows, *_wide_split(k))
     _check_kept_codes(abi, rows, k)
+
+
+# Many wide rows, on both sides of the lines from which 13 ... 16 waves take two lanes per block again (6144, 4096, 3072 rows) and up to which 13 do
+# with RMSNorm (4096): the same codes and scales as 512 rows at a time, which take one lane per block (with RMSNorm 256 at a time).
+@pytest.mark.parametrize("k,rows,norm", [
+    (12320, 6143, False), (12320, 6150, False), (13312, 6144, False), (13344, 4095, False), (14336, 4100, False), (14368, 3071, False),
+    (15360, 3080, False), (15392, 3072, False), (16384, 3100, False), (12320, 4096, True), (13312, 4100, True)])
+def test_many_wide_rows_match_a_few_at_a_time(abi, k, rows, norm):
+    split = _wide_split(k)
+    _say("many wide rows", rows, *split)
+    g = torch.Generator().manual_seed(rows + k)
+    few = torch.randn(700, k, generator=g).to(torch.bfloat16)
+    few[:, ::97] *= 30
+    x = few.to(DEV)[torch.randint(700, (rows,), generator=g).to(DEV)]
+    idx = H.random_index(k, 3).to(DEV)
+    gamma = (1 + 0.1 * torch.randn(k, generator=g)).to(torch.bfloat16).to(DEV) if norm else None
+    quantize = (lambda v: abi.rmsnorm_reorder_quantize_x(v, gamma, 1e-5, idx, *split)) if norm else (lambda v: abi.reorder_quantize_x(v, idx, *split))
+    got, step = quantize(x), 256 if norm else 512
+    for r in range(0, rows, step):
+        part = quantize(x[r:r + step])
+        n = min(step, rows - r)
+        for a, b in zip(got[:3], part[:3]):
+            assert torch.equal(a[r:r + n], b)
+        for a, b, kseg in zip(got[3:], part[3:], split):
+            a, b = (t.cpu().numpy() for t in (a[abi.sf_offset(r, 0, kseg):], b))
+            np.testing.assert_array_equal(mo.sf_gather(a, n, kseg), mo.sf_gather(b, n, kseg))
 
 
 def _adversarial(k):
