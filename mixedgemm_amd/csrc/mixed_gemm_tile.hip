@@ -17,6 +17,7 @@
 //   M = 512, N = 4096, K = 4096: 16.6 / 19.6 -> 10.0 / 12.0;  N = 1024, K = 8192: 27.6 / 34.8 -> 11.6 / 13.2
 //   M = 64, N = 14336, K = 4096: 16.4 / 16.8 -> 8.8 / 9.3;   M = 128: 16.8 / 20.1 -> 10.1 / 12.3
 //   M = 1024, N = 4096, K = 4096: 17.0 / 19.7 -> 14.5 / 16.5
+// and, with batches copied as rows of their stages (BatchRow): K = 14336, M = 256 17.5 / 18.7;  M = 1024, K = 4096 12.6 / 13.1
 // (from HBM: M = 256 10.6 / 10.8 and 30 / 30, M = 512 12.5 / 15.2 and 16.1 / 16.0, M = 64 13.7 / 14.1, M = 1024 17.6 / 19.2)
 // Tiles of 256 x 128 with the same division of work were level with the mixed waves of the 256 x 256 kernel (M = 2048, N =
 // 4096, K = 12288: 57.6 against 56.3 us: 15 % fewer cycles at a clock as much lower; the chip is at its power limit there), tiles of
@@ -91,17 +92,16 @@ __device__ __forceinline__ void drain() {
 __device__ __forceinline__ void wait_lds() { __builtin_amdgcn_s_waitcnt(0xC07F); }
 
 // Geometry of an instance.  TF x TT: the workgroup's tile; WT: tile-major weights; a batch of WS stages per barrier, each the
-// work of 8 / WS math waves (WF along the features).
-template <int TF_, int TT_, int WF_, int WS_, bool WT_>
+// work of 8 / WS math waves (WF along the features); ROWS: batches of one segment lie as rows of WS stages (BatchRow).
+template <int TF_, int TT_, int WF_, int WS_, bool WT_, bool ROWS_>
 struct Geo {
   static constexpr int TF = TF_, TT = TT_, WF = WF_, WS = WS_;
-  static constexpr bool WT = WT_;
+  static constexpr bool WT = WT_, ROWS = ROWS_;
   static constexpr int WM = kMathWaves / WF / WS;                          // math waves along tokens
   static constexpr int TN = TF / 32 / WF, TM = TT / 32 / WM;               // a wave's 32 x 32 tiles
-  // a stage in LDS: 1 KB of scales (32 pieces of the features, 32 of the tokens), weights, tokens
-  static constexpr int kW = 1024, kX = kW + TF * 64;
-  static constexpr int kSlot = kX + TT * 128;
-  static constexpr int kBatch = WS * kSlot;
+  // a batch in LDS: per stage 1 KB of scales (32 pieces of the features, 32 of the tokens), then the weights, then the tokens
+  static constexpr int kW = WS * 1024, kX = kW + WS * TF * 64;
+  static constexpr int kBatch = kX + WS * TT * 128;
   static constexpr int NB = kRingBytes / kBatch < 8 ? kRingBytes / kBatch : 8;   // batches in the ring
   // the partial sums on their way out: per stage of a batch, fp32 rows of tokens
   static constexpr int kPitch = TF * 4 + 16, kPart = TT * kPitch;
@@ -115,11 +115,16 @@ struct TileCtx {
 };
 
 // ---------------------------------------------------------------------------------------------
-// Copies of one whole stage, dealt to the four copy waves.  Weights and E2M1 tokens: 16 rows x 64 B per copy, the 16-byte
-// pieces of row r permuted by XOR with r / 4, E4M3: 8 rows x 128 B, permuted by XOR with r / 2, E3M2: rows of 96 B one after the other,
+// Copies, dealt to the four copy waves.  A cache line is 128 bytes, a stage of a row of E2M1 codes 64, of E3M2 96: a batch whose stages are
+// all of one segment is copied (and lies in LDS) as rows of WS stages, so that its lines are asked for once, in one piece (BatchRow).
+// Stage by stage, every row's every line was fetched by two copies a batch or more apart: GEMM alone, tile-major / row-major weights,
+// all E2M1, us: M = 256, N = 4096, K = 14336 17.2 -> 15.2 / - ; M = 512, N = 4096, K = 4096 8.9 -> 8.6 / 10.2 -> 8.7; M = 1024 11.9 -> 11.0 /
+// 13.5 -> 11.1; M = 244, N = 12416, K = 13824, default plan - / 64.8 -> 48.3.  Short launches do not gain (batch_rows).
+// A batch of two segments, and a last, partial one, go stage by stage: weights and E2M1 tokens 16 rows x 64 B per copy, the 16-byte
+// pieces of row r permuted by XOR with r / 4, E3M2: rows of 96 B one after the other,
 // their pieces rotated by one in rows 8 ... 15 of every 16: the 16 rows that a fragment read touches at a time lie on different
-// banks (E3M2 rows as they are: 0.85 instead of 0.36 us per stage of 128 x 128).  Scales: the two atoms of 128 rows that hold the
-// tile's rows, one copy.
+// banks (E3M2 rows as they are: 0.85 instead of 0.36 us per stage of 128 x 128).  E4M3 always goes stage by stage, a line per row: 8 rows x
+// 128 B, permuted by XOR with r / 2.  Scales: the two atoms of 128 rows that hold the tile's rows, one copy per stage.
 // Tile-major weights (16 KB per 256 features and stage: 1 KB per j = feature % 16, in it 64 bytes per feature / 16, even ones
 // first): a copy takes what the tile's features have of 128 / TF blocks of 1 KB, whole lines, and row i of a 32-row fragment is the
 // feature that WeightRows says.  (A workgroup has consecutive features: with whole 1 KB blocks, i.e. every other run of eight, two
@@ -163,50 +168,81 @@ struct WeightRows {
   }
 };
 
+// n / P for a piece's number n < 2^15
+template <int P>
+__device__ __forceinline__ int row_of(int n) {
+  static_assert(P == 8 || P == 16 || P == 6 || P == 12 || P == 24, "pieces per row");
+  if constexpr ((P & (P - 1)) == 0) return n / P;
+  else return (int)(__umul24((unsigned)n, 43691u) >> (P == 6 ? 18 : P == 12 ? 19 : 20));   // 43691 * 6 = 2^18 + 2
+}
+
+// Rows of a batch of one segment in LDS: BYTES per stage, WS stages, in 16-byte pieces; which piece lies where in its row depends on the
+// row such that the 16 rows read at a time (see WeightRows) are on 16 different sixteenths of the 256 bytes of all banks: a power of two
+// of pieces is permuted by XOR, 12 and 24 (E3M2) are rotated by as many steps as rows 12 and 24 pieces apart leave between them.
+template <int BYTES, class G>
+struct BatchRow {
+  static constexpr int P = G::WS * BYTES / 16, bytes = 16 * P;
+  static_assert(P == 8 || P == 12 || P == 16 || P == 24, "pieces per row");
+  static __device__ __forceinline__ int key(int row) { return P == 16 ? row & 15 : P == 12 ? (row >> 2) & 3 : (row >> 1) & 7; }
+  static __device__ __forceinline__ int place(int piece, int row) {   // of a piece in the row
+    if constexpr ((P & (P - 1)) == 0) return piece ^ key(row);
+    const int at = piece + key(row);
+    return at >= P ? at - P : at;
+  }
+  static __device__ __forceinline__ int piece(int at, int row) {      // that lies there
+    if constexpr ((P & (P - 1)) == 0) return at ^ key(row);
+    const int p = at - key(row);
+    return p < 0 ? p + P : p;
+  }
+};
+
 template <int FMT, class G>
-constexpr int kTokenCopiesAll = G::TT * Form<FMT>::row / 1024;
+constexpr int kTokenCopiesAll = G::TT * Form<FMT>::row / 1024;   // per stage
 // copies that every copy wave issues per whole batch, at least (a stage of a later segment has as many or more)
 template <class G>
 constexpr int kBatchCopies = G::WS * (G::TF / 64) + G::WS * kTokenCopiesAll<kFmtE2M1, G> / kCopyWaves + G::WS / kCopyWaves;
 
 template <int FMT, class G>
-struct StageCopy {
+struct SegCopy {
+  static constexpr bool kRows = G::ROWS && FMT != kFmtE4M3;   // whole batches as rows of WS stages
   static constexpr int NW = G::TF / 64, NX = kTokenCopiesAll<FMT, G>, KX = (NX + kCopyWaves - 1) / kCopyWaves;
+  static constexpr int BW = G::WS * NW, BX = G::WS * NX / kCopyWaves;   // of a whole batch
+  static_assert(G::WS * NX % kCopyWaves == 0, "a batch's token copies are dealt evenly");
+  typedef BatchRow<64, G> WRow;
+  typedef BatchRow<kRows ? Form<FMT>::row : 64, G> XRow;
   const uint8_t *w, *x;         // bases of the next stage
   const uint8_t* sc;            // this lane's scale piece
-  unsigned vw[NW], vx[KX];
+  unsigned vw[NW], vx[KX], bw[BW], bx[BX];
   int wave;
 
-  // token copies come in fours, a last pair is dealt to waves 0, 1 and 2, 3 in turn
+  // token copies of a stage come in fours, a last pair is dealt to waves 0, 1 and 2, 3 in turn
   static_assert(NX % 2 == 0, "token copies in pairs");
   __device__ __forceinline__ int block(int k) const { return (k + 1) * kCopyWaves <= NX ? wave + kCopyWaves * k : (wave & 1) + kCopyWaves * k; }
 
+  // the bases, and what batches copied as rows need
   __device__ __forceinline__ void init(const TileCtx<G>& c, const TileSeg& s, int wave_) {
     wave = wave_;
-    const int r = c.lane >> 2, p = (c.lane & 3) ^ ((c.lane >> 4) & 3);
+    const unsigned pitch = (unsigned)s.blk * (Form<FMT>::row / 4);
+    x = s.a + (size_t)c.m0 * pitch;
     if constexpr (G::WT) {
       w = s.b + (size_t)(c.n0 >> 8) * s.whole * 16384;
 #pragma unroll
       for (int k = 0; k < NW; ++k) vw[k] = WeightRows<G>::tiled_offset(wave + kCopyWaves * k, c.lane, c.n0);
     } else {
       w = s.b + (size_t)c.n0 * s.blk * 16;
+      if constexpr (kRows) {
 #pragma unroll
-      for (int k = 0; k < NW; ++k) vw[k] = (unsigned)min(16 * (wave + kCopyWaves * k) + r, c.last_col) * (unsigned)s.blk * 16u + p * 16;
+        for (int k = 0; k < BW; ++k) {
+          const int chunk = 64 * (wave + kCopyWaves * k) + c.lane, row = row_of<WRow::P>(chunk);
+          bw[k] = __umul24(min(row, c.last_col), 16 * s.blk) + WRow::piece(chunk - row * WRow::P, row) * 16;
+        }
+      }
     }
-    const unsigned pitch = (unsigned)s.blk * (Form<FMT>::row / 4);
-    x = s.a + (size_t)c.m0 * pitch;
+    if constexpr (kRows) {
 #pragma unroll
-    for (int k = 0; k < KX; ++k) {
-      const int b = block(k);
-      if constexpr (FMT == kFmtE2M1) {
-        vx[k] = (unsigned)min(16 * b + r, c.last_row) * pitch + p * 16;
-      } else if constexpr (FMT == kFmtE3M2) {   // the pieces of rows 8 ... 15 of every 16 rotated by one
-        const int chunk = 64 * b + c.lane, row = chunk / 6, at = chunk % 6;
-        const int piece = (row & 8) ? (at == 0 ? 5 : at - 1) : at;
-        vx[k] = (unsigned)min(row, c.last_row) * pitch + piece * 16;
-      } else {
-        const int row = 8 * b + (c.lane >> 3);
-        vx[k] = (unsigned)min(row, c.last_row) * pitch + (((c.lane & 7) ^ ((row >> 1) & 7)) * 16);
+      for (int k = 0; k < BX; ++k) {
+        const int chunk = 64 * (wave + kCopyWaves * k) + c.lane, row = row_of<XRow::P>(chunk);
+        bx[k] = __umul24(min(row, c.last_row), pitch) + XRow::piece(chunk - row * XRow::P, row) * 16;
       }
     }
     const int katoms = (s.blk + 3) >> 2;
@@ -214,19 +250,69 @@ struct StageCopy {
     const uint8_t* const of_rows = s.sfa + (size_t)(c.m0 >> 7) * katoms * 512;
     sc = c.lane < 32 ? of_features + WeightRows<G>::scale_piece(c.lane) * 16 : of_rows + (c.lane & 31) * 16;
   }
-
-  // the next stage, t-th of all, into a slot.  What does not divide by the copy waves goes to other ones in every stage.
-  __device__ __forceinline__ void issue(int t, unsigned slot) {
+  // what single stages need
+  __device__ __forceinline__ void init_stages(const TileCtx<G>& c, const TileSeg& s) {
+    const int r = c.lane >> 2, p = (c.lane & 3) ^ ((c.lane >> 4) & 3);
+    if constexpr (!G::WT) {
 #pragma unroll
-    for (int k = 0; k < NW; ++k) copy_at(w, vw[k], slot + G::kW + 1024u * (wave + kCopyWaves * k));
+      for (int k = 0; k < NW; ++k) vw[k] = __umul24(min(16 * (wave + kCopyWaves * k) + r, c.last_col), 16 * s.blk) + p * 16;
+    }
+    const unsigned pitch = (unsigned)s.blk * (Form<FMT>::row / 4);
+#pragma unroll
+    for (int k = 0; k < KX; ++k) {
+      const int b = block(k);
+      if constexpr (FMT == kFmtE2M1) {
+        vx[k] = __umul24(min(16 * b + r, c.last_row), pitch) + p * 16;
+      } else if constexpr (FMT == kFmtE3M2) {   // the pieces of rows 8 ... 15 of every 16 rotated by one
+        const int chunk = 64 * b + c.lane, row = row_of<6>(chunk), at = chunk - row * 6;
+        const int piece = (row & 8) ? (at == 0 ? 5 : at - 1) : at;
+        vx[k] = __umul24(min(row, c.last_row), pitch) + piece * 16;
+      } else {
+        const int row = 8 * b + (c.lane >> 3);
+        vx[k] = __umul24(min(row, c.last_row), pitch) + (((c.lane & 7) ^ ((row >> 1) & 7)) * 16);
+      }
+    }
+  }
+
+  // What does not divide by the copy waves goes to other ones in every stage (t: of all stages).
+  __device__ __forceinline__ void scales(int t, unsigned at) {
+    const int turn = 2 * (~t & 1) + ((t >> 1) & 1);   // every wave once in four stages
+    if (turn == wave) copy_lane(sc, at);
+    sc += 512;
+  }
+  // the next stage, t-th of all, as stage u of a batch
+  __device__ __forceinline__ void issue(int t, int u, unsigned batch) {
+#pragma unroll
+    for (int k = 0; k < NW; ++k) copy_at(w, vw[k], batch + G::kW + G::TF * 64u * u + 1024u * (wave + kCopyWaves * k));
 #pragma unroll
     for (int k = 0; k < KX; ++k)
-      if ((k + 1) * kCopyWaves <= NX || (wave >> 1) == (t & 1)) copy_at(x, vx[k], slot + G::kX + 1024u * block(k));
-    const int turn = 2 * (~t & 1) + ((t >> 1) & 1);   // every wave once in four stages
-    if (turn == wave) copy_lane(sc, slot);
+      if ((k + 1) * kCopyWaves <= NX || (wave >> 1) == (t & 1)) copy_at(x, vx[k], batch + G::kX + G::TT * 128u * u + 1024u * block(k));
+    scales(t, batch + 1024u * u);
     w += G::WT ? 16384 : 64;
     x += Form<FMT>::row;
-    sc += 512;
+  }
+  // the next WS stages
+  __device__ __forceinline__ void issue_batch(int t, unsigned batch) {
+    if constexpr (!kRows) {
+#pragma unroll
+      for (int u = 0; u < G::WS; ++u) issue(t + u, u, batch);
+    } else {
+      if constexpr (G::WT) {
+#pragma unroll
+        for (int u = 0; u < G::WS; ++u)
+#pragma unroll
+          for (int k = 0; k < NW; ++k) copy_at(w + u * 16384, vw[k], batch + G::kW + G::TF * 64u * u + 1024u * (wave + kCopyWaves * k));
+      } else {
+#pragma unroll
+        for (int k = 0; k < BW; ++k) copy_at(w, bw[k], batch + G::kW + 1024u * (wave + kCopyWaves * k));
+      }
+#pragma unroll
+      for (int k = 0; k < BX; ++k) copy_at(x, bx[k], batch + G::kX + 1024u * (wave + kCopyWaves * k));
+#pragma unroll
+      for (int u = 0; u < G::WS; ++u) scales(t + u, batch + 1024u * u);
+      w += G::WS * (G::WT ? 16384 : 64);
+      x += G::WS * Form<FMT>::row;
+    }
   }
 };
 
@@ -239,35 +325,71 @@ struct TileFrags {
   typename Form<FMT>::frag x[G::TM];
 };
 
-template <class G>
-struct ReadAt {   // per-lane LDS offsets inside a slot
-  int w, x4, x6, x8, sw, sx;
-  int xor4, xor8, xorw;
-  int p6a, p6b, h6a, h6b;   // E3M2: the lane's whole and half piece of K half 0, 1
+// Per-lane offsets inside a batch of what a wave reads of its stage; [..][H]: of K half H.  Rows of WS stages (ROWS) or of one.
+struct ReadAt {
+  int w[2], x[2], h[2];   // 16-byte pieces of weights and tokens, 8-byte ones of E3M2 tokens (E4M3: x[H] and, 32 bytes off under XOR, h[H])
 };
+template <int FMT, bool ROWS, class G>
+__device__ __forceinline__ ReadAt read_at(int i, int g, int wf, int wm, int ws) {
+  ReadAt at;
+  const int T0 = wf * G::TN, row0 = wm * G::TM * 32;
+#pragma unroll
+  for (int H = 0; H < 2; ++H) {
+    if constexpr (ROWS && !G::WT) {
+      typedef BatchRow<64, G> Row;
+      at.w[H] = G::kW + (T0 * 32 + i) * Row::bytes + Row::place(4 * ws + 2 * H + g, i) * 16;
+    } else {
+      at.w[H] = G::kW + ws * G::TF * 64 + WeightRows<G>::lds(T0, i) + (((2 * H + g) ^ (G::WT ? i & 3 : (i >> 2) & 3)) * 16);
+    }
+    if constexpr (ROWS) {
+      typedef BatchRow<Form<FMT>::row, G> Row;
+      const int x = G::kX + (row0 + i) * Row::bytes;
+      if constexpr (FMT == kFmtE2M1) {
+        at.x[H] = x + Row::place(4 * ws + 2 * H + g, i) * 16;
+        at.h[H] = 0;
+      } else {   // block 2H is piece 3H and the first half of piece 3H + 1, block 2H + 1 the other half and piece 3H + 2
+        at.x[H] = x + Row::place(6 * ws + 3 * H + 2 * g, i) * 16;
+        at.h[H] = x + Row::place(6 * ws + 3 * H + 1, i) * 16 + 8 * g;
+      }
+    } else {
+      const int x = G::kX + ws * G::TT * 128 + (row0 + i) * Form<FMT>::row;
+      if constexpr (FMT == kFmtE2M1) {
+        at.x[H] = x + (((2 * H + g) ^ ((i >> 2) & 3)) * 16);
+        at.h[H] = 0;
+      } else if constexpr (FMT == kFmtE3M2) {
+        const int turn = (i >> 3) & 1;
+        auto piece = [&](int p) { return (p + turn == 6 ? 0 : p + turn) * 16; };
+        at.x[H] = x + piece(3 * H + 2 * g);
+        at.h[H] = x + piece(3 * H + 1) + 8 * g;
+      } else {   // K [16g, 16g+16) and [32+16g, ...) of the half
+        at.x[H] = x + (((4 * H + g) ^ ((i >> 1) & 7)) * 16);
+        at.h[H] = x + (((4 * H + 2 + g) ^ ((i >> 1) & 7)) * 16);
+      }
+    }
+  }
+  return at;
+}
 
 __device__ __forceinline__ v8i widened(v4i v) { return __builtin_shufflevector(v, v, 0, 1, 2, 3, -1, -1, -1, -1); }
 __device__ __forceinline__ v8i widened(v6i v) { return __builtin_shufflevector(v, v, 0, 1, 2, 3, 4, 5, -1, -1); }
 __device__ __forceinline__ v8i widened(v8i v) { return v; }
 
-template <int FMT, int H, class G>
-__device__ __forceinline__ void read_half(TileFrags<FMT, G>& f, const uint8_t* slot, const ReadAt<G>& r, int g) {
-  const int piece = ((2 * H + g) ^ r.xor4) * 16, wpiece = ((2 * H + g) ^ r.xorw) * 16;
+template <int FMT, int H, bool ROWS, class G>
+__device__ __forceinline__ void read_half(TileFrags<FMT, G>& f, const uint8_t* batch, const ReadAt& r, int g) {
+  constexpr int kWTile = ROWS && !G::WT ? 32 * BatchRow<64, G>::bytes : 2048;
+  constexpr int kXTile = 32 * Form<FMT>::row * (ROWS ? G::WS : 1);
 #pragma unroll
-  for (int t = 0; t < G::TN; ++t) f.w[t] = *reinterpret_cast<const v4i*>(slot + r.w + t * 2048 + wpiece);
+  for (int t = 0; t < G::TN; ++t) f.w[t] = *reinterpret_cast<const v4i*>(batch + r.w[H] + t * kWTile);
 #pragma unroll
   for (int t = 0; t < G::TM; ++t) {
+    const v4i a = *reinterpret_cast<const v4i*>(batch + r.x[H] + t * kXTile);
     if constexpr (FMT == kFmtE2M1) {
-      f.x[t] = *reinterpret_cast<const v4i*>(slot + r.x4 + t * 2048 + piece);
+      f.x[t] = a;
     } else if constexpr (FMT == kFmtE3M2) {
-      // block 2H is piece 3H and the first half of piece 3H + 1, block 2H + 1 the other half and piece 3H + 2
-      const uint8_t* row = slot + r.x6 + t * 3072;
-      const v4i a = *reinterpret_cast<const v4i*>(row + (H ? r.p6b : r.p6a));
-      const v2i b = *reinterpret_cast<const v2i*>(row + (H ? r.h6b : r.h6a));
+      const v2i b = *reinterpret_cast<const v2i*>(batch + r.h[H] + t * kXTile);
       f.x[t] = g ? v6i{b[0], b[1], a[0], a[1], a[2], a[3]} : v6i{a[0], a[1], a[2], a[3], b[0], b[1]};
-    } else {   // K [16g, 16g+16) and [32+16g, ...) of the half
-      const v4i a = *reinterpret_cast<const v4i*>(slot + r.x8 + t * 4096 + ((4 * H + g) ^ r.xor8) * 16);
-      const v4i b = *reinterpret_cast<const v4i*>(slot + r.x8 + t * 4096 + ((4 * H + 2 + g) ^ r.xor8) * 16);
+    } else {
+      const v4i b = *reinterpret_cast<const v4i*>(batch + r.h[H] + t * kXTile);
       f.x[t] = __builtin_shufflevector(a, b, 0, 1, 2, 3, 4, 5, 6, 7);
     }
   }
@@ -284,9 +406,9 @@ struct RawScales {
   int w, x;
 };
 template <class G>
-__device__ __forceinline__ void read_scales(RawScales<G>& s, const uint8_t* slot, const ReadAt<G>& r) {
-  s.w = *reinterpret_cast<const int*>(slot + r.sw);
-  s.x = *reinterpret_cast<const int*>(slot + r.sx);
+__device__ __forceinline__ void read_scales(RawScales<G>& s, const uint8_t* batch, int sw, int sx) {
+  s.w = *reinterpret_cast<const int*>(batch + sw);
+  s.x = *reinterpret_cast<const int*>(batch + sx);
 }
 __device__ __forceinline__ void both_halves(int v, int& lower, int& upper) {
   const auto p = __builtin_amdgcn_permlane32_swap((unsigned)v, (unsigned)v, false, false);
@@ -402,10 +524,10 @@ __device__ __forceinline__ void pin_plan(const TilePlan& p, const Epilogue& ep, 
                "s"(p.order.div2), "s"(p.order.magic), "s"(p.order.grid_x), "s"(p.order.tiles), "s"(ep.bias), "s"(ep.n_out), "s"(d));
 }
 
-template <int TF, int TT, int WF, int WS, bool WT, bool REM>
+template <int TF, int TT, int WF, int WS, bool WT, bool REM, bool ROWS>
 __global__ void __launch_bounds__(64 * kTileWaves)
 mixed_gemm_tile_kernel(TilePlan plan, Epilogue ep, uint16_t* __restrict__ d) {
-  typedef Geo<TF, TT, WF, WS, WT> G;
+  typedef Geo<TF, TT, WF, WS, WT, ROWS> G;
   constexpr int NB = G::NB;
   extern __shared__ __align__(16) uint8_t lds[];
   const unsigned lds0 = (unsigned)(size_t)(__attribute__((address_space(3))) uint8_t*)lds;
@@ -425,83 +547,102 @@ mixed_gemm_tile_kernel(TilePlan plan, Epilogue ep, uint16_t* __restrict__ d) {
 
   if (wave < kCopyWaves) {
     // ------------------------------------------------------------------ copy waves
-    StageCopy<kFmtE2M1, G> k4;
-    StageCopy<kFmtE3M2, G> k6;
-    StageCopy<kFmtE4M3, G> k8;
-    unsigned slot = lds0;
+    SegCopy<kFmtE2M1, G> k4;
+    SegCopy<kFmtE3M2, G> k6;
+    SegCopy<kFmtE4M3, G> k8;
+    unsigned batch = lds0;
     const unsigned ring_end = lds0 + NB * G::kBatch;
     auto advance = [&]() __attribute__((always_inline)) {
-      slot += G::kSlot;
-      slot = slot == ring_end ? lds0 : slot;
+      batch += G::kBatch;
+      batch = batch == ring_end ? lds0 : batch;
     };
     // The first NB batches at once, then one more behind each barrier.  Before the barrier that hands over a batch, all but
     // the copies of the NB - 2 younger ones have landed (kBatchCopies each at least; a last, partial one is counted as none).
     constexpr int LB = kBatchCopies<G>;
-    auto stages = [&](auto& k, int& t, int last) __attribute__((always_inline)) {
-      for (; t < last; ++t) {
-        k.issue(t, slot);
+    // whole batches of one segment that end by stage `last`
+    auto whole = [&](auto& k, int& t, int last) __attribute__((always_inline)) {
+      for (; t + WS <= last; t += WS) {
+        k.issue_batch(t, batch);
         advance();
       }
     };
-    // whole batches of one segment
+    // the same behind a barrier each
     auto stream = [&](auto& k, int& t, int last) __attribute__((always_inline)) {
       for (; t + WS <= last; t += WS) {
         wait_vm<(NB - 2) * LB>();
         workgroup_barrier();
-#pragma unroll
-        for (int u = 0; u < WS; ++u) {
-          k.issue(t + u, slot);
-          advance();
-        }
+        k.issue_batch(t, batch);
+        advance();
       }
     };
-    // a run of stages whatever their segments
-    auto mixed = [&](int& t, int last) __attribute__((always_inline)) {
-      stages(k4, t, min(last, t6));
-      stages(k6, t, min(last, t8));
-      stages(k8, t, last);
+    // stages up to `last`, whatever their segments, one by one: whole batches but for the last one of all
+    auto one_by_one = [&](int& t, int last) __attribute__((always_inline)) {
+      auto stages = [&](auto& k, int end) __attribute__((always_inline)) {
+        for (; t < end; ++t) {
+          k.issue(t, t % WS, batch);
+          if (t % WS == WS - 1) advance();
+        }
+      };
+      stages(k4, min(last, t6));
+      stages(k6, min(last, t8));
+      stages(k8, last);
+    };
+    // batches up to stage `last` (a whole number of them, or all), whatever their segments
+    auto fill = [&](int& t, int last) __attribute__((always_inline)) {
+      if constexpr (!ROWS) {
+        one_by_one(t, last);
+      } else {
+        whole(k4, t, min(last, t6));
+        if (t < t6 && t < last) one_by_one(t, min(last, t + WS));
+        whole(k6, t, min(last, t8));
+        if (t < t8 && t < last) one_by_one(t, min(last, t + WS));
+        whole(k8, t, last);
+        if (t < last) one_by_one(t, last);
+      }
     };
     int t = 0;
     constexpr int kFirst = NB * WS;
-    k4.init(c, plan.s4, wave);
-    const bool short4 = t6 < kFirst;
-    if (short4) {
+    auto init_rest = [&]() __attribute__((always_inline)) {
+      if (ROWS && t6 % WS) k4.init_stages(c, plan.s4);
       k6.init(c, plan.s6, wave);
+      if (!ROWS || t6 % WS || t8 % WS) k6.init_stages(c, plan.s6);
       k8.init(c, plan.s8, wave);
-    }
-    if (total >= kFirst) {
+      k8.init_stages(c, plan.s8);
+    };
+    k4.init(c, plan.s4, wave);
+    if constexpr (!ROWS) k4.init_stages(c, plan.s4);
+    const bool short4 = t6 < kFirst;
+    if (short4) init_rest();
+    if (ROWS || total >= kFirst) {   // (batch_rows)
       // two batches, then the multiplying starts on the first of them, then the rest of the ring
-      mixed(t, 2 * WS);
+      fill(t, 2 * WS);
       wait_vm<LB>();
       workgroup_barrier();   // batch 0 has landed
-      mixed(t, kFirst);
-      if (!short4) {
-        k6.init(c, plan.s6, wave);
-        k8.init(c, plan.s8, wave);
-      }
+      fill(t, kFirst);
+      if (!short4) init_rest();
       stream(k4, t, t6);
       if (t < t6 && t + WS <= total) {   // a batch of two or three segments
         wait_vm<(NB - 2) * LB>();
         workgroup_barrier();
-        mixed(t, t + WS);
+        one_by_one(t, t + WS);
       }
       stream(k6, t, t8);
       if (t < t8 && t + WS <= total) {
         wait_vm<(NB - 2) * LB>();
         workgroup_barrier();
-        mixed(t, t + WS);
+        one_by_one(t, t + WS);
       }
       stream(k8, t, total);
       if (t < total) {   // the last, partial batch
         wait_vm<(NB - 2) * LB>();
         workgroup_barrier();
-        mixed(t, total);
+        one_by_one(t, total);
         drain<NB - 2, LB, 1>();
       } else {
         drain<NB - 2, LB, 0>();
       }
     } else {   // all of them at once
-      mixed(t, total);
+      fill(t, total);
       wait_vm<0>();
       for (int q = 0; q <= batches; ++q) workgroup_barrier();
     }
@@ -509,24 +650,8 @@ mixed_gemm_tile_kernel(TilePlan plan, Epilogue ep, uint16_t* __restrict__ d) {
     // ------------------------------------------------------------------ math waves
     const int mw = wave - kCopyWaves, wf = mw % WF, wm = (mw / WF) % G::WM, ws = mw / (WF * G::WM);
     const int i = c.lane & 31, g = c.lane >> 5;
-    ReadAt<G> at;
-    at.xor4 = (i >> 2) & 3;
-    at.xor8 = (i >> 1) & 7;
-    at.xorw = WT ? i & 3 : (i >> 2) & 3;
-    at.w = G::kW + WeightRows<G>::lds(wf * G::TN, i);
-    at.x4 = G::kX + (wm * G::TM) * 2048 + i * 64;
-    at.x6 = G::kX + (wm * G::TM) * 3072 + i * 96;
-    {
-      const int turn = (i >> 3) & 1;
-      auto piece = [&](int p) { return (p + turn == 6 ? 0 : p + turn) * 16; };
-      at.p6a = piece(2 * g);
-      at.p6b = piece(3 + 2 * g);
-      at.h6a = piece(1) + 8 * g;
-      at.h6b = piece(4) + 8 * g;
-    }
-    at.x8 = G::kX + (wm * G::TM) * 4096 + i * 128;
-    at.sw = WeightRows<G>::scale(wf * G::TN + g, i, (c.n0 & 127) >> 5);
-    at.sx = 512 + i * 16 + (((c.m0 & 127) >> 5) + wm * G::TM + (G::TM == 2 ? g : 0)) * 4;
+    const int sw = ws * 1024 + WeightRows<G>::scale(wf * G::TN + g, i, (c.n0 & 127) >> 5);
+    const int sx = ws * 1024 + 512 + i * 16 + (((c.m0 & 127) >> 5) + wm * G::TM + (G::TM == 2 ? g : 0)) * 4;
 
     v16f acc[G::TN][G::TM];
 #pragma unroll
@@ -540,51 +665,77 @@ mixed_gemm_tile_kernel(TilePlan plan, Epilogue ep, uint16_t* __restrict__ d) {
       rest_half<1, G>(acc, c, plan, wf, wm, ws, g);
     }
     workgroup_barrier();   // batch 0 has landed
-    const uint8_t* slot = lds + ws * G::kSlot;
-    const uint8_t* const ring_end = slot + NB * G::kBatch;
-    // This wave's stages of one segment.  Everything between two barriers is one basic block with its order fixed by scheduling
-    // barriers: an MFMA, the reads of the next half, the other MFMAs (the compiler would sink them behind the barrier).
-    auto run = [&](auto fmt_c, int stages) __attribute__((always_inline)) {
+    const uint8_t* batch = lds;
+    const uint8_t* const ring_end = lds + NB * G::kBatch;
+    auto next_batch = [&]() __attribute__((always_inline)) {
+      batch += G::kBatch;
+      batch = batch == ring_end ? lds : batch;
+    };
+    // This wave's stages of `stages` batches, all of one format.  Everything between two barriers is one basic block with its order fixed by
+    // scheduling barriers: an MFMA, the reads of the next half, the other MFMAs (the compiler would sink them behind the barrier).
+    auto run = [&](auto fmt_c, auto rows_c, int stages) __attribute__((always_inline)) {
       constexpr int FMT = decltype(fmt_c)::value;
+      constexpr bool BY_ROWS = decltype(rows_c)::value, RUN = BY_ROWS || FMT == kFmtE4M3 || !ROWS;
       if (stages == 0) return;
+      int row = i;
+      asm volatile("" : "+v"(row));   // the addresses of this format only: those of all five would be kept from the start
+      const ReadAt at = read_at<FMT, BY_ROWS, G>(row, g, wf, wm, ws);
       TileFrags<FMT, G> fa, fb, fn;
       RawScales<G> raw;
       TileScales<G> sc;
-      read_scales<G>(raw, slot, at);
-      read_half<FMT, 0, G>(fa, slot, at, g);
+      read_scales<G>(raw, batch, sw, sx);
+      read_half<FMT, 0, BY_ROWS, G>(fa, batch, at, g);
       auto first_half = [&]() __attribute__((always_inline)) {
         wait_lds();
         sc = shifted<G>(raw, g);
         multiply<FMT, 0, G, 0, 1>(acc, fa, sc);
         __builtin_amdgcn_sched_barrier(0);
-        read_half<FMT, 1, G>(fb, slot, at, g);
+        read_half<FMT, 1, BY_ROWS, G>(fb, batch, at, g);
         __builtin_amdgcn_sched_barrier(0);
         multiply<FMT, 0, G, 1, G::TN * G::TM>(acc, fa, sc);
         __builtin_amdgcn_sched_barrier(0);
         wait_lds();
         workgroup_barrier();   // the next batch has landed; this one is in registers
-        slot += G::kBatch;
-        slot = slot == ring_end ? slot - NB * G::kBatch : slot;
+        next_batch();
         __builtin_amdgcn_sched_barrier(0);
         multiply<FMT, 1, G, 0, 1>(acc, fb, sc);
         __builtin_amdgcn_sched_barrier(0);
       };
-      for (int q = 1; q < stages; ++q) {
-        first_half();
-        read_scales<G>(raw, slot, at);
-        read_half<FMT, 0, G>(fn, slot, at, g);
-        __builtin_amdgcn_sched_barrier(0);
-        multiply<FMT, 1, G, 1, G::TN * G::TM>(acc, fb, sc);
-        __builtin_amdgcn_sched_barrier(0);
-        fa = fn;
-      }
+      if constexpr (RUN) {
+        for (int q = 1; q < stages; ++q) {
+          first_half();
+          read_scales<G>(raw, batch, sw, sx);
+          read_half<FMT, 0, BY_ROWS, G>(fn, batch, at, g);
+          __builtin_amdgcn_sched_barrier(0);
+          multiply<FMT, 1, G, 1, G::TN * G::TM>(acc, fb, sc);
+          __builtin_amdgcn_sched_barrier(0);
+          fa = fn;
+        }
+      }   // (else a single stage)
       first_half();
       multiply<FMT, 1, G, 1, G::TN * G::TM>(acc, fb, sc);
     };
+    const std::integral_constant<int, kFmtE2M1> f4;
+    const std::integral_constant<int, kFmtE3M2> f6;
+    const std::integral_constant<int, kFmtE4M3> f8;
+    const std::true_type rows;
+    const std::false_type single;
+    // Batches [0, e4) are all E2M1, [b6, e6) all E3M2; e4 if it is below b6 has stages of several segments, and so has e6 where E3M2
+    // ends inside it.  (E4M3 stages are the last of every wave.)
+    const int e4 = t6 / WS, b6 = (t6 + WS - 1) / WS, e6 = max(t8 / WS, b6);
     auto mine = [&](int t) { return (max(t - ws, 0) + WS - 1) / WS; };   // of the first t stages
-    run(std::integral_constant<int, kFmtE2M1>{}, mine(t6));
-    run(std::integral_constant<int, kFmtE3M2>{}, mine(t8) - mine(t6));
-    run(std::integral_constant<int, kFmtE4M3>{}, mine(total) - mine(t8));
+    const int first = e4 * WS + ws, second = e6 * WS + ws;
+    if constexpr (ROWS) {
+      run(f4, rows, e4);
+      run(f4, single, first < t6);
+      run(f6, single, e4 < b6 && first >= t6 && first < t8);
+      run(f6, rows, e6 - b6);
+      run(f6, single, second < t8);
+    } else {
+      run(f4, single, mine(t6));
+      run(f6, single, mine(t8) - mine(t6));
+    }
+    run(f8, single, mine(total) - mine(t8));
     if (mine(total) < batches) workgroup_barrier();
 
     // Nothing reads or fills the ring any more.  The partial sums to LDS, as rows of tokens: a lane holds token i of its 32 x 32
@@ -644,13 +795,30 @@ mixed_gemm_tile_kernel(TilePlan plan, Epilogue ep, uint16_t* __restrict__ d) {
   }
 }
 
+// Whether batches of one segment are copied as rows of WS stages.  The lines it saves against what it costs once (more offsets before the
+// first copies, batches that are not whole in code of their own): one by one / as rows, us, tile-major, row-major weights, default plan:
+//   64 x 64, M = 256, N = 4096: 16 stages 5.53 / 6.03, 5.45 / 6.02; 28 7.36 / 7.44, 7.78 / 7.66; 32 8.06 / 7.81, 8.47 / 8.07; 64 12.5 / 11.1;
+//     112 19.8 / 17.5, 22.3 / 18.7
+//   128 x 64, M = 512: 8 stages 5.30 / 5.72, 5.43 / 5.83; 16 6.63 / 7.00, 7.24 / 7.19; 32 9.52 / 9.47, 11.5 / 10.1; 48 13.9 / 14.1; 64 15.3 / 14.4
+//     (its weights are most of its bytes: whole lines already where they are tile-major)
+//   128 x 128, M = 1024: 8 stages 6.77 / 7.12, 7.11 / 7.36; 16 9.24 / 9.10, 10.1 / 9.24; 32 13.7 / 12.6, 15.4 / 13.1; 48 20.6 / 19.8
+// (Least where a row of codes is not whole lines, K = 3072 and 5120: there the stages of a batch still end in the middle of one.)
+constexpr bool batch_rows(int tf, int tt, bool w_tiled, int stages) {
+  return stages >= (tf == 64 ? 32 : tt == 64 && w_tiled ? 56 : 16);
+}
+
 template <int TF, int TT, int WF, int WS>
 hipError_t launch_geo(const TilePlan& p, bool w_tiled, bool rem, const Epilogue& ep, uint16_t* d, hipStream_t stream) {
-  const auto kernel = w_tiled ? (rem ? mixed_gemm_tile_kernel<TF, TT, WF, WS, true, true> : mixed_gemm_tile_kernel<TF, TT, WF, WS, true, false>)
-                              : (rem ? mixed_gemm_tile_kernel<TF, TT, WF, WS, false, true> : mixed_gemm_tile_kernel<TF, TT, WF, WS, false, false>);
+  auto of = [&](auto rows_c) {
+    constexpr bool ROWS = decltype(rows_c)::value;
+    return w_tiled ? (rem ? mixed_gemm_tile_kernel<TF, TT, WF, WS, true, true, ROWS> : mixed_gemm_tile_kernel<TF, TT, WF, WS, true, false, ROWS>)
+                   : (rem ? mixed_gemm_tile_kernel<TF, TT, WF, WS, false, true, ROWS> : mixed_gemm_tile_kernel<TF, TT, WF, WS, false, false, ROWS>);
+  };
+  const auto kernel = batch_rows(TF, TT, w_tiled, p.total) ? of(std::true_type()) : of(std::false_type());
   static_assert((int64_t)kMostTilesAcross * 64 * kTileWaves < (int64_t)1 << 32, "threads along a dimension of the grid");
-  typedef Geo<TF, TT, WF, WS, false> G;
+  typedef Geo<TF, TT, WF, WS, false, false> G;
   constexpr int kLds = G::NB * G::kBatch;
+  static_assert(!batch_rows(TF, TT, false, G::NB * WS - 1) && !batch_rows(TF, TT, true, G::NB * WS - 1), "with rows the ring is filled at least once");
   if (hipError_t e = allow_dynamic_lds(reinterpret_cast<const void*>(kernel), kLds); e != hipSuccess) return e;
   hipLaunchKernelGGL(kernel, dim3(p.order.grid_x, grid_rows(p.order)), dim3(64 * kTileWaves), kLds, stream, p, ep, d);
   return hipGetLastError();

@@ -942,6 +942,28 @@ def test_small_tiles_refill_their_ring(abi, tf, tt, m, n, kn, ks, ko):
     _check_small_tiles(abi, m, n, kn, ks, ko)
 
 
+# Batches of one segment copied as rows of their stages: 2 and 4 stages per batch, segments that begin and end inside a batch (one, two
+# and three of them in it), rows of codes that are and are not whole lines, single segments, blocks past the whole stages; and on either
+# side of the line (16 stages, 64 x 64: 32, 128 x 64 on tile-major weights: 56) the same one by one.
+ROW_SHAPES = [
+    (64, 64, 262, 256, 2944, 1152, 640), (64, 64, 267, 200, 2176, 256, 1792), (64, 64, 257, 256, 0, 4224, 0), (64, 64, 321, 256, 4224, 0, 0),
+    (64, 64, 290, 256, 640, 1408, 2304), (64, 64, 262, 256, 1824, 928, 1568), (64, 64, 262, 256, 2048, 1024, 1024), (64, 64, 262, 256, 1920, 1024, 1024),
+    (64, 64, 262, 256, 1952, 928, 800),
+    (128, 64, 145, 5632, 4224, 2432, 640), (128, 64, 137, 5632, 3232, 3104, 1280), (128, 64, 145, 5632, 3712, 2560, 896), (128, 64, 145, 5632, 3584, 2560, 896),
+    (128, 64, 460, 2304, 896, 512, 640), (128, 64, 296, 3328, 1152, 384, 384), (128, 64, 145, 5632, 1184, 448, 416),
+    (128, 128, 399, 4864, 1152, 640, 384), (128, 128, 390, 5120, 1184, 288, 800), (128, 128, 399, 4864, 0, 2176, 128), (128, 128, 399, 4864, 1152, 0, 1152),
+    (128, 128, 399, 4864, 1024, 512, 384), (128, 128, 390, 5120, 1056, 544, 416), (128, 128, 399, 4864, 1024, 512, 512),
+]
+
+
+@pytest.mark.parametrize("tf,tt,m,n,kn,ks,ko", ROW_SHAPES)
+def test_small_tiles_copied_as_rows_of_a_batch(abi, tf, tt, m, n, kn, ks, ko):
+    _say("rows of a batch", tf, tt, m, n, kn, ks, ko)
+    cus = torch.cuda.get_device_properties(0).multi_processor_count
+    assert abi.gemm_kernel(m, n, kn, ks, ko, False, cus) == ("tile", tf, tt)
+    _check_small_tiles(abi, m, n, kn, ks, ko)
+
+
 @pytest.mark.parametrize("m", [1, 8, 16, 17])
 def test_row_major_weights_of_more_than_4_gb(abi, m):
     """Features behind the first 2^32 bytes of a segment's codes are multiplied with their own rows.  All scales are 1 and the sums
