@@ -833,11 +833,14 @@ struct TilePlanChoice { int tf, tt; double us; };
 // Fitted to 450 measured calls each (17 ... 2600 tokens, N 384 ... 28672, K 1024 ... 18944, tile-major weights; rms error 10 %,
 // before the runs of tiles per XCD of tile_order.h, which made launches of other than 8 n tiles up to 1.4 times as fast):
 // the tile taken is in the mean 0.5 % slower than the best of the three.  Long launches are held back by the clock that the power
-// limit leaves: no faster than the table's PFLOP/s on whole tiles (M = 1894, N = 8448, K = 13824: 198 us where the sum says 135, 170
-// on 256 x 256 tiles; over 55 calls of 35 ... 135 us the choice against those is then the faster one every time).
+// limit leaves: no faster than the table's PFLOP/s on whole tiles.  128 x 128: 2.9 with batches copied as rows (2.3 before: M = 1894, N = 8448,
+// K = 13824 198 us where the sum says 135).  Of 130 drawn calls that 2.3 sent to the whole-tile kernel and 2.9 does not, 126 are faster here, all 1.26
+// times in the mean, on row-major weights up to 1.9 times (M = 1355, N = 2688, K = 18944 94.5 -> 49.9 us; tile-major M = 1381, N = 5632,
+// K = 7488 44.9 -> 40.9), four slower: many tokens of few feature tiles (M = 6430, N = 1280, K = 12288 65 -> 77).  With 3.3 the
+// further ones gain 2 % in the mean.
 TilePlanChoice mixed_gemm_tile_plan(int M, int N, int KN, int KS, int KO, int cus) {
   static const struct { int tf, tt; double fixed, round, stage, fill, mb, rest, pflops; } kTiles[] = {
-      {128, 128, 2.87, -0.24, 0.260, 0.075, 0.41, 1.8, 2.3}, {128, 64, 1.47, 1.29, 0.170, 0.051, 0.39, 1.0, 2.0}, {64, 64, 1.55, 1.07, 0.125, 0.039, 0.46, 0.9, 1.5}};
+      {128, 128, 2.87, -0.24, 0.260, 0.075, 0.41, 1.8, 2.9}, {128, 64, 1.47, 1.29, 0.170, 0.051, 0.39, 1.0, 2.0}, {64, 64, 1.55, 1.07, 0.125, 0.039, 0.46, 0.9, 1.5}};
   const int stages = KN / 128 + KS / 128 + KO / 128;
   const bool rest = ((KN | KS | KO) & 127) != 0;
   TilePlanChoice best = {0, 0, 0.0};

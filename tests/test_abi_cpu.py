@@ -338,6 +338,8 @@ def test_segments_of_4_gb_of_row_major_weights_never_meet_32_bit_offsets(abi, cu
     (149, 20480, 2304, 1152, 128, True), (171, 20480, 11008, 0, 0, True),
     # ... and where small tiles are the faster ones
     (49, 9600, 1024, 0, 0, False), (85, 8192, 640, 256, 128, False), (140, 18944, 5120, 2816, 256, False), (136, 18944, 11968, 0, 128, False),
+    # long launches: held back by the power limit, but less than the whole-tile kernel
+    (738, 5376, 7680, 4224, 384, False), (1345, 2944, 8576, 4800, 448, False), (1051, 3584, 7680, 4224, 384, False), (5147, 4096, 7680, 4224, 384, True),
 ])
 def test_small_tiles_are_not_taken_where_they_were_measured_slower(abi, m, n, kn, ks, ko, others):
     for tiled in (False, True):
