@@ -53,7 +53,7 @@ def _stale(target: str, deps: list[str]) -> bool:
 # Kernels whose loads and LDS copies are inline assembly that the compiler does not count: a register such a load
 # is still to fill must never be moved or spilled, so these kernels must compile without scratch memory.  (The
 # whole-tile GEMM is listed for speed: a spill inside its K loop costs more than anything else there.)
-NO_SCRATCH_KERNELS = ("mixed_gemm_decode_kernel", "reorder_quant_dma_kernel", "mixed_gemm_256_kernel",
+NO_SCRATCH_KERNELS = ("mixed_gemm_decode_kernel", "reorder_quant_dma_kernel", "reorder_quant_part_kernel", "mixed_gemm_256_kernel",
                       "mixed_gemm_256_tail_kernel", "mixed_gemm_tile_kernel")
 
 

@@ -504,6 +504,110 @@ reorder_quant_dma_kernel(const uint8_t* __restrict__ x, const int16_t* __restric
   while (i < count) run(run, std::integral_constant<int, 0>{});
 }
 
+// ---------------------------------------------------------------------------------------------
+// Few rows: a workgroup quantizes 16 T channels of one row (two lanes per block) and nothing else.  A call of few rows is the latency of
+// one: launch, index and row on their way, gather, arithmetic, stores.  Here a long row's last three are spread over several CUs -- each
+// copies the whole row, since the gathered channels may lie anywhere in it, but only its part of the index --, and a short one is spared
+// the schedule and the ring of rows.  The launch grid is 8 x parts x rows / 8: workgroups go to the 8 XCDs round-robin, so the parts
+// of a row share an L2, which fetches it once (dealt out one by one, 128 rows of 14336 took 5.1 us instead of 3.5, of 28672 10.1 instead of 5.9).
+// us, rows in the caches, the kernel above -> T = 256:
+//   rows 16: K = 1024 2.65 -> 2.50, 4096 3.04 -> 2.82, 8192 3.25 -> 2.76, 14336 4.08 -> 2.96, 18944 4.79 -> 3.11, 28672 5.39 -> 3.17
+//   rows 128: K = 1024 2.69 -> 2.54, 4096 3.19 -> 2.98, 8192 3.33 -> 2.87, 14336 4.38 -> 3.48, 18944 5.07 -> 4.10
+// Layer calls, us: M = 32, N = 4096, K = 14336 13.6 -> 12.3; M = 100, N = K = 8192 16.6 -> 14.7 (some of it the GEMM's).
+// With RMSNorm: rows 16: K = 2048 3.54 -> 3.35, 5120 4.30 -> 3.80, 8192 4.50 -> 4.01, 14336 5.78 -> 4.45.  (Gathering in front of the
+// sum, with a barrier more, is level.)
+// ---------------------------------------------------------------------------------------------
+template <int T, bool KEEP, bool NORM>
+__global__ void __launch_bounds__(T)
+reorder_quant_part_kernel(const uint8_t* __restrict__ x, const int16_t* __restrict__ idx, int rows, int K, int KN, int KS, int KO,
+                          uint8_t* __restrict__ qn, uint8_t* __restrict__ qs, uint8_t* __restrict__ qo, uint8_t* __restrict__ sfn,
+                          uint8_t* __restrict__ sfs, uint8_t* __restrict__ sfo, const uint8_t* __restrict__ gamma, float eps, double inv_k) {
+  extern __shared__ __align__(16) uint8_t lds[];
+  __shared__ double row_sums[NORM ? T / 64 : 1];   // RMSNorm: the waves' sums of squares
+  const int tid = threadIdx.x, row = (int)blockIdx.z * 8 + (int)blockIdx.x;
+  if (row >= rows) return;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const unsigned lds0 = (unsigned)(size_t)(__attribute__((address_space(3))) uint8_t*)lds;
+  const int b = (int)blockIdx.y * (T / 2) + (tid >> 1), half = tid & 1;
+  const bool has_block = b < (K >> 5);
+  v4u iv[2];
+  const v4u* ip = reinterpret_cast<const v4u*>(idx + (size_t)(has_block ? b : 0) * 32 + half * 16);
+  asm volatile("global_load_dwordx4 %0, %1, off" : "=v"(iv[0]) : "v"(ip) : "memory");
+  asm volatile("global_load_dwordx4 %0, %1, off" : "=v"(iv[1]) : "v"(ip + 1) : "memory");
+  const uint8_t* base = x + (size_t)row * K * 2;
+  const int nchunks = K >> 3, copies = (nchunks + T - 1) / T;
+  for (int it = 0; it < copies; ++it)   // (past the row's end: its last piece again, into the padding)
+    dma16(base, (unsigned)min(it * T + tid, nchunks - 1) * 16u, lds0 + (unsigned)(it * T * 16 + wave * 1024));
+  const unsigned weights = (unsigned)copies * T * 16;   // RMSNorm: its weight, behind the row
+  if constexpr (NORM)
+    for (int it = 0; it < copies; ++it)
+      dma16(gamma, (unsigned)min(it * T + tid, nchunks - 1) * 16u, lds0 + weights + (unsigned)(it * T * 16 + wave * 1024));
+
+  const int nbn = KN >> 5, nbs = KS >> 5;
+  const int seg = b < nbn ? 0 : (b < nbn + nbs ? 1 : 2);
+  const int j = seg == 0 ? b : (seg == 1 ? b - nbn : b - nbn - nbs);
+  const int kseg = seg == 0 ? KN : (seg == 1 ? KS : KO);
+  const int fmt = seg == 0 ? kFmtE2M1 : (seg == 1 ? kFmtE3M2 : kFmtE4M3);
+  const int blk_bytes = fmt == kFmtE2M1 ? 16 : (fmt == kFmtE3M2 ? 24 : 32);
+  uint8_t* q = (seg == 0 ? qn : (seg == 1 ? qs : qo)) + (size_t)row * ((kseg >> 5) * blk_bytes) + j * blk_bytes;
+  uint8_t* sf = (seg == 0 ? sfn : (seg == 1 ? sfs : sfo)) + sf_offset(row, j, (kseg + 127) >> 7);
+  wait_vm(copies * (NORM ? 2 : 1));   // the index
+  asm volatile("" : "+v"(iv[0]), "+v"(iv[1]));
+  unsigned ga[16], u[16];
+#pragma unroll
+  for (int p = 0; p < 16; ++p) {
+    const unsigned pair = iv[p >> 3][(p & 7) >> 1];
+    ga[p] = lds0 + min((p & 1) ? pair >> 16 : pair & 0xffffu, (unsigned)(K - 1)) * 2u;   // an entry outside [0, K): channel K - 1
+    u[p] = 0u;
+  }
+  if constexpr (NORM) {   // every workgroup of a row sums all of it, a lane what it copied
+    wait_vm(copies);
+    double part[4] = {0.0, 0.0, 0.0, 0.0};
+    for (int it = 0; it < copies; ++it) {
+      const v4u a = *reinterpret_cast<const v4u*>(lds + (size_t)(it * T + tid) * 16);
+      if (it * T + tid < nchunks) {
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          const double lo = (double)__uint_as_float(a[e] << 16), hi = (double)__uint_as_float(a[e] & 0xffff0000u);
+          part[e] = __builtin_fma(lo, lo, part[e]);
+          part[e] = __builtin_fma(hi, hi, part[e]);
+        }
+      }
+    }
+    const double sum = wave_sum((part[0] + part[1]) + (part[2] + part[3]));
+    if ((tid & 63) == 0) row_sums[tid >> 6] = sum;
+    __builtin_amdgcn_s_waitcnt(0xC07F);   // lgkmcnt(0): the sum is in the LDS
+  }
+  wait_vm_imm<0>();
+  asm volatile("s_barrier" ::: "memory");
+  if (has_block) {
+    gather16<0>(u, ga, 0u);
+    [[maybe_unused]] unsigned gw[NORM ? 16 : 1];
+    [[maybe_unused]] float rn = 0.0f;
+    if constexpr (NORM) {
+#pragma unroll
+      for (int p = 0; p < 16; ++p) {
+        ga[p] += weights;
+        gw[p] = 0u;
+      }
+      gather16<0>(gw, ga, 0u);
+      double tot = 0.0;
+#pragma unroll
+      for (int w = 0; w < T / 64; ++w) tot += row_sums[w];
+      rn = rms_scale(tot, K, inv_k, eps);
+      gather_wait(gw);
+    }
+    gather_wait(u);
+    float f[16];
+#pragma unroll
+    for (int p = 0; p < 16; ++p) f[p] = __uint_as_float(u[p]);
+    if constexpr (NORM)
+#pragma unroll
+      for (int p = 0; p < 16; p += 2) rms_apply(f[p], f[p + 1], gw[p], gw[p + 1], rn);
+    quantize_half(f, fmt, half, StoreHalf<KEEP>{q, sf, half});
+  }
+}
+
 }  // namespace
 
 // gamma != nullptr: RMSNorm with that weight and eps before the gather (activations only).  src_rows != 0 (weights only):
@@ -564,15 +668,27 @@ hipError_t launch_reorder_quant(const void* x, const int16_t* idx, int rows, int
   // 23.8; K = 12288 16 6.25, 5.75 / 5.85, 5.45, 2048 30.4, 24.4 / 31.3, 24.7; K = 14336 128 6.35, 6.6 / 6.85, 6.65, 256 6.6, 6.85 / 7.3, 7.05, 257 10.3, 9.35 / 11.7, 9.5, 2048
   // 31.9, 28.4 / 33.0, 28.7; K = 12800 4096 51.0, 50.8 / 52.1, 51.0, 8192 93.8, 96.5 / 94.6, 96.6 (up to K = 15360: the LDS offsets of its three rows are
   // immediates).
-  // Codes kept for the GEMM that follows, gain of two lanes per layer call (N = 4096): 9 and 10 waves, 1 ... 128 rows 1 ... 5 % / 0 ... 3 %, 512 -2 % / -1 %, 2048 and
+  // (Fewer rows than CUs without RMSNorm do not get here: few_rows.)  Codes kept for the GEMM that follows, gain of two lanes per layer call (N = 4096): 9 and 10 waves, 1 ... 128 rows 1 ... 5 % / 0 ... 3 %, 512 -2 % / -1 %, 2048 and
   // 4096 -1 % / 0.5 %; 11 and 12, 1 ... 900 rows 0 ... 4 % / 0 ... 4 %, from 1300 on 0 / 1 %; 13 ... 16, up to 256 rows 0 ... 2 % / 0 ... 2 %, 512 -1 % / 0, 2048 and 4096 -2 % / -1 ... 1 %.
   auto two_lanes = [&](int t2, bool norm, bool kept) {
     const int64_t r = rows, cus = lim.cus;
     if (norm) return t2 <= 768 || (t2 <= 960 && r > cus && (t2 > 832 || r <= 16 * cus));
     if (t2 > 1024) return false;
-    if (t2 < 704) return 2 * r <= cus || (!kept && 2 * r >= 5 * cus && r <= 4 * cus);
+    if (t2 < 704) return !kept && 2 * r >= 5 * cus && r <= 4 * cus;
     if (t2 <= 768) return kept || r <= cus || r >= 4 * cus;
     return r <= cus || (!kept && r >= (t2 == 832 ? 24 : t2 == 896 ? 16 : 12) * cus);
+  };
+  // Fewer rows than CUs go to the kernel for few rows (from there on the workgroups of the other one are arranged so that an L2 puts the lines
+  // of scales together: K = 4096, 256 rows 3.01 us there, 3.06 here, 255 rows 3.32 and 3.10); of more than 20480 channels three quarters as many (K =
+  // 28672, 192 rows 6.60, 6.35, 255 7.16, 7.43).  Above 16384 channels and a workgroup of 4096 channels per CU with 8192 channels in each (K = 18944,
+  // 64 rows 3.66 with 4096, 3.55, 255 5.85, 5.18 (the other kernel 5.93); K = 28672, 64 rows 3.89, 3.62, 128 5.88, 4.70 (5.92)).  With RMSNorm, where
+  // every workgroup of a row sums all of it, at most a workgroup per CU (K = 8192, 128 rows 4.61, 4.14, 255 4.73, 4.98; K = 18944, 64 rows
+  // 6.92, 8.49), and not 2048 < K <= 4096 (3.72, 3.67, but a layer call of M = 8, N = 14336, K = 4096 10.7 -> 10.9 launched one by one).
+  const int64_t parts_of_4096 = (int64_t)rows * ((K + 4095) >> 12);
+  auto few_rows = [&](bool norm) {
+    // (the copies of the norm's weight want it aligned)
+    if (norm) return (K <= 2048 || K > 4096) && parts_of_4096 <= lim.cus && (reinterpret_cast<uintptr_t>(gamma) & 15u) == 0;
+    return K > 20480 ? (int64_t)rows * 4 <= (int64_t)lim.cus * 3 : rows < lim.cus;
   };
   // keep: the codes stay in the L2 for the kernel that reads them next (activations only); norm: RMSNorm of the row
   // before the gather (activations only; its codes are always kept: what follows a norm is the layer's GEMM)
@@ -581,6 +697,25 @@ hipError_t launch_reorder_quant(const void* x, const int16_t* idx, int rows, int
     constexpr bool KP = decltype(keep_c)::value;
     constexpr bool NM = decltype(norm_c)::value;
     const int t2 = ((K >> 4) + 63) & ~63;   // two lanes per block: K/16 lanes, rounded up to whole waves
+    if constexpr (!IS_W) {
+      auto parts = [&](auto t_c) {
+        constexpr int T = decltype(t_c)::value;
+        const auto kernel = reorder_quant_part_kernel<T, KP, NM>;
+        const int lds = ((K >> 3) + T - 1) / T * T * 16 * (NM ? 2 : 1);   // the row, and the RMSNorm's weight
+        if (lds > usable) { err = hipErrorInvalidValue; return; }
+        err = allow_dynamic_lds(reinterpret_cast<const void*>(kernel), usable);
+        if (err != hipSuccess) return;
+        hipLaunchKernelGGL(kernel, dim3(8, ((K >> 4) + T - 1) / T, (rows + 7) / 8), dim3(T), (size_t)lds, stream, xb, idx, rows, K, KN, KS, KO, qn, qs, qo,
+                           sfn, sfs, sfo, reinterpret_cast<const uint8_t*>(gm), eps, 1.0 / K);
+        err = hipGetLastError();
+      };
+      if (few_rows(NM)) {
+        if constexpr (!NM) {
+          if (K > 16384 && parts_of_4096 > lim.cus) return parts(std::integral_constant<int, 512>{});
+        }
+        return parts(std::integral_constant<int, 256>{});
+      }
+    }
     if (K <= 8192) {
       switch (t2) {
         case 64: launch_dma(reorder_quant_dma_kernel<16, 64, kNS, IS_W, 64, KP, NM, TI>, 16, kNS, 64, kPerCu); break;

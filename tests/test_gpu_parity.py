@@ -90,6 +90,21 @@ def test_wide_rows_with_two_lanes_per_block(abi, k, rows):
         _check_kept_codes(abi, rows, k)
 
 
+# Few rows: parts of 4096 channels, and of 8192 of more than 16384 and of enough rows (44 of 24576, 52 of 20480), whole and not; as many rows as
+# an XCD group of 8 and one to either side; on both sides of the lines to the other kernel (256 rows; above 20480 channels 192; with RMSNorm as
+# many workgroups as CUs: 128 rows of 8192, 42 of 24576); every workgroup size of that one up to K = 8192 behind them.
+@pytest.mark.parametrize("rows,k", [
+    (1, 32), (7, 96), (8, 4096), (9, 4128), (1, 8192), (15, 8224), (64, 12288), (85, 12288), (86, 12320), (17, 16384), (51, 16416), (52, 16416), (16, 20480),
+    (53, 20480), (42, 24576), (43, 24576), (191, 20512), (192, 20512), (193, 20512), (31, 32736), (40, 32736), (128, 8192), (129, 8192), (255, 2080), (255, 4096),
+    (256, 4096), (255, 5152), (256, 32), (256, 1056), (256, 2080), (256, 3104), (256, 4128), (256, 5152), (256, 6176), (256, 7200)])
+def test_few_rows(abi, rows, k):
+    split = _wide_split(k)
+    test_reorder_quantize_matches_oracle(abi, "x", rows, *split)
+    test_rmsnorm_reorder_quantize_matches_oracle(abi, rows, *split, 1e-5)
+    if rows <= 64:
+        _check_kept_codes(abi, rows, k)
+
+
 # The same instances with more rows than both slots of every workgroup hold, so that slots are filled again and the RMSNorm's sums change
 # places: one workgroup per CU has three or four of 900 rows (9 and 10 waves: of 1000 without RMSNorm), two per CU, with 11 and 12 waves and no
 # RMSNorm, two or three of 1100.
