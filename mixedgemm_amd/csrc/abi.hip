@@ -11,12 +11,12 @@ namespace mg {
 template <bool IS_W>
 hipError_t launch_reorder_quant(const void* x, const int16_t* idx, int rows, int K, int KN, int KS, int KO, uint8_t* qn,
                                 uint8_t* qs, uint8_t* qo, uint8_t* sfn, uint8_t* sfs, uint8_t* sfo, const void* gamma,
-                                float eps, bool keep_codes, int src_rows, unsigned* verdict, hipStream_t stream);
+                                float eps, bool keep_codes, int a_staged, int src_rows, unsigned* verdict, hipStream_t stream);
 void mixed_gemm_choice(int M, int N, int KN, int KS, int KO, bool w_tiled, int cus, int out[3]);
 hipError_t launch_mixed_gemm(const uint8_t* an, const uint8_t* bn, const uint8_t* as_, const uint8_t* bs,
                              const uint8_t* ao, const uint8_t* bo, const uint8_t* sfan, const uint8_t* sfbn,
                              const uint8_t* sfas, const uint8_t* sfbs, const uint8_t* sfao, const uint8_t* sfbo, int M,
-                             int a_rows, int N, int KN, int KS, int KO, unsigned flags, Epilogue ep, void* d,
+                             int a_rows, int a_staged, int N, int KN, int KS, int KO, unsigned flags, Epilogue ep, void* d,
                              hipStream_t stream);
 hipError_t launch_token_linear(const void* x, const int16_t* idx, const void* gamma, float eps, const uint8_t* bn, const uint8_t* bs,
                                const uint8_t* bo, const uint8_t* sfbn, const uint8_t* sfbs, const uint8_t* sfbo, int M, int N,
@@ -44,7 +44,7 @@ int check_split(int rows, int KN, int KS, int KO) {
 template <bool IS_W>
 int reorder_quantize(const void* x, const int16_t* idx, int rows, int K, int KN, int KS, int KO, uint8_t* qn,
                      uint8_t* qs, uint8_t* qo, uint8_t* sfn, uint8_t* sfs, uint8_t* sfo, void* stream,
-                     const void* gamma = nullptr, float eps = 0.0f, bool keep_codes = false, int src_rows = 0,
+                     const void* gamma = nullptr, float eps = 0.0f, bool keep_codes = false, int a_staged = 0, int src_rows = 0,
                      unsigned* verdict = nullptr) {
   if (int s = check_split(rows, KN, KS, KO)) return s;
   if (K != KN + KS + KO) return MG_ERR_BAD_SHAPE;
@@ -52,7 +52,7 @@ int reorder_quantize(const void* x, const int16_t* idx, int rows, int K, int KN,
   if (!ptr_ok(x, true) || !ptr_ok(idx, true)) return MG_ERR_BAD_POINTER;
   if (!ptr_ok(qn, KN > 0) || !ptr_ok(qs, KS > 0) || !ptr_ok(qo, KO > 0)) return MG_ERR_BAD_POINTER;
   if ((KN > 0 && !sfn) || (KS > 0 && !sfs) || (KO > 0 && !sfo)) return MG_ERR_BAD_POINTER;
-  return (int)mg::launch_reorder_quant<IS_W>(x, idx, rows, K, KN, KS, KO, qn, qs, qo, sfn, sfs, sfo, gamma, eps, keep_codes, src_rows,
+  return (int)mg::launch_reorder_quant<IS_W>(x, idx, rows, K, KN, KS, KO, qn, qs, qo, sfn, sfs, sfo, gamma, eps, keep_codes, a_staged, src_rows,
                                              verdict, static_cast<hipStream_t>(stream));
 }
 
@@ -90,7 +90,7 @@ hipError_t scratch_ptr(uint8_t** out) {
 int mixed_gemm(const uint8_t* an, const uint8_t* bn, const uint8_t* as_, const uint8_t* bs, const uint8_t* ao,
                      const uint8_t* bo, const uint8_t* sfan, const uint8_t* sfbn, const uint8_t* sfas,
                      const uint8_t* sfbs, const uint8_t* sfao, const uint8_t* sfbo, int M, int a_rows, int N, int KN,
-                     int KS, int KO, unsigned flags, const void* bias_bf16, int n_out, void* d_bf16, void* stream) {
+                     int KS, int KO, unsigned flags, const void* bias_bf16, int n_out, void* d_bf16, void* stream, int a_staged = 0) {
   if (int s = check_split(M, KN, KS, KO)) return s;
   if (N < 0 || a_rows < M) return MG_ERR_BAD_SHAPE;
   if (flags & ~MG_FLAG_W_TILED) return MG_ERR_BAD_SHAPE;
@@ -104,7 +104,7 @@ int mixed_gemm(const uint8_t* an, const uint8_t* bn, const uint8_t* as_, const u
     return MG_ERR_BAD_POINTER;
   if ((KN > 0 && (!sfan || !sfbn)) || (KS > 0 && (!sfas || !sfbs)) || (KO > 0 && (!sfao || !sfbo)))
     return MG_ERR_BAD_POINTER;
-  return (int)mg::launch_mixed_gemm(an, bn, as_, bs, ao, bo, sfan, sfbn, sfas, sfbs, sfao, sfbo, M, a_rows, N, KN, KS, KO,
+  return (int)mg::launch_mixed_gemm(an, bn, as_, bs, ao, bo, sfan, sfbn, sfas, sfbs, sfao, sfbo, M, a_rows, a_staged, N, KN, KS, KO,
                                     flags, mg::Epilogue{static_cast<const uint16_t*>(bias_bf16), n_out}, d_bf16, static_cast<hipStream_t>(stream));
 }
 
@@ -133,7 +133,7 @@ int mg_reorder_quantize_w_tiled(const void* w_bf16, const int16_t* idx, int n, i
                                 uint8_t* qs, uint8_t* qo, uint8_t* sfn, uint8_t* sfs, uint8_t* sfo, void* stream) {
   if (int s = check_split(N, KN, KS, KO)) return s;
   if (n <= 0 || n > N || N - n >= 256 || N % 256 != 0) return MG_ERR_BAD_SHAPE;
-  return reorder_quantize<true>(w_bf16, idx, N, K, KN, KS, KO, qn, qs, qo, sfn, sfs, sfo, stream, nullptr, 0.0f, false, n);
+  return reorder_quantize<true>(w_bf16, idx, N, K, KN, KS, KO, qn, qs, qo, sfn, sfs, sfo, stream, nullptr, 0.0f, false, 0, n);
 }
 
 int mg_pack_weights(const void* w_bf16, const int16_t* idx, int n, int N, int K, int KN, int KS, int KO, unsigned flags, uint8_t* qn,
@@ -141,7 +141,7 @@ int mg_pack_weights(const void* w_bf16, const int16_t* idx, int n, int N, int K,
   const bool tiled = (flags & MG_FLAG_W_TILED) != 0;
   if ((flags & ~MG_FLAG_W_TILED) != 0 || n <= 0 || n > N || (tiled ? N - n >= 256 || N % 256 != 0 : n != N)) return MG_ERR_BAD_SHAPE;
   if (verdict == nullptr || K <= 0) return verdict == nullptr ? MG_ERR_BAD_POINTER : MG_ERR_BAD_SHAPE;
-  return reorder_quantize<true>(w_bf16, idx, N, K, KN, KS, KO, qn, qs, qo, sfn, sfs, sfo, stream, nullptr, 0.0f, false, tiled ? n : 0, verdict);
+  return reorder_quantize<true>(w_bf16, idx, N, K, KN, KS, KO, qn, qs, qo, sfn, sfs, sfo, stream, nullptr, 0.0f, false, 0, tiled ? n : 0, verdict);
 }
 
 int mg_mixed_gemm_ex(const uint8_t* an, const uint8_t* bn, const uint8_t* as_, const uint8_t* bs, const uint8_t* ao,
@@ -232,12 +232,20 @@ int mg_linear(const void* x_bf16, const void* gamma_bf16, float eps, const int16
   uint8_t* sfn = p; p += align256(mg_sf_bytes(R, KN, MG_OPERAND_A));
   uint8_t* sfs = p; p += align256(mg_sf_bytes(R, KS, MG_OPERAND_A));
   uint8_t* sfo = p;
+  // Whole tiles get their codes stage by stage, in whole lines (see launch_reorder_quant): nobody else reads the workspace.
+  int staged = 0, choice[3];
+  if (M >= 256) {
+    mg::DeviceLimits lim;
+    if (hipError_t e = mg::device_limits(&lim); e != hipSuccess) return (int)e;
+    mg::mixed_gemm_choice(M, N, KN, KS, KO, tiled, lim.cus, choice);
+    if (choice[0] == MG_KERNEL_WHOLE) staged = R;
+  }
   // the GEMM reads the codes next: ordinary stores, so that they are in the L2 when it starts
   if (int s = reorder_quantize<false>(x_bf16, idx, M, KN + KS + KO, KN, KS, KO, qn, qs, qo, sfn, sfs, sfo, stream, gamma_bf16, eps,
-                                      /*keep_codes=*/true))
+                                      /*keep_codes=*/true, staged))
     return s;
   return mixed_gemm(qn, bn, qs, bs, qo, bo, sfn, sfbn, sfs, sfbs, sfo, sfbo, M, R, N, KN, KS, KO, flags, bias_bf16, n_out, d_bf16,
-                    stream);
+                    stream, staged);
 }
 
 int mg_fused_norm_linear(const void* x_bf16, const void* gamma_bf16, float eps, const int16_t* idx, const uint8_t* bn,

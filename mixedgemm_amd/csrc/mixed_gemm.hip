@@ -1291,7 +1291,7 @@ bool mixed_gemm_256_supported(int M, int N, int KN, int KS, int KO);
 hipError_t launch_mixed_gemm_256(const uint8_t* an, const uint8_t* bn, const uint8_t* as_, const uint8_t* bs,
                                  const uint8_t* ao, const uint8_t* bo, const uint8_t* sfan, const uint8_t* sfbn,
                                  const uint8_t* sfas, const uint8_t* sfbs, const uint8_t* sfao, const uint8_t* sfbo,
-                                 int m_store, int a_rows, int N, int KN, int KS, int KO, bool w_tiled, Epilogue ep,
+                                 int m_store, int a_rows, int a_staged, int N, int KN, int KS, int KO, bool w_tiled, Epilogue ep,
                                  void* d, hipStream_t stream);
 
 // tiles of 64 or 128 features x 64 or 128 tokens (mixed_gemm_tile.hip)
@@ -1402,11 +1402,12 @@ void mixed_gemm_choice(int M, int N, int KN, int KS, int KO, bool w_tiled, int c
   }
 }
 
-// a_rows: token rows for which the activation codes and scales are readable (>= M)
+// a_rows: token rows for which the activation codes and scales are readable (>= M).  a_staged: the codes are stage by stage, of so many rows
+// (see launch_reorder_quant); for the whole-tile kernel alone.
 hipError_t launch_mixed_gemm(const uint8_t* an, const uint8_t* bn, const uint8_t* as_, const uint8_t* bs,
                              const uint8_t* ao, const uint8_t* bo, const uint8_t* sfan, const uint8_t* sfbn,
                              const uint8_t* sfas, const uint8_t* sfbs, const uint8_t* sfao, const uint8_t* sfbo, int M,
-                             int a_rows, int N, int KN, int KS, int KO, unsigned flags, Epilogue ep, void* d,
+                             int a_rows, int a_staged, int N, int KN, int KS, int KO, unsigned flags, Epilogue ep, void* d,
                              hipStream_t stream) {
   if (M == 0 || N == 0) return hipSuccess;
   const bool w_tiled = (flags & 1u) != 0;   // MG_FLAG_W_TILED
@@ -1418,6 +1419,7 @@ hipError_t launch_mixed_gemm(const uint8_t* an, const uint8_t* bn, const uint8_t
   DeviceLimits lim;
   if (hipError_t e = device_limits(&lim); e != hipSuccess) return e;
   const GemmChoice c = choose_gemm(d4, d6, d8, M, N, KN, KS, KO, w_tiled, lim.cus);
+  if (a_staged != 0 && c.kernel != GemmKernel::kWhole) return hipErrorInvalidValue;
   switch (c.kernel) {
     case GemmKernel::kDecode:
       return launch_decode(d4, d6, d8, M, N, w_tiled, c.decode_f, c.lds, ep, static_cast<uint16_t*>(d), stream);
@@ -1427,7 +1429,7 @@ hipError_t launch_mixed_gemm(const uint8_t* an, const uint8_t* bn, const uint8_t
       return launch_mixed_gemm_tile(an, bn, as_, bs, ao, bo, sfan, sfbn, sfas, sfbs, sfao, sfbo, M, a_rows, N, KN, KS, KO, w_tiled,
                                     c.tile, ep, d, stream);
     case GemmKernel::kWhole:
-      return launch_mixed_gemm_256(an, bn, as_, bs, ao, bo, sfan, sfbn, sfas, sfbs, sfao, sfbo, M, a_rows, N, KN, KS, KO, w_tiled,
+      return launch_mixed_gemm_256(an, bn, as_, bs, ao, bo, sfan, sfbn, sfas, sfbs, sfao, sfbo, M, a_rows, a_staged, N, KN, KS, KO, w_tiled,
                                    ep, d, stream);
     default: return hipErrorInvalidValue;
   }

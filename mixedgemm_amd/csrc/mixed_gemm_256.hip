@@ -64,6 +64,7 @@ struct Plan {
   int blk0, blk1, blk2;               // 32-element blocks per segment (row pitches and scale atoms; up to 3 more than 4 * st)
   int total;                          // stages over all segments
   int w_tiled;                        // weights in tile-major order (see tile_weights_kernel): a copy reads 1 KB of consecutive bytes
+  int a_staged;                       // activation codes stage by stage, rows of the buffer (0: row-major, see launch_reorder_quant)
 };
 
 __device__ __forceinline__ const uint8_t* uni(const uint8_t* p) {
@@ -223,11 +224,11 @@ struct LaneOffsets {
 
 struct StageBases {
   const uint8_t *w, *x, *s;
-  unsigned ldb, lda;
+  unsigned ldb, lda, xstep;   // weight and token rows; from a stage of the tokens to the next
   int seg;   // -1: no such stage
   bool tiled;   // tile-major weights
 
-  __device__ __forceinline__ StageBases() : w(nullptr), x(nullptr), s(nullptr), ldb(0), lda(0), seg(-1), tiled(false) {}
+  __device__ __forceinline__ StageBases() : w(nullptr), x(nullptr), s(nullptr), ldb(0), lda(0), xstep(0), seg(-1), tiled(false) {}
 
   __device__ __forceinline__ StageBases(const Plan& plan, int q, const Ctx& c) {
     int ql;
@@ -241,7 +242,8 @@ struct StageBases {
     const unsigned nst = (blk + 3) >> 2;   // scale atoms along K
     const unsigned rb = sg == 0 ? 64 : (sg == 1 ? 96 : 128);
     ldb = blk * 16;
-    lda = blk * (rb >> 2);
+    lda = plan.a_staged ? rb : blk * (rb >> 2);
+    xstep = plan.a_staged ? (unsigned)plan.a_staged * rb : rb;
     tiled = plan.w_tiled != 0;
     if (plan.w_tiled) {
       // 16 KB per (feature tile, stage), 1 KB per copy block: the wave's 4 blocks are consecutive
@@ -252,7 +254,7 @@ struct StageBases {
       w = pb + (size_t)c.n0 * ldb + (size_t)ql * 64;   // the lanes' offsets carry the wave's rows
     }
     // the tile's first token row (the lanes' offsets carry the wave's rows); E4M3: K half wave / 4
-    x = pa + (size_t)c.m0 * lda + (size_t)ql * rb + (sg == 2 ? (c.wave >> 2) * 64 : 0);
+    x = pa + (size_t)c.m0 * lda + (size_t)ql * xstep + (sg == 2 ? (c.wave >> 2) * 64 : 0);
     s = c.wave < 4 ? psb + ((size_t)(c.n0 >> 7) * nst + ql) * 512 : psa + ((size_t)(c.m0 >> 7) * nst + ql) * 512;
   }
 };
@@ -317,7 +319,7 @@ struct LeanCopy {
   static constexpr int NV = kSteps ? 1 : NX;
   const uint8_t *w, *x, *s;        // bases of the stage being copied
   unsigned lds_w, lds_x, lds_s;    // LDS offsets of the wave's first weight / token block and scale atom pair in buffer 0
-  unsigned lda;
+  unsigned lda, xstep;
   unsigned vw[WC], vx[NV], vs, vlin;
 
   __device__ __forceinline__ void init(const Plan& plan, int q, const LaneOffsets&, const Ctx& c) {
@@ -333,6 +335,7 @@ struct LeanCopy {
       for (int k = 0; k < WC; ++k) vw[k] = lo.woff(k, b.ldb);
     }
     lda = __builtin_amdgcn_readfirstlane(b.lda);
+    xstep = __builtin_amdgcn_readfirstlane(b.xstep);
     if constexpr (kSteps) {
       const int row0 = lo.prow + 4 * (c.wave & 3);
       vx[0] = lo.xoff<TM>(2, 0, b.lda) | (unsigned)min(max(lo.last_row - row0, 0), NX - 1);
@@ -349,7 +352,7 @@ struct LeanCopy {
 
   __device__ __forceinline__ void advance() {
     w += WT ? 16384 : 64;
-    x += Fmt<FMT>::row_bytes;
+    x += xstep;
     s += 512;
   }
 
@@ -764,7 +767,7 @@ template <int FMT, int TM>
 __device__ __forceinline__ void remainder_load(RemainderHalf<FMT, TM>& f, int h, const uint8_t* __restrict__ a,
                                                const uint8_t* __restrict__ b, const uint8_t* __restrict__ sfa,
                                                const uint8_t* __restrict__ sfb, int blk, bool w_tiled, int tiles_n,
-                                               const Ctx& c) {
+                                               int a_staged, const Ctx& c) {
   const int r = blk & 3, q = blk >> 2;
   // weights: row-major rows of blk blocks, or (tile-major) the r blocks past the whole stages as rows of
   // r blocks behind the tiled part; with r == 0 nothing is used and any valid address will do
@@ -774,7 +777,10 @@ __device__ __forceinline__ void remainder_load(RemainderHalf<FMT, TM>& f, int h,
   constexpr int XB = Fmt<FMT>::row_bytes / 4;   // token bytes per block
   const int i = c.lane & 31, g = c.lane >> 5;
   const int katoms = (blk + 3) >> 2;
-  const unsigned lda = (unsigned)blk * XB;
+  // tokens: likewise rows of r blocks behind the whole stages where those are stage by stage
+  const uint8_t* const xbase = a_staged && r ? a + (size_t)a_staged * q * (4 * XB) : a;
+  const unsigned lda = (unsigned)(a_staged ? r : blk) * XB;
+  const int xfirst = a_staged ? 4 * q : 0;
   const int kb = 2 * h + g;
   const int kbc = min(4 * q + kb, blk - 1);           // a block that exists
   const int kb1 = min(4 * q + 2 * h + 1, blk - 1);    // E4M3: the second block of the half
@@ -788,18 +794,19 @@ __device__ __forceinline__ void remainder_load(RemainderHalf<FMT, TM>& f, int h,
   for (int t = 0; t < TM; ++t) {
     const unsigned m = c.m0 + min(c.wm * (32 * TM) + t * 32 + i, c.rows_avail - 1);   // rows past the last readable one are never stored
     f.sx[t] = sfa[sf_offset(m, kbc, katoms)];
-    const uint8_t* xr = a + (size_t)m * lda;
+    const uint8_t* xr = xbase + (size_t)m * lda;
+    const int kx = max(kbc - xfirst, 0);
     if constexpr (FMT == kFmtE2M1) {
-      f.x[t] = *reinterpret_cast<const v4i*>(xr + (size_t)kbc * 16);
+      f.x[t] = *reinterpret_cast<const v4i*>(xr + (size_t)kx * 16);
     } else if constexpr (FMT == kFmtE3M2) {
-      const v2i* p = reinterpret_cast<const v2i*>(xr + (size_t)kbc * 24);
+      const v2i* p = reinterpret_cast<const v2i*>(xr + (size_t)kx * 24);
       const v2i p0 = p[0], p1 = p[1], p2 = p[2];
       f.x[t] = v6i{p0[0], p0[1], p1[0], p1[1], p2[0], p2[1]};
     } else {
       // K [16g, 16g+16) of the half lies in block 2h, K [32+16g, ...) in block 2h+1
       const int kb0 = min(4 * q + 2 * h, blk - 1);
-      const v4i pa = *reinterpret_cast<const v4i*>(xr + (size_t)kb0 * 32 + g * 16);
-      const v4i pb = *reinterpret_cast<const v4i*>(xr + (size_t)kb1 * 32 + g * 16);
+      const v4i pa = *reinterpret_cast<const v4i*>(xr + (size_t)max(kb0 - xfirst, 0) * 32 + g * 16);
+      const v4i pb = *reinterpret_cast<const v4i*>(xr + (size_t)max(kb1 - xfirst, 0) * 32 + g * 16);
       f.x[t] = __builtin_shufflevector(pa, pb, 0, 1, 2, 3, 4, 5, 6, 7);
     }
   }
@@ -924,6 +931,7 @@ __device__ __forceinline__ Plan start_workgroup(const Plan& plan_arg, int first_
   plan.blk2 = __builtin_amdgcn_readfirstlane(plan_arg.blk2);
   plan.total = __builtin_amdgcn_readfirstlane(plan_arg.total);
   plan.w_tiled = WT ? 1 : 0;
+  plan.a_staged = __builtin_amdgcn_readfirstlane(plan_arg.a_staged);
   return plan;
 }
 
@@ -982,9 +990,9 @@ __device__ __forceinline__ void compute_tile(const Plan& plan, int tile_n, int t
   RemainderHalf<kFmtE3M2, TM> s0;
   RemainderHalf<kFmtE4M3, TM> o0;
   if constexpr (REM) {
-    if ((plan.blk0 & 3) > 0) remainder_load<kFmtE2M1>(p0, 0, plan.a0, plan.b0, plan.sfa0, plan.sfb0, plan.blk0, WT, tiles_n, c);
-    if ((plan.blk1 & 3) > 0) remainder_load<kFmtE3M2>(s0, 0, plan.a1, plan.b1, plan.sfa1, plan.sfb1, plan.blk1, WT, tiles_n, c);
-    if ((plan.blk2 & 3) > 0) remainder_load<kFmtE4M3>(o0, 0, plan.a2, plan.b2, plan.sfa2, plan.sfb2, plan.blk2, WT, tiles_n, c);
+    if ((plan.blk0 & 3) > 0) remainder_load<kFmtE2M1>(p0, 0, plan.a0, plan.b0, plan.sfa0, plan.sfb0, plan.blk0, WT, tiles_n, plan.a_staged, c);
+    if ((plan.blk1 & 3) > 0) remainder_load<kFmtE3M2>(s0, 0, plan.a1, plan.b1, plan.sfa1, plan.sfb1, plan.blk1, WT, tiles_n, plan.a_staged, c);
+    if ((plan.blk2 & 3) > 0) remainder_load<kFmtE4M3>(o0, 0, plan.a2, plan.b2, plan.sfa2, plan.sfb2, plan.blk2, WT, tiles_n, plan.a_staged, c);
     __builtin_amdgcn_sched_barrier(0);
   }
   // prologue: stages 0 and 1 and the first copies of stage 2 in flight; wait for stage 0 only.  The copies go out
@@ -1046,9 +1054,9 @@ __device__ __forceinline__ void compute_tile(const Plan& plan, int tile_n, int t
     RemainderHalf<kFmtE2M1, TM> p1;
     RemainderHalf<kFmtE3M2, TM> s1;
     RemainderHalf<kFmtE4M3, TM> o1;
-    if ((plan.blk0 & 3) > 2) remainder_load<kFmtE2M1>(p1, 1, plan.a0, plan.b0, plan.sfa0, plan.sfb0, plan.blk0, WT, tiles_n, c);
-    if ((plan.blk1 & 3) > 2) remainder_load<kFmtE3M2>(s1, 1, plan.a1, plan.b1, plan.sfa1, plan.sfb1, plan.blk1, WT, tiles_n, c);
-    if ((plan.blk2 & 3) > 2) remainder_load<kFmtE4M3>(o1, 1, plan.a2, plan.b2, plan.sfa2, plan.sfb2, plan.blk2, WT, tiles_n, c);
+    if ((plan.blk0 & 3) > 2) remainder_load<kFmtE2M1>(p1, 1, plan.a0, plan.b0, plan.sfa0, plan.sfb0, plan.blk0, WT, tiles_n, plan.a_staged, c);
+    if ((plan.blk1 & 3) > 2) remainder_load<kFmtE3M2>(s1, 1, plan.a1, plan.b1, plan.sfa1, plan.sfb1, plan.blk1, WT, tiles_n, plan.a_staged, c);
+    if ((plan.blk2 & 3) > 2) remainder_load<kFmtE4M3>(o1, 1, plan.a2, plan.b2, plan.sfa2, plan.sfb2, plan.blk2, WT, tiles_n, plan.a_staged, c);
     __builtin_amdgcn_sched_barrier(0);
     if ((plan.blk0 & 3) > 2) remainder_mfma<kFmtE2M1>(acc, p1, 1, plan.blk0, c);
     if ((plan.blk1 & 3) > 2) remainder_mfma<kFmtE3M2>(acc, s1, 1, plan.blk1, c);
@@ -1282,11 +1290,11 @@ static tail_kernel_t select_tail_kernel(int nlast) {
 hipError_t launch_mixed_gemm_256(const uint8_t* an, const uint8_t* bn, const uint8_t* as_, const uint8_t* bs,
                                  const uint8_t* ao, const uint8_t* bo, const uint8_t* sfan, const uint8_t* sfbn,
                                  const uint8_t* sfas, const uint8_t* sfbs, const uint8_t* sfao, const uint8_t* sfbo,
-                                 int m_store, int a_rows, int N, int KN, int KS, int KO, bool w_tiled, Epilogue ep,
+                                 int m_store, int a_rows, int a_staged, int N, int KN, int KS, int KO, bool w_tiled, Epilogue ep,
                                  void* d, hipStream_t stream) {
   // m_store tokens are computed in whole tiles of 256 or 128 token rows; rows past m_store are computed but not
   // stored; the activation buffers are read up to row a_rows - 1 only
-  if (m_store <= 0 || a_rows < m_store) return hipErrorInvalidValue;
+  if (m_store <= 0 || a_rows < m_store || (a_staged != 0 && a_staged < a_rows)) return hipErrorInvalidValue;
   DeviceLimits lim;
   if (hipError_t e = device_limits(&lim); e != hipSuccess) return e;
   const int tokens = tile_tokens(m_store, ep.n_out, lim.cus);
@@ -1328,6 +1336,7 @@ hipError_t launch_mixed_gemm_256(const uint8_t* an, const uint8_t* bn, const uin
   p.blk0 = KN / 32; p.blk1 = KS / 32; p.blk2 = KO / 32;
   p.total = p.st0 + p.st1 + p.st2;
   p.w_tiled = w_tiled ? 1 : 0;
+  p.a_staged = a_staged;
   if (w_tiled && N % kT != 0) return hipErrorInvalidValue;
   const int tiles_n = (ep.n_out + kT - 1) / kT, tiles_m = M / tokens;
   // more tiles than CUs: staggered start (see the kernel), up to kStartSkew ticks of the shader's clock counter

@@ -211,7 +211,7 @@ __global__ void __launch_bounds__(MAXT)
 reorder_quant_dma_kernel(const uint8_t* __restrict__ x, const int16_t* __restrict__ idx, int rows, int K, int KN, int KS,
                          int KO, uint8_t* __restrict__ qn, uint8_t* __restrict__ qs, uint8_t* __restrict__ qo,
                          uint8_t* __restrict__ sfn, uint8_t* __restrict__ sfs, uint8_t* __restrict__ sfo, RowSchedule sched,
-                         const uint16_t* __restrict__ gamma, float eps, double inv_k, int src_rows,
+                         const uint16_t* __restrict__ gamma, float eps, double inv_k, int src_rows, int a_staged,
                          unsigned* __restrict__ verdict) {
   extern __shared__ __align__(16) uint8_t lds[];
   __shared__ double row_sums[NORM ? 2 : 1][NORM ? MAXT / 64 : 1];   // RMSNorm: the waves' sums of squares, by row parity
@@ -325,6 +325,13 @@ reorder_quant_dma_kernel(const uint8_t* __restrict__ x, const int16_t* __restric
   if constexpr (TILED) {
     qbase = (seg == 0 ? qn : (seg == 1 ? qs : qo)) + (in_tile ? (size_t)(j >> 2) * 16384 : (size_t)rows * whole * 64) + (j & 3) * 16;
     pitch = in_tile ? (size_t)whole * 16384 : (size_t)((kseg >> 5) & 3) * 16;   // per tile, or per row
+  }
+  if constexpr (KEEP) {
+    if (a_staged != 0) {   // stage by stage
+      const bool in_stage = (j >> 2) < whole;
+      qbase = (seg == 0 ? qn : (seg == 1 ? qs : qo)) + (size_t)(in_stage ? j >> 2 : whole) * a_staged * (4 * blk_bytes) + (j & 3) * blk_bytes;
+      pitch = (size_t)(in_stage ? 4 : (kseg >> 5) & 3) * blk_bytes;
+    }
   }
   uint8_t* sfbase = seg == 0 ? sfn : (seg == 1 ? sfs : sfo);
 
@@ -610,12 +617,19 @@ reorder_quant_part_kernel(const uint8_t* __restrict__ x, const int16_t* __restri
 
 }  // namespace
 
+// a_staged != 0 (activations whose codes are kept): the codes of a segment stage by stage, as a GEMM on whole tiles copies them -- per whole
+// 128-wide stage `a_staged` rows (at least `rows`) of 64, 96 or 128 bytes one after the other, behind them rows of the blocks past the last whole
+// stage.  A copy of 16 rows is then one run of whole lines; row-major, a row's 64 bytes of a stage are half a line and its 96 bytes lie in
+// two, so that the GEMM fetched every line of E2M1 codes twice.  A row's stores are 64-byte pieces apart here, and the rows that share
+// a line are neighbours, on one XCD.  Layer calls, us, row-major -> stage by stage, one layer over and over / six in turn: M = 777, N = 5000, K = 5120 all
+// E2M1 30.2 -> 28.4 / 30.2 -> 28.2; M = 2048, N = 4096, K = 14336 77.5 -> 76.3 / 85.2 -> 79.8, row-major weights 88.7 -> 82.9 / 103 -> 95; M = 4096, N =
+// 14336, K = 4096 126.2 -> 123.7 / 131.0 -> 126.7; M = 4096, N = K = 5120 74.9 -> 70.8 / 78.7 -> 73.0; the same bits in all of them.
 // gamma != nullptr: RMSNorm with that weight and eps before the gather (activations only).  src_rows != 0 (weights only):
 // codes in tile-major order, x has src_rows rows and the result `rows`, a multiple of 256.  verdict (weights only): 16 words, see the kernel.
 template <bool IS_W>
 hipError_t launch_reorder_quant(const void* x, const int16_t* idx, int rows, int K, int KN, int KS, int KO, uint8_t* qn,
                                 uint8_t* qs, uint8_t* qo, uint8_t* sfn, uint8_t* sfs, uint8_t* sfo,
-                                const void* gamma, float eps, bool keep_codes, int src_rows, unsigned* verdict, hipStream_t stream) {
+                                const void* gamma, float eps, bool keep_codes, int a_staged, int src_rows, unsigned* verdict, hipStream_t stream) {
   if (rows == 0 || K == 0) return hipSuccess;
   if ((gamma != nullptr && IS_W) || (verdict != nullptr && !IS_W) || (src_rows != 0 && (!IS_W || src_rows > rows || rows % 256 != 0))) return hipErrorInvalidValue;
   const uint16_t* gm = static_cast<const uint16_t*>(gamma);
@@ -645,7 +659,7 @@ hipError_t launch_reorder_quant(const void* x, const int16_t* idx, int rows, int
     err = allow_dynamic_lds(reinterpret_cast<const void*>(kernel), usable);
     if (err != hipSuccess) return;
     hipLaunchKernelGGL(kernel, dim3(grid), dim3(nthreads), (size_t)lds, stream, xb, idx, rows, K, KN, KS, KO, qn, qs, qo, sfn,
-                       sfs, sfo, sched, gm, eps, 1.0 / K, src_rows, verdict);
+                       sfs, sfo, sched, gm, eps, 1.0 / K, src_rows, a_staged, verdict);
     err = hipGetLastError();
   };
   // Measured on M = 4096 ... 16384 rows of K = 3584 ... 18944: two row slots per workgroup, and per CU up to four
@@ -709,7 +723,7 @@ hipError_t launch_reorder_quant(const void* x, const int16_t* idx, int rows, int
                            sfn, sfs, sfo, reinterpret_cast<const uint8_t*>(gm), eps, 1.0 / K);
         err = hipGetLastError();
       };
-      if (few_rows(NM)) {
+      if (a_staged == 0 && few_rows(NM)) {
         if constexpr (!NM) {
           if (K > 16384 && parts_of_4096 > lim.cus) return parts(std::integral_constant<int, 512>{});
         }
@@ -773,8 +787,8 @@ hipError_t launch_reorder_quant(const void* x, const int16_t* idx, int rows, int
 }
 
 template hipError_t launch_reorder_quant<false>(const void*, const int16_t*, int, int, int, int, int, uint8_t*, uint8_t*,
-                                                uint8_t*, uint8_t*, uint8_t*, uint8_t*, const void*, float, bool, int, unsigned*, hipStream_t);
+                                                uint8_t*, uint8_t*, uint8_t*, uint8_t*, const void*, float, bool, int, int, unsigned*, hipStream_t);
 template hipError_t launch_reorder_quant<true>(const void*, const int16_t*, int, int, int, int, int, uint8_t*, uint8_t*,
-                                               uint8_t*, uint8_t*, uint8_t*, uint8_t*, const void*, float, bool, int, unsigned*, hipStream_t);
+                                               uint8_t*, uint8_t*, uint8_t*, uint8_t*, const void*, float, bool, int, int, unsigned*, hipStream_t);
 
 }  // namespace mg

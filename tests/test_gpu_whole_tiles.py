@@ -96,3 +96,28 @@ def test_every_instance_of_the_whole_tile_kernel(abi, m, n, kn, ks, ko):
 @pytest.mark.parametrize("kn,ks,ko", [(480, 448, 160), (384, 384, 256)])
 def test_rows_up_to_the_last_one_on_whole_tiles(abi, m, n, kn, ks, ko):
     _check(abi, m, n, kn, ks, ko)
+
+
+# A layer call hands the codes of its tokens to whole tiles stage by stage, matmul gets them row by row: the same bits.  Ragged tokens and features, 256 x 256,
+# 256 x 128 and both in one launch; one to three segments, 1 to 3 blocks past the whole stages; one lane per block from 16416 channels on.
+@pytest.mark.parametrize("m,n", [(2304, 3840), (300, 18944), (511, 28672), (4300, 4104)])
+@pytest.mark.parametrize("kn,ks,ko", [(512, 0, 0), (0, 512, 0), (0, 0, 512), (1024, 0, 128), (544, 448, 416), (480, 416, 160), (384, 384, 256), (10272, 5120, 1024),
+                                      (12832, 6400, 1280)])
+@pytest.mark.parametrize("norm", [False, True])
+def test_layer_calls_on_whole_tiles_equal_quantize_then_gemm(abi, m, n, kn, ks, ko, norm):
+    print("staged codes", m, n, kn, ks, ko, norm, flush=True)
+    cus = torch.cuda.get_device_properties(0).multi_processor_count
+    assert abi.gemm_kernel(m, n, kn, ks, ko, False, cus)[0] == "whole" or (m == 300 and kn > 10000)   # (small tiles)
+    k, g = kn + ks + ko, torch.Generator(device=DEV).manual_seed(m + kn)
+    x = torch.randn(m, k, device=DEV, generator=g)
+    x[:, ::37] *= 30
+    x, w = x.to(torch.bfloat16), (torch.randn(n, k, device=DEV, generator=g) * 0.02).to(torch.bfloat16)
+    idx = torch.randperm(k, device=DEV, generator=g).to(torch.int16)
+    gamma = (1 + 0.1 * torch.randn(k, device=DEV, generator=g)).to(torch.bfloat16)
+    b = abi.reorder_quantize_w(w, idx, kn, ks, ko)
+    a = abi.rmsnorm_reorder_quantize_x(x, gamma, 1e-5, idx, kn, ks, ko) if norm else abi.reorder_quantize_x(x, idx, kn, ks, ko)
+    kw = dict(norm_weight=gamma, eps=1e-5) if norm else {}
+    want = abi.matmul(a[0], b[0], a[1], b[1], a[2], b[2], *[t for pair in zip(a[3:], b[3:]) for t in pair])
+    assert torch.equal(abi.fused_linear(x, idx, *b, kn, ks, ko, **kw), want)
+    if abi.weights_tileable(n, kn, ks, ko):
+        assert torch.equal(abi.fused_linear(x, idx, *abi.tile_weights(*b[:3]), *b[3:], kn, ks, ko, w_tiled=True, **kw), want)
