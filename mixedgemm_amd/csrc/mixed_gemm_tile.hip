@@ -836,7 +836,8 @@ struct TilePlanChoice { int tf, tt; double us; };
 // limit leaves: no faster than the table's PFLOP/s on whole tiles.  128 x 128: 2.9 with batches copied as rows (2.3 before: M = 1894, N = 8448,
 // K = 13824 198 us where the sum says 135).  Of 130 drawn calls that 2.3 sent to the whole-tile kernel and 2.9 does not, 126 are faster here, all 1.26
 // times in the mean, on row-major weights up to 1.9 times (M = 1355, N = 2688, K = 18944 94.5 -> 49.9 us; tile-major M = 1381, N = 5632,
-// K = 7488 44.9 -> 40.9), four slower: many tokens of few feature tiles (M = 6430, N = 1280, K = 12288 65 -> 77).  With 3.3 the
+// K = 7488 44.9 -> 40.9), four slower, many tokens of few feature tiles, which runs along the features (cheapest_order) have made the faster ones
+// too (M = 6430, N = 1280, K = 12288 65 -> 77, now 50 as all MXFP4, 73 -> 78 -> 60 on row-major weights).  With 3.3 the
 // further ones gain 2 % in the mean.
 TilePlanChoice mixed_gemm_tile_plan(int M, int N, int KN, int KS, int KO, int cus) {
   static const struct { int tf, tt; double fixed, round, stage, fill, mb, rest, pflops; } kTiles[] = {
@@ -869,7 +870,7 @@ hipError_t launch_mixed_gemm_tile(const uint8_t* an, const uint8_t* bn, const ui
   p.N = N;
   p.m_store = m_store;
   p.a_rows = a_rows;
-  p.order = tile_order(ceil_div(ep.n_out, tf), ceil_div(m_store, tt), tf, tt);
+  p.order = cheapest_order(ceil_div(ep.n_out, tf), ceil_div(m_store, tt), tf, tt);
   const bool rem = ((KN | KS | KO) & 127) != 0;
   uint16_t* out = static_cast<uint16_t*>(d);
   if (tf == 128 && tt == 128) return launch_geo<128, 128, 2, 2>(p, w_tiled, rem, ep, out, stream);

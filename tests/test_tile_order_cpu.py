@@ -45,3 +45,14 @@ def test_grids_of_more_tiles_than_one_row_of_workgroups_takes(check):
     most = 1 << 22
     grids = [(most - 1, 1), (most, 1), (most + 1, 1), (1, most + 1), (5593752, 1), (11187503, 1), (2, 4194305), (3001, 2003)]
     assert check([(n, m, *f) for n, m in grids for f in FORMS]) == []
+
+
+def test_every_tile_of_the_order_with_the_fewest_bytes(tmp_path):
+    exe = str(tmp_path / "cheapest_order_check")
+    subprocess.check_call(["hipcc", "-x", "hip", "--offload-arch=gfx950", "-O2", "-std=c++17", os.path.join(os.path.dirname(SRC), "cheapest_order_check.cpp"), "-o", exe])
+    rng = random.Random(4)
+    grids = [(n, m, *f) for n in range(1, 31) for m in range(1, 61) for f in FORMS] + [(10, 51, 128, 128), (5, 30819, 128, 128), (1003, 2089, 128, 128)]
+    grids += [(rng.randrange(1, 300), rng.randrange(1, 3000), *rng.choice(FORMS)) for _ in range(200)]
+    text = "".join(f"{n} {m} {tf} {tt}\n" for n, m, tf, tt in grids)
+    out = subprocess.run([exe], input=text, capture_output=True, text=True, check=True).stdout.splitlines()
+    assert len(out) == 1 and int(out[0].split()[0]) > 300, out
