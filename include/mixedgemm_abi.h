@@ -151,7 +151,7 @@ int mg_padded_rows(int M);
  * Activation reorder-quantize followed by the mixed GEMM on the same stream
  * (the sequence src/bindings.cpp:69-186 then :9-67 performs with a device-wide
  * synchronize in between; bench_reorder_gemm.cu:163-167 times the same pair).
- * `workspace` receives the quantized activations and their scales;
+ * `workspace` receives the quantized activations and their scales, in the order in which the GEMM of the shape reads them;
  * mg_fused_workspace_bytes(M, KN, KS, KO) bytes, 256-byte aligned.
  */
 int mg_fused_linear(const void* x_bf16, const int16_t* idx,

@@ -1300,7 +1300,7 @@ TilePlanChoice mixed_gemm_tile_plan(int M, int N, int KN, int KS, int KO, int cu
 hipError_t launch_mixed_gemm_tile(const uint8_t* an, const uint8_t* bn, const uint8_t* as_, const uint8_t* bs,
                                   const uint8_t* ao, const uint8_t* bo, const uint8_t* sfan, const uint8_t* sfbn,
                                   const uint8_t* sfas, const uint8_t* sfbs, const uint8_t* sfao, const uint8_t* sfbo,
-                                  int m_store, int a_rows, int N, int KN, int KS, int KO, bool w_tiled, const TilePlanChoice& choice,
+                                  int m_store, int a_rows, int a_staged, int N, int KN, int KS, int KO, bool w_tiled, const TilePlanChoice& choice,
                                   Epilogue ep, void* d, hipStream_t stream);
 
 // Rough launch time of the whole-tile kernel in microseconds for fewer than 256 tokens, only to choose between the kernels: as
@@ -1403,7 +1403,7 @@ void mixed_gemm_choice(int M, int N, int KN, int KS, int KO, bool w_tiled, int c
 }
 
 // a_rows: token rows for which the activation codes and scales are readable (>= M).  a_staged: the codes are stage by stage, of so many rows
-// (see launch_reorder_quant); for the whole-tile kernel alone.
+// (see launch_reorder_quant); for whole and small tiles alone.
 hipError_t launch_mixed_gemm(const uint8_t* an, const uint8_t* bn, const uint8_t* as_, const uint8_t* bs,
                              const uint8_t* ao, const uint8_t* bo, const uint8_t* sfan, const uint8_t* sfbn,
                              const uint8_t* sfas, const uint8_t* sfbs, const uint8_t* sfao, const uint8_t* sfbo, int M,
@@ -1419,14 +1419,14 @@ hipError_t launch_mixed_gemm(const uint8_t* an, const uint8_t* bn, const uint8_t
   DeviceLimits lim;
   if (hipError_t e = device_limits(&lim); e != hipSuccess) return e;
   const GemmChoice c = choose_gemm(d4, d6, d8, M, N, KN, KS, KO, w_tiled, lim.cus);
-  if (a_staged != 0 && c.kernel != GemmKernel::kWhole) return hipErrorInvalidValue;
+  if (a_staged != 0 && c.kernel != GemmKernel::kWhole && c.kernel != GemmKernel::kTile) return hipErrorInvalidValue;
   switch (c.kernel) {
     case GemmKernel::kDecode:
       return launch_decode(d4, d6, d8, M, N, w_tiled, c.decode_f, c.lds, ep, static_cast<uint16_t*>(d), stream);
     case GemmKernel::kSkinny:
       return launch_skinny(d4, d6, d8, M, N, w_tiled, c.skinny, ep, static_cast<uint16_t*>(d), stream);
     case GemmKernel::kTile:
-      return launch_mixed_gemm_tile(an, bn, as_, bs, ao, bo, sfan, sfbn, sfas, sfbs, sfao, sfbo, M, a_rows, N, KN, KS, KO, w_tiled,
+      return launch_mixed_gemm_tile(an, bn, as_, bs, ao, bo, sfan, sfbn, sfas, sfbs, sfao, sfbo, M, a_rows, a_staged, N, KN, KS, KO, w_tiled,
                                     c.tile, ep, d, stream);
     case GemmKernel::kWhole:
       return launch_mixed_gemm_256(an, bn, as_, bs, ao, bo, sfan, sfbn, sfas, sfbs, sfao, sfbo, M, a_rows, a_staged, N, KN, KS, KO, w_tiled,

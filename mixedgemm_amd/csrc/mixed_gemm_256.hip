@@ -100,7 +100,7 @@ __device__ __forceinline__ int seg_of(const Plan& p, int q, int& local) {
 constexpr int kFmtNone = -1;   // "no stage": copies of a stage past the end of K
 
 template <int FMT> struct Fmt;
-template <> struct Fmt<kFmtNone> { static constexpr int seg = 3, row_bytes = 0, x_copies = 0; typedef v4i xfrag; };
+template <> struct Fmt<kFmtNone> { static constexpr int x_copies = 0; typedef v4i xfrag; };
 template <> struct Fmt<kFmtE2M1> { static constexpr int seg = 0, row_bytes = 64, x_copies = 4; typedef v4i xfrag; };
 template <> struct Fmt<kFmtE3M2> { static constexpr int seg = 1, row_bytes = 96, x_copies = 6; typedef v6i xfrag; };
 template <> struct Fmt<kFmtE4M3> { static constexpr int seg = 2, row_bytes = 128, x_copies = 8; typedef v8i xfrag; };

@@ -50,6 +50,7 @@ struct TilePlan {
   int N;          // weight rows
   int m_store;    // token rows that are stored
   int a_rows;     // token rows that may be read
+  int a_staged;   // the token codes are stage by stage, of so many rows (0: row-major, see launch_reorder_quant)
   TileOrder order;   // workgroup -> tile
 };
 
@@ -213,6 +214,7 @@ struct SegCopy {
   const uint8_t *w, *x;         // bases of the next stage
   const uint8_t* sc;            // this lane's scale piece
   unsigned vw[NW], vx[KX], bw[BW], bx[BX];
+  unsigned xstep;               // from a stage of the tokens to the next
   int wave;
 
   // token copies of a stage come in fours, a last pair is dealt to waves 0, 1 and 2, 3 in turn
@@ -220,9 +222,10 @@ struct SegCopy {
   __device__ __forceinline__ int block(int k) const { return (k + 1) * kCopyWaves <= NX ? wave + kCopyWaves * k : (wave & 1) + kCopyWaves * k; }
 
   // the bases, and what batches copied as rows need
-  __device__ __forceinline__ void init(const TileCtx<G>& c, const TileSeg& s, int wave_) {
+  __device__ __forceinline__ void init(const TileCtx<G>& c, const TileSeg& s, int a_staged, int wave_) {
     wave = wave_;
-    const unsigned pitch = (unsigned)s.blk * (Form<FMT>::row / 4);
+    const unsigned pitch = a_staged ? Form<FMT>::row : (unsigned)s.blk * (Form<FMT>::row / 4);
+    xstep = a_staged ? (unsigned)a_staged * Form<FMT>::row : Form<FMT>::row;
     x = s.a + (size_t)c.m0 * pitch;
     if constexpr (G::WT) {
       w = s.b + (size_t)(c.n0 >> 8) * s.whole * 16384;
@@ -251,13 +254,13 @@ struct SegCopy {
     sc = c.lane < 32 ? of_features + WeightRows<G>::scale_piece(c.lane) * 16 : of_rows + (c.lane & 31) * 16;
   }
   // what single stages need
-  __device__ __forceinline__ void init_stages(const TileCtx<G>& c, const TileSeg& s) {
+  __device__ __forceinline__ void init_stages(const TileCtx<G>& c, const TileSeg& s, int a_staged) {
     const int r = c.lane >> 2, p = (c.lane & 3) ^ ((c.lane >> 4) & 3);
     if constexpr (!G::WT) {
 #pragma unroll
       for (int k = 0; k < NW; ++k) vw[k] = __umul24(min(16 * (wave + kCopyWaves * k) + r, c.last_col), 16 * s.blk) + p * 16;
     }
-    const unsigned pitch = (unsigned)s.blk * (Form<FMT>::row / 4);
+    const unsigned pitch = a_staged ? Form<FMT>::row : (unsigned)s.blk * (Form<FMT>::row / 4);
 #pragma unroll
     for (int k = 0; k < KX; ++k) {
       const int b = block(k);
@@ -289,7 +292,7 @@ struct SegCopy {
       if ((k + 1) * kCopyWaves <= NX || (wave >> 1) == (t & 1)) copy_at(x, vx[k], batch + G::kX + G::TT * 128u * u + 1024u * block(k));
     scales(t, batch + 1024u * u);
     w += G::WT ? 16384 : 64;
-    x += Form<FMT>::row;
+    x += xstep;
   }
   // the next WS stages
   __device__ __forceinline__ void issue_batch(int t, unsigned batch) {
@@ -447,7 +450,7 @@ struct Rest {
   TileScales<G> sc;
 };
 template <int FMT, int H, class G>
-__device__ __forceinline__ void rest_load(Rest<FMT, G>& r, const TileCtx<G>& c, const TileSeg& s, int N, int wf, int wm) {
+__device__ __forceinline__ void rest_load(Rest<FMT, G>& r, const TileCtx<G>& c, const TileSeg& s, int N, int a_staged, int wf, int wm) {
   const int rem = s.blk & 3;
   const int i = c.lane & 31, g = c.lane >> 5, q = s.blk >> 2, katoms = (s.blk + 3) >> 2;
   const int kb = 4 * q + min(2 * H + g, rem - 1), kb0 = 4 * q + 2 * H, kb1 = 4 * q + min(2 * H + 1, rem - 1);   // blocks that exist
@@ -461,7 +464,9 @@ __device__ __forceinline__ void rest_load(Rest<FMT, G>& r, const TileCtx<G>& c, 
 #pragma unroll
   for (int t = 0; t < G::TM; ++t) {
     const int m = c.m0 + min((wm * G::TM + t) * 32 + i, c.last_row);
-    const uint8_t* row = s.a + (size_t)m * s.blk * (Form<FMT>::row / 4);
+    // (behind codes that are stage by stage: rows of the rem blocks; row points to where the row's first block would be)
+    const uint8_t* row = a_staged ? s.a + (size_t)a_staged * q * Form<FMT>::row + (size_t)m * rem * (Form<FMT>::row / 4) - (size_t)q * Form<FMT>::row
+                                  : s.a + (size_t)m * s.blk * (Form<FMT>::row / 4);
     r.sc.x[t] = s.sfa[sf_offset(m, kb, katoms)];
     if constexpr (FMT == kFmtE2M1) {
       r.f.x[t] = *reinterpret_cast<const v4i*>(row + (size_t)kb * 16);
@@ -506,9 +511,9 @@ __device__ __forceinline__ void rest_half(v16f (&acc)[G::TN][G::TM], const TileC
   Rest<kFmtE2M1, G> r4;
   Rest<kFmtE3M2, G> r6;
   Rest<kFmtE4M3, G> r8;
-  if (has4) rest_load<kFmtE2M1, H, G>(r4, c, p.s4, p.N, wf, wm);
-  if (has6) rest_load<kFmtE3M2, H, G>(r6, c, p.s6, p.N, wf, wm);
-  if (has8) rest_load<kFmtE4M3, H, G>(r8, c, p.s8, p.N, wf, wm);
+  if (has4) rest_load<kFmtE2M1, H, G>(r4, c, p.s4, p.N, p.a_staged, wf, wm);
+  if (has6) rest_load<kFmtE3M2, H, G>(r6, c, p.s6, p.N, p.a_staged, wf, wm);
+  if (has8) rest_load<kFmtE4M3, H, G>(r8, c, p.s8, p.N, p.a_staged, wf, wm);
   __builtin_amdgcn_sched_barrier(0);
   if (has4) rest_multiply<kFmtE2M1, H, G>(acc, r4, p.s4, g);
   if (has6) rest_multiply<kFmtE3M2, H, G>(acc, r6, p.s6, g);
@@ -520,7 +525,7 @@ __device__ __forceinline__ void rest_half(v16f (&acc)[G::TN][G::TM], const TileC
 __device__ __forceinline__ void pin_plan(const TilePlan& p, const Epilogue& ep, const uint16_t* d) {
   asm volatile("" : : "s"(p.s4.a), "s"(p.s4.b), "s"(p.s4.sfa), "s"(p.s4.sfb), "s"(p.s4.blk), "s"(p.s4.whole), "s"(p.s6.a), "s"(p.s6.b),
                "s"(p.s6.sfa), "s"(p.s6.sfb), "s"(p.s6.blk), "s"(p.s6.whole), "s"(p.s8.a), "s"(p.s8.b), "s"(p.s8.sfa), "s"(p.s8.sfb),
-               "s"(p.s8.blk), "s"(p.s8.whole), "s"(p.total), "s"(p.N), "s"(p.m_store), "s"(p.a_rows), "s"(p.order.xlog), "s"(p.order.div),
+               "s"(p.s8.blk), "s"(p.s8.whole), "s"(p.total), "s"(p.N), "s"(p.m_store), "s"(p.a_rows), "s"(p.a_staged), "s"(p.order.xlog), "s"(p.order.div),
                "s"(p.order.div2), "s"(p.order.magic), "s"(p.order.grid_x), "s"(p.order.tiles), "s"(ep.bias), "s"(ep.n_out), "s"(d));
 }
 
@@ -602,15 +607,16 @@ mixed_gemm_tile_kernel(TilePlan plan, Epilogue ep, uint16_t* __restrict__ d) {
     };
     int t = 0;
     constexpr int kFirst = NB * WS;
+    const int a_staged = ROWS ? 0 : plan.a_staged;
     auto init_rest = [&]() __attribute__((always_inline)) {
-      if (ROWS && t6 % WS) k4.init_stages(c, plan.s4);
-      k6.init(c, plan.s6, wave);
-      if (!ROWS || t6 % WS || t8 % WS) k6.init_stages(c, plan.s6);
-      k8.init(c, plan.s8, wave);
-      k8.init_stages(c, plan.s8);
+      if (ROWS && t6 % WS) k4.init_stages(c, plan.s4, a_staged);
+      k6.init(c, plan.s6, a_staged, wave);
+      if (!ROWS || t6 % WS || t8 % WS) k6.init_stages(c, plan.s6, a_staged);
+      k8.init(c, plan.s8, a_staged, wave);
+      k8.init_stages(c, plan.s8, a_staged);
     };
-    k4.init(c, plan.s4, wave);
-    if constexpr (!ROWS) k4.init_stages(c, plan.s4);
+    k4.init(c, plan.s4, a_staged, wave);
+    if constexpr (!ROWS) k4.init_stages(c, plan.s4, a_staged);
     const bool short4 = t6 < kFirst;
     if (short4) init_rest();
     if (ROWS || total >= kFirst) {   // (batch_rows)
@@ -814,7 +820,8 @@ hipError_t launch_geo(const TilePlan& p, bool w_tiled, bool rem, const Epilogue&
     return w_tiled ? (rem ? mixed_gemm_tile_kernel<TF, TT, WF, WS, true, true, ROWS> : mixed_gemm_tile_kernel<TF, TT, WF, WS, true, false, ROWS>)
                    : (rem ? mixed_gemm_tile_kernel<TF, TT, WF, WS, false, true, ROWS> : mixed_gemm_tile_kernel<TF, TT, WF, WS, false, false, ROWS>);
   };
-  const auto kernel = batch_rows(TF, TT, w_tiled, p.total) ? of(std::true_type()) : of(std::false_type());
+  // (codes that are stage by stage are whole lines as they are)
+  const auto kernel = p.a_staged == 0 && batch_rows(TF, TT, w_tiled, p.total) ? of(std::true_type()) : of(std::false_type());
   static_assert((int64_t)kMostTilesAcross * 64 * kTileWaves < (int64_t)1 << 32, "threads along a dimension of the grid");
   typedef Geo<TF, TT, WF, WS, false, false> G;
   constexpr int kLds = G::NB * G::kBatch;
@@ -858,10 +865,10 @@ TilePlanChoice mixed_gemm_tile_plan(int M, int N, int KN, int KS, int KO, int cu
 hipError_t launch_mixed_gemm_tile(const uint8_t* an, const uint8_t* bn, const uint8_t* as_, const uint8_t* bs,
                                   const uint8_t* ao, const uint8_t* bo, const uint8_t* sfan, const uint8_t* sfbn,
                                   const uint8_t* sfas, const uint8_t* sfbs, const uint8_t* sfao, const uint8_t* sfbo,
-                                  int m_store, int a_rows, int N, int KN, int KS, int KO, bool w_tiled, const TilePlanChoice& choice,
+                                  int m_store, int a_rows, int a_staged, int N, int KN, int KS, int KO, bool w_tiled, const TilePlanChoice& choice,
                                   Epilogue ep, void* d, hipStream_t stream) {
   const int tf = choice.tf, tt = choice.tt;
-  if (m_store <= 0 || a_rows < m_store) return hipErrorInvalidValue;
+  if (m_store <= 0 || a_rows < m_store || (a_staged != 0 && a_staged < a_rows)) return hipErrorInvalidValue;
   TilePlan p;
   p.s4 = {an, bn, sfan, sfbn, KN / 32, KN / 128};
   p.s6 = {as_, bs, sfas, sfbs, KS / 32, KS / 128};
@@ -870,6 +877,7 @@ hipError_t launch_mixed_gemm_tile(const uint8_t* an, const uint8_t* bn, const ui
   p.N = N;
   p.m_store = m_store;
   p.a_rows = a_rows;
+  p.a_staged = a_staged;
   p.order = cheapest_order(ceil_div(ep.n_out, tf), ceil_div(m_store, tt), tf, tt);
   const bool rem = ((KN | KS | KO) & 127) != 0;
   uint16_t* out = static_cast<uint16_t*>(d);

@@ -524,11 +524,12 @@ reorder_quant_dma_kernel(const uint8_t* __restrict__ x, const int16_t* __restric
 // With RMSNorm: rows 16: K = 2048 3.54 -> 3.35, 5120 4.30 -> 3.80, 8192 4.50 -> 4.01, 14336 5.78 -> 4.45.  (Gathering in front of the
 // sum, with a barrier more, is level.)
 // ---------------------------------------------------------------------------------------------
-template <int T, bool KEEP, bool NORM>
+// STAGED: the codes stage by stage (see launch_reorder_quant; as an argument 0.2 us of every other call).
+template <int T, bool KEEP, bool NORM, bool STAGED>
 __global__ void __launch_bounds__(T)
 reorder_quant_part_kernel(const uint8_t* __restrict__ x, const int16_t* __restrict__ idx, int rows, int K, int KN, int KS, int KO,
                           uint8_t* __restrict__ qn, uint8_t* __restrict__ qs, uint8_t* __restrict__ qo, uint8_t* __restrict__ sfn,
-                          uint8_t* __restrict__ sfs, uint8_t* __restrict__ sfo, const uint8_t* __restrict__ gamma, float eps, double inv_k) {
+                          uint8_t* __restrict__ sfs, uint8_t* __restrict__ sfo, const uint8_t* __restrict__ gamma, float eps, double inv_k, int a_staged) {
   extern __shared__ __align__(16) uint8_t lds[];
   __shared__ double row_sums[NORM ? T / 64 : 1];   // RMSNorm: the waves' sums of squares
   const int tid = threadIdx.x, row = (int)blockIdx.z * 8 + (int)blockIdx.x;
@@ -557,6 +558,12 @@ reorder_quant_part_kernel(const uint8_t* __restrict__ x, const int16_t* __restri
   const int fmt = seg == 0 ? kFmtE2M1 : (seg == 1 ? kFmtE3M2 : kFmtE4M3);
   const int blk_bytes = fmt == kFmtE2M1 ? 16 : (fmt == kFmtE3M2 ? 24 : 32);
   uint8_t* q = (seg == 0 ? qn : (seg == 1 ? qs : qo)) + (size_t)row * ((kseg >> 5) * blk_bytes) + j * blk_bytes;
+  if constexpr (STAGED) {
+    const int whole = kseg >> 7;
+    const bool in_stage = (j >> 2) < whole;
+    q = (seg == 0 ? qn : (seg == 1 ? qs : qo)) + (size_t)(in_stage ? j >> 2 : whole) * a_staged * (4 * blk_bytes) +
+        (size_t)row * ((in_stage ? 4 : (kseg >> 5) & 3) * blk_bytes) + (j & 3) * blk_bytes;
+  }
   uint8_t* sf = (seg == 0 ? sfn : (seg == 1 ? sfs : sfo)) + sf_offset(row, j, (kseg + 127) >> 7);
   wait_vm(copies * (NORM ? 2 : 1));   // the index
   asm volatile("" : "+v"(iv[0]), "+v"(iv[1]));
@@ -617,13 +624,15 @@ reorder_quant_part_kernel(const uint8_t* __restrict__ x, const int16_t* __restri
 
 }  // namespace
 
-// a_staged != 0 (activations whose codes are kept): the codes of a segment stage by stage, as a GEMM on whole tiles copies them -- per whole
+// a_staged != 0 (activations whose codes are kept): the codes of a segment stage by stage, as a GEMM on tiles copies them -- per whole
 // 128-wide stage `a_staged` rows (at least `rows`) of 64, 96 or 128 bytes one after the other, behind them rows of the blocks past the last whole
 // stage.  A copy of 16 rows is then one run of whole lines; row-major, a row's 64 bytes of a stage are half a line and its 96 bytes lie in
 // two, so that the GEMM fetched every line of E2M1 codes twice.  A row's stores are 64-byte pieces apart here, and the rows that share
 // a line are neighbours, on one XCD.  Layer calls, us, row-major -> stage by stage, one layer over and over / six in turn: M = 777, N = 5000, K = 5120 all
 // E2M1 30.2 -> 28.4 / 30.2 -> 28.2; M = 2048, N = 4096, K = 14336 77.5 -> 76.3 / 85.2 -> 79.8, row-major weights 88.7 -> 82.9 / 103 -> 95; M = 4096, N =
-// 14336, K = 4096 126.2 -> 123.7 / 131.0 -> 126.7; M = 4096, N = K = 5120 74.9 -> 70.8 / 78.7 -> 73.0; the same bits in all of them.
+// 14336, K = 4096 126.2 -> 123.7 / 131.0 -> 126.7; M = 4096, N = K = 5120 74.9 -> 70.8 / 78.7 -> 73.0.  On small tiles (tile-major weights; before, long
+// launches copied batches of rows): M = 256, N = K = 4096 10.9 -> 10.5 / 11.4 -> 11.0, M = 1024 19.6 -> 19.0 / 19.8 -> 19.4; M = 700, N = 4096, K = 5120 21.1
+// -> 19.6 / 21.2 -> 19.5; M = 140, N = 18944, K = 8192 32.2 -> 30.7 / 44.5 -> 42.8.  The same bits in all of them.
 // gamma != nullptr: RMSNorm with that weight and eps before the gather (activations only).  src_rows != 0 (weights only):
 // codes in tile-major order, x has src_rows rows and the result `rows`, a multiple of 256.  verdict (weights only): 16 words, see the kernel.
 template <bool IS_W>
@@ -714,16 +723,19 @@ hipError_t launch_reorder_quant(const void* x, const int16_t* idx, int rows, int
     if constexpr (!IS_W) {
       auto parts = [&](auto t_c) {
         constexpr int T = decltype(t_c)::value;
-        const auto kernel = reorder_quant_part_kernel<T, KP, NM>;
+        auto kernel = reorder_quant_part_kernel<T, KP, NM, false>;
+        if constexpr (KP) {
+          if (a_staged != 0) kernel = reorder_quant_part_kernel<T, KP, NM, true>;
+        }
         const int lds = ((K >> 3) + T - 1) / T * T * 16 * (NM ? 2 : 1);   // the row, and the RMSNorm's weight
         if (lds > usable) { err = hipErrorInvalidValue; return; }
         err = allow_dynamic_lds(reinterpret_cast<const void*>(kernel), usable);
         if (err != hipSuccess) return;
         hipLaunchKernelGGL(kernel, dim3(8, ((K >> 4) + T - 1) / T, (rows + 7) / 8), dim3(T), (size_t)lds, stream, xb, idx, rows, K, KN, KS, KO, qn, qs, qo,
-                           sfn, sfs, sfo, reinterpret_cast<const uint8_t*>(gm), eps, 1.0 / K);
+                           sfn, sfs, sfo, reinterpret_cast<const uint8_t*>(gm), eps, 1.0 / K, a_staged);
         err = hipGetLastError();
       };
-      if (a_staged == 0 && few_rows(NM)) {
+      if (few_rows(NM)) {
         if constexpr (!NM) {
           if (K > 16384 && parts_of_4096 > lim.cus) return parts(std::integral_constant<int, 512>{});
         }

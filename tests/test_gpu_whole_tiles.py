@@ -105,9 +105,24 @@ def test_rows_up_to_the_last_one_on_whole_tiles(abi, m, n, kn, ks, ko):
                                       (12832, 6400, 1280)])
 @pytest.mark.parametrize("norm", [False, True])
 def test_layer_calls_on_whole_tiles_equal_quantize_then_gemm(abi, m, n, kn, ks, ko, norm):
-    print("staged codes", m, n, kn, ks, ko, norm, flush=True)
     cus = torch.cuda.get_device_properties(0).multi_processor_count
     assert abi.gemm_kernel(m, n, kn, ks, ko, False, cus)[0] == "whole" or (m == 300 and kn > 10000)   # (small tiles)
+    _check_layer_call(abi, m, n, kn, ks, ko, norm)
+
+
+# The same on small tiles of tile-major weights: every tile, fewer and more than 256 tokens (two quantizers), one to three segments that begin and end
+# inside a batch, 1 to 3 blocks past the whole stages, few and many stages.
+@pytest.mark.parametrize("tf,tt,m,n", [(64, 64, 262, 256), (64, 64, 70, 5632), (128, 64, 145, 5632), (128, 64, 460, 2304), (128, 128, 399, 4864)])
+@pytest.mark.parametrize("kn,ks,ko", [(1664, 640, 384), (1632, 736, 544), (2432, 0, 256), (0, 2176, 384), (2560, 1408, 128), (4160, 2144, 288)])
+@pytest.mark.parametrize("norm", [False, True])
+def test_layer_calls_on_small_tiles_equal_quantize_then_gemm(abi, tf, tt, m, n, kn, ks, ko, norm):
+    cus = torch.cuda.get_device_properties(0).multi_processor_count
+    assert abi.gemm_kernel(m, n, kn, ks, ko, True, cus)[0] == "tile"
+    _check_layer_call(abi, m, n, kn, ks, ko, norm)
+
+
+def _check_layer_call(abi, m, n, kn, ks, ko, norm):
+    print("staged codes", m, n, kn, ks, ko, norm, flush=True)
     k, g = kn + ks + ko, torch.Generator(device=DEV).manual_seed(m + kn)
     x = torch.randn(m, k, device=DEV, generator=g)
     x[:, ::37] *= 30
