@@ -33,7 +33,7 @@ OBJ_DIR = os.path.join(EXT_DIR, "obj")
 
 HIP_SOURCES = ["abi.hip", "reorder_quant.hip", "mixed_gemm.hip", "mixed_gemm_256.hip", "mixed_gemm_tile.hip", "calibrate.hip"]
 BENCH_SOURCES = ["bench_kernels.hip"]
-HIP_HEADERS = ["mg_common.h", "quantize.h", "tile_order.h", os.path.join(ROOT, "include", "mixedgemm_abi.h")]
+HIP_HEADERS = ["mg_common.h", "quantize.h", "staged_codes.h", "tile_order.h", os.path.join(ROOT, "include", "mixedgemm_abi.h")]
 
 HIPCC_FLAGS = [
     "--offload-arch=gfx950", "-O3", "-std=c++17", "-fPIC",

@@ -4,6 +4,7 @@
 #include "../../include/mixedgemm_abi.h"
 
 #include "mg_common.h"
+#include "staged_codes.h"
 
 #include <vector>
 
@@ -232,14 +233,13 @@ int mg_linear(const void* x_bf16, const void* gamma_bf16, float eps, const int16
   uint8_t* sfn = p; p += align256(mg_sf_bytes(R, KN, MG_OPERAND_A));
   uint8_t* sfs = p; p += align256(mg_sf_bytes(R, KS, MG_OPERAND_A));
   uint8_t* sfo = p;
-  // Whole tiles, and small ones on tile-major weights, get their codes stage by stage, in whole lines (see launch_reorder_quant): nobody else
-  // reads the workspace.  (On row-major weights small tiles copy batches of rows, weights and tokens alike.)
+  // The GEMMs on tiles get their codes stage by stage: nobody else reads the workspace.
   int staged = 0, choice[3];
   if (M > 16) {
     mg::DeviceLimits lim;
     if (hipError_t e = mg::device_limits(&lim); e != hipSuccess) return (int)e;
     mg::mixed_gemm_choice(M, N, KN, KS, KO, tiled, lim.cus, choice);
-    if (choice[0] == MG_KERNEL_WHOLE || (choice[0] == MG_KERNEL_TILE && tiled)) staged = R;
+    staged = mg::staged_rows(choice[0], tiled, R);
   }
   // the GEMM reads the codes next: ordinary stores, so that they are in the L2 when it starts
   if (int s = reorder_quantize<false>(x_bf16, idx, M, KN + KS + KO, KN, KS, KO, qn, qs, qo, sfn, sfs, sfo, stream, gamma_bf16, eps,

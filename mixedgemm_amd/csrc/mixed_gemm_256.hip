@@ -21,6 +21,7 @@
 // too short for that run a generic body whose copy format is a run-time, wave-uniform value.
 // The result tile is transposed through LDS so that stores write 256 contiguous bytes per row.
 #include "mg_common.h"
+#include "staged_codes.h"
 
 #include <type_traits>
 
@@ -1294,7 +1295,7 @@ hipError_t launch_mixed_gemm_256(const uint8_t* an, const uint8_t* bn, const uin
                                  void* d, hipStream_t stream) {
   // m_store tokens are computed in whole tiles of 256 or 128 token rows; rows past m_store are computed but not
   // stored; the activation buffers are read up to row a_rows - 1 only
-  if (m_store <= 0 || a_rows < m_store || (a_staged != 0 && a_staged < a_rows)) return hipErrorInvalidValue;
+  if (m_store <= 0 || a_rows < m_store || (a_staged != 0 && (a_staged < a_rows || !staged_in_reach(a_staged)))) return hipErrorInvalidValue;
   DeviceLimits lim;
   if (hipError_t e = device_limits(&lim); e != hipSuccess) return e;
   const int tokens = tile_tokens(m_store, ep.n_out, lim.cus);

@@ -23,6 +23,7 @@
 // 4096, K = 12288: 57.6 against 56.3 us: 15 % fewer cycles at a clock as much lower; the chip is at its power limit there), tiles of
 // 64 and 128 x 32 slower than 64 x 64 at every shape tried.
 #include "mg_common.h"
+#include "staged_codes.h"
 #include "tile_order.h"
 
 #include <type_traits>
@@ -868,7 +869,7 @@ hipError_t launch_mixed_gemm_tile(const uint8_t* an, const uint8_t* bn, const ui
                                   int m_store, int a_rows, int a_staged, int N, int KN, int KS, int KO, bool w_tiled, const TilePlanChoice& choice,
                                   Epilogue ep, void* d, hipStream_t stream) {
   const int tf = choice.tf, tt = choice.tt;
-  if (m_store <= 0 || a_rows < m_store || (a_staged != 0 && a_staged < a_rows)) return hipErrorInvalidValue;
+  if (m_store <= 0 || a_rows < m_store || (a_staged != 0 && (a_staged < a_rows || !staged_in_reach(a_staged)))) return hipErrorInvalidValue;
   TilePlan p;
   p.s4 = {an, bn, sfan, sfbn, KN / 32, KN / 128};
   p.s6 = {as_, bs, sfas, sfbs, KS / 32, KS / 128};
