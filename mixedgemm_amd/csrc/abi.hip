@@ -235,7 +235,7 @@ int mg_linear(const void* x_bf16, const void* gamma_bf16, float eps, const int16
   uint8_t* sfo = p;
   // The GEMMs on tiles get their codes stage by stage: nobody else reads the workspace.
   int staged = 0, choice[3];
-  if (M > 16) {
+  if (M > 16 && KN + KS + KO > 0 && ptr_ok(x_bf16, true) && ptr_ok(idx, true)) {   // (else there is nothing to quantize, or the call below refuses it)
     mg::DeviceLimits lim;
     if (hipError_t e = mg::device_limits(&lim); e != hipSuccess) return (int)e;
     mg::mixed_gemm_choice(M, N, KN, KS, KO, tiled, lim.cus, choice);

@@ -296,6 +296,16 @@ def test_static_entry_point_refuses_what_does_not_fit(abi):
 
 
 # ------------------------------------------------------------------ which kernel a shape runs on
+@pytest.mark.parametrize("m", [1, 16, 17, 300])
+def test_layer_calls_say_what_is_wrong_before_they_ask_for_the_device(abi, m):
+    lib, good = abi.lib(), 1 << 20   # (an address that nothing reads)
+
+    def call(x=good, idx=good, d=good, kn=256):
+        ws = lib.mg_fused_workspace_bytes(m, kn, 0, 0)
+        return lib.mg_linear(x, None, 0.0, idx, *[good] * 6, None, m, 256, 256, kn, 0, 0, 0, d, good, ws, None)
+    assert call(x=None) == call(x=good + 2) == call(idx=None) == call(idx=good + 2) == call(kn=0, d=None) == 10002
+
+
 def test_gemm_kernel_query(abi):
     import torch  # noqa: F401
     assert abi.gemm_kernel(0, 256, 128, 0, 0) == ("none", 0, 0) and abi.gemm_kernel(4, 0, 128, 0, 0) == ("none", 0, 0)
