@@ -206,13 +206,15 @@ struct RowSchedule {
 // tiles) are quantized as zeros.  A row's stores are then 64-byte pieces 16 KB apart instead of one run; the two rows that
 // share a line go to workgroups of one XCD, whose L2 joins them, and the pass is as fast as the row-major one:
 // W[14336, 4096] 38.7 us for quantizing and tiling one after the other, 24.6 in one pass (6.0 TB/s of what it has to move).
-template <int EPL, int T, int NS, bool IS_W, int MAXT, bool KEEP = false, bool NORM = false, bool TILED = false>
+// STAGED: the codes stage by stage (see launch_reorder_quant).  (Asked for at run time, every call whose codes are kept paid for it, most where the launch is all
+// there is: M = 8, N = 14336, K = 4096 with RMSNorm 10.80 us, 10.75 without.)
+template <int EPL, int T, int NS, bool IS_W, int MAXT, bool KEEP = false, bool NORM = false, bool TILED = false, bool STAGED = false>
 __global__ void __launch_bounds__(MAXT)
 reorder_quant_dma_kernel(const uint8_t* __restrict__ x, const int16_t* __restrict__ idx, int rows, int K, int KN, int KS,
                          int KO, uint8_t* __restrict__ qn, uint8_t* __restrict__ qs, uint8_t* __restrict__ qo,
                          uint8_t* __restrict__ sfn, uint8_t* __restrict__ sfs, uint8_t* __restrict__ sfo, RowSchedule sched,
-                         const uint16_t* __restrict__ gamma, float eps, double inv_k, int src_rows, int a_staged,
-                         unsigned* __restrict__ verdict) {
+                         const uint16_t* __restrict__ gamma, float eps, double inv_k, int src_rows, unsigned* __restrict__ verdict,
+                         int a_staged) {
   extern __shared__ __align__(16) uint8_t lds[];
   __shared__ double row_sums[NORM ? 2 : 1][NORM ? MAXT / 64 : 1];   // RMSNorm: the waves' sums of squares, by row parity
   static_assert(EPL == 32 || EPL == 16, "one or two lanes per block");
@@ -326,12 +328,10 @@ reorder_quant_dma_kernel(const uint8_t* __restrict__ x, const int16_t* __restric
     qbase = (seg == 0 ? qn : (seg == 1 ? qs : qo)) + (in_tile ? (size_t)(j >> 2) * 16384 : (size_t)rows * whole * 64) + (j & 3) * 16;
     pitch = in_tile ? (size_t)whole * 16384 : (size_t)((kseg >> 5) & 3) * 16;   // per tile, or per row
   }
-  if constexpr (KEEP) {
-    if (a_staged != 0) {   // stage by stage
-      const bool in_stage = (j >> 2) < whole;
-      qbase = (seg == 0 ? qn : (seg == 1 ? qs : qo)) + (size_t)(in_stage ? j >> 2 : whole) * a_staged * (4 * blk_bytes) + (j & 3) * blk_bytes;
-      pitch = (size_t)(in_stage ? 4 : (kseg >> 5) & 3) * blk_bytes;
-    }
+  if constexpr (STAGED) {
+    const bool in_stage = (j >> 2) < whole;
+    qbase = (seg == 0 ? qn : (seg == 1 ? qs : qo)) + (size_t)(in_stage ? j >> 2 : whole) * a_staged * (4 * blk_bytes) + (j & 3) * blk_bytes;
+    pitch = (size_t)(in_stage ? 4 : (kseg >> 5) & 3) * blk_bytes;
   }
   uint8_t* sfbase = seg == 0 ? sfn : (seg == 1 ? sfs : sfo);
 
@@ -641,6 +641,7 @@ hipError_t launch_reorder_quant(const void* x, const int16_t* idx, int rows, int
                                 const void* gamma, float eps, bool keep_codes, int a_staged, int src_rows, unsigned* verdict, hipStream_t stream) {
   if (rows == 0 || K == 0) return hipSuccess;
   if ((gamma != nullptr && IS_W) || (verdict != nullptr && !IS_W) || (src_rows != 0 && (!IS_W || src_rows > rows || rows % 256 != 0))) return hipErrorInvalidValue;
+  if (a_staged != 0 && (IS_W || !keep_codes || a_staged < rows)) return hipErrorInvalidValue;
   const uint16_t* gm = static_cast<const uint16_t*>(gamma);
   const int threads = ((K >> 5) + 63) & ~63;
   const uint8_t* xb = static_cast<const uint8_t*>(x);
@@ -668,7 +669,7 @@ hipError_t launch_reorder_quant(const void* x, const int16_t* idx, int rows, int
     err = allow_dynamic_lds(reinterpret_cast<const void*>(kernel), usable);
     if (err != hipSuccess) return;
     hipLaunchKernelGGL(kernel, dim3(grid), dim3(nthreads), (size_t)lds, stream, xb, idx, rows, K, KN, KS, KO, qn, qs, qo, sfn,
-                       sfs, sfo, sched, gm, eps, 1.0 / K, src_rows, a_staged, verdict);
+                       sfs, sfo, sched, gm, eps, 1.0 / K, src_rows, verdict, a_staged);
     err = hipGetLastError();
   };
   // Measured on M = 4096 ... 16384 rows of K = 3584 ... 18944: two row slots per workgroup, and per CU up to four
@@ -715,7 +716,9 @@ hipError_t launch_reorder_quant(const void* x, const int16_t* idx, int rows, int
   };
   // keep: the codes stay in the L2 for the kernel that reads them next (activations only); norm: RMSNorm of the row
   // before the gather (activations only; its codes are always kept: what follows a norm is the layer's GEMM)
-  auto dispatch = [&](auto keep_c, auto norm_c, auto tiled_c) {
+  // staged: those codes stage by stage
+  auto dispatch = [&](auto keep_c, auto norm_c, auto tiled_c, auto staged_c) {
+    constexpr bool ST = decltype(staged_c)::value;
     constexpr bool TI = decltype(tiled_c)::value;
     constexpr bool KP = decltype(keep_c)::value;
     constexpr bool NM = decltype(norm_c)::value;
@@ -723,10 +726,7 @@ hipError_t launch_reorder_quant(const void* x, const int16_t* idx, int rows, int
     if constexpr (!IS_W) {
       auto parts = [&](auto t_c) {
         constexpr int T = decltype(t_c)::value;
-        auto kernel = reorder_quant_part_kernel<T, KP, NM, false>;
-        if constexpr (KP) {
-          if (a_staged != 0) kernel = reorder_quant_part_kernel<T, KP, NM, true>;
-        }
+        const auto kernel = reorder_quant_part_kernel<T, KP, NM, ST>;
         const int lds = ((K >> 3) + T - 1) / T * T * 16 * (NM ? 2 : 1);   // the row, and the RMSNorm's weight
         if (lds > usable) { err = hipErrorInvalidValue; return; }
         err = allow_dynamic_lds(reinterpret_cast<const void*>(kernel), usable);
@@ -744,20 +744,20 @@ hipError_t launch_reorder_quant(const void* x, const int16_t* idx, int rows, int
     }
     if (K <= 8192) {
       switch (t2) {
-        case 64: launch_dma(reorder_quant_dma_kernel<16, 64, kNS, IS_W, 64, KP, NM, TI>, 16, kNS, 64, kPerCu); break;
-        case 128: launch_dma(reorder_quant_dma_kernel<16, 128, kNS, IS_W, 128, KP, NM, TI>, 16, kNS, 128, kPerCu); break;
-        case 192: launch_dma(reorder_quant_dma_kernel<16, 192, kNS, IS_W, 192, KP, NM, TI>, 16, kNS, 192, kPerCu); break;
-        case 256: launch_dma(reorder_quant_dma_kernel<16, 256, kNS, IS_W, 256, KP, NM, TI>, 16, kNS, 256, kPerCu); break;
-        case 320: launch_dma(reorder_quant_dma_kernel<16, 320, kNS, IS_W, 320, KP, NM, TI>, 16, kNS, 320, kPerCu); break;
-        case 384: launch_dma(reorder_quant_dma_kernel<16, 384, kNS, IS_W, 384, KP, NM, TI>, 16, kNS, 384, kPerCu); break;
-        case 448: launch_dma(reorder_quant_dma_kernel<16, 448, kNS, IS_W, 448, KP, NM, TI>, 16, kNS, 448, kPerCu); break;
-        default: launch_dma(reorder_quant_dma_kernel<16, 512, kNS, IS_W, 512, KP, NM, TI>, 16, kNS, 512, kPerCu); break;
+        case 64: launch_dma(reorder_quant_dma_kernel<16, 64, kNS, IS_W, 64, KP, NM, TI, ST>, 16, kNS, 64, kPerCu); break;
+        case 128: launch_dma(reorder_quant_dma_kernel<16, 128, kNS, IS_W, 128, KP, NM, TI, ST>, 16, kNS, 128, kPerCu); break;
+        case 192: launch_dma(reorder_quant_dma_kernel<16, 192, kNS, IS_W, 192, KP, NM, TI, ST>, 16, kNS, 192, kPerCu); break;
+        case 256: launch_dma(reorder_quant_dma_kernel<16, 256, kNS, IS_W, 256, KP, NM, TI, ST>, 16, kNS, 256, kPerCu); break;
+        case 320: launch_dma(reorder_quant_dma_kernel<16, 320, kNS, IS_W, 320, KP, NM, TI, ST>, 16, kNS, 320, kPerCu); break;
+        case 384: launch_dma(reorder_quant_dma_kernel<16, 384, kNS, IS_W, 384, KP, NM, TI, ST>, 16, kNS, 384, kPerCu); break;
+        case 448: launch_dma(reorder_quant_dma_kernel<16, 448, kNS, IS_W, 448, KP, NM, TI, ST>, 16, kNS, 448, kPerCu); break;
+        default: launch_dma(reorder_quant_dma_kernel<16, 512, kNS, IS_W, 512, KP, NM, TI, ST>, 16, kNS, 512, kPerCu); break;
       }
     } else if (!IS_W && two_lanes(t2, NM, KP)) {
       if constexpr (!IS_W) {
         auto wide = [&](auto t_c) {
           constexpr int T2 = decltype(t_c)::value;
-          launch_dma(reorder_quant_dma_kernel<16, T2, kNS, IS_W, T2, KP, NM, TI>, 16, kNS, T2, kPerCu, !NM && (T2 == 704 || T2 == 768) ? 24 : 16);
+          launch_dma(reorder_quant_dma_kernel<16, T2, kNS, IS_W, T2, KP, NM, TI, ST>, 16, kNS, T2, kPerCu, !NM && (T2 == 704 || T2 == 768) ? 24 : 16);
         };
         switch (t2) {
           case 576: wide(std::integral_constant<int, 576>{}); break;
@@ -776,24 +776,28 @@ hipError_t launch_reorder_quant(const void* x, const int16_t* idx, int rows, int
       // one lane per block: the workgroups are large enough as it is, and LDS (two rows per workgroup) bounds how
       // many a CU holds
       switch (threads) {
-        case 320: launch_dma(reorder_quant_dma_kernel<32, 320, kNS, IS_W, 320, KP, NM, TI>, 32, kNS, 320, kPerCu); break;
-        case 384: launch_dma(reorder_quant_dma_kernel<32, 384, kNS, IS_W, 384, KP, NM, TI>, 32, kNS, 384, kPerCu); break;
-        case 448: launch_dma(reorder_quant_dma_kernel<32, 448, kNS, IS_W, 448, KP, NM, TI>, 32, kNS, 448, kPerCu); break;
-        case 512: launch_dma(reorder_quant_dma_kernel<32, 512, kNS, IS_W, 512, KP, NM, TI>, 32, kNS, 512, kPerCu); break;
-        case 576: launch_dma(reorder_quant_dma_kernel<32, 576, kNS, IS_W, 576, KP, NM, TI>, 32, kNS, 576, kPerCu); break;
-        default: launch_dma(reorder_quant_dma_kernel<32, 640, kNS, IS_W, 640, KP, NM, TI>, 32, kNS, 640, kPerCu); break;
+        case 320: launch_dma(reorder_quant_dma_kernel<32, 320, kNS, IS_W, 320, KP, NM, TI, ST>, 32, kNS, 320, kPerCu); break;
+        case 384: launch_dma(reorder_quant_dma_kernel<32, 384, kNS, IS_W, 384, KP, NM, TI, ST>, 32, kNS, 384, kPerCu); break;
+        case 448: launch_dma(reorder_quant_dma_kernel<32, 448, kNS, IS_W, 448, KP, NM, TI, ST>, 32, kNS, 448, kPerCu); break;
+        case 512: launch_dma(reorder_quant_dma_kernel<32, 512, kNS, IS_W, 512, KP, NM, TI, ST>, 32, kNS, 512, kPerCu); break;
+        case 576: launch_dma(reorder_quant_dma_kernel<32, 576, kNS, IS_W, 576, KP, NM, TI, ST>, 32, kNS, 576, kPerCu); break;
+        default: launch_dma(reorder_quant_dma_kernel<32, 640, kNS, IS_W, 640, KP, NM, TI, ST>, 32, kNS, 640, kPerCu); break;
       }
     } else {
-      launch_dma(reorder_quant_dma_kernel<32, 0, 2, IS_W, 1024, KP, NM, TI>, 32, 2, threads, kPerCu);
+      launch_dma(reorder_quant_dma_kernel<32, 0, 2, IS_W, 1024, KP, NM, TI, ST>, 32, 2, threads, kPerCu);
     }
   };
+  const std::true_type yes;
+  const std::false_type no;
   if constexpr (IS_W) {
-    if (src_rows != 0) dispatch(std::false_type{}, std::false_type{}, std::true_type{});
-    else dispatch(std::false_type{}, std::false_type{}, std::false_type{});
+    if (src_rows != 0) dispatch(no, no, yes, no);
+    else dispatch(no, no, no, no);
   } else {
-    if (gamma != nullptr) dispatch(std::true_type{}, std::true_type{}, std::false_type{});
-    else if (keep_codes) dispatch(std::true_type{}, std::false_type{}, std::false_type{});
-    else dispatch(std::false_type{}, std::false_type{}, std::false_type{});
+    if (a_staged != 0 && gamma != nullptr) dispatch(yes, yes, no, yes);
+    else if (a_staged != 0) dispatch(yes, no, no, yes);
+    else if (gamma != nullptr) dispatch(yes, yes, no, no);
+    else if (keep_codes) dispatch(yes, no, no, no);
+    else dispatch(no, no, no, no);
   }
   return err;
 }

@@ -121,6 +121,18 @@ def test_layer_calls_on_small_tiles_equal_quantize_then_gemm(abi, tf, tt, m, n, 
     _check_layer_call(abi, m, n, kn, ks, ko, norm)
 
 
+# Codes stage by stage out of every instance of the quantizer for many rows: its workgroup sizes with two lanes per block and with one, without RMSNorm
+# and with it, one row per workgroup and two; the last stage of every segment is not whole.
+@pytest.mark.parametrize("m", [256, 261, 531])
+@pytest.mark.parametrize("k", [1024 * i - 32 for i in range(1, 17)] + [18400, 20448, 20512, 32736])
+@pytest.mark.parametrize("norm", [False, True])
+def test_layer_calls_of_every_width_equal_quantize_then_gemm(abi, m, k, norm):
+    kn, ko = k * 5 // 8 // 128 * 128 + 32, max(k // 8 // 128, 1) * 128 + 96
+    cus = torch.cuda.get_device_properties(0).multi_processor_count
+    assert abi.weights_tileable(256, kn, k - kn - ko, ko) and abi.gemm_kernel(m, 256, kn, k - kn - ko, ko, True, cus)[0] == "tile"
+    _check_layer_call(abi, m, 256, kn, k - kn - ko, ko, norm)
+
+
 def _check_layer_call(abi, m, n, kn, ks, ko, norm):
     print("staged codes", m, n, kn, ks, ko, norm, flush=True)
     k, g = kn + ks + ko, torch.Generator(device=DEV).manual_seed(m + kn)
