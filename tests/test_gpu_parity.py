@@ -105,6 +105,23 @@ def test_few_rows(abi, rows, k):
         _check_kept_codes(abi, rows, k)
 
 
+# As many rows as CUs and more, which the kernel for few rows above does not take: the codes kept in the caches for the GEMM of a layer call, row by row, out of
+# every workgroup size with two lanes per block and with one (at most 255 rows, those of the wide rows and of a single token above included, are few).
+@pytest.mark.parametrize("rows", [256, 257, 641])
+@pytest.mark.parametrize("k", [1024, 2048, 3072, 4096, 5120, 6144, 7168, 8192, 8224, 9248, 10240, 10272, 11264, 11296, 12288, 12320, 13344, 14368, 15392, 16384,
+                               16416, 18432, 18944, 20480, 20512])
+def test_kept_codes_of_many_rows(abi, rows, k):
+    _say("kept codes", rows, k, 0, 0)
+    _check_kept_codes(abi, rows, k)
+
+
+# Rows of up to 1023 blocks, each with a workgroup of a size known at run time (704 and 1024 lanes), without RMSNorm: row by row and kept.
+@pytest.mark.parametrize("rows,k", [(193, 22560), (193, 32736), (257, 32736), (520, 32736)])
+def test_widest_rows(abi, rows, k):
+    test_reorder_quantize_matches_oracle(abi, "x", rows, *_wide_split(k))
+    _check_kept_codes(abi, rows, k)
+
+
 # The same instances with more rows than both slots of every workgroup hold, so that slots are filled again and the RMSNorm's sums change
 # places: one workgroup per CU has three or four of 900 rows (9 and 10 waves: of 1000 without RMSNorm), two per CU, with 11 and 12 waves and no
 # RMSNorm, two or three of 1100.

@@ -133,6 +133,30 @@ def test_layer_calls_of_every_width_equal_quantize_then_gemm(abi, m, k, norm):
     _check_layer_call(abi, m, 256, kn, k - kn - ko, ko, norm)
 
 
+# Codes stage by stage out of every instance of the quantizer for fewer rows than CUs: parts of 256 lanes, one to four of a row, and of 512, three and
+# four (more than 256 parts of more than 16384 channels), with RMSNorm where that takes the kernel; on small tiles of each size and on whole ones; segments
+# that end in a whole stage and 1 to 3 blocks behind one.
+@pytest.mark.parametrize("kernel,m,n,kn,ks,ko", [
+    (("tile", 64, 64), 52, 8448, 11808, 6496, 640), (("tile", 64, 64), 52, 12544, 11776, 6560, 608), (("tile", 128, 64), 100, 12544, 12832, 6400, 1280),
+    (("tile", 128, 64), 100, 12544, 12800, 6720, 992), (("tile", 64, 64), 190, 2816, 20448, 10240, 2048), (("tile", 64, 64), 51, 8448, 11808, 6496, 640),
+    (("tile", 64, 64), 64, 8448, 8960, 4928, 448), (("tile", 64, 64), 60, 8448, 8992, 4896, 448), (("tile", 64, 64), 200, 2816, 2560, 1408, 128),
+    (("tile", 128, 64), 200, 4352, 2592, 1376, 160), (("tile", 128, 128), 255, 8448, 1632, 736, 544), (("tile", 64, 64), 255, 2816, 1248, 608, 192),
+    (("whole", 256, 256), 200, 16640, 2560, 1408, 128), (("whole", 256, 256), 255, 16640, 1120, 544, 384)])
+@pytest.mark.parametrize("norm", [False, True])
+def test_layer_calls_of_few_rows_equal_quantize_then_gemm(abi, kernel, m, n, kn, ks, ko, norm):
+    cus = torch.cuda.get_device_properties(0).multi_processor_count
+    assert abi.weights_tileable(n, kn, ks, ko) and abi.gemm_kernel(m, n, kn, ks, ko, True, cus) == kernel
+    _check_layer_call(abi, m, n, kn, ks, ko, norm)
+
+
+# The tiles that the layer calls above are meant for.
+@pytest.mark.parametrize("tf,tt,m,n", [(64, 64, 262, 256), (64, 64, 70, 5632), (128, 64, 145, 5632), (128, 64, 460, 2304), (128, 128, 399, 4864)])
+@pytest.mark.parametrize("kn,ks,ko", [(1664, 640, 384), (1632, 736, 544), (2432, 0, 256), (0, 2176, 384), (2560, 1408, 128), (4160, 2144, 288)])
+def test_layer_calls_take_their_small_tile(abi, tf, tt, m, n, kn, ks, ko):
+    cus = torch.cuda.get_device_properties(0).multi_processor_count
+    assert abi.gemm_kernel(m, n, kn, ks, ko, True, cus) == ("tile", tf, tt)
+
+
 def _check_layer_call(abi, m, n, kn, ks, ko, norm):
     print("staged codes", m, n, kn, ks, ko, norm, flush=True)
     k, g = kn + ks + ko, torch.Generator(device=DEV).manual_seed(m + kn)
