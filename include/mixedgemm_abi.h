@@ -151,8 +151,13 @@ int mg_padded_rows(int M);
  * Activation reorder-quantize followed by the mixed GEMM on the same stream
  * (the sequence src/bindings.cpp:69-186 then :9-67 performs with a device-wide
  * synchronize in between; bench_reorder_gemm.cu:163-167 times the same pair).
- * `workspace` receives the quantized activations and their scales, in the order in which the GEMM of the shape reads them;
- * mg_fused_workspace_bytes(M, KN, KS, KO) bytes, 256-byte aligned.
+ * `workspace`: mg_fused_workspace_bytes(M, KN, KS, KO) bytes, 256-byte aligned.  It receives the quantized activations and their
+ * scales, unless the call is done in one launch (few tokens), which writes nothing there: with R = mg_padded_rows(M), the codes of
+ * the E2M1, E3M2 and E4M3 segments, room for R rows each, then the scales of the three, mg_sf_bytes(R, kseg, MG_OPERAND_A) each,
+ * every part on the next multiple of 256 bytes.  Scales are as mg_reorder_quantize_x writes them, and so are codes, row by row, but
+ * for more than 16 tokens and R < 2^25 where mg_gemm_kernel says MG_KERNEL_WHOLE, or MG_KERNEL_TILE on tile-major weights: there
+ * each whole 128-wide stage of a segment has R rows of its 64, 96 or 128 bytes one after the other, stage after stage, and the 1 to
+ * 3 blocks past the last whole stage follow as R rows of their own.  Rows M and up are not written.
  */
 int mg_fused_linear(const void* x_bf16, const int16_t* idx,
                     const uint8_t* bn, const uint8_t* bs, const uint8_t* bo,
