@@ -627,8 +627,8 @@ reorder_quant_part_kernel(const uint8_t* __restrict__ x, const int16_t* __restri
 // a_staged != 0 (activations whose codes are kept): the codes of a segment stage by stage, as a GEMM on tiles copies them -- per whole
 // 128-wide stage `a_staged` rows (at least `rows`) of 64, 96 or 128 bytes one after the other, behind them rows of the blocks past the last whole
 // stage.  A copy of 16 rows is then one run of whole lines; row-major, a row's 64 bytes of a stage are half a line and its 96 bytes lie in
-// two, so that the GEMM fetched every line of E2M1 codes twice.  A row's stores are 64-byte pieces apart here, and the rows that share
-// a line are neighbours, on one XCD.  Layer calls, us, row-major -> stage by stage, one layer over and over / six in turn: M = 777, N = 5000, K = 5120 all
+// two, so that the GEMM fetched every line of E2M1 codes twice.  A row's stores are 64-byte pieces apart here; of neighbouring rows that share
+// a line, the kernel for many rows has runs of eight on one XCD, whose L2 puts the lines together, the one for few rows each on another XCD, as parts of lines.  Layer calls, us, row-major -> stage by stage, one layer over and over / six in turn: M = 777, N = 5000, K = 5120 all
 // E2M1 30.2 -> 28.4 / 30.2 -> 28.2; M = 2048, N = 4096, K = 14336 77.5 -> 76.3 / 85.2 -> 79.8, row-major weights 88.7 -> 82.9 / 103 -> 95; M = 4096, N =
 // 14336, K = 4096 126.2 -> 123.7 / 131.0 -> 126.7; M = 4096, N = K = 5120 74.9 -> 70.8 / 78.7 -> 73.0.  On small tiles (tile-major weights; before, long
 // launches copied batches of rows): M = 256, N = K = 4096 10.9 -> 10.5 / 11.4 -> 11.0, M = 1024 19.6 -> 19.0 / 19.8 -> 19.4; M = 700, N = 4096, K = 5120 21.1
@@ -680,27 +680,27 @@ hipError_t launch_reorder_quant(const void* x, const int16_t* idx, int rows, int
   // Activations of 8192 < K <= 16384 with two lanes per block as well, i.e. 9 ... 16 waves per workgroup, where that is the faster way or level with the
   // rows in the caches, where the kernel before left them, and from HBM (us, one lane per block against two, from the caches / from HBM; two runs of one
   // side differ by 1 %).  Without RMSNorm:
-  //   9 and 10 waves, one workgroup per CU: K = 9216 rows 16 4.35 against 4.05 / 3.95 against 3.7, 128 4.55, 4.25 / 4.35, 4.3, 256 4.4, 4.4 / 4.4, 4.45, 512
-  //     5.05, 5.4 / 6.1, 6.35, 640 7.2, 6.75 / 7.9, 7.55, 1024 8.2, 7.8 / 10.4, 8.9, 1025 8.2, 8.55 / 10.4, 9.4, 1600 9.9, 11.4 / 12.4, 12.25, 4096 22.2, 22.7 /
+  //   9 and 10 waves, one workgroup per CU: K = 9216 rows 256 4.4 against 4.4 / 4.4 against 4.45, 512 5.05, 5.4 / 6.1, 6.35, 640 7.2, 6.75 / 7.9, 7.55, 1024 8.2, 7.8 / 10.4, 8.9, 1025 8.2, 8.55 / 10.4, 9.4, 1600 9.9, 11.4 / 12.4, 12.25, 4096 22.2, 22.7 /
   //     24.6, 23.25; K = 10240 1024 8.1, 8.1 / 10.9, 9.3, 2048 13.1, 13.9 / 15.0, 14.4 (three per CU: 2048 rows of 9216 15 % slower than one lane);
-  //   11 and 12 waves, two per CU: K = 12288 rows 16 4.35, 4.15 / 3.95, 3.85, 256 4.55, 4.35 / 4.85, 4.65, 512 5.3, 5.6 / 6.9, 6.4, 1024 7.8, 7.6 / 10.0, 9.15, 1600
+  //   11 and 12 waves, two per CU: K = 12288 rows 256 4.55, 4.35 / 4.85, 4.65, 512 5.3, 5.6 / 6.9, 6.4, 1024 7.8, 7.6 / 10.0, 9.15, 1600
   //     11.0, 11.5 / 13.15, 12.4, 2048 13.7, 12.9 / 15.2, 14.2, 8192 45.9, 40.0 / 52.3, 49.1; K = 11008 1700 10.45, 10.7 / 12.55, 12.1, 4096 22.6, 20.8 / 25.4, 23.9;
-  //   13 ... 16 waves, one per CU: K = 14336 rows 16 4.45, 4.4 / 4.1, 4.15, 256 4.75, 4.75 / 5.2, 5.1, 320 5.5, 6.1 / 7.1, 6.95, 1024 9.1, 9.3 / 11.4, 11.3, 1600 12.8, 14.9 /
+  //   13 ... 16 waves, one per CU: K = 14336 rows 256 4.75, 4.75 / 5.2, 5.1, 320 5.5, 6.1 / 7.1, 6.95, 1024 9.1, 9.3 / 11.4, 11.3, 1600 12.8, 14.9 /
   //     15.3, 15.6, 3500 24.3, 24.6 / 27.7, 26.4, 4096 27.1, 27.2 / 32.0, 29.8, 8192 52.0, 49.5 / 61.3, 55.3; K = 12800 4096 25.3, 26.0 / 28.85, 27.15, 6144 36.4, 36.1 / 42.55,
   //     38.2; K = 15360 2560 20.1, 19.6 / 23.4, 22.2, K = 16384 2048 17.0, 17.35 / 20.2, 19.3, 3072 24.2, 22.9 / 27.6, 26.0 (two per CU: up to 15 % slower).
-  // With RMSNorm, whose form for one lane per block normalizes the row in place: K = 9216 rows 16 5.6, 5.5 / 5.4, 5.3, 512 9.8, 8.4 / 11.0, 8.8, 2048 28.5, 23.55 / 29.6,
-  // 23.8; K = 12288 16 6.25, 5.75 / 5.85, 5.45, 2048 30.4, 24.4 / 31.3, 24.7; K = 14336 128 6.35, 6.6 / 6.85, 6.65, 256 6.6, 6.85 / 7.3, 7.05, 257 10.3, 9.35 / 11.7, 9.5, 2048
+  // With RMSNorm, whose form for one lane per block normalizes the row in place: K = 9216 rows 512 9.8, 8.4 / 11.0, 8.8, 2048 28.5, 23.55 / 29.6,
+  // 23.8; K = 12288 2048 30.4, 24.4 / 31.3, 24.7; K = 14336 128 6.35, 6.6 / 6.85, 6.65, 256 6.6, 6.85 / 7.3, 7.05, 257 10.3, 9.35 / 11.7, 9.5, 2048
   // 31.9, 28.4 / 33.0, 28.7; K = 12800 4096 51.0, 50.8 / 52.1, 51.0, 8192 93.8, 96.5 / 94.6, 96.6 (up to K = 15360: the LDS offsets of its three rows are
   // immediates).
-  // (Fewer rows than CUs without RMSNorm do not get here: few_rows.)  Codes kept for the GEMM that follows, gain of two lanes per layer call (N = 4096): 9 and 10 waves, 1 ... 128 rows 1 ... 5 % / 0 ... 3 %, 512 -2 % / -1 %, 2048 and
-  // 4096 -1 % / 0.5 %; 11 and 12, 1 ... 900 rows 0 ... 4 % / 0 ... 4 %, from 1300 on 0 / 1 %; 13 ... 16, up to 256 rows 0 ... 2 % / 0 ... 2 %, 512 -1 % / 0, 2048 and 4096 -2 % / -1 ... 1 %.
+  // Codes kept for the GEMM that follows, gain of two lanes per layer call (N = 4096): 9 and 10 waves, 512 rows -2 % / -1 %, 2048 and 4096 -1 % / 0.5 %; 11 and 12, up
+  // to 900 rows 0 ... 4 % / 0 ... 4 %, from 1300 on 0 / 1 %; 13 ... 16, 256 rows 0 ... 2 % / 0 ... 2 %, 512 -1 % / 0, 2048 and 4096 -2 % / -1 ... 1 %.
   auto two_lanes = [&](int t2, bool norm, bool kept) {
     const int64_t r = rows, cus = lim.cus;
     if (norm) return t2 <= 768 || (t2 <= 960 && r > cus && (t2 > 832 || r <= 16 * cus));
     if (t2 > 1024) return false;
+    // (no RMSNorm: fewer rows than CUs have gone to few_rows)
     if (t2 < 704) return !kept && 2 * r >= 5 * cus && r <= 4 * cus;
-    if (t2 <= 768) return kept || r <= cus || r >= 4 * cus;
-    return r <= cus || (!kept && r >= (t2 == 832 ? 24 : t2 == 896 ? 16 : 12) * cus);
+    if (t2 <= 768) return kept || r == cus || r >= 4 * cus;
+    return r == cus || (!kept && r >= (t2 == 832 ? 24 : t2 == 896 ? 16 : 12) * cus);
   };
   // Fewer rows than CUs go to the kernel for few rows (from there on the workgroups of the other one are arranged so that an L2 puts the lines
   // of scales together: K = 4096, 256 rows 3.01 us there, 3.06 here, 255 rows 3.32 and 3.10); of more than 20480 channels three quarters as many (K =
@@ -757,7 +757,10 @@ hipError_t launch_reorder_quant(const void* x, const int16_t* idx, int rows, int
       if constexpr (!IS_W) {
         auto wide = [&](auto t_c) {
           constexpr int T2 = decltype(t_c)::value;
-          launch_dma(reorder_quant_dma_kernel<16, T2, kNS, IS_W, T2, KP, NM, TI, ST>, 16, kNS, T2, kPerCu, !NM && (T2 == 704 || T2 == 768) ? 24 : 16);
+          if constexpr (NM ? T2 <= 960 : !KP || T2 >= 704)   // what two_lanes sends here
+            launch_dma(reorder_quant_dma_kernel<16, T2, kNS, IS_W, T2, KP, NM, TI, ST>, 16, kNS, T2, kPerCu, !NM && (T2 == 704 || T2 == 768) ? 24 : 16);
+          else
+            err = hipErrorInvalidValue;
         };
         switch (t2) {
           case 576: wide(std::integral_constant<int, 576>{}); break;
@@ -767,21 +770,26 @@ hipError_t launch_reorder_quant(const void* x, const int16_t* idx, int rows, int
           case 832: wide(std::integral_constant<int, 832>{}); break;
           case 896: wide(std::integral_constant<int, 896>{}); break;
           case 960: wide(std::integral_constant<int, 960>{}); break;
-          default:
-            if constexpr (!NM) wide(std::integral_constant<int, 1024>{});
-            break;
+          default: wide(std::integral_constant<int, 1024>{}); break;
         }
       }
     } else if (K <= 20480) {
       // one lane per block: the workgroups are large enough as it is, and LDS (two rows per workgroup) bounds how
       // many a CU holds
+      auto one_lane = [&](auto t_c) {
+        constexpr int T = decltype(t_c)::value;
+        if constexpr (NM ? T > 384 : !KP || T != 384)   // what two_lanes leaves
+          launch_dma(reorder_quant_dma_kernel<32, T, kNS, IS_W, T, KP, NM, TI, ST>, 32, kNS, T, kPerCu);
+        else
+          err = hipErrorInvalidValue;
+      };
       switch (threads) {
-        case 320: launch_dma(reorder_quant_dma_kernel<32, 320, kNS, IS_W, 320, KP, NM, TI, ST>, 32, kNS, 320, kPerCu); break;
-        case 384: launch_dma(reorder_quant_dma_kernel<32, 384, kNS, IS_W, 384, KP, NM, TI, ST>, 32, kNS, 384, kPerCu); break;
-        case 448: launch_dma(reorder_quant_dma_kernel<32, 448, kNS, IS_W, 448, KP, NM, TI, ST>, 32, kNS, 448, kPerCu); break;
-        case 512: launch_dma(reorder_quant_dma_kernel<32, 512, kNS, IS_W, 512, KP, NM, TI, ST>, 32, kNS, 512, kPerCu); break;
-        case 576: launch_dma(reorder_quant_dma_kernel<32, 576, kNS, IS_W, 576, KP, NM, TI, ST>, 32, kNS, 576, kPerCu); break;
-        default: launch_dma(reorder_quant_dma_kernel<32, 640, kNS, IS_W, 640, KP, NM, TI, ST>, 32, kNS, 640, kPerCu); break;
+        case 320: one_lane(std::integral_constant<int, 320>{}); break;
+        case 384: one_lane(std::integral_constant<int, 384>{}); break;
+        case 448: one_lane(std::integral_constant<int, 448>{}); break;
+        case 512: one_lane(std::integral_constant<int, 512>{}); break;
+        case 576: one_lane(std::integral_constant<int, 576>{}); break;
+        default: one_lane(std::integral_constant<int, 640>{}); break;
       }
     } else {
       launch_dma(reorder_quant_dma_kernel<32, 0, 2, IS_W, 1024, KP, NM, TI, ST>, 32, 2, threads, kPerCu);
