@@ -206,15 +206,16 @@ struct RowSchedule {
 // tiles) are quantized as zeros.  A row's stores are then 64-byte pieces 16 KB apart instead of one run; the two rows that
 // share a line go to workgroups of one XCD, whose L2 joins them, and the pass is as fast as the row-major one:
 // W[14336, 4096] 38.7 us for quantizing and tiling one after the other, 24.6 in one pass (6.0 TB/s of what it has to move).
-// STAGED: the codes stage by stage (see launch_reorder_quant).  (Asked for at run time, every call whose codes are kept paid for it, most where the launch is all
-// there is: M = 8, N = 14336, K = 4096 with RMSNorm 10.80 us, 10.75 without.)
-template <int EPL, int T, int NS, bool IS_W, int MAXT, bool KEEP = false, bool NORM = false, bool TILED = false, bool STAGED = false>
+// STAGED: a_staged says whether the codes go stage by stage (see launch_reorder_quant), without a branch, and the addresses are worked out while the index
+// is on its way.  Behind the wait for it, where the compiler does that by itself (with an instance for each order, too), M = 1055, N = 384, K = 4096 with RMSNorm
+// is 14.35 us instead of 14.12, M = 1024, N = K = 4096 18.3 instead of 18.05.
+template <int EPL, int T, int NS, bool IS_W, int MAXT, bool KEEP = false, bool NORM = false, bool TILED = false, bool STAGED = KEEP>
 __global__ void __launch_bounds__(MAXT)
 reorder_quant_dma_kernel(const uint8_t* __restrict__ x, const int16_t* __restrict__ idx, int rows, int K, int KN, int KS,
                          int KO, uint8_t* __restrict__ qn, uint8_t* __restrict__ qs, uint8_t* __restrict__ qo,
                          uint8_t* __restrict__ sfn, uint8_t* __restrict__ sfs, uint8_t* __restrict__ sfo, RowSchedule sched,
-                         const uint16_t* __restrict__ gamma, float eps, double inv_k, int src_rows, unsigned* __restrict__ verdict,
-                         int a_staged) {
+                         const uint16_t* __restrict__ gamma, float eps, double inv_k, int src_rows, int a_staged,
+                         unsigned* __restrict__ verdict) {
   extern __shared__ __align__(16) uint8_t lds[];
   __shared__ double row_sums[NORM ? 2 : 1][NORM ? MAXT / 64 : 1];   // RMSNorm: the waves' sums of squares, by row parity
   static_assert(EPL == 32 || EPL == 16, "one or two lanes per block");
@@ -328,12 +329,13 @@ reorder_quant_dma_kernel(const uint8_t* __restrict__ x, const int16_t* __restric
     qbase = (seg == 0 ? qn : (seg == 1 ? qs : qo)) + (in_tile ? (size_t)(j >> 2) * 16384 : (size_t)rows * whole * 64) + (j & 3) * 16;
     pitch = in_tile ? (size_t)whole * 16384 : (size_t)((kseg >> 5) & 3) * 16;   // per tile, or per row
   }
-  if constexpr (STAGED) {
-    const bool in_stage = (j >> 2) < whole;
-    qbase = (seg == 0 ? qn : (seg == 1 ? qs : qo)) + (size_t)(in_stage ? j >> 2 : whole) * a_staged * (4 * blk_bytes) + (j & 3) * blk_bytes;
-    pitch = (size_t)(in_stage ? 4 : (kseg >> 5) & 3) * blk_bytes;
-  }
   uint8_t* sfbase = seg == 0 ? sfn : (seg == 1 ? sfs : sfo);
+  // Stage by stage: of a_staged rows each.  Row by row (0) is the same with one row, but for the pitch: no branch.
+  if constexpr (STAGED) {
+    qbase = (seg == 0 ? qn : (seg == 1 ? qs : qo)) + (size_t)(j >> 2) * max(a_staged, 1) * (4 * blk_bytes) + (j & 3) * blk_bytes;
+    pitch = (size_t)(a_staged == 0 ? kseg >> 5 : (j >> 2) < whole ? 4 : (kseg >> 5) & 3) * blk_bytes;
+    asm volatile("" : "+v"(qbase), "+v"(pitch), "+v"(sfbase));   // before the wait for the index
+  }
 
   // ---- the index entries are the oldest requests: they are there when at most the row copies are in flight
   wait_vm(kPieces * min(NS, count) + (kLate ? kPieces : 0));
@@ -669,7 +671,7 @@ hipError_t launch_reorder_quant(const void* x, const int16_t* idx, int rows, int
     err = allow_dynamic_lds(reinterpret_cast<const void*>(kernel), usable);
     if (err != hipSuccess) return;
     hipLaunchKernelGGL(kernel, dim3(grid), dim3(nthreads), (size_t)lds, stream, xb, idx, rows, K, KN, KS, KO, qn, qs, qo, sfn,
-                       sfs, sfo, sched, gm, eps, 1.0 / K, src_rows, verdict, a_staged);
+                       sfs, sfo, sched, gm, eps, 1.0 / K, src_rows, a_staged, verdict);
     err = hipGetLastError();
   };
   // Measured on M = 4096 ... 16384 rows of K = 3584 ... 18944: two row slots per workgroup, and per CU up to four
@@ -707,7 +709,8 @@ hipError_t launch_reorder_quant(const void* x, const int16_t* idx, int rows, int
   // 28672, 192 rows 6.60, 6.35, 255 7.16, 7.43).  Above 16384 channels and a workgroup of 4096 channels per CU with 8192 channels in each (K = 18944,
   // 64 rows 3.66 with 4096, 3.55, 255 5.85, 5.18 (the other kernel 5.93); K = 28672, 64 rows 3.89, 3.62, 128 5.88, 4.70 (5.92)).  With RMSNorm, where
   // every workgroup of a row sums all of it, at most a workgroup per CU (K = 8192, 128 rows 4.61, 4.14, 255 4.73, 4.98; K = 18944, 64 rows
-  // 6.92, 8.49), and not 2048 < K <= 4096 (3.72, 3.67, but a layer call of M = 8, N = 14336, K = 4096 10.7 -> 10.9 launched one by one).
+  // 6.92, 8.49), and not 2048 < K <= 4096, on one measurement (alone 3.72, 3.67, but the layer call M = 8, N = 14336, K = 4096 10.7 -> 10.9 launched one by one; other
+  // sizes of that band were not timed).
   const int64_t parts_of_4096 = (int64_t)rows * ((K + 4095) >> 12);
   auto few_rows = [&](bool norm) {
     // (the copies of the norm's weight want it aligned)
@@ -716,9 +719,7 @@ hipError_t launch_reorder_quant(const void* x, const int16_t* idx, int rows, int
   };
   // keep: the codes stay in the L2 for the kernel that reads them next (activations only); norm: RMSNorm of the row
   // before the gather (activations only; its codes are always kept: what follows a norm is the layer's GEMM)
-  // staged: those codes stage by stage
-  auto dispatch = [&](auto keep_c, auto norm_c, auto tiled_c, auto staged_c) {
-    constexpr bool ST = decltype(staged_c)::value;
+  auto dispatch = [&](auto keep_c, auto norm_c, auto tiled_c) {
     constexpr bool TI = decltype(tiled_c)::value;
     constexpr bool KP = decltype(keep_c)::value;
     constexpr bool NM = decltype(norm_c)::value;
@@ -726,7 +727,10 @@ hipError_t launch_reorder_quant(const void* x, const int16_t* idx, int rows, int
     if constexpr (!IS_W) {
       auto parts = [&](auto t_c) {
         constexpr int T = decltype(t_c)::value;
-        const auto kernel = reorder_quant_part_kernel<T, KP, NM, ST>;
+        auto kernel = reorder_quant_part_kernel<T, KP, NM, false>;
+        if constexpr (KP) {
+          if (a_staged != 0) kernel = reorder_quant_part_kernel<T, KP, NM, true>;
+        }
         const int lds = ((K >> 3) + T - 1) / T * T * 16 * (NM ? 2 : 1);   // the row, and the RMSNorm's weight
         if (lds > usable) { err = hipErrorInvalidValue; return; }
         err = allow_dynamic_lds(reinterpret_cast<const void*>(kernel), usable);
@@ -744,21 +748,21 @@ hipError_t launch_reorder_quant(const void* x, const int16_t* idx, int rows, int
     }
     if (K <= 8192) {
       switch (t2) {
-        case 64: launch_dma(reorder_quant_dma_kernel<16, 64, kNS, IS_W, 64, KP, NM, TI, ST>, 16, kNS, 64, kPerCu); break;
-        case 128: launch_dma(reorder_quant_dma_kernel<16, 128, kNS, IS_W, 128, KP, NM, TI, ST>, 16, kNS, 128, kPerCu); break;
-        case 192: launch_dma(reorder_quant_dma_kernel<16, 192, kNS, IS_W, 192, KP, NM, TI, ST>, 16, kNS, 192, kPerCu); break;
-        case 256: launch_dma(reorder_quant_dma_kernel<16, 256, kNS, IS_W, 256, KP, NM, TI, ST>, 16, kNS, 256, kPerCu); break;
-        case 320: launch_dma(reorder_quant_dma_kernel<16, 320, kNS, IS_W, 320, KP, NM, TI, ST>, 16, kNS, 320, kPerCu); break;
-        case 384: launch_dma(reorder_quant_dma_kernel<16, 384, kNS, IS_W, 384, KP, NM, TI, ST>, 16, kNS, 384, kPerCu); break;
-        case 448: launch_dma(reorder_quant_dma_kernel<16, 448, kNS, IS_W, 448, KP, NM, TI, ST>, 16, kNS, 448, kPerCu); break;
-        default: launch_dma(reorder_quant_dma_kernel<16, 512, kNS, IS_W, 512, KP, NM, TI, ST>, 16, kNS, 512, kPerCu); break;
+        case 64: launch_dma(reorder_quant_dma_kernel<16, 64, kNS, IS_W, 64, KP, NM, TI>, 16, kNS, 64, kPerCu); break;
+        case 128: launch_dma(reorder_quant_dma_kernel<16, 128, kNS, IS_W, 128, KP, NM, TI>, 16, kNS, 128, kPerCu); break;
+        case 192: launch_dma(reorder_quant_dma_kernel<16, 192, kNS, IS_W, 192, KP, NM, TI>, 16, kNS, 192, kPerCu); break;
+        case 256: launch_dma(reorder_quant_dma_kernel<16, 256, kNS, IS_W, 256, KP, NM, TI>, 16, kNS, 256, kPerCu); break;
+        case 320: launch_dma(reorder_quant_dma_kernel<16, 320, kNS, IS_W, 320, KP, NM, TI>, 16, kNS, 320, kPerCu); break;
+        case 384: launch_dma(reorder_quant_dma_kernel<16, 384, kNS, IS_W, 384, KP, NM, TI>, 16, kNS, 384, kPerCu); break;
+        case 448: launch_dma(reorder_quant_dma_kernel<16, 448, kNS, IS_W, 448, KP, NM, TI>, 16, kNS, 448, kPerCu); break;
+        default: launch_dma(reorder_quant_dma_kernel<16, 512, kNS, IS_W, 512, KP, NM, TI>, 16, kNS, 512, kPerCu); break;
       }
     } else if (!IS_W && two_lanes(t2, NM, KP)) {
       if constexpr (!IS_W) {
         auto wide = [&](auto t_c) {
           constexpr int T2 = decltype(t_c)::value;
           if constexpr (NM ? T2 <= 960 : !KP || T2 >= 704)   // what two_lanes sends here
-            launch_dma(reorder_quant_dma_kernel<16, T2, kNS, IS_W, T2, KP, NM, TI, ST>, 16, kNS, T2, kPerCu, !NM && (T2 == 704 || T2 == 768) ? 24 : 16);
+            launch_dma(reorder_quant_dma_kernel<16, T2, kNS, IS_W, T2, KP, NM, TI>, 16, kNS, T2, kPerCu, !NM && (T2 == 704 || T2 == 768) ? 24 : 16);
           else
             err = hipErrorInvalidValue;
         };
@@ -779,7 +783,7 @@ hipError_t launch_reorder_quant(const void* x, const int16_t* idx, int rows, int
       auto one_lane = [&](auto t_c) {
         constexpr int T = decltype(t_c)::value;
         if constexpr (NM ? T > 384 : !KP || T != 384)   // what two_lanes leaves
-          launch_dma(reorder_quant_dma_kernel<32, T, kNS, IS_W, T, KP, NM, TI, ST>, 32, kNS, T, kPerCu);
+          launch_dma(reorder_quant_dma_kernel<32, T, kNS, IS_W, T, KP, NM, TI>, 32, kNS, T, kPerCu);
         else
           err = hipErrorInvalidValue;
       };
@@ -792,20 +796,23 @@ hipError_t launch_reorder_quant(const void* x, const int16_t* idx, int rows, int
         default: one_lane(std::integral_constant<int, 640>{}); break;
       }
     } else {
-      launch_dma(reorder_quant_dma_kernel<32, 0, 2, IS_W, 1024, KP, NM, TI, ST>, 32, 2, threads, kPerCu);
+      launch_dma(reorder_quant_dma_kernel<32, 0, 2, IS_W, 1024, KP, NM, TI>, 32, 2, threads, kPerCu);
     }
   };
   const std::true_type yes;
   const std::false_type no;
   if constexpr (IS_W) {
-    if (src_rows != 0) dispatch(no, no, yes, no);
-    else dispatch(no, no, no, no);
+    if (src_rows != 0) dispatch(no, no, yes);
+    else dispatch(no, no, no);
   } else {
-    if (a_staged != 0 && gamma != nullptr) dispatch(yes, yes, no, yes);
-    else if (a_staged != 0) dispatch(yes, no, no, yes);
-    else if (gamma != nullptr) dispatch(yes, yes, no, no);
-    else if (keep_codes) dispatch(yes, no, no, no);
-    else dispatch(no, no, no, no);
+    // Up to 16 rows, whose GEMMs take codes row by row and whose launch is all there is, nobody asks for their order: M = 8, N = 14336, K = 4096 with
+    // RMSNorm 10.75 us instead of 10.85 (other widths go to few_rows).
+    const bool decoded = gamma != nullptr && a_staged == 0 && rows <= 16 && K > 2048 && K <= 4096;
+    if (gamma != nullptr && !decoded) dispatch(yes, yes, no);
+    else if (keep_codes && !decoded) dispatch(yes, no, no);
+    else if (!decoded) dispatch(no, no, no);
+    else if (K <= 3072) launch_dma(reorder_quant_dma_kernel<16, 192, kNS, IS_W, 192, true, true, false, false>, 16, kNS, 192, kPerCu);
+    else launch_dma(reorder_quant_dma_kernel<16, 256, kNS, IS_W, 256, true, true, false, false>, 16, kNS, 256, kPerCu);
   }
   return err;
 }
