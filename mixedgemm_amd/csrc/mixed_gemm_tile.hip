@@ -3,22 +3,23 @@
 //
 // What bounded such launches on 256 x 128 tiles was not the memory (a tile alone on the chip took 0.30 us per stage of 128 K elements):
 // a global -> LDS copy holds the wave that issues it for ~64 cycles (its addresses go out one per cycle; a CU accepts one
-// from each of its SIMDs at a time, 1 KB per 16 cycles in all, whatever rows it is put together from, as long as the lines are in
-// the L2), so that waves that copy and multiply in turn leave the matrix cores idle.  Here four waves, one per SIMD, issue
-// all copies, eight waves, two per SIMD, read fragments and multiply, and one barrier hands over WS stages at a time, each of them the
-// work of 8 / WS of the math waves (fragments are read once per 2 x 2 tiles of 32 x 32 rather than once per 1 x 2).
-// What bounds it now: with many stages the copies (address unit busy 72 % of the cycles on tile-major and 77 % on row-major weights at
-// M = 256, N = 4096, K = 14336, where the matrix cores are 19 and 16 %, the LDS's fragment reads 25 %), with 32 stages latency as well
-// (address unit 45 ... 65 %, waves waiting 50 ... 63 %; M = 1024, N = K = 4096: matrix cores 29 and 25 %).  Clock stamps of an instrumented
-// build: 64 x 64 tiles, K = 4096, one per CU: 270 cycles per stage, of which 64 are MFMAs' (150 without copies); a launch of them takes 1.2
+// from each of its SIMDs at a time, 1 KB per 16 cycles in all where it is put together from whole lines that are in the L2), so that waves that
+// copy and multiply in turn leave the matrix cores idle.  Here four waves, one per SIMD, issue all copies, eight waves, two per SIMD, read
+// fragments and multiply, and one barrier hands over WS stages at a time, each of them the work of 8 / WS of the math waves (fragments are read
+// once per 2 x 2 tiles of 32 x 32 rather than once per 1 x 2).
+// What bounds it now: with many stages the copies (M = 256, N = 4096, K = 14336: address unit busy 65 ... 69 % of the cycles, matrix cores 18 ... 21 %, the
+// LDS's fragment reads 24 ... 28 %), with 32 stages latency as well (address unit 36 ... 51 %, waves waiting 52 ... 68 %; M = 1024, N = K = 4096: matrix
+// cores 27 ... 32 %).  An instruction takes the address unit 19 ... 26 cycles with the tokens' codes stage by stage, 22 ... 32 row by row, of which 1 ... 11 and
+// 10 ... 34 % are stalls on the cache behind it.  Clock stamps of an instrumented build, copies stage by stage of codes row by
+// row: 64 x 64 tiles, K = 4096, one per CU: 270 cycles per stage, of which 64 are MFMAs' (150 without copies); a launch of them takes 1.2
 // us until the first stages have landed, 2.7 us for 20 E2M1 and 1.3 for 12 later stages, 1.2 us to add the partial sums and store.
 // Tile-major / row-major weights, of two or three layers in turn in the caches, before (skinny kernel or 256 x 128 tiles) -> now, us:
 //   M = 256, N = 4096, K = 4096: 16.4 / 19.6 -> 8.3 / 8.6;   K = 14336: 45.6 / 59.9 -> 20.2 / 22.3
 //   M = 512, N = 4096, K = 4096: 16.6 / 19.6 -> 10.0 / 12.0;  N = 1024, K = 8192: 27.6 / 34.8 -> 11.6 / 13.2
 //   M = 64, N = 14336, K = 4096: 16.4 / 16.8 -> 8.8 / 9.3;   M = 128: 16.8 / 20.1 -> 10.1 / 12.3
 //   M = 1024, N = 4096, K = 4096: 17.0 / 19.7 -> 14.5 / 16.5
-// and, with batches copied as rows of their stages (BatchRow): K = 14336, M = 256 17.5 / 18.7;  M = 1024, K = 4096 12.6 / 13.1
-// (from HBM: M = 256 10.6 / 10.8 and 30 / 30, M = 512 12.5 / 15.2 and 16.1 / 16.0, M = 64 13.7 / 14.1, M = 1024 17.6 / 19.2)
+// (from HBM: M = 256 10.6 / 10.8 and 30 / 30, M = 512 12.5 / 15.2 and 16.1 / 16.0, M = 64 13.7 / 14.1, M = 1024 17.6 / 19.2), all of these
+// stage by stage on row-major codes; with batches copied as rows of their stages (BatchRow): K = 14336, M = 256 17.5 / 18.7;  M = 1024, K = 4096 12.6 / 13.1
 // Tiles of 256 x 128 with the same division of work were level with the mixed waves of the 256 x 256 kernel (M = 2048, N =
 // 4096, K = 12288: 57.6 against 56.3 us: 15 % fewer cycles at a clock as much lower; the chip is at its power limit there), tiles of
 // 64 and 128 x 32 slower than 64 x 64 at every shape tried.

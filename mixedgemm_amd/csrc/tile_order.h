@@ -50,10 +50,11 @@ inline TileOrder tile_order(int tiles_n, int tiles_m, int tf, int tt) {
   return o;
 }
 
-// What the small-tile GEMM is launched with: tile_order, but runs along the features where those of an XCD are fewer operand bytes per stage (many
+// What the small-tile GEMM is launched with: tile_order, but runs along the features where those of an XCD are four fifths of the operand bytes per stage or less (many
 // tokens of few features: 51 x 10 tiles in runs along the tokens had every L2 fetch nearly all tokens).  GEMM alone, us: M = 6430, N = 1280, K = 12288 66.0 -> 50.5
 // (tile-major), 78.0 -> 60.2 (row-major); M = 3694, N = 896, K = 7872 26.8 -> 21.0; M = 2874, N = 1152, K = 4096 12.6 -> 10.8; M = 1339, N = 640, K = 1792 6.3 -> 5.4; of
-// 76 calls of 256 ... 6500 tokens 26 have such runs and gain 7 % in the mean, the others are as before.
+// 76 calls of 256 ... 6500 tokens 26 have such runs and gain 7 % in the mean, the others are as before.  Only where they are a fifth fewer: 14 calls with 2 ... 19 %
+// fewer are level either way (at most 3 %, 0.5 % in the mean, as much as two runs of one side).
 inline TileOrder cheapest_order(int tiles_n, int tiles_m, int tf, int tt) {
   TileOrder o = tile_order(tiles_n, tiles_m, tf, tt);
   if (o.xlog >= 0) return o;
