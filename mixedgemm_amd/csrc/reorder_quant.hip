@@ -7,12 +7,11 @@
 //   scale  = 2^e, e = min{e : amax <= MAX * 2^e}  (= ceil(log2(amax/MAX)), :180),
 //            0.5 for an all-zero block (:179); E8M0 byte = e + 127
 //   code   = RNE_fmt( bf16( clamp( roundf(x / scale) ) ) )   (:221-248)
-// The design is not the reference's: a workgroup stages R rows at a time into
-// LDS in channel-major order with the R rows of one channel adjacent, so one
-// 2R-byte LDS read fetches a gathered channel for all R rows; one lane owns one
-// 32-element block (no cross-lane reduction), the scale exponent comes from
-// integer arithmetic on the float bits, and the element conversion is done by
-// the gfx950 cvt_scalef32 instructions on the already integer-rounded values.
+// The design is not the reference's: rows go global -> LDS directly, as they are
+// in memory, one or two lanes own a 32-element block and gather its channels
+// from there, the scale exponent comes from integer arithmetic on the float
+// bits, and the element conversion is done by the gfx950 cvt_scalef32
+// instructions on the already integer-rounded values.
 #include <type_traits>
 
 #include "mg_common.h"
@@ -631,7 +630,7 @@ reorder_quant_part_kernel(const uint8_t* __restrict__ x, const int16_t* __restri
 // stage.  A copy of 16 rows is then one run of whole lines; row-major, a row's 64 bytes of a stage are half a line and its 96 bytes lie in
 // two, so that the GEMM fetched every line of E2M1 codes twice.  A row's stores are 64-byte pieces apart here; of neighbouring rows that share
 // a line, the kernel for many rows has runs of eight on one XCD, whose L2 puts the lines together, the one for few rows each on another XCD, as parts of lines.  Layer calls, us, row-major -> stage by stage, one layer over and over / six in turn: M = 777, N = 5000, K = 5120 all
-// E2M1 30.2 -> 28.4 / 30.2 -> 28.2; M = 2048, N = 4096, K = 14336 77.5 -> 76.3 / 85.2 -> 79.8, row-major weights 88.7 -> 82.9 / 103 -> 95; M = 4096, N =
+// E2M1 30.2 -> 28.4 / 30.2 -> 28.2; M = 2048, N = 4096, K = 14336 level (0.99 ... 1.014 times as fast over four machines) / 85.2 -> 79.8, row-major weights 88.7 -> 82.9 / 103 -> 95; M = 4096, N =
 // 14336, K = 4096 126.2 -> 123.7 / 131.0 -> 126.7; M = 4096, N = K = 5120 74.9 -> 70.8 / 78.7 -> 73.0.  On small tiles (tile-major weights; before, long
 // launches copied batches of rows): M = 256, N = K = 4096 10.9 -> 10.5 / 11.4 -> 11.0, M = 1024 19.6 -> 19.0 / 19.8 -> 19.4; M = 700, N = 4096, K = 5120 21.1
 // -> 19.6 / 21.2 -> 19.5; M = 140, N = 18944, K = 8192 32.2 -> 30.7 / 44.5 -> 42.8.  The same bits in all of them.
